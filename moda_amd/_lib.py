@@ -117,6 +117,24 @@ def load():
     return lib
 
 
+_host = None
+
+
+def host():
+    """The native host module (csrc/host.cpp), loaded once, after the kernel library it calls."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise MissingLibraryError(
+                f"{os.path.join(_HERE, '_host.so')} does not load ({e}): build it with "
+                f"`make -C {os.path.join(_HERE, 'csrc')}`. moda_amd has no Python fallback for it.") from e
+        _host = module
+    return _host
+
+
 def check(rc: int, what: str):
     if rc != 0:
         msg = load().moda_hip_strerror(rc).decode()

@@ -12,7 +12,9 @@ argument meaning, assertions and return conventions -- on top of the C ABI of
   * ``parallel_attn`` (fla/ops/attn/parallel.py:678-730), the plain causal comparator.
 
 Tensors stay torch tensors; torch is used for allocation, streams and autograd
-only.  Every compute step is a HIP kernel of the shared library.
+only.  Every compute step is a HIP kernel of the shared library; the host work of
+a call (contract checks, descriptor, allocation, launch, autograd node) is native
+(``csrc/host.cpp``), this file is the interface.
 """
 from __future__ import annotations
 
@@ -34,21 +36,15 @@ _DTYPES = {torch.bfloat16: _lib.BF16, torch.float16: _lib.FP16, torch.float32: _
 # 10-bit mantissa (TF32) and accumulates in fp32 -- fp16 has the same mantissa; its range (6e-8 .. 65504) is the
 # caller's responsibility, "bf16" trades three mantissa bits for the fp32 range.
 _FP32_COMPUTE = "fp32"
-_FP32_COMPUTE_TYPES = {"fp16": torch.float16, "bf16": torch.bfloat16}
 
 
 def set_fp32_compute(mode: str) -> str:
     """Choose how fp32 tensors are computed ("fp32", "fp16" or "bf16", see above); returns the previous setting."""
     global _FP32_COMPUTE
     assert mode in ("fp32", "fp16", "bf16"), f"unknown fp32 compute mode {mode!r}"
+    _lib.host().set_fp32_compute({"fp32": _lib.FP32, "fp16": _lib.FP16, "bf16": _lib.BF16}[mode])
     previous, _FP32_COMPUTE = _FP32_COMPUTE, mode
     return previous
-
-
-def _narrowed(*xs):
-    """fp32 tensors -> the 16-bit compute type chosen with set_fp32_compute (None stays None)."""
-    t = _FP32_COMPUTE_TYPES[_FP32_COMPUTE]
-    return tuple(None if x is None else x.to(t) for x in xs)
 
 
 # Query rows per chunk of the chunk-visible variant when the caller does not
@@ -76,18 +72,23 @@ def _packed(cu_seqlens, q: torch.Tensor, rows_per_token: int) -> Optional[Packed
     (the longest sequence sizes the launch); pass the returned PackedBatch instead of the tensor to reuse it."""
     if cu_seqlens is None or isinstance(cu_seqlens, PackedBatch):
         return cu_seqlens
-    assert q.shape[0] == 1, "with cu_seqlens all sequences share one packed row axis: batch size must be 1"
-    assert cu_seqlens.dim() == 1 and cu_seqlens.numel() >= 1, "cu_seqlens must be a vector of n+1 offsets"
-    host = cu_seqlens.detach().to("cpu", torch.int64)
-    lens = host[1:] - host[:-1]
-    assert int(host[0]) == 0 and bool((lens >= 0).all()), "cu_seqlens must start at 0 and not decrease"
-    total = int(host[-1])
-    assert total * rows_per_token == q.shape[1], (
-        f"cu_seqlens ends at {total} base tokens but q holds {q.shape[1]} rows "
-        f"({rows_per_token} per token)")
-    cu = cu_seqlens.detach().to(device=q.device, dtype=torch.int32).contiguous()
-    host_arr = (ctypes.c_int32 * host.numel())(*host.tolist())
-    return PackedBatch(cu, int(lens.numel()), int(lens.max()) if lens.numel() else 0, total, host_arr)
+    p = _lib.host().pack(cu_seqlens, q, rows_per_token)
+    return PackedBatch(p.cu, p.n, p.max_len, p.total, (ctypes.c_int32 * (p.n + 1))(*p.host))
+
+
+def _native_packed(p: Optional[PackedBatch]):
+    if p is None:
+        return None
+    return _lib.host().Packed(p.cu, p.n, p.max_len, p.total, list(p.host) if p.host is not None else [])
+
+
+def _offsets(cu_seqlens):
+    """``cu_seqlens`` of a public call -> the two arguments the native call takes it as: a tensor, or a PackedBatch."""
+    if cu_seqlens is None:
+        return None, None
+    if isinstance(cu_seqlens, PackedBatch):
+        return None, _native_packed(cu_seqlens)
+    return cu_seqlens, None
 
 
 def _ptr(x: Optional[torch.Tensor]):
@@ -96,28 +97,6 @@ def _ptr(x: Optional[torch.Tensor]):
 
 def _stream(x: torch.Tensor):
     return ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
-
-
-def _usable(x: Optional[torch.Tensor], vec16: bool = True) -> Optional[torch.Tensor]:
-    """Return ``x`` if the kernels can read it in place (unit inner stride, 16-byte
-    aligned rows), else a contiguous copy -- the reference's ``@contiguous``
-    (fla/utils.py:130-164) made a copy of every non-contiguous input.  ``vec16=False``: the
-    vector-ALU kernels, which load element by element and take any non-negative strides."""
-    if x is None:
-        return None
-    if not vec16:
-        ok = x.dim() == 4 and (x.stride(3) == 1 or x.shape[3] == 1) and all(x.stride(i) >= 0 for i in range(3))
-        return x if ok else x.contiguous()
-    m = 16 // x.element_size()
-    ok = (
-        x.dim() == 4
-        and (x.stride(3) == 1 or x.shape[3] == 1)
-        and all(x.stride(i) % m == 0 for i in range(3))
-        and x.data_ptr() % 16 == 0
-        and all(x.stride(i) >= 0 for i in range(3))
-        and x.stride(1) * x.element_size() < (1 << 24)  # row offsets inside a tile are 32-bit
-    )
-    return x if ok else x.contiguous()
 
 
 def _matrix_core_path(q: torch.Tensor, val: torch.Tensor, packed: Optional["PackedBatch"] = None) -> bool:
@@ -195,92 +174,15 @@ def _desc(mode, q, k, v, kd, vd, G, L, chunk_tokens, scale, o=None, do=None, dq=
     return d
 
 
-def _same_dtype(*xs):
-    dt = None
-    for x in xs:
-        if x is None:
-            continue
-        if dt is None:
-            dt = x.dtype
-        elif x.dtype != dt:
-            raise TypeError(f"all tensors must share one dtype, got {dt} and {x.dtype}")
-
-
 def _check_shapes(mode, q, k, v, kd, vd, G, o=None, do=None, lse=None):
-    """The C ABI takes bare pointers: it derives every extent from ``k`` (or ``q``), ``G`` and the depth
-    row count and cannot see what the buffers really hold.  A mismatch would be an out-of-bounds access
-    on the device, so every extent is checked here, before any launch.  Returns ``(T, L)``."""
-    assert q.dim() == 4, "q must be [B, rows, heads, D]"
-    B = q.shape[0]
-    assert G >= 1, "moda_group_num must be positive"
-    if mode == _lib.DEPTH_ONLY:
-        assert k is None and v is None, "depth-only attention takes no sequence k/v"
-        assert kd is not None and vd is not None, "depth-only attention needs the depth k/v"
-        assert q.shape[1] % G == 0, "query rows must be a multiple of moda_group_num"
-        T, H = q.shape[1] // G, kd.shape[2]
-        assert q.shape[2] == H, "q and depth k/v must have the same number of heads"
-    else:
-        assert k is not None and v is not None and k.dim() == 4 and v.dim() == 4, "k, v must be [B, T, H, D]"
-        T, H = k.shape[1], k.shape[2]
-        assert k.shape[0] == B and v.shape[0] == B, "batch sizes of q, k, v differ"
-        assert v.shape[1] == T and v.shape[2] == H, "k and v must agree in tokens and heads"
-        assert k.shape[3] == q.shape[3], "q and k must share the head dim"
-        if mode == _lib.PLAIN_GQA:
-            assert q.shape[1] == T and q.shape[2] == H * G, "plain GQA: q must be [B, T, H*G, D]"
-        else:
-            assert q.shape[2] == H, "folded layout: q and k must have the same number of heads"
-            assert q.shape[1] == T * G, f"q holds {q.shape[1]} rows, expected T*moda_group_num = {T * G}"
-    L = 0
-    if kd is not None or vd is not None:
-        assert kd is not None and vd is not None, "depth k and v must be given together"
-        assert kd.dim() == 4 and vd.dim() == 4, "depth k/v must be [B, T*L, H, D]"
-        assert kd.shape[0] == B and vd.shape[0] == B, "depth k/v batch size differs from q"
-        assert kd.shape[2] == H and vd.shape[2] == H, "depth k/v head count mismatch"
-        assert kd.shape[3] == q.shape[3], "depth k must share q's head dim"
-        assert vd.shape[1] == kd.shape[1], "depth k and v must have the same number of rows"
-        if T > 0:
-            assert kd.shape[1] % T == 0, "depth rows must be T * L"
-            L = kd.shape[1] // T
-        else:
-            assert kd.shape[1] == 0, "depth rows must be T * L"
-        if v is not None:
-            assert vd.shape[3] == v.shape[3], "v and depth v must share the value head dim"
-    Dv = (vd if mode == _lib.DEPTH_ONLY else v).shape[3]
-    for name, x in (("o", o), ("do", do)):
-        if x is not None:
-            assert tuple(x.shape) == (B, q.shape[1], q.shape[2], Dv), f"{name} must be {(B, q.shape[1], q.shape[2], Dv)}"
-    if lse is not None:
-        assert tuple(lse.shape) == (B, q.shape[1], q.shape[2]) and lse.dtype == torch.float32, \
-            "lse must be fp32 [B, rows, heads]"
-    return T, L
+    """Every extent the kernels derive from ``k`` (or ``q``), ``G`` and the depth row count, checked against what the
+    tensors hold.  Returns ``(T, L)``."""
+    return _lib.host().check_shapes(mode, q, k, v, kd, vd, G, o, do, lse)
 
 
 def _raw_fwd(mode, q, k, v, kd, vd, scale, G, chunk_tokens=0, depth_valid=None, packed=None):
     """Launch the forward kernels. Returns (o, lse)."""
-    if q.dtype == torch.float32 and _FP32_COMPUTE != "fp32":
-        o, lse = _raw_fwd(mode, *_narrowed(q, k, v, kd, vd), scale, G, chunk_tokens, depth_valid, packed)
-        return o.float(), lse
-    _check_shapes(mode, q, k, v, kd, vd, G)
-    _check_device(q)
-    _same_dtype(q, k, v, kd, vd)
-    vec16 = _matrix_core_path(q, vd if mode == _lib.DEPTH_ONLY else v, packed)
-    q, k, v, kd, vd = (_usable(x, vec16) for x in (q, k, v, kd, vd))
-    src = kd if mode == _lib.DEPTH_ONLY else k
-    T = q.shape[1] // G if mode == _lib.DEPTH_ONLY else k.shape[1]
-    L = (kd.shape[1] // T) if (kd is not None and T > 0) else 0
-    if kd is not None and T == 0:
-        L = 0
-    val = vd if mode == _lib.DEPTH_ONLY else v
-    o = torch.empty(q.shape[0], q.shape[1], q.shape[2], val.shape[-1], dtype=val.dtype, device=q.device)
-    lse = torch.empty(q.shape[0], q.shape[1], q.shape[2], dtype=torch.float32, device=q.device)
-    if L == 0:
-        kd = vd = None
-    d = _desc(mode, q, k, v, kd, vd, G, L, chunk_tokens, scale, o=o, depth_valid=depth_valid, packed=packed)
-    with torch.cuda.device(q.device):
-        rc = _lib.load().moda_hip_fwd(ctypes.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(kd), _ptr(vd), _ptr(o),
-                                      _ptr(lse), _stream(q))
-    _lib.check(rc, "moda_hip_fwd")
-    return o, lse
+    return _lib.host().forward(mode, q, k, v, kd, vd, scale, G, chunk_tokens, depth_valid, _native_packed(packed))
 
 
 def _raw_bwd(mode, q, k, v, kd, vd, o, lse, do, scale, G, chunk_tokens=0, stages=_lib.STAGE_ALL, out=None, ws=None,
@@ -291,52 +193,8 @@ def _raw_bwd(mode, q, k, v, kd, vd, o, lse, do, scale, G, chunk_tokens=0, stages
     value) and ``ws`` (a workspace tensor) let the caller reuse buffers across calls.
     ``accumulate_depth``: the depth gradients are ADDED to the ``dkd, dvd`` given in ``out`` (slots
     ``>= depth_valid`` untouched) instead of overwriting them."""
-    assert not accumulate_depth or (out is not None and out[3] is not None and out[4] is not None), \
-        "accumulate_depth needs the gradient buffers to add to"
-    if q.dtype == torch.float32 and _FP32_COMPUTE != "fp32":
-        # 16-bit gradients from the matrix kernels (without the accumulate flag: the slots without data come back
-        # as zeros), widened into the caller's fp32 buffers or added to them
-        got = _raw_bwd(mode, *_narrowed(q, k, v, kd, vd, o), lse, *_narrowed(do), scale, G, chunk_tokens, stages,
-                       None, None, depth_valid, packed, False)
-        if out is None:
-            return tuple(None if g_ is None else g_.float() for g_ in got)
-        for i, (dst, g_) in enumerate(zip(out, got)):
-            if dst is not None:
-                dst.add_(g_) if (accumulate_depth and i >= 3) else dst.copy_(g_)
-        return tuple(out)
-    _check_shapes(mode, q, k, v, kd, vd, G, o=o, do=do, lse=lse)
-    _check_device(q)
-    _same_dtype(q, k, v, kd, vd, o, do)
-    vec16 = _matrix_core_path(q, vd if mode == _lib.DEPTH_ONLY else v, packed)
-    q, k, v, kd, vd, o, do = (_usable(x, vec16) for x in (q, k, v, kd, vd, o, do))
-    lse = lse.contiguous()
-    T = q.shape[1] // G if mode == _lib.DEPTH_ONLY else k.shape[1]
-    L = (kd.shape[1] // T) if (kd is not None and T > 0) else 0
-    if out is not None:
-        dq, dk, dv, dkd, dvd = out
-        for g_, x_ in ((dq, q), (dk, k), (dv, v), (dkd, kd), (dvd, vd)):
-            assert (g_ is None) == (x_ is None) and (g_ is None or (g_.shape == x_.shape and g_.dtype == x_.dtype)), \
-                "reused gradient buffers must match their inputs in shape and dtype"
-    else:
-        dq = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-        dk = torch.empty(k.shape, dtype=k.dtype, device=q.device) if k is not None else None
-        dv = torch.empty(v.shape, dtype=v.dtype, device=q.device) if v is not None else None
-        dkd = torch.empty(kd.shape, dtype=kd.dtype, device=q.device) if kd is not None else None
-        dvd = torch.empty(vd.shape, dtype=vd.dtype, device=q.device) if vd is not None else None
-    kd_a, vd_a, dkd_a, dvd_a = (kd, vd, dkd, dvd) if L > 0 else (None, None, None, None)
-    d = _desc(mode, q, k, v, kd_a, vd_a, G, L, chunk_tokens, scale, o=o, do=do, dq=dq, dk=dk, dv=dv, dkd=dkd_a,
-              dvd=dvd_a, depth_valid=depth_valid, packed=packed, accumulate_depth=accumulate_depth and L > 0)
-    lib = _lib.load()
-    nbytes = lib.moda_hip_bwd_workspace_bytes(ctypes.byref(d))
-    if ws is None:
-        ws = torch.empty(max(int(nbytes), 4), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
-        rc = lib.moda_hip_bwd_stages(ctypes.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(kd_a), _ptr(vd_a), _ptr(o),
-                                     _ptr(lse), _ptr(do), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dkd_a), _ptr(dvd_a),
-                                     _ptr(ws), ctypes.c_size_t(ws.numel() * ws.element_size()), int(stages),
-                                     _stream(q))
-    _lib.check(rc, "moda_hip_bwd")
-    return dq, dk, dv, dkd, dvd
+    return _lib.host().backward(mode, q, k, v, kd, vd, o, lse, do, scale, G, chunk_tokens, depth_valid,
+                                _native_packed(packed), int(stages), out, ws, accumulate_depth)
 
 
 def bwd_workspace(mode, q, k, v, kd, vd, G, chunk_tokens=0, packed=None) -> torch.Tensor:
@@ -395,102 +253,42 @@ def parallel_moda_bwd(q, k, v, o, g_cumsum, lse, do, scale=None, chunk_size=128,
     return dq, dk, dv, None, dkd, dvd
 
 
-def _autograd_forward(ctx, fwd_impl, q, k, v, g, scale, cu_seqlens, cached_k, cached_v, moda_group_num, **kw):
+def _refuse_decay(g, q):
+    """``g`` (the reference's decay) is part of the signatures and unsupported, like there."""
+    assert g.shape[:3] == q.shape[:3], "g must be [B,T_q,HQ]"
     assert g is None, "g is not supported in this version"
-    packed = _packed(cu_seqlens, q, moda_group_num)
-    has_depth = cached_k is not None and cached_v is not None
-    if not has_depth:
-        cached_k = cached_v = None
-    o, lse = fwd_impl(q=q, k=k, v=v, g_cumsum=None, scale=scale, cu_seqlens=packed, cached_k=cached_k,
-                      cached_v=cached_v, moda_group_num=moda_group_num, **kw)
-    ctx.packed = packed
-    ctx.save_for_backward(q, k, v, o, lse, *([cached_k, cached_v] if has_depth else []))
-    ctx.has_depth = has_depth
-    ctx.scale = scale
-    ctx.moda_group_num = moda_group_num
-    ctx.kw = kw
-    return o.to(q.dtype), lse
 
 
-def _autograd_backward(ctx, bwd_impl, do):
-    if ctx.has_depth:
-        q, k, v, o, lse, cached_k, cached_v = ctx.saved_tensors
-    else:
-        q, k, v, o, lse = ctx.saved_tensors
-        cached_k = cached_v = None
-    dq, dk, dv, _, dkd, dvd = bwd_impl(q=q, k=k, v=v, o=o, g_cumsum=None, lse=lse, do=do.to(o.dtype), scale=ctx.scale,
-                                       cu_seqlens=ctx.packed, cached_k=cached_k, cached_v=cached_v,
-                                       moda_group_num=ctx.moda_group_num, **ctx.kw)
-    if not ctx.has_depth:
-        dkd = dvd = None
-    return dq.to(q), dk.to(k), dv.to(v), dkd, dvd
-
-
-class ParallelMixtureOfDepthAttentionFunction(torch.autograd.Function):
-    """moda_v14.py:2649-2789: 14 inputs, 14 gradients, gradient into ``lse`` ignored."""
+class ParallelMixtureOfDepthAttentionFunction:
+    """moda_v14.py:2649-2789, by its ``apply``: differentiable in q, k, v, cached_k, cached_v; the gradient into
+    ``lse`` is ignored.  (The autograd node itself is native: csrc/host.cpp, Attend.)"""
 
     @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda")
-    def forward(ctx, q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, is_causal=True,
-                group_bs=None, group_warps=None, depth_bs=None, depth_warps=None, depth_valid=None):
-        o, lse = _autograd_forward(ctx, parallel_moda_fwd, q, k, v, g, scale, cu_seqlens, cached_k, cached_v,
-                                   moda_group_num, is_causal=is_causal, depth_valid=depth_valid)
-        ctx.mark_non_differentiable(lse)
-        return o, lse
-
-    @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
-    def backward(ctx, do, dlse_unused):
-        dq, dk, dv, dkd, dvd = _autograd_backward(ctx, parallel_moda_bwd, do)
-        return dq, dk, dv, None, None, None, dkd, dvd, None, None, None, None, None, None, None
+    def apply(q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, is_causal=True,
+              group_bs=None, group_warps=None, depth_bs=None, depth_warps=None, depth_valid=None):
+        assert g is None, "g is not supported in this version"
+        cu, packed = _offsets(cu_seqlens)
+        return _lib.host().attend(_lib.CAUSAL if is_causal else _lib.NONCAUSAL, q, k, v, cached_k, cached_v, scale,
+                                  moda_group_num, 0, depth_valid, cu, packed, False, 128)
 
 
-def _prepare_inputs(api_name, q, k, v, g, cached_k, cached_v, scale, moda_group_num, head_first,
-                    return_depth_grads, warn_shape):
-    """Shared argument contract of parallel_moda (moda_v14.py:2817-2871) and
-    parallel_moda_chunk_visible (moda_v16.py:3496-3565)."""
-    if head_first:
-        q = q.transpose(1, 2)
-        k = k.transpose(1, 2)
-        v = v.transpose(1, 2)
-        if g is not None:
-            g = g.transpose(1, 2)
-        if cached_k is not None and cached_v is not None:
-            cached_k = cached_k.transpose(1, 2)
-            cached_v = cached_v.transpose(1, 2)
-    elif warn_shape and q.shape[1] < q.shape[2]:
-        warnings.warn(
-            f"[{api_name}] detected seq_len({q.shape[1]}) < num_heads({q.shape[2]}). "
-            "input may be in head_first format while head_first=True is not set."
-        )
-    B, T_q, HQ, Kdim = q.shape
-    T_kv = k.shape[1]
-    H = k.shape[2]
-    assert HQ == H, (
-        "Implicit head-dimension GQA is not allowed. "
-        "Please fold grouping only into `moda_group_num`: "
-        "use q.shape[2] == k.shape[2] and set T_q = T_kv * moda_group_num."
+def _head_last(*xs):
+    return tuple(x if x is None else x.transpose(1, 2) for x in xs)
+
+
+def _warn_layout(api_name, q):
+    warnings.warn(
+        f"[{api_name}] detected seq_len({q.shape[1]}) < num_heads({q.shape[2]}). "
+        "input may be in head_first format while head_first=True is not set.", stacklevel=3
     )
-    if scale is None:
-        scale = Kdim ** -0.5
-    if moda_group_num > 1:
-        assert T_q == T_kv * moda_group_num, "When moda_group_num > 1, T_q must equal T_kv * moda_group_num"
-    else:
-        assert T_q == T_kv, "When moda_group_num=1, T_q must equal T_kv"
-    if cached_k is not None and cached_v is not None:
-        assert cached_k.shape[0] == B and cached_v.shape[0] == B
-        assert cached_k.shape[2] == H and cached_v.shape[2] == H, "cached_k/v head count mismatch"
-        assert cached_k.shape[1] % T_kv == 0, "cached_k time dimension must be T_kv * L"
-        L = cached_k.shape[1] // T_kv
-        assert cached_v.shape[1] == T_kv * L, "cached_v shape mismatch"
-        if (cached_k.requires_grad or cached_v.requires_grad) and not return_depth_grads:
-            warnings.warn(
-                "cached_k/v requires gradients, but return_depth_grads=False. "
-                "Gradients are still computed and returned."
-            )
-    if g is not None:
-        assert g.shape[:3] == (B, T_q, HQ), "g must be [B,T_q,HQ]"
-    return q, k, v, g, cached_k, cached_v, scale
+
+
+def _warn_depth_grads(cached_k, cached_v):
+    if cached_k is not None and cached_v is not None and (cached_k.requires_grad or cached_v.requires_grad):
+        warnings.warn(
+            "cached_k/v requires gradients, but return_depth_grads=False. "
+            "Gradients are still computed and returned.", stacklevel=3
+        )
 
 
 def parallel_moda(q, k, v, g=None, cached_k=None, cached_v=None, scale=None, cu_seqlens=None, moda_group_num=1,
@@ -509,13 +307,18 @@ def parallel_moda(q, k, v, g=None, cached_k=None, cached_v=None, scale=None, cu_
     zero, and a preallocated cache (``DepthCache``) need not be rebuilt per layer.  The other slots are
     never read: they may hold anything (an uninitialised ``torch.empty`` buffer included).
     """
-    q, k, v, g, cached_k, cached_v, scale = _prepare_inputs(
-        "parallel_moda", q, k, v, g, cached_k, cached_v, scale, moda_group_num, head_first, return_depth_grads,
-        warn_shape)
-    o, lse = ParallelMixtureOfDepthAttentionFunction.apply(
-        q, k, v, g, scale, cu_seqlens, cached_k, cached_v, moda_group_num, is_causal, group_bs, group_warps, depth_bs,
-        depth_warps, depth_valid)
-    return (o, lse) if need_lse else o
+    if head_first:
+        q, k, v, g, cached_k, cached_v = _head_last(q, k, v, g, cached_k, cached_v)
+    elif warn_shape and q.shape[1] < q.shape[2]:
+        _warn_layout("parallel_moda", q)
+    if not return_depth_grads:
+        _warn_depth_grads(cached_k, cached_v)
+    if g is not None:
+        _refuse_decay(g, q)
+    cu, packed = _offsets(cu_seqlens)
+    out = _lib.host().attend(_lib.CAUSAL if is_causal else _lib.NONCAUSAL, q, k, v, cached_k, cached_v, scale,
+                             moda_group_num, 0, depth_valid, cu, packed, True, 128)
+    return out if need_lse else out[0]
 
 
 # ---------------------------------------------------------------------------
@@ -560,23 +363,16 @@ def parallel_moda_chunk_visible_bwd(q, k, v, o, g_cumsum, lse, do, scale=None, c
     return dq, dk, dv, None, dkd, dvd
 
 
-class ParallelMixtureOfDepthAttentionChunkVisibleFunction(torch.autograd.Function):
-    """moda_v16.py:3456-3493 (9 inputs)."""
+class ParallelMixtureOfDepthAttentionChunkVisibleFunction:
+    """moda_v16.py:3456-3493, by its ``apply``."""
 
     @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda")
-    def forward(ctx, q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1,
-                chunk_rows=None, depth_valid=None):
-        o, lse = _autograd_forward(ctx, parallel_moda_chunk_visible_fwd, q, k, v, g, scale, cu_seqlens, cached_k,
-                                   cached_v, moda_group_num, chunk_rows=chunk_rows, depth_valid=depth_valid)
-        ctx.mark_non_differentiable(lse)
-        return o, lse
-
-    @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
-    def backward(ctx, do, dlse_unused):
-        dq, dk, dv, dkd, dvd = _autograd_backward(ctx, parallel_moda_chunk_visible_bwd, do)
-        return dq, dk, dv, None, None, None, dkd, dvd, None, None, None
+    def apply(q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, chunk_rows=None,
+              depth_valid=None):
+        assert g is None, "g is not supported in this version"
+        cu, packed = _offsets(cu_seqlens)
+        return _lib.host().attend(_lib.CHUNK_VISIBLE, q, k, v, cached_k, cached_v, scale, moda_group_num,
+                                  _chunk_tokens(moda_group_num, chunk_rows), depth_valid, cu, packed, False, 0)
 
 
 def parallel_moda_chunk_visible(q, k, v, g=None, cached_k=None, cached_v=None, scale=None, cu_seqlens=None,
@@ -589,12 +385,18 @@ def parallel_moda_chunk_visible(q, k, v, g=None, cached_k=None, cached_v=None, s
     ``Cb = 64 // moda_group_num``.  The four ``customized_*`` arguments are accepted and dropped exactly as the
     reference's wrapper drops them (moda_v16.py:3646-3650: a chunk is 64 query rows whatever they say);
     ``chunk_rows``, which the reference does not have, selects another chunk size in query rows."""
-    q, k, v, g, cached_k, cached_v, scale = _prepare_inputs(
-        "parallel_moda_chunk_visible", q, k, v, g, cached_k, cached_v, scale, moda_group_num, head_first,
-        return_depth_grads, warn_shape)
-    o, lse = ParallelMixtureOfDepthAttentionChunkVisibleFunction.apply(
-        q, k, v, g, scale, cu_seqlens, cached_k, cached_v, moda_group_num, chunk_rows, depth_valid)
-    return (o, lse) if need_lse else o
+    if head_first:
+        q, k, v, g, cached_k, cached_v = _head_last(q, k, v, g, cached_k, cached_v)
+    elif warn_shape and q.shape[1] < q.shape[2]:
+        _warn_layout("parallel_moda_chunk_visible", q)
+    if not return_depth_grads:
+        _warn_depth_grads(cached_k, cached_v)
+    if g is not None:
+        _refuse_decay(g, q)
+    cu, packed = _offsets(cu_seqlens)
+    out = _lib.host().attend(_lib.CHUNK_VISIBLE, q, k, v, cached_k, cached_v, scale, moda_group_num,
+                             _chunk_tokens(moda_group_num, chunk_rows), depth_valid, cu, packed, True, 0)
+    return out if need_lse else out[0]
 
 
 # ---------------------------------------------------------------------------
@@ -624,30 +426,18 @@ def parallel_fda_bwd(q, o, g_cumsum, lse, do, scale=None, chunk_size=128, cu_seq
     return dq, None, dkd, dvd
 
 
-class ParallelFlashDepthAttentionFunction(torch.autograd.Function):
-    """fda_v12.py:1207-1338 (13 inputs; the k, v slots must be None)."""
+class ParallelFlashDepthAttentionFunction:
+    """fda_v12.py:1207-1338, by its ``apply`` (the k, v slots must be None)."""
 
     @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda")
-    def forward(ctx, q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, group_bs=None,
-                group_warps=None, depth_bs=None, depth_warps=None):
+    def apply(q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, group_bs=None,
+              group_warps=None, depth_bs=None, depth_warps=None):
         assert g is None, "g is not supported in this version"
         assert k is None and v is None, "Flash Depth Attention does not accept legacy k/v; pass None"
-        ctx.packed = _packed(cu_seqlens, q, moda_group_num)
-        o, lse = parallel_fda_fwd(q, None, scale, ctx.packed, cached_k, cached_v, moda_group_num)
-        ctx.save_for_backward(q, o, lse, cached_k, cached_v)
-        ctx.scale = scale
-        ctx.moda_group_num = moda_group_num
-        ctx.mark_non_differentiable(lse)
-        return o.to(q.dtype), lse
-
-    @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
-    def backward(ctx, do, dlse_unused):
-        q, o, lse, cached_k, cached_v = ctx.saved_tensors
-        dq, _, dkd, dvd = parallel_fda_bwd(q, o, None, lse, do.to(o.dtype), ctx.scale, cu_seqlens=ctx.packed,
-                                           cached_k=cached_k, cached_v=cached_v, moda_group_num=ctx.moda_group_num)
-        return dq.to(q), None, None, None, None, None, dkd, dvd, None, None, None, None, None
+        assert cached_k is not None and cached_v is not None, "Flash Depth Attention requires cached_k/cached_v"
+        cu, packed = _offsets(cu_seqlens)
+        return _lib.host().attend(_lib.DEPTH_ONLY, q, None, None, cached_k, cached_v, scale, moda_group_num, 0, None,
+                                  cu, packed, False, 128)
 
 
 def parallel_fda(q, k=None, v=None, g=None, cached_k=None, cached_v=None, scale=None, cu_seqlens=None,
@@ -657,46 +447,17 @@ def parallel_fda(q, k=None, v=None, g=None, cached_k=None, cached_v=None, scale=
     """Depth-only attention; signature of fda_v12.py:1346-1368."""
     assert k is None and v is None, "Flash Depth Attention does not accept legacy k/v; pass None"
     if head_first:
-        q = q.transpose(1, 2)
-        if g is not None:
-            g = g.transpose(1, 2)
-        if cached_k is not None and cached_v is not None:
-            cached_k = cached_k.transpose(1, 2)
-            cached_v = cached_v.transpose(1, 2)
+        q, g, cached_k, cached_v = _head_last(q, g, cached_k, cached_v)
     elif warn_shape and q.shape[1] < q.shape[2]:
-        warnings.warn(
-            f"[parallel_fda] detected seq_len({q.shape[1]}) < num_heads({q.shape[2]}). "
-            "input may be in head_first format while head_first=True is not set."
-        )
-    B, T_q, HQ, Kdim = q.shape
-    assert cached_k is not None and cached_v is not None, "Flash Depth Attention requires cached_k/cached_v"
-    assert moda_group_num > 0
-    assert T_q % moda_group_num == 0, "T_q must be divisible by moda_group_num"
-    T_kv = T_q // moda_group_num
-    H = cached_k.shape[2]
-    assert HQ == H, (
-        "Implicit head-dimension GQA is not allowed. "
-        "Please fold grouping only into `moda_group_num`: "
-        "use q.shape[2] == cached_k.shape[2] and set T_q = T_kv * moda_group_num."
-    )
-    if scale is None:
-        scale = Kdim ** -0.5
-    assert cached_k.shape[0] == B and cached_v.shape[0] == B
-    assert cached_k.shape[2] == H and cached_v.shape[2] == H, "cached_k/v head count mismatch"
-    assert cached_k.shape[1] % T_kv == 0, "cached_k time dimension must be T_kv * L"
-    L = cached_k.shape[1] // T_kv
-    assert L > 0
-    assert cached_v.shape[1] == T_kv * L, "cached_v shape mismatch"
-    if (cached_k.requires_grad or cached_v.requires_grad) and not return_depth_grads:
-        warnings.warn(
-            "cached_k/v requires gradients, but return_depth_grads=False. "
-            "Gradients are still computed and returned."
-        )
+        _warn_layout("parallel_fda", q)
+    if not return_depth_grads:
+        _warn_depth_grads(cached_k, cached_v)
     if g is not None:
-        assert g.shape[:3] == (B, T_q, HQ), "g must be [B,T_q,HQ]"
-    o, lse = ParallelFlashDepthAttentionFunction.apply(q, k, v, g, scale, cu_seqlens, cached_k, cached_v,
-                                                       moda_group_num, group_bs, group_warps, depth_bs, depth_warps)
-    return (o, lse) if need_lse else o
+        _refuse_decay(g, q)
+    cu, packed = _offsets(cu_seqlens)
+    out = _lib.host().attend(_lib.DEPTH_ONLY, q, None, None, cached_k, cached_v, scale, moda_group_num, 0, None, cu,
+                             packed, True, 128)
+    return out if need_lse else out[0]
 
 
 # ---------------------------------------------------------------------------
@@ -756,25 +517,17 @@ def parallel_attn_bwd(q, k, v, o, g_cumsum, lse, do, scale=None, chunk_size=128,
     return dq, dk, dv, None
 
 
-class ParallelAttentionFunction(torch.autograd.Function):
-    """fla/ops/attn/parallel.py:632-675."""
+class ParallelAttentionFunction:
+    """fla/ops/attn/parallel.py:632-675, by its ``apply``."""
 
     @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda")
-    def forward(ctx, q, k, v, g, scale, cu_seqlens):
+    def apply(q, k, v, g, scale, cu_seqlens):
         assert g is None, "g is not supported"
-        ctx.packed = _packed(cu_seqlens, q, 1)
-        o, lse = parallel_attn_fwd(q, k, v, None, scale, ctx.packed)
-        ctx.save_for_backward(q, k, v, o, lse)
-        ctx.scale = scale
-        return o.to(q.dtype)
-
-    @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
-    def backward(ctx, do):
-        q, k, v, o, lse = ctx.saved_tensors
-        dq, dk, dv, _ = parallel_attn_bwd(q, k, v, o, None, lse, do.to(o.dtype), ctx.scale, cu_seqlens=ctx.packed)
-        return dq.to(q), dk.to(k), dv.to(v), None, None, None
+        assert q.shape[2] % k.shape[2] == 0, "HQ must be a multiple of H"
+        assert q.shape[1] == k.shape[1]
+        cu, packed = _offsets(cu_seqlens)
+        return _lib.host().attend(_lib.PLAIN_GQA, q, k, v, None, None, scale, q.shape[2] // k.shape[2], 0, None, cu,
+                                  packed, False, 0)[0]
 
 
 def parallel_attn(q, k, v, g=None, scale=None, cu_seqlens=None, head_first=False):
@@ -788,6 +541,4 @@ def parallel_attn(q, k, v, g=None, scale=None, cu_seqlens=None, head_first=False
         warnings.warn(
             f"Input tensor shape suggests potential format mismatch: seq_len ({q.shape[1]}) < num_heads ({q.shape[2]}). "
         )
-    if scale is None:
-        scale = k.shape[-1] ** -0.5
     return ParallelAttentionFunction.apply(q, k, v, g, scale, cu_seqlens)
