@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <initializer_list>
 #include <string.h>
 
 #include "../../include/moda_hip.h"
@@ -15,6 +16,7 @@ hipError_t launch_delta(const KArgs& a, int dtype, int hd, hipStream_t stream);
 hipError_t launch_dq(const KArgs& a, int dtype, int hd, hipStream_t stream);
 hipError_t launch_dkv(const KArgs& a, int dtype, int hd, hipStream_t stream);
 hipError_t launch_generic(const KArgs& a, int dtype, int D, int Dv, int which, hipStream_t stream);
+hipError_t launch_fp32(const KArgs& a, int which, hipStream_t stream);
 hipError_t launch_reorg(void* const* layers, int64_t n_layers, int64_t slot0, int64_t L_total, int64_t n_tokens,
                         int64_t row_bytes, void* cache, bool to_cache, hipStream_t stream);
 }  // namespace moda
@@ -45,6 +47,19 @@ bool row_stride_ok(const moda_hip_strides& s, int esize) { return s.t >= 0 && s.
 bool mapped_span_ok(const KArgs& a, const moda_hip_strides& s, int esize) {
   if (a.L == 0 || a.Lv == a.L) return true;
   return (int64_t)(64 / a.Lv + 2) * a.L * s.t * esize < (1ll << 31);
+}
+
+// The fp32 matrix kernels move 16-byte pieces of rows; fp32 tensors that are not laid out for that run on the vector-ALU
+// kernels, which ask for element alignment only (the host therefore does not copy fp32 views).
+struct TensorAt {
+  const void* p;
+  const moda_hip_strides& s;
+};
+bool fp32_matrix(const moda_hip_desc* d, const KArgs& a, std::initializer_list<TensorAt> tensors) {
+  if (d->dtype != MODA_HIP_FP32 || a.D > 128 || a.Dv > 128) return false;
+  for (const TensorAt& t : tensors)
+    if (t.p && !aligned(t.p, t.s, 4, true)) return false;
+  return true;
 }
 
 int value_dim(const moda_hip_desc* d) { return (int)(d->Dv > 0 ? d->Dv : d->D); }
@@ -288,8 +303,13 @@ int moda_hip_fwd(const moda_hip_desc* d, const void* q, const void* k, const voi
   a.skd = cvt(d->kd);
   a.svd = cvt(d->vd);
   a.so = cvt(d->o);
-  hipError_t e = use_mfma(d) ? moda::launch_fwd(a, d->dtype, tile_width(d), (hipStream_t)stream)
-                             : moda::launch_generic(a, d->dtype, (int)d->D, value_dim(d), 0, (hipStream_t)stream);
+  hipError_t e;
+  if (use_mfma(d))
+    e = moda::launch_fwd(a, d->dtype, tile_width(d), (hipStream_t)stream);
+  else if (fp32_matrix(d, a, {{q, d->q}, {k, d->k}, {v, d->v}, {kd, d->kd}, {vd, d->vd}, {o, d->o}}))
+    e = moda::launch_fp32(a, 0, (hipStream_t)stream);
+  else
+    e = moda::launch_generic(a, d->dtype, (int)d->D, value_dim(d), 0, (hipStream_t)stream);
   return e == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
 }
 
@@ -440,6 +460,12 @@ int moda_hip_bwd_stages(const moda_hip_desc* d, const void* q, const void* k, co
     if ((stages & MODA_HIP_STAGE_DELTA) && !a.own_delta) e = moda::launch_delta(a, d->dtype, tile_width(d), s);
     if (e == hipSuccess && (stages & MODA_HIP_STAGE_DQ)) e = moda::launch_dq(a, d->dtype, tile_width(d), s);
     if (e == hipSuccess && (stages & MODA_HIP_STAGE_DKV)) e = moda::launch_dkv(a, d->dtype, tile_width(d), s);
+  } else if (fp32_matrix(d, a, {{q, d->q}, {k, d->k}, {v, d->v}, {kd, d->kd}, {vd, d->vd}, {o, d->o}, {d_o, d->d_o}, {dq, d->dq},
+                                {dk, d->dk}, {dv, d->dv}, {dkd, d->dkd}, {dvd, d->dvd}})) {
+    // the dQ kernel forms the row sums for the dK/dV kernel; a dK/dV stage that runs alone has them formed first
+    if (stages & MODA_HIP_STAGE_DQ) e = moda::launch_fp32(a, 1, s);
+    if (e == hipSuccess && !(stages & MODA_HIP_STAGE_DQ) && stages) e = moda::launch_fp32(a, 3, s);
+    if (e == hipSuccess && (stages & MODA_HIP_STAGE_DKV)) e = moda::launch_fp32(a, 2, s);
   } else {
     // the generic kernels recompute delta inline; the DELTA stage is a no-op for them
     if (stages & MODA_HIP_STAGE_DQ) e = moda::launch_generic(a, d->dtype, (int)d->D, value_dim(d), 1, s);

@@ -215,6 +215,69 @@ def test_variants(gpu_device, case):
     compare_all(got, ref, dtype, str(case))
 
 
+# fp32 tensors on the fp32 matrix kernels (head dims up to 128; wider ones and rows that are not 16-byte aligned stay on
+# the vector-ALU kernels): one row, block edges (15, 16, 17), more blocks than a workgroup has waves, head dims below,
+# at and just above a tile width, groups that do not divide a block, several blocks of depth slots per wave group
+FP32 = [
+    # B, T, H, D, Dv, L, G, mode, chunk_tokens
+    (1, 1, 1, 64, 64, 3, 2, "causal", 0),
+    (2, 15, 2, 64, 64, 0, 1, "causal", 0),
+    (1, 16, 1, 128, 128, 5, 1, "noncausal", 0),
+    (1, 17, 3, 4, 4, 7, 3, "causal", 0),
+    (2, 129, 2, 60, 68, 9, 2, "noncausal", 0),
+    (1, 300, 2, 128, 128, 12, 4, "causal", 0),
+    (1, 145, 1, 124, 36, 4, 8, "causal", 0),
+    (1, 70, 2, 64, 64, 70, 1, "depth_only", 0),
+    (1, 200, 2, 64, 64, 3, 2, "chunk_visible", 32),
+    (1, 77, 1, 128, 64, 5, 4, "chunk_visible", 16),
+    (1, 40, 1, 132, 132, 2, 2, "causal", 0),
+]
+
+
+@pytest.mark.parametrize("case", FP32, ids=lambda c: f"{c[7]}-T{c[1]}-D{c[3]}-Dv{c[4]}-L{c[5]}-G{c[6]}")
+def test_fp32_kernels(gpu_device, case):
+    """Relative L2 error within 1e-5: sums of at most a few thousand fp32 products on both sides (rounding 6e-8 each,
+    errors adding up as the square root of their number, a few e-6), elementwise as every fp32 case.  A dK/dV stage
+    that runs alone forms its row sums itself; a view with rows off the 16-byte grid takes the other kernels."""
+    from moda_amd import _lib, ops
+
+    B, T, H, D, Dv, L, G, mode, cb = case
+    say(f"[fp32] {case}")
+    inp = oracle.make_inputs(B, T, H, D, L, G, seed=61, dtype=torch.float32, std=0.5, depth_only=(mode == "depth_only"), Dv=Dv)
+    sc = D ** -0.5
+    ref = oracle.moda_dense_fwd_bwd(inp, sc, G, mode, cb)
+    dev = to_dev(inp, gpu_device)
+    got = run_hip(dev, sc, G, mode, cb)
+    compare_all(got, ref, torch.float32, str(case))
+    for n in ("o", "dq", "dk", "dv", "dkd", "dvd"):
+        if ref[n] is not None and ref[n].norm() > 1e-3:
+            assert numerics(got[n], ref[n])[2] <= 1e-5, (case, n)
+    m = MODE_ID[mode]
+    xs = [dev[n] for n in ("q", "k", "v", "kd", "vd")]
+    alone = ops._raw_bwd(m, *xs, got["o"], got["lse"], dev["do"], sc, G, cb, stages=_lib.STAGE_DKV)
+    for i, n in enumerate(("dk", "dv", "dkd", "dvd"), 1):
+        assert (got[n] is None and alone[i] is None) or torch.equal(got[n], alone[i]), n
+    shifted = {k: x if x is None else torch.empty(x.numel() + 1, device=x.device)[1:].view(x.shape).copy_(x) for k, x in dev.items()}
+    compare_all(run_hip(shifted, sc, G, mode, cb), ref, torch.float32, str(case) + " off the 16-byte grid")
+
+
+def test_fp32_plain_gqa(gpu_device):
+    """Head-dim GQA in fp32: several query heads per kv head in one dK/dV workgroup."""
+    import moda_amd
+
+    gen = torch.Generator().manual_seed(5)
+    q, k, v, do = (torch.randn(2, 83, h, 64, generator=gen) for h in (6, 2, 2, 6))
+    xs = [x.clone().requires_grad_() for x in (q, k, v)]
+    s = torch.einsum("bthd,bshd->bhts", xs[0], xs[1].repeat_interleave(3, 2)) * 64 ** -0.5
+    s = s.masked_fill(torch.ones(83, 83).triu(1).bool(), float("-inf"))
+    o_ref = torch.einsum("bhts,bshd->bthd", s.softmax(-1), xs[2].repeat_interleave(3, 2))
+    ref = torch.autograd.grad(o_ref, xs, do)
+    ys = [x.to(gpu_device).requires_grad_() for x in (q, k, v)]
+    o = moda_amd.parallel_attn(*ys)
+    for got, want in zip((o, *torch.autograd.grad(o, ys, do.to(gpu_device))), (o_ref, *ref)):
+        assert numerics(got, want)[2] <= 1e-5
+
+
 @pytest.mark.parametrize("case", [
     # (B, T, H, D, L, G, mode, chunk tokens, compute type)
     (1, 256, 4, 64, 4, 2, "causal", 0, "fp16"),          # the fp32 plumbing configuration of the benchmark list
