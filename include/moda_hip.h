@@ -97,7 +97,9 @@ enum moda_hip_flag {
    * (vision_tasks/deit/models.py:361-390 does both for every layer).  Still one writer per row and
    * no atomics.  Every mode with a depth stream takes it.
    */
-  MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS = 1
+  MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS = 1,
+  /* dkd, dvd: slots >= L_valid are left alone (implied by the flag above); without it they are zeroed */
+  MODA_HIP_FLAG_KEEP_DEPTH_SLOTS = 2
 };
 
 typedef struct moda_hip_strides {
@@ -232,6 +234,41 @@ int moda_hip_depth_reorg_fwd(const void* const* layers, int64_t n_layers, int64_
 int moda_hip_depth_reorg_bwd(const void* d_cache, int64_t n_layers, int64_t slot0, int64_t L_total,
                              int64_t B, int64_t T, int64_t H, int64_t D, int32_t dtype,
                              void* const* d_layers, void* stream);
+
+/*
+ * One layer's K and V against slot `slot` of the two token-major caches [B, T*L_total, H, D], both in one launch.  The
+ * layer tensors are [B, T, H, D] with element strides {b, t, h} and unit inner stride (views are taken as they are), the
+ * caches contiguous.  _push: the slot receives the layer (the append of a forward pass).  _slot_add: the layer
+ * tensors receive the sum of themselves and the slot (a layer's own dk, dv and what later layers' attention sent to
+ * its slot).
+ */
+int moda_hip_depth_push(const void* k, const void* v, const moda_hip_strides* sk, const moda_hip_strides* sv, int64_t slot,
+                        int64_t L_total, int64_t B, int64_t T, int64_t H, int64_t D, int32_t dtype,
+                        void* cache_k, void* cache_v, void* stream);
+int moda_hip_depth_slot_add(void* dk, void* dv, const moda_hip_strides* sdk, const moda_hip_strides* sdv, int64_t slot,
+                            int64_t L_total, int64_t B, int64_t T, int64_t H, int64_t D, int32_t dtype,
+                            const void* d_cache_k, const void* d_cache_v, void* stream);
+
+/*
+ * The dense pieces of a transformer block around the attention call, 16-bit types, fp32 sums.
+ *
+ * moda_hip_linear: y = x W^T + bias for up to three outputs that share the input (x [rows, K], row stride ldx; W [n, K]
+ * contiguous; each output [rows, n] with row stride ldy), then optionally the exact GELU, or a residual
+ * (same shape and row stride ld_res) added to the rounded result.  K a multiple of 64, n of 8,
+ * x, W, y, residual rows on 16-byte boundaries (bias: 8 bytes); MODA_HIP_EUNSUPPORTED / MODA_HIP_EALIGN otherwise.
+ * `residual` may be the output itself (single part).
+ * moda_hip_layer_norm: y = (x - mean) / sqrt(var + eps) * weight + bias over rows of `dim` (a multiple of 8, at most 4096).
+ */
+typedef struct moda_hip_linear_part {
+  const void* w;
+  const void* bias; /* may be NULL */
+  void* y;
+  int64_t ldy, n;
+} moda_hip_linear_part;
+int moda_hip_linear(int32_t dtype, int64_t rows, int64_t K, const void* x, int64_t ldx, const moda_hip_linear_part* parts,
+                    int32_t n_parts, const void* residual, int64_t ld_res, int32_t gelu, void* stream);
+int moda_hip_layer_norm(int32_t dtype, int64_t rows, int64_t dim, const void* x, const void* weight, const void* bias, float eps,
+                        void* y, void* stream);
 
 /*
  * Which kernels a descriptor runs on: 1 = the matrix-core kernels (tensor rows must then be 16-byte aligned, see

@@ -28,6 +28,10 @@ EXPORTS = (
     "moda_hip_bwd_static",
     "moda_hip_depth_reorg_fwd",
     "moda_hip_depth_reorg_bwd",
+    "moda_hip_depth_push",
+    "moda_hip_depth_slot_add",
+    "moda_hip_linear",
+    "moda_hip_layer_norm",
     "moda_hip_uses_matrix_cores",
     "moda_hip_strerror",
     "moda_hip_version",

@@ -657,8 +657,8 @@ __global__ __launch_bounds__(256) void depth_cols_kernel(const KArgs a_in) {
   uint16_t* dv_out = a.dvd + b * a.sdvd.b + hkv * a.sdvd.h + c * a.sdvd.t + 8 * sub;
   // lanes past a tensor's head dim carry zeros and store nothing (keys and values may differ in width)
   const bool in_k = 8 * sub < a.D, in_v = 8 * sub < a.Dv;
-  if (slot >= a.Lv) {  // a slot without data: zero gradient, or (accumulating) somebody else's sum to leave alone
-    if (a.accum_depth) return;
+  if (slot >= a.Lv) {  // a slot without data: zero gradient, or (keep_slots) somebody else's sum to leave alone
+    if (a.keep_slots) return;
     const i32x4 z = {0, 0, 0, 0};
     if (in_k) *reinterpret_cast<i32x4*>(dk_out) = z;
     if (in_v) *reinterpret_cast<i32x4*>(dv_out) = z;
@@ -744,8 +744,8 @@ __global__ __launch_bounds__(256) void depth_cols_handed_kernel(const KArgs a_in
   uint16_t* dk_out = a.dkd + b * a.sdkd.b + hkv * a.sdkd.h + c * a.sdkd.t + 8 * sub;
   uint16_t* dv_out = a.dvd + b * a.sdvd.b + hkv * a.sdvd.h + c * a.sdvd.t + 8 * sub;
   const bool in_k = 8 * sub < a.D, in_v = 8 * sub < a.Dv;
-  if (slot >= a.Lv) {  // a slot without data: zero gradient, or (accumulating) somebody else's sum to leave alone
-    if (a.accum_depth) return;
+  if (slot >= a.Lv) {  // a slot without data: zero gradient, or (keep_slots) somebody else's sum to leave alone
+    if (a.keep_slots) return;
     const i32x4 z = {0, 0, 0, 0};
     if (in_k) *reinterpret_cast<i32x4*>(dk_out) = z;
     if (in_v) *reinterpret_cast<i32x4*>(dv_out) = z;
@@ -839,8 +839,8 @@ __global__ __launch_bounds__(256) void depth_token_handed_kernel(const KArgs a_i
     float dk[8], dv[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) dk[i] = dv[i] = 0.f;
-    if (slot >= a.Lv) {  // a slot without data: zero gradient, or (accumulating) somebody else's sum to leave alone
-      if (a.accum_depth) continue;
+    if (slot >= a.Lv) {  // a slot without data: zero gradient, or (keep_slots) somebody else's sum to leave alone
+      if (a.keep_slots) continue;
     } else {
 #pragma unroll
       for (int g = 0; g < GMAX; g++) {
@@ -979,7 +979,7 @@ hipError_t launch_dkv_t(const KArgs& a, hipStream_t stream) {
       if (er != hipSuccess) return er;
     }
   }
-  if (a.L > 0 && (a.chunk || in_dq) && a.Lv != a.L && !a.accum_depth && (int64_t)a.B * a.T > 0) {
+  if (a.L > 0 && (a.chunk || in_dq) && a.Lv != a.L && !a.keep_slots && (int64_t)a.B * a.T > 0) {
     // packed batch: one row axis of all sequences (its length is the row-sum pitch / G), else B x T * L rows
     const int64_t rows = a.cu ? (int64_t)(a.delta_pitch / a.Gf) * a.L : (int64_t)a.T * a.L;
     const int batches = a.cu ? 1 : a.B;

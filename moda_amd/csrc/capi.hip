@@ -19,6 +19,12 @@ hipError_t launch_generic(const KArgs& a, int dtype, int D, int Dv, int which, h
 hipError_t launch_fp32(const KArgs& a, int which, hipStream_t stream);
 hipError_t launch_reorg(void* const* layers, int64_t n_layers, int64_t slot0, int64_t L_total, int64_t n_tokens,
                         int64_t row_bytes, void* cache, bool to_cache, hipStream_t stream);
+hipError_t launch_slot(void* const (&layer)[2], const int64_t (&strides)[2][3], void* const (&cache)[2], int64_t slot, int64_t L_total,
+                       int64_t B, int64_t T, int64_t H, int64_t D, int dtype, bool to_cache, hipStream_t stream);
+hipError_t launch_linear(int dtype, int64_t rows, int64_t K, const void* x, int64_t ldx, const moda_hip_linear_part* parts, int n_parts,
+                         const void* residual, int64_t ld_res, bool gelu, int compute_units, hipStream_t stream);
+hipError_t launch_layer_norm(int dtype, int64_t rows, int64_t dim, const void* x, const void* weight, const void* bias, float eps, void* y,
+                             hipStream_t stream);
 }  // namespace moda
 
 using moda::KArgs;
@@ -94,7 +100,7 @@ int fill_geometry(const moda_hip_desc* d, KArgs& a) {
   if (d->mode == MODA_HIP_DEPTH_ONLY && d->L == 0) return MODA_HIP_EINVAL;
   if (d->mode == MODA_HIP_CHUNK_VISIBLE && d->L > 0 && d->chunk_tokens <= 0) return MODA_HIP_EINVAL;
   if (d->L_valid < 0 || d->L_valid > d->L) return MODA_HIP_EINVAL;
-  if (d->flags & ~(int32_t)MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS) return MODA_HIP_EINVAL;
+  if (d->flags & ~(int32_t)(MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS | MODA_HIP_FLAG_KEEP_DEPTH_SLOTS)) return MODA_HIP_EINVAL;
   // 32-bit index space used for rows and flattened depth columns inside the kernels
   if (d->T * d->G >= (1ll << 30) || d->T * (d->L > 0 ? d->L : 1) >= (1ll << 30) || d->B * d->H * d->G >= (1ll << 20))
     return MODA_HIP_EUNSUPPORTED;
@@ -117,6 +123,7 @@ int fill_geometry(const moda_hip_desc* d, KArgs& a) {
   a.causal = d->mode == MODA_HIP_CAUSAL || d->mode == MODA_HIP_CHUNK_VISIBLE || plain;
   a.chunk = d->mode == MODA_HIP_CHUNK_VISIBLE;
   a.accum_depth = (d->flags & MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS) ? 1 : 0;
+  a.keep_slots = d->flags ? 1 : 0;
   a.nqt = (a.Tq + 127) / 128;
   a.scale = d->scale;
   a.delta_pitch = a.Tq;
@@ -501,6 +508,64 @@ int moda_hip_depth_reorg_bwd(const void* d_cache, int64_t n_layers, int64_t slot
   if (B * T >= (1ll << 31)) return MODA_HIP_EUNSUPPORTED;
   hipError_t e = moda::launch_reorg(d_layers, n_layers, slot0, L_total, B * T, H * D * elem_size(dtype),
                                     const_cast<void*>(d_cache), false, (hipStream_t)stream);
+  return e == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
+}
+
+static int depth_slot(void* k, void* v, const moda_hip_strides* sk, const moda_hip_strides* sv, int64_t slot, int64_t L_total, int64_t B,
+                      int64_t T, int64_t H, int64_t D, int32_t dtype, void* cache_k, void* cache_v, bool to_cache, void* stream) {
+  if (slot < 0 || slot >= L_total || B < 0 || T < 0 || H <= 0 || D <= 0 || B * T >= (1ll << 31) || H >= (1ll << 31) || D >= (1ll << 31))
+    return MODA_HIP_EINVAL;
+  if (dtype < MODA_HIP_BF16 || dtype > MODA_HIP_FP32) return MODA_HIP_EINVAL;
+  if (B * T == 0) return MODA_HIP_OK;
+  if (!k || !v || !sk || !sv || !cache_k || !cache_v) return MODA_HIP_EINVAL;
+  void* const layer[2] = {k, v};
+  void* const cache[2] = {cache_k, cache_v};
+  const int64_t strides[2][3] = {{sk->b, sk->t, sk->h}, {sv->b, sv->t, sv->h}};
+  const hipError_t e = moda::launch_slot(layer, strides, cache, slot, L_total, B, T, H, D, dtype, to_cache, (hipStream_t)stream);
+  return e == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
+}
+int moda_hip_depth_push(const void* k, const void* v, const moda_hip_strides* sk, const moda_hip_strides* sv, int64_t slot,
+                        int64_t L_total, int64_t B, int64_t T, int64_t H, int64_t D, int32_t dtype, void* cache_k, void* cache_v,
+                        void* stream) {
+  return depth_slot(const_cast<void*>(k), const_cast<void*>(v), sk, sv, slot, L_total, B, T, H, D, dtype, cache_k, cache_v, true, stream);
+}
+int moda_hip_depth_slot_add(void* dk, void* dv, const moda_hip_strides* sdk, const moda_hip_strides* sdv, int64_t slot, int64_t L_total,
+                            int64_t B, int64_t T, int64_t H, int64_t D, int32_t dtype, const void* d_cache_k, const void* d_cache_v,
+                            void* stream) {
+  return depth_slot(dk, dv, sdk, sdv, slot, L_total, B, T, H, D, dtype, const_cast<void*>(d_cache_k), const_cast<void*>(d_cache_v), false,
+                    stream);
+}
+
+int moda_hip_linear(int32_t dtype, int64_t rows, int64_t K, const void* x, int64_t ldx, const moda_hip_linear_part* parts, int32_t n_parts,
+                    const void* residual, int64_t ld_res, int32_t gelu, void* stream) {
+  if ((dtype != MODA_HIP_BF16 && dtype != MODA_HIP_FP16) || rows < 0 || K <= 0 || n_parts < 1 || n_parts > 3 || !parts) return MODA_HIP_EINVAL;
+  if (rows == 0) return MODA_HIP_OK;
+  if (!x || (residual && n_parts != 1)) return MODA_HIP_EINVAL;
+  if (K % 64 != 0 || rows >= (1ll << 30) || ldx >= (1ll << 22) || K >= (1ll << 22)) return MODA_HIP_EUNSUPPORTED;
+  if ((uintptr_t)x % 16 != 0 || ldx % 8 != 0 || ldx < K || (residual && ((uintptr_t)residual % 16 != 0 || ld_res % 8 != 0)))
+    return MODA_HIP_EALIGN;
+  for (int i = 0; i < n_parts; i++) {
+    const moda_hip_linear_part& p = parts[i];
+    if (!p.w || !p.y || p.n <= 0 || p.n >= (1ll << 24)) return MODA_HIP_EINVAL;
+    if (p.n % 8 != 0) return MODA_HIP_EUNSUPPORTED;
+    if ((uintptr_t)p.w % 16 != 0 || (uintptr_t)p.y % 16 != 0 || p.ldy % 8 != 0 || (uintptr_t)p.bias % 8 != 0) return MODA_HIP_EALIGN;
+  }
+  int cus = 0;
+  const int rc = check_device(&cus);
+  if (rc) return rc;
+  const hipError_t e = moda::launch_linear(dtype, rows, K, x, ldx, parts, n_parts, residual, ld_res, gelu != 0, cus, (hipStream_t)stream);
+  return e == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
+}
+
+int moda_hip_layer_norm(int32_t dtype, int64_t rows, int64_t dim, const void* x, const void* weight, const void* bias, float eps, void* y,
+                        void* stream) {
+  if ((dtype != MODA_HIP_BF16 && dtype != MODA_HIP_FP16) || rows < 0 || dim <= 0) return MODA_HIP_EINVAL;
+  if (rows == 0) return MODA_HIP_OK;
+  if (!x || !weight || !bias || !y) return MODA_HIP_EINVAL;
+  if (dim % 8 != 0 || dim > 4096 || rows >= (1ll << 31)) return MODA_HIP_EUNSUPPORTED;
+  for (const void* p : {x, weight, bias, (const void*)y})
+    if ((uintptr_t)p % 16 != 0) return MODA_HIP_EALIGN;
+  const hipError_t e = moda::launch_layer_norm(dtype, rows, dim, x, weight, bias, eps, y, (hipStream_t)stream);
   return e == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
 }
 

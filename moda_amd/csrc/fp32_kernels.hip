@@ -457,7 +457,7 @@ __global__ __launch_bounds__(64 * kFp32ColWaves<HD>, HD <= 64 ? 2 : 1) void fp32
         if (d < a.Dv) *reinterpret_cast<f32x4*>(dvp + d) = y;
       }
     // the lane group of a token's last filled slot also clears the rows of the slots without data
-    if (a.Lv != a.L && !a.accum_depth && c % a.Lv == a.Lv - 1) {
+    if (a.Lv != a.L && !a.keep_slots && c % a.Lv == a.Lv - 1) {
       const f32x4 z = {0.f, 0.f, 0.f, 0.f};
       for (int slot = a.Lv; slot < a.L; slot++) {
         dkp += a.sdkd.t;

@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256) void generic_col_kernel(const KArgs a_in, cons
     qlo = w * a.Gf;
     qhi = a.chunk ? min(a.T, (w / a.Cb + 1) * a.Cb) * a.Gf : (w + 1) * a.Gf;
     if (col - w * a.L >= a.Lv) {  // a slot without data: no row sees it
-      if (a.accum_depth) return;  // accumulating: the row holds somebody else's sum
+      if (a.keep_slots) return;  // the row may hold somebody else's sum
       qhi = qlo;                  // its gradients are zero
     }
   }

@@ -289,21 +289,24 @@ std::pair<Tensor, Tensor> forward(const Call& c, Tensor q, Tensor k, Tensor v, T
 }
 
 typedef std::array<Tensor, 5> Grads;  // dq, dk, dv, dkd, dvd
+// what happens to dkd, dvd: overwritten; added to, slots >= depth_valid untouched; overwritten, those slots untouched
+enum DepthGrads { kOverwrite = 0, kAccumulate = MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS, kKeepSlots = MODA_HIP_FLAG_KEEP_DEPTH_SLOTS };
 
-// `out`: gradient buffers to write to (undefined entries where the input is), else allocated here; `ws`: workspace to
-// use, else allocated here; `accumulate`: dkd, dvd of `out` are added to (slots >= depth_valid untouched).
+// `out`: gradient buffers to write to (an undefined entry is allocated here like all of them without `out`); `ws`:
+// workspace to use, else allocated here.
 Grads backward(const Call& c, Tensor q, Tensor k, Tensor v, Tensor kd, Tensor vd, Tensor o, Tensor lse, Tensor d_o, int stages,
-               const Grads* out, Tensor ws, bool accumulate) {
+               const Grads* out, Tensor ws, DepthGrads depth_grads) {
+  const bool accumulate = depth_grads == kAccumulate;
   CONTRACT(!accumulate || (out && (*out)[3].defined() && (*out)[4].defined()), "accumulate_depth needs the gradient buffers to add to");
   if (narrows(q)) {
     // 16-bit gradients from the matrix kernels (without the accumulate flag: the slots without data come back as
     // zeros), widened into the caller's fp32 buffers or added to them
     Grads g = backward(c, narrowed(q), narrowed(k), narrowed(v), narrowed(kd), narrowed(vd), narrowed(o), lse, narrowed(d_o), stages,
-                       nullptr, Tensor(), false);
+                       nullptr, Tensor(), kOverwrite);
     for (int i = 0; i < 5; i++) {
-      if (!out) {
+      if (!out || !(*out)[i].defined()) {
         if (g[i].defined()) g[i] = g[i].to(at::kFloat);
-      } else if ((*out)[i].defined()) {
+      } else {
         if (accumulate && i >= 3)
           (*out)[i].add_(g[i]);
         else
@@ -323,10 +326,9 @@ Grads backward(const Call& c, Tensor q, Tensor k, Tensor v, Tensor kd, Tensor vd
   const Tensor* ins[5] = {&q, &k, &v, &kd, &vd};
   Grads g;
   for (int i = 0; i < 5; i++) {
-    if (out) {
+    if (out && (*out)[i].defined()) {
       g[i] = (*out)[i];
-      CONTRACT(g[i].defined() == ins[i]->defined() &&
-                   (!g[i].defined() || (g[i].sizes() == ins[i]->sizes() && g[i].scalar_type() == ins[i]->scalar_type())),
+      CONTRACT(ins[i]->defined() && g[i].sizes() == ins[i]->sizes() && g[i].scalar_type() == ins[i]->scalar_type(),
                "reused gradient buffers must match their inputs in shape and dtype");
     } else if (ins[i]->defined()) {
       g[i] = at::empty(ins[i]->sizes(), ins[i]->options());
@@ -334,7 +336,7 @@ Grads backward(const Call& c, Tensor q, Tensor k, Tensor v, Tensor kd, Tensor vd
   }
   Grads to = g;  // what the library sees: no depth gradients of an empty stream
   if (e.L == 0) kd = vd = to[3] = to[4] = Tensor();
-  if (accumulate && e.L > 0) d.flags = MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS;
+  if (e.L > 0) d.flags = depth_grads;
   d.q = strides_of(q);
   d.k = strides_of(k);
   d.v = strides_of(v);
@@ -377,7 +379,7 @@ struct Attend : torch::autograd::Function<Attend> {
     const auto call = c10::static_intrusive_pointer_cast<Call>(ctx->saved_data["call"].toCapsule());
     if (!grads[0].defined()) return variable_list(6);
     Grads g = ::backward(*call, s[0], s[1], s[2], s[3], s[4], s[5], s[6], grads[0].to(s[5].scalar_type()), MODA_HIP_STAGE_ALL,
-                         nullptr, Tensor(), false);
+                         nullptr, Tensor(), kOverwrite);
     return {g[0], g[1], g[2], g[3], g[4], Tensor()};
   }
 };
@@ -444,6 +446,279 @@ py::tuple attend(int mode, const Tensor& q, const OptTensor& k, const OptTensor&
   return py::make_tuple(r[0], r[1]);
 }
 
+// ------------------------------------------------------------------------------------------------------------------
+// depth stream of a training step (moda_amd/modules.py: DepthStream)
+// ------------------------------------------------------------------------------------------------------------------
+
+// Unit inner stride is all the slot kernels ask of a layer tensor.
+Tensor layer_view(const Tensor& x) { return x.stride(3) == 1 || x.size(3) == 1 ? x : x.contiguous(); }
+
+void check_layer(const Tensor& x, const Tensor& cache, int64_t L_total) {
+  CONTRACT(x.dim() == 4, "a layer must be a [B, T, H, D] tensor");
+  CONTRACT(cache.is_contiguous() && has_shape(cache, {x.size(0), x.size(1) * L_total, x.size(2), x.size(3)}),
+           "cache must be a contiguous ", shape_text({x.size(0), x.size(1) * L_total, x.size(2), x.size(3)}), " tensor");
+  CONTRACT(x.scalar_type() == cache.scalar_type() && x.device() == cache.device(), "layers and cache must share dtype and device");
+}
+
+// one layer's K and V into slot `slot` of the caches
+void depth_push(const Tensor& k_in, const Tensor& v_in, const Tensor& cache_k, const Tensor& cache_v, int64_t slot, int64_t L_total) {
+  check_layer(k_in, cache_k, L_total);
+  check_layer(v_in, cache_v, L_total);
+  CONTRACT(k_in.sizes() == v_in.sizes(), "a layer's k and v must agree in shape");
+  CONTRACT(slot >= 0 && slot < L_total, "slots out of range");
+  check_device(cache_k);
+  const Tensor k = layer_view(k_in), v = layer_view(v_in);
+  const moda_hip_strides sk = strides_of(k), sv = strides_of(v);
+  c10::OptionalDeviceGuard guard(k.device());
+  check_rc(moda_hip_depth_push(in_ptr(k), in_ptr(v), &sk, &sv, slot, L_total, k.size(0), k.size(1), k.size(2), k.size(3), dtype_code(k),
+                               out_ptr(cache_k), out_ptr(cache_v), stream_of(k)),
+           "moda_hip_depth_push");
+}
+
+// Cache and gradient buffers of one forward / backward pass, [B, T * L, H, D] each, allocated by the first push and never
+// initialised: slots are read once written.  The backward calls run from the last layer to the first; the first of
+// them overwrites the gradients of the slots it saw (`written`), the others, which saw fewer, add to theirs.
+struct StreamBuffers : torch::CustomClassHolder {
+  Tensor k, v, gk, gv;
+  int64_t L = 0, written = 0;
+};
+// An attention call of the stream: what it saw, and the slot its own k, v were pushed to afterwards (-1: none).
+struct StreamCall : torch::CustomClassHolder {
+  Call call;
+  c10::intrusive_ptr<StreamBuffers> buf;
+  int64_t n = 0, slot = -1;
+};
+
+// A tensor that carries no data, only the order of the stream's operations (autograd runs them last to first).
+Tensor order_token(const Tensor& like) { return at::empty({0}, like.options().dtype(at::kFloat)); }
+
+// Attention over the sequence and the first n slots of the cache (which is not an autograd input: its gradient goes to
+// the buffers).  Where the layer's k, v themselves went to a slot, their gradient is the call's own plus that slot's,
+// complete by the time this node runs.
+struct StreamAttend : torch::autograd::Function<StreamAttend> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& /*token*/,
+                               const c10::intrusive_ptr<StreamCall>& call) {
+    const bool depth = call->n > 0;
+    auto r = ::forward(call->call, q, k, v, depth ? call->buf->k : Tensor(), depth ? call->buf->v : Tensor());
+    ctx->save_for_backward({q, k, v, r.first, r.second});
+    ctx->saved_data["call"] = c10::IValue::make_capsule(call);
+    ctx->set_materialize_grads(false);
+    return {r.first, order_token(q)};
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    const variable_list s = ctx->get_saved_variables();
+    const auto call = c10::static_intrusive_pointer_cast<StreamCall>(ctx->saved_data["call"].toCapsule());
+    StreamBuffers& buf = *call->buf;
+    const Tensor &q = s[0], &k = s[1], &v = s[2], &o = s[3], &lse = s[4];
+    const Tensor d_o = grads[0].defined() ? grads[0].to(o.scalar_type()) : at::zeros_like(o);
+    const int64_t n = call->n;
+    Grads g;
+    if (n > 0) {
+      bool first = buf.written == 0;
+      if (first && narrows(q)) {  // gradients computed in another type arrive as sums
+        buf.gk.zero_();
+        buf.gv.zero_();
+        first = false;
+      }
+      const Grads into{Tensor(), Tensor(), Tensor(), buf.gk, buf.gv};
+      g = ::backward(call->call, q, k, v, buf.k, buf.v, o, lse, d_o, MODA_HIP_STAGE_ALL, &into, Tensor(), first ? kKeepSlots : kAccumulate);
+      buf.written = std::max(buf.written, n);
+    } else {
+      g = ::backward(call->call, q, k, v, {}, {}, o, lse, d_o, MODA_HIP_STAGE_ALL, nullptr, Tensor(), kOverwrite);
+    }
+    if (call->slot >= 0 && call->slot < buf.written) {
+      const moda_hip_strides sk = strides_of(g[1]), sv = strides_of(g[2]);
+      c10::OptionalDeviceGuard guard(k.device());
+      check_rc(moda_hip_depth_slot_add(out_ptr(g[1]), out_ptr(g[2]), &sk, &sv, call->slot, buf.L, k.size(0), k.size(1), k.size(2), k.size(3),
+                                       dtype_code(k), in_ptr(buf.gk), in_ptr(buf.gv), stream_of(k)),
+               "moda_hip_depth_slot_add");
+    }
+    return {g[0], g[1], g[2], Tensor(), Tensor()};
+  }
+};
+
+// K/V pushed without having been attended over by their own layer: their gradient is their slot's.
+struct StreamPush : torch::autograd::Function<StreamPush> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& k, const Tensor& /*v*/, const Tensor& /*token*/,
+                               const c10::intrusive_ptr<StreamCall>& call) {
+    ctx->saved_data["call"] = c10::IValue::make_capsule(call);
+    ctx->set_materialize_grads(false);
+    return {order_token(k)};
+  }
+  static variable_list backward(AutogradContext* ctx, const variable_list&) {
+    const auto call = c10::static_intrusive_pointer_cast<StreamCall>(ctx->saved_data["call"].toCapsule());
+    const StreamBuffers& buf = *call->buf;
+    const int64_t B = buf.k.size(0), T = buf.k.size(1) / buf.L, H = buf.k.size(2), D = buf.k.size(3);
+    auto slot = [&](const Tensor& g) {
+      if (call->slot >= buf.written) return at::zeros({B, T, H, D}, g.options());
+      return g.view({B, T, buf.L, H, D}).select(2, call->slot).contiguous();
+    };
+    return {slot(buf.gk), slot(buf.gv), Tensor(), Tensor()};
+  }
+};
+
+class TrainStream {
+ public:
+  explicit TrainStream(int64_t max_layers) : buf_(c10::make_intrusive<StreamBuffers>()) { buf_->L = max_layers; }
+
+  Tensor attend(const Tensor& q, const Tensor& k, const Tensor& v, double scale, int64_t G, int mode, int64_t chunk_tokens) {
+    py::gil_scoped_release nogil;
+    auto call = c10::make_intrusive<StreamCall>();
+    call->call.mode = mode;
+    call->call.scale = scale;
+    call->call.G = G;
+    call->call.chunk_tokens = chunk_tokens;
+    if (n_ > 0) call->call.depth_valid = n_;
+    call->buf = buf_;
+    call->n = n_;
+    const variable_list r = StreamAttend::apply(q, k, v, token_.defined() ? OptTensor(token_) : OptTensor(), call);
+    token_ = r[1];
+    last_ = r[0].requires_grad() ? call : c10::intrusive_ptr<StreamCall>();
+    last_k_ = k;
+    last_v_ = v;
+    return r[0];
+  }
+
+  void push(const Tensor& k, const Tensor& v) {
+    py::gil_scoped_release nogil;
+    CONTRACT(k.dim() == 4, "k must be [B, T, H, D]");
+    if (!buf_->k.defined()) {
+      buf_->k = at::empty({k.size(0), k.size(1) * buf_->L, k.size(2), k.size(3)}, k.options());
+      for (Tensor* x : {&buf_->v, &buf_->gk, &buf_->gv}) *x = at::empty_like(buf_->k);
+    }
+    depth_push(k, v, buf_->k, buf_->v, n_, buf_->L);
+    if (at::GradMode::is_enabled()) {
+      if (last_ && k.is_same(last_k_) && v.is_same(last_v_)) {
+        last_->slot = n_;
+      } else if (k.requires_grad() || v.requires_grad()) {
+        auto call = c10::make_intrusive<StreamCall>();
+        call->buf = buf_;
+        call->slot = n_;
+        token_ = StreamPush::apply(k, v, token_.defined() ? token_ : order_token(k), call)[0];
+      }
+    }
+    last_.reset();
+    last_k_ = last_v_ = Tensor();
+    n_++;
+  }
+
+ private:
+  c10::intrusive_ptr<StreamBuffers> buf_;
+  c10::intrusive_ptr<StreamCall> last_;  // the latest attention call, until something is pushed
+  Tensor token_, last_k_, last_v_;
+  int64_t n_ = 0;
+};
+
+// ------------------------------------------------------------------------------------------------------------------
+// a stack of blocks without gradients (moda_amd/modules.py: MoDAStack)
+// ------------------------------------------------------------------------------------------------------------------
+
+struct Block {
+  Tensor norm1_w, norm1_b, q_w, q_b, kv_w, kv_b, proj_w, proj_b, norm2_w, norm2_b, fc1_w, fc1_b, fc2_w, fc2_b, kv_ffn_w, kv_ffn_b;
+  double eps1, eps2;
+};
+
+// Forward pass of all blocks of one stack, launches only: the residual stream, one depth cache and four work tensors
+// are all there is.  A layer's K and V are projected straight into their slot of the cache, where its own attention reads
+// them as the sequence and later layers as a depth slot.  Returns nothing where a kernel's contract is not met (the
+// caller then runs the modules one by one): 16-bit types, widths the linear kernel takes, 16-byte rows.
+std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>& blocks, int64_t heads, int64_t kv_heads, bool is_causal,
+                                    int64_t chunk_tokens, bool post_norm) {
+  const auto type = x_in.scalar_type();
+  if (!x_in.is_cuda() || x_in.dim() != 3 || (type != at::kBFloat16 && type != at::kHalf) || x_in.numel() == 0) return {};
+  const int64_t B = x_in.size(0), N = x_in.size(1), C = x_in.size(2), hd = C / heads, kv = kv_heads * hd, M = B * N;
+  if (hd % 8 != 0 || hd > 256 || C % 64 != 0 || C > 4096) return {};
+  const int64_t hidden = blocks[0].fc1_w.size(0);
+  auto fits = [&](const Tensor& x, std::initializer_list<int64_t> shape) {
+    return x.defined() && has_shape(x, shape) && x.scalar_type() == type && x.device() == x_in.device() && x.is_contiguous() &&
+           (uintptr_t)x.const_data_ptr() % 16 == 0;
+  };
+  auto bias_fits = [&](const Tensor& x, int64_t n) { return !x.defined() || fits(x, {n}); };
+  if (hidden % 64 != 0) return {};
+  int64_t L = 0;
+  for (const Block& b : blocks) {
+    if (!(fits(b.norm1_w, {C}) && fits(b.norm1_b, {C}) && fits(b.norm2_w, {C}) && fits(b.norm2_b, {C}) && fits(b.q_w, {C, C}) &&
+          fits(b.kv_w, {2 * kv, C}) && fits(b.proj_w, {C, C}) && fits(b.fc1_w, {hidden, C}) && fits(b.fc2_w, {C, hidden}) &&
+          bias_fits(b.q_b, C) && bias_fits(b.kv_b, 2 * kv) && bias_fits(b.proj_b, C) && bias_fits(b.fc1_b, hidden) && bias_fits(b.fc2_b, C) &&
+          bias_fits(b.kv_ffn_b, 2 * kv) && (!b.kv_ffn_w.defined() || fits(b.kv_ffn_w, {2 * kv, C}))))
+      return {};
+    L += b.kv_ffn_w.defined() ? 2 : 1;
+  }
+  c10::OptionalDeviceGuard guard(x_in.device());
+  void* stream = stream_of(x_in);
+  const int dt = type == at::kHalf ? MODA_HIP_FP16 : MODA_HIP_BF16;
+  const int64_t es = 2;
+  const auto opt = x_in.options().requires_grad(false);
+  const Tensor x0 = x_in.contiguous();
+  if ((uintptr_t)x0.const_data_ptr() % 16 != 0) return {};
+  Tensor x = at::empty({B, N, C}, opt), x1 = at::empty({M, C}, opt), h = at::empty({M, C}, opt), q = at::empty({M, C}, opt),
+         hid = at::empty({M, hidden}, opt), ck = at::empty({B, N * L, kv}, opt), cv = at::empty({B, N * L, kv}, opt),
+         lse = at::empty({M * heads}, opt.dtype(at::kFloat));
+  auto part = [&](const Tensor& w, const Tensor& b, int64_t first, int64_t n, void* y, int64_t ldy) {
+    return moda_hip_linear_part{(const char*)in_ptr(w) + first * w.size(1) * es, b.defined() ? (const char*)in_ptr(b) + first * es : nullptr, y,
+                                ldy, n};
+  };
+  auto linear = [&](const void* in, int64_t K, std::initializer_list<moda_hip_linear_part> parts, const void* residual, bool gelu) {
+    check_rc(moda_hip_linear(dt, M, K, in, K, parts.begin(), (int32_t)parts.size(), residual, C, gelu, stream), "moda_hip_linear");
+  };
+  auto norm = [&](const void* in, const Tensor& w, const Tensor& b, double eps, const Tensor& out) {
+    check_rc(moda_hip_layer_norm(dt, M, C, in, in_ptr(w), in_ptr(b), (float)eps, out_ptr(out), stream), "moda_hip_layer_norm");
+  };
+  auto slot_of = [&](const Tensor& cache, int64_t slot) { return (char*)out_ptr(cache) + slot * kv * es; };
+
+  moda_hip_desc d = {};
+  d.struct_size = sizeof(d);
+  d.dtype = dt;
+  d.mode = chunk_tokens > 0 ? MODA_HIP_CHUNK_VISIBLE : is_causal ? MODA_HIP_CAUSAL : MODA_HIP_NONCAUSAL;
+  d.B = B;
+  d.T = N;
+  d.H = kv_heads;
+  d.G = heads / kv_heads;
+  d.D = d.Dv = hd;
+  d.chunk_tokens = chunk_tokens;
+  d.scale = (float)(1.0 / std::sqrt((double)hd));
+  d.q = d.o = {N * C, kv, hd};
+  d.k = d.v = {N * L * kv, L * kv, hd};
+  d.kd = d.vd = {N * L * kv, kv, hd};
+
+  const void* cur = in_ptr(x0);  // the residual stream
+  int64_t n = 0;                 // filled slots
+  for (const Block& b : blocks) {
+    const void* in = cur;
+    if (!post_norm) {
+      norm(cur, b.norm1_w, b.norm1_b, b.eps1, h);
+      in = in_ptr(h);
+    }
+    char *ks = slot_of(ck, n), *vs = slot_of(cv, n);
+    linear(in, C, {part(b.q_w, b.q_b, 0, C, out_ptr(q), C), part(b.kv_w, b.kv_b, 0, kv, ks, L * kv), part(b.kv_w, b.kv_b, kv, kv, vs, L * kv)},
+           nullptr, false);
+    d.L = n > 0 ? L : 0;
+    d.L_valid = (int32_t)n;
+    check_rc(moda_hip_fwd(&d, in_ptr(q), ks, vs, n > 0 ? in_ptr(ck) : nullptr, n > 0 ? in_ptr(cv) : nullptr, out_ptr(h),
+                          (float*)out_ptr(lse), stream),
+             "moda_hip_fwd");
+    linear(in_ptr(h), C, {part(b.proj_w, b.proj_b, 0, C, out_ptr(x1), C)}, cur, false);
+    if (post_norm) {
+      norm(in_ptr(x1), b.norm1_w, b.norm1_b, b.eps1, x1);
+      linear(in_ptr(x1), C, {part(b.fc1_w, b.fc1_b, 0, hidden, out_ptr(hid), hidden)}, nullptr, true);
+      linear(in_ptr(hid), hidden, {part(b.fc2_w, b.fc2_b, 0, C, out_ptr(h), C)}, in_ptr(x1), false);
+      norm(in_ptr(h), b.norm2_w, b.norm2_b, b.eps2, x);
+    } else {
+      norm(in_ptr(x1), b.norm2_w, b.norm2_b, b.eps2, h);
+      linear(in_ptr(h), C, {part(b.fc1_w, b.fc1_b, 0, hidden, out_ptr(hid), hidden)}, nullptr, true);
+      linear(in_ptr(hid), hidden, {part(b.fc2_w, b.fc2_b, 0, C, out_ptr(x), C)}, in_ptr(x1), false);
+    }
+    cur = in_ptr(x);
+    n++;
+    if (b.kv_ffn_w.defined()) {
+      linear(cur, C, {part(b.kv_ffn_w, b.kv_ffn_b, 0, kv, slot_of(ck, n), L * kv), part(b.kv_ffn_w, b.kv_ffn_b, kv, kv, slot_of(cv, n), L * kv)},
+             nullptr, false);
+      n++;
+    }
+  }
+  return x;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -463,6 +738,20 @@ PYBIND11_MODULE(_host, m) {
       .def_readonly("max_len", &Packed::max_len)
       .def_readonly("total", &Packed::total)
       .def_readonly("host", &Packed::host);
+  py::class_<TrainStream>(m, "TrainStream").def(py::init<int64_t>()).def("attend", &TrainStream::attend).def("push", &TrainStream::push);
+  m.def("depth_push", &depth_push);
+  m.def("stack_forward", [](const Tensor& x, const std::vector<std::vector<OptTensor>>& params, const std::vector<std::array<double, 2>>& eps,
+                            int64_t heads, int64_t kv_heads, bool is_causal, int64_t chunk_tokens, bool post_norm) {
+    std::vector<Block> blocks;
+    for (size_t i = 0; i < params.size(); i++) {
+      std::array<Tensor, 16> t;
+      for (size_t j = 0; j < 16; j++) t[j] = value(params[i].at(j));
+      blocks.push_back(Block{t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], t[10], t[11], t[12], t[13], t[14], t[15], eps[i][0], eps[i][1]});
+    }
+    py::gil_scoped_release nogil;
+    std::optional<Tensor> y = stack_forward(x, blocks, heads, kv_heads, is_causal, chunk_tokens, post_norm);
+    return y.has_value() ? OptTensor(*y) : OptTensor();
+  });
   m.def("set_fp32_compute", [](int code) { fp32_compute.store(code); });
   m.def("pack", &pack);
   m.def("check_shapes", [](int mode, const Tensor& q, const OptTensor& k, const OptTensor& v, const OptTensor& kd, const OptTensor& vd,
@@ -492,7 +781,8 @@ PYBIND11_MODULE(_host, m) {
       if (out.has_value())
         for (int i = 0; i < 5; i++) buffers[i] = value((*out)[i]);
       const Grads g = backward(*make_call(mode, scale, G, chunk_tokens, depth_valid, std::move(packed)), q, value(k), value(v),
-                               value(kd), value(vd), o, lse, d_o, stages, out.has_value() ? &buffers : nullptr, value(ws), accumulate);
+                               value(kd), value(vd), o, lse, d_o, stages, out.has_value() ? &buffers : nullptr, value(ws),
+                               accumulate ? kAccumulate : kOverwrite);
       for (int i = 0; i < 5; i++) r[i] = optional(g[i]);
     }
     return py::make_tuple(r[0], r[1], r[2], r[3], r[4]);

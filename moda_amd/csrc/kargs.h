@@ -26,7 +26,8 @@ struct KArgs {
   int Lv;    // slots per token that hold data, 1 <= Lv <= L: slots l >= Lv are invisible
   int Cb;    // chunk-visible: tokens per chunk
   int has_seq, causal, chunk;
-  int accum_depth;  // dkd, dvd += (slots l >= Lv untouched) instead of = (slots l >= Lv zeroed)
+  int accum_depth;  // dkd, dvd += instead of =
+  int keep_slots;   // slots l >= Lv of dkd, dvd untouched (always when accumulating) instead of zeroed
   int own_delta;    // the dQ kernel forms the row sums of o * do itself and leaves them in `delta` for the later kernels
   // Outside chunk-visible mode a query row sees the Lv depth slots of its own token only.  When the dQ kernel walks
   // them (its waves' own depth columns) it leaves the rounded P and dS of those (row, slot) pairs here,

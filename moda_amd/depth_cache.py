@@ -111,8 +111,7 @@ class DepthCache:
             assert tuple(x.shape) == self.shape, f"{name} must be {self.shape} like the cache, got {tuple(x.shape)}"
             assert x.dtype == self.k.dtype and x.device == self.k.device, \
                 f"{name} must have the cache's dtype ({self.k.dtype}) and device"
-        _reorg_fwd([k.contiguous()], self.k, self.n, self.L_max)
-        _reorg_fwd([v.contiguous()], self.v, self.n, self.L_max)
+        _lib.host().depth_push(k, v, self.k, self.v, self.n, self.L_max)
         self.n += 1
 
     def filled(self):

@@ -12,8 +12,9 @@ back): one token-major cache is preallocated per forward pass and each layer's K
 slot once.
   * With gradients flowing, a second buffer of the same shape collects the depth gradients: the backward
     of the attention that saw ``n`` slots adds its share to slots ``< n`` (the kernels' accumulate mode),
-    and the gradient of a layer's K/V is the slice of that buffer for its slot, read when autograd
-    reaches the layer.  Neither direction touches a slot more than once per consumer.
+    and the gradient of a layer's K/V is its own attention's plus the slice of that buffer for its slot,
+    joined when autograd reaches the layer.  Neither direction touches a slot more than once per consumer.
+    The autograd nodes and the bookkeeping are native (csrc/host.cpp: TrainStream).
   * Without gradients only the cache is kept.
   * ``inplace=False`` keeps the reference's behaviour (rebuild per layer, differentiable ``stack_depth``).
 """
@@ -25,75 +26,8 @@ import torch
 from torch import nn
 
 from . import _lib
-from .depth_cache import DepthCache, _reorg_bwd, _reorg_fwd, stack_depth
-from .ops import _chunk_tokens, _raw_bwd, _raw_fwd, parallel_moda, parallel_moda_chunk_visible
-
-
-class _TrainBuffers:
-    """Cache and gradient accumulators of one forward/backward pass, ``[B, T*L_max, H, D]`` each.  The
-    accumulators start as zeros; the cache needs no initialisation (the kernels never read a slot that has not
-    been written: ``depth_valid``)."""
-
-    def __init__(self, B, T, L_max, H, D, dtype, device):
-        self.shape, self.L_max = (B, T, H, D), L_max
-        self.k = torch.empty(B, T * L_max, H, D, dtype=dtype, device=device)
-        self.v = torch.empty_like(self.k)
-        self.gk = torch.zeros_like(self.k)
-        self.gv = torch.zeros_like(self.k)
-
-
-class _StreamAttention(torch.autograd.Function):
-    """parallel_moda over the sequence and the first ``n`` slots of the stream's cache.  The cache is not an
-    autograd input: its gradient goes to the stream's accumulators, from where ``_StreamPush.backward`` of the
-    layer that owns a slot hands it on.  ``token`` chains the stream's operations so that autograd runs
-    their backward passes in reverse order whatever else connects the layers."""
-
-    @staticmethod
-    @torch.amp.custom_fwd(device_type="cuda")
-    def forward(ctx, q, k, v, token, buf, n, scale, G, mode, chunk_tokens):
-        o, lse = _raw_fwd(mode, q, k, v, buf.k if n else None, buf.v if n else None, scale, G, chunk_tokens,
-                          depth_valid=n if n else None)
-        ctx.save_for_backward(q, k, v, o, lse)
-        ctx.buf, ctx.n, ctx.scale, ctx.G, ctx.mode, ctx.chunk_tokens = buf, n, scale, G, mode, chunk_tokens
-        ctx.set_materialize_grads(False)
-        ctx.mark_non_differentiable(lse)
-        return o, lse, token.new_zeros(())
-
-    @staticmethod
-    @torch.amp.custom_bwd(device_type="cuda")
-    def backward(ctx, do, _dlse, _dtoken):
-        q, k, v, o, lse = ctx.saved_tensors
-        buf, n = ctx.buf, ctx.n
-        do = torch.zeros_like(o) if do is None else do.to(o.dtype)
-        mode, cb = ctx.mode, ctx.chunk_tokens
-        dq, dk, dv = torch.empty_like(q), torch.empty(k.shape, dtype=k.dtype, device=k.device), \
-            torch.empty(v.shape, dtype=v.dtype, device=v.device)
-        if n:
-            _raw_bwd(mode, q, k, v, buf.k, buf.v, o, lse, do, ctx.scale, ctx.G, cb, out=(dq, dk, dv, buf.gk, buf.gv),
-                     depth_valid=n, accumulate_depth=True)
-        else:
-            _raw_bwd(mode, q, k, v, None, None, o, lse, do, ctx.scale, ctx.G, cb, out=(dq, dk, dv, None, None))
-        return dq, dk, dv, None, None, None, None, None, None, None
-
-
-class _StreamPush(torch.autograd.Function):
-    """Writes one layer's K/V into slot ``slot`` of the cache; its backward returns what the attention calls
-    that saw the slot have added to the gradient accumulators (all of them ran before: see ``token``)."""
-
-    @staticmethod
-    def forward(ctx, k, v, token, buf, slot):
-        _reorg_fwd([k.contiguous()], buf.k, slot, buf.L_max)
-        _reorg_fwd([v.contiguous()], buf.v, slot, buf.L_max)
-        ctx.buf, ctx.slot = buf, slot
-        ctx.set_materialize_grads(False)
-        return token.new_zeros(())
-
-    @staticmethod
-    def backward(ctx, _dtoken):
-        buf = ctx.buf
-        (gk,) = _reorg_bwd(buf.gk, 1, ctx.slot, buf.L_max, buf.shape)
-        (gv,) = _reorg_bwd(buf.gv, 1, ctx.slot, buf.L_max, buf.shape)
-        return gk, gv, None, None, None
+from .depth_cache import DepthCache, stack_depth
+from .ops import _chunk_tokens, parallel_moda, parallel_moda_chunk_visible
 
 
 class DepthStream:
@@ -113,8 +47,7 @@ class DepthStream:
         self.max_layers = int(max_layers)
         self._layers: List[Tuple[torch.Tensor, torch.Tensor]] = []
         self._cache: Optional[DepthCache] = None
-        self._train: Optional[_TrainBuffers] = None
-        self._token: Optional[torch.Tensor] = None
+        self._train = None  # native TrainStream, from the first call with gradients flowing
         self._n = 0
         self._inplace: Optional[bool] = inplace
         self._mode: Optional[str] = None  # 'train' | 'infer' | 'rebuild', fixed by the first push
@@ -135,19 +68,21 @@ class DepthStream:
     def push(self, k: torch.Tensor, v: torch.Tensor):
         assert self._n < self.max_layers, "depth stream is full"
         self._decide(k, v)
-        B, T, H, D = k.shape
         if self._mode == "train":
-            if self._train is None:
-                self._train = _TrainBuffers(B, T, self.max_layers, H, D, k.dtype, k.device)
-                self._token = torch.zeros((), device=k.device)
-            self._token = _StreamPush.apply(k, v, self._token, self._train, self._n)
+            self._native().push(k, v)
         elif self._mode == "infer":
             if self._cache is None:
+                B, T, H, D = k.shape
                 self._cache = DepthCache(B, T, self.max_layers, H, D, k.dtype, k.device)
             self._cache.append(k.detach(), v.detach())
         else:
             self._layers.append((k, v))
         self._n += 1
+
+    def _native(self):
+        if self._train is None:
+            self._train = _lib.host().TrainStream(self.max_layers)
+        return self._train
 
     def context(self):
         self._used_context = True
@@ -175,14 +110,9 @@ class DepthStream:
                 "To keep depth alignment consistent with backward, BT % moda_group_num must be 0"
             if scale is None:
                 scale = q.shape[-1] ** -0.5
-            if self._token is None:
-                self._token = torch.zeros((), device=q.device)
-            buf = self._train if self._n else None
             mode = _lib.CHUNK_VISIBLE if chunk_visible else _lib.CAUSAL if is_causal else _lib.NONCAUSAL
             cb = _chunk_tokens(moda_group_num, chunk_rows) if chunk_visible else 0
-            o, _, self._token = _StreamAttention.apply(q, k, v, self._token, buf, self._n, scale, moda_group_num,
-                                                       mode, cb)
-            return o
+            return self._native().attend(q, k, v, scale, moda_group_num, mode, cb)
         if self._n == 0:
             dk = dv = n = None
         elif self._mode == "infer":
@@ -285,7 +215,63 @@ class MoDAStack(nn.Module):
             blk.mlp = nn.Sequential(nn.Linear(dim, hidden), nn.GELU(), nn.Linear(hidden, dim))
             self.blocks.append(blk)
 
+    def _plain_parameters(self):
+        """Parameters and norm epsilons of every block for the native forward pass, or None when a block is not what
+        the constructor made: a replaced, subclassed, patched or hooked module, blocks that differ, active dropout."""
+        params, eps, first = [], [], None
+        for blk in self.blocks:
+            sub = blk._modules
+            attn, mlp = sub["attn"], sub["mlp"]
+            parts = attn._modules
+            if type(attn) is not MoDAAttention or type(mlp) is not nn.Sequential or len(mlp) != 3:
+                return None
+            q, kv, proj, drop, kv_ffn = (parts.get(n) for n in ("q", "kv", "proj", "proj_drop", "kv_ffn"))
+            norm1, norm2 = sub["norm1"], sub["norm2"]
+            fc1, act, fc2 = mlp._modules.values()
+            linears = (q, kv, proj, fc1, fc2) if kv_ffn is None else (q, kv, proj, fc1, fc2, kv_ffn)
+            if not (all(type(m) is nn.Linear for m in linears) and type(norm1) is nn.LayerNorm and type(norm2) is nn.LayerNorm
+                    and type(act) is nn.GELU and act.approximate == "none" and type(drop) is nn.Dropout):
+                return None
+            if (drop.training and drop.p > 0) or (self.ffn_kv and kv_ffn is None):
+                return None
+            for m in (attn, mlp, norm1, norm2, act, drop, *linears):
+                if m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__:
+                    return None
+            what = (attn.num_heads, attn.num_kv_heads, attn.is_causal, attn.chunk_rows, attn.scale)
+            if first is None:
+                first = what
+            if what != first or attn.scale != attn.head_dim ** -0.5:
+                return None
+            tensors = [p for m in (norm1, q, kv, proj, norm2, fc1, fc2) for p in (m._parameters["weight"], m._parameters["bias"])]
+            tensors += [None, None] if kv_ffn is None or not self.ffn_kv else [kv_ffn._parameters["weight"], kv_ffn._parameters["bias"]]
+            if not all(t is None or type(t) is nn.Parameter for t in tensors):
+                return None
+            params.append(tensors)
+            eps.append((norm1.eps, norm2.eps))
+        return (params, eps) if params else None
+
+    def _forward_native(self, x):
+        """The whole stack as kernel launches from native code (csrc/host.cpp: stack_forward), for calls through which
+        no gradient flows; None where the modules have to run one by one.  Twelve blocks of width 256 on 64 x 197
+        tokens issue some 200 framework operations of about 10 us host time each when run as modules."""
+        attn = self.blocks[0].attn if len(self.blocks) else None
+        if (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or type(attn) is not MoDAAttention
+                or nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks
+                or type(x) is not torch.Tensor or x.dim() != 3 or x.shape[-1] != attn.num_heads * attn.head_dim):
+            return None
+        if 128 % attn.moda_group_num or (attn.chunk_rows is not None and not attn.is_causal):
+            return None  # attend() refuses these
+        plain = self._plain_parameters()
+        if plain is None:
+            return None
+        cb = 0 if attn.chunk_rows is None else _chunk_tokens(attn.moda_group_num, attn.chunk_rows)
+        return _lib.host().stack_forward(x, plain[0], plain[1], attn.num_heads, attn.num_kv_heads, bool(attn.is_causal), cb, self.post_norm)
+
     def forward(self, x, inplace_cache: Optional[bool] = None):
+        if inplace_cache is not False:
+            y = self._forward_native(x)
+            if y is not None:
+                return y
         stream = DepthStream(len(self.blocks) * (2 if self.ffn_kv else 1), inplace=inplace_cache)
         for blk in self.blocks:
             if self.post_norm:
