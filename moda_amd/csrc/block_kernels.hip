@@ -24,16 +24,32 @@ struct LinearArgs {
 
 enum Epilogue { kBias, kGelu, kResidual };
 
+// The exact GELU, x Phi(x) = max(x, 0) - |x| / 2 erfc(|x| / sqrt 2).  erfc(z) = exp(-z^2) t R(t) with t = 1 / (1 + 0.38 z):
+// R is a degree-6 fit of erfcx(z) / t over [0, 12], relative error 1.1e-6 -- three hundred times below a rounding to 11
+// bits, in both tails.  A fifth of the instructions of erff, which took two thirds of the launch.
+__device__ __forceinline__ float gelu(float x) {
+  const float a = fminf(fabsf(x), 14.f);  // beyond, the second term is below 1e-43
+  const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(a, 0.38f * 0.70710678f, 1.f));
+  float r = -0.12541133165359497f;
+  r = __builtin_fmaf(r, t, 0.3360145092010498f);
+  r = __builtin_fmaf(r, t, -0.06988266855478287f);
+  r = __builtin_fmaf(r, t, 0.24781261384487152f);
+  r = __builtin_fmaf(r, t, 0.18060259521007538f);
+  r = __builtin_fmaf(r, t, 0.21657583117485046f);
+  r = __builtin_fmaf(r, t, 0.2142874300479889f);
+  return (x < 0.f ? 0.f : x) - 0.5f * a * t * r * fast_exp2(a * a * (-0.5f * kLog2e));
+}
+
 // y = x W^T: both operands have the summation index innermost, so a k step is a 64-element-wide tile of each, staged
 // like the attention kernels' 64-wide tiles.  Four waves share a BM (rows) x BN (features) output tile, two by two.
 // The features sit on the matrix instruction's A side: a lane then holds four consecutive features of one row.
 //
-// Sized for a vision model's linears (12 608 rows, K 256 .. 1024), where a launch is a few microseconds and the k loop
-// 4 to 16 steps: what counts is enough workgroups for every compute unit's two or three places, not a large tile.
+// Sized for a vision model's linears (12 608 rows, K 256 .. 1024), where a launch is 8 to 20 us and the k loop 4 to 16
+// steps: what counts is enough workgroups in flight to cover each one's start and end, not a large tile.
 // The feature tiles of one row tile go to one XCD (blocks b, b + 8, b + 16, ... share an L2), which reads x once.
-template <typename T, int BM, int BN, Epilogue EPI>
+template <typename T, int BM, int BN, int NST, Epilogue EPI>
 __global__ __launch_bounds__(256, 2) void linear_kernel(const LinearArgs a) {
-  constexpr int NST = BM + BN > 192 ? 2 : 3, DIST = NST - 1, MB = BN / 32, NB = BM / 32, STAGE = (BM + BN) * 64;
+  constexpr int DIST = NST - 1, MB = BN / 32, NB = BM / 32, STAGE = (BM + BN) * 64;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   lds_ptr smem = (lds_ptr)smem_raw;
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, q4 = lane >> 4;
@@ -125,7 +141,7 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(const LinearArgs a) {
       }
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        if (EPI == kGelu) x[i] = 0.5f * x[i] * (1.f + erff(x[i] * 0.70710678118654752f));
+        if (EPI == kGelu) x[i] = gelu(x[i]);
         if (EPI == kResidual) x[i] += res[i];
       }
       i32x2 w;
@@ -190,18 +206,18 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const uint16_t* x, cons
 
 namespace {
 
-template <typename T, int BM, int BN, Epilogue EPI>
+template <typename T, int BM, int BN, int NST, Epilogue EPI>
 hipError_t launch_linear_t(LinearArgs a, hipStream_t stream) {
-  constexpr size_t smem = (size_t)(BM + BN > 192 ? 2 : 3) * (BM + BN) * 64 * sizeof(uint16_t);
+  constexpr size_t smem = (size_t)NST * (BM + BN) * 64 * sizeof(uint16_t);
   static LdsAttrState attr;
-  const hipError_t e = allow_dynamic_lds(attr, reinterpret_cast<const void*>(&linear_kernel<T, BM, BN, EPI>), smem);
+  const hipError_t e = allow_dynamic_lds(attr, reinterpret_cast<const void*>(&linear_kernel<T, BM, BN, NST, EPI>), smem);
   if (e != hipSuccess) return e;
   a.m_tiles = (a.rows + BM - 1) / BM;
   a.n_tiles = 0;
   for (int i = 0; i < a.n_parts; i++) a.part[i].tile_end = a.n_tiles += (a.part[i].n + BN - 1) / BN;
   const int64_t nblk = 8ll * ((a.m_tiles + 7) / 8) * a.n_tiles;
   if (nblk >= (1ll << 31)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((linear_kernel<T, BM, BN, EPI>), dim3((unsigned)nblk), dim3(256), smem, stream, a);
+  hipLaunchKernelGGL((linear_kernel<T, BM, BN, NST, EPI>), dim3((unsigned)nblk), dim3(256), smem, stream, a);
   return hipGetLastError();
 }
 
@@ -212,10 +228,15 @@ hipError_t launch_linear_e(const LinearArgs& a, int cus, hipStream_t stream) {
     for (int i = 0; i < a.n_parts; i++) t += (a.part[i].n + bn - 1) / bn;
     return t * ((a.rows + bm - 1) / bm);
   };
-  // the largest tile that still gives every compute unit its two workgroups
-  if (tiles(128, 128) >= 2ll * cus) return launch_linear_t<T, 128, 128, EPI>(a, stream);
-  if (tiles(128, 64) >= 2ll * cus) return launch_linear_t<T, 128, 64, EPI>(a, stream);
-  return launch_linear_t<T, 64, 64, EPI>(a, stream);
+  // Measured at 1 900 .. 12 608 rows, K 128 .. 3 072.  A 128 x 128 tile where its grid is one full round of two
+  // workgroups per compute unit (12 608 x 512 -> 512: 17 us, others 18 - 24); 128 x 64 where that still gives two each
+  // (256 -> 384: 8.7 us), with a third stage in flight for a long k loop in one round (1024 -> 256: 14.6 against
+  // 15.9 us); else small tiles, five workgroups per compute unit.
+  const int64_t large = tiles(128, 128), tall = tiles(128, 64);
+  if (large >= cus + cus / 4 && large <= 2ll * cus) return launch_linear_t<T, 128, 128, 2, EPI>(a, stream);
+  if (tall >= 2ll * cus) return launch_linear_t<T, 128, 64, 2, EPI>(a, stream);
+  if (tall > cus && a.K >= 512) return launch_linear_t<T, 128, 64, 3, EPI>(a, stream);
+  return launch_linear_t<T, 64, 64, 2, EPI>(a, stream);
 }
 
 template <typename T>

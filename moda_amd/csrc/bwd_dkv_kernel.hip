@@ -97,13 +97,6 @@ __global__ __launch_bounds__(512) void dkv_kernel(const KArgs a_in) {
     }
   }
 
-  // The register operands above must have arrived before the tile loads start: those are issued
-  // behind the compiler's back, and a load it still believes pending would cost a vmcnt(0) in every
-  // trip of the main loop.
-  asm volatile("" ::: "memory");  // keep the loads above this point
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  asm volatile("" ::: "memory");
-
   // visible query-row interval of this lane's columns
   int qlo[NB], qhi[NB];
 #pragma unroll
@@ -194,7 +187,11 @@ __global__ __launch_bounds__(512) void dkv_kernel(const KArgs a_in) {
   if (feeding) prep();
 #pragma unroll
   for (int k = 0; k < kParts; k++) part(k);
+  // The tile loads are issued behind the compiler's back, and a register operand it still believes pending would cost
+  // a vmcnt(0) in every trip of the main loop: both kinds are waited for here, once, having travelled together.
+  asm volatile("" ::: "memory");
   Loader::wait_all();
+  asm volatile("" ::: "memory");
   __syncthreads();
 
   // Query tiles whose rows ALL see ALL 128 columns of this workgroup need no masking and no

@@ -126,11 +126,6 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
     dlo[nb] = vis.dlo;
     dhi[nb] = vis.dhi;
   }
-  // the register operands must have arrived before the tile loads (issued behind the compiler's back) start
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  asm volatile("" ::: "memory");
-
   // Depth columns a wave alone can see are not streamed through the workgroup's ring: each wave fetches its own
   // rows' span after the sequence tiles (see the end of the kernel), when a 32-column K and V tile per wave fit.
   constexpr bool OWN_FITS = Shape::W * 64 * HD * 2 <= 128 * 1024;
@@ -197,7 +192,11 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
 #pragma unroll
   for (int j = 0; j < DIST; j++)
     if (j < ntiles) issue(j);
-  wait_tile(0);
+  // The tile loads are issued behind the compiler's back, and a register operand it still believes pending would cost
+  // a vmcnt(0) in every trip of the main loop: both kinds are waited for here, once, having travelled together.
+  asm volatile("" ::: "memory");
+  Loader::wait_all();
+  asm volatile("" ::: "memory");
   __syncthreads();
   int c_st = 0;
 
@@ -570,7 +569,7 @@ hipError_t launch_dq_t_shape(const KArgs& a, hipStream_t stream) {
   // which the gradients leave
   constexpr size_t ring = (size_t)Shape::NST * 2 * 64 * HD * sizeof(uint16_t),
                    own = (size_t)Shape::W * (HD <= kDepthGradsInDqMaxWidth ? 2 * 64 + 16 : 64) * HD * sizeof(uint16_t);
-  constexpr size_t smem = (size_t)Shape::W * 64 * HD * sizeof(uint16_t) <= 128 * 1024 ? std::max(ring, own) : ring;
+  constexpr size_t smem = (ADDR & 4) == 0 && (size_t)Shape::W * 64 * HD * sizeof(uint16_t) <= 128 * 1024 ? std::max(ring, own) : ring;
   static LdsAttrState attr;
   const hipError_t ea = allow_dynamic_lds(attr, reinterpret_cast<const void*>(&dq_kernel<T, HD, Shape, ADDR>), smem);
   if (ea != hipSuccess) return ea;
@@ -584,10 +583,15 @@ hipError_t launch_dq_t_shape(const KArgs& a, hipStream_t stream) {
 
 template <typename T, int HD, int ADDR>
 hipError_t launch_dq_t_addr(const KArgs& a, bool small, hipStream_t stream) {
-  if constexpr (HD > 128) return launch_dq_t_shape<T, HD, RowWide, ADDR>(a, stream);  // one shape for the wide tiles
-  else {
-    if (ADDR & 1) return launch_dq_t_shape<T, HD, RowLarge, ADDR>(a, stream);  // slices wider than 2 GiB: never a small launch
-    if (small) return launch_dq_t_shape<T, HD, RowSmall<HD>, ADDR>(a, stream);
+  if constexpr (HD <= 64) {
+    const ShortRows rows = (ADDR & 3) ? ShortRows::kNone : pick_short_rows(a.Tq, (long long)a.B * a.Hq, a.causal, a.compute_units);
+    if (rows == ShortRows::kTwoStages) return launch_dq_t_shape<T, HD, RowShort, ADDR & ~3>(a, stream);
+    if (rows == ShortRows::kThreeStages) return launch_dq_t_shape<T, HD, RowShort3, ADDR & ~3>(a, stream);
+    return launch_dq_t_shape<T, HD, RowSmall<HD>, ADDR>(a, stream);
+  } else if constexpr (HD > 128) {
+    return launch_dq_t_shape<T, HD, RowWide, ADDR>(a, stream);  // one shape for the wide tiles
+  } else {
+    if (small && !(ADDR & 1)) return launch_dq_t_shape<T, HD, RowSmall<HD>, ADDR & ~1>(a, stream);  // slices wider than 2 GiB: never small
     return launch_dq_t_shape<T, HD, RowLarge, ADDR>(a, stream);
   }
 }
@@ -598,7 +602,8 @@ hipError_t launch_dq_t(const KArgs& a, hipStream_t stream) {
   const int64_t span = 2 * std::max(std::max((int64_t)a.T * a.sk.t, (int64_t)a.T * a.sv.t),
                                     std::max((int64_t)a.T * a.L * a.skd.t, (int64_t)a.T * a.L * a.svd.t));
   const bool wide = span > 0x7fffffffll;
-  const bool small = use_small_rows(a.Tq, (long long)a.B * a.Hq, a.compute_units);
+  const bool small = a.cu ? use_small_rows(a.delta_pitch, a.Hq, a.compute_units)  // the rows there are, not those of the grid
+                          : use_small_rows(a.Tq, (long long)a.B * a.Hq, a.compute_units);
   switch ((wide ? 1 : 0) | (a.cu ? 2 : 0) | (a.L == 0 ? 4 : 0) | (a.L > 0 && a.Lv != a.L ? 8 : 0)) {
     case 0: return launch_dq_t_addr<T, HD, 0>(a, small, stream);
     case 1: return launch_dq_t_addr<T, HD, 1>(a, small, stream);

@@ -31,13 +31,12 @@ using FwdLarge = RowLargePP;
 // ADDR bit 0: a (batch, head) slice is wider than 2 GiB (descriptors anchored per tile instead of 32-bit
 // offsets inside the slice); bit 1: packed variable-length batch; bit 2: no depth stream; bit 3: partially filled
 // depth stream (only Lv of a token's L slots hold data: depth tiles are loaded through the slot mapping)
+// On the 64-wide tiles the registers of three waves per SIMD are enough (168, no spills).
 template <typename T, int HD, typename Shape, int ADDR>
-__global__ __launch_bounds__(64 * Shape::W, 2) void fwd_kernel(const KArgs a_in) {
+__global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(const KArgs a_in) {
   constexpr int BM = 32 * Shape::W, BN = 64, KK = HD / 16, DB = HD / 32, NT = 64 * Shape::W, NST = Shape::NST,
                 DIST = Shape::DIST;
   constexpr bool PP = Shape::PP;
-  // on the 64-wide tiles the waves' own depth columns go through two sets of private tiles (see the end of the kernel)
-  constexpr bool TWO_OWN_SETS = HD <= 64;
   static_assert(NST >= DIST + 1 + (PP ? 1 : 0) && DIST >= 1 && DIST <= 2,
                 "ring must hold the tile in use, the tiles in flight and (ping-pong) the previous tile");
   static_assert(2 * NST >= Shape::W, "the ring must be large enough for one 32-column K tile and V tile per wave");
@@ -74,13 +73,6 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void fwd_kernel(const KArgs a_in)
       Qr[kk] = (valid && 16 * kk + 8 * g < a.D) ? *reinterpret_cast<const i32x4*>(qp + 16 * kk) : z;
     }
   }
-
-  // The register operands above must have arrived before the tile loads start: those are issued
-  // behind the compiler's back, and a load it still believes pending would cost a vmcnt(0) in every
-  // trip of the main loop.
-  asm volatile("" ::: "memory");  // keep the loads above this point
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  asm volatile("" ::: "memory");
 
   // per-row visible column intervals [lo, hi) for the two phases
   const RowVis vis = row_visibility(a, r, Ld);
@@ -155,7 +147,11 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void fwd_kernel(const KArgs a_in)
 #pragma unroll
   for (int j = 0; j < DIST; j++)
     if (j < ntiles) issue(j);
-  wait_tile(0);
+  // The tile loads are issued behind the compiler's back, and a register operand it still believes pending would cost
+  // a vmcnt(0) in every trip of the main loop: both kinds are waited for here, once, having travelled together.
+  asm volatile("" ::: "memory");
+  Loader::wait_all();
+  asm volatile("" ::: "memory");
   __syncthreads();
   int c_st = 0;  // ring stage of the tile being consumed
 
@@ -361,25 +357,6 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void fwd_kernel(const KArgs a_in)
       fetch(Kt, kdp, a.skd.t, c_beg, a.D);
       fetch(Vt, vdp, a.svd.t, c_beg, a.Dv);
       const std::integral_constant<int, 1> one{};
-      if constexpr (TWO_OWN_SETS) {
-        // room for two sets of private tiles: the rows of tile j + 1 travel while tile j is worked on
-        constexpr int SET = Shape::W * 2 * 32 * HD;
-        for (int j = 0; j < nh; j++) {
-          const int col0 = c_beg + 32 * j;
-          lds_ptr Kc = Kt + (j & 1) * SET, Vc = Vt + (j & 1) * SET;
-          Own::template wait_but<0>();
-          if (j + 1 < nh) {
-            fetch(Kt + ((j + 1) & 1) * SET, kdp, a.skd.t, col0 + 32, a.D);
-            fetch(Vt + ((j + 1) & 1) * SET, vdp, a.svd.t, col0 + 32, a.Dv);
-          }
-          front(std::true_type{}, one, Kc, col0, dlo, dhi, []() {});
-          TrPipe<T, HD, 2, 2> pv1;
-          const i32x4 P1[2] = {P[0], P[1]};
-          pv1.prefetch(oa, Vc);
-          pv1.run(oa, Vc, P1, o);
-          Own::reads_done();  // this set may be loaded over in the next trip
-        }
-      } else {
       for (int j = 0; j < nh; j++) {
         const int col0 = c_beg + 32 * j;
         const bool more = j + 1 < nh;
@@ -397,7 +374,6 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void fwd_kernel(const KArgs a_in)
         pv1.run(oa, Vt, P1, o);
         Own::reads_done();
         if (more) fetch(Vt, vdp, a.svd.t, col0 + 32, a.Dv);
-      }
       }
     }
   }
@@ -462,13 +438,6 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void fwd_wide_kernel(const KArgs 
     dlo[nb] = vis.dlo;
     dhi[nb] = vis.dhi;
   }
-
-  // The register operands above must have arrived before the tile loads start: those are issued
-  // behind the compiler's back, and a load it still believes pending would cost a vmcnt(0) in every
-  // trip of the main loop.
-  asm volatile("" ::: "memory");  // keep the loads above this point
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  asm volatile("" ::: "memory");
 
   // the workgroup's column tiles: depth columns always stream through the ring here
   const RowTilePlan plan = row_tile_plan(a, qt, BM, BN, a.L > 0);
@@ -544,7 +513,11 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void fwd_wide_kernel(const KArgs 
 #pragma unroll
   for (int j = 0; j < DIST; j++)
     if (j < ntiles) issue(j);
-  wait_tile(0);
+  // The tile loads are issued behind the compiler's back, and a register operand it still believes pending would cost
+  // a vmcnt(0) in every trip of the main loop: both kinds are waited for here, once, having travelled together.
+  asm volatile("" ::: "memory");
+  Loader::wait_all();
+  asm volatile("" ::: "memory");
   __syncthreads();
   int c_st = 0;  // ring stage of the tile being consumed
 
@@ -683,10 +656,7 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void fwd_wide_kernel(const KArgs 
 
 template <typename T, int HD, typename Shape, int ADDR>
 hipError_t launch_fwd_t_shape(const KArgs& a, hipStream_t stream) {
-  // the ring, or (64-wide tiles) two sets of a private 32-column K tile and V tile per wave, whichever is larger
-  constexpr size_t ring = (size_t)Shape::NST * 2 * 64 * HD * sizeof(uint16_t);
-  constexpr size_t own = HD <= 64 ? (size_t)2 * Shape::W * 2 * 32 * HD * sizeof(uint16_t) : 0;
-  constexpr size_t smem = ring > own ? ring : own;
+  constexpr size_t smem = (size_t)Shape::NST * 2 * 64 * HD * sizeof(uint16_t);  // the ring
   static LdsAttrState attr;
   const hipError_t ea = allow_dynamic_lds(attr, reinterpret_cast<const void*>(&fwd_kernel<T, HD, Shape, ADDR>), smem);
   if (ea != hipSuccess) return ea;
@@ -715,10 +685,14 @@ hipError_t launch_fwd_wide(const KArgs& a, hipStream_t stream) {
 
 template <typename T, int HD, int ADDR>
 hipError_t launch_fwd_t_addr(const KArgs& a, bool small, hipStream_t stream) {
-  if constexpr (HD > 128) return launch_fwd_wide<T, HD, ADDR & 11>(a, stream);
-  else {
-    if (ADDR & 1) return launch_fwd_t_shape<T, HD, FwdLarge, ADDR>(a, stream);  // slices wider than 2 GiB: never a small launch
-    if (small) return launch_fwd_t_shape<T, HD, RowSmall<HD>, ADDR>(a, stream);
+  if constexpr (HD <= 64) {
+    if (!(ADDR & 3) && pick_short_rows(a.Tq, (long long)a.B * a.Hq, a.causal, a.compute_units) == ShortRows::kTwoStages)
+      return launch_fwd_t_shape<T, HD, RowShort, ADDR & ~3>(a, stream);
+    return launch_fwd_t_shape<T, HD, RowSmall<HD>, ADDR>(a, stream);
+  } else if constexpr (HD > 128) {
+    return launch_fwd_wide<T, HD, ADDR & 11>(a, stream);
+  } else {
+    if (small && !(ADDR & 1)) return launch_fwd_t_shape<T, HD, RowSmall<HD>, ADDR & ~1>(a, stream);  // slices wider than 2 GiB: never small
     return launch_fwd_t_shape<T, HD, FwdLarge, ADDR>(a, stream);
   }
 }
@@ -729,7 +703,8 @@ hipError_t launch_fwd_t(const KArgs& a, hipStream_t stream) {
   const int64_t span = 2 * std::max(std::max((int64_t)a.T * a.sk.t, (int64_t)a.T * a.sv.t),
                                     std::max((int64_t)a.T * a.L * a.skd.t, (int64_t)a.T * a.L * a.svd.t));
   const bool wide = span > 0x7fffffffll;
-  const bool small = use_small_rows(a.Tq, (long long)a.B * a.Hq, a.compute_units);
+  const bool small = a.cu ? use_small_rows(a.delta_pitch, a.Hq, a.compute_units)  // the rows there are, not those of the grid
+                          : use_small_rows(a.Tq, (long long)a.B * a.Hq, a.compute_units);
   switch ((wide ? 1 : 0) | (a.cu ? 2 : 0) | (a.L == 0 ? 4 : 0) | (a.L > 0 && a.Lv != a.L ? 8 : 0)) {
     case 0: return launch_fwd_t_addr<T, HD, 0>(a, small, stream);
     case 1: return launch_fwd_t_addr<T, HD, 1>(a, small, stream);

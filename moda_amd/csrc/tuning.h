@@ -6,12 +6,16 @@ namespace moda {
 // Waves per workgroup (16 * NB query rows each; NB matters to the 16x16x32 kernels only), LDS ring stages of one 64-column K tile + V tile, and how
 // many tiles ahead the global->LDS loads run.
 //
-// RowLarge is the throughput shape: 256 query rows share every K/V tile.  RowSmall is for problems
-// with few query rows per (batch, head), where the large shape leaves compute units without a
-// workgroup and makes every wave sit through the barriers of depth tiles that only other waves of
-// its workgroup touch: fewer rows per workgroup mean more workgroups and a depth range that is
-// mostly the wave's own.  Its wave count is the smallest one whose tile loader covers a multiple
-// of 16 rows per pass (the LDS swizzle repeats every 16 rows).
+// 128-wide tiles: RowLarge is the throughput shape, 256 query rows share every K/V tile, one workgroup per compute unit.
+// RowSmall<128> is for problems with few query rows per (batch, head), where the large shape leaves compute units
+// without a workgroup and makes every wave sit through the barriers of depth tiles that only other waves of its
+// workgroup touch.
+//
+// 64-wide tiles: four waves (128 rows) with two ring stages of 16 KB are the better shape at every size.  Two
+// workgroups of the dQ kernel and three of the forward kernel (whose registers then fit three waves per SIMD) share a
+// compute unit and cover each other's softmax, depth phase, start and end, where the eight-wave workgroup of
+// the 128-wide tiles is alone: forward 2.87 -> 2.47 ms and dQ 3.71 -> 3.57 ms at 16 K tokens, 64 query heads, 64 slots;
+// 181 -> 145 us and 217 -> 187 us at 3 x 4 144 tokens, 16 query heads without a depth stream.
 struct RowLarge {
   static constexpr int W = 8, NST = 3, DIST = 2, NB = 2;
   static constexpr bool PP = false;
@@ -23,15 +27,18 @@ struct RowLargePP {
   static constexpr bool PP = true;
 };
 template <int HD>
-struct RowSmall;
-template <>
-struct RowSmall<64> {
-  static constexpr int W = 2, NST = 3, DIST = 2, NB = 2;  // 48 KB of LDS: three workgroups per compute unit
+struct RowSmall {
+  static constexpr int W = 4, NST = 2, DIST = 1, NB = 2;  // 64 KB of LDS at 128, 32 KB at 64
   static constexpr bool PP = false;
 };
-template <>
-struct RowSmall<128> {
-  static constexpr int W = 4, NST = 2, DIST = 1, NB = 2;  // 64 KB of LDS: two workgroups per compute unit
+// 64-wide tiles, short sequences: two waves, for a row count whose last 128-row tile would be half empty.
+struct RowShort {
+  static constexpr int W = 2, NST = 2, DIST = 1, NB = 2;
+  static constexpr bool PP = false;
+};
+// ... and with a third ring stage, for dQ launches of equal, HBM-bound workgroups (see pick_short_rows).
+struct RowShort3 {
+  static constexpr int W = 2, NST = 3, DIST = 2, NB = 2;
   static constexpr bool PP = false;
 };
 
@@ -42,11 +49,28 @@ struct RowWide {
   static constexpr bool PP = false;
 };
 
-// Host side: the small shape is used when the large one would not even give every compute unit
+// Host side, 128-wide tiles: the small shape is used when the large one would not even give every compute unit
 // two workgroups.
 inline bool use_small_rows(long long rows_per_head, long long heads, int compute_units) {
   const long long large_blocks = (rows_per_head + 32 * RowLarge::W - 1) / (32 * RowLarge::W) * heads;
   return large_blocks < 2ll * compute_units;
+}
+
+// Host side, 64-wide tiles: which two-wave shape a launch takes instead of the four-wave one.
+enum class ShortRows { kNone, kTwoStages, kThreeStages };
+// RowShort: an odd number of 64-row tiles per head, few enough for the half-empty 128-row tile to count (at 16 tiles
+// it is 3 % of the rows), and more 128-row workgroups than compute units (fewer run side by side anyway).
+// 64 x 197 tokens, four query rows each, six slots: dQ 24.3 -> 22.7 us; 101 x 257, two heads of two: 92 -> 90 us.
+// RowShort3: equal workgroups (not causal) in few rounds finish with a nearly empty last round unless their count fits.
+// Three ring stages allow three workgroups per compute unit instead of four: taken when that wastes fewer places.
+// 64 x 197 tokens, six heads, twelve slots (1536 workgroups: two rounds of 768, one and a half of 1024): dQ 127 -> 119 us.
+inline ShortRows pick_short_rows(long long rows_per_head, long long heads, bool causal, int compute_units) {
+  const long long tiles = (rows_per_head + 63) / 64, n = tiles * heads;
+  const long long three = 3ll * compute_units, four = 4ll * compute_units;
+  const auto places = [n](long long slots) { return (n + slots - 1) / slots * slots; };
+  if (!causal && n > four && places(four) <= 3 * four && places(three) < places(four)) return ShortRows::kThreeStages;
+  if (tiles % 2 == 1 && tiles <= 16 && (tiles + 1) / 2 * heads > compute_units) return ShortRows::kTwoStages;
+  return ShortRows::kNone;
 }
 
 }  // namespace moda
