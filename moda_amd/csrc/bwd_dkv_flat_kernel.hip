@@ -7,11 +7,15 @@
 //   S = Q K^T, dP - delta = dO V^T (accumulators preset with -delta), P = exp2(S c - lse), dS = P (dP - delta),
 //   dV^T += dO^T P, dK^T += Q^T dS.
 // P stays in fp32 until dS is formed (one rounding on the dK path) and nothing travels between waves.  With 26 KB of
-// LDS and no mailbox, three workgroups share a compute unit where dkv_kernel fits one: a launch of a few hundred
-// column tiles of a short sequence (a vision model's 197 tokens) runs in one round of workgroups instead of three,
-// and a launch with many column tiles keeps twelve waves per compute unit busy instead of eight.  A launch of few
-// tiles over a long sequence is bound by its heaviest tile, where the eight waves of dkv_kernel are faster; on the
-// 128-wide tiles this structure spills.  geometry.h: takes_dkv_flat says which launches come here.
+// LDS and no mailbox, three workgroups share a compute unit where dkv_kernel fits one: twelve waves per compute unit
+// instead of eight cover each other's softmax, start and end.  On the 128-wide tiles this structure spills.
+//
+// SPLIT: the query rows of long column tiles are cut into segments of about equal length (geometry.h: dkv_split_plan),
+// which leave fp32 partial sums for dkv_reduce_kernel: without them the launch ends with the heaviest tile.
+//
+// RW (row waves): the four waves share the SAME 32 columns and take 32 rows each of every 128-row query tile; their
+// accumulators meet in LDS, in wave order, before the rows are written.  For short launches with too few 128-column
+// tiles to fill the machine (geometry.h: dkv_flat_row_waves): four times the workgroups, a quarter of the trips.
 #include <type_traits>
 
 #include "geometry.h"
@@ -22,10 +26,12 @@
 namespace moda {
 
 // VARLEN: packed variable-length batch (a workgroup enters its sequence; column tiles past its end leave at once)
-template <typename T, int HD, bool VARLEN>
-__global__ __launch_bounds__(256, 3) void dkv_flat_kernel(const KArgs a_in) {
-  constexpr int NB = 2, BM = 32, MBLK = BM / 16, BN = 4 * 16 * NB, KS = HD / 32, MB = HD / 16, NST = 3, DIST = 2;
-  constexpr int SP = 64;  // floats per statistic and stage (one wave-wide load each)
+template <typename T, int HD, bool VARLEN, bool SPLIT, int RW = 1>
+__global__ __launch_bounds__(256, RW == 1 ? 3 : 2) void dkv_flat_kernel(const KArgs a_in) {
+  static_assert(RW == 1 || (RW == 4 && !VARLEN && !SPLIT), "four row waves: fixed length, no segments");
+  constexpr int NB = 2, WM = 32, BM = WM * RW, MBLK = WM / 16, BN = 4 / RW * 16 * NB, KS = HD / 32, MB = HD / 16;
+  constexpr int NST = RW == 1 ? 3 : 2, DIST = NST - 1;  // ring stages, tiles in flight
+  constexpr int SP = RW == 1 ? 64 : BM;  // floats per statistic and stage (wave-wide loads)
   extern __shared__ __align__(16) unsigned char smem_raw[];
   lds_ptr ring = (lds_ptr)smem_raw;                                      // [NST]: Q tile, dO tile
   MODA_LDS float* stat = (MODA_LDS float*)(ring + NST * 2 * BM * HD);    // [NST][2][SP]: lse, minus delta
@@ -37,15 +43,17 @@ __global__ __launch_bounds__(256, 3) void dkv_flat_kernel(const KArgs a_in) {
   const int ct = blockIdx.x / BHk;
   int b = bh / a_in.Hkv;
   const int hkv = bh % a_in.Hkv;
+  const int seq_index = b;
   SeqArgs<VARLEN> seq(a_in, b);
   const KArgs& a = seq.a;
-  const ColTilePlan plan = col_tile_plan(a_in, a, ct, BN, BM, VARLEN, 1);
-  if (VARLEN && !plan.active) return;  // a tile beyond this sequence of a variable-length batch
+  const ColTilePlan plan = col_tile_plan(a_in, a, ct, BN, BM, VARLEN, SPLIT ? a.dkv_split : 1);
+  if ((VARLEN || SPLIT) && !plan.active) return;  // a tile beyond its sequence, or a segment beyond its tile
+  const int cw = RW == 1 ? wave : 0, rw = RW == 1 ? 0 : wave;  // the wave's column block, its rows of a query tile
   int c[NB];
   bool valid[NB];
 #pragma unroll
   for (int nb = 0; nb < NB; nb++) {
-    c[nb] = plan.c_first + wave * (16 * NB) + 16 * nb + n;
+    c[nb] = plan.c_first + cw * (16 * NB) + 16 * nb + n;
     valid[nb] = c[nb] < a.T;
   }
   i32x4 Kr[NB][KS], Vr[NB][KS];
@@ -83,7 +91,8 @@ __global__ __launch_bounds__(256, 3) void dkv_flat_kernel(const KArgs a_in) {
   const bool st_lse = (wave & 1) == 0;
   const char* stb = st_lse ? (const char*)(a.lse + (int64_t)b * a.Tq * a.Hq + hkv) : (const char*)(a.delta + ((int64_t)b * a.Hq + hkv) * (VARLEN ? a.delta_pitch : a.Tq));
   const uint32_t st_row = st_lse ? (uint32_t)a.Hq * 4u : 4u;
-  const int voff_stat = lane * (int)st_row;
+  const int st_first = SP == 64 ? 0 : (wave >> 1) * 64;  // first row this wave fetches of a tile's statistics
+  const int voff_stat = (st_first + lane) * (int)st_row;
   int ld_st = 0;
   auto issue = [&](int it) {  // trip `it` consumes query tile nqt - 1 - it
     const int f_q0 = (qt0 + nqt - 1 - it) * BM;
@@ -92,11 +101,11 @@ __global__ __launch_bounds__(256, 3) void dkv_flat_kernel(const KArgs a_in) {
     ld.load(Qt + BM * HD, dob, a.sdo.t, f_q0, a.Tq, a.Dv);
     const int rows = imax(imin(a.Tq - f_q0, BM), 0);
     const i32x4 rs = rsrc_words(stb + (int64_t)f_q0 * st_row, rows > 0 ? (uint32_t)(rows - 1) * st_row + 4u : 0u);
-    lds_dma<4>(rs, (uint32_t)(uintptr_t)(stat + ld_st * 2 * SP + (st_lse ? 0 : SP)), voff_stat, 0);
+    lds_dma<4>(rs, (uint32_t)(uintptr_t)(stat + ld_st * 2 * SP + (st_lse ? 0 : SP) + st_first), voff_stat, 0);
     ld_st = (ld_st + 1 == NST) ? 0 : ld_st + 1;
   };
   auto wait_tile = [&](int next) {
-    if (next + 1 < nqt)
+    if (DIST == 2 && next + 1 < nqt)
       Loader::template wait_but<LPT>();
     else
       Loader::wait_all();
@@ -119,9 +128,9 @@ __global__ __launch_bounds__(256, 3) void dkv_flat_kernel(const KArgs a_in) {
 
   auto tile = [&](auto masked, int st, int q0) {
     constexpr bool MASKED = decltype(masked)::value;
-    lds_cptr Qs = ring + st * 2 * BM * HD;
+    lds_cptr Qs = ring + st * 2 * BM * HD + rw * (WM * HD);
     lds_cptr dOs = Qs + BM * HD;
-    MODA_LDS const float* lse_s = stat + st * 2 * SP;
+    MODA_LDS const float* lse_s = stat + st * 2 * SP + rw * WM;
     MODA_LDS const float* del_s = lse_s + SP;
     f32x4 s[MBLK][NB], dp[MBLK][NB];
 #pragma unroll
@@ -163,7 +172,7 @@ __global__ __launch_bounds__(256, 3) void dkv_flat_kernel(const KArgs a_in) {
         for (int j = 0; j < 4; j++) {
           float p = fast_exp2(__builtin_fmaf(s[m][nb][j], sc, -lv[j]));
           if (MASKED) {
-            const int qr = q0 + 16 * m + slot_base(q4) + j;
+            const int qr = q0 + rw * WM + 16 * m + slot_base(q4) + j;
             p = (qr >= qlo[nb] && qr < qhi[nb]) ? p : 0.f;
           }
           s[m][nb][j] = p;
@@ -182,7 +191,7 @@ __global__ __launch_bounds__(256, 3) void dkv_flat_kernel(const KArgs a_in) {
     pk.run(oa, Qs, DS, dk);
   };
 
-  // query tiles whose rows all see all 128 columns need no masking: for causal keys those at or past the last
+  // query tiles whose rows all see all columns of the workgroup need no masking: for causal keys those at or past the last
   // column's first visible row (padding rows past Tq carry zero Q, dO, lse, delta and contribute nothing)
   const int first_free_qt = a.causal ? ((imin(a.T, plan.c_first + BN) - 1) * a.Gf + BM - 1) / BM - qt0 : 0;
   int it = 0, c_st = 0;
@@ -201,6 +210,55 @@ __global__ __launch_bounds__(256, 3) void dkv_flat_kernel(const KArgs a_in) {
     __syncthreads();
   }
 
+  if constexpr (RW > 1) {
+    // [which][d][nb] blocks of all waves through the ring (which every wave has done reading): wave w adds up and writes
+    // a quarter of them
+    static_assert(NST * 2 * BM * HD * 2 >= 4 * 2 * MB * NB * 1024 && 2 * MB % RW == 0, "the exchange fits the ring");
+    MODA_LDS f32x4* ex = (MODA_LDS f32x4*)ring;
+#pragma unroll
+    for (int d = 0; d < MB; d++)
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) {
+        ex[((rw * 2 * MB + d) * NB + nb) * 64 + lane] = dk[d][nb];
+        ex[((rw * 2 * MB + MB + d) * NB + nb) * 64 + lane] = dv[d][nb];
+      }
+    __syncthreads();
+    const bool is_v = rw >= RW / 2;
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) {
+      uint16_t* outp = is_v ? a.dv + b * a.sdv.b + hkv * a.sdv.h + (int64_t)c[nb] * a.sdv.t
+                            : a.dk + b * a.sdk.b + hkv * a.sdk.h + (int64_t)c[nb] * a.sdk.t;
+#pragma unroll
+      for (int i = 0; i < 2 * MB / RW; i++) {
+        const int blk = rw * (2 * MB / RW) + i, d = blk % MB;
+        f32x4 sum = ex[(blk * NB + nb) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < RW; w++) sum += ex[((w * 2 * MB + blk) * NB + nb) * 64 + lane];
+        sum *= is_v ? 1.f : a.scale;
+        i32x2 w;
+        w[0] = pack2<T>(sum[0], sum[1]);
+        w[1] = pack2<T>(sum[2], sum[3]);
+        if (valid[nb] && 16 * d + 4 * q4 < (is_v ? a.Dv : a.D)) *reinterpret_cast<i32x2*>(outp + 16 * d + 4 * q4) = w;
+      }
+    }
+    return;
+  }
+  if (SPLIT && plan.nsegs > 1) {  // a row segment: fp32 partial sums, added up by dkv_reduce_kernel
+    const int64_t pitch = part_rows(a), plane = (int64_t)(VARLEN ? 1 : a.B) * a.Hkv * pitch * HD;
+    const int first = VARLEN ? a_in.cu[seq_index] : 0;
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++)
+      if (valid[nb]) {
+        float* kp = a.dkv_part + plan.seg * plane + (((int64_t)b * a.Hkv + hkv) * pitch + first + c[nb]) * HD + 4 * q4;
+        float* vp = kp + a.dkv_split * plane;
+#pragma unroll
+        for (int d = 0; d < MB; d++) {
+          *reinterpret_cast<f32x4*>(kp + 16 * d) = dk[d][nb] * a.scale;
+          *reinterpret_cast<f32x4*>(vp + 16 * d) = dv[d][nb];
+        }
+      }
+    return;
+  }
 #pragma unroll
   for (int nb = 0; nb < NB; nb++)
     if (valid[nb]) {
@@ -219,23 +277,31 @@ __global__ __launch_bounds__(256, 3) void dkv_flat_kernel(const KArgs a_in) {
     }
 }
 
-template <typename T, int HD, bool VARLEN>
+template <typename T, int HD, bool VARLEN, bool SPLIT, int RW = 1>
 hipError_t launch_dkv_flat_t(const KArgs& a, hipStream_t stream) {
-  constexpr size_t smem = (size_t)3 * 2 * 32 * HD * sizeof(uint16_t) + 3 * 2 * 64 * sizeof(float);
+  constexpr size_t smem = (RW == 1 ? (size_t)3 * (2 * 32 * HD * sizeof(uint16_t) + 2 * 64 * sizeof(float))
+                                   : (size_t)2 * (2 * 32 * RW * HD * sizeof(uint16_t) + 2 * 32 * RW * sizeof(float)));
   static LdsAttrState attr;
-  const hipError_t ea = allow_dynamic_lds(attr, reinterpret_cast<const void*>(&dkv_flat_kernel<T, HD, VARLEN>), smem);
+  const hipError_t ea = allow_dynamic_lds(attr, reinterpret_cast<const void*>(&dkv_flat_kernel<T, HD, VARLEN, SPLIT, RW>), smem);
   if (ea != hipSuccess) return ea;
-  const int64_t nblk = dkv_flat_blocks(a);
+  const int64_t nblk = dkv_flat_blocks(a, 128 / RW) * (SPLIT ? a.dkv_split : 1);
   if (nblk == 0) return hipSuccess;
   if (nblk >= (1ll << 31)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((dkv_flat_kernel<T, HD, VARLEN>), dim3((unsigned)nblk), dim3(256), smem, stream, a);
+  hipLaunchKernelGGL((dkv_flat_kernel<T, HD, VARLEN, SPLIT, RW>), dim3((unsigned)nblk), dim3(256), smem, stream, a);
   return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_dkv_flat_as(const KArgs& a, hipStream_t stream) {
+  const bool split = a.dkv_split > 1;
+  if (a.cu) return split ? launch_dkv_flat_t<T, 64, true, true>(a, stream) : launch_dkv_flat_t<T, 64, true, false>(a, stream);
+  if (dkv_flat_row_waves(a)) return launch_dkv_flat_t<T, 64, false, false, 4>(a, stream);
+  return split ? launch_dkv_flat_t<T, 64, false, true>(a, stream) : launch_dkv_flat_t<T, 64, false, false>(a, stream);
 }
 
 // dtype: 0 bf16, 1 fp16; 64-wide tiles only (the caller asks takes_dkv_flat first)
 hipError_t launch_dkv_flat(const KArgs& a, int dtype, hipStream_t stream) {
-  if (a.cu) return dtype == 0 ? launch_dkv_flat_t<BF16, 64, true>(a, stream) : launch_dkv_flat_t<FP16, 64, true>(a, stream);
-  return dtype == 0 ? launch_dkv_flat_t<BF16, 64, false>(a, stream) : launch_dkv_flat_t<FP16, 64, false>(a, stream);
+  return dtype == 0 ? launch_dkv_flat_as<BF16>(a, stream) : launch_dkv_flat_as<FP16>(a, stream);
 }
 
 }  // namespace moda

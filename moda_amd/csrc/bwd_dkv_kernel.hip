@@ -30,11 +30,10 @@
 
 namespace moda {
 
-// SPLIT: the launch cuts the query rows of every sequence column tile into a.dkv_split segments (a variant of
-// its own: the extra index arithmetic costs the long-sequence instantiation scalar registers it cannot spare)
+// SPLIT: the launch cuts the query rows of long sequence column tiles into segments (a variant of its own: the extra
+// index arithmetic costs the long-sequence instantiation scalar registers it cannot spare)
 template <typename T, int HD, bool VARLEN, bool SPLIT = false>
 __global__ __launch_bounds__(512) void dkv_kernel(const KArgs a_in) {
-  static_assert(!(VARLEN && SPLIT), "packed batches are not split");
   // 16-column halves per wave, query rows per streamed tile: halved for the 256-wide tiles, whose operands and
   // accumulators would not fit the register file (and whose three-stage ring would not fit the LDS) otherwise
   constexpr int NB = HD > 128 ? 1 : 2, BM = HD > 128 ? 32 : 64, MBLK = BM / 16;
@@ -58,13 +57,14 @@ __global__ __launch_bounds__(512) void dkv_kernel(const KArgs a_in) {
   const int ct = blockIdx.x / BHk;
   int b = bh / a_in.Hkv;
   const int hkv = bh % a_in.Hkv;
+  const int seq_index = b;
   SeqArgs<VARLEN> seq(a_in, b);
   const KArgs& a = seq.a;
   // sequence tiles come `nseg` workgroups each (row segments of one column tile are neighbours in the grid, the
   // heaviest column tile first), then the depth tiles
   const int nseg = SPLIT ? a.dkv_split : 1;
   const ColTilePlan plan = col_tile_plan(a_in, a, ct, BN, BM, VARLEN, nseg);
-  if (VARLEN && !plan.active) return;  // a tile beyond this sequence of a variable-length batch
+  if ((VARLEN || SPLIT) && !plan.active) return;  // a tile beyond its sequence, or a segment beyond its tile
   const bool dep = plan.dep;
   const int ncols = plan.ncols, seg = plan.seg, c_first = plan.c_first;
   int c[NB];
@@ -359,15 +359,16 @@ __global__ __launch_bounds__(512) void dkv_kernel(const KArgs a_in) {
   else
     role_loop(std::true_type{});
 
-  if (SPLIT && !dep) {
+  if (SPLIT && !dep && plan.nsegs > 1) {
     // a row segment: fp32 partial sums, added up by dkv_reduce_kernel
-    const int64_t plane = (int64_t)a.B * a.Hkv * a.T * HD;
+    const int64_t pitch = part_rows(a), plane = (int64_t)(VARLEN ? 1 : a.B) * a.Hkv * pitch * HD;
+    const int first = VARLEN ? a_in.cu[seq_index] : 0;
     const float mul = role_b ? a.scale : 1.f;
 #pragma unroll
     for (int nb = 0; nb < NB; nb++)
       if (valid[nb]) {
         float* outp = a.dkv_part + ((int64_t)(role_b ? 0 : 1) * nseg + seg) * plane +
-                      (((int64_t)b * a.Hkv + hkv) * a.T + c[nb]) * HD;
+                      (((int64_t)b * a.Hkv + hkv) * pitch + first + c[nb]) * HD;
 #pragma unroll
         for (int d = 0; d < MB; d++) *reinterpret_cast<f32x4*>(outp + 16 * d + 4 * q4) = acc[d][nb] * mul;
       }
@@ -898,26 +899,32 @@ __global__ __launch_bounds__(256) void zero_unfilled_slots_kernel(const KArgs a,
 }
 
 // Adds the fp32 partial sums of the row segments (in segment order: the result does not depend on which
-// workgroup finished first) and writes dk, dv in the tensor type.  One thread per 8 head-dim elements.
-template <typename T, int HD>
-__global__ __launch_bounds__(256) void dkv_reduce_kernel(const KArgs a) {
-  constexpr int TPR = HD / 8;
-  const int64_t rows = (int64_t)a.B * a.Hkv * a.T;
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t row = gid / TPR;
-  if (row >= rows) return;
-  const int sub = (int)(gid % TPR);
-  const int c = (int)(row % a.T);
-  const int bh = (int)(row / a.T);
-  const int b = bh / a.Hkv, hkv = bh % a.Hkv;
-  const int64_t plane = rows * HD;
+// workgroup finished first) and writes dk, dv in the tensor type.  One thread per 8 head-dim elements.  BN, BM: the
+// column and query tiles of the launch that left them; its tiles of one segment have written their rows themselves.
+template <typename T, int HD, bool VARLEN>
+__global__ __launch_bounds__(256) void dkv_reduce_kernel(const KArgs a_in, int BN, int BM) {
+  constexpr int TPR = HD / 8, RPB = 256 / TPR;
+  const int BHk = a_in.B * a_in.Hkv;
+  const int bh = blockIdx.x % BHk;
+  int b = bh / a_in.Hkv;
+  const int hkv = bh % a_in.Hkv, sub = threadIdx.x % TPR;
+  const int first = VARLEN ? a_in.cu[b] : 0;
+  SeqArgs<VARLEN> seq(a_in, b);
+  const KArgs& a = seq.a;
+  const int c = (int)(blockIdx.x / BHk) * RPB + threadIdx.x / TPR;
+  if (c >= a.T) return;
+  const int c_first = c / BN * BN, row0 = a.causal ? c_first * a.Gf : 0;
+  const int nsegs = tile_segments(a, (a.Tq + BM - 1) / BM - row0 / BM, a.dkv_split);
+  if (nsegs == 1) return;
+  const int64_t pitch = part_rows(a), plane = (int64_t)(VARLEN ? 1 : a.B) * a.Hkv * pitch * HD;
+  const int64_t row = ((int64_t)b * a.Hkv + hkv) * pitch + first + c;
 #pragma unroll
   for (int which = 0; which < 2; which++) {  // 0: dk, 1: dv
     const float* src = a.dkv_part + (int64_t)which * a.dkv_split * plane + row * HD + 8 * sub;
     float s[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) s[i] = 0.f;
-    for (int sg = 0; sg < a.dkv_split; sg++) {
+    for (int sg = 0; sg < nsegs; sg++) {
       const f32x4 lo = *reinterpret_cast<const f32x4*>(src + sg * plane);
       const f32x4 hi = *reinterpret_cast<const f32x4*>(src + sg * plane + 4);
 #pragma unroll
@@ -941,41 +948,40 @@ template <typename T, int HD>
 hipError_t launch_dkv_t(const KArgs& a, hipStream_t stream) {
   constexpr int NB = HD > 128 ? 1 : 2, BM = HD > 128 ? 32 : 64, BN = 64 * NB;  // as in dkv_kernel
   constexpr size_t smem = 3 * 2 * BM * HD * sizeof(uint16_t) + 2 * 4 * (BM / 32) * NB * 64 * 16 + 3 * 2 * 64 * sizeof(float);
-  static LdsAttrState attr;
-  static LdsAttrState attr_packed;
-  static LdsAttrState attr_split;
-  const int nseg = a.cu ? 1 : a.dkv_split;
-  const hipError_t ea =
-      a.cu       ? allow_dynamic_lds(attr_packed, reinterpret_cast<const void*>(&dkv_kernel<T, HD, true>), smem)
-      : nseg > 1 ? allow_dynamic_lds(attr_split, reinterpret_cast<const void*>(&dkv_kernel<T, HD, false, true>), smem)
-                 : allow_dynamic_lds(attr, reinterpret_cast<const void*>(&dkv_kernel<T, HD, false>), smem);
-  if (ea != hipSuccess) return ea;
-  // depth columns: vector kernel, except in chunk-visible mode where a column has up to G*Cb visible rows
-  const bool in_dq = depth_grads_in_dq(a, HD);  // the dQ launch has formed the depth slots' dK and dV already
-  const bool depth_by_columns = a.L > 0 && !a.chunk && !in_dq;
   const int64_t n_seq_tiles = a.has_seq ? (a.T + BN - 1) / BN : 0;
-  const bool depth_by_chunks = moda::depth_by_chunks(a, HD);
+  const int nseg = a.dkv_split;
+  const bool flat = takes_dkv_flat(a, HD);
   const int64_t nblk = col_kernel_blocks(a, HD, BN, nseg);
   if (nblk >= (1ll << 31)) return hipErrorInvalidValue;
-  if (nblk > 0 && takes_dkv_flat(a, HD, nseg)) {
+  if (nblk > 0 && flat) {
     const hipError_t e = launch_dkv_flat(a, std::is_same<T, FP16>::value ? 1 : 0, stream);
     if (e != hipSuccess) return e;
   } else if (nblk > 0) {
+    const auto go = [&](auto kernel, LdsAttrState& attr) {
+      const hipError_t e = allow_dynamic_lds(attr, reinterpret_cast<const void*>(kernel), smem);
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL(kernel, dim3((unsigned)nblk), dim3(512), smem, stream, a);
+      return hipGetLastError();
+    };
+    static LdsAttrState attr[4];
+    const hipError_t e = a.cu ? (nseg > 1 ? go(&dkv_kernel<T, HD, true, HD <= 128>, attr[0]) : go(&dkv_kernel<T, HD, true>, attr[1]))
+                              : (nseg > 1 ? go(&dkv_kernel<T, HD, false, true>, attr[2]) : go(&dkv_kernel<T, HD, false>, attr[3]));
+    if (e != hipSuccess) return e;
+  }
+  if (nseg > 1 && n_seq_tiles > 0) {
+    const int rpb = 256 / (HD / 8), bm = flat ? 32 : BM;
+    const dim3 grid((unsigned)(((int64_t)a.T + rpb - 1) / rpb * a.B * a.Hkv));
     if (a.cu)
-      hipLaunchKernelGGL((dkv_kernel<T, HD, true>), dim3((unsigned)nblk), dim3(512), smem, stream, a);
-    else if (nseg > 1)
-      hipLaunchKernelGGL((dkv_kernel<T, HD, false, true>), dim3((unsigned)nblk), dim3(512), smem, stream, a);
+      hipLaunchKernelGGL((dkv_reduce_kernel<T, HD, true>), grid, dim3(256), 0, stream, a, BN, bm);
     else
-      hipLaunchKernelGGL((dkv_kernel<T, HD, false>), dim3((unsigned)nblk), dim3(512), smem, stream, a);
+      hipLaunchKernelGGL((dkv_reduce_kernel<T, HD, false>), grid, dim3(256), 0, stream, a, BN, bm);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (nseg > 1 && n_seq_tiles > 0) {
-      const int64_t nthreads = (int64_t)a.B * a.Hkv * a.T * (HD / 8);
-      hipLaunchKernelGGL((dkv_reduce_kernel<T, HD>), dim3((unsigned)((nthreads + 255) / 256)), dim3(256), 0, stream, a);
-      const hipError_t er = hipGetLastError();
-      if (er != hipSuccess) return er;
-    }
   }
+  // depth columns: vector kernel, except in chunk-visible mode where a column has up to G*Cb visible rows
+  const bool in_dq = depth_grads_in_dq(a, HD);  // the dQ launch has formed the depth slots' dK and dV already
+  const bool depth_by_columns = a.L > 0 && !a.chunk && !in_dq;
+  const bool depth_by_chunks = moda::depth_by_chunks(a, HD);
   if (a.L > 0 && (a.chunk || in_dq) && a.Lv != a.L && !a.keep_slots && (int64_t)a.B * a.T > 0) {
     // packed batch: one row axis of all sequences (its length is the row-sum pitch / G), else B x T * L rows
     const int64_t rows = a.cu ? (int64_t)(a.delta_pitch / a.Gf) * a.L : (int64_t)a.T * a.L;

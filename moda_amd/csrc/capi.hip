@@ -154,18 +154,10 @@ size_t delta_bytes_exact(const KArgs& a) {
 }
 size_t delta_bytes(const KArgs& a) { return (delta_bytes_exact(a) + 255) / 256 * 256; }
 
-// Row segments per column tile of the sequence dK/dV kernel (see KArgs::dkv_split).  A launch whose column
-// tiles cannot give every compute unit two workgroups is cut further along the query rows, as long as a
-// segment keeps at least 16 query tiles.  Sized for the 256 compute units of a whole MI355X whatever the
-// partition mode, so that the workspace size depends on the descriptor alone.
-int desired_dkv_split(const moda_hip_desc* d, const KArgs& a) {
-  if (!use_mfma(d) || a.cu || !a.has_seq || a.T == 0) return 1;
-  const int cols = widest_dim(d) > 128 ? 64 : 128, rows = widest_dim(d) > 128 ? 32 : 64;  // the kernel's column tile and query tile
-  const int64_t tiles = (int64_t)((a.T + cols - 1) / cols) * a.B * a.Hkv;
-  const int64_t query_tiles = (a.Tq + rows - 1) / rows;
-  int s = 1;
-  while (tiles * s < 512 && s < 8 && query_tiles / (2 * s) >= 16) s *= 2;
-  return s;
+// Row segments of the sequence dK/dV launch (geometry.h: dkv_split_plan).
+moda::DkvSplit desired_dkv_split(const moda_hip_desc* d, const KArgs& a) {
+  if (!use_mfma(d)) return {1, 0};
+  return moda::dkv_split_plan(a, tile_width(d));
 }
 
 // P and dS of the (query row, depth slot) pairs, handed from the dQ kernel to the depth-gradient kernel (see
@@ -177,7 +169,7 @@ size_t depth_handover_bytes(const moda_hip_desc* d, const KArgs& a) {
 }
 
 size_t dkv_part_bytes(const moda_hip_desc* d, const KArgs& a, int split) {
-  return split > 1 ? (size_t)2 * split * a.B * a.Hkv * a.T * tile_width(d) * sizeof(float) : 0;
+  return split > 1 ? (size_t)2 * split * (a.cu ? 1 : a.B) * a.Hkv * moda::part_rows(a) * tile_width(d) * sizeof(float) : 0;
 }
 
 // The current device must be a gfx950; reports its compute-unit count.  One entry per device is cached.
@@ -323,7 +315,7 @@ int moda_hip_fwd(const moda_hip_desc* d, const void* q, const void* k, const voi
 size_t moda_hip_bwd_workspace_bytes(const moda_hip_desc* d) {
   KArgs a;
   if (fill_geometry(d, a)) return 0;
-  const size_t part = dkv_part_bytes(d, a, desired_dkv_split(d, a));
+  const size_t part = dkv_part_bytes(d, a, desired_dkv_split(d, a).nseg);
   const size_t hand = depth_handover_bytes(d, a);
   // the row sums, then (each optional) the handed-over depth scores and the partial sums of the row split
   return (part || hand) ? delta_bytes(a) + hand + part : delta_bytes_exact(a);
@@ -420,10 +412,12 @@ int moda_hip_bwd_stages(const moda_hip_desc* d, const void* q, const void* k, co
     // between the row sums and the partial sums
     size_t hand = depth_handover_bytes(d, a);
     if (delta_bytes(a) + hand > workspace_bytes) hand = 0;
-    int split = desired_dkv_split(d, a);
-    while (split > 1 && delta_bytes(a) + hand + dkv_part_bytes(d, a, split) > workspace_bytes) split /= 2;
-    if ((uintptr_t)workspace % 16 != 0) split = 1;  // the partial sums are written and read 16 bytes at a time
-    a.dkv_split = split;
+    moda::DkvSplit split = desired_dkv_split(d, a);
+    const int most = split.nseg;
+    while (split.nseg > 1 && delta_bytes(a) + hand + dkv_part_bytes(d, a, split.nseg) > workspace_bytes) split.nseg /= 2;
+    if ((uintptr_t)workspace % 16 != 0) split.nseg = 1;  // the partial sums are written and read 16 bytes at a time
+    a.dkv_split = split.nseg;
+    a.dkv_seg_tiles = (split.seg_tiles * most + split.nseg - 1) / split.nseg;  // fewer segments: longer ones
     a.dkv_part = (float*)((char*)workspace + delta_bytes(a) + hand);
     if (hand) {
       a.depth_p = (uint16_t*)((char*)workspace + delta_bytes(a));

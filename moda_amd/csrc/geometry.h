@@ -135,13 +135,18 @@ MODA_HD void q_interval(const KArgs& a, bool dep, int col, int& lo, int& hi) {
 // What column-tile workgroup `ct` of a (batch, kv head) does.  `grid`: the launch's argument block (T of the
 // longest sequence), `a`: the one rebased on the workgroup's sequence; nseg: row segments per sequence tile.
 struct ColTilePlan {
-  bool active;  // false: a tile beyond this sequence of a variable-length batch
+  bool active;  // false: a tile beyond this sequence of a variable-length batch, or a segment a tile does without
   bool dep;     // depth columns (else sequence keys)
   int ncols;    // columns of the (batch, head): T or T * L
-  int seg;      // row segment of a split sequence tile
+  int seg;      // row segment of a split sequence tile ...
+  int nsegs;    // ... out of this many (1: the workgroup writes the gradients itself)
   int c_first;  // first column
   int qt0, nqt; // query tiles qt0 .. qt0 + nqt - 1 (BM rows each), streamed from the last one down
 };
+// row segments of a sequence column tile that sees `nqt` query tiles
+MODA_HD int tile_segments(const KArgs& grid, int nqt, int nseg) {
+  return grid.dkv_seg_tiles > 0 ? imax(1, imin(nseg, (nqt + grid.dkv_seg_tiles - 1) / grid.dkv_seg_tiles)) : nseg;
+}
 MODA_HD ColTilePlan col_tile_plan(const KArgs& grid, const KArgs& a, int ct, int BN, int BM, bool varlen, int nseg) {
   ColTilePlan p;
   // the grid holds the sequence tiles of the longest sequence (nseg workgroups each: the row segments of one
@@ -161,6 +166,7 @@ MODA_HD ColTilePlan col_tile_plan(const KArgs& grid, const KArgs& a, int ct, int
   p.c_first = tile * BN;
   if (varlen && p.c_first >= p.ncols) p.active = false;
   p.qt0 = p.nqt = 0;
+  p.nsegs = 1;
   if (!p.active) return p;
   int wg_lo, wg_hi, tmp;
   q_interval(a, p.dep, p.c_first, wg_lo, tmp);
@@ -168,7 +174,9 @@ MODA_HD ColTilePlan col_tile_plan(const KArgs& grid, const KArgs& a, int ct, int
   p.qt0 = wg_lo / BM;
   p.nqt = (wg_hi + BM - 1) / BM - p.qt0;
   if (nseg > 1 && !p.dep) {  // this workgroup's share of the column tile's query tiles
-    const int lo = (int)((int64_t)p.nqt * p.seg / nseg), hi = (int)((int64_t)p.nqt * (p.seg + 1) / nseg);
+    p.nsegs = tile_segments(grid, p.nqt, nseg);
+    if (p.seg >= p.nsegs) p.active = false;
+    const int lo = (int)((int64_t)p.nqt * p.seg / p.nsegs), hi = (int)((int64_t)p.nqt * (p.seg + 1) / p.nsegs);
     p.qt0 += lo;
     p.nqt = hi - lo;
   }
@@ -192,17 +200,52 @@ inline int64_t col_kernel_blocks(const KArgs& a, int HD, int BN, int nseg) {
   const int64_t n_dep_tiles = (a.L > 0 && a.chunk && !depth_by_chunks(a, HD)) ? ((int64_t)a.T * a.Lv + BN - 1) / BN : 0;
   return (n_seq_tiles * nseg + n_dep_tiles) * a.B * a.Hkv;
 }
-// Sequence dK/dV on the 64-wide tiles: dkv_flat_kernel (three workgroups per compute unit, where dkv_kernel fits
-// one) takes a launch of sequence-key column tiles -- kv head = query head, no row segments -- when the
-// tiles see few query rows each (the launch waits for memory, not for the matrix pipe) or when there are enough of
-// them to fill every compute unit's three places (measured: 18-35 % faster from 768 tiles up, at any sequence
-// length; 16-25 % slower at 512 tiles of 16 K rows, where the heaviest tile's trips set the time).
-constexpr int kDkvFlatMaxRows = 512;
-inline int64_t dkv_flat_blocks(const KArgs& a) { return a.has_seq ? (int64_t)((a.T + 127) / 128) * a.B * a.Hkv : 0; }
-inline bool takes_dkv_flat(const KArgs& a, int HD, int nseg) {
-  return HD == 64 && a.has_seq && a.hdiv == 1 && nseg == 1 && a.compute_units > 0 &&
-         col_kernel_blocks(a, HD, 128, 1) == dkv_flat_blocks(a) &&
-         (a.Tq <= kDkvFlatMaxRows || dkv_flat_blocks(a) >= 3ll * a.compute_units);
+// Sequence dK/dV on the 64-wide tiles: dkv_flat_kernel (three workgroups per compute unit, where dkv_kernel fits one)
+// takes every launch of sequence-key column tiles whose kv head is the query head.
+inline int64_t dkv_flat_blocks(const KArgs& a, int BN = 128) { return a.has_seq ? (int64_t)((a.T + BN - 1) / BN) * a.B * a.Hkv : 0; }
+inline bool takes_dkv_flat(const KArgs& a, int HD) {
+  return HD == 64 && a.has_seq && a.hdiv == 1 && col_kernel_blocks(a, HD, 128, 1) == dkv_flat_blocks(a);
+}
+// ... with the four waves on the SAME 32 columns and a quarter of every 128-row query tile each, for short launches whose
+// 128-column tiles would leave compute units idle (64 x 197 tokens of four query rows: 128 tiles; the twelve layers of a
+// depth stream 925 -> 810 us).  Longer ones are cut into segments, which re-read the query rows less.
+constexpr int kDkvRowWavesMaxRows = 1024;
+inline bool dkv_flat_row_waves(const KArgs& a) {
+  return !a.cu && a.Tq <= kDkvRowWavesMaxRows && dkv_flat_blocks(a) <= 256;
+}
+
+// Row segments of the sequence dK/dV launch (KArgs::dkv_split, dkv_seg_tiles): a launch ends with its longest workgroup,
+// and one with few column tiles leaves compute units idle.  Sized for 256 compute units whatever the partition mode, so
+// that the workspace size depends on the problem alone.
+// Launches with two column tiles per compute unit (dkv_flat_kernel: per workgroup place) are not cut: dispatched heaviest
+// first they balance by themselves, and the partial sums only cost (16 K tokens, sixteen query heads on four: 4.07 -> 4.97
+// ms; head dim 64, 64 heads: 10.4 -> 10.9 ms).  Below that:
+// dkv_kernel, fixed length: the same power of two for every tile, segments of the heaviest of at least 16 trips (a trip:
+// one query tile of one query head).  3057 tokens, 32 query heads on four: 538 -> 430 us when the heads count as trips.
+// Packed batches and dkv_flat_kernel: segments of equal length, three quarters of a place's share of all trips (0.35 to 1
+// measure within 4 %).  A packed batch counts as one of equal, longest sequences.  Eight sequences of 200 - 3000
+// tokens, head dim 64: 974 -> 705 us; five of 168 - 2600, head dim 128: 651 -> 242 us; 6000 tokens, four heads of
+// four, head dim 64: 497 -> 430 us.
+struct DkvSplit {
+  int nseg, seg_tiles;
+};
+inline DkvSplit dkv_split_plan(const KArgs& a, int HD) {
+  const bool flat = takes_dkv_flat(a, HD);
+  if (!a.has_seq || a.T == 0 || (flat && dkv_flat_row_waves(a))) return {1, 0};
+  const int BN = HD > 128 ? 64 : 128, BM = flat || HD > 128 ? 32 : 64;
+  const int64_t tiles = (int64_t)((a.T + BN - 1) / BN) * a.Hkv * (a.cu ? imax(1, part_rows(a) / a.T) : a.B);
+  const int64_t nqt = (a.Tq + BM - 1) / BM;
+  if (tiles >= (flat ? 768 : 512)) return {1, 0};
+  if (!flat && !a.cu) {
+    int s = 1;
+    while (tiles * s < 512 && s < 8 && nqt * a.hdiv / (2 * s) >= 16 && nqt >= 4 * s) s *= 2;
+    return {s, 0};
+  }
+  const int64_t trips = tiles * (a.causal ? (nqt + 1) / 2 : nqt) * a.hdiv / (flat ? 768 : 256);  // of one place
+  const int64_t least = flat ? 24 : 40;  // trips that pay for a workgroup's start, end and partial sums
+  const int64_t seg = imax((int)((trips * 3 / 4 > least ? trips * 3 / 4 : least) / a.hdiv), (int)((nqt + 15) / 16));
+  const int64_t n = seg > 0 ? (nqt + seg - 1) / seg : nqt;
+  return n > 1 ? DkvSplit{(int)n, (int)imax(1, (int)seg)} : DkvSplit{1, 0};
 }
 inline int64_t delta_kernel_blocks(const KArgs& a, int rows_per_block) {
   return (int64_t)((a.Tq + rows_per_block - 1) / rows_per_block) * a.B * a.Hq;

@@ -35,10 +35,12 @@ struct KArgs {
   // times Lv; inside it slot-major, the token's Gf rows side by side), and the depth-gradient kernel forms dkd, dvd
   // from them and the rows of q, do without reading kd, vd again.  Null: no room in the workspace, or another route.
   uint16_t *depth_p, *depth_ds;
-  // Sequence dK/dV of launches too small to fill the device: the query rows of every column tile are cut into
-  // `dkv_split` segments, one workgroup each, which leave fp32 partial sums in `dkv_part`
-  // ([2 (dk, dv)][dkv_split][B][Hkv][T][D]); a second kernel adds them in segment order.  1 = no split.
-  int dkv_split;
+  // Sequence dK/dV of launches that few or unequal column tiles would leave unbalanced: the query rows of a column tile
+  // are cut into at most `dkv_split` segments of about `dkv_seg_tiles` query tiles (0: always `dkv_split` segments), one
+  // workgroup each, which leave fp32 partial sums in `dkv_part` ([2 (dk, dv)][dkv_split][B][Hkv][part_rows(a)][tile
+  // width]); a second kernel adds them in segment order.  A column tile of one segment writes its gradients itself.
+  // 1 = no split.
+  int dkv_split, dkv_seg_tiles;
   float* dkv_part;
   int nqt;   // query tiles per (batch, query head)
   float scale;
@@ -48,6 +50,9 @@ struct KArgs {
   const int32_t* cu;
   int delta_pitch;  // query rows per head in `delta`: Tq, or the packed total
 };
+
+// Key rows per head and batch entry of `dkv_part` (a packed batch: all sequences on one axis, one batch entry).
+__host__ __device__ __forceinline__ int part_rows(const KArgs& a) { return a.cu ? a.delta_pitch / a.Gf : a.T; }
 
 // Variable-length batches: rebases every tensor on the first row of sequence `b` and shrinks T / Tq to the
 // sequence's length, so that the code after it addresses the sequence as batch 0 of a fixed-length problem.

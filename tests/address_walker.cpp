@@ -439,18 +439,18 @@ void walk_dkv(const KArgs& a_in) {
   const uint32_t lds_bytes = 3 * 2 * BM * HD * 2 + 2 * 4 * (BM / 32) * NB * 64 * 16 + 3 * 2 * 64 * 4;
   const uint32_t stat_byte = NST * 2 * BM * HD * 2 + 2 * 4 * NP * 64 * 16;
   const bool varlen = a_in.cu != nullptr;
-  const int nseg = varlen ? 1 : a_in.dkv_split;
+  const int nseg = a_in.dkv_split;
   const int BHk = a_in.B * a_in.Hkv;
   const int64_t nblk = col_kernel_blocks(a_in, HD, BN, nseg);
   typedef AsyncTileLoader<HD, BM, 512> Loader;
   for (int64_t block = 0; block < nblk; block++) {
     const int bh = (int)(block % BHk), ct = (int)(block / BHk);
     int b = bh / a_in.Hkv;
-    const int hkv = bh % a_in.Hkv;
+    const int hkv = bh % a_in.Hkv, first = varlen ? a_in.cu[b] : 0;
     const KArgs a = seq_args(a_in, b);
     const ColTilePlan plan = col_tile_plan(a_in, a, ct, BN, BM, varlen, nseg);
     if (!plan.active) {
-      if (!varlen) fail("dkv_kernel: inactive column tile in a fixed-length launch");
+      if (!varlen && nseg == 1) fail("dkv_kernel: inactive column tile in a fixed-length launch");
       continue;
     }
     const bool dep = plan.dep;
@@ -470,10 +470,10 @@ void walk_dkv(const KArgs& a_in) {
           if (valid && 32 * ks + 8 * q4 < (role_b ? a.Dv : a.D)) check_access(sname, src + crow * st + 32 * ks + 8 * q4, 16, false);
         if (!valid) continue;
         ctx("dkv_kernel", (int)block, wave, lane, "gradient rows");
-        if (nseg > 1 && !dep) {  // a row segment: fp32 partial sums, all HD columns of the tile width
-          const int64_t plane = (int64_t)a.B * a.Hkv * a.T * HD;
+        if (plan.nsegs > 1 && !dep) {  // a row segment: fp32 partial sums, all HD columns of the tile width
+          const int64_t pitch = part_rows(a), plane = (int64_t)(varlen ? 1 : a.B) * a.Hkv * pitch * HD;
           float* pp = a.dkv_part + ((int64_t)(role_b ? 0 : 1) * nseg + plan.seg) * plane +
-                      (((int64_t)b * a.Hkv + hkv) * a.T + c) * HD;
+                      (((int64_t)b * a.Hkv + hkv) * pitch + first + c) * HD;
           for (int d = 0; d < MB; d++) check_access("part", pp + 16 * d + 4 * q4, 16, true);
           continue;
         }
@@ -524,31 +524,34 @@ void walk_dkv(const KArgs& a_in) {
   }
 }
 
-// dkv_flat_kernel: four waves, a wave's 32 columns with K and V in registers, query tiles of 32 rows
-template <int HD>
+// dkv_flat_kernel: four waves, a wave's 32 columns with K and V in registers, query tiles of 32 rows; or (RW = 4) the
+// waves on the same 32 columns, 32 rows each of a query tile of 128
+template <int HD, int RW>
 void walk_dkv_flat(const KArgs& a_in) {
-  constexpr int NB = 2, BM = 32, BN = 4 * 16 * NB, KS = HD / 32, MB = HD / 16, NST = 3, SP = 64;
-  const uint32_t lds_bytes = 3 * 2 * 32 * HD * 2 + 3 * 2 * 64 * 4;
+  constexpr int NB = 2, BM = 32 * RW, BN = 4 / RW * 16 * NB, KS = HD / 32, MB = HD / 16, NST = RW == 1 ? 3 : 2, SP = RW == 1 ? 64 : BM;
+  const uint32_t lds_bytes = NST * 2 * BM * HD * 2 + NST * 2 * SP * 4;
+  const int nseg = a_in.dkv_split;
+  if (RW > 1 && nseg > 1) fail("dkv_flat_kernel: row waves and segments");
   const uint32_t stat_byte = NST * 2 * BM * HD * 2;
   const bool varlen = a_in.cu != nullptr;
   const int BHk = a_in.B * a_in.Hkv;
-  const int64_t nblk = dkv_flat_blocks(a_in);
+  const int64_t nblk = dkv_flat_blocks(a_in, BN) * nseg;
   typedef AsyncTileLoader<HD, BM, 256> Loader;
   for (int64_t block = 0; block < nblk; block++) {
     const int bh = (int)(block % BHk), ct = (int)(block / BHk);
     int b = bh / a_in.Hkv;
-    const int hkv = bh % a_in.Hkv;
+    const int hkv = bh % a_in.Hkv, first = varlen ? a_in.cu[b] : 0;
     const KArgs a = seq_args(a_in, b);
-    const ColTilePlan plan = col_tile_plan(a_in, a, ct, BN, BM, varlen, 1);
+    const ColTilePlan plan = col_tile_plan(a_in, a, ct, BN, BM, varlen, nseg);
     if (!plan.active) {
-      if (!varlen) fail("dkv_flat_kernel: inactive column tile in a fixed-length launch");
+      if (!varlen && nseg == 1) fail("dkv_flat_kernel: inactive column tile in a fixed-length launch");
       continue;
     }
     if (plan.dep) fail("dkv_flat_kernel: column tile %d is not a sequence tile", ct);
     for (int tid = 0; tid < 256; tid++) {
       const int lane = tid & 63, n = lane & 15, q4 = lane >> 4, wave = tid >> 6;
       for (int nb = 0; nb < NB; nb++) {
-        const int c = plan.c_first + wave * (16 * NB) + 16 * nb + n;
+        const int c = plan.c_first + (RW == 1 ? wave : 0) * (16 * NB) + 16 * nb + n;
         if (c >= a.T) continue;
         ctx("dkv_flat_kernel", (int)block, wave, lane, "stationary K and V rows");
         for (int ks = 0; ks < KS; ks++) {
@@ -558,9 +561,19 @@ void walk_dkv_flat(const KArgs& a_in) {
         ctx("dkv_flat_kernel", (int)block, wave, lane, "gradient rows");
         uint16_t* dkp = a.dk + b * a.sdk.b + hkv * a.sdk.h + (int64_t)c * a.sdk.t + 4 * q4;
         uint16_t* dvp = a.dv + b * a.sdv.b + hkv * a.sdv.h + (int64_t)c * a.sdv.t + 4 * q4;
+        if (plan.nsegs > 1) {
+          const int64_t pitch = part_rows(a), plane = (int64_t)(varlen ? 1 : a.B) * a.Hkv * pitch * HD;
+          float* kp = a.dkv_part + plan.seg * plane + (((int64_t)b * a.Hkv + hkv) * pitch + first + c) * HD + 4 * q4;
+          for (int d = 0; d < MB; d++) {
+            check_access("part", kp + 16 * d, 16, true);
+            check_access("part", kp + nseg * plane + 16 * d, 16, true);
+          }
+          continue;
+        }
         for (int d = 0; d < MB; d++) {
-          if (16 * d + 4 * q4 < a.D) check_access("dk", dkp + 16 * d, 8, true);
-          if (16 * d + 4 * q4 < a.Dv) check_access("dv", dvp + 16 * d, 8, true);
+          if (RW > 1 && d / (MB / 2) != (wave & 1)) continue;  // waves 0, 1 write dk, waves 2, 3 dv, half the blocks each
+          if ((RW == 1 || wave < 2) && 16 * d + 4 * q4 < a.D) check_access("dk", dkp + 16 * d, 8, true);
+          if ((RW == 1 || wave >= 2) && 16 * d + 4 * q4 < a.Dv) check_access("dv", dvp + 16 * d, 8, true);
         }
       }
       Loader ld;
@@ -582,11 +595,12 @@ void walk_dkv_flat(const KArgs& a_in) {
                     ld.lane_offset((int)a.sdo.t * 2, a.Dv), Loader::rows_before(i) * (int)a.sdo.t * 2, 16,
                     Qt + (uint32_t)(BM * HD + ld.lds_elems(i)) * 2, lds_bytes, ld.pads(a.Dv));
         }
-        const int rows = imax(imin(a.Tq - f_q0, BM), 0);
+        const int rows = imax(imin(a.Tq - f_q0, BM), 0), st_first = RW == 1 ? 0 : (wave >> 1) * 64;
         if (rows == 0) fail("dkv_flat_kernel: empty query tile at row %d (Tq %d)", f_q0, a.Tq);
         ctx("dkv_flat_kernel", (int)block, wave, lane, st_lse ? "query tile lse" : "query tile row sums");
-        check_dma(st_lse ? "lse" : "delta", stb + (int64_t)f_q0 * st_row, (uint32_t)(rows - 1) * st_row + 4u, lane * (int)st_row, 0, 4,
-                  stat_byte + (uint32_t)(ld_st * 2 * SP + (st_lse ? 0 : SP)) * 4, lds_bytes, false);
+        check_dma(st_lse ? "lse" : "delta", stb + (int64_t)f_q0 * st_row, (uint32_t)(rows - 1) * st_row + 4u,
+                  (st_first + lane) * (int)st_row, 0, 4, stat_byte + (uint32_t)(ld_st * 2 * SP + (st_lse ? 0 : SP) + st_first) * 4,
+                  lds_bytes, false);
         ld_st = (ld_st + 1) % NST;
       }
     }
@@ -595,23 +609,31 @@ void walk_dkv_flat(const KArgs& a_in) {
 
 // the partial sums of the row segments -> dk, dv
 template <int HD>
-void walk_reduce(const KArgs& a) {
-  constexpr int TPR = HD / 8;
-  const int64_t rows = (int64_t)a.B * a.Hkv * a.T, plane = rows * HD;
-  const int64_t nthreads = rows * TPR;
-  for (int64_t gid = 0; gid < (nthreads + 255) / 256 * 256; gid++) {
-    const int64_t row = gid / TPR;
-    if (row >= rows) continue;
-    const int sub = (int)(gid % TPR), c = (int)(row % a.T), bh = (int)(row / a.T), b = bh / a.Hkv, hkv = bh % a.Hkv;
-    ctx("dkv_reduce_kernel", (int)(gid / 256), (int)(gid % 256) >> 6, (int)(gid & 63), "partial sums and dk, dv rows");
-    for (int which = 0; which < 2; which++) {
-      const float* src = a.dkv_part + (int64_t)which * a.dkv_split * plane + row * HD + 8 * sub;
-      for (int sg = 0; sg < a.dkv_split; sg++) check_access("part", src + sg * plane, 32, false);
-      uint16_t* outp = which == 0 ? a.dk + b * a.sdk.b + hkv * a.sdk.h + (int64_t)c * a.sdk.t
-                                  : a.dv + b * a.sdv.b + hkv * a.sdv.h + (int64_t)c * a.sdv.t;
-      if (8 * sub < (which == 0 ? a.D : a.Dv)) check_access(which == 0 ? "dk" : "dv", outp + 8 * sub, 16, true);
+void walk_reduce(const KArgs& a_in, int BN, int BM) {
+  constexpr int TPR = HD / 8, RPB = 256 / TPR;
+  const int BHk = a_in.B * a_in.Hkv;
+  const int64_t nblk = ((int64_t)a_in.T + RPB - 1) / RPB * BHk;
+  for (int64_t block = 0; block < nblk; block++)
+    for (int tid = 0; tid < 256; tid++) {
+      const int bh = (int)(block % BHk), hkv = bh % a_in.Hkv, sub = tid % TPR, c = (int)(block / BHk) * RPB + tid / TPR;
+      int b = bh / a_in.Hkv;
+      const int first = a_in.cu ? a_in.cu[b] : 0;
+      const KArgs a = seq_args(a_in, b);
+      if (c >= a.T) continue;
+      const int row0 = a.causal ? c / BN * BN * a.Gf : 0;
+      const int nsegs = tile_segments(a, (a.Tq + BM - 1) / BM - row0 / BM, a.dkv_split);
+      if (nsegs == 1) continue;
+      const int64_t pitch = part_rows(a), plane = (int64_t)(a.cu ? 1 : a.B) * a.Hkv * pitch * HD;
+      const int64_t row = ((int64_t)b * a.Hkv + hkv) * pitch + first + c;
+      ctx("dkv_reduce_kernel", (int)block, tid >> 6, tid & 63, "partial sums and dk, dv rows");
+      for (int which = 0; which < 2; which++) {
+        const float* src = a.dkv_part + (int64_t)which * a.dkv_split * plane + row * HD + 8 * sub;
+        for (int sg = 0; sg < nsegs; sg++) check_access("part", src + sg * plane, 32, false);
+        uint16_t* outp = which == 0 ? a.dk + b * a.sdk.b + hkv * a.sdk.h + (int64_t)c * a.sdk.t
+                                    : a.dv + b * a.sdv.b + hkv * a.sdv.h + (int64_t)c * a.sdv.t;
+        if (8 * sub < (which == 0 ? a.D : a.Dv)) check_access(which == 0 ? "dk" : "dv", outp + 8 * sub, 16, true);
+      }
     }
-  }
 }
 
 // chunk-visible depth columns by whole chunks (tile widths up to 128)
@@ -854,14 +876,20 @@ void walk_all(const Case& c, const KArgs& a) {
     require_full("hand_p");
     require_full("hand_ds");
   }
-  if (takes_dkv_flat(a, HD, a.cu ? 1 : a.dkv_split)) {
-    if constexpr (HD == 64) walk_dkv_flat<HD>(a);
+  const bool flat = takes_dkv_flat(a, HD);
+  if (flat) {
+    if constexpr (HD == 64) {
+      if (dkv_flat_row_waves(a))
+        walk_dkv_flat<HD, 4>(a);
+      else
+        walk_dkv_flat<HD, 1>(a);
+    }
   } else {
     walk_dkv<HD>(a);
   }
   if (a.dkv_split > 1 && a.has_seq) {
-    require_full("part");
-    walk_reduce<HD>(a);
+    if (a.dkv_seg_tiles == 0) require_full("part");  // otherwise short tiles have fewer segments, or none
+    walk_reduce<HD>(a, HD > 128 ? 64 : 128, flat || HD > 128 ? 32 : 64);
   }
   if (a.has_seq) {
     require_full("dk");
@@ -923,8 +951,14 @@ int main(int argc, char** argv) {
   }
   KArgs a = make_args(c);
   a.dkv_split = split > 0 && !c.packed ? split : 1;
+  if (split < 0) {  // the library's own rule
+    const DkvSplit plan = dkv_split_plan(a, c.HD);
+    a.dkv_split = plan.nseg;
+    a.dkv_seg_tiles = plan.seg_tiles;
+    printf("segments=%d ", plan.nseg);
+  }
   if (a.dkv_split > 1)
-    a.dkv_part = (float*)add_region("part", 20, (uint64_t)2 * a.dkv_split * a.B * a.Hkv * a.T * c.HD * 4, 4, true);
+    a.dkv_part = (float*)add_region("part", 20, (uint64_t)2 * a.dkv_split * (a.cu ? 1 : a.B) * a.Hkv * part_rows(a) * c.HD * 4, 4, true);
   switch (c.HD) {
     case 64: walk_all<64>(c, a); break;
     case 128: walk_all<128>(c, a); break;

@@ -156,3 +156,25 @@ def test_row_split_launch(walker):
     for split in (2, 4, 8):
         rc, out = run(walker, (4096,), 1, 128, 0, 2, "causal", packed=False, B=1, split=split)
         assert rc == 0 and out.startswith("OK"), out
+
+
+@pytest.mark.parametrize("case", [
+    # lengths, H, D, L, G, mode, chunk tokens, packed, B, segments expected
+    ((2048,), 2, 128, 2, 4, "causal", 0, False, 1, True),
+    ((1100,), 2, 64, 0, 4, "causal", 0, False, 1, True),        # 64-wide tiles, ragged last tile
+    ((1000,), 3, 64, 2, 2, "noncausal", 0, False, 1, True),     # more than 1024 query rows: no row waves
+    ((3000, 1, 300, 0, 777), 1, 128, 2, 4, "causal", 0, True, 1, True),
+    ((3000, 130, 64, 0, 1), 1, 64, 2, 4, "causal", 0, True, 1, True),
+    ((1500, 700), 1, 96, 0, 8, "plain", 0, True, 1, True),      # head-dim GQA, padded head dim
+    ((900, 100), 1, 128, 2, 8, "chunk_visible", 40, True, 1, True),  # sequence segments and depth column tiles in one launch
+    ((197,), 1, 64, 3, 4, "noncausal", 0, False, 5, False),     # row waves
+    ((250,), 2, 64, 0, 4, "causal", 0, False, 3, False),        # ... with a diagonal
+    ((33,), 1, 40, 2, 3, "noncausal", 0, False, 2, False),      # ... one short query tile, padded head dim
+], ids=lambda c: f"{c[5]}-{'_'.join(map(str, c[0]))}-D{c[2]}G{c[4]}")
+def test_balanced_row_segments_and_row_waves(walker, case):
+    """The rule that cuts long column tiles into segments (tiles of one segment write their gradients themselves), and
+    the short launches whose waves share their columns: every access in bounds, every gradient row written once."""
+    lengths, H, D, L, G, mode, cb, packed, B, split = case
+    rc, out = run(walker, lengths, H, D, L, G, mode, cb, packed=packed, B=B, split=-1)
+    assert rc == 0 and "OK" in out, out
+    assert (int(out.split("segments=")[1].split()[0]) > 1) == split, out

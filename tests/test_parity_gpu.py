@@ -927,6 +927,24 @@ def test_row_split_sequence_gradients(gpu_device, case):
         assert ((a.float() - b_.float()).abs() <= 2.0 ** -6 * b_.float().abs() + 2e-3).all()
 
 
+@pytest.mark.parametrize("case", [
+    # (B, T, H, D, L, G, mode, dtype): short launches of the 64-wide tiles, whose waves share their columns
+    (2, 33, 1, 64, 2, 4, "noncausal", torch.bfloat16),      # one query tile and a row or two of the next, short column tile
+    (1, 256, 2, 64, 3, 4, "causal", torch.float16),         # 1024 query rows: the most that come here
+    (3, 95, 2, 40, 0, 3, "causal", torch.bfloat16),         # padded head dim, rows not a multiple of the tile
+    # ... and one row per head more: equal segments, single-segment tiles at the end
+    (1, 257, 2, 64, 3, 4, "causal", torch.float16),
+    (1, 1300, 1, 64, 1, 2, "noncausal", torch.bfloat16),
+])
+def test_short_and_segmented_launches_of_the_narrow_tiles(gpu_device, case):
+    B, T, H, D, L, G, mode, dtype = case
+    say(f"CASE narrow sequence gradients {case}")
+    inp = oracle.make_inputs(B, T, H, D, L, G, seed=89, dtype=dtype, std=0.5)
+    ref = oracle.moda_dense_fwd_bwd(inp, D ** -0.5, G, mode, 0)
+    got = run_hip(to_dev(inp, gpu_device), D ** -0.5, G, mode)
+    compare_all(got, ref, dtype, f"narrow {case}")
+
+
 def test_hip_graph_capture_and_replay(gpu_device):
     """Forward + backward captured in a HIP graph (the library allocates nothing and clears nothing, so
     every launch is capturable) and replayed with new inputs; every replay is checked against eager."""
@@ -1116,6 +1134,17 @@ def test_random_sweep_packed(gpu_device, seed):
     """Random packed batches on the 64- and 128-wide tiles: empty and one-token sequences, chunks below and above
     one query tile, every mode."""
     test_packed_variable_length_batches(gpu_device, _random_packed_case(7000 + seed))
+
+
+@pytest.mark.parametrize("case", [
+    # long sequences in a small batch: their key tiles are cut along the query rows, those of the short ones are not
+    ((1700, 0, 1, 130), 1, 128, 2, 2, "causal", 0, torch.bfloat16),
+    ((1700, 65, 300), 1, 64, 2, 2, "causal", 0, torch.float16),
+    ((700, 129), 2, 64, 0, 4, "noncausal", 0, torch.bfloat16),
+    ((1000, 33), 1, 96, 2, 4, "chunk_visible", 40, torch.bfloat16),
+], ids=lambda c: f"{c[5]}-{'_'.join(map(str, c[0]))}-D{c[2]}")
+def test_packed_batches_cut_along_the_query_rows(gpu_device, case):
+    test_packed_variable_length_batches(gpu_device, case)
 
 
 def test_packed_batch_equals_separate_calls_bitwise(gpu_device):
