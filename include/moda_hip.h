@@ -99,7 +99,12 @@ enum moda_hip_flag {
    */
   MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS = 1,
   /* dkd, dvd: slots >= L_valid are left alone (implied by the flag above); without it they are zeroed */
-  MODA_HIP_FLAG_KEEP_DEPTH_SLOTS = 2
+  MODA_HIP_FLAG_KEEP_DEPTH_SLOTS = 2,
+  /* backward, with either flag above: dk, dv get the gradient that slot L_valid of dkd, dvd holds added -- the layer's
+   * own slot of a stream whose later layers have run their backward.  In the launch that forms dk, dv, before their
+   * rounding; MODA_HIP_EUNSUPPORTED, with nothing launched, where that launch does not do it (it does on 16-bit types,
+   * head dims up to 64, kv head = query head, fixed length): use moda_hip_depth_slot_add then. */
+  MODA_HIP_FLAG_ADD_OWN_SLOT = 4
 };
 
 typedef struct moda_hip_strides {

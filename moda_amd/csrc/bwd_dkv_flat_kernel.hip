@@ -210,6 +210,16 @@ __global__ __launch_bounds__(256, RW == 1 ? 3 : 2) void dkv_flat_kernel(const KA
     __syncthreads();
   }
 
+  auto own_slot_row = [&](bool is_v, int col) -> const uint16_t* {  // this lane's part of slot Lv of the column's token
+    const int64_t row = (int64_t)col * a.L + a.Lv;
+    return (is_v ? a.dvd + b * a.sdvd.b + hkv * a.sdvd.h + row * a.sdvd.t : a.dkd + b * a.sdkd.b + hkv * a.sdkd.h + row * a.sdkd.t) + 4 * q4;
+  };
+  auto add_own = [&](f32x4& x, const i32x2& w) {
+    float f[4];
+    unpack2<T>(w[0], f[0], f[1]);
+    unpack2<T>(w[1], f[2], f[3]);
+    x += f32x4{f[0], f[1], f[2], f[3]};
+  };
   if constexpr (RW > 1) {
     // [which][d][nb] blocks of all waves through the ring (which every wave has done reading): wave w adds up and writes
     // a quarter of them
@@ -222,8 +232,20 @@ __global__ __launch_bounds__(256, RW == 1 ? 3 : 2) void dkv_flat_kernel(const KA
         ex[((rw * 2 * MB + d) * NB + nb) * 64 + lane] = dk[d][nb];
         ex[((rw * 2 * MB + MB + d) * NB + nb) * 64 + lane] = dv[d][nb];
       }
-    __syncthreads();
     const bool is_v = rw >= RW / 2;
+    i32x2 own[NB][2 * MB / RW];  // the layer's own slot: on its way while the accumulators are exchanged
+    if (a.own_slot) {
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) {
+        const uint16_t* slot = own_slot_row(is_v, c[nb]);
+#pragma unroll
+        for (int i = 0; i < 2 * MB / RW; i++) {
+          const int d = (rw * (2 * MB / RW) + i) % MB;
+          own[nb][i] = valid[nb] && 16 * d + 4 * q4 < (is_v ? a.Dv : a.D) ? *reinterpret_cast<const i32x2*>(slot + 16 * d) : i32x2{0, 0};
+        }
+      }
+    }
+    __syncthreads();
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
       uint16_t* outp = is_v ? a.dv + b * a.sdv.b + hkv * a.sdv.h + (int64_t)c[nb] * a.sdv.t
@@ -235,6 +257,7 @@ __global__ __launch_bounds__(256, RW == 1 ? 3 : 2) void dkv_flat_kernel(const KA
 #pragma unroll
         for (int w = 1; w < RW; w++) sum += ex[((w * 2 * MB + blk) * NB + nb) * 64 + lane];
         sum *= is_v ? 1.f : a.scale;
+        if (a.own_slot) add_own(sum, own[nb][i]);
         i32x2 w;
         w[0] = pack2<T>(sum[0], sum[1]);
         w[1] = pack2<T>(sum[2], sum[3]);
@@ -266,9 +289,14 @@ __global__ __launch_bounds__(256, RW == 1 ? 3 : 2) void dkv_flat_kernel(const KA
       uint16_t* dvp = a.dv + b * a.sdv.b + hkv * a.sdv.h + (int64_t)c[nb] * a.sdv.t + 4 * q4;
 #pragma unroll
       for (int d = 0; d < MB; d++) {
+        dk[d][nb] *= a.scale;
+        if (!VARLEN && a.own_slot) {
+          if (16 * d + 4 * q4 < a.D) add_own(dk[d][nb], *reinterpret_cast<const i32x2*>(own_slot_row(false, c[nb]) + 16 * d));
+          if (16 * d + 4 * q4 < a.Dv) add_own(dv[d][nb], *reinterpret_cast<const i32x2*>(own_slot_row(true, c[nb]) + 16 * d));
+        }
         i32x2 w;
-        w[0] = pack2<T>(dk[d][nb][0] * a.scale, dk[d][nb][1] * a.scale);
-        w[1] = pack2<T>(dk[d][nb][2] * a.scale, dk[d][nb][3] * a.scale);
+        w[0] = pack2<T>(dk[d][nb][0], dk[d][nb][1]);
+        w[1] = pack2<T>(dk[d][nb][2], dk[d][nb][3]);
         if (16 * d + 4 * q4 < a.D) *reinterpret_cast<i32x2*>(dkp + 16 * d) = w;
         w[0] = pack2<T>(dv[d][nb][0], dv[d][nb][1]);
         w[1] = pack2<T>(dv[d][nb][2], dv[d][nb][3]);

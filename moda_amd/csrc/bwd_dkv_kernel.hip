@@ -934,6 +934,18 @@ __global__ __launch_bounds__(256) void dkv_reduce_kernel(const KArgs a_in, int B
       }
     }
     i32x4 w;
+    if (!VARLEN && a.own_slot && 8 * sub < (which == 0 ? a.D : a.Dv)) {
+      const int64_t slot = (int64_t)c * a.L + a.Lv;
+      w = *reinterpret_cast<const i32x4*>((which == 0 ? a.dkd + b * a.sdkd.b + hkv * a.sdkd.h + slot * a.sdkd.t
+                                                      : a.dvd + b * a.sdvd.b + hkv * a.sdvd.h + slot * a.sdvd.t) + 8 * sub);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        float lo, hi;
+        unpack2<T>(w[i], lo, hi);
+        s[2 * i] += lo;
+        s[2 * i + 1] += hi;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < 4; i++) w[i] = pack2<T>(s[2 * i], s[2 * i + 1]);
     uint16_t* outp = which == 0 ? a.dk + b * a.sdk.b + hkv * a.sdk.h + (int64_t)c * a.sdk.t

@@ -100,7 +100,8 @@ int fill_geometry(const moda_hip_desc* d, KArgs& a) {
   if (d->mode == MODA_HIP_DEPTH_ONLY && d->L == 0) return MODA_HIP_EINVAL;
   if (d->mode == MODA_HIP_CHUNK_VISIBLE && d->L > 0 && d->chunk_tokens <= 0) return MODA_HIP_EINVAL;
   if (d->L_valid < 0 || d->L_valid > d->L) return MODA_HIP_EINVAL;
-  if (d->flags & ~(int32_t)(MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS | MODA_HIP_FLAG_KEEP_DEPTH_SLOTS)) return MODA_HIP_EINVAL;
+  if (d->flags & ~(int32_t)(MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS | MODA_HIP_FLAG_KEEP_DEPTH_SLOTS | MODA_HIP_FLAG_ADD_OWN_SLOT))
+    return MODA_HIP_EINVAL;
   // 32-bit index space used for rows and flattened depth columns inside the kernels
   if (d->T * d->G >= (1ll << 30) || d->T * (d->L > 0 ? d->L : 1) >= (1ll << 30) || d->B * d->H * d->G >= (1ll << 20))
     return MODA_HIP_EUNSUPPORTED;
@@ -122,8 +123,9 @@ int fill_geometry(const moda_hip_desc* d, KArgs& a) {
   a.has_seq = d->mode != MODA_HIP_DEPTH_ONLY;
   a.causal = d->mode == MODA_HIP_CAUSAL || d->mode == MODA_HIP_CHUNK_VISIBLE || plain;
   a.chunk = d->mode == MODA_HIP_CHUNK_VISIBLE;
+  a.own_slot = (d->flags & MODA_HIP_FLAG_ADD_OWN_SLOT) ? 1 : 0;
   a.accum_depth = (d->flags & MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS) ? 1 : 0;
-  a.keep_slots = d->flags ? 1 : 0;
+  a.keep_slots = (d->flags & (MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS | MODA_HIP_FLAG_KEEP_DEPTH_SLOTS)) ? 1 : 0;
   a.nqt = (a.Tq + 127) / 128;
   a.scale = d->scale;
   a.delta_pitch = a.Tq;
@@ -350,6 +352,10 @@ int moda_hip_bwd_stages(const moda_hip_desc* d, const void* q, const void* k, co
   int rc = fill_geometry(d, a);
   if (rc) return rc;
   if (stages < 0 || stages > MODA_HIP_STAGE_ALL) return MODA_HIP_EINVAL;
+  if (a.own_slot) {
+    if (a.L == 0 || a.Lv >= a.L || !a.keep_slots) return MODA_HIP_EINVAL;
+    if (!use_mfma(d) || a.cu || !moda::takes_dkv_flat(a, tile_width(d))) return MODA_HIP_EUNSUPPORTED;
+  }
   const int es = elem_size(d->dtype);
   if (per_sequence(d) && (int64_t)a.B * a.Tq * a.Hq > 0) {
     MODA_REQ_PTR(lse);

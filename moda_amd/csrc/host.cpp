@@ -293,11 +293,14 @@ typedef std::array<Tensor, 5> Grads;  // dq, dk, dv, dkd, dvd
 enum DepthGrads { kOverwrite = 0, kAccumulate = MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS, kKeepSlots = MODA_HIP_FLAG_KEEP_DEPTH_SLOTS };
 
 // `out`: gradient buffers to write to (an undefined entry is allocated here like all of them without `out`); `ws`:
-// workspace to use, else allocated here.
+// workspace to use, else allocated here.  `add_own_slot`: in, dk and dv are to have slot depth_valid of dkd, dvd added; out,
+// whether they have.
 Grads backward(const Call& c, Tensor q, Tensor k, Tensor v, Tensor kd, Tensor vd, Tensor o, Tensor lse, Tensor d_o, int stages,
-               const Grads* out, Tensor ws, DepthGrads depth_grads) {
+               const Grads* out, Tensor ws, DepthGrads depth_grads, bool* add_own_slot = nullptr) {
   const bool accumulate = depth_grads == kAccumulate;
   CONTRACT(!accumulate || (out && (*out)[3].defined() && (*out)[4].defined()), "accumulate_depth needs the gradient buffers to add to");
+  const bool own_slot = add_own_slot && *add_own_slot && !narrows(q);
+  if (add_own_slot) *add_own_slot = false;
   if (narrows(q)) {
     // 16-bit gradients from the matrix kernels (without the accumulate flag: the slots without data come back as
     // zeros), widened into the caller's fp32 buffers or added to them
@@ -352,10 +355,22 @@ Grads backward(const Call& c, Tensor q, Tensor k, Tensor v, Tensor kd, Tensor vd
   c10::OptionalDeviceGuard guard(q.device());
   if (!ws.defined())
     ws = at::empty({std::max<int64_t>((int64_t)moda_hip_bwd_workspace_bytes(&d), 4)}, q.options().dtype(at::kByte));
-  check_rc(moda_hip_bwd_stages(&d, in_ptr(q), in_ptr(k), in_ptr(v), in_ptr(kd), in_ptr(vd), in_ptr(o), (const float*)in_ptr(lse),
+  auto launch = [&] {
+    return moda_hip_bwd_stages(&d, in_ptr(q), in_ptr(k), in_ptr(v), in_ptr(kd), in_ptr(vd), in_ptr(o), (const float*)in_ptr(lse),
                                in_ptr(d_o), out_ptr(to[0]), out_ptr(to[1]), out_ptr(to[2]), out_ptr(to[3]), out_ptr(to[4]),
-                               out_ptr(ws), (size_t)ws.nbytes(), stages, stream_of(q)),
-           "moda_hip_bwd");
+                               out_ptr(ws), (size_t)ws.nbytes(), stages, stream_of(q));
+  };
+  if (own_slot) {
+    d.flags |= MODA_HIP_FLAG_ADD_OWN_SLOT;
+    const int rc = launch();
+    if (rc != MODA_HIP_EUNSUPPORTED) {
+      check_rc(rc, "moda_hip_bwd");
+      *add_own_slot = true;
+      return g;
+    }
+    d.flags &= ~MODA_HIP_FLAG_ADD_OWN_SLOT;
+  }
+  check_rc(launch(), "moda_hip_bwd");
   return g;
 }
 
@@ -513,6 +528,8 @@ struct StreamAttend : torch::autograd::Function<StreamAttend> {
     const Tensor d_o = grads[0].defined() ? grads[0].to(o.scalar_type()) : at::zeros_like(o);
     const int64_t n = call->n;
     Grads g;
+    const bool join = call->slot >= 0 && call->slot < buf.written;  // later layers have seen this one's slot
+    bool joined = join && call->slot == n;
     if (n > 0) {
       bool first = buf.written == 0;
       if (first && narrows(q)) {  // gradients computed in another type arrive as sums
@@ -521,12 +538,14 @@ struct StreamAttend : torch::autograd::Function<StreamAttend> {
         first = false;
       }
       const Grads into{Tensor(), Tensor(), Tensor(), buf.gk, buf.gv};
-      g = ::backward(call->call, q, k, v, buf.k, buf.v, o, lse, d_o, MODA_HIP_STAGE_ALL, &into, Tensor(), first ? kKeepSlots : kAccumulate);
+      g = ::backward(call->call, q, k, v, buf.k, buf.v, o, lse, d_o, MODA_HIP_STAGE_ALL, &into, Tensor(), first ? kKeepSlots : kAccumulate,
+                     &joined);
       buf.written = std::max(buf.written, n);
     } else {
       g = ::backward(call->call, q, k, v, {}, {}, o, lse, d_o, MODA_HIP_STAGE_ALL, nullptr, Tensor(), kOverwrite);
+      joined = false;
     }
-    if (call->slot >= 0 && call->slot < buf.written) {
+    if (join && !joined) {
       const moda_hip_strides sk = strides_of(g[1]), sv = strides_of(g[2]);
       c10::OptionalDeviceGuard guard(k.device());
       check_rc(moda_hip_depth_slot_add(out_ptr(g[1]), out_ptr(g[2]), &sk, &sv, call->slot, buf.L, k.size(0), k.size(1), k.size(2), k.size(3),

@@ -1555,3 +1555,37 @@ def test_depth_reorg_round_trip_full_size(gpu_device):
     for a, b in zip(layers, back):
         assert torch.equal(a, b)
     assert torch.equal(cache.view(B, T, L, H, D)[:, :, 7], layers[7])
+
+
+@pytest.mark.parametrize("case", [
+    # (B, T, H, G, D): layer gradients that join their slot's in the launch that forms them
+    (2, 50, 1, 4, 64),       # waves that share their columns, one query tile and a part
+    (1, 601, 2, 2, 64),      # row segments: in the kernel that adds them up, or in the tiles of one segment
+    (43, 1100, 2, 1, 40),    # whole column tiles, padded head dim
+    (1, 70, 2, 2, 128),      # the wider tiles: in a launch of its own
+])
+def test_stream_layers_join_their_slot_gradient(gpu_device, case):
+    """Three layers through one depth stream against the same calls on stacked caches, whose gradients torch adds up.
+    Both round a layer's own gradient and its slot's to bf16 (2^-8), the reference their sum once more."""
+    import moda_amd
+
+    B, T, H, G, D = case
+    say(f"CASE stream slots {case}")
+    gen = torch.Generator(device=gpu_device).manual_seed(5)
+    rn = lambda *s: (0.5 * torch.randn(*s, generator=gen, device=gpu_device)).bfloat16().requires_grad_(True)
+    layers = [(rn(B, T * G, H, D), rn(B, T, H, D), rn(B, T, H, D)) for _ in range(3)]
+    flat = [x for layer in layers for x in layer]
+    do = [rn(B, T * G, H, D).detach() for _ in range(3)]
+    stream, outs = moda_amd.DepthStream(3), []
+    for q, k, v in layers:
+        outs.append(stream.attend(q, k, v, moda_group_num=G, is_causal=False))
+        stream.push(k, v)
+    got = torch.autograd.grad(outs, flat, do)
+    outs = []
+    for n, (q, k, v) in enumerate(layers):
+        kd = moda_amd.stack_depth([l[1] for l in layers[:n]]) if n else None
+        vd = moda_amd.stack_depth([l[2] for l in layers[:n]]) if n else None
+        outs.append(moda_amd.parallel_moda(q, k, v, cached_k=kd, cached_v=vd, moda_group_num=G, is_causal=False))
+    ref = torch.autograd.grad(outs, flat, do)
+    for i, (a, b) in enumerate(zip(got, ref)):
+        assert (a.float() - b.float()).norm() <= 2.0 ** -7 * b.float().norm(), (i, case)
