@@ -103,7 +103,8 @@ enum moda_hip_flag {
   /* backward, with either flag above: dk, dv get the gradient that slot L_valid of dkd, dvd holds added -- the layer's
    * own slot of a stream whose later layers have run their backward.  In the launch that forms dk, dv, before their
    * rounding; MODA_HIP_EUNSUPPORTED, with nothing launched, where that launch does not do it (it does on 16-bit types,
-   * head dims up to 64, kv head = query head, fixed length): use moda_hip_depth_slot_add then. */
+   * head dims up to 64, kv head = query head, fixed length, launches that are cut along the query rows or short): use
+   * moda_hip_depth_slot_add then. */
   MODA_HIP_FLAG_ADD_OWN_SLOT = 4
 };
 

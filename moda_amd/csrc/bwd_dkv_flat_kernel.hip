@@ -289,14 +289,15 @@ __global__ __launch_bounds__(256, RW == 1 ? 3 : 2) void dkv_flat_kernel(const KA
       uint16_t* dvp = a.dv + b * a.sdv.b + hkv * a.sdv.h + (int64_t)c[nb] * a.sdv.t + 4 * q4;
 #pragma unroll
       for (int d = 0; d < MB; d++) {
-        dk[d][nb] *= a.scale;
-        if (!VARLEN && a.own_slot) {
+        if (SPLIT) dk[d][nb] *= a.scale;
+        if (SPLIT && !VARLEN && a.own_slot) {  // (not in the instantiation of the long launches: 0.7 % of their time)
           if (16 * d + 4 * q4 < a.D) add_own(dk[d][nb], *reinterpret_cast<const i32x2*>(own_slot_row(false, c[nb]) + 16 * d));
           if (16 * d + 4 * q4 < a.Dv) add_own(dv[d][nb], *reinterpret_cast<const i32x2*>(own_slot_row(true, c[nb]) + 16 * d));
         }
         i32x2 w;
-        w[0] = pack2<T>(dk[d][nb][0], dk[d][nb][1]);
-        w[1] = pack2<T>(dk[d][nb][2], dk[d][nb][3]);
+        const float mul = SPLIT ? 1.f : a.scale;
+        w[0] = pack2<T>(dk[d][nb][0] * mul, dk[d][nb][1] * mul);
+        w[1] = pack2<T>(dk[d][nb][2] * mul, dk[d][nb][3] * mul);
         if (16 * d + 4 * q4 < a.D) *reinterpret_cast<i32x2*>(dkp + 16 * d) = w;
         w[0] = pack2<T>(dv[d][nb][0], dv[d][nb][1]);
         w[1] = pack2<T>(dv[d][nb][2], dv[d][nb][3]);

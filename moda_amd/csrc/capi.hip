@@ -423,6 +423,7 @@ int moda_hip_bwd_stages(const moda_hip_desc* d, const void* q, const void* k, co
     while (split.nseg > 1 && delta_bytes(a) + hand + dkv_part_bytes(d, a, split.nseg) > workspace_bytes) split.nseg /= 2;
     if ((uintptr_t)workspace % 16 != 0) split.nseg = 1;  // the partial sums are written and read 16 bytes at a time
     a.dkv_split = split.nseg;
+    if (a.own_slot && split.nseg == 1 && !moda::dkv_flat_row_waves(a)) return MODA_HIP_EUNSUPPORTED;
     a.dkv_seg_tiles = (split.seg_tiles * most + split.nseg - 1) / split.nseg;  // fewer segments: longer ones
     a.dkv_part = (float*)((char*)workspace + delta_bytes(a) + hand);
     if (hand) {
