@@ -259,17 +259,64 @@ def _refuse_decay(g, q):
     assert g is None, "g is not supported in this version"
 
 
-class ParallelMixtureOfDepthAttentionFunction:
-    """moda_v14.py:2649-2789, by its ``apply``: differentiable in q, k, v, cached_k, cached_v; the gradient into
-    ``lse`` is ignored.  (The autograd node itself is native: csrc/host.cpp, Attend.)"""
+class _AttentionFunction(torch.autograd.Function):
+    """What the four operators' autograd Functions share.  ``apply`` of one of them builds the native node of the same
+    computation (csrc/host.cpp, Attend), which costs a tenth of the host time; a class derived from one of them runs
+    its own ``forward`` and ``backward`` as any Function does.  The gradient into ``lse`` is ignored."""
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        return cls._attend(*args, **kwargs) if cls in _NATIVE_FUNCTIONS else super().apply(*args, **kwargs)
 
     @staticmethod
-    def apply(q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, is_causal=True,
-              group_bs=None, group_warps=None, depth_bs=None, depth_warps=None, depth_valid=None):
+    def _run(ctx, mode, q, k, v, cached_k, cached_v, scale, moda_group_num, chunk_tokens, depth_valid, cu_seqlens):
+        if cached_k is None or cached_v is None:
+            cached_k = cached_v = None
+        packed = _packed(cu_seqlens, q, 1 if mode == _lib.PLAIN_GQA else moda_group_num)
+        scale = q.shape[-1] ** -0.5 if scale is None else scale
+        o, lse = _raw_fwd(mode, q, k, v, cached_k, cached_v, scale, moda_group_num, chunk_tokens, depth_valid, packed)
+        ctx.save_for_backward(q, k, v, cached_k, cached_v, o, lse)
+        ctx.call = (mode, scale, moda_group_num, chunk_tokens, depth_valid, packed)
+        ctx.set_materialize_grads(False)
+        return o, lse
+
+    @staticmethod
+    def _gradients(ctx, do):
+        if do is None:
+            return (None,) * 5
+        mode, scale, G, chunk_tokens, depth_valid, packed = ctx.call
+        q, k, v, cached_k, cached_v, o, lse = ctx.saved_tensors
+        return _raw_bwd(mode, q, k, v, cached_k, cached_v, o, lse, do.to(o.dtype), scale, G, chunk_tokens,
+                        depth_valid=depth_valid, packed=packed)
+
+
+class ParallelMixtureOfDepthAttentionFunction(_AttentionFunction):
+    """moda_v14.py:2649-2789: differentiable in q, k, v, cached_k, cached_v."""
+
+    @staticmethod
+    def _attend(q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, is_causal=True,
+                group_bs=None, group_warps=None, depth_bs=None, depth_warps=None, depth_valid=None):
         assert g is None, "g is not supported in this version"
         cu, packed = _offsets(cu_seqlens)
         return _lib.host().attend(_lib.CAUSAL if is_causal else _lib.NONCAUSAL, q, k, v, cached_k, cached_v, scale,
                                   moda_group_num, 0, depth_valid, cu, packed, False, 128)
+
+    @staticmethod
+    @torch.amp.custom_fwd(device_type="cuda")
+    def forward(ctx, q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, is_causal=True,
+                group_bs=None, group_warps=None, depth_bs=None, depth_warps=None, depth_valid=None):
+        assert g is None, "g is not supported in this version"
+        _assert_group_tile(moda_group_num)
+        o, lse = _AttentionFunction._run(ctx, _lib.CAUSAL if is_causal else _lib.NONCAUSAL, q, k, v, cached_k, cached_v,
+                                         scale, moda_group_num, 0, depth_valid, cu_seqlens)
+        ctx.mark_non_differentiable(lse)
+        return o, lse
+
+    @staticmethod
+    @torch.amp.custom_bwd(device_type="cuda")
+    def backward(ctx, do, dlse):
+        dq, dk, dv, dkd, dvd = _AttentionFunction._gradients(ctx, do)
+        return dq, dk, dv, None, None, None, dkd, dvd, None, None, None, None, None, None, None
 
 
 def _head_last(*xs):
@@ -363,16 +410,32 @@ def parallel_moda_chunk_visible_bwd(q, k, v, o, g_cumsum, lse, do, scale=None, c
     return dq, dk, dv, None, dkd, dvd
 
 
-class ParallelMixtureOfDepthAttentionChunkVisibleFunction:
-    """moda_v16.py:3456-3493, by its ``apply``."""
+class ParallelMixtureOfDepthAttentionChunkVisibleFunction(_AttentionFunction):
+    """moda_v16.py:3456-3493."""
 
     @staticmethod
-    def apply(q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, chunk_rows=None,
-              depth_valid=None):
+    def _attend(q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, chunk_rows=None,
+                depth_valid=None):
         assert g is None, "g is not supported in this version"
         cu, packed = _offsets(cu_seqlens)
         return _lib.host().attend(_lib.CHUNK_VISIBLE, q, k, v, cached_k, cached_v, scale, moda_group_num,
                                   _chunk_tokens(moda_group_num, chunk_rows), depth_valid, cu, packed, False, 0)
+
+    @staticmethod
+    @torch.amp.custom_fwd(device_type="cuda")
+    def forward(ctx, q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, chunk_rows=None,
+                depth_valid=None):
+        assert g is None, "g is not supported in this version"
+        o, lse = _AttentionFunction._run(ctx, _lib.CHUNK_VISIBLE, q, k, v, cached_k, cached_v, scale, moda_group_num,
+                                         _chunk_tokens(moda_group_num, chunk_rows), depth_valid, cu_seqlens)
+        ctx.mark_non_differentiable(lse)
+        return o, lse
+
+    @staticmethod
+    @torch.amp.custom_bwd(device_type="cuda")
+    def backward(ctx, do, dlse):
+        dq, dk, dv, dkd, dvd = _AttentionFunction._gradients(ctx, do)
+        return dq, dk, dv, None, None, None, dkd, dvd, None, None, None
 
 
 def parallel_moda_chunk_visible(q, k, v, g=None, cached_k=None, cached_v=None, scale=None, cu_seqlens=None,
@@ -426,18 +489,39 @@ def parallel_fda_bwd(q, o, g_cumsum, lse, do, scale=None, chunk_size=128, cu_seq
     return dq, None, dkd, dvd
 
 
-class ParallelFlashDepthAttentionFunction:
-    """fda_v12.py:1207-1338, by its ``apply`` (the k, v slots must be None)."""
+class ParallelFlashDepthAttentionFunction(_AttentionFunction):
+    """fda_v12.py:1207-1338 (the k, v slots must be None)."""
 
     @staticmethod
-    def apply(q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, group_bs=None,
-              group_warps=None, depth_bs=None, depth_warps=None):
+    def _check(k, v, g, cached_k, cached_v):
         assert g is None, "g is not supported in this version"
         assert k is None and v is None, "Flash Depth Attention does not accept legacy k/v; pass None"
         assert cached_k is not None and cached_v is not None, "Flash Depth Attention requires cached_k/cached_v"
+
+    @staticmethod
+    def _attend(q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, group_bs=None,
+                group_warps=None, depth_bs=None, depth_warps=None):
+        ParallelFlashDepthAttentionFunction._check(k, v, g, cached_k, cached_v)
         cu, packed = _offsets(cu_seqlens)
         return _lib.host().attend(_lib.DEPTH_ONLY, q, None, None, cached_k, cached_v, scale, moda_group_num, 0, None,
                                   cu, packed, False, 128)
+
+    @staticmethod
+    @torch.amp.custom_fwd(device_type="cuda")
+    def forward(ctx, q, k, v, g, scale, cu_seqlens, cached_k=None, cached_v=None, moda_group_num=1, group_bs=None,
+                group_warps=None, depth_bs=None, depth_warps=None):
+        ParallelFlashDepthAttentionFunction._check(k, v, g, cached_k, cached_v)
+        _assert_group_tile(moda_group_num)
+        o, lse = _AttentionFunction._run(ctx, _lib.DEPTH_ONLY, q, None, None, cached_k, cached_v, scale, moda_group_num,
+                                         0, None, cu_seqlens)
+        ctx.mark_non_differentiable(lse)
+        return o, lse
+
+    @staticmethod
+    @torch.amp.custom_bwd(device_type="cuda")
+    def backward(ctx, do, dlse):
+        dq, _, _, dkd, dvd = _AttentionFunction._gradients(ctx, do)
+        return dq, None, None, None, None, None, dkd, dvd, None, None, None, None, None
 
 
 def parallel_fda(q, k=None, v=None, g=None, cached_k=None, cached_v=None, scale=None, cu_seqlens=None,
@@ -517,17 +601,37 @@ def parallel_attn_bwd(q, k, v, o, g_cumsum, lse, do, scale=None, chunk_size=128,
     return dq, dk, dv, None
 
 
-class ParallelAttentionFunction:
-    """fla/ops/attn/parallel.py:632-675, by its ``apply``."""
+class ParallelAttentionFunction(_AttentionFunction):
+    """fla/ops/attn/parallel.py:632-675."""
 
     @staticmethod
-    def apply(q, k, v, g, scale, cu_seqlens):
+    def _check(q, k, g):
         assert g is None, "g is not supported"
         assert q.shape[2] % k.shape[2] == 0, "HQ must be a multiple of H"
         assert q.shape[1] == k.shape[1]
+
+    @staticmethod
+    def _attend(q, k, v, g, scale, cu_seqlens):
+        ParallelAttentionFunction._check(q, k, g)
         cu, packed = _offsets(cu_seqlens)
         return _lib.host().attend(_lib.PLAIN_GQA, q, k, v, None, None, scale, q.shape[2] // k.shape[2], 0, None, cu,
                                   packed, False, 0)[0]
+
+    @staticmethod
+    @torch.amp.custom_fwd(device_type="cuda")
+    def forward(ctx, q, k, v, g, scale, cu_seqlens):
+        ParallelAttentionFunction._check(q, k, g)
+        return _AttentionFunction._run(ctx, _lib.PLAIN_GQA, q, k, v, None, None, scale, q.shape[2] // k.shape[2], 0, None,
+                                       cu_seqlens)[0]
+
+    @staticmethod
+    @torch.amp.custom_bwd(device_type="cuda")
+    def backward(ctx, do):
+        return *_AttentionFunction._gradients(ctx, do)[:3], None, None, None
+
+
+_NATIVE_FUNCTIONS = frozenset((ParallelMixtureOfDepthAttentionFunction, ParallelMixtureOfDepthAttentionChunkVisibleFunction,
+                               ParallelFlashDepthAttentionFunction, ParallelAttentionFunction))
 
 
 def parallel_attn(q, k, v, g=None, scale=None, cu_seqlens=None, head_first=False):

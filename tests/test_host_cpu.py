@@ -398,3 +398,48 @@ def test_fp32_compute_setting():
     with pytest.raises(AssertionError):
         moda_amd.set_fp32_compute("tf32")
     assert moda_amd.set_fp32_compute("fp32") == "fp32"
+
+
+def _function_calls():
+    """The operators' autograd Functions with arguments of a small call each, and which of them are tensors."""
+    import moda_amd
+
+    g = torch.Generator().manual_seed(2)
+    r = lambda *s: torch.randn(*s, generator=g, dtype=torch.float64)
+    q, k, v, kd, vd = r(1, 8, 2, 4), r(1, 4, 2, 4), r(1, 4, 2, 4), r(1, 12, 2, 4), r(1, 12, 2, 4)
+    return [(moda_amd.ParallelMixtureOfDepthAttentionFunction, [q, k, v, None, 0.5, None, kd, vd, 2]),
+            (moda_amd.ParallelMixtureOfDepthAttentionChunkVisibleFunction, [q, k, v, None, 0.5, None, kd, vd, 2]),
+            (moda_amd.ParallelFlashDepthAttentionFunction, [q, None, None, None, 0.5, None, kd, vd, 2]),
+            (moda_amd.ParallelAttentionFunction, [r(1, 4, 4, 4), k, v, None, 0.5, None])]
+
+
+def _stub_kernels(monkeypatch):
+    """Stand-ins for the launches: an output that depends on every input, a gradient that names the input it is of."""
+    from moda_amd import ops
+
+    def fwd(mode, q, k, v, kd, vd, scale, G, chunk_tokens=0, depth_valid=None, packed=None):
+        o = q * scale + sum(x.sum() for x in (k, v, kd, vd) if x is not None)
+        return o, o.sum(-1)
+
+    def bwd(mode, q, k, v, kd, vd, o, lse, do, scale, G, chunk_tokens=0, **kw):
+        return tuple(None if x is None else torch.full_like(x, 10.0 * (i + 1)) for i, x in enumerate((q, k, v, kd, vd)))
+
+    monkeypatch.setattr(ops, "_raw_fwd", fwd)
+    monkeypatch.setattr(ops, "_raw_bwd", bwd)
+
+
+def test_operator_functions_are_autograd_functions(monkeypatch):
+    """The Functions the reference's modules export are torch.autograd.Functions with a forward and a backward of their
+    own, which a class derived from one of them runs; every gradient arrives at the input it belongs to."""
+    _stub_kernels(monkeypatch)
+    for cls, args in _function_calls():
+        assert issubclass(cls, torch.autograd.Function)
+        assert "forward" in cls.__dict__ and "backward" in cls.__dict__
+        xs = [x.clone().requires_grad_() if isinstance(x, torch.Tensor) else x for x in args]
+        out = type("Derived", (cls,), {}).apply(*xs)
+        o = out[0] if isinstance(out, tuple) else out
+        assert o.grad_fn is not None and (not isinstance(out, tuple) or not out[1].requires_grad)
+        o.sum().backward()
+        order = [xs[i] for i in (0, 1, 2, 6, 7) if i < len(xs)]
+        for i, x in enumerate(order):
+            assert x is None or (x.grad == 10.0 * (i + 1)).all(), (cls.__name__, i)

@@ -1589,3 +1589,27 @@ def test_stream_layers_join_their_slot_gradient(gpu_device, case):
     ref = torch.autograd.grad(outs, flat, do)
     for i, (a, b) in enumerate(zip(got, ref)):
         assert (a.float() - b.float()).norm() <= 2.0 ** -7 * b.float().norm(), (i, case)
+
+
+def test_derived_autograd_functions_match_the_native_node(gpu_device):
+    """A class derived from an operator's autograd Function runs the Function's own forward and backward; the class
+    itself builds the native node.  Same launches, so the same bits."""
+    import moda_amd
+
+    gen = torch.Generator(device=gpu_device).manual_seed(3)
+    rn = lambda *s: (0.5 * torch.randn(*s, generator=gen, device=gpu_device)).bfloat16()
+    q, k, v, kd, vd = rn(1, 140, 2, 64), rn(1, 70, 2, 64), rn(1, 70, 2, 64), rn(1, 210, 2, 64), rn(1, 210, 2, 64)
+    cu = torch.tensor([0, 30, 70], device=gpu_device)
+    for cls, args in ((moda_amd.ParallelMixtureOfDepthAttentionFunction, [q, k, v, None, None, cu, kd, vd, 2, False]),
+                      (moda_amd.ParallelMixtureOfDepthAttentionChunkVisibleFunction, [q, k, v, None, 0.1, None, kd, vd, 2]),
+                      (moda_amd.ParallelFlashDepthAttentionFunction, [q, None, None, None, None, None, kd, vd, 2]),
+                      (moda_amd.ParallelAttentionFunction, [rn(1, 70, 4, 64), k, v, None, None, cu])):
+        results = []
+        for f in (cls, type("Derived", (cls,), {})):
+            xs = [x.detach().clone().requires_grad_(x.is_floating_point()) if isinstance(x, torch.Tensor) else x for x in args]
+            out = f.apply(*xs)
+            out = out if isinstance(out, tuple) else (out,)
+            grads = torch.autograd.grad(out[0].float().square().sum(), [x for x in xs if isinstance(x, torch.Tensor) and x.requires_grad])
+            results.append([*out, *grads])
+        for a, b in zip(*results):
+            assert torch.equal(a, b), cls.__name__
