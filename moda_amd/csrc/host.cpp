@@ -778,6 +778,8 @@ PYBIND11_MODULE(_host, m) {
     const Extent e = check_shapes(mode, q, value(k), value(v), value(kd), value(vd), G, value(o), value(d_o), value(lse));
     return py::make_tuple(e.T, e.L);
   });
+  m.def("check_folded_contract", [](int mode, const Tensor& q, const OptTensor& k, const OptTensor& cached_k, const OptTensor& cached_v,
+                                    int64_t G) { check_folded_contract(mode, q, value(k), value(cached_k), value(cached_v), G); });
   m.def("attend", &attend);
   m.def("forward", [](int mode, const Tensor& q, const OptTensor& k, const OptTensor& v, const OptTensor& kd, const OptTensor& vd,
                       double scale, int64_t G, int64_t chunk_tokens, std::optional<int64_t> depth_valid,

@@ -37,7 +37,8 @@ class DepthStream:
     the sequence and over everything pushed so far), then ``stream.push(k, v)`` with the layer's
     ``[B, T, H, D]`` tensors (any number of pushes per layer, e.g. K/V projected from the FFN output as
     well).  ``max_layers`` sizes the cache.  ``inplace=None`` keeps one cache in place (with gradient
-    accumulators when gradients flow), ``inplace=False`` rebuilds the cache per layer as the reference does.
+    accumulators when gradients flow), ``inplace=False`` rebuilds the cache per layer as the reference does; so does a
+    stream whose first push ``torch.jit.trace`` records (what writes a cache in place leaves nothing to replay).
 
     ``context()`` -> ``(cached_k, cached_v, depth_valid)`` is the lower-level access for callers that
     invoke ``parallel_moda`` themselves; with gradients flowing it uses the rebuilding path (the in-place
@@ -60,7 +61,7 @@ class DepthStream:
         if self._mode is not None:
             return
         grads = torch.is_grad_enabled() and (k.requires_grad or v.requires_grad)
-        if self._inplace is False or (grads and self._used_context):
+        if self._inplace is False or (grads and self._used_context) or torch.jit.is_tracing():
             self._mode = "rebuild"
         else:
             self._mode = "train" if grads else "infer"
@@ -80,6 +81,8 @@ class DepthStream:
         self._n += 1
 
     def _native(self):
+        if torch.jit.is_tracing():
+            raise RuntimeError("a depth stream that began in place cannot be traced: create it inside the traced function")
         if self._train is None:
             self._train = _lib.host().TrainStream(self.max_layers)
         return self._train
@@ -102,7 +105,8 @@ class DepthStream:
         chunk_visible = chunk_rows is not None
         assert not chunk_visible or is_causal, "chunk-visible attention is causal"
         if self._mode == "train" or (self._mode is None and self._inplace is not False and not self._used_context
-                                     and torch.is_grad_enabled() and (q.requires_grad or k.requires_grad)):
+                                     and not torch.jit.is_tracing() and torch.is_grad_enabled()
+                                     and (q.requires_grad or k.requires_grad)):
             # the same argument contract as parallel_moda, which is bypassed here
             assert q.shape[2] == k.shape[2] and q.shape[1] == k.shape[1] * moda_group_num, \
                 "q must be [B, T*moda_group_num, H, D] for k [B, T, H, D]"
@@ -255,7 +259,8 @@ class MoDAStack(nn.Module):
         no gradient flows; None where the modules have to run one by one.  Twelve blocks of width 256 on 64 x 197
         tokens issue some 200 framework operations of about 10 us host time each when run as modules."""
         attn = self.blocks[0].attn if len(self.blocks) else None
-        if (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or type(attn) is not MoDAAttention
+        if (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing()
+                or type(attn) is not MoDAAttention
                 or nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks
                 or type(x) is not torch.Tensor or x.dim() != 3 or x.shape[-1] != attn.num_heads * attn.head_dim):
             return None

@@ -262,11 +262,15 @@ def _refuse_decay(g, q):
 class _AttentionFunction(torch.autograd.Function):
     """What the four operators' autograd Functions share.  ``apply`` of one of them builds the native node of the same
     computation (csrc/host.cpp, Attend), which costs a tenth of the host time; a class derived from one of them runs
-    its own ``forward`` and ``backward`` as any Function does.  The gradient into ``lse`` is ignored."""
+    its own ``forward`` and ``backward`` as any Function does.  So do all of them while ``torch.jit.trace`` records: a
+    Function is recorded as one operation that runs again on replay, of the native node only its empty output
+    tensors would be.  The gradient into ``lse`` is ignored."""
 
     @classmethod
     def apply(cls, *args, **kwargs):
-        return cls._attend(*args, **kwargs) if cls in _NATIVE_FUNCTIONS else super().apply(*args, **kwargs)
+        if cls in _NATIVE_FUNCTIONS and not torch.jit.is_tracing():
+            return cls._attend(*args, **kwargs)
+        return super().apply(*args, **kwargs)
 
     @staticmethod
     def _run(ctx, mode, q, k, v, cached_k, cached_v, scale, moda_group_num, chunk_tokens, depth_valid, cu_seqlens):
@@ -362,9 +366,14 @@ def parallel_moda(q, k, v, g=None, cached_k=None, cached_v=None, scale=None, cu_
         _warn_depth_grads(cached_k, cached_v)
     if g is not None:
         _refuse_decay(g, q)
-    cu, packed = _offsets(cu_seqlens)
-    out = _lib.host().attend(_lib.CAUSAL if is_causal else _lib.NONCAUSAL, q, k, v, cached_k, cached_v, scale,
-                             moda_group_num, 0, depth_valid, cu, packed, True, 128)
+    mode = _lib.CAUSAL if is_causal else _lib.NONCAUSAL
+    if torch.jit.is_tracing():
+        _lib.host().check_folded_contract(mode, q, k, cached_k, cached_v, moda_group_num)
+        out = ParallelMixtureOfDepthAttentionFunction.apply(q, k, v, None, scale, cu_seqlens, cached_k, cached_v, moda_group_num,
+                                                            is_causal, None, None, None, None, depth_valid)
+    else:
+        cu, packed = _offsets(cu_seqlens)
+        out = _lib.host().attend(mode, q, k, v, cached_k, cached_v, scale, moda_group_num, 0, depth_valid, cu, packed, True, 128)
     return out if need_lse else out[0]
 
 
@@ -456,9 +465,14 @@ def parallel_moda_chunk_visible(q, k, v, g=None, cached_k=None, cached_v=None, s
         _warn_depth_grads(cached_k, cached_v)
     if g is not None:
         _refuse_decay(g, q)
-    cu, packed = _offsets(cu_seqlens)
-    out = _lib.host().attend(_lib.CHUNK_VISIBLE, q, k, v, cached_k, cached_v, scale, moda_group_num,
-                             _chunk_tokens(moda_group_num, chunk_rows), depth_valid, cu, packed, True, 0)
+    if torch.jit.is_tracing():
+        _lib.host().check_folded_contract(_lib.CHUNK_VISIBLE, q, k, cached_k, cached_v, moda_group_num)
+        out = ParallelMixtureOfDepthAttentionChunkVisibleFunction.apply(q, k, v, None, scale, cu_seqlens, cached_k, cached_v,
+                                                                        moda_group_num, chunk_rows, depth_valid)
+    else:
+        cu, packed = _offsets(cu_seqlens)
+        out = _lib.host().attend(_lib.CHUNK_VISIBLE, q, k, v, cached_k, cached_v, scale, moda_group_num,
+                                 _chunk_tokens(moda_group_num, chunk_rows), depth_valid, cu, packed, True, 0)
     return out if need_lse else out[0]
 
 
@@ -538,9 +552,13 @@ def parallel_fda(q, k=None, v=None, g=None, cached_k=None, cached_v=None, scale=
         _warn_depth_grads(cached_k, cached_v)
     if g is not None:
         _refuse_decay(g, q)
-    cu, packed = _offsets(cu_seqlens)
-    out = _lib.host().attend(_lib.DEPTH_ONLY, q, None, None, cached_k, cached_v, scale, moda_group_num, 0, None, cu,
-                             packed, True, 128)
+    if torch.jit.is_tracing():
+        _lib.host().check_folded_contract(_lib.DEPTH_ONLY, q, None, cached_k, cached_v, moda_group_num)
+        out = ParallelFlashDepthAttentionFunction.apply(q, None, None, None, scale, cu_seqlens, cached_k, cached_v, moda_group_num)
+    else:
+        cu, packed = _offsets(cu_seqlens)
+        out = _lib.host().attend(_lib.DEPTH_ONLY, q, None, None, cached_k, cached_v, scale, moda_group_num, 0, None, cu,
+                                 packed, True, 128)
     return out if need_lse else out[0]
 
 

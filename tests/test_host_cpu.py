@@ -443,3 +443,67 @@ def test_operator_functions_are_autograd_functions(monkeypatch):
         order = [xs[i] for i in (0, 1, 2, 6, 7) if i < len(xs)]
         for i, x in enumerate(order):
             assert x is None or (x.grad == 10.0 * (i + 1)).all(), (cls.__name__, i)
+
+
+def test_a_traced_operator_is_recorded_as_an_operation(monkeypatch):
+    """torch.jit.trace records an operator as one operation, which runs again on replay (the native node's launches
+    write through bare pointers: of it only the empty output tensors would be recorded)."""
+    import moda_amd
+    from moda_amd import _lib, ops
+
+    _stub_kernels(monkeypatch)
+    real, replays = _lib.host(), []
+
+    class Host:  # the native call of a replay, on the stand-ins
+        def attend(self, mode, q, k, v, kd, vd, scale, G, *_):
+            replays.append(mode)
+            return ops._raw_fwd(mode, q, k, v, kd, vd, q.shape[-1] ** -0.5 if scale is None else scale, G)
+
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+    monkeypatch.setattr(_lib, "host", lambda host=Host(): host)
+    r = lambda *s: torch.randn(*s, dtype=torch.float64)
+    for f, shapes in (
+            (lambda q, k, v, kd, vd: moda_amd.parallel_moda(q, k, v, cached_k=kd, cached_v=vd, moda_group_num=2), "qkvde"),
+            (lambda q, k, v, kd, vd: moda_amd.parallel_moda_chunk_visible(q, k, v, cached_k=kd, cached_v=vd, moda_group_num=2,
+                                                                          need_lse=True), "qkvde"),
+            (lambda q, kd, vd: moda_amd.parallel_fda(q, cached_k=kd, cached_v=vd, moda_group_num=2), "qde"),
+            (lambda q, k, v: moda_amd.parallel_attn(q, k, v), "kkv")):
+        dims = {"q": (1, 8, 2, 4), "k": (1, 4, 2, 4), "v": (1, 4, 2, 4), "d": (1, 12, 2, 4), "e": (1, 12, 2, 4)}
+        traced = torch.jit.trace(f, tuple(r(*dims[s]) for s in shapes), check_trace=False)
+        assert "^Parallel" in str(traced.graph)
+        xs = [r(*dims[s]) for s in shapes]
+        del replays[:]
+        got, want = traced(*xs), f(*xs)
+        assert len(replays) == 2  # the replay and the eager call
+        for a, b in zip(*((x if isinstance(x, tuple) else (x,)) for x in (got, want))):
+            assert torch.equal(a, b)
+    with pytest.raises(AssertionError, match="T_q must equal T_kv"):  # the argument contract holds while recording
+        torch.jit.trace(lambda q, k: moda_amd.parallel_moda(q, k, k), (r(1, 8, 2, 4), r(1, 4, 2, 4)))
+
+
+def test_a_traced_depth_stream_is_rebuilt_not_written_in_place(monkeypatch):
+    import moda_amd
+    from moda_amd import modules
+
+    monkeypatch.setattr(modules, "stack_depth", lambda xs: torch.stack(xs, 2).flatten(1, 2))
+    monkeypatch.setattr(modules, "parallel_moda", lambda q, k, v, cached_k=None, cached_v=None, **kw:
+                        q + k + v + (0 if cached_k is None else (cached_k + cached_v).sum(1, keepdim=True)))
+
+    def f(q, k, v):
+        s = moda_amd.DepthStream(3)
+        for _ in range(3):
+            q = s.attend(q, k, v)
+            s.push(k, v)
+        return q
+
+    r = lambda: torch.randn(1, 4, 2, 4, dtype=torch.float64, requires_grad=True)
+    traced = torch.jit.trace(f, (r(), r(), r()), check_trace=False)
+    q, k, v = r(), r(), r()
+    d = (k + v).sum(1, keepdim=True)
+    assert torch.allclose(traced(q, k, v), q + 3 * (k + v) + 3 * d)
+    outer = moda_amd.DepthStream(2)  # began in place, outside
+    outer._mode = "train"
+    with pytest.raises(RuntimeError, match="cannot be traced"):
+        torch.jit.trace(lambda q: outer.attend(q, q, q), (r(),))

@@ -1613,3 +1613,46 @@ def test_derived_autograd_functions_match_the_native_node(gpu_device):
             results.append([*out, *grads])
         for a, b in zip(*results):
             assert torch.equal(a, b), cls.__name__
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_traced_callers_replay(gpu_device, grad):
+    """What torch.jit.trace records of the operators, a depth stream and a stack of blocks computes new inputs on replay:
+    the same kernels on the same values, so the eager result bit for bit (the traced stack runs its modules on a
+    rebuilt cache: also against eager on the modules with the rebuilt cache)."""
+    import moda_amd
+
+    gen = torch.Generator(device=gpu_device).manual_seed(8)
+    rn = lambda *s: (0.5 * torch.randn(*s, generator=gen, device=gpu_device)).bfloat16().requires_grad_(grad)
+    new = lambda: (rn(1, 100, 2, 64), rn(1, 50, 2, 64), rn(1, 50, 2, 64), rn(1, 150, 2, 64), rn(1, 150, 2, 64))
+    stack = moda_amd.MoDAStack(128, 3, 2, 1).to(gpu_device, torch.bfloat16).requires_grad_(False)
+
+    def streamed(q, k, v, *_):
+        s = moda_amd.DepthStream(2)
+        outs = []
+        for i in range(2):
+            outs.append(s.attend(q * (i + 1), k, v, moda_group_num=2))
+            s.push(k, v)
+        return tuple(outs)
+
+    calls = (lambda q, k, v, kd, vd: moda_amd.parallel_moda(q, k, v, cached_k=kd, cached_v=vd, moda_group_num=2, need_lse=True),
+             lambda q, k, v, kd, vd: moda_amd.parallel_moda_chunk_visible(q, k, v, cached_k=kd, cached_v=vd, moda_group_num=2),
+             lambda q, k, v, kd, vd: moda_amd.parallel_fda(q, cached_k=kd, cached_v=vd, moda_group_num=2),
+             lambda q, k, v, kd, vd: moda_amd.parallel_attn(q[:, :50], k, v),
+             streamed,
+             lambda q, k, v, kd, vd: stack(q.reshape(1, 100, 128), inplace_cache=None if torch.jit.is_tracing() else False))
+    with torch.set_grad_enabled(grad):
+        for i, f in enumerate(calls):
+            traced = torch.jit.trace(f, new(), check_trace=False)
+            xs = new()
+            for _ in range(2):
+                got, want = traced(*xs), f(*xs)
+                got, want = (x if isinstance(x, tuple) else (x,) for x in (got, want))
+                for a, b in zip(got, want):
+                    assert torch.equal(a, b), i
+            if grad:
+                ga, gb = (torch.autograd.grad(sum(o.float().square().sum() for o in r if o.requires_grad), xs, allow_unused=True)
+                          for r in (got, want))
+                for a, b in zip(ga, gb):
+                    # the two streams add a layer's two gradients up in different orders: a rounding of each and of their sum
+                    assert (a is None and b is None) or (a.float() - b.float()).norm() <= 2.0 ** -7 * b.float().norm(), i
