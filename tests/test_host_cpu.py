@@ -507,3 +507,39 @@ def test_a_traced_depth_stream_is_rebuilt_not_written_in_place(monkeypatch):
     outer._mode = "train"
     with pytest.raises(RuntimeError, match="cannot be traced"):
         torch.jit.trace(lambda q: outer.attend(q, q, q), (r(),))
+
+
+def _native_stack(monkeypatch):
+    """A small stack of blocks whose native forward pass answers with a mark instead of launching anything."""
+    import moda_amd
+    from moda_amd import _lib
+
+    real, mark = _lib.host(), torch.zeros(1)
+
+    class Host:
+        def stack_forward(self, *_):
+            return mark
+
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+    monkeypatch.setattr(_lib, "host", lambda host=Host(): host)
+    return moda_amd.MoDAStack(64, 2, 2, 1).eval(), torch.zeros(1, 4, 64), mark
+
+
+def _runs_modules(model, x):
+    with torch.no_grad(), pytest.raises(RuntimeError, match="no CPU path"):  # the modules' attention says so
+        model(x)
+
+
+def test_stack_of_dual_tensors_is_left_to_the_modules(monkeypatch):
+    """no_grad leaves forward-mode differentiation on: the native forward pass has no tangents, the modules refuse them."""
+    import torch.autograd.forward_ad as fwAD
+
+    model, x, mark = _native_stack(monkeypatch)
+    with torch.no_grad():
+        assert model(x) is mark
+    with fwAD.dual_level():
+        _runs_modules(model, fwAD.make_dual(x, torch.ones_like(x)))
+    with torch.no_grad():
+        assert model(x) is mark

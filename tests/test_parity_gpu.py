@@ -1656,3 +1656,26 @@ def test_traced_callers_replay(gpu_device, grad):
                 for a, b in zip(ga, gb):
                     # the two streams add a layer's two gradients up in different orders: a rounding of each and of their sum
                     assert (a is None and b is None) or (a.float() - b.float()).norm() <= 2.0 ** -7 * b.float().norm(), i
+
+
+def test_forward_mode_tangents_are_refused_not_dropped(gpu_device):
+    """Forward-mode differentiation is not implemented: operators and a stack of blocks refuse a dual input
+    under no_grad too; values without a tangent pass while a level is open."""
+    import torch.autograd.forward_ad as fwAD
+
+    import moda_amd
+
+    x = torch.randn(2, 50, 128, device=gpu_device).bfloat16()
+    stack = moda_amd.MoDAStack(128, 2, 2, 1).to(gpu_device, torch.bfloat16).requires_grad_(False)
+    q = x.view(2, 50, 2, 64)
+    with torch.no_grad():
+        want = stack(x)
+        with fwAD.dual_level():
+            dual = fwAD.make_dual(x, torch.ones_like(x))
+            with pytest.raises(RuntimeError):  # by a module of the stack, which one says so is torch's affair
+                stack(dual)
+            with pytest.raises(RuntimeError, match="jvp"):
+                moda_amd.parallel_moda(dual.view(2, 50, 2, 64), q, q)
+            got = stack(x)
+    # the modules round the layers' results where the native pass does; sums in another order
+    assert (got.float() - want.float()).norm() <= 1.5e-2 * want.float().norm()
