@@ -257,11 +257,12 @@ class MoDAStack(nn.Module):
     def _forward_native(self, x):
         """The whole stack as kernel launches from native code (csrc/host.cpp: stack_forward), for calls through which
         no gradient flows, backward or forward (an open level of forward-mode differentiation: no_grad does not close
-        it); None where the modules have to run one by one.  Twelve blocks of width 256 on 64 x 197
-        tokens issue some 200 framework operations of about 10 us host time each when run as modules."""
+        it), and while nothing watches the framework's operations (a dispatch mode); None where the modules have to
+        run one by one.  Twelve blocks of width 256 on 64 x 197 tokens issue some 200 framework operations of about
+        10 us host time each when run as modules."""
         attn = self.blocks[0].attn if len(self.blocks) else None
         if (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing()
-                or torch.autograd.forward_ad._current_level >= 0 or type(attn) is not MoDAAttention
+                or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() or type(attn) is not MoDAAttention
                 or nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks
                 or type(x) is not torch.Tensor or x.dim() != 3 or x.shape[-1] != attn.num_heads * attn.head_dim):
             return None

@@ -543,3 +543,22 @@ def test_stack_of_dual_tensors_is_left_to_the_modules(monkeypatch):
         _runs_modules(model, fwAD.make_dual(x, torch.ones_like(x)))
     with torch.no_grad():
         assert model(x) is mark
+
+
+def test_stack_under_a_dispatch_mode_is_left_to_the_modules(monkeypatch):
+    """A dispatch mode is there to see the framework's operations, which the native forward pass does not issue."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    seen = []
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    model, x, mark = _native_stack(monkeypatch)
+    with Watch():
+        _runs_modules(model, x)
+    assert any("addmm" in s or "linear" in s for s in seen)
+    with torch.no_grad():
+        assert model(x) is mark
