@@ -5,6 +5,7 @@
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/utils/pybind.h>
 
@@ -374,6 +375,26 @@ Grads backward(const Call& c, Tensor q, Tensor k, Tensor v, Tensor kd, Tensor vd
   return g;
 }
 
+// What a backward node refuses.  The translator at the end of this file sees calls from Python only; the engine that runs
+// the nodes hands a Python error on as it is and makes a RuntimeError of any other.
+[[noreturn]] void throw_python(PyObject* type, const char* what) {
+  py::gil_scoped_acquire gil;
+  PyErr_SetString(type, what);
+  python_error error;
+  error.persist();
+  throw error;
+}
+template <typename F>
+variable_list in_engine(F&& node) {
+  try {
+    return node();
+  } catch (const ContractError& e) {
+    throw_python(PyExc_AssertionError, e.what());
+  } catch (const py::type_error& e) {
+    throw_python(PyExc_TypeError, e.what());
+  }
+}
+
 Tensor value(const OptTensor& x) { return x.has_value() ? *x : Tensor(); }
 OptTensor optional(const Tensor& x) { return x.defined() ? OptTensor(x) : OptTensor(); }
 
@@ -390,6 +411,9 @@ struct Attend : torch::autograd::Function<Attend> {
     return {r.first, r.second};
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    return in_engine([&] { return gradients(ctx, grads); });
+  }
+  static variable_list gradients(AutogradContext* ctx, const variable_list& grads) {
     const variable_list s = ctx->get_saved_variables();
     const auto call = c10::static_intrusive_pointer_cast<Call>(ctx->saved_data["call"].toCapsule());
     if (!grads[0].defined()) return variable_list(6);
@@ -521,6 +545,9 @@ struct StreamAttend : torch::autograd::Function<StreamAttend> {
     return {r.first, order_token(q)};
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
+    return in_engine([&] { return gradients(ctx, grads); });
+  }
+  static variable_list gradients(AutogradContext* ctx, const variable_list& grads) {
     const variable_list s = ctx->get_saved_variables();
     const auto call = c10::static_intrusive_pointer_cast<StreamCall>(ctx->saved_data["call"].toCapsule());
     StreamBuffers& buf = *call->buf;

@@ -1679,3 +1679,28 @@ def test_forward_mode_tangents_are_refused_not_dropped(gpu_device):
             got = stack(x)
     # the modules round the layers' results where the native pass does; sums in another order
     assert (got.float() - want.float()).norm() <= 1.5e-2 * want.float().norm()
+
+
+def test_what_a_backward_refuses_arrives_as_the_same_exception(gpu_device):
+    """A violated argument contract is an AssertionError, mixed dtypes are a TypeError, in a backward pass (here: saved
+    tensors that come back changed) as in a call.  Everything is refused before a launch."""
+    import moda_amd
+
+    rn = lambda *s: torch.randn(*s, device=gpu_device).bfloat16().requires_grad_()
+
+    def operator(q, k, v):
+        return moda_amd.parallel_moda(q, k, v, moda_group_num=2)
+
+    def stream(q, k, v):
+        s = moda_amd.DepthStream(1)
+        o = s.attend(q, k, v, moda_group_num=2)
+        s.push(k, v)
+        return o
+
+    for call in (operator, stream):
+        for change, error, match in ((lambda x: x.float(), TypeError, "share one dtype"),
+                                     (lambda x: x[:, :32], AssertionError, "expected T\\*moda_group_num")):
+            with torch.autograd.graph.saved_tensors_hooks(lambda x: x, lambda x: change(x) if x.shape[1] == 64 else x):
+                o = call(rn(1, 128, 2, 64), rn(1, 64, 2, 64), rn(1, 64, 2, 64))
+            with pytest.raises(error, match=match):
+                o.float().sum().backward()
