@@ -7,6 +7,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <array>
@@ -515,11 +516,19 @@ void depth_push(const Tensor& k_in, const Tensor& v_in, const Tensor& cache_k, c
 }
 
 // Cache and gradient buffers of one forward / backward pass, [B, T * L, H, D] each, allocated by the first push and never
-// initialised: slots are read once written.  The backward calls run from the last layer to the first; the first of
-// them overwrites the gradients of the slots it saw (`written`), the others, which saw fewer, add to theirs.
+// initialised: slots are read once written.  The nodes of a backward pass run from the last layer to the first; the first
+// attention call among them overwrites the gradients of the slots it saw (`written`), the others, which saw fewer, add to
+// theirs.  Another pass over a retained graph starts over, however much of the stream the one before it reached.
 struct StreamBuffers : torch::CustomClassHolder {
   Tensor k, v, gk, gv;
   int64_t L = 0, written = 0;
+  int pass = -1;  // the engine's number of the pass that `written` is about
+
+  void enter_pass() {
+    const int id = torch::autograd::get_current_graph_task_id();
+    if (id != pass) written = 0;
+    pass = id;
+  }
 };
 // An attention call of the stream: what it saw, and the slot its own k, v were pushed to afterwards (-1: none).
 struct StreamCall : torch::CustomClassHolder {
@@ -551,6 +560,7 @@ struct StreamAttend : torch::autograd::Function<StreamAttend> {
     const variable_list s = ctx->get_saved_variables();
     const auto call = c10::static_intrusive_pointer_cast<StreamCall>(ctx->saved_data["call"].toCapsule());
     StreamBuffers& buf = *call->buf;
+    buf.enter_pass();
     const Tensor &q = s[0], &k = s[1], &v = s[2], &o = s[3], &lse = s[4];
     const Tensor d_o = grads[0].defined() ? grads[0].to(o.scalar_type()) : at::zeros_like(o);
     const int64_t n = call->n;
@@ -593,7 +603,8 @@ struct StreamPush : torch::autograd::Function<StreamPush> {
   }
   static variable_list backward(AutogradContext* ctx, const variable_list&) {
     const auto call = c10::static_intrusive_pointer_cast<StreamCall>(ctx->saved_data["call"].toCapsule());
-    const StreamBuffers& buf = *call->buf;
+    StreamBuffers& buf = *call->buf;
+    buf.enter_pass();
     const int64_t B = buf.k.size(0), T = buf.k.size(1) / buf.L, H = buf.k.size(2), D = buf.k.size(3);
     auto slot = [&](const Tensor& g) {
       if (call->slot >= buf.written) return at::zeros({B, T, H, D}, g.options());

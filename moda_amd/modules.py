@@ -42,7 +42,7 @@ class DepthStream:
 
     ``context()`` -> ``(cached_k, cached_v, depth_valid)`` is the lower-level access for callers that
     invoke ``parallel_moda`` themselves; with gradients flowing it uses the rebuilding path (the in-place
-    gradient path needs ``attend``).  One backward pass per forward pass: the accumulators are consumed by it."""
+    gradient path needs ``attend``).  Each backward pass over the stream's graph fills the accumulators anew."""
 
     def __init__(self, max_layers: int, inplace: Optional[bool] = None):
         self.max_layers = int(max_layers)

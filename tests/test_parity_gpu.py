@@ -1704,3 +1704,47 @@ def test_what_a_backward_refuses_arrives_as_the_same_exception(gpu_device):
                 o = call(rn(1, 128, 2, 64), rn(1, 64, 2, 64), rn(1, 64, 2, 64))
             with pytest.raises(error, match=match):
                 o.float().sum().backward()
+
+
+@pytest.mark.parametrize("case", [
+    # B, T, H, G, D, dtype: own slots joined in the dK/dV launch, in a launch of their own, fp32
+    (2, 50, 1, 4, 64, torch.bfloat16),
+    (1, 70, 2, 2, 128, torch.bfloat16),
+    (1, 40, 2, 2, 64, torch.float32),
+])
+def test_every_backward_pass_over_a_stream_is_its_own(gpu_device, case):
+    """Passes over a retained graph, the first of them from an early layer: each returns what the same pass over stacked
+    caches does (bounds: test_stream_layers_join_their_slot_gradient; fp32: sums in another order).  The gradient buffers
+    are not initialised, and a later pass reaches slots that no earlier one wrote: they are filled with NaN by hand."""
+    import moda_amd
+
+    B, T, H, G, D, dtype = case
+    say(f"CASE stream passes {case}")
+    gen = torch.Generator(device=gpu_device).manual_seed(6)
+    rn = lambda *s: (0.5 * torch.randn(*s, generator=gen, device=gpu_device)).to(dtype).requires_grad_(True)
+    layers = [(rn(B, T * G, H, D), rn(B, T, H, D), rn(B, T, H, D)) for _ in range(4)]
+    # K/V that no attention call saw go into the stream between the third and the fourth layer
+    extra = (rn(B, T, H, D), rn(B, T, H, D))
+    flat = [x for layer in layers for x in layer] + list(extra)
+    do = [rn(B, T * G, H, D).detach() for _ in range(4)]
+    poison = [torch.full((B, T * 5, H, D), float("nan"), dtype=dtype, device=gpu_device) for _ in range(4)]
+    del poison  # the stream's buffers come from this memory
+    stream, outs = moda_amd.DepthStream(5), []
+    for i, (q, k, v) in enumerate(layers):
+        outs.append(stream.attend(q, k, v, moda_group_num=G, is_causal=False))
+        stream.push(k, v)
+        if i == 2:
+            stream.push(*extra)
+    seen, want = [], []
+    for i, (q, k, v) in enumerate(layers):
+        kd, vd = (moda_amd.stack_depth([l[j] for l in seen]) if seen else None for j in (0, 1))
+        want.append(moda_amd.parallel_moda(q, k, v, cached_k=kd, cached_v=vd, moda_group_num=G, is_causal=False))
+        seen += [(k, v)] + ([extra] if i == 2 else [])
+    bound = 2.0 ** -7 if dtype is torch.bfloat16 else 2e-6
+    for upto in (2, 4, 1, 3, 4):
+        got, ref = (torch.autograd.grad(o[:upto], flat, do[:upto], retain_graph=True, allow_unused=True) for o in (outs, want))
+        for i, (a, b) in enumerate(zip(got, ref)):
+            if b is None:  # the stream's order edges may reach further: what they bring is nothing
+                assert a is None or not a.any(), (upto, i)
+            else:
+                assert (a.float() - b.float()).norm() <= bound * b.float().norm(), (upto, i)
