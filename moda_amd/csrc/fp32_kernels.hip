@@ -89,6 +89,46 @@ __device__ __forceinline__ void accumulate(f32x4 (&acc)[HD / 64][4], const f32x4
       for (int j = 0; j < 4; j++) acc[h][j] = mfma_f32(x[i][h][j], w[i], acc[h][j]);
 }
 
+// The same where not every column sees every row (`see`: the lane's column sees row 4 q + i).  The weight of an unseen
+// pair is zero, which takes a finite row out of the product but not one with an infinity or a NaN in it: 0 x those is
+// NaN, and a later token's value would reach an earlier token's result.  A block that holds such a value is added up
+// pair by pair, unseen pairs left out.  Finding out costs HD / 4 vector instructions beside HD / 4 matrix instructions
+// of 32 cycles, in blocks on an edge of what is visible and in depth blocks only.
+template <int HD>
+__device__ __forceinline__ void accumulate_seen(f32x4 (&acc)[HD / 64][4], const f32x4 (&x)[4][HD / 64], const f32x4& w, const bool (&see)[4],
+                                                int n, int q) {
+  float z = 0.f;
+  if (!__all(see[0] && see[1] && see[2] && see[3]))
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int h = 0; h < HD / 64; h++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) z = __builtin_fmaf(x[i][h][j], 0.f, z);
+  if (!__any(z != 0.f)) {  // NaN as soon as one of them is not finite
+    accumulate<HD>(acc, x, w);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+#pragma unroll 1
+    for (int g = 0; g < 4; g++) {  // row 4 g + i; its element 64 h + 16 q + 4 m + j is with lane 4 q + m of the rows' group g
+      const float weight = __shfl(w[i], 16 * g + n, 64);
+      const bool seen = __shfl((int)see[i], 16 * g + n, 64) != 0;
+#pragma unroll
+      for (int h = 0; h < HD / 64; h++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+#pragma unroll
+          for (int m = 0; m < 4; m++) {
+            const float v = __shfl(x[i][h][j], 16 * g + 4 * q + m, 64);
+            acc[h][j][m] = seen ? __builtin_fmaf(v, weight, acc[h][j][m]) : acc[h][j][m];
+          }
+          __builtin_amdgcn_sched_barrier(0);  // a few values at a time: the registers of this path are those of the kernel
+        }
+    }
+}
+
 template <int HD>
 __device__ __forceinline__ void clear(f32x4 (&acc)[HD / 64][4]) {
 #pragma unroll
@@ -219,7 +259,7 @@ __global__ __launch_bounds__(64 * kFp32RowWaves, 2) void fp32_fwd_kernel(const K
       p[i] = see[i] ? exp2f(s[i] - ref) : 0.f;
       l += p[i];
     }
-    accumulate<HD>(o, V, p);
+    accumulate_seen<HD>(o, V, p, see, n, q);
   }
   l = quad_sum_f32(l);
   leave_partial<HD>(part + wave * 16 * kPartRow<HD>, o, n, q);
@@ -312,12 +352,14 @@ __global__ __launch_bounds__(64 * kFp32RowWaves, 2) void fp32_dq_kernel(const KA
     __builtin_amdgcn_sched_barrier(0);
     const int lo = x.dep ? vis.dlo : 0, hi = x.dep ? vis.dhi : vis.shi;
     f32x4 ds;
+    bool see[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int c = x.col0 + 4 * q + i;
-      ds[i] = (c >= lo && c < hi) ? exp2f(__builtin_fmaf(s[i], sc, -lse)) * dp[i] : 0.f;
+      see[i] = c >= lo && c < hi;
+      ds[i] = see[i] ? exp2f(__builtin_fmaf(s[i], sc, -lse)) * dp[i] : 0.f;
     }
-    accumulate<HD>(dq, KT, ds);
+    accumulate_seen<HD>(dq, KT, ds, see, n, q);
   }
   leave_partial<HD>(part + wave * 16 * kPartRow<HD>, dq, n, q);
   __syncthreads();
@@ -427,16 +469,18 @@ __global__ __launch_bounds__(64 * kFp32ColWaves<HD>, HD <= 64 ? 2 : 1) void fp32
     const f32x4 s = scores<HD>(Q, K, f32x4{0.f, 0.f, 0.f, 0.f});
     const f32x4 dp = scores<HD>(dO, V, f32x4{neg_delta[0], neg_delta[1], neg_delta[2], neg_delta[3]});
     f32x4 p, ds;
+    bool see[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int r = x.r0 + 4 * q + i;
-      p[i] = (r >= qlo && r < qhi) ? exp2f(__builtin_fmaf(s[i], sc, -lse[i])) : 0.f;
-      ds[i] = p[i] * dp[i];
+      see[i] = r >= qlo && r < qhi;
+      p[i] = see[i] ? exp2f(__builtin_fmaf(s[i], sc, -lse[i])) : 0.f;
+      ds[i] = see[i] ? p[i] * dp[i] : 0.f;
     }
     if (blk + step < nblk) load_rows(blk + step);
     __builtin_amdgcn_sched_barrier(0);
-    accumulate<HD>(dv, dOT, p);
-    accumulate<HD>(dk, QT, ds);
+    accumulate_seen<HD>(dv, dOT, p, see, n, q);
+    accumulate_seen<HD>(dk, QT, ds, see, n, q);
   }
 
   if (dep) {

@@ -1748,3 +1748,51 @@ def test_every_backward_pass_over_a_stream_is_its_own(gpu_device, case):
                 assert a is None or not a.any(), (upto, i)
             else:
                 assert (a.float() - b.float()).norm() <= bound * b.float().norm(), (upto, i)
+
+
+@pytest.mark.parametrize("case", [
+    # T, D, L, G, mode, chunk_tokens: head dims at both tile widths and padded, several waves' blocks, ragged edges
+    (70, 64, 3, 2, "causal", 0),
+    (150, 128, 2, 1, "causal", 0),
+    (41, 36, 5, 4, "noncausal", 0),
+    (90, 64, 2, 2, "chunk_visible", 16),
+    (50, 128, 20, 3, "depth_only", 0),
+    (40, 160, 2, 2, "causal", 0),   # the vector-ALU kernels
+])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_fp32_non_finite_values_stay_with_the_rows_that_see_them(gpu_device, case, value):
+    """A NaN or an infinity in one row of one input reaches only what depends on it by the visible mask: the output rows
+    that see the column, the gradients of those rows, and of the columns such a row sees.  Everything else is what it is
+    without the value (sums in another order: a few roundings of 6e-8)."""
+    T, D, L, G, mode, cb = case
+    say(f"CASE fp32 non-finite {case} {value}")
+    inp = to_dev(oracle.make_inputs(1, T, 1, D, L, G, seed=17, dtype=torch.float32, std=0.5, depth_only=mode == "depth_only"), gpu_device)
+    vis = oracle.visible_mask(T, G, L, mode, cb).to(gpu_device)  # [rows, T + T * L], depth-only: no sequence column seen
+    clean = run_hip(inp, D ** -0.5, G, mode, cb)
+    t0 = T // 2 + 3
+    for name, row in (("k", t0), ("v", t0), ("kd", t0 * L + L - 1), ("vd", t0 * L), ("q", t0 * G + G - 1), ("do", t0 * G)):
+        if inp[name] is None:
+            continue
+        bad = dict(inp)
+        bad[name] = inp[name].clone()
+        bad[name][0, row, 0, D // 3] = value
+        got = run_hip(bad, D ** -0.5, G, mode, cb)
+        rows = torch.zeros(T * G, dtype=torch.bool, device=gpu_device)  # rows whose output may differ
+        if name in ("k", "v", "kd", "vd"):
+            rows = vis[:, row if name in ("k", "v") else T + row].clone()
+        elif name == "q":
+            rows[row] = True
+        back = rows.clone()  # ... and whose gradient may
+        if name == "do":
+            back[row] = True
+        cols = vis[back].any(0)
+        if name in ("k", "v", "kd", "vd"):
+            cols[row if name in ("k", "v") else T + row] = True
+        hit = {"o": rows, "lse": rows, "dq": back, "dk": cols[:T], "dv": cols[:T], "dkd": cols[T:], "dvd": cols[T:]}
+        assert value == value or name in ("do", "k", "kd", "q") or not torch.isfinite(got["o"][0, rows]).all(-1).any()
+        for n, mask in hit.items():
+            if clean[n] is None:
+                continue
+            a, b = got[n][0, ~mask].float(), clean[n][0, ~mask].float()
+            assert torch.isfinite(a).all(), (name, n)
+            assert (a - b).abs().max() <= 1e-5 * clean[n].abs().max() if a.numel() else True, (name, n)
