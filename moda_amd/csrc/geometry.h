@@ -222,16 +222,18 @@ inline bool dkv_flat_row_waves(const KArgs& a) {
 // ms; head dim 64, 64 heads: 10.4 -> 10.9 ms).  Below that:
 // dkv_kernel, fixed length: the same power of two for every tile, segments of the heaviest of at least 16 trips (a trip:
 // one query tile of one query head).  3057 tokens, 32 query heads on four: 538 -> 430 us when the heads count as trips.
-// Packed batches and dkv_flat_kernel: segments of equal length, three quarters of a place's share of all trips (0.35 to 1
-// measure within 4 %).  A packed batch counts as one of equal, longest sequences.  Eight sequences of 200 - 3000
-// tokens, head dim 64: 974 -> 705 us; five of 168 - 2600, head dim 128: 651 -> 242 us; 6000 tokens, four heads of
-// four, head dim 64: 497 -> 430 us.
+// dkv_kernel, packed, tiles wider than 64: not cut.  There a packed batch returns bit for bit what separate calls return
+// that have no room for segments, and that is kept although the cut is faster (a training step of 2600 + 168 + 900 + 400
+// + 1500 tokens, four heads of four, eight slots: 329 us cut, 435 not; of 6000 + 3000 + 500, two heads of four: 641, 894).
+// The rest (dkv_flat_kernel; packed batches on the 64-wide tiles): segments of equal length, three quarters of a place's
+// share of all trips (0.35 to 1 measure within 4 %).  A packed batch counts as one of equal, longest sequences.  Eight
+// sequences of 200 - 3000 tokens, head dim 64: 974 -> 705 us; 6000 tokens, four heads of four, head dim 64: 497 -> 430 us.
 struct DkvSplit {
   int nseg, seg_tiles;
 };
 inline DkvSplit dkv_split_plan(const KArgs& a, int HD) {
   const bool flat = takes_dkv_flat(a, HD);
-  if (!a.has_seq || a.T == 0 || (flat && dkv_flat_row_waves(a))) return {1, 0};
+  if (!a.has_seq || a.T == 0 || (flat && dkv_flat_row_waves(a)) || (a.cu && HD > 64)) return {1, 0};
   const int BN = HD > 128 ? 64 : 128, BM = flat || HD > 128 ? 32 : 64;
   const int64_t tiles = (int64_t)((a.T + BN - 1) / BN) * a.Hkv * (a.cu ? imax(1, part_rows(a) / a.T) : a.B);
   const int64_t nqt = (a.Tq + BM - 1) / BM;

@@ -163,10 +163,12 @@ def test_row_split_launch(walker):
     ((2048,), 2, 128, 2, 4, "causal", 0, False, 1, True),
     ((1100,), 2, 64, 0, 4, "causal", 0, False, 1, True),        # 64-wide tiles, ragged last tile
     ((1000,), 3, 64, 2, 2, "noncausal", 0, False, 1, True),     # more than 1024 query rows: no row waves
-    ((3000, 1, 300, 0, 777), 1, 128, 2, 4, "causal", 0, True, 1, True),
+    ((3000, 1, 300, 0, 777), 1, 128, 2, 4, "causal", 0, True, 1, False),  # packed on the wider tiles: one pass
     ((3000, 130, 64, 0, 1), 1, 64, 2, 4, "causal", 0, True, 1, True),
-    ((1500, 700), 1, 96, 0, 8, "plain", 0, True, 1, True),      # head-dim GQA, padded head dim
-    ((900, 100), 1, 128, 2, 8, "chunk_visible", 40, True, 1, True),  # sequence segments and depth column tiles in one launch
+    ((1500, 700), 1, 96, 0, 8, "plain", 0, True, 1, False),     # head-dim GQA, padded head dim
+    ((1500, 700), 1, 48, 0, 8, "plain", 0, True, 1, True),      # ... on the 64-wide tiles
+    ((900, 100), 1, 128, 2, 8, "chunk_visible", 40, True, 1, False),
+    ((900, 100), 1, 64, 2, 8, "chunk_visible", 40, True, 1, True),   # sequence segments and depth column tiles in one launch
     ((197,), 1, 64, 3, 4, "noncausal", 0, False, 5, False),     # row waves
     ((250,), 2, 64, 0, 4, "causal", 0, False, 3, False),        # ... with a diagonal
     ((33,), 1, 40, 2, 3, "noncausal", 0, False, 2, False),      # ... one short query tile, padded head dim

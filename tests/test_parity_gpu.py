@@ -1137,7 +1137,8 @@ def test_random_sweep_packed(gpu_device, seed):
 
 
 @pytest.mark.parametrize("case", [
-    # long sequences in a small batch: their key tiles are cut along the query rows, those of the short ones are not
+    # long sequences in a small batch: on the 64-wide tiles their key tiles are cut along the query rows, those of the
+    # short ones are not
     ((1700, 0, 1, 130), 1, 128, 2, 2, "causal", 0, torch.bfloat16),
     ((1700, 65, 300), 1, 64, 2, 2, "causal", 0, torch.float16),
     ((700, 129), 2, 64, 0, 4, "noncausal", 0, torch.bfloat16),
@@ -1170,6 +1171,41 @@ def test_packed_batch_equals_separate_calls_bitwise(gpu_device):
         assert torch.equal(o[:, a * G:b * G], one["o"]) and torch.equal(lse[:, a * G:b * G], one["lse"]), i
         for n, key in (("q", "dq"), ("k", "dk"), ("v", "dv"), ("kd", "dkd"), ("vd", "dvd")):
             assert torch.equal(leaf[n].grad[:, a * mult[n]:b * mult[n]], one[key]), (i, n)
+
+
+@pytest.mark.parametrize("case", [
+    # lengths, H, D, L, G, mode, chunk: few key tiles, long enough that a fixed-length call of theirs is cut
+    ((1700, 0, 1, 130), 1, 128, 2, 2, "causal", 0),
+    ((1000, 33), 1, 96, 2, 4, "chunk_visible", 40),
+    ((900, 1300), 2, 128, 0, 4, "noncausal", 0),
+    ((700, 64), 1, 160, 3, 4, "causal", 0),
+], ids=lambda c: f"{c[5]}-{'_'.join(map(str, c[0]))}-D{c[2]}")
+def test_small_packed_batches_of_long_sequences_equal_separate_calls_bitwise(gpu_device, case):
+    """Head dims above 64: every result of a packed batch is, bit for bit, that of separate calls whose workspace has no
+    room for row segments."""
+    import moda_amd
+
+    lengths, H, D, L, G, mode, cb = case
+    cu = _cu(lengths)
+    inp = to_dev(oracle.make_inputs(1, cu[-1], H, D, L, G, seed=43, dtype=torch.bfloat16, std=0.5), gpu_device)
+    leaf = {n: inp[n].clone().requires_grad_(True) for n in ("q", "k", "v", "kd", "vd") if inp[n] is not None}
+    common = dict(cached_k=leaf.get("kd"), cached_v=leaf.get("vd"), moda_group_num=G, need_lse=True,
+                  cu_seqlens=torch.tensor(cu, device=gpu_device))
+    if mode == "chunk_visible":
+        o, lse = moda_amd.parallel_moda_chunk_visible(leaf["q"], leaf["k"], leaf["v"], chunk_rows=cb * G, **common)
+    else:
+        o, lse = moda_amd.parallel_moda(leaf["q"], leaf["k"], leaf["v"], is_causal=mode == "causal", **common)
+    o.backward(inp["do"])
+    mult = {"q": G, "k": 1, "v": 1, "kd": L, "vd": L}
+    for a, b in zip(cu[:-1], cu[1:]):
+        if a == b:
+            continue
+        part = {n: None if inp[n] is None else inp[n][:, a * m:b * m] for n, m in mult.items()}
+        part["do"] = inp["do"][:, a * G:b * G]
+        one = run_hip(part, D ** -0.5, G, mode, cb, row_sums_only=D > 128, no_row_split=D <= 128)
+        assert torch.equal(o[:, a * G:b * G], one["o"]) and torch.equal(lse[:, a * G:b * G], one["lse"]), (a, b)
+        for n, x in leaf.items():
+            assert torch.equal(x.grad[:, a * mult[n]:b * mult[n]], one["d" + n]), (a, b, n)
 
 
 def test_packed_batch_on_the_narrow_tiles_against_separate_calls(gpu_device):
