@@ -675,16 +675,33 @@ struct Block {
   double eps1, eps2;
 };
 
+// Whether the blocks run as native launches, by who is faster (four blocks, 64 .. 50 432 tokens, times of the modules over
+// ours).  Up to width 512 we are: 1.2 - 3.9, replayed from a captured graph 1.13 - 1.6.  Above, the library's products are the
+// faster kernels (width 1024, 12 608 tokens: 2246 against 1915 us; 2048: 7.6 against 5.6 ms; 4096, 197 tokens: 2294 against 908
+// us), and what is left to gain is the modules' host time, some 170 us a block, where that is more than the launches take:
+// width 1024 up to 3 152 tokens 1.1 - 2.1, 1280 up to 788 tokens 1.4 - 1.75 (3 152: 0.81), 1536 up to 197 tokens 1.16 - 1.5 (788:
+// 0.97).  A captured graph has no host time: 1024 at 197 tokens replays at 0.89.
+bool stack_runs_native(int64_t rows, int64_t width, void* stream) {
+  if (width <= 512) return true;
+  if (rows * width > (width <= 1024 ? 3 << 20 : width <= 1536 ? 1 << 20 : 0)) return false;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing((hipStream_t)stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+}
+
 // Forward pass of all blocks of one stack, launches only: the residual stream, one depth cache and four work tensors
 // are all there is.  A layer's K and V are projected straight into their slot of the cache, where its own attention reads
 // them as the sequence and later layers as a depth slot.  Returns nothing where a kernel's contract is not met (the
-// caller then runs the modules one by one): 16-bit types, widths the linear kernel takes, 16-byte rows.
+// caller then runs the modules one by one): 16-bit types, widths the linear kernel takes, 16-byte rows; or where the
+// modules are faster.
 std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>& blocks, int64_t heads, int64_t kv_heads, bool is_causal,
                                     int64_t chunk_tokens, bool post_norm) {
   const auto type = x_in.scalar_type();
   if (!x_in.is_cuda() || x_in.dim() != 3 || (type != at::kBFloat16 && type != at::kHalf) || x_in.numel() == 0) return {};
   const int64_t B = x_in.size(0), N = x_in.size(1), C = x_in.size(2), hd = C / heads, kv = kv_heads * hd, M = B * N;
-  if (hd % 8 != 0 || hd > 256 || C % 64 != 0 || C > 4096) return {};
+  if (hd % 8 != 0 || hd > 256 || C % 64 != 0) return {};
+  c10::OptionalDeviceGuard guard(x_in.device());
+  void* stream = stream_of(x_in);
+  if (!stack_runs_native(M, C, stream)) return {};
   const int64_t hidden = blocks[0].fc1_w.size(0);
   auto fits = [&](const Tensor& x, std::initializer_list<int64_t> shape) {
     return x.defined() && has_shape(x, shape) && x.scalar_type() == type && x.device() == x_in.device() && x.is_contiguous() &&
@@ -701,8 +718,6 @@ std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>
       return {};
     L += b.kv_ffn_w.defined() ? 2 : 1;
   }
-  c10::OptionalDeviceGuard guard(x_in.device());
-  void* stream = stream_of(x_in);
   const int dt = type == at::kHalf ? MODA_HIP_FP16 : MODA_HIP_BF16;
   const int64_t es = 2;
   const auto opt = x_in.options().requires_grad(false);

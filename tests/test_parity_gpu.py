@@ -1832,3 +1832,44 @@ def test_fp32_non_finite_values_stay_with_the_rows_that_see_them(gpu_device, cas
             a, b = got[n][0, ~mask].float(), clean[n][0, ~mask].float()
             assert torch.isfinite(a).all(), (name, n)
             assert (a - b).abs().max() <= 1e-5 * clean[n].abs().max() if a.numel() else True, (name, n)
+
+
+@pytest.mark.parametrize("case", [
+    # width, heads, batch, tokens, mlp ratio, native in an eager call, in a captured one
+    (512, 8, 3, 150, 4.0, True, True),
+    (576, 9, 2, 70, 3.0, True, False),
+    (768, 12, 4, 1024, 1.0, True, False),      # 768 * 4096 = 3 * 2^20
+    (768, 12, 1, 4097, 1.0, False, False),
+    (1024, 8, 1, 197, 4.0, True, False),
+    (1536, 12, 1, 600, 2.0, True, False),
+    (1536, 12, 1, 700, 1.0, False, False),
+    (1600, 8, 1, 10, 1.0, False, False),
+])
+def test_stack_widths_and_which_of_them_run_as_native_launches(gpu_device, case):
+    """The rule by size, and both ways through the blocks against the same blocks in fp32 on the same 16-bit weights: the
+    native pass rounds where the modules round, so neither is further off than the other by more than noise."""
+    import moda_amd
+
+    C, heads, B, N, ratio, eager, captured = case
+    say(f"CASE stack widths {case}")
+    torch.manual_seed(1)
+    m = moda_amd.MoDAStack(C, 2, heads, heads, mlp_ratio=ratio).to(gpu_device, torch.bfloat16).eval()
+    x = (0.5 * torch.randn(B, N, C, device=gpu_device)).bfloat16()
+    with torch.no_grad():
+        y = m._forward_native(x)
+        assert (y is not None) == eager
+        m(x)
+        torch.cuda.synchronize()
+        with torch.cuda.graph(torch.cuda.CUDAGraph()):
+            again = m._forward_native(x)
+            assert (again is not None) == captured
+        stream = moda_amd.DepthStream(2)
+        z = x
+        for blk in m.blocks:
+            a, k, v = blk.attn(blk.norm1(z), stream=stream)
+            z = z + a
+            z = z + blk.mlp(blk.norm2(z))
+            stream.push(k, v)
+        exact = m.float()(x.float())
+    off = lambda t: ((t.float() - exact).norm() / exact.norm()).item()
+    assert off(m.bfloat16()(x) if y is None else y) <= max(1.1 * off(z), 2.0 ** -8), (off(z), y is None or off(y))
