@@ -1873,3 +1873,40 @@ def test_stack_widths_and_which_of_them_run_as_native_launches(gpu_device, case)
         exact = m.float()(x.float())
     off = lambda t: ((t.float() - exact).norm() / exact.norm()).item()
     assert off(m.bfloat16()(x) if y is None else y) <= max(1.1 * off(z), 2.0 ** -8), (off(z), y is None or off(y))
+
+
+def _linear(x, parts, residual=None, gelu=False, ldx=None, K=None):
+    """moda_hip_linear through the C entry point; parts: (w, bias, y).  Returns its code."""
+    import ctypes
+
+    from moda_amd import _lib
+
+    class Part(ctypes.Structure):
+        _fields_ = [("w", ctypes.c_void_p), ("bias", ctypes.c_void_p), ("y", ctypes.c_void_p), ("ldy", ctypes.c_int64), ("n", ctypes.c_int64)]
+
+    arr = (Part * len(parts))(*(Part(w.data_ptr(), None if b is None else b.data_ptr(), y.data_ptr(), y.stride(0), w.shape[0]) for w, b, y in parts))
+    i64, ptr = ctypes.c_int64, ctypes.c_void_p
+    return _lib.load().moda_hip_linear(
+        {torch.bfloat16: 0, torch.float16: 1}[x.dtype], i64(x.shape[0]), i64(x.shape[1] if K is None else K), ptr(x.data_ptr()),
+        i64(x.stride(0) if ldx is None else ldx), arr, len(parts), ptr(None if residual is None else residual.data_ptr()),
+        i64(0 if residual is None else residual.stride(0)), int(gelu), ptr(torch.cuda.current_stream().cuda_stream))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gelu_over_the_whole_range(gpu_device, dtype):
+    """The fused GELU of every 16-bit value (given as a bias onto a zero product) against fp64: one rounding of the result,
+    2^-8 or 2^-11 relative, beside the fit's error, or half of the smallest result there is; infinities and NaN
+    as torch has them."""
+    v = torch.arange(-32768, 32768, device=gpu_device).to(torch.int16).view(dtype)
+    x, w = torch.zeros(3, 64, device=gpu_device, dtype=dtype), torch.randn(v.numel(), 64, device=gpu_device).to(dtype)
+    y = torch.empty(3, v.numel(), device=gpu_device, dtype=dtype)
+    assert _linear(x, [(w, v, y)], gelu=True) == 0
+    want = 0.5 * v.double() * torch.special.erfc(v.double() * -0.5 ** 0.5)  # (1 + erf cancels in the lower tail)
+    like = torch.nn.functional.gelu(v.float())
+    for row in y:
+        assert torch.equal(row.isnan(), like.isnan()) and torch.equal(row.isinf(), like.to(dtype).isinf())
+        ok = like.isfinite() & like.to(dtype).isfinite()
+        rel = 2.0 ** -8 if dtype is torch.bfloat16 else 2.0 ** -11
+        tiny = 2.0 ** -25 if dtype is torch.float16 else 2.0 ** -126  # bf16: fp32's subnormals are flushed
+        err = (row.double() - want).abs()[ok]
+        assert (err <= (rel + 8e-6) * want.abs()[ok] + tiny).all(), (err - (rel + 8e-6) * want.abs()[ok]).max()
