@@ -262,7 +262,7 @@ int moda_hip_depth_slot_add(void* dk, void* dv, const moda_hip_strides* sdk, con
  * contiguous; each output [rows, n] with row stride ldy), then optionally the exact GELU, or a residual
  * (same shape and row stride ld_res) added to the rounded result.  K a multiple of 64, n of 8,
  * x, W, y, residual rows on 16-byte boundaries (bias: 8 bytes); MODA_HIP_EUNSUPPORTED / MODA_HIP_EALIGN otherwise.
- * `residual` may be the output itself (single part).
+ * `residual` may be the output itself (single part, no GELU: MODA_HIP_EINVAL otherwise).
  * moda_hip_layer_norm: y = (x - mean) / sqrt(var + eps) * weight + bias over rows of `dim` (a multiple of 8, at most 4096).
  */
 typedef struct moda_hip_linear_part {

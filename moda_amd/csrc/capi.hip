@@ -541,7 +541,7 @@ int moda_hip_linear(int32_t dtype, int64_t rows, int64_t K, const void* x, int64
                     const void* residual, int64_t ld_res, int32_t gelu, void* stream) {
   if ((dtype != MODA_HIP_BF16 && dtype != MODA_HIP_FP16) || rows < 0 || K <= 0 || n_parts < 1 || n_parts > 3 || !parts) return MODA_HIP_EINVAL;
   if (rows == 0) return MODA_HIP_OK;
-  if (!x || (residual && n_parts != 1)) return MODA_HIP_EINVAL;
+  if (!x || (residual && (n_parts != 1 || gelu))) return MODA_HIP_EINVAL;
   if (K % 64 != 0 || rows >= (1ll << 30) || ldx >= (1ll << 22) || K >= (1ll << 22)) return MODA_HIP_EUNSUPPORTED;
   if ((uintptr_t)x % 16 != 0 || ldx % 8 != 0 || ldx < K || (residual && ((uintptr_t)residual % 16 != 0 || ld_res % 8 != 0)))
     return MODA_HIP_EALIGN;

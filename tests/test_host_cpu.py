@@ -562,3 +562,39 @@ def test_stack_under_a_dispatch_mode_is_left_to_the_modules(monkeypatch):
     assert any("addmm" in s or "linear" in s for s in seen)
     with torch.no_grad():
         assert model(x) is mark
+
+
+def test_dense_entry_points_refuse_what_their_kernels_cannot_take():
+    """Codes of moda_hip_linear and moda_hip_layer_norm, all returned before a device is looked at (nothing is read)."""
+    from moda_amd import _lib
+
+    lib = _lib.load()
+    i64, ptr = ctypes.c_int64, ctypes.c_void_p
+
+    class Part(ctypes.Structure):
+        _fields_ = [("w", ptr), ("bias", ptr), ("y", ptr), ("ldy", i64), ("n", i64)]
+
+    def linear(dtype=0, rows=4, K=64, x=0x1000, ldx=64, n_parts=1, residual=None, ld_res=64, gelu=0, **part):
+        p = dict(w=0x2000, bias=0x3000, y=0x4000, ldy=64, n=64)
+        p.update(part)
+        parts = (Part * 3)(*(Part(*(p[k] for k in ("w", "bias", "y", "ldy", "n"))) for _ in range(3)))
+        return lib.moda_hip_linear(dtype, i64(rows), i64(K), ptr(x), i64(ldx), parts, n_parts, ptr(residual), i64(ld_res), gelu, None)
+
+    def norm(dtype=0, rows=4, dim=64, x=0x1000, w=0x2000, b=0x3000, y=0x4000):
+        return lib.moda_hip_layer_norm(dtype, i64(rows), i64(dim), ptr(x), ptr(w), ptr(b), ctypes.c_float(1e-6), ptr(y), None)
+
+    assert linear(rows=0) == 0 and norm(rows=0) == 0
+    for bad in (dict(dtype=2), dict(dtype=-1), dict(rows=-1), dict(K=0), dict(n_parts=0), dict(n_parts=4), dict(x=None), dict(w=None),
+                dict(y=None), dict(n=0), dict(residual=0x5000, n_parts=2), dict(residual=0x5000, gelu=1)):
+        assert linear(**bad) == -1, bad
+    for bad in (dict(K=96, ldx=96), dict(n=60), dict(rows=1 << 30), dict(ldx=1 << 22)):
+        assert linear(**bad) == -2, bad
+    for bad in (dict(x=0x1008), dict(ldx=68), dict(ldx=56), dict(w=0x2008), dict(y=0x4002), dict(ldy=68), dict(bias=0x3004),
+                dict(residual=0x5008), dict(residual=0x5000, ld_res=68)):
+        assert linear(**bad) == -3, bad
+    for bad in (dict(dtype=2), dict(rows=-1), dict(dim=0), dict(x=None), dict(w=None), dict(b=None), dict(y=None)):
+        assert norm(**bad) == -1, bad
+    for bad in (dict(dim=60), dict(dim=4104), dict(rows=1 << 31)):
+        assert norm(**bad) == -2, bad
+    for bad in (dict(x=0x1008), dict(w=0x2008), dict(b=0x3008), dict(y=0x4008)):
+        assert norm(**bad) == -3, bad
