@@ -598,3 +598,66 @@ def test_dense_entry_points_refuse_what_their_kernels_cannot_take():
         assert norm(**bad) == -2, bad
     for bad in (dict(x=0x1008), dict(w=0x2008), dict(b=0x3008), dict(y=0x4008)):
         assert norm(**bad) == -3, bad
+
+
+@pytest.mark.parametrize("way", ["forward hook", "forward pre-hook", "global hook", "dropout", "replaced activation", "tanh GELU",
+                                 "derived linear", "patched forward", "derived attention", "swapped parameter", "blocks that differ",
+                                 "another scale", "autocast", "gradients", "derived tensor", "rebuilt cache"])
+def test_ways_back_from_the_native_stack_to_its_modules(monkeypatch, way):
+    """What the native forward pass does not do, the modules do: a stack runs them as soon as one is not what the
+    constructor made, is hooked, drops out, or the call asks for more than values."""
+    import moda_amd
+
+    model, x, mark = _native_stack(monkeypatch)
+    with torch.no_grad():
+        assert model(x) is mark
+    blk, nn = model.blocks[1], torch.nn
+    if way == "forward hook":
+        blk.norm2.register_forward_hook(lambda *a: None)
+    elif way == "forward pre-hook":
+        blk.attn.kv.register_forward_pre_hook(lambda *a: None)
+    elif way == "dropout":
+        blk.attn.proj_drop.p = 0.1
+        with torch.no_grad():
+            assert model(x) is mark  # not active in evaluation
+        model.train()
+    elif way == "replaced activation":
+        blk.mlp[1] = nn.SiLU()
+    elif way == "tanh GELU":
+        blk.mlp[1] = nn.GELU(approximate="tanh")
+    elif way == "derived linear":
+        class Linear(nn.Linear):
+            pass
+        blk.attn.q = Linear(64, 64)
+    elif way == "patched forward":
+        blk.mlp[2].forward = lambda h: h[..., :64]
+    elif way == "derived attention":
+        class Attention(moda_amd.MoDAAttention):
+            pass
+        blk.attn = Attention(64, 2, 1, qkv_bias=True)
+    elif way == "swapped parameter":
+        blk.norm1._parameters["weight"] = torch.ones(64)
+    elif way == "blocks that differ":
+        blk.attn.is_causal = True
+    elif way == "another scale":
+        for b in model.blocks:
+            b.attn.scale = 1.0
+    if way == "global hook":
+        handle = nn.modules.module.register_module_forward_pre_hook(lambda *a: None)
+        try:
+            _runs_modules(model, x)
+        finally:
+            handle.remove()
+    elif way == "autocast":
+        monkeypatch.setattr(torch, "is_autocast_enabled", lambda device: device == "cuda")  # (off on a host without a GPU)
+        _runs_modules(model, x)
+    elif way == "gradients":
+        with pytest.raises(RuntimeError, match="no CPU path"):
+            model(x)
+    elif way == "derived tensor":
+        _runs_modules(model, nn.Parameter(x))
+    elif way == "rebuilt cache":
+        with torch.no_grad(), pytest.raises(RuntimeError, match="no CPU path"):
+            model(x, inplace_cache=False)
+    else:
+        _runs_modules(model, x)

@@ -1910,3 +1910,75 @@ def test_gelu_over_the_whole_range(gpu_device, dtype):
         tiny = 2.0 ** -25 if dtype is torch.float16 else 2.0 ** -126  # bf16: fp32's subnormals are flushed
         err = (row.double() - want).abs()[ok]
         assert (err <= (rel + 8e-6) * want.abs()[ok] + tiny).all(), (err - (rel + 8e-6) * want.abs()[ok]).max()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [
+    # rows, K, features of each part: the smallest call and ragged edges of the 64 x 64 tile, three parts; then grids that
+    # take the 128 x 128, the two-stage and the three-stage 128 x 64 tile (a short last tile on both axes each)
+    (1, 64, (8,)),
+    (65, 192, (72, 24, 136)),
+    (129, 64, (64, 8)),
+    (4999, 128, (1000,)),
+    (8187, 64, (504,)),
+    (8187, 576, (184, 120)),
+], ids=str)
+def test_linear_against_fp64(gpu_device, case, dtype):
+    """Every tile and epilogue of the linear kernel.  Bound: u |y| for each rounding to 16 bits (u = 2^-8, 2^-11; the layer's
+    own result first, then GELU's, whose slope is at most 1.13, or the sum's), and K 2^-24 sum |x| |w| for the fp32 sums.
+    Rows of input and output are further apart than they are long; what lies between the output rows stays."""
+    rows, K, parts = case
+    say(f"CASE linear {case} {dtype}")
+    u = 2.0 ** -8 if dtype is torch.bfloat16 else 2.0 ** -11
+    gen = torch.Generator(device=gpu_device).manual_seed(rows)
+    rn = lambda *s: torch.randn(*s, generator=gen, device=gpu_device).to(dtype)
+    x = rn(rows, K + 16)[:, :K]
+    for epilogue in ("plain", "bias", "gelu", "residual", "inplace") if len(parts) == 1 else ("plain", "bias", "gelu"):
+        ws, bs = [rn(n, K) for n in parts], [None if epilogue == "plain" else rn(n) for n in parts]
+        outs = [torch.full((rows, n + 8), 7.0, device=gpu_device, dtype=dtype) for n in parts]
+        residual = rn(rows, parts[0] + 24)[:, :parts[0]] if epilogue == "residual" else outs[0][:, :parts[0]] if epilogue == "inplace" else None
+        res = None if residual is None else residual.double().clone()
+        assert _linear(x, [(w, b, y[:, :w.shape[0]]) for w, b, y in zip(ws, bs, outs)], residual, epilogue == "gelu") == 0
+        for w, b, y in zip(ws, bs, outs):
+            n = w.shape[0]
+            lin = x.double() @ w.double().t() + (0 if b is None else b.double())
+            err = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + 2.0 ** -23 * lin.abs()
+            want = lin
+            if epilogue == "gelu":
+                want, err = 0.5 * lin * torch.special.erfc(lin * -0.5 ** 0.5), 1.13 * (err + u * lin.abs()) + 1e-6
+            elif res is not None:
+                want, err = lin + res, err + u * lin.abs()
+            bound = (err + u * (want.abs() + err)) * 1.001 + (2.0 ** -25 if dtype is torch.float16 else 0)
+            assert ((y[:, :n].double() - want).abs() <= bound).all(), (epilogue, ((y[:, :n].double() - want).abs() / bound).max())
+            assert (y[:, n:] == 7.0).all(), epilogue
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dim", [8, 128, 136, 256, 264, 512, 520, 1024, 1032, 2048, 2056, 4096])
+def test_layer_norm_against_fp64(gpu_device, dim, dtype):
+    """Every row width class of the layer-norm kernel at its ends, rows that do not fill a workgroup, in place as well.
+    Bound: one rounding to 16 bits, u |y|, and 2^-20 of the largest term for the fp32 arithmetic."""
+    import ctypes
+
+    from moda_amd import _lib
+
+    u = 2.0 ** -8 if dtype is torch.bfloat16 else 2.0 ** -11
+    gen = torch.Generator(device=gpu_device).manual_seed(dim)
+    rn = lambda *s: torch.randn(*s, generator=gen, device=gpu_device)
+    w, b = rn(dim).to(dtype), rn(dim).to(dtype)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    for rows in (1, 3, 67):
+        x = (rn(rows, dim) * 2 + 3).to(dtype)
+        y = torch.full((rows + 1, dim), 7.0, device=gpu_device, dtype=dtype)
+        place = torch.cat([x, y[:1]])
+        for src, dst in ((x, y), (place, place)):
+            rc = _lib.load().moda_hip_layer_norm({torch.bfloat16: 0, torch.float16: 1}[dtype], ctypes.c_int64(rows), ctypes.c_int64(dim), ptr(src),
+                                                 ptr(w), ptr(b), ctypes.c_float(1e-6), ptr(dst),
+                                                 ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+            assert rc == 0
+        want = torch.nn.functional.layer_norm(x.double(), (dim,), w.double(), b.double(), 1e-6)
+        unit = torch.nn.functional.layer_norm(x.double(), (dim,), None, None, 1e-6)
+        bound = u * want.abs() + 2.0 ** -20 * ((3 + unit.abs()) * w.double().abs() + b.double().abs())
+        for got in (y, place):
+            assert ((got[:rows].double() - want).abs() <= bound).all(), (rows, ((got[:rows].double() - want).abs() / bound).max())
+            assert (got[rows:] == 7.0).all()
