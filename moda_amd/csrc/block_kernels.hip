@@ -4,8 +4,10 @@
 #include <algorithm>
 
 #include "../../include/moda_hip.h"
+#include "geometry.h"
 #include "tile.h"
 #include "tile16.h"
+#include "tuning.h"
 
 namespace moda {
 
@@ -47,7 +49,6 @@ __device__ __forceinline__ float gelu(float x) {
 //
 // Sized for a vision model's linears (12 608 rows, K 256 .. 1024), where a launch is 8 to 20 us and the k loop 4 to 16
 // steps: what counts is enough workgroups in flight to cover each one's start and end, not a large tile.
-// The feature tiles of one row tile go to one XCD (blocks b, b + 8, b + 16, ... share an L2), which reads x once.
 template <typename T, int BM, int BN, int NST, Epilogue EPI>
 __global__ __launch_bounds__(256, 2) void linear_kernel(const LinearArgs a) {
   constexpr int DIST = NST - 1, MB = BN / 32, NB = BM / 32, STAGE = (BM + BN) * 64;
@@ -55,9 +56,8 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(const LinearArgs a) {
   lds_ptr smem = (lds_ptr)smem_raw;
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, q4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wf = wave & 1;
-  const int slot = blockIdx.x >> 3;
-  const int mt = (blockIdx.x & 7) + 8 * (slot / a.n_tiles);
-  int nt = slot % a.n_tiles;
+  const int mt = linear_row_tile(blockIdx.x, a.n_tiles);
+  int nt = linear_feature_tile(blockIdx.x, a.n_tiles);
   if (mt >= a.m_tiles) return;
   int pi = 0;
   if (a.n_parts > 1 && nt >= a.part[0].tile_end) pi = (a.n_parts > 2 && nt >= a.part[1].tile_end) ? 2 : 1;
@@ -216,7 +216,7 @@ hipError_t launch_linear_t(LinearArgs a, hipStream_t stream) {
   a.m_tiles = (a.rows + BM - 1) / BM;
   a.n_tiles = 0;
   for (int i = 0; i < a.n_parts; i++) a.part[i].tile_end = a.n_tiles += (a.part[i].n + BN - 1) / BN;
-  const int64_t nblk = 8ll * ((a.m_tiles + 7) / 8) * a.n_tiles;
+  const int64_t nblk = linear_blocks(a.m_tiles, a.n_tiles);
   if (nblk >= (1ll << 31)) return hipErrorInvalidValue;
   hipLaunchKernelGGL((linear_kernel<T, BM, BN, NST, EPI>), dim3((unsigned)nblk), dim3(256), smem, stream, a);
   return hipGetLastError();
@@ -224,20 +224,14 @@ hipError_t launch_linear_t(LinearArgs a, hipStream_t stream) {
 
 template <typename T, Epilogue EPI>
 hipError_t launch_linear_e(const LinearArgs& a, int cus, hipStream_t stream) {
-  auto tiles = [&](int bm, int bn) {
-    int64_t t = 0;
-    for (int i = 0; i < a.n_parts; i++) t += (a.part[i].n + bn - 1) / bn;
-    return t * ((a.rows + bm - 1) / bm);
-  };
-  // Measured at 1 900 .. 12 608 rows, K 128 .. 3 072.  A 128 x 128 tile where its grid is one full round of two
-  // workgroups per compute unit (12 608 x 512 -> 512: 17 us, others 18 - 24); 128 x 64 where that still gives two each
-  // (256 -> 384: 8.7 us), with a third stage in flight for a long k loop in one round (1024 -> 256: 14.6 against
-  // 15.9 us); else small tiles, five workgroups per compute unit.
-  const int64_t large = tiles(128, 128), tall = tiles(128, 64);
-  if (large >= cus + cus / 4 && large <= 2ll * cus) return launch_linear_t<T, 128, 128, 2, EPI>(a, stream);
-  if (tall >= 2ll * cus) return launch_linear_t<T, 128, 64, 2, EPI>(a, stream);
-  if (tall > cus && a.K >= 512) return launch_linear_t<T, 128, 64, 3, EPI>(a, stream);
-  return launch_linear_t<T, 64, 64, 2, EPI>(a, stream);
+  int features[3];
+  for (int i = 0; i < a.n_parts; i++) features[i] = a.part[i].n;
+  switch (pick_linear_tile(a.rows, a.K, features, a.n_parts, cus)) {
+    case LinearTile::k128x128: return launch_linear_t<T, 128, 128, 2, EPI>(a, stream);
+    case LinearTile::k128x64: return launch_linear_t<T, 128, 64, 2, EPI>(a, stream);
+    case LinearTile::k128x64ThreeStages: return launch_linear_t<T, 128, 64, 3, EPI>(a, stream);
+    default: return launch_linear_t<T, 64, 64, 2, EPI>(a, stream);
+  }
 }
 
 template <typename T>

@@ -34,6 +34,7 @@ namespace moda {
 // index arithmetic costs the long-sequence instantiation scalar registers it cannot spare)
 template <typename T, int HD, bool VARLEN, bool SPLIT = false>
 __global__ __launch_bounds__(512) void dkv_kernel(const KArgs a_in) {
+  static_assert(!(VARLEN && SPLIT) || HD <= 64, "packed batches on the wider tiles are summed in one pass");
   // 16-column halves per wave, query rows per streamed tile: halved for the 256-wide tiles, whose operands and
   // accumulators would not fit the register file (and whose three-stage ring would not fit the LDS) otherwise
   constexpr int NB = HD > 128 ? 1 : 2, BM = HD > 128 ? 32 : 64, MBLK = BM / 16;
@@ -976,15 +977,15 @@ hipError_t launch_dkv_t(const KArgs& a, hipStream_t stream) {
       return hipGetLastError();
     };
     static LdsAttrState attr[4];
-    const hipError_t e = a.cu ? (nseg > 1 ? go(&dkv_kernel<T, HD, true, HD <= 128>, attr[0]) : go(&dkv_kernel<T, HD, true>, attr[1]))
+    const hipError_t e = a.cu ? (nseg > 1 ? go(&dkv_kernel<T, HD, true, HD <= 64>, attr[0]) : go(&dkv_kernel<T, HD, true>, attr[1]))
                               : (nseg > 1 ? go(&dkv_kernel<T, HD, false, true>, attr[2]) : go(&dkv_kernel<T, HD, false>, attr[3]));
     if (e != hipSuccess) return e;
   }
   if (nseg > 1 && n_seq_tiles > 0) {
     const int rpb = 256 / (HD / 8), bm = flat ? 32 : BM;
     const dim3 grid((unsigned)(((int64_t)a.T + rpb - 1) / rpb * a.B * a.Hkv));
-    if (a.cu)
-      hipLaunchKernelGGL((dkv_reduce_kernel<T, HD, true>), grid, dim3(256), 0, stream, a, BN, bm);
+    if (HD <= 64 && a.cu)
+      hipLaunchKernelGGL((dkv_reduce_kernel<T, HD, HD <= 64>), grid, dim3(256), 0, stream, a, BN, bm);
     else
       hipLaunchKernelGGL((dkv_reduce_kernel<T, HD, false>), grid, dim3(256), 0, stream, a, BN, bm);
     const hipError_t e = hipGetLastError();

@@ -187,6 +187,14 @@ MODA_HD ColTilePlan col_tile_plan(const KArgs& grid, const KArgs& a, int ct, int
 MODA_HD int query_tile_rows(const KArgs& a, int f_q0, int BM) { return imax(imin(a.Tq - f_q0, BM), 0); }
 
 // ---------------------------------------------------------------------------------------------------
+// Linear layers: the feature tiles of one row tile go to one XCD (blocks b, b + 8, b + 16, ... share an L2), which reads
+// its input rows once.  Row tiles past the last one have nothing to do.
+// ---------------------------------------------------------------------------------------------------
+MODA_HD int linear_row_tile(unsigned block, int n_tiles) { return (int)(block & 7) + 8 * ((int)(block >> 3) / n_tiles); }
+MODA_HD int linear_feature_tile(unsigned block, int n_tiles) { return (int)(block >> 3) % n_tiles; }
+inline int64_t linear_blocks(int m_tiles, int n_tiles) { return 8ll * ((m_tiles + 7) / 8) * n_tiles; }
+
+// ---------------------------------------------------------------------------------------------------
 // Launch grids (host side), one place for the launchers and the walker.
 // ---------------------------------------------------------------------------------------------------
 inline int64_t row_kernel_blocks(const KArgs& a, int rows_per_block) {

@@ -16,10 +16,14 @@
 //     voffset + soffset does not wrap 32 bits (the range check the kernels rely on compares that sum with
 //     num_records); a lane whose chunk lies past the tensors' head dim is out of range; the 64 LDS slots the load
 //     fills lie inside the launch's dynamic LDS allocation;
-//   * coverage: every element of o, lse, dq, dk, dv, dkd, dvd and of the row-sum workspace is written exactly once.
+//   * coverage: every element of o, lse, dq, dk, dv, dkd, dvd and of the row-sum workspace is written exactly once;
+//     every partial sum of a row segment that is read was written once, and every one that was written is read.
 //
 // usage: address_walker HD D Dv H G L Lv mode(0..4) chunk_tokens row_segments packed B_or_n len0 [len1 ...]
 //   packed = 0: a fixed-length batch of B sequences of len0 tokens; packed = 1: n sequences on one packed axis.
+//   environment: WALKER_FP32=1 walks the fp32 matrix kernels instead; WALKER_OWN_SLOT=1 a backward that leaves the slots
+//   without data alone and adds slot Lv of the depth gradients to dk, dv.
+// usage: address_walker linear rows K gelu n0 [n1 n2]   |   norm rows dim   |   slot B T H D L slot wide to_cache
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
@@ -50,6 +54,7 @@ struct Region {
 
 std::map<std::string, Region> g_regions;
 long long g_checked = 0, g_dma_in = 0, g_dma_out = 0;
+bool g_fp32 = false, g_own_slot = false;
 std::string g_ctx;
 
 [[noreturn]] void fail(const char* fmt, ...) {
@@ -125,6 +130,18 @@ void check_dma(const char* name, const void* desc_base, uint32_t num_records, in
     fail("LDS target %u (+%d) beyond the %u bytes of dynamic LDS", lds_byte, 64 * bytes, lds_limit);
 }
 
+// partial sums of row segments: written once before they are read, and then marked so that the rest can be found
+long long g_partials_read = 0;
+void read_partials(const float* p, int n) {
+  check_access("part", p, 4ull * n, false);
+  Region& r = region("part");
+  for (uint64_t i = ((uint64_t)p - r.base) / 4; i < ((uint64_t)p - r.base) / 4 + n; i++) {
+    if (r.writes[i] != 1) fail("partial sum %llu read %s", (unsigned long long)i, r.writes[i] ? "twice" : "that no segment wrote");
+    r.writes[i] = 2;
+    g_partials_read++;
+  }
+}
+
 struct Case {
   int HD, D, Dv, H, G, L, Lv, mode, cb, packed, nseq;
   std::vector<int> len;
@@ -160,25 +177,27 @@ KArgs make_args(const Case& c) {
   a.delta_pitch = c.packed ? (int)qrows : a.Tq;
   a.own_delta = 1;  // a whole backward: the dQ kernel forms the row sums (the delta kernel is walked as well)
   auto strides = [&](int64_t rows, int heads, int dim) { return Str3{rows * heads * dim, (int64_t)heads * dim, (int64_t)dim}; };
-  // bytes of a dense [Bt, rows, heads, dim] tensor of 16-bit elements
-  auto bytes = [&](int64_t rows, int heads, int dim) { return (uint64_t)Bt * rows * heads * dim * 2; };
+  a.own_slot = a.keep_slots = g_own_slot ? 1 : 0;
+  // a dense [Bt, rows, heads, dim] tensor
+  const int es = g_fp32 ? 4 : 2;
+  auto bytes = [&](int64_t rows, int heads, int dim) { return (uint64_t)Bt * rows * heads * dim * es; };
   int idx = 0;
-  a.q = add_region("q", idx++, bytes(qrows, a.Hq, c.D), 2, false);
-  a.o = add_region("o", idx++, bytes(qrows, a.Hq, c.Dv), 2, true);
+  a.q = add_region("q", idx++, bytes(qrows, a.Hq, c.D), es, false);
+  a.o = add_region("o", idx++, bytes(qrows, a.Hq, c.Dv), es, true);
   a.out_o = (uint16_t*)a.o;
-  a.d_o = add_region("do", idx++, bytes(qrows, a.Hq, c.Dv), 2, false);
-  a.dq = (uint16_t*)add_region("dq", idx++, bytes(qrows, a.Hq, c.D), 2, true);
-  a.k = add_region("k", idx++, bytes(T, c.H, c.D), 2, false);
-  a.v = add_region("v", idx++, bytes(T, c.H, c.Dv), 2, false);
-  a.dk = (uint16_t*)add_region("dk", idx++, bytes(T, c.H, c.D), 2, true);
-  a.dv = (uint16_t*)add_region("dv", idx++, bytes(T, c.H, c.Dv), 2, true);
-  a.kd = add_region("kd", idx++, bytes((int64_t)T * c.L, c.H, c.D), 2, false);
-  a.vd = add_region("vd", idx++, bytes((int64_t)T * c.L, c.H, c.Dv), 2, false);
-  a.dkd = (uint16_t*)add_region("dkd", idx++, bytes((int64_t)T * c.L, c.H, c.D), 2, true);
-  a.dvd = (uint16_t*)add_region("dvd", idx++, bytes((int64_t)T * c.L, c.H, c.Dv), 2, true);
+  a.d_o = add_region("do", idx++, bytes(qrows, a.Hq, c.Dv), es, false);
+  a.dq = (uint16_t*)add_region("dq", idx++, bytes(qrows, a.Hq, c.D), es, true);
+  a.k = add_region("k", idx++, bytes(T, c.H, c.D), es, false);
+  a.v = add_region("v", idx++, bytes(T, c.H, c.Dv), es, false);
+  a.dk = (uint16_t*)add_region("dk", idx++, bytes(T, c.H, c.D), es, true);
+  a.dv = (uint16_t*)add_region("dv", idx++, bytes(T, c.H, c.Dv), es, true);
+  a.kd = add_region("kd", idx++, bytes((int64_t)T * c.L, c.H, c.D), es, false);
+  a.vd = add_region("vd", idx++, bytes((int64_t)T * c.L, c.H, c.Dv), es, false);
+  a.dkd = (uint16_t*)add_region("dkd", idx++, bytes((int64_t)T * c.L, c.H, c.D), es, true);
+  a.dvd = (uint16_t*)add_region("dvd", idx++, bytes((int64_t)T * c.L, c.H, c.Dv), es, true);
   a.lse = (float*)add_region("lse", idx++, (uint64_t)Bt * qrows * a.Hq * 4, 4, true);
   a.delta = (float*)add_region("delta", idx++, (uint64_t)(c.packed ? 1 : c.nseq) * a.Hq * a.delta_pitch * 4, 4, true);
-  if (depth_scores_from_dq(a, c.HD)) {  // P and dS of the (query row, slot) pairs, handed from dQ to the depth-gradient kernel
+  if (!g_fp32 && depth_scores_from_dq(a, c.HD)) {  // P and dS of the (query row, slot) pairs, handed from dQ to the depth-gradient kernel
     const uint64_t n = (uint64_t)(c.packed ? 1 : c.nseq) * a.Hq * a.delta_pitch * a.Lv * 2;
     a.depth_p = (uint16_t*)add_region("hand_p", idx++, n, 2, true);
     a.depth_ds = (uint16_t*)add_region("hand_ds", idx++, n, 2, true);
@@ -328,8 +347,7 @@ void walk_row_kernel(const KArgs& a_in, bool dq, int rows_per_wave, bool own_pos
             const int col0 = span.c_beg + 32 * j;
             const int nrows = imin(32, span.c_end - col0);
             // where the dQ kernel forms the depth gradients it alternates between two sets of private tiles
-            // ... and so does the forward kernel on the 64-wide tiles
-            const uint32_t set = ((dq && depth_grads_in_dq(a, HD)) || (!dq && HD <= 64)) ? (uint32_t)(j & 1) * Shape::W * 64 * HD * 2 : 0u;
+            const uint32_t set = dq && depth_grads_in_dq(a, HD) ? (uint32_t)(j & 1) * Shape::W * 64 * HD * 2 : 0u;
             for (int i = 0; i < Own::N; i++) {
               if (a.Lv != a.L) {
                 const int w0 = col0 / a.Lv, l0 = col0 - w0 * a.Lv;
@@ -570,8 +588,14 @@ void walk_dkv_flat(const KArgs& a_in) {
           }
           continue;
         }
+        const int64_t slot = (int64_t)c * a.L + a.Lv;  // the layer's own, joined where the launch has been asked to
+        if (a.own_slot && RW == 1 && nseg == 1) fail("dkv_flat_kernel: the long launches' kernel does not add an own slot");
         for (int d = 0; d < MB; d++) {
           if (RW > 1 && d / (MB / 2) != (wave & 1)) continue;  // waves 0, 1 write dk, waves 2, 3 dv, half the blocks each
+          if (a.own_slot && (RW == 1 || wave < 2) && 16 * d + 4 * q4 < a.D)
+            check_access("dkd", a.dkd + b * a.sdkd.b + hkv * a.sdkd.h + slot * a.sdkd.t + 4 * q4 + 16 * d, 8, false);
+          if (a.own_slot && (RW == 1 || wave >= 2) && 16 * d + 4 * q4 < a.Dv)
+            check_access("dvd", a.dvd + b * a.sdvd.b + hkv * a.sdvd.h + slot * a.sdvd.t + 4 * q4 + 16 * d, 8, false);
           if ((RW == 1 || wave < 2) && 16 * d + 4 * q4 < a.D) check_access("dk", dkp + 16 * d, 8, true);
           if ((RW == 1 || wave >= 2) && 16 * d + 4 * q4 < a.Dv) check_access("dv", dvp + 16 * d, 8, true);
         }
@@ -628,9 +652,16 @@ void walk_reduce(const KArgs& a_in, int BN, int BM) {
       ctx("dkv_reduce_kernel", (int)block, tid >> 6, tid & 63, "partial sums and dk, dv rows");
       for (int which = 0; which < 2; which++) {
         const float* src = a.dkv_part + (int64_t)which * a.dkv_split * plane + row * HD + 8 * sub;
-        for (int sg = 0; sg < nsegs; sg++) check_access("part", src + sg * plane, 32, false);
+        for (int sg = 0; sg < nsegs; sg++) read_partials(src + sg * plane, 8);
         uint16_t* outp = which == 0 ? a.dk + b * a.sdk.b + hkv * a.sdk.h + (int64_t)c * a.sdk.t
                                     : a.dv + b * a.sdv.b + hkv * a.sdv.h + (int64_t)c * a.sdv.t;
+        if (a.own_slot && 8 * sub < (which == 0 ? a.D : a.Dv)) {
+          const int64_t slot = (int64_t)c * a.L + a.Lv;
+          if (which == 0)
+            check_access("dkd", a.dkd + b * a.sdkd.b + hkv * a.sdkd.h + slot * a.sdkd.t + 8 * sub, 16, false);
+          else
+            check_access("dvd", a.dvd + b * a.sdvd.b + hkv * a.sdvd.h + slot * a.sdvd.t + 8 * sub, 16, false);
+        }
         if (8 * sub < (which == 0 ? a.D : a.Dv)) check_access(which == 0 ? "dk" : "dv", outp + 8 * sub, 16, true);
       }
     }
@@ -751,7 +782,7 @@ void walk_depth_cols(const KArgs& a_in) {
       uint16_t* dk_out = a.dkd + b * a.sdkd.b + hkv * a.sdkd.h + c * a.sdkd.t + 8 * sub;
       uint16_t* dv_out = a.dvd + b * a.sdvd.b + hkv * a.sdvd.h + c * a.sdvd.t + 8 * sub;
       if (slot >= a.Lv) {
-        if (!a.accum_depth) {
+        if (!a.keep_slots) {
           if (in_k) check_access("dkd", dk_out, 16, true);
           if (in_v) check_access("dvd", dv_out, 16, true);
         }
@@ -802,7 +833,7 @@ void walk_depth_tokens(const KArgs& a_in) {
       }
       const int64_t blk = (((int64_t)b * a.Hq + hkv) * a.delta_pitch + (int64_t)w * a.Gf) * a.Lv;
       for (int slot = 0; slot < a.L; slot++) {
-        if (slot >= a.Lv && a.accum_depth) continue;
+        if (slot >= a.Lv && a.keep_slots) continue;
         if (slot < a.Lv)
           for (int g = 0; g < a.Gf; g++) {
             check_access("hand_p", a.depth_p + blk + (int64_t)slot * a.Gf + g, 2, false);
@@ -827,29 +858,335 @@ void require_full(const char* name) {
   for (size_t i = 0; i < r.writes.size(); i++)
     if (r.writes[i] != 1) fail("%s unit %zu written %d times after the launch", name, i, (int)r.writes[i]);
 }
+// the depth gradients: rows of slots that hold data once, the others once or (keep_slots) not at all
+void require_depth_rows(const char* name, const KArgs& a, int dim) {
+  Region& r = region(name);
+  if (!r.track) return;
+  for (size_t i = 0; i < r.writes.size(); i++) {
+    const int want = a.keep_slots && (int)(i / ((size_t)a.Hkv * dim) % a.L) >= a.Lv ? 0 : 1;
+    if (r.writes[i] != want) fail("%s unit %zu written %d times after the launch, not %d", name, i, (int)r.writes[i], want);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// fp32 matrix kernels: 16-row (or 16-column) tiles, operands straight from global memory
+// ---------------------------------------------------------------------------------------------------------------
+template <int HD>
+void walk_fp32(const KArgs& a_in) {
+  constexpr int KS = HD / 16, H4 = HD / 64, W = 8, CW = HD <= 64 ? 8 : 4, PART = 16 * (HD + 4);
+  const bool full = a_in.D == HD && a_in.Dv == HD;
+  auto f = [](const uint16_t* p) { return (const float*)p; };
+  // the 16-byte pieces of one row as a score operand (lane group q) and as a second product's operand (lane n)
+  auto score = [&](const char* name, const float* row, int q, int d) {
+    for (int s = 0; s < KS; s++) check_access(name, row + (full || 16 * s + 4 * q < d ? 16 * s + 4 * q : 0), 16, false);
+  };
+  auto sum = [&](const char* name, const float* row, int n, int d) {
+    for (int h = 0; h < H4; h++) check_access(name, row + (full || 64 * h + 4 * n < d ? 64 * h + 4 * n : 0), 16, false);
+  };
+  auto partial = [&](int first, uint32_t lds_bytes) {  // a wave's accumulators on their way to LDS
+    for (int n = 0; n < 16; n++)
+      if ((uint32_t)(first + n * (HD + 4) + HD) * 4 > lds_bytes) fail("partial results past the LDS allocation");
+  };
+  for (int which = 0; which < 3; which++) {  // forward, row sums alone, dQ
+    const char* kname = which == 0 ? "fp32_fwd_kernel" : which == 1 ? "fp32_delta_kernel" : "fp32_dq_kernel";
+    const uint32_t lds_bytes = W * PART * 4 + (which == 0 ? W * 32 * 4 : 0);
+    const int64_t nblk = (int64_t)((a_in.Tq + 15) / 16) * a_in.B * a_in.Hq;
+    const int BH = a_in.B * a_in.Hq;
+    for (int64_t block = 0; block < nblk; block++) {
+      int b = (int)(block % BH) / a_in.Hq;
+      const int hq = (int)(block % BH) % a_in.Hq, hkv = hq / a_in.hdiv;
+      KArgs a = a_in;
+      enter_sequence(a, b, 2);
+      const int qt = which == 1 ? (int)(block / BH) : query_tile_of((int)block, BH, 16, a_in.Tq);
+      if (which != 1 && qt * 16 >= a.Tq) continue;
+      if (a.Tq == 0) continue;
+      const RowTilePlan plan = row_tile_plan(a, qt, 16, 16, a.L > 0);
+      const int nblocks = which == 1 ? 0 : plan.n_seq + plan.n_dep;
+      for (int tid = 0; tid < (which == 1 ? 64 : 64 * W); tid++) {
+        const int lane = tid & 63, n = lane & 15, q = lane >> 4, wave = tid >> 6;
+        const int r = qt * 16 + n, rc = imin(r, a.Tq - 1);
+        ctx(kname, (int)block, wave, lane, "rows of q, do, o and their statistics");
+        if (which != 1) score("q", f(a.q) + b * a.sq.b + hq * a.sq.h + (int64_t)rc * a.sq.t, q, a.D);
+        if (which != 0) {
+          score("do", f(a.d_o) + b * a.sdo.b + hq * a.sdo.h + (int64_t)rc * a.sdo.t, q, a.Dv);
+          score("o", f(a.o) + b * a.so.b + hq * a.so.h + (int64_t)rc * a.so.t, q, a.Dv);
+        }
+        if (which == 2) check_access("lse", a.lse + ((int64_t)b * a.Tq + rc) * a.Hq + hq, 4, false);
+        if (which != 0 && wave == 0 && q == 0 && r < a.Tq)
+          check_access("delta", a.delta + ((int64_t)b * a.Hq + hq) * a.delta_pitch + r, 4, true);
+        for (int blk = wave; blk < nblocks; blk += W) {
+          const bool dep = blk >= plan.n_seq;
+          const int col0 = dep ? plan.dep0 + (blk - plan.n_seq) * 16 : blk * 16, ncols = dep ? a.T * a.Lv : a.T;
+          auto row_of = [&](int c) { return dep ? depth_row_of(a, imin(c, ncols - 1)) : (int64_t)imin(c, ncols - 1); };
+          const char *kn = dep ? "kd" : "k", *vn = dep ? "vd" : "v";
+          const float* kp = dep ? f(a.kd) + b * a.skd.b + hkv * a.skd.h : f(a.k) + b * a.sk.b + hkv * a.sk.h;
+          const float* vp = dep ? f(a.vd) + b * a.svd.b + hkv * a.svd.h : f(a.v) + b * a.sv.b + hkv * a.sv.h;
+          const int64_t ks = dep ? a.skd.t : a.sk.t, vs = dep ? a.svd.t : a.sv.t;
+          ctx(kname, (int)block, wave, lane, dep ? "depth columns" : "sequence columns");
+          if (dep && row_of(col0 + n) % a.L >= a.Lv) fail("depth row of a slot without data");
+          score(kn, kp + row_of(col0 + n) * ks, q, a.D);
+          if (which == 2) score(vn, vp + row_of(col0 + n) * vs, q, a.Dv);
+          for (int i = 0; i < 4; i++) {
+            if (which == 0)
+              sum(vn, vp + row_of(col0 + 4 * q + i) * vs, n, a.Dv);
+            else
+              sum(kn, kp + row_of(col0 + 4 * q + i) * ks, n, a.D);
+          }
+        }
+        if (which == 1) continue;
+        if (lane == 0) partial(wave * PART, W * PART * 4);
+        if (which == 0 && (uint32_t)(W * PART + (wave * 16 + n) * 2 + 2) * 4 > lds_bytes) fail("row statistics past the LDS allocation");
+        const int row = tid / (HD / 4), d = (tid % (HD / 4)) * 4;
+        ctx(kname, (int)block, wave, lane, "result row");
+        if (tid >= 16 * HD / 4 || qt * 16 + row >= a.Tq) continue;
+        const int64_t ro = qt * 16 + row;
+        if (which == 0 && d < a.Dv) check_access("o", f(a.out_o) + b * a.so.b + hq * a.so.h + ro * a.so.t + d, 16, true);
+        if (which == 0 && d == 0) check_access("lse", a.lse + ((int64_t)b * a.Tq + ro) * a.Hq + hq, 4, true);
+        if (which == 2 && d < a.D) check_access("dq", f(a.dq) + b * a.sdq.b + hq * a.sdq.h + ro * a.sdq.t + d, 16, true);
+      }
+    }
+    if (which == 0) {
+      require_full("o");
+      require_full("lse");
+    } else {
+      require_full("delta");
+      if (which == 1) reset_writes("delta");
+    }
+    if (which == 2) require_full("dq");
+  }
+  // dK/dV
+  const int BHk = a_in.B * a_in.Hkv, n_seq_tiles = a_in.has_seq ? (a_in.T + 15) / 16 : 0;
+  const int64_t ndep = ((int64_t)a_in.T * a_in.Lv + 16 * CW - 1) / (16 * CW), nblk = (n_seq_tiles + ndep) * BHk;
+  for (int64_t block = 0; block < nblk; block++) {
+    const int hkv = (int)(block % BHk) % a_in.Hkv, tile = (int)(block / BHk);
+    int b = (int)(block % BHk) / a_in.Hkv;
+    KArgs a = a_in;
+    enter_sequence(a, b, 2);
+    const bool dep = tile >= n_seq_tiles;
+    const int ncols = dep ? a.T * a.Lv : a.T;
+    for (int tid = 0; tid < 64 * CW; tid++) {
+      const int lane = tid & 63, n = lane & 15, q = lane >> 4, wave = tid >> 6;
+      const int c0 = dep ? ((tile - n_seq_tiles) * CW + wave) * 16 : tile * 16;
+      if (c0 >= ncols) continue;
+      const int c = c0 + n, cc = imin(c, ncols - 1);
+      const int64_t crow = dep ? depth_row_of(a, cc) : (int64_t)cc;
+      ctx("fp32_dkv_kernel", (int)block, wave, lane, "stationary K and V rows");
+      score(dep ? "kd" : "k", dep ? f(a.kd) + b * a.skd.b + hkv * a.skd.h + crow * a.skd.t : f(a.k) + b * a.sk.b + hkv * a.sk.h + crow * a.sk.t, q, a.D);
+      score(dep ? "vd" : "v", dep ? f(a.vd) + b * a.svd.b + hkv * a.svd.h + crow * a.svd.t : f(a.v) + b * a.sv.b + hkv * a.sv.h + crow * a.sv.t, q, a.Dv);
+      int lo, hi, unused;
+      q_interval(a, dep, c0, lo, unused);
+      q_interval(a, dep, imin(ncols, c0 + 16) - 1, unused, hi);
+      const int r_first = lo / 16 * 16, nrb = (hi - r_first + 15) / 16, nb = nrb * a.hdiv;
+      ctx("fp32_dkv_kernel", (int)block, wave, lane, "query rows and their statistics");
+      for (int blk = dep ? 0 : wave; blk < nb; blk += dep ? 1 : CW) {
+        const int hq = hkv * a.hdiv + blk / nrb, r0 = r_first + blk % nrb * 16;
+        const float *qp = f(a.q) + b * a.sq.b + hq * a.sq.h, *dop = f(a.d_o) + b * a.sdo.b + hq * a.sdo.h;
+        const int64_t r = imin(r0 + n, a.Tq - 1);
+        score("q", qp + r * a.sq.t, q, a.D);
+        score("do", dop + r * a.sdo.t, q, a.Dv);
+        for (int i = 0; i < 4; i++) {
+          const int64_t ri = imin(r0 + 4 * q + i, a.Tq - 1);
+          check_access("lse", a.lse + ((int64_t)b * a.Tq + ri) * a.Hq + hq, 4, false);
+          check_access("delta", a.delta + ((int64_t)b * a.Hq + hq) * a.delta_pitch + ri, 4, false);
+          sum("q", qp + ri * a.sq.t, n, a.D);
+          sum("do", dop + ri * a.sdo.t, n, a.Dv);
+        }
+      }
+      ctx("fp32_dkv_kernel", (int)block, wave, lane, "gradient rows");
+      if (dep) {
+        if (c >= ncols) continue;
+        const float *dkp = f(a.dkd) + b * a.sdkd.b + hkv * a.sdkd.h + crow * a.sdkd.t, *dvp = f(a.dvd) + b * a.sdvd.b + hkv * a.sdvd.h + crow * a.sdvd.t;
+        for (int h = 0; h < H4; h++)
+          for (int i = 0; i < 4; i++) {
+            const int d = 64 * h + 16 * q + 4 * i;
+            if (d < a.D) check_access("dkd", dkp + d, 16, true);
+            if (d < a.Dv) check_access("dvd", dvp + d, 16, true);
+          }
+        if (a.Lv != a.L && !a.keep_slots && c % a.Lv == a.Lv - 1)
+          for (int slot = a.Lv; slot < a.L; slot++) {
+            dkp += a.sdkd.t;
+            dvp += a.sdvd.t;
+            for (int d = 4 * q; d < a.D; d += 16) check_access("dkd", dkp + d, 16, true);
+            for (int d = 4 * q; d < a.Dv; d += 16) check_access("dvd", dvp + d, 16, true);
+          }
+        continue;
+      }
+      if (lane == 0) partial((CW + wave) * PART, 2 * CW * PART * 4);
+      for (int e = tid; e < 2 * 16 * HD / 4; e += 64 * CW) {
+        const int w = e / (16 * HD / 4), row = e % (16 * HD / 4) / (HD / 4), d = (e % (HD / 4)) * 4;
+        if (c0 + row >= ncols || d >= (w ? a.Dv : a.D)) continue;
+        if (w)
+          check_access("dv", f(a.dv) + b * a.sdv.b + hkv * a.sdv.h + (int64_t)(c0 + row) * a.sdv.t + d, 16, true);
+        else
+          check_access("dk", f(a.dk) + b * a.sdk.b + hkv * a.sdk.h + (int64_t)(c0 + row) * a.sdk.t + d, 16, true);
+      }
+    }
+  }
+  if (a_in.has_seq) {
+    require_full("dk");
+    require_full("dv");
+  }
+  if (a_in.L > 0) {
+    require_depth_rows("dkd", a_in, a_in.D);
+    require_depth_rows("dvd", a_in, a_in.Dv);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// linear layers, layer norm, depth slots
+// ---------------------------------------------------------------------------------------------------------------
+template <int BM, int BN, int NST>
+void walk_linear_tiles(int rows, int K, const std::vector<int>& parts, bool residual) {
+  constexpr int MB = BN / 32, NB = BM / 32;
+  const uint32_t lds_bytes = NST * (BM + BN) * 64 * 2;
+  const int64_t ldx = K + 8, ldy_pad = 16;
+  int idx = 0;
+  const uint16_t* x = add_region("x", idx++, ((int64_t)(rows - 1) * ldx + K) * 2, 2, false);  // nothing behind the last row
+  std::vector<const uint16_t*> w, bias, y;
+  std::vector<int> end;
+  std::vector<std::string> names;
+  for (size_t i = 0; i < parts.size(); i++) {
+    const std::string k = std::to_string(i);
+    w.push_back(add_region(("w" + k).c_str(), idx++, (int64_t)parts[i] * K * 2, 2, false));
+    bias.push_back(add_region(("bias" + k).c_str(), idx++, (int64_t)parts[i] * 2, 2, false));
+    y.push_back(add_region(("y" + k).c_str(), idx++, ((int64_t)(rows - 1) * (parts[i] + ldy_pad) + parts[i]) * 2, 2, true));
+    end.push_back((end.empty() ? 0 : end.back()) + (parts[i] + BN - 1) / BN);
+  }
+  const uint16_t* res = add_region("residual", idx++, residual ? (int64_t)rows * parts[0] * 2 : 0, 2, false);
+  const int m_tiles = (rows + BM - 1) / BM, n_tiles = end.back();
+  typedef AsyncTileLoader<64, BM, 256> LoadX;
+  typedef AsyncTileLoader<64, BN, 256> LoadW;
+  for (int64_t block = 0; block < linear_blocks(m_tiles, n_tiles); block++) {
+    const int mt = linear_row_tile((unsigned)block, n_tiles);
+    int nt = linear_feature_tile((unsigned)block, n_tiles), pi = 0;
+    if (mt >= m_tiles) continue;
+    while (nt >= end[pi]) pi++;
+    const int n = parts[pi], ldy = n + (int)ldy_pad;
+    if (pi > 0) nt -= end[pi - 1];
+    const int r0 = mt * BM, f0 = nt * BN;
+    const std::string wn = "w" + std::to_string(pi), bn = "bias" + std::to_string(pi), yn = "y" + std::to_string(pi);
+    for (int tid = 0; tid < 256; tid++) {
+      const int lane = tid & 63, ln = lane & 15, q4 = lane >> 4, wave = tid >> 6, wm = wave >> 1, wf = wave & 1;
+      LoadX lx;
+      LoadW lw;
+      lx.init(tid);
+      lw.init(tid);
+      ctx("linear_kernel", (int)block, wave, lane, "operand tiles");
+      for (int it = 0; it < K / 64; it++) {
+        const uint32_t xs = (uint32_t)(it % NST) * (BM + BN) * 64 * 2;
+        for (int i = 0; i < LoadX::N; i++)
+          check_dma("x", x + it * 64 + (int64_t)r0 * ldx, LoadX::anchored_bytes(ldx, r0, rows), lx.lane_offset((int)ldx * 2, 64),
+                    LoadX::rows_before(i) * (int)ldx * 2, 16, xs + (uint32_t)lx.lds_elems(i) * 2, lds_bytes, false);
+        for (int i = 0; i < LoadW::N; i++)
+          check_dma(wn.c_str(), w[pi] + it * 64 + (int64_t)f0 * K, LoadW::anchored_bytes(K, f0, n), lw.lane_offset(K * 2, 64),
+                    LoadW::rows_before(i) * K * 2, 16, xs + BM * 64 * 2 + (uint32_t)lw.lds_elems(i) * 2, lds_bytes, false);
+      }
+      ctx("linear_kernel", (int)block, wave, lane, "results");
+      for (int mb = 0; mb < MB; mb++) {
+        const int f = f0 + wf * (BN / 2) + 16 * mb + slot_base(q4);
+        if (f >= n) continue;
+        check_access(bn.c_str(), bias[pi] + f, 8, false);
+        for (int nb = 0; nb < NB; nb++) {
+          const int r = r0 + wm * (BM / 2) + 16 * nb + slot_base(ln >> 2) + (ln & 3);
+          if (r >= rows) continue;
+          if (residual) check_access("residual", res + (int64_t)r * n + f, 8, false);
+          check_access(yn.c_str(), y[pi] + (int64_t)r * ldy + f, 8, true);
+        }
+      }
+    }
+  }
+  for (size_t i = 0; i < parts.size(); i++) {
+    Region& r = region(("y" + std::to_string(i)).c_str());
+    for (size_t u = 0; r.track && u < r.writes.size(); u++) {
+      const int want = (int)(u % (size_t)(parts[i] + ldy_pad)) < parts[i] ? 1 : 0;
+      if (r.writes[u] != want) fail("%s unit %zu written %d times, not %d", r.name.c_str(), u, (int)r.writes[u], want);
+    }
+  }
+}
+void walk_linear(int rows, int K, bool gelu, const std::vector<int>& parts) {
+  const bool residual = parts.size() == 1 && !gelu;
+  switch (pick_linear_tile(rows, K, parts.data(), (int)parts.size(), 256)) {
+    case LinearTile::k128x128: printf("128x128 "); return walk_linear_tiles<128, 128, 2>(rows, K, parts, residual);
+    case LinearTile::k128x64: printf("128x64 "); return walk_linear_tiles<128, 64, 2>(rows, K, parts, residual);
+    case LinearTile::k128x64ThreeStages: printf("128x64,3 "); return walk_linear_tiles<128, 64, 3>(rows, K, parts, residual);
+    default: printf("64x64 "); return walk_linear_tiles<64, 64, 2>(rows, K, parts, residual);
+  }
+}
+
+void walk_norm(int rows, int dim) {
+  const int lpr = dim <= 128 ? 16 : dim <= 256 ? 32 : 64, ch = dim <= 512 ? 1 : dim <= 1024 ? 2 : dim <= 2048 ? 4 : 8;
+  const uint16_t* x = add_region("x", 0, (int64_t)rows * dim * 2, 2, false);
+  const uint16_t* w = add_region("weight", 1, (int64_t)dim * 2, 2, false);
+  const uint16_t* b = add_region("bias", 2, (int64_t)dim * 2, 2, false);
+  const uint16_t* y = add_region("y", 3, (int64_t)rows * dim * 2, 2, true);
+  const int rpb = 256 / lpr;
+  for (int block = 0; block < (rows + rpb - 1) / rpb; block++)
+    for (int tid = 0; tid < 256; tid++) {
+      const int row = block * rpb + tid / lpr;
+      if (row >= rows) continue;
+      ctx("layer_norm_kernel", block, tid >> 6, tid & 63, "row, weight, bias");
+      for (int c = 0; c < ch; c++) {
+        const int e = (c * lpr + tid % lpr) * 8;
+        if (e >= dim) continue;
+        check_access("x", x + (int64_t)row * dim + e, 16, false);
+        check_access("weight", w + e, 16, false);
+        check_access("bias", b + e, 16, false);
+        check_access("y", y + (int64_t)row * dim + e, 16, true);
+      }
+    }
+  require_full("y");
+}
+
+// one layer's K and V (views of one projection: rows 2 H D + 8 elements apart) against slot `slot` of the caches
+void walk_slot(int64_t B, int64_t T, int64_t H, int64_t D, int64_t L, int64_t slot, bool wide, bool to_cache) {
+  const int64_t st = 2 * H * D + 8, sb = T * st, piece = wide ? 16 : 2, per_row = D * 2 / piece, units = B * T * H * per_row;
+  for (int i = 0; i < 2; i++) {
+    const uint16_t* layer = add_region(i ? "v" : "k", 2 * i, (((B - 1) * T + T - 1) * st + H * D) * 2, 2, !to_cache);
+    const uint16_t* cache = add_region(i ? "cache_v" : "cache_k", 2 * i + 1, B * T * L * H * D * 2, 2, to_cache);
+    for (int64_t u = 0; u < (units + 255) / 256 * 256; u++) {
+      if (u >= units) continue;
+      const int64_t w = u % per_row, row = u / per_row, tok = row / H, h = row - tok * H, b = tok / T, t = tok - b * T;
+      ctx("slot_kernel", (int)(u / 256), (int)(u % 256) >> 6, (int)(u & 63), to_cache ? "layer into its slot" : "slot onto its layer");
+      check_access(i ? "v" : "k", (const char*)layer + (b * sb + t * st + h * D) * 2 + w * piece, piece, !to_cache);
+      check_access(i ? "cache_v" : "cache_k", (const char*)cache + (slot + tok * L) * H * D * 2 + (h * per_row + w) * piece, piece, to_cache);
+    }
+    Region& c = region(to_cache ? (i ? "cache_v" : "cache_k") : (i ? "v" : "k"));
+    for (size_t u = 0; u < c.writes.size(); u++) {
+      const int want = to_cache ? (int64_t)u / (H * D) % L == slot : (int64_t)u % st < H * D;
+      if (c.writes[u] != want) fail("%s unit %zu written %d times, not %d", c.name.c_str(), u, (int)c.writes[u], want);
+    }
+  }
+}
 
 template <int HD>
 void walk_all(const Case& c, const KArgs& a) {
-  const bool packed = a.cu != nullptr;
   // byte span of the widest streamed (batch, head) slice decides the addressing variant (as the launchers do)
   const int64_t span = 2 * std::max(std::max((int64_t)a.T * a.sk.t, (int64_t)a.T * a.sv.t),
                                     std::max((int64_t)a.T * a.L * a.skd.t, (int64_t)a.T * a.L * a.svd.t));
   const bool wide_addr = span > 0x7fffffffll;
   if (wide_addr) fail("slices beyond 2 GiB are not walked (the fake tensors would not fit the walker's write maps)");
-  const bool small = use_small_rows(a.Tq, (long long)a.B * a.Hq, a.compute_units);
+  const bool small = a.cu ? use_small_rows(a.delta_pitch, a.Hq, a.compute_units) : use_small_rows(a.Tq, (long long)a.B * a.Hq, a.compute_units);
+  const ShortRows rows = a.cu ? ShortRows::kNone : pick_short_rows(a.Tq, (long long)a.B * a.Hq, a.causal, a.compute_units);
   // ---- forward
   g_ctx = "forward";
-  auto fwd_lds = [&](int W, int NST) {  // the ring, or (64-wide tiles) two sets of private tiles per wave
-    const uint32_t ring = (uint32_t)NST * 2 * 64 * HD * 2, own = HD <= 64 ? 2u * W * 2 * 32 * HD * 2 : 0u;
-    return std::max(ring, own);
+  const auto ring = [](int NST) { return (uint32_t)NST * 2 * 64 * HD * 2; };
+  const auto fwd = [&](auto shape, const char* name) {
+    typedef decltype(shape) Shape;
+    printf("%s ", name);
+    walk_row_kernel<HD, Shape, false>(a, false, HD > 128 ? 16 : 32, HD <= 128, ring(Shape::NST), name);
   };
   if constexpr (HD > 128) {
-    walk_row_kernel<HD, RowWide, false>(a, false, 16, false, RowWide::NST * 2 * 64 * HD * 2, "fwd_wide_kernel");
+    fwd(RowWide{}, "fwd_wide_kernel");
+  } else if constexpr (HD <= 64) {
+    if (rows == ShortRows::kTwoStages)
+      fwd(RowShort{}, "fwd_kernel(short)");
+    else
+      fwd(RowSmall<HD>{}, "fwd_kernel(small)");
   } else {
     if (small)
-      walk_row_kernel<HD, RowSmall<HD>, false>(a, false, 32, true, fwd_lds(RowSmall<HD>::W, RowSmall<HD>::NST), "fwd_kernel(small)");
+      fwd(RowSmall<HD>{}, "fwd_kernel(small)");
     else
-      walk_row_kernel<HD, RowLargePP, false>(a, false, 32, true, fwd_lds(RowLargePP::W, RowLargePP::NST), "fwd_kernel");
+      fwd(RowLargePP{}, "fwd_kernel");
   }
   require_full("o");
   require_full("lse");
@@ -858,17 +1195,27 @@ void walk_all(const Case& c, const KArgs& a) {
   walk_delta<HD>(a);
   require_full("delta");
   reset_writes("delta");
-  auto ring_or_own = [&](int W, int NST) {
-    const uint32_t ring = (uint32_t)NST * 2 * 64 * HD * 2, own = (uint32_t)W * (HD <= kDepthGradsInDqMaxWidth ? 2 * 64 + 16 : 64) * HD * 2;
-    return (uint32_t)W * 64 * HD * 2 <= 128 * 1024 ? std::max(ring, own) : ring;
+  const auto dq = [&](auto shape, const char* name) {
+    typedef decltype(shape) Shape;
+    const uint32_t own = (uint32_t)Shape::W * (HD <= kDepthGradsInDqMaxWidth ? 2 * 64 + 16 : 64) * HD * 2;
+    const bool own_fits = a.L > 0 && (uint32_t)Shape::W * 64 * HD * 2 <= 128 * 1024;
+    printf("%s ", name);
+    walk_row_kernel<HD, Shape, false>(a, true, HD > 128 ? 16 : 32, HD <= 128, own_fits ? std::max(ring(Shape::NST), own) : ring(Shape::NST), name);
   };
   if constexpr (HD > 128) {
-    walk_row_kernel<HD, RowWide, false>(a, true, 16, false, ring_or_own(RowWide::W, RowWide::NST), "dq_kernel(wide)");
+    dq(RowWide{}, "dq_kernel(wide)");
+  } else if constexpr (HD <= 64) {
+    if (rows == ShortRows::kTwoStages)
+      dq(RowShort{}, "dq_kernel(short)");
+    else if (rows == ShortRows::kThreeStages)
+      dq(RowShort3{}, "dq_kernel(short, three stages)");
+    else
+      dq(RowSmall<HD>{}, "dq_kernel(small)");
   } else {
     if (small)
-      walk_row_kernel<HD, RowSmall<HD>, false>(a, true, 32, true, ring_or_own(RowSmall<HD>::W, RowSmall<HD>::NST), "dq_kernel(small)");
+      dq(RowSmall<HD>{}, "dq_kernel(small)");
     else
-      walk_row_kernel<HD, RowLarge, false>(a, true, 32, true, ring_or_own(RowLarge::W, RowLarge::NST), "dq_kernel");
+      dq(RowLarge{}, "dq_kernel");
   }
   require_full("dq");
   require_full("delta");
@@ -877,6 +1224,7 @@ void walk_all(const Case& c, const KArgs& a) {
     require_full("hand_ds");
   }
   const bool flat = takes_dkv_flat(a, HD);
+  if (a.own_slot && !flat) fail("only dkv_flat_kernel's launches add an own slot");
   if (flat) {
     if constexpr (HD == 64) {
       if (dkv_flat_row_waves(a))
@@ -888,15 +1236,17 @@ void walk_all(const Case& c, const KArgs& a) {
     walk_dkv<HD>(a);
   }
   if (a.dkv_split > 1 && a.has_seq) {
-    if (a.dkv_seg_tiles == 0) require_full("part");  // otherwise short tiles have fewer segments, or none
     walk_reduce<HD>(a, HD > 128 ? 64 : 128, flat || HD > 128 ? 32 : 64);
+    for (uint8_t w : region("part").writes)  // (short tiles have fewer segments, or none: their places stay empty)
+      if (w == 1) fail("a partial sum that no column adds up");
+    if (g_partials_read == 0) fail("row segments without partial sums");
   }
   if (a.has_seq) {
     require_full("dk");
     require_full("dv");
   }
   if (a.L > 0) {
-    if ((a.chunk || depth_grads_in_dq(a, HD)) && a.Lv != a.L) walk_zero_unfilled<HD>(a);
+    if ((a.chunk || depth_grads_in_dq(a, HD)) && a.Lv != a.L && !a.keep_slots) walk_zero_unfilled<HD>(a);
     if (a.chunk) {
       if constexpr (HD <= 128) {
         if (depth_by_chunks(a, HD)) walk_chunk_depth<HD>(a);
@@ -907,16 +1257,28 @@ void walk_all(const Case& c, const KArgs& a) {
       else
         walk_depth_cols<HD>(a);
     }
-    require_full("dkd");
-    require_full("dvd");
+    require_depth_rows("dkd", a, a.D);
+    require_depth_rows("dvd", a, a.Dv);
   }
-  (void)packed;
   (void)c;
 }
 
 }  // namespace
 
 int main(int argc, char** argv) {
+  const auto arg = [&](int i) { return i < argc ? atoi(argv[i]) : 0; };
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "linear" || what == "norm" || what == "slot") {
+    std::vector<int> parts;
+    for (int i = 5; i < argc; i++) parts.push_back(arg(i));
+    if (what == "linear") walk_linear(arg(2), arg(3), arg(4) != 0, parts);
+    if (what == "norm") walk_norm(arg(2), arg(3));
+    if (what == "slot") walk_slot(arg(2), arg(3), arg(4), arg(5), arg(6), arg(7), arg(8) != 0, arg(9) != 0);
+    printf("OK checked=%lld\n", g_checked);
+    return 0;
+  }
+  g_fp32 = getenv("WALKER_FP32") != nullptr;
+  g_own_slot = getenv("WALKER_OWN_SLOT") != nullptr;
   if (argc < 14) {
     fprintf(stderr, "usage: %s HD D Dv H G L Lv mode chunk_tokens split packed n len0 [len1 ...]\n", argv[0]);
     return 2;
@@ -959,6 +1321,12 @@ int main(int argc, char** argv) {
   }
   if (a.dkv_split > 1)
     a.dkv_part = (float*)add_region("part", 20, (uint64_t)2 * a.dkv_split * (a.cu ? 1 : a.B) * a.Hkv * part_rows(a) * c.HD * 4, 4, true);
+  if (g_fp32) {
+    if (c.HD > 128) return 2;
+    c.HD == 64 ? walk_fp32<64>(a) : walk_fp32<128>(a);
+    printf("OK checked=%lld\n", g_checked);
+    return 0;
+  }
   switch (c.HD) {
     case 64: walk_all<64>(c, a); break;
     case 128: walk_all<128>(c, a); break;

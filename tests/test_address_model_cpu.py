@@ -5,7 +5,8 @@ kernels' own index arithmetic (``moda_amd/csrc/geometry.h``, ``kargs.h``, ``tile
 and walks every (workgroup, wave, lane, trip) of a forward + backward launch: register operand loads, every tile
 descriptor with each lane's vector and scalar offset (the lanes that fetch past the tensors' head dim included),
 the row-statistics loads, the LDS targets against the launch's dynamic LDS size, and all stores; every output
-element must be written exactly once.
+element must be written exactly once.  The fp32 matrix kernels, the linear, layer-norm and depth-slot kernels are walked
+the same way.
 
 The first case is the packed batch that once ended in a GPU memory fault on the packed instantiations of the
 256-wide kernels (switched off since).  The walk finds every access of it inside its tensor: the fault is not an
@@ -112,7 +113,7 @@ FIXED = [
 
 def test_the_packed_wide_case_that_faulted_stays_inside_its_tensors(walker):
     rc, out = run(walker, **FAULTED)
-    assert rc == 0 and out.startswith("OK"), out
+    assert rc == 0 and "OK checked" in out, out
     # ... and the walk is not vacuous: the same launch over tensors that are one row short is reported, whichever
     # tensor it is (a read through a tile descriptor, a register load, a store)
     for name, cut in (("kd", 192 * 2), ("q", 192 * 2), ("dvd", 192 * 2), ("lse", 4), ("delta", 4), ("do", 16), ("o", 8)):
@@ -124,14 +125,14 @@ def test_the_packed_wide_case_that_faulted_stays_inside_its_tensors(walker):
 def test_packed_batches(walker, case):
     lengths, H, D, L, G, mode, cb = case
     rc, out = run(walker, lengths, H, D, L, G, mode, cb)
-    assert rc == 0 and out.startswith("OK"), out
+    assert rc == 0 and "OK checked" in out, out
 
 
 @pytest.mark.parametrize("case", FIXED, ids=lambda c: f"{c[6]}-B{c[0]}T{c[1]}H{c[2]}D{c[3]}L{c[4]}G{c[5]}")
 def test_fixed_length_batches(walker, case):
     B, T, H, D, L, G, mode, cb, Lv = case
     rc, out = run(walker, (T,), H, D, L, G, mode, cb, packed=False, B=B, Lv=Lv)
-    assert rc == 0 and out.startswith("OK"), out
+    assert rc == 0 and "OK checked" in out, out
 
 
 @pytest.mark.parametrize("case", [
@@ -147,7 +148,7 @@ def test_fixed_length_batches(walker, case):
 def test_value_head_dim_differs(walker, case):
     B, T, H, D, Dv, L, G, mode, cb, Lv = case
     rc, out = run(walker, (T,), H, D, L, G, mode, cb, packed=False, B=B, Lv=Lv, Dv=Dv)
-    assert rc == 0 and out.startswith("OK"), out
+    assert rc == 0 and "OK checked" in out, out
 
 
 def test_row_split_launch(walker):
@@ -155,7 +156,7 @@ def test_row_split_launch(walker):
     segment stay inside q, do, lse and the row sums."""
     for split in (2, 4, 8):
         rc, out = run(walker, (4096,), 1, 128, 0, 2, "causal", packed=False, B=1, split=split)
-        assert rc == 0 and out.startswith("OK"), out
+        assert rc == 0 and "OK checked" in out, out
 
 
 @pytest.mark.parametrize("case", [
@@ -180,3 +181,84 @@ def test_balanced_row_segments_and_row_waves(walker, case):
     rc, out = run(walker, lengths, H, D, L, G, mode, cb, packed=packed, B=B, split=-1)
     assert rc == 0 and "OK" in out, out
     assert (int(out.split("segments=")[1].split()[0]) > 1) == split, out
+
+
+@pytest.mark.parametrize("case", [
+    # B, T, H, D, L, G, mode, launches of the forward and dQ kernels on the 64-wide tiles
+    (257, 33, 1, 64, 2, 1, "noncausal", "fwd_kernel(short) dq_kernel(short)"),            # one 64-row tile a head
+    (130, 70, 2, 40, 0, 2, "causal", "fwd_kernel(short) dq_kernel(short)"),
+    (1100, 20, 1, 64, 1, 1, "noncausal", "fwd_kernel(small) dq_kernel(short, three stages)"),
+    (300, 50, 2, 64, 3, 2, "noncausal", "fwd_kernel(small) dq_kernel(short, three stages)"),
+    (2, 300, 2, 64, 3, 4, "causal", "fwd_kernel(small) dq_kernel(small)"),
+], ids=lambda c: f"{c[6]}-B{c[0]}T{c[1]}")
+def test_launch_shapes_of_the_narrow_tiles(walker, case):
+    B, T, H, D, L, G, mode, shapes = case
+    rc, out = run(walker, (T,), H, D, L, G, mode, packed=False, B=B)
+    assert rc == 0 and out.startswith(shapes + " OK"), out
+
+
+@pytest.mark.parametrize("case", [
+    # T, H, D, L, Lv, G, B: a backward that adds slot Lv of the depth gradients: row waves, row segments
+    (197, 1, 64, 3, 1, 4, 3),
+    (1100, 2, 40, 4, 2, 4, 1),
+])
+def test_own_slot_rows(walker, case):
+    T, H, D, L, Lv, G, B = case
+    args = dict(lengths=(T,), H=H, D=D, L=L, G=G, mode="noncausal", packed=False, B=B, Lv=Lv, split=-1)
+    rc, out = run(walker, env={"WALKER_OWN_SLOT": "1"}, **args)
+    assert rc == 0 and "OK checked" in out, out
+    rc, out = run(walker, env={"WALKER_OWN_SLOT": "1", "WALKER_SHRINK": f"dkd:{2 * H * D * L}"}, **args)
+    assert rc == 1 and "VIOLATION" in out, out
+
+
+FP32 = [
+    # lengths, H, D, Dv, L, Lv, G, mode, chunk tokens, packed, B
+    ((1,), 1, 64, 64, 3, 0, 2, "causal", 0, False, 1),
+    ((15,), 2, 64, 64, 0, 0, 1, "causal", 0, False, 2),
+    ((17,), 3, 4, 4, 7, 0, 3, "causal", 0, False, 1),
+    ((129,), 2, 60, 68, 9, 4, 2, "noncausal", 0, False, 2),
+    ((300,), 2, 128, 128, 12, 0, 4, "causal", 0, False, 1),
+    ((145,), 1, 124, 36, 4, 3, 8, "causal", 0, False, 1),
+    ((70,), 2, 64, 64, 70, 0, 1, "depth_only", 0, False, 1),
+    ((200,), 2, 64, 64, 3, 2, 2, "chunk_visible", 32, False, 1),
+    ((83,), 2, 64, 64, 0, 0, 3, "plain", 0, False, 2),
+    ((40, 0, 1, 133), 2, 64, 64, 3, 0, 2, "causal", 0, True, 1),
+    ((17, 90), 1, 128, 64, 5, 2, 4, "chunk_visible", 16, True, 1),
+    ((50, 3), 1, 100, 100, 2, 0, 1, "depth_only", 0, True, 1),
+]
+
+
+@pytest.mark.parametrize("case", FP32, ids=lambda c: f"{c[7]}-{'_'.join(map(str, c[0]))}-D{c[2]}-Dv{c[3]}-L{c[4]}")
+def test_fp32_kernels(walker, case):
+    lengths, H, D, Dv, L, Lv, G, mode, cb, packed, B = case
+    args = dict(lengths=lengths, H=H, D=D, Dv=Dv, L=L, G=G, mode=mode, cb=cb, packed=packed, B=B, Lv=Lv)
+    rc, out = run(walker, env={"WALKER_FP32": "1"}, **args)
+    assert rc == 0 and "OK checked" in out, out
+    for name, cut in (("q", 16), ("lse", 4), ("do", 16), *((("kd", 16),) if L else (("k", 16),))):
+        rc, out = run(walker, env={"WALKER_FP32": "1", "WALKER_SHRINK": f"{name}:{cut}"}, **args)
+        if Lv and name == "kd":
+            continue  # the last slot holds no data: nobody reads it
+        assert rc == 1 and "VIOLATION" in out, (name, out)
+
+
+@pytest.mark.parametrize("case", [
+    # which: arguments, what the rule has to choose
+    (("linear", 1, 64, 0, 8), "64x64"),
+    (("linear", 65, 192, 0, 72, 24, 136), "64x64"),
+    (("linear", 4999, 64, 1, 1000), "128x128"),
+    (("linear", 8187, 64, 0, 504), "128x64 "),
+    (("linear", 8187, 576, 1, 184, 120), "128x64,3"),
+    *((("norm", rows, dim), "") for dim in (8, 136, 512, 520, 1032, 4096) for rows in (1, 37)),
+    *((("slot", 2, 33, 3, 40, 4, 2, wide, to_cache), "") for wide in (0, 1) for to_cache in (0, 1)),
+], ids=lambda c: "-".join(map(str, c[0])) if isinstance(c, tuple) and isinstance(c[0], tuple) else None)
+def test_dense_and_slot_kernels(walker, case):
+    args, chosen = case
+    for shrink, want in ((None, 0), (f"{'y' if args[0] == 'norm' else 'y0' if args[0] == 'linear' else 'cache_v' if args[-1] else 'v'}:8", 1)):
+        e = dict(os.environ)
+        if shrink:
+            e["WALKER_SHRINK"] = shrink
+        if shrink and args[0] == "slot" and args[-1]:
+            e["WALKER_SHRINK"] = f"cache_v:{2 * 3 * 40 * 2}"  # behind the slot that is written lies one more
+        r = subprocess.run([walker, *map(str, args)], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, env=e, timeout=600)
+        out = r.stdout + r.stderr
+        assert r.returncode == want and out.startswith(chosen) and ("VIOLATION" if want else "OK checked") in out, out
