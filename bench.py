@@ -94,8 +94,8 @@ def make_device_inputs(B, T, Hkv, G, D, L, mode, dev, seed=0):
 
 def bench_fp32_config(dev, steps=20):
     """The benchmark's fp32 configuration (causal, B=1, T=256, H=Hkv=4, D=64, L=4; the reference's CPU-runnable case):
-    forward + backward on fp32 tensors, in exact fp32 on the vector-ALU kernels (the default) and rounded to fp16
-    operands on the matrix kernels (moda_amd.set_fp32_compute("fp16"))."""
+    forward + backward on fp32 tensors, in exact fp32 on the fp32 matrix kernels (the default) and rounded to fp16
+    operands on the 16-bit ones (moda_amd.set_fp32_compute("fp16"))."""
     import torch
     from moda_amd import _lib, ops
 
@@ -104,7 +104,7 @@ def bench_fp32_config(dev, steps=20):
     rn = lambda *s: torch.randn(*s, generator=gen, device=dev, dtype=torch.float32)
     q, k, v, kd, vd, do = rn(B, T, H, D) * D ** -0.5, rn(B, T, H, D), rn(B, T, H, D), rn(B, T * L, H, D), rn(B, T * L, H, D), rn(B, T, H, D)
     out = {"workload": f"c1: causal fp32 B={B} T={T} Hq={H} Hkv={H} G=1 D={D} L={L}"}
-    for setting, key in (("fp32", "ms_exact_fp32_vector_alu"), ("fp16", "ms_fp16_operands_matrix_kernels")):
+    for setting, key in (("fp32", "ms_exact_fp32"), ("fp16", "ms_fp16_operands_matrix_kernels")):
         previous = ops.set_fp32_compute(setting)
         try:
             def step():
@@ -322,13 +322,10 @@ def depth_gradient_kernel(mode, D, G):
     return "depth_cols_kernel"
 
 
-def sequence_dkv_kernel(B, T, Hkv, G, D, compute_units=256):
-    """Name of the launch that forms dk, dv of the sequence keys (moda_amd/csrc/geometry.h: takes_dkv_flat,
-    moda_amd/csrc/capi.hip: desired_dkv_split): short launches on the 64-wide tiles go to the kernel without the
-    role split when they are short or have at least three column tiles per compute unit."""
-    tiles = -(-T // 128) * B * Hkv
-    split = tiles < 512 and (-(-T * G // 64)) // 2 >= 16
-    return "dkv_flat_kernel" if D <= 64 and not split and (T * G <= 512 or tiles >= 3 * compute_units) else "dkv_kernel"
+def sequence_dkv_kernel(D):
+    """Name of the launch that forms dk, dv of the sequence keys in the folded layout (moda_amd/csrc/geometry.h:
+    takes_dkv_flat): on the 64-wide tiles the kernel without the role split."""
+    return "dkv_flat_kernel" if D <= 64 else "dkv_kernel"
 
 
 def recorded_traffic(workload):
@@ -548,7 +545,7 @@ def main():
         mb = min_hbm_bytes(B, T, Hkv, G, D, L, mode)
         gbs = mb / (r["ms_step"] * 1e-3) / 1e9
         whole = sum(v["bytes"] for k, v in traffic.items() if k != "reorg_kernel") if traffic else None
-        launches = ["fwd_kernel", "dq_kernel"] + ([sequence_dkv_kernel(B, T, Hkv, G, D)] if mode != "depth_only" else []) \
+        launches = ["fwd_kernel", "dq_kernel"] + ([sequence_dkv_kernel(D)] if mode != "depth_only" else []) \
             + ([depth_kernel] if depth_kernel else [])
         roofline = {"bound": "hbm", "kernel": " + ".join(launches),
                     "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": gbs / PEAK_HBM_GBS,

@@ -7,8 +7,9 @@
  * elements; the innermost (head-dim) stride is always 1.  For the matrix-core
  * kernels (bf16/fp16, head dims D and Dv multiples of 8 up to 256) every row must be 16-byte
  * aligned (base pointer and all strides multiples of 8 elements) and a row
- * stride must stay below 16 MiB; every other combination runs on vector-ALU
- * kernels that need element alignment only.  All work is enqueued on the hipStream_t passed
+ * stride must stay below 16 MiB.  Every other combination needs element alignment
+ * only: fp32 with head dims up to 128 and 16-byte rows runs on the fp32 matrix
+ * instruction, the rest on vector-ALU kernels.  All work is enqueued on the hipStream_t passed
  * as `stream` (NULL = the legacy default stream); nothing synchronises the
  * host.  The library keeps no mutable state except where a function says so,
  * apart from one flag per kernel variant and device: the first launch of a
@@ -278,7 +279,7 @@ int moda_hip_layer_norm(int32_t dtype, int64_t rows, int64_t dim, const void* x,
 
 /*
  * Which kernels a descriptor runs on: 1 = the matrix-core kernels (tensor rows must then be 16-byte aligned, see
- * the top of this file), 0 = the vector-ALU kernels (element alignment), negative = the descriptor's error code.
+ * the top of this file), 0 = the fp32 or the vector-ALU kernels (element alignment), negative = the descriptor's error code.
  * No counterpart in the reference; lets a host wrapper decide whether an input needs a contiguous copy without
  * repeating the library's rule.  Touches no device.
  */

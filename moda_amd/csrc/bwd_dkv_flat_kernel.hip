@@ -1,5 +1,5 @@
-// Backward, key side, sequence keys of fixed-length launches on the 64-wide tiles: the same products as dkv_kernel
-// (moda_v14.py:874-1248, fla/ops/attn/parallel.py:299-440) without the split into two roles.
+// Backward, key side, sequence keys on the 64-wide tiles where the key head is the query head, fixed-length and packed: the
+// same products as dkv_kernel (moda_v14.py:874-1248, fla/ops/attn/parallel.py:299-440) without the split into two roles.
 //
 // A workgroup of FOUR waves owns 128 key columns of one (batch, kv head), a wave 32 of them with K AND V in
 // registers and BOTH accumulators, dK^T and dV^T; the query rows come by in tiles of 32 (one summation step of the

@@ -1,10 +1,11 @@
-// Reference-grade kernels for everything the MFMA kernels do not cover: fp32
-// tensors, head dims other than 64/128 (any D <= 256, D % 4 == 0) and a value
-// head dim Dv that differs from the key head dim D.  Same
+// Reference-grade kernels for what the matrix kernels do not cover: 16-bit head
+// dims that are not a multiple of 8, fp32 above head dim 128 or with rows off
+// the 16-byte grid (any D, Dv <= 256, multiples of 4), and packed batches with
+// head dims above 128 that come without host offsets.  Same
 // math, same visible sets and the same base-2 conventions as the MFMA kernels,
 // all arithmetic in fp32 on the vector ALU; one 64-lane wave per query row
 // (forward, dQ) or per key / depth column (dK, dV).  Not tuned: meant for small
-// problems such as the reference's fp32 self-test shapes (moda_v14.py:2917).
+// problems.
 #include "kargs.h"
 #include "tile.h"
 

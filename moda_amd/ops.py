@@ -29,8 +29,9 @@ from ._lib import Desc, Strides
 
 _DTYPES = {torch.bfloat16: _lib.BF16, torch.float16: _lib.FP16, torch.float32: _lib.FP32}
 
-# How fp32 tensors are computed.  "fp32": in fp32 on the vector-ALU kernels (exact to fp32 rounding, two orders of
-# magnitude slower than the matrix kernels).  "fp16" / "bf16": the inputs are rounded to that type, the matrix
+# How fp32 tensors are computed.  "fp32": fp32 products and sums throughout, on the fp32 matrix instruction (head dims up
+# to 128, rows on the 16-byte grid; 2 x 4096 tokens, 16 query heads, head dim 128: 9.5 ms forward and backward, through
+# fp16 1.1 ms) or on the vector ALU.  "fp16" / "bf16": the inputs are rounded to that type, the 16-bit matrix
 # kernels run, the results are widened again.  "fp16" is what the reference's own fp32 path amounts to: its
 # tl.dot calls (moda_v14.py:188, 209, 699-712) take the default input precision, which rounds fp32 operands to a
 # 10-bit mantissa (TF32) and accumulates in fp32 -- fp16 has the same mantissa; its range (6e-8 .. 65504) is the
