@@ -196,6 +196,9 @@ class MoDAAttention(nn.Module):
         return x, k, v
 
 
+_MISSING = object()
+
+
 class MoDAStack(nn.Module):
     """``depth`` blocks (attention + MLP) chained through one ``DepthStream``: the body of
     ``MoDAVisionTransformer.forward_features`` (vision_tasks/deit/models.py:376-390) without the patch
@@ -224,13 +227,10 @@ class MoDAStack(nn.Module):
         the constructor made: a replaced, subclassed, patched or hooked module, blocks that differ, active dropout."""
         params, eps, first = [], [], None
         for blk in self.blocks:
-            sub = blk._modules
-            attn, mlp = sub["attn"], sub["mlp"]
-            parts = attn._modules
+            attn, mlp, norm1, norm2 = (blk._modules.get(n) for n in ("attn", "mlp", "norm1", "norm2"))  # none: wrapped
             if type(attn) is not MoDAAttention or type(mlp) is not nn.Sequential or len(mlp) != 3:
                 return None
-            q, kv, proj, drop, kv_ffn = (parts.get(n) for n in ("q", "kv", "proj", "proj_drop", "kv_ffn"))
-            norm1, norm2 = sub["norm1"], sub["norm2"]
+            q, kv, proj, drop, kv_ffn = (attn._modules.get(n) for n in ("q", "kv", "proj", "proj_drop", "kv_ffn"))
             fc1, act, fc2 = mlp._modules.values()
             linears = (q, kv, proj, fc1, fc2) if kv_ffn is None else (q, kv, proj, fc1, fc2, kv_ffn)
             if not (all(type(m) is nn.Linear for m in linears) and type(norm1) is nn.LayerNorm and type(norm2) is nn.LayerNorm
@@ -246,8 +246,9 @@ class MoDAStack(nn.Module):
                 first = what
             if what != first or attn.scale != attn.head_dim ** -0.5:
                 return None
-            tensors = [p for m in (norm1, q, kv, proj, norm2, fc1, fc2) for p in (m._parameters["weight"], m._parameters["bias"])]
-            tensors += [None, None] if kv_ffn is None or not self.ffn_kv else [kv_ffn._parameters["weight"], kv_ffn._parameters["bias"]]
+            # a replica, and a module whose parameters are slices of one flat tensor, hold them as plain attributes
+            tensors = [m._parameters.get(n, _MISSING) for m in (norm1, q, kv, proj, norm2, fc1, fc2) for n in ("weight", "bias")]
+            tensors += [None if kv_ffn is None or not self.ffn_kv else kv_ffn._parameters.get(n, _MISSING) for n in ("weight", "bias")]
             if not all(t is None or type(t) is nn.Parameter for t in tensors):
                 return None
             params.append(tensors)

@@ -661,3 +661,38 @@ def test_ways_back_from_the_native_stack_to_its_modules(monkeypatch, way):
             model(x, inplace_cache=False)
     else:
         _runs_modules(model, x)
+
+
+@pytest.mark.parametrize("way", ["wrapped block", "wrapped attention", "replicas", "plain tensors"])
+def test_a_stack_whose_modules_are_wrapped_runs_them(monkeypatch, way):
+    """What training and sharding wrappers make of a model: a module that stands in front of a block, replicas and flattened
+    parameters, which are attributes and no longer entries of the module's parameters."""
+
+    class Wrapper(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner = inner
+
+        def forward(self, *args, **kwargs):
+            return self.inner(*args, **kwargs)
+
+        def __getattr__(self, name):
+            try:
+                return super().__getattr__(name)
+            except AttributeError:
+                return getattr(self.inner, name)
+
+    model, x, _ = _native_stack(monkeypatch)
+    if way == "wrapped block":
+        model.blocks[0] = Wrapper(model.blocks[0])
+    elif way == "wrapped attention":
+        model.blocks[1].attn = Wrapper(model.blocks[1].attn)
+    else:
+        attn = model.blocks[1].attn
+        linear = attn.q._replicate_for_data_parallel() if way == "replicas" else attn.q
+        for name in ("weight", "bias"):
+            value = getattr(attn.q, name).detach().clone()
+            linear._parameters.pop(name, None)
+            setattr(linear, name, value)
+        attn._modules["q"] = linear
+    _runs_modules(model, x)
