@@ -99,7 +99,7 @@ std::shared_ptr<Packed> pack(const Tensor& cu_seqlens, const Tensor& q, int64_t 
 }
 
 // What a call is besides its tensors.
-struct Call : torch::CustomClassHolder {
+struct Call : c10::intrusive_ptr_target {
   int mode = 0;
   double scale = 1.0;
   int64_t G = 1, chunk_tokens = 0;
@@ -399,28 +399,40 @@ variable_list in_engine(F&& node) {
 Tensor value(const OptTensor& x) { return x.has_value() ? *x : Tensor(); }
 OptTensor optional(const Tensor& x) { return x.defined() ? OptTensor(x) : OptTensor(); }
 
+// What a node keeps from its forward pass besides tensors, in the node's saved data: a tensor that owns it.  Compiled
+// autograd, which replays nodes from a graph of its own, carries tensors through that graph; capsules it refuses.
+template <typename State>
+Tensor owning(const c10::intrusive_ptr<State>& state) {
+  auto* kept = new c10::intrusive_ptr<State>(state);
+  return at::from_blob(kept, {(int64_t)sizeof(*kept)}, [kept](void*) { delete kept; }, at::TensorOptions().dtype(at::kByte));
+}
+template <typename State>
+c10::intrusive_ptr<State> owned(AutogradContext* ctx) {
+  return *static_cast<const c10::intrusive_ptr<State>*>(ctx->saved_data["state"].toTensor().const_data_ptr());
+}
+
 // The autograd node of every operator (moda_v14.py:2649-2789, moda_v16.py:3456-3493, fda_v12.py:1207-1338,
-// fla/ops/attn/parallel.py:632-675): gradient into lse ignored.
+// fla/ops/attn/parallel.py:632-675).  lse has no gradient and is no output of the node: it leaves by the pointer.
 struct Attend : torch::autograd::Function<Attend> {
   static variable_list forward(AutogradContext* ctx, const Tensor& q, const OptTensor& k, const OptTensor& v, const OptTensor& kd,
-                               const OptTensor& vd, const c10::intrusive_ptr<Call>& call) {
+                               const OptTensor& vd, const c10::intrusive_ptr<Call>& call, Tensor* lse) {
     auto r = ::forward(*call, q, value(k), value(v), value(kd), value(vd));
+    *lse = r.second;
     ctx->save_for_backward({q, value(k), value(v), value(kd), value(vd), r.first, r.second});
-    ctx->saved_data["call"] = c10::IValue::make_capsule(call);
+    ctx->saved_data["state"] = owning(call);
     ctx->set_materialize_grads(false);
-    ctx->mark_non_differentiable({r.second});
-    return {r.first, r.second};
+    return {r.first};
   }
   static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
     return in_engine([&] { return gradients(ctx, grads); });
   }
   static variable_list gradients(AutogradContext* ctx, const variable_list& grads) {
     const variable_list s = ctx->get_saved_variables();
-    const auto call = c10::static_intrusive_pointer_cast<Call>(ctx->saved_data["call"].toCapsule());
-    if (!grads[0].defined()) return variable_list(6);
+    const auto call = owned<Call>(ctx);
+    if (!grads[0].defined()) return variable_list(7);
     Grads g = ::backward(*call, s[0], s[1], s[2], s[3], s[4], s[5], s[6], grads[0].to(s[5].scalar_type()), MODA_HIP_STAGE_ALL,
                          nullptr, Tensor(), kOverwrite);
-    return {g[0], g[1], g[2], g[3], g[4], Tensor()};
+    return {g[0], g[1], g[2], g[3], g[4], Tensor(), Tensor()};
   }
 };
 
@@ -471,7 +483,7 @@ void check_folded_contract(int mode, const Tensor& q, const Tensor& k, const Ten
 py::tuple attend(int mode, const Tensor& q, const OptTensor& k, const OptTensor& v, const OptTensor& kd, const OptTensor& vd,
                  std::optional<double> scale, int64_t G, int64_t chunk_tokens, std::optional<int64_t> depth_valid,
                  const OptTensor& cu_seqlens, std::shared_ptr<Packed> packed, bool folded, int64_t group_rows) {
-  variable_list r;
+  Tensor o, lse;
   {
     py::gil_scoped_release nogil;
     if (folded) check_folded_contract(mode, q, value(k), value(kd), value(vd), G);
@@ -480,10 +492,10 @@ py::tuple attend(int mode, const Tensor& q, const OptTensor& k, const OptTensor&
              "To keep depth alignment consistent with backward, BT % moda_group_num must be 0");
     const bool has_depth = kd.has_value() && vd.has_value();  // one without the other counts as none
     const double sc = scale.has_value() ? *scale : 1.0 / std::sqrt((double)q.size(-1));
-    r = Attend::apply(q, k, v, has_depth ? kd : OptTensor(), has_depth ? vd : OptTensor(),
-                      make_call(mode, sc, G, chunk_tokens, depth_valid, std::move(packed)));
+    o = Attend::apply(q, k, v, has_depth ? kd : OptTensor(), has_depth ? vd : OptTensor(),
+                      make_call(mode, sc, G, chunk_tokens, depth_valid, std::move(packed)), &lse)[0];
   }
-  return py::make_tuple(r[0], r[1]);
+  return py::make_tuple(o, lse);
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -519,7 +531,7 @@ void depth_push(const Tensor& k_in, const Tensor& v_in, const Tensor& cache_k, c
 // initialised: slots are read once written.  The nodes of a backward pass run from the last layer to the first; the first
 // attention call among them overwrites the gradients of the slots it saw (`written`), the others, which saw fewer, add to
 // theirs.  Another pass over a retained graph starts over, however much of the stream the one before it reached.
-struct StreamBuffers : torch::CustomClassHolder {
+struct StreamBuffers : c10::intrusive_ptr_target {
   Tensor k, v, gk, gv;
   int64_t L = 0, written = 0;
   int pass = -1;  // the engine's number of the pass that `written` is about
@@ -531,7 +543,7 @@ struct StreamBuffers : torch::CustomClassHolder {
   }
 };
 // An attention call of the stream: what it saw, and the slot its own k, v were pushed to afterwards (-1: none).
-struct StreamCall : torch::CustomClassHolder {
+struct StreamCall : c10::intrusive_ptr_target {
   Call call;
   c10::intrusive_ptr<StreamBuffers> buf;
   int64_t n = 0, slot = -1;
@@ -549,7 +561,7 @@ struct StreamAttend : torch::autograd::Function<StreamAttend> {
     const bool depth = call->n > 0;
     auto r = ::forward(call->call, q, k, v, depth ? call->buf->k : Tensor(), depth ? call->buf->v : Tensor());
     ctx->save_for_backward({q, k, v, r.first, r.second});
-    ctx->saved_data["call"] = c10::IValue::make_capsule(call);
+    ctx->saved_data["state"] = owning(call);
     ctx->set_materialize_grads(false);
     return {r.first, order_token(q)};
   }
@@ -558,7 +570,7 @@ struct StreamAttend : torch::autograd::Function<StreamAttend> {
   }
   static variable_list gradients(AutogradContext* ctx, const variable_list& grads) {
     const variable_list s = ctx->get_saved_variables();
-    const auto call = c10::static_intrusive_pointer_cast<StreamCall>(ctx->saved_data["call"].toCapsule());
+    const auto call = owned<StreamCall>(ctx);
     StreamBuffers& buf = *call->buf;
     buf.enter_pass();
     const Tensor &q = s[0], &k = s[1], &v = s[2], &o = s[3], &lse = s[4];
@@ -597,12 +609,12 @@ struct StreamAttend : torch::autograd::Function<StreamAttend> {
 struct StreamPush : torch::autograd::Function<StreamPush> {
   static variable_list forward(AutogradContext* ctx, const Tensor& k, const Tensor& /*v*/, const Tensor& /*token*/,
                                const c10::intrusive_ptr<StreamCall>& call) {
-    ctx->saved_data["call"] = c10::IValue::make_capsule(call);
+    ctx->saved_data["state"] = owning(call);
     ctx->set_materialize_grads(false);
     return {order_token(k)};
   }
   static variable_list backward(AutogradContext* ctx, const variable_list&) {
-    const auto call = c10::static_intrusive_pointer_cast<StreamCall>(ctx->saved_data["call"].toCapsule());
+    const auto call = owned<StreamCall>(ctx);
     StreamBuffers& buf = *call->buf;
     buf.enter_pass();
     const int64_t B = buf.k.size(0), T = buf.k.size(1) / buf.L, H = buf.k.size(2), D = buf.k.size(3);

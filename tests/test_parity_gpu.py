@@ -1981,3 +1981,34 @@ def test_layer_norm_against_fp64(gpu_device, dim, dtype):
         for got in (y, place):
             assert ((got[:rows].double() - want).abs() <= bound).all(), (rows, ((got[:rows].double() - want).abs() / bound).max())
             assert (got[rows:] == 7.0).all()
+
+
+def test_compiled_autograd_replays_the_native_nodes(gpu_device):
+    """Compiled autograd builds a graph of the backward pass and runs the nodes from it: same launches, same bits, also when
+    the graph is reused for another pass."""
+    import moda_amd
+    import torch._dynamo.compiled_autograd as compiled
+
+    gen = torch.Generator(device=gpu_device).manual_seed(4)
+    rn = lambda *s: (0.5 * torch.randn(*s, generator=gen, device=gpu_device)).bfloat16().requires_grad_()
+    cu = torch.tensor([0, 20, 64], device=gpu_device)
+
+    def operator(q, k, v):
+        return moda_amd.parallel_moda(q, k, v, moda_group_num=2, cu_seqlens=cu).float().square().sum()
+
+    def stream(q, k, v):
+        s, total = moda_amd.DepthStream(3), 0
+        for i in range(3):
+            total = total + s.attend(q * (i + 1), k, v, moda_group_num=2).float().square().sum()
+            s.push(k, v)
+        return total
+
+    for call in (operator, stream):
+        for _ in range(2):
+            xs = [rn(1, 128, 2, 64), rn(1, 64, 2, 64), rn(1, 64, 2, 64)]
+            want = torch.autograd.grad(call(*xs), xs)
+            total = call(*xs)
+            with compiled._enable(lambda graph: graph):
+                total.backward()
+            for x, w in zip(xs, want):
+                assert torch.equal(x.grad, w), call.__name__
