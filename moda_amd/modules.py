@@ -27,7 +27,7 @@ from torch import nn
 
 from . import _lib
 from .depth_cache import DepthCache, stack_depth
-from .ops import _chunk_tokens, parallel_moda, parallel_moda_chunk_visible
+from .ops import _chunk_tokens, _tracing, parallel_moda, parallel_moda_chunk_visible
 
 
 class DepthStream:
@@ -61,7 +61,7 @@ class DepthStream:
         if self._mode is not None:
             return
         grads = torch.is_grad_enabled() and (k.requires_grad or v.requires_grad)
-        if self._inplace is False or (grads and self._used_context) or torch.jit.is_tracing():
+        if self._inplace is False or (grads and self._used_context) or _tracing():
             self._mode = "rebuild"
         else:
             self._mode = "train" if grads else "infer"
@@ -81,7 +81,7 @@ class DepthStream:
         self._n += 1
 
     def _native(self):
-        if torch.jit.is_tracing():
+        if _tracing():
             raise RuntimeError("a depth stream that began in place cannot be traced: create it inside the traced function")
         if self._train is None:
             self._train = _lib.host().TrainStream(self.max_layers)
@@ -105,7 +105,7 @@ class DepthStream:
         chunk_visible = chunk_rows is not None
         assert not chunk_visible or is_causal, "chunk-visible attention is causal"
         if self._mode == "train" or (self._mode is None and self._inplace is not False and not self._used_context
-                                     and not torch.jit.is_tracing() and torch.is_grad_enabled()
+                                     and not _tracing() and torch.is_grad_enabled()
                                      and (q.requires_grad or k.requires_grad)):
             # the same argument contract as parallel_moda, which is bypassed here
             assert q.shape[2] == k.shape[2] and q.shape[1] == k.shape[1] * moda_group_num, \
@@ -262,7 +262,7 @@ class MoDAStack(nn.Module):
         run one by one.  Twelve blocks of width 256 on 64 x 197 tokens issue some 200 framework operations of about
         10 us host time each when run as modules."""
         attn = self.blocks[0].attn if len(self.blocks) else None
-        if (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or torch.jit.is_tracing()
+        if (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or _tracing()
                 or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() or type(attn) is not MoDAAttention
                 or nn.modules.module._global_forward_hooks or nn.modules.module._global_forward_pre_hooks
                 or type(x) is not torch.Tensor or x.dim() != 3 or x.shape[-1] != attn.num_heads * attn.head_dim):

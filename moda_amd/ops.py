@@ -27,6 +27,8 @@ import torch
 from . import _lib
 from ._lib import Desc, Strides
 
+_tracing = torch._C._get_tracing_state  # true while torch.jit.trace records (torch.jit.is_tracing takes twice as long)
+
 _DTYPES = {torch.bfloat16: _lib.BF16, torch.float16: _lib.FP16, torch.float32: _lib.FP32}
 
 # How fp32 tensors are computed.  "fp32": fp32 products and sums throughout, on the fp32 matrix instruction (head dims up
@@ -269,7 +271,7 @@ class _AttentionFunction(torch.autograd.Function):
 
     @classmethod
     def apply(cls, *args, **kwargs):
-        if cls in _NATIVE_FUNCTIONS and not torch.jit.is_tracing():
+        if cls in _NATIVE_FUNCTIONS and not _tracing():
             return cls._attend(*args, **kwargs)
         return super().apply(*args, **kwargs)
 
@@ -368,7 +370,7 @@ def parallel_moda(q, k, v, g=None, cached_k=None, cached_v=None, scale=None, cu_
     if g is not None:
         _refuse_decay(g, q)
     mode = _lib.CAUSAL if is_causal else _lib.NONCAUSAL
-    if torch.jit.is_tracing():
+    if _tracing():
         _lib.host().check_folded_contract(mode, q, k, cached_k, cached_v, moda_group_num)
         out = ParallelMixtureOfDepthAttentionFunction.apply(q, k, v, None, scale, cu_seqlens, cached_k, cached_v, moda_group_num,
                                                             is_causal, None, None, None, None, depth_valid)
@@ -466,7 +468,7 @@ def parallel_moda_chunk_visible(q, k, v, g=None, cached_k=None, cached_v=None, s
         _warn_depth_grads(cached_k, cached_v)
     if g is not None:
         _refuse_decay(g, q)
-    if torch.jit.is_tracing():
+    if _tracing():
         _lib.host().check_folded_contract(_lib.CHUNK_VISIBLE, q, k, cached_k, cached_v, moda_group_num)
         out = ParallelMixtureOfDepthAttentionChunkVisibleFunction.apply(q, k, v, None, scale, cu_seqlens, cached_k, cached_v,
                                                                         moda_group_num, chunk_rows, depth_valid)
@@ -553,7 +555,7 @@ def parallel_fda(q, k=None, v=None, g=None, cached_k=None, cached_v=None, scale=
         _warn_depth_grads(cached_k, cached_v)
     if g is not None:
         _refuse_decay(g, q)
-    if torch.jit.is_tracing():
+    if _tracing():
         _lib.host().check_folded_contract(_lib.DEPTH_ONLY, q, None, cached_k, cached_v, moda_group_num)
         out = ParallelFlashDepthAttentionFunction.apply(q, None, None, None, scale, cu_seqlens, cached_k, cached_v, moda_group_num)
     else:
