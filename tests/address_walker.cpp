@@ -55,12 +55,16 @@ struct Region {
 std::map<std::string, Region> g_regions;
 long long g_checked = 0, g_dma_in = 0, g_dma_out = 0;
 bool g_fp32 = false, g_own_slot = false;
-std::string g_ctx;
+struct Where {  // put into words when there is something to say
+  const char* kernel;
+  int block, wave, lane;
+  const char* what;
+} g_where = {"", 0, 0, 0, ""};
 
 [[noreturn]] void fail(const char* fmt, ...) {
   va_list ap;
   va_start(ap, fmt);
-  fprintf(stdout, "VIOLATION [%s] ", g_ctx.c_str());
+  fprintf(stdout, "VIOLATION [%s block %d wave %d lane %d: %s] ", g_where.kernel, g_where.block, g_where.wave, g_where.lane, g_where.what);
   vfprintf(stdout, fmt, ap);
   fprintf(stdout, "\n");
   va_end(ap);
@@ -220,9 +224,7 @@ KArgs seq_args(const KArgs& in, int& b) {
 }
 
 void ctx(const char* kernel, int block, int wave, int lane, const char* what) {
-  char buf[256];
-  snprintf(buf, sizeof(buf), "%s block %d wave %d lane %d: %s", kernel, block, wave, lane, what);
-  g_ctx = buf;
+  g_where = {kernel, block, wave, lane, what};
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1168,7 +1170,6 @@ void walk_all(const Case& c, const KArgs& a) {
   const bool small = a.cu ? use_small_rows(a.delta_pitch, a.Hq, a.compute_units) : use_small_rows(a.Tq, (long long)a.B * a.Hq, a.compute_units);
   const ShortRows rows = a.cu ? ShortRows::kNone : pick_short_rows(a.Tq, (long long)a.B * a.Hq, a.causal, a.compute_units);
   // ---- forward
-  g_ctx = "forward";
   const auto ring = [](int NST) { return (uint32_t)NST * 2 * 64 * HD * 2; };
   const auto fwd = [&](auto shape, const char* name) {
     typedef decltype(shape) Shape;
