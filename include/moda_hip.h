@@ -278,6 +278,41 @@ int moda_hip_layer_norm(int32_t dtype, int64_t rows, int64_t dim, const void* x,
                         void* y, void* stream);
 
 /*
+ * What a transformer block does with a row between its attention call and the next block's, in one launch:
+ *   y = residual + proj(attention);  y = y + fc2(gelu(fc1(mid_norm(y)));  x = y;  parts = W end_norm(y)        (post_norm 0)
+ *   y = mid_norm(residual + proj(attention));  y = end_norm(y + fc2(gelu(fc1(y))));  x = y;  parts = W y          (post_norm 1)
+ * rounded to 16 bits wherever one of the pieces above hands a result on.  attention, residual, x: [rows, width] contiguous
+ * (x may be the residual); parts: up to three projections as in moda_hip_linear, n_parts 0: none (end_norm is then not
+ * read where post_norm is 0).  width 128, 256, 384 or 512, hidden a multiple of 128, each part's n of 16: MODA_HIP_EUNSUPPORTED
+ * otherwise (use the pieces).  Pointers on 16-byte boundaries (biases: 8; they may be NULL).
+ * All weights (proj, fc1, fc2, parts) as moda_hip_pack_weights leaves them.
+ */
+typedef struct moda_hip_block_tail_args {
+  int32_t struct_size, dtype;
+  int64_t rows, width, hidden;
+  const void *attention, *residual;
+  void* x;
+  const void *proj_w, *proj_b, *fc1_w, *fc1_b, *fc2_w, *fc2_b;
+  const void *mid_norm_w, *mid_norm_b, *end_norm_w, *end_norm_b;
+  const void* gelu_table;
+  float mid_norm_eps, end_norm_eps;
+  int32_t post_norm, n_parts;
+  moda_hip_linear_part parts[3];
+} moda_hip_block_tail_args;
+/* the weights of a block tail are packed copies: n matrices [rows n][k], n a multiple of 16, k of 32, 16-byte boundaries, each
+ * to n * k elements at `packed` (the 16-row blocks one after the other, so rows from a multiple of 16 on start at their
+ * own multiple of k); n >= 1.  gelu_table (MODA_HIP_GELU_TABLE_BYTES, 16-byte boundary, or NULL) receives the table that bf16
+ * block tails read. */
+#define MODA_HIP_GELU_TABLE_BYTES 21504
+typedef struct moda_hip_weight {
+  const void* w;
+  void* packed;
+  int64_t n, k;
+} moda_hip_weight;
+int moda_hip_pack_weights(const moda_hip_weight* weights, int32_t n, void* gelu_table, void* stream);
+int moda_hip_block_tail(const moda_hip_block_tail_args* args, void* stream);
+
+/*
  * Which kernels a descriptor runs on: 1 = the matrix-core kernels (tensor rows must then be 16-byte aligned, see
  * the top of this file), 0 = the fp32 or the vector-ALU kernels (element alignment), negative = the descriptor's error code.
  * No counterpart in the reference; lets a host wrapper decide whether an input needs a contiguous copy without

@@ -4,6 +4,7 @@
 #include <algorithm>
 
 #include "../../include/moda_hip.h"
+#include "block.h"
 #include "geometry.h"
 #include "tile.h"
 #include "tile16.h"
@@ -25,24 +26,6 @@ struct LinearArgs {
 };
 
 enum Epilogue { kBias, kGelu, kResidual };
-
-// The exact GELU, x Phi(x) = max(x, 0) - |x| / 2 erfc(|x| / sqrt 2).  erfc(z) = exp(-z^2) t R(t) with t = 1 / (1 + 0.38 z):
-// R is a degree-6 fit of erfcx(z) / t over [0, 12], relative error 1.1e-6 -- three hundred times below a rounding to 11
-// bits, in both tails.  A fifth of the instructions of erff, which took two thirds of the launch.  The first term is
-// x - min(x, 0), which is NaN for minus infinity, as -inf (1 + erf(-inf)) is.  The clamp is a median, which takes a value
-// as it comes, where fminf has it made canonical first: one instruction less, what the other form of the first term costs.
-__device__ __forceinline__ float gelu(float x) {
-  const float a = __builtin_amdgcn_fmed3f(fabsf(x), 0.f, 14.f);  // beyond, the second term is below 1e-43
-  const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(a, 0.38f * 0.70710678f, 1.f));
-  float r = -0.12541133165359497f;
-  r = __builtin_fmaf(r, t, 0.3360145092010498f);
-  r = __builtin_fmaf(r, t, -0.06988266855478287f);
-  r = __builtin_fmaf(r, t, 0.24781261384487152f);
-  r = __builtin_fmaf(r, t, 0.18060259521007538f);
-  r = __builtin_fmaf(r, t, 0.21657583117485046f);
-  r = __builtin_fmaf(r, t, 0.2142874300479889f);
-  return (x - fminf(x, 0.f)) - 0.5f * a * t * r * fast_exp2(a * a * (-0.5f * kLog2e));
-}
 
 // y = x W^T: both operands have the summation index innermost, so a k step is a 64-element-wide tile of each, staged
 // like the attention kernels' 64-wide tiles.  Four waves share a BM (rows) x BN (features) output tile, two by two.

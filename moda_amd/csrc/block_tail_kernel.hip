@@ -1,0 +1,568 @@
+// Everything a transformer block does with a row between two attention calls, in one launch: output projection and
+// residual, layer norm, MLP with exact GELU and residual, layer norm and the projections of the next block.  All of it is
+// local to a row, so a workgroup takes BM rows through the whole chain; what one step hands to the next stays in
+// registers and LDS.  As separate launches (block_kernels.hip) the same rows went to memory and back six times, the
+// hidden activations of the MLP, four times as wide, among them: 12 608 rows of width 256 took 69 us in seven launches
+// (projection 9, norm 6, MLP 23 + 15, norm 6, next projections 10.5), here 32.8.
+//
+// Eight waves share the BM rows and divide the features of every product.  The weights sit on the matrix instruction's A
+// side (M = features) and go from memory (L2 after the first workgroup of an XCD) straight into the registers that it
+// reads: no two waves of a workgroup read the same weight, so LDS would only add a trip.  The rows sit on the B side
+// (N = rows) and come from LDS, where all waves read them.  A lane ends up with four consecutive features of a row.
+//
+// 64 rows where they give each compute unit a workgroup, else 32: a compute unit takes in 64 bytes of weights a cycle, and with
+// 32 rows it waits for them.  (Two workgroups of 32 rows a compute unit instead: 48 us.)
+//
+// What bounds it, per 64 rows at width 256, hidden 1024, a next block with 384 projected features, measured cycles of 63 k: the
+// MLP's products 21 k (16 k of matrix instructions), its activation 9.4 k, waiting for each other 4 k; rows in 5 k, the two
+// projections 9 k, norms and residuals 11 k, rows out 5 k.  The activation's vector work does not overlap with the products:
+// run beside the next chunk's first product, or with the two waves of a SIMD half a chunk apart, it needs more registers than
+// there are (72 spilled, 44 us; with half the weights in flight 37).
+#include <type_traits>
+
+#include "../../include/moda_hip.h"
+#include "block.h"
+#include "tile.h"
+#include "tile16.h"
+#include "tuning.h"
+
+namespace moda {
+
+struct TailPart {
+  const uint16_t *w, *bias;
+  uint16_t* y;
+  int64_t ldy;
+  int n, block_end;  // output features; 16-feature blocks of this part and of those before it
+};
+struct TailArgs {
+  const uint16_t *h, *res;  // attention output, residual stream
+  uint16_t* x;              // residual stream after the block
+  int rows, hidden, n_parts;
+  const uint16_t *proj_w, *proj_b, *fc1_w, *fc1_b, *fc2_w, *fc2_b;
+  // layer norms: after the projection, and after the MLP (before-norm blocks: the next block's first norm)
+  const uint16_t *mid_w, *mid_b, *end_w, *end_b;
+  float mid_eps, end_eps;
+  const float* gelu_table;  // bf16: written with the packed weights
+  TailPart part[3];  // projections of the next block
+};
+
+namespace {
+
+#define MODA_INLINE __attribute__((always_inline))  // lambdas: what they capture stays in registers
+
+// workgroup barrier that waits for this wave's LDS accesses only: weights on their way to registers stay on their way
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// GELU of a packed pair of 16-bit values.  A bf16 value has 2 x 2688 magnitudes between 2^-17 and 16, outside of which Phi is
+// 0.5 or 0 and 1 to 3e-6 relative: x Phi(x) with Phi from a table in LDS, 8 vector instructions an element where the
+// formula (which fp16 takes) has 22, 6.5 k cycles for 64 rows x 256 features against 2.4 k (the launch 40 -> 32.7 us).
+constexpr int kGeluHalf = 21 * 128, kGeluTable = 2 * kGeluHalf, kGeluFirst = (127 - 17) << 7;
+template <typename T>
+constexpr int table_bytes() {
+  return std::is_same<T, BF16>::value ? kGeluTable * 4 : 0;
+}
+template <typename T>
+__device__ __forceinline__ int activated(int w, MODA_LDS const char* table) {
+  float x[2];
+  unpack2<T>(w, x[0], x[1]);
+  if constexpr (table_bytes<T>() > 0) {
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    const u16x2 first = {kGeluFirst, kGeluFirst}, last = {kGeluHalf - 1, kGeluHalf - 1}, other = {4 * kGeluHalf, 4 * kGeluHalf};
+    const u16x2 mag = __builtin_bit_cast(u16x2, w & 0x7fff7fff), sign = __builtin_bit_cast(u16x2, (int)(((unsigned)w >> 15) & 0x10001u));
+    const u16x2 at = __builtin_elementwise_min(__builtin_elementwise_sub_sat(mag, first), last) * (unsigned short)4 + sign * other;
+    const unsigned bytes = __builtin_bit_cast(unsigned, at);
+    x[0] *= *reinterpret_cast<MODA_LDS const float*>(table + (bytes & 0xffffu));
+    x[1] *= *reinterpret_cast<MODA_LDS const float*>(table + (bytes >> 16));
+    return pack2<T>(x[0], x[1]);
+  } else {
+    return pack2<T>(gelu(x[0]), gelu(x[1]));
+  }
+}
+
+// sum over the TPR neighbouring lanes (8 or 16) of a row
+template <int TPR>
+__device__ __forceinline__ float lane_group_sum(float v) {
+  static_assert(TPR == 8 || TPR == 16, "half or whole rows of sixteen lanes");
+#if defined(__HIP_DEVICE_COMPILE__)
+  auto add = [&](auto ctrl) {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  add(std::integral_constant<int, 0xB1>{});   // quad_perm 1, 0, 3, 2
+  add(std::integral_constant<int, 0x4E>{});   // quad_perm 2, 3, 0, 1
+  add(std::integral_constant<int, 0x141>{});  // row_half_mirror
+  if (TPR == 16) add(std::integral_constant<int, 0x140>{});  // row_mirror
+#endif
+  return v;
+}
+
+// Rows of W 16-bit elements in LDS, 16-byte chunks swizzled as Tile<> has them for rows of 256 bytes and more.
+template <int W>
+struct Rows {
+  static_assert(W % 128 == 0, "rows start at bank 0");
+  __device__ __forceinline__ static int swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+  __device__ __forceinline__ static int off(int row, int chunk) { return row * W + ((chunk ^ swz(row)) << 3); }
+  // B operand of rows row0 + sigma(0..15), features 32 ks .. +31 (see Operand16); base: off(sigma(n), q4 + 4 j) for j = 0..3
+  __device__ __forceinline__ static i32x4 operand(lds_cptr tile, const int (&base)[4], int row0, int ks) {
+    return *reinterpret_cast<MODA_LDS const i32x4*>(tile + base[ks & 3] + row0 * W + (ks >> 2) * 128);
+  }
+};
+
+// acc[mb][nb] += weights (MB blocks of 16 features) x rows (NB blocks of 16), K innermost.  PF steps of 32 of the weights
+// are on their way; start() sends for the first ones, before what produces the rows.
+template <typename T, int MB, int NB>
+struct Product {
+  static constexpr int PF = MB <= 3 ? 4 : 2;
+  i32x4 w[PF][MB];
+  const uint16_t* base[MB];  // wave-uniform: packed block of the features, at the first step of the sum
+  uint32_t voff;             // this lane's byte offset
+
+  __device__ __forceinline__ i32x4 get(int mb, int ks) const {
+    typedef __attribute__((address_space(1))) const i32x4* vec;
+    return *(vec)((__attribute__((address_space(1))) const char*)base[mb] + (size_t)voff + (size_t)ks * 1024);
+  }
+  __device__ __forceinline__ void start() {
+#pragma unroll
+    for (int j = 0; j < PF; j++)
+#pragma unroll
+      for (int mb = 0; mb < MB; mb++) w[j][mb] = get(mb, j);
+  }
+  template <int W>
+  __device__ __forceinline__ static void rows(i32x4 (&x)[NB], lds_cptr tile, const int (&rbase)[4], int ks) {
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) x[nb] = Rows<W>::operand(tile, rbase, 16 * nb, ks);
+  }
+  __device__ __forceinline__ void step(const i32x4 (&wj)[MB], const i32x4 (&x)[NB], f32x4 (&acc)[MB][NB]) const {
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+      for (int mb = 0; mb < MB; mb++) acc[mb][nb] = mfma16<T>(wj[mb], x[nb], acc[mb][nb]);
+  }
+  // nk: steps of 32, a multiple of four.  The rows' operands of the next step are on their way while this one's products run.
+  template <int W>
+  __device__ __forceinline__ void run(lds_cptr tile, const int (&rbase)[4], int nk, f32x4 (&acc)[MB][NB]) {
+    i32x4 x[2][NB];
+    rows<W>(x[0], tile, rbase, 0);
+    for (int k0 = 0; k0 < nk; k0 += 4) {
+      lds_cptr at = tile + k0 * 32;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        if (j < 3 || k0 + 4 < nk) rows<W>(x[(j + 1) & 1], at, rbase, j + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        step(w[j % PF], x[j & 1], acc);
+        if (k0 + j + PF < nk) {
+#pragma unroll
+          for (int mb = 0; mb < MB; mb++) w[j % PF][mb] = get(mb, k0 + j + PF);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+};
+
+}  // namespace
+
+template <typename T, int C, int NB, bool POST>
+__global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
+  constexpr int BM = 16 * NB, MB2 = C / 128, MB1 = 2, HC = 128 * MB1, CH = C / 8, TPR = 512 / BM, NL = CH / TPR;
+  static_assert(CH % TPR == 0, "a row's chunks over the threads of the row");
+  extern __shared__ __align__(16) unsigned char tail_smem[];
+  MODA_LDS const char* table = (MODA_LDS const char*)(lds_ptr)tail_smem;  // kGeluTable floats (bf16)
+  lds_ptr X = (lds_ptr)tail_smem + (table_bytes<T>() / 2);  // [BM][C]: the block's rows
+  lds_ptr H = X + BM * C;          // [BM][C] attention output, then two stages of [BM][HC] hidden activations
+  const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, q4 = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r0 = blockIdx.x * BM;
+  const int sigma = slot_base(n >> 2) + (n & 3);  // tile row of a 16-row block that lane column n stands for
+  int xbase[4], hbase[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    xbase[j] = Rows<C>::off(sigma, 4 * j + q4);
+    hbase[j] = Rows<HC>::off(sigma, 4 * j + q4);
+  }
+  const i32x2 none = {0, 0};
+  auto unpack4 = [](const i32x2& w, float (&f)[4]) {
+    unpack2<T>(w[0], f[0], f[1]);
+    unpack2<T>(w[1], f[2], f[3]);
+  };
+  auto pack4 = [](const float (&f)[4]) {
+    i32x2 w;
+    w[0] = pack2<T>(f[0], f[1]);
+    w[1] = pack2<T>(f[2], f[3]);
+    return w;
+  };
+  auto zero = [](auto& acc) {
+    for (auto& row : acc)
+      for (auto& x : row) x = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  const int f2 = wave * 16 * MB2;  // this wave's features of a C-wide product
+  // a bias's pieces at feature f of this wave, four features a lane
+  auto pieces = [&](const uint16_t* bias, int f, auto& to) MODA_INLINE {
+#pragma unroll
+    for (int mb = 0; mb < (int)(sizeof(to) / sizeof(to[0])); mb++)
+      to[mb] = bias ? *reinterpret_cast<const i32x2*>(bias + f + 16 * mb + 4 * q4) : none;
+  };
+
+  // Attention output, projection weights, residual and GELU table set out together, by rows (a load in the products' layout
+  // would touch sixteen rows in each quarter of its lanes).
+  Product<T, MB2, NB> proj;
+  proj.voff = lane * 16;
+  i32x2 bias2[MB2];
+  {
+    constexpr int N = BM * CH / 512, NT = table_bytes<T>() / 16;
+    static_assert(BM * CH % 512 == 0, "whole passes");
+    i32x4 v[N], res[N], tab[(NT + 511) / 512 + 1];
+    auto fetch = [&](const uint16_t* from, i32x4 (&to)[N]) MODA_INLINE {  // past the last row: that row's again, never stored
+#pragma unroll
+      for (int j = 0; j < N; j++) {
+        const int row = r0 + (tid + 512 * j) / CH;
+        to[j] = *reinterpret_cast<const i32x4*>(from + (int64_t)(row < a.rows ? row : a.rows - 1) * C + (tid + 512 * j) % CH * 8);
+      }
+    };
+    auto leave = [&](lds_ptr tile, const i32x4 (&from)[N]) MODA_INLINE {
+#pragma unroll
+      for (int j = 0; j < N; j++) *reinterpret_cast<MODA_LDS i32x4*>(tile + Rows<C>::off((tid + 512 * j) / CH, (tid + 512 * j) % CH)) = from[j];
+    };
+    fetch(a.h, v);
+#pragma unroll
+    for (int mb = 0; mb < MB2; mb++) proj.base[mb] = a.proj_w + (size_t)(f2 + 16 * mb) * C;
+    proj.start();
+    fetch(a.res, res);
+#pragma unroll
+    for (int j = 0; j < (NT + 511) / 512; j++) tab[j] = reinterpret_cast<const i32x4*>(a.gelu_table)[tid + 512 * j < NT ? tid + 512 * j : 0];
+    pieces(a.proj_b, f2, bias2);
+    leave(H, v);
+    leave(X, res);
+#pragma unroll
+    for (int j = 0; j < (NT + 511) / 512; j++)
+      if (tid + 512 * j < NT) reinterpret_cast<MODA_LDS i32x4*>((lds_ptr)tail_smem)[tid + 512 * j] = tab[j];
+  }
+  i32x2 keep[MB2][NB];  // this lane's pieces of what the MLP's result is added to, rounded
+  lds_barrier();
+  f32x4 acc[MB2][NB];
+  // (rows 16 apart share their swizzle: one address per feature block)
+  auto own_piece = [&](int mb, int nb) { return X + Rows<C>::off(sigma, (f2 >> 3) + 2 * mb + (q4 >> 1)) + 4 * (q4 & 1) + 16 * nb * C; };
+  // + bias, rounded as the linear layer's result, + keep, rounded: into keep and the row tile
+  auto add_keep = [&]() MODA_INLINE {
+#pragma unroll
+    for (int mb = 0; mb < MB2; mb++) {
+      float b[4];
+      unpack4(bias2[mb], b);
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) {
+        float x[4], k[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = acc[mb][nb][i] + b[i];
+        unpack4(pack4(x), x);
+        unpack4(keep[mb][nb], k);
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] += k[i];
+        keep[mb][nb] = pack4(x);
+        *reinterpret_cast<MODA_LDS i32x2*>(own_piece(mb, nb)) = keep[mb][nb];
+      }
+    }
+  };
+  // Layer norm of the row tile in place, TPR threads a row; `out`: the rows also go there, normalised (POST) or as they
+  // were.  Parameters are fetched ahead of the barrier, by fetch_norm.
+  const int lrow = tid / TPR, lsub = tid % TPR;
+  i32x4 wv[NL], bv[NL];
+  auto fetch_norm = [&](const uint16_t* weight, const uint16_t* bias) MODA_INLINE {
+#pragma unroll
+    for (int j = 0; j < NL; j++) {
+      wv[j] = *reinterpret_cast<const i32x4*>(weight + (lsub + TPR * j) * 8);
+      bv[j] = *reinterpret_cast<const i32x4*>(bias + (lsub + TPR * j) * 8);
+    }
+  };
+  auto layer_norm = [&](bool normalise, float eps, uint16_t* out) MODA_INLINE {
+    auto load8 = [](const i32x4& v, float (&f)[8]) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) unpack2<T>(v[i], f[2 * i], f[2 * i + 1]);
+    };
+    lds_barrier();
+    float f[NL][8], s = 0.f;
+    i32x4 raw[NL];
+#pragma unroll
+    for (int j = 0; j < NL; j++) {
+      raw[j] = *reinterpret_cast<MODA_LDS const i32x4*>(X + Rows<C>::off(lrow, lsub + TPR * j));
+      load8(raw[j], f[j]);
+#pragma unroll
+      for (int i = 0; i < 8; i++) s += f[j][i];
+    }
+    const bool store = out && r0 + lrow < a.rows;
+    if (!POST && store) {
+#pragma unroll
+      for (int j = 0; j < NL; j++) *reinterpret_cast<i32x4*>(out + (int64_t)(r0 + lrow) * C + (lsub + TPR * j) * 8) = raw[j];
+    }
+    if (normalise) {
+      const float mean = lane_group_sum<TPR>(s) / C;
+      float v = 0.f;
+#pragma unroll
+      for (int j = 0; j < NL; j++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          const float d = f[j][i] - mean;
+          v = __builtin_fmaf(d, d, v);
+        }
+      const float rstd = rsqrtf(lane_group_sum<TPR>(v) / C + eps);
+#pragma unroll
+      for (int j = 0; j < NL; j++) {
+        float w[8], b[8];
+        load8(wv[j], w);
+        load8(bv[j], b);
+        i32x4 o;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          o[i] = pack2<T>((f[j][2 * i] - mean) * rstd * w[2 * i] + b[2 * i], (f[j][2 * i + 1] - mean) * rstd * w[2 * i + 1] + b[2 * i + 1]);
+        *reinterpret_cast<MODA_LDS i32x4*>(X + Rows<C>::off(lrow, lsub + TPR * j)) = o;
+        if (POST && store) *reinterpret_cast<i32x4*>(out + (int64_t)(r0 + lrow) * C + (lsub + TPR * j) * 8) = o;
+      }
+    }
+    lds_barrier();
+  };
+
+  auto read_keep = [&]() MODA_INLINE {
+#pragma unroll
+    for (int mb = 0; mb < MB2; mb++)
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) keep[mb][nb] = *reinterpret_cast<MODA_LDS const i32x2*>(own_piece(mb, nb));
+  };
+  zero(acc);
+  proj.template run<C>(H, xbase, C / 32, acc);
+  read_keep();  // (the pieces that add_keep overwrites are the ones this lane reads)
+  // this wave's features of the hidden chunk that starts at c0: f1 = c0 + wave * 16 * MB1, none in a short last chunk
+  Product<T, MB1, NB> fc1;
+  fc1.voff = lane * 16;
+  i32x2 bias1[MB1];
+  auto has_features = [&](int c0) { return c0 + wave * 16 * MB1 < a.hidden; };
+  auto start_fc1 = [&](int c0) MODA_INLINE {
+    if (!has_features(c0)) return;
+    const int f1 = c0 + wave * 16 * MB1;
+#pragma unroll
+    for (int mb = 0; mb < MB1; mb++) fc1.base[mb] = a.fc1_w + (size_t)(f1 + 16 * mb) * C;
+    fc1.start();
+    pieces(a.fc1_b, f1, bias1);
+  };
+  start_fc1(0);
+  fetch_norm(a.mid_w, a.mid_b);
+  add_keep();
+  layer_norm(true, a.mid_eps, nullptr);
+  if (POST) read_keep();
+
+  // MLP, HC hidden features at a time; two stages of hidden activations, so that one barrier a chunk is enough
+  zero(acc);
+  Product<T, MB2, NB> fc2;
+  fc2.voff = lane * 16;
+  lds_ptr Hs = H;
+  for (int c0 = 0; c0 < a.hidden; c0 += HC) {
+    if (has_features(c0)) {
+      f32x4 hid[MB1][NB];
+#pragma unroll
+      for (int mb = 0; mb < MB1; mb++) {  // sums start from the bias
+        float b[4];
+        unpack4(bias1[mb], b);
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) hid[mb][nb] = f32x4{b[0], b[1], b[2], b[3]};
+      }
+      fc1.template run<C>(X, xbase, C / 32, hid);
+#pragma unroll
+      for (int mb = 0; mb < MB1; mb++)
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) {
+          i32x2 w;  // the linear layer's own result is a 16-bit value, as it is when the layers run one by one
+          w[0] = activated<T>(pack2<T>(hid[mb][nb][0], hid[mb][nb][1]), table);
+          w[1] = activated<T>(pack2<T>(hid[mb][nb][2], hid[mb][nb][3]), table);
+          *reinterpret_cast<MODA_LDS i32x2*>(Hs + Rows<HC>::off(sigma, wave * 2 * MB1 + 2 * mb + (q4 >> 1)) + 4 * (q4 & 1) + 16 * nb * HC) = w;
+        }
+    }
+#pragma unroll
+    for (int mb = 0; mb < MB2; mb++) fc2.base[mb] = a.fc2_w + (size_t)(f2 + 16 * mb) * a.hidden + c0 * 16;
+    fc2.start();
+    lds_barrier();
+    const int left = a.hidden - c0;
+    fc2.template run<HC>(Hs, hbase, (left < HC ? left : HC) / 32, acc);
+    if (c0 + HC < a.hidden) start_fc1(c0 + HC);
+    Hs = Hs == H ? H + BM * HC : H;
+  }
+  pieces(a.fc2_b, f2, bias2);
+  const bool end_norm = POST || a.n_parts > 0;
+  if (end_norm) fetch_norm(a.end_w, a.end_b);
+  add_keep();
+  layer_norm(end_norm, a.end_eps, a.x);
+  if (a.n_parts == 0) return;
+
+  // Projections of the next block: 8 MBQ blocks of 16 features a turn, MBQ a wave, so many that one turn is enough where
+  // four are.  Results leave through LDS, by rows.
+  const int end0 = a.part[0].block_end, end1 = a.n_parts > 1 ? a.part[1].block_end : end0, blocks = a.part[a.n_parts - 1].block_end;
+  auto projections = [&](auto side_by_side) MODA_INLINE {
+    constexpr int MBQ = decltype(side_by_side)::value, W = 128 * MBQ;
+#pragma unroll 1
+    for (int first = 0; first < blocks; first += 8 * MBQ) {
+      Product<T, MBQ, NB> next;
+      next.voff = lane * 16;
+      i32x2 bias[MBQ];
+#pragma unroll
+      for (int mb = 0; mb < MBQ; mb++) {
+        const int want = first + wave * MBQ + mb, blk = want < blocks ? want : blocks - 1;  // past the last block: that one again, not stored
+        const int pi = blk < end0 ? 0 : blk < end1 ? 1 : 2, f = 16 * (blk - (pi == 0 ? 0 : pi == 1 ? end0 : end1));
+        next.base[mb] = (pi == 0 ? a.part[0].w : pi == 1 ? a.part[1].w : a.part[2].w) + (size_t)f * C;
+        const uint16_t* bp = pi == 0 ? a.part[0].bias : pi == 1 ? a.part[1].bias : a.part[2].bias;
+        bias[mb] = bp ? *reinterpret_cast<const i32x2*>(bp + f + 4 * q4) : none;
+      }
+      next.start();
+      if (first > 0) lds_barrier();  // the results of the turn before are read
+      f32x4 out[MBQ][NB];
+      zero(out);
+      next.template run<C>(X, xbase, C / 32, out);
+#pragma unroll
+      for (int mb = 0; mb < MBQ; mb++) {
+        float b[4];
+        unpack4(bias[mb], b);
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) {
+          float x[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++) x[i] = out[mb][nb][i] + b[i];
+          *reinterpret_cast<MODA_LDS i32x2*>(H + Rows<W>::off(sigma, 2 * (wave * MBQ + mb) + (q4 >> 1)) + 4 * (q4 & 1) + 16 * nb * W) = pack4(x);
+        }
+      }
+      lds_barrier();
+      const int chunks = 2 * (blocks - first < 8 * MBQ ? blocks - first : 8 * MBQ);  // of 8 features a row
+      if (r0 + lrow < a.rows)
+#pragma unroll 2
+        for (int ch = lsub; ch < chunks; ch += TPR) {
+          const int blk = first + (ch >> 1), f = 8 * (2 * first + ch);
+          uint16_t* y = blk < end0 ? a.part[0].y + f : blk < end1 ? a.part[1].y + (f - 16 * end0) : a.part[2].y + (f - 16 * end1);
+          const int64_t ldy = blk < end0 ? a.part[0].ldy : blk < end1 ? a.part[1].ldy : a.part[2].ldy;
+          *reinterpret_cast<i32x4*>(y + (r0 + lrow) * ldy) = *reinterpret_cast<MODA_LDS const i32x4*>(H + Rows<W>::off(lrow, ch));
+        }
+    }
+  };
+  if (blocks <= 16)
+    projections(std::integral_constant<int, 2>{});
+  else if (blocks <= 24)
+    projections(std::integral_constant<int, 3>{});
+  else
+    projections(std::integral_constant<int, 4>{});
+}
+
+// Weights [n][k] into the order in which the products above read them: blocks of 16 features, per block the steps of 32 of
+// the sum, per step the 1 KB of a wave's A operand, lane by lane.  In their own order a wave's load touches sixteen rows in each
+// quarter of its lanes, sixteen cache lines where packed it touches two, and a compute unit takes in 13 bytes a cycle instead
+// of 64 (12 608 rows, width 256: 61 us, packed 42 at the time).  Twelve blocks are packed in one launch of 7 us.
+// The last row of workgroups fills the GELU table: Phi of the bf16 values from 2^-17 to 16, then of their negatives.
+constexpr int kPackMatrices = 96;
+struct PackArgs {
+  int n;
+  float* gelu_table;
+  struct Matrix {
+    const uint16_t* w;
+    uint16_t* to;
+    int blocks, steps;
+  } m[kPackMatrices];
+};
+__global__ __launch_bounds__(256) void pack_weights_kernel(const PackArgs a) {
+  if ((int)blockIdx.y == a.n) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < kGeluTable; i += gridDim.x * 256) {
+      const unsigned bits = (unsigned)(kGeluFirst + i % kGeluHalf) << 16;
+      const double x = __builtin_bit_cast(float, bits) * (i < kGeluHalf ? 1.0 : -1.0);
+      a.gelu_table[i] = (float)(0.5 * erfc(-x * 0.70710678118654752440));
+    }
+    return;
+  }
+  const PackArgs::Matrix m = a.m[blockIdx.y];
+  const int lane = threadIdx.x & 63, item = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (item >= m.blocks * m.steps) return;
+  const int blk = item / m.steps, ks = item - blk * m.steps;
+  const i32x4 v = *reinterpret_cast<const i32x4*>(m.w + ((int64_t)(blk * 16 + (lane & 15)) * m.steps + ks) * 32 + (lane >> 4) * 8);
+  *reinterpret_cast<i32x4*>(m.to + ((int64_t)item * 64 + lane) * 8) = v;
+}
+
+namespace {
+
+template <typename T, int C, int NB, bool POST>
+hipError_t launch_tail_t(const TailArgs& a, hipStream_t stream) {
+  constexpr int BM = 16 * NB, HC = 256;
+  constexpr size_t smem = table_bytes<T>() + (size_t)BM * (C + (C > 2 * HC ? C : 2 * HC)) * sizeof(uint16_t);
+  static LdsAttrState attr;
+  const hipError_t e = allow_dynamic_lds(attr, reinterpret_cast<const void*>(&block_tail_kernel<T, C, NB, POST>), smem);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((block_tail_kernel<T, C, NB, POST>), dim3((unsigned)((a.rows + BM - 1) / BM)), dim3(512), smem, stream, a);
+  return hipGetLastError();
+}
+
+template <typename T, int C>
+hipError_t launch_tail_c(const TailArgs& a, bool post, int cus, hipStream_t stream) {
+  if (a.rows <= 32 * cus) return post ? launch_tail_t<T, C, 2, true>(a, stream) : launch_tail_t<T, C, 2, false>(a, stream);
+  return post ? launch_tail_t<T, C, 4, true>(a, stream) : launch_tail_t<T, C, 4, false>(a, stream);
+}
+
+template <typename T>
+hipError_t launch_tail(const TailArgs& a, int width, bool post, int cus, hipStream_t stream) {
+  switch (width) {
+    case 128: return launch_tail_c<T, 128>(a, post, cus, stream);
+    case 256: return launch_tail_c<T, 256>(a, post, cus, stream);
+    case 384: return launch_tail_c<T, 384>(a, post, cus, stream);
+    case 512: return launch_tail_c<T, 512>(a, post, cus, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace
+
+hipError_t launch_pack_weights(const moda_hip_weight* w, int n, float* gelu_table, hipStream_t stream) {
+  for (int first = 0; first < n; first += kPackMatrices) {
+    PackArgs a = {};
+    int64_t most = 0;
+    const int count = n - first < kPackMatrices ? n - first : kPackMatrices;
+    for (int i = 0; i < count; i++) {
+      const moda_hip_weight& x = w[first + i];
+      a.m[i] = PackArgs::Matrix{(const uint16_t*)x.w, (uint16_t*)x.packed, (int)x.n / 16, (int)x.k / 32};
+      const int64_t items = (x.n / 16) * (x.k / 32);
+      most = items > most ? items : most;
+    }
+    a.n = count;
+    a.gelu_table = first == 0 ? gelu_table : nullptr;
+    hipLaunchKernelGGL(pack_weights_kernel, dim3((unsigned)((most + 3) / 4), count + (a.gelu_table ? 1 : 0)), dim3(256), 0, stream, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+hipError_t launch_block_tail(const moda_hip_block_tail_args* t, int compute_units, hipStream_t stream) {
+  TailArgs a = {};
+  auto in = [](const void* p) { return (const uint16_t*)p; };
+  a.h = in(t->attention);
+  a.res = in(t->residual);
+  a.x = (uint16_t*)t->x;
+  a.rows = (int)t->rows;
+  a.hidden = (int)t->hidden;
+  a.n_parts = t->n_parts;
+  a.proj_w = in(t->proj_w);
+  a.proj_b = in(t->proj_b);
+  a.fc1_w = in(t->fc1_w);
+  a.fc1_b = in(t->fc1_b);
+  a.fc2_w = in(t->fc2_w);
+  a.fc2_b = in(t->fc2_b);
+  a.mid_w = in(t->mid_norm_w);
+  a.mid_b = in(t->mid_norm_b);
+  a.end_w = in(t->end_norm_w);
+  a.end_b = in(t->end_norm_b);
+  a.mid_eps = t->mid_norm_eps;
+  a.end_eps = t->end_norm_eps;
+  a.gelu_table = (const float*)t->gelu_table;
+  int end = 0;
+  for (int i = 0; i < t->n_parts; i++) {
+    const moda_hip_linear_part& p = t->parts[i];
+    end += (int)p.n / 16;
+    a.part[i] = TailPart{in(p.w), in(p.bias), (uint16_t*)p.y, p.ldy, (int)p.n, end};
+  }
+  return t->dtype == 0 ? launch_tail<BF16>(a, (int)t->width, t->post_norm != 0, compute_units, stream)
+                       : launch_tail<FP16>(a, (int)t->width, t->post_norm != 0, compute_units, stream);
+}
+
+}  // namespace moda

@@ -25,6 +25,8 @@ hipError_t launch_linear(int dtype, int64_t rows, int64_t K, const void* x, int6
                          const void* residual, int64_t ld_res, bool gelu, int compute_units, hipStream_t stream);
 hipError_t launch_layer_norm(int dtype, int64_t rows, int64_t dim, const void* x, const void* weight, const void* bias, float eps, void* y,
                              hipStream_t stream);
+hipError_t launch_pack_weights(const moda_hip_weight* w, int n, float* gelu_table, hipStream_t stream);
+hipError_t launch_block_tail(const moda_hip_block_tail_args* args, int compute_units, hipStream_t stream);
 }  // namespace moda
 
 using moda::KArgs;
@@ -568,6 +570,50 @@ int moda_hip_layer_norm(int32_t dtype, int64_t rows, int64_t dim, const void* x,
     if ((uintptr_t)p % 16 != 0) return MODA_HIP_EALIGN;
   const hipError_t e = moda::launch_layer_norm(dtype, rows, dim, x, weight, bias, eps, y, (hipStream_t)stream);
   return e == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
+}
+
+int moda_hip_pack_weights(const moda_hip_weight* w, int32_t n, void* gelu_table, void* stream) {
+  if (!w || n < 1) return MODA_HIP_EINVAL;
+  if ((uintptr_t)gelu_table % 16 != 0) return MODA_HIP_EALIGN;
+  for (int i = 0; i < n; i++) {
+    if (!w[i].w || !w[i].packed || w[i].n <= 0 || w[i].k <= 0) return MODA_HIP_EINVAL;
+    if (w[i].n % 16 != 0 || w[i].k % 32 != 0 || w[i].n >= (1 << 20) || w[i].k >= (1 << 20) || w[i].n * w[i].k >= (1ll << 31))
+      return MODA_HIP_EUNSUPPORTED;
+    if ((uintptr_t)w[i].w % 16 != 0 || (uintptr_t)w[i].packed % 16 != 0) return MODA_HIP_EALIGN;
+  }
+  const int rc = check_device();
+  if (rc) return rc;
+  return moda::launch_pack_weights(w, n, (float*)gelu_table, (hipStream_t)stream) == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
+}
+
+int moda_hip_block_tail(const moda_hip_block_tail_args* t, void* stream) {
+  if (!t || t->struct_size != (int32_t)sizeof(*t) || (t->dtype != MODA_HIP_BF16 && t->dtype != MODA_HIP_FP16)) return MODA_HIP_EINVAL;
+  if (t->rows < 0 || t->width <= 0 || t->hidden <= 0 || t->n_parts < 0 || t->n_parts > 3) return MODA_HIP_EINVAL;
+  if (t->rows == 0) return MODA_HIP_OK;
+  if (t->dtype == MODA_HIP_BF16 && !t->gelu_table) return MODA_HIP_EINVAL;
+  if ((uintptr_t)t->gelu_table % 16 != 0) return MODA_HIP_EALIGN;
+  const bool end_norm = t->post_norm || t->n_parts > 0;
+  for (const void* p : {t->attention, t->residual, (const void*)t->x, t->proj_w, t->fc1_w, t->fc2_w, t->mid_norm_w, t->mid_norm_b,
+                        end_norm ? t->end_norm_w : t->x, end_norm ? t->end_norm_b : t->x})
+    if (!p) return MODA_HIP_EINVAL;
+  if ((t->width != 128 && t->width != 256 && t->width != 384 && t->width != 512) || t->hidden % 128 != 0 || t->hidden >= (1 << 20) ||
+      t->rows >= (1ll << 30))
+    return MODA_HIP_EUNSUPPORTED;
+  for (const void* p : {t->attention, t->residual, (const void*)t->x, t->proj_w, t->fc1_w, t->fc2_w, t->mid_norm_w, t->mid_norm_b,
+                        end_norm ? t->end_norm_w : t->x, end_norm ? t->end_norm_b : t->x})
+    if ((uintptr_t)p % 16 != 0) return MODA_HIP_EALIGN;
+  for (const void* p : {t->proj_b, t->fc1_b, t->fc2_b})
+    if ((uintptr_t)p % 8 != 0) return MODA_HIP_EALIGN;
+  for (int i = 0; i < t->n_parts; i++) {
+    const moda_hip_linear_part& p = t->parts[i];
+    if (!p.w || !p.y || p.n <= 0) return MODA_HIP_EINVAL;
+    if (p.n % 16 != 0 || p.n >= (1 << 20)) return MODA_HIP_EUNSUPPORTED;
+    if ((uintptr_t)p.w % 16 != 0 || (uintptr_t)p.y % 16 != 0 || p.ldy % 8 != 0 || (uintptr_t)p.bias % 8 != 0) return MODA_HIP_EALIGN;
+  }
+  int cus = 0;
+  const int rc = check_device(&cus);
+  if (rc) return rc;
+  return moda::launch_block_tail(t, cus, (hipStream_t)stream) == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
 }
 
 int moda_hip_uses_matrix_cores(const moda_hip_desc* d) {

@@ -700,6 +700,19 @@ bool stack_runs_native(int64_t rows, int64_t width, void* stream) {
   return hipStreamIsCapturing((hipStream_t)stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
 }
 
+// Whether a block's dense part runs as one launch (moda_hip_block_tail) or as its pieces.  Eight blocks, 64 x 197 tokens,
+// one launch / pieces: width 128 268 / 455 us, 256 407 / 660, 384 735 / 1005, 512 1110 / 1284.  A workgroup takes 64 rows through
+// all of a block's weights (32 where that still fits one round), so few rows cost what a full round of 256 workgroups
+// does, and a round that is mostly empty as much as a full one: up to width 256 that is still the faster way (4 x 50 tokens
+// 187 / 272 and 272 / 335; 64 x 257, one workgroup too many for a round, 388 / 519 and 683 / 838), above only when the last
+// round is well filled (384: 64 x 145 tokens 670 / 845, 4 x 50 452 / 411; 512: 64 x 145 979 / 1036, in fp16 1134 / 1038, 4 x 50
+// 618 / 446, 64 x 257 2084 / 1839).
+bool tail_is_one_launch(int64_t rows, int64_t width, int64_t hidden, int64_t kv) {
+  if ((width != 128 && width != 256 && width != 384 && width != 512) || hidden % 128 != 0 || kv % 16 != 0) return false;
+  const int64_t last = ((rows + 63) / 64 - 1) % 256 + 1;
+  return width <= 256 || last >= (width <= 384 ? 128 : 192);
+}
+
 // Forward pass of all blocks of one stack, launches only: the residual stream, one depth cache and four work tensors
 // are all there is.  A layer's K and V are projected straight into their slot of the cache, where its own attention reads
 // them as the sequence and later layers as a depth slot.  Returns nothing where a kernel's contract is not met (the
@@ -735,8 +748,9 @@ std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>
   const auto opt = x_in.options().requires_grad(false);
   const Tensor x0 = x_in.contiguous();
   if ((uintptr_t)x0.const_data_ptr() % 16 != 0) return {};
-  Tensor x = at::empty({B, N, C}, opt), x1 = at::empty({M, C}, opt), h = at::empty({M, C}, opt), q = at::empty({M, C}, opt),
-         hid = at::empty({M, hidden}, opt), ck = at::empty({B, N * L, kv}, opt), cv = at::empty({B, N * L, kv}, opt),
+  const bool tails = tail_is_one_launch(M, C, hidden, kv);
+  Tensor x = at::empty({B, N, C}, opt), h = at::empty({M, C}, opt), q = at::empty({M, C}, opt), x1 = tails ? Tensor() : at::empty({M, C}, opt),
+         hid = tails ? Tensor() : at::empty({M, hidden}, opt), ck = at::empty({B, N * L, kv}, opt), cv = at::empty({B, N * L, kv}, opt),
          lse = at::empty({M * heads}, opt.dtype(at::kFloat));
   auto part = [&](const Tensor& w, const Tensor& b, int64_t first, int64_t n, void* y, int64_t ldy) {
     return moda_hip_linear_part{(const char*)in_ptr(w) + first * w.size(1) * es, b.defined() ? (const char*)in_ptr(b) + first * es : nullptr, y,
@@ -765,32 +779,100 @@ std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>
   d.k = d.v = {N * L * kv, L * kv, hd};
   d.kd = d.vd = {N * L * kv, kv, hd};
 
+  auto projections = [&](const Block& b, int64_t slot) {
+    char *ks = slot_of(ck, slot), *vs = slot_of(cv, slot);
+    return std::array<moda_hip_linear_part, 3>{part(b.q_w, b.q_b, 0, C, out_ptr(q), C), part(b.kv_w, b.kv_b, 0, kv, ks, L * kv),
+                                               part(b.kv_w, b.kv_b, kv, kv, vs, L * kv)};
+  };
+  // packed copies of the weights, in the order proj, fc1, fc2, q, kv of each block (the first block's q, kv are not packed),
+  // and the table behind them
+  Tensor packed;
+  const int64_t block_elems = C * C + 2 * hidden * C + C * C + 2 * kv * C;
+  auto packed_at = [&](size_t i) { return (char*)out_ptr(packed) + (int64_t)i * block_elems * es; };
+  if (tails) {
+    packed = at::empty({(int64_t)blocks.size() * block_elems + MODA_HIP_GELU_TABLE_BYTES / es}, opt);
+    std::vector<moda_hip_weight> weights;
+    for (size_t i = 0; i < blocks.size(); i++) {
+      const Block& b = blocks[i];
+      char* to = packed_at(i);
+      for (const Tensor* w : {&b.proj_w, &b.fc1_w, &b.fc2_w, &b.q_w, &b.kv_w}) {
+        if (i > 0 || (w != &b.q_w && w != &b.kv_w)) weights.push_back({in_ptr(*w), to, w->size(0), w->size(1)});
+        to += w->numel() * es;
+      }
+    }
+    check_rc(moda_hip_pack_weights(weights.data(), (int32_t)weights.size(), packed_at(blocks.size()), stream), "moda_hip_pack_weights");
+  }
+
   const void* cur = in_ptr(x0);  // the residual stream
   int64_t n = 0;                 // filled slots
-  for (const Block& b : blocks) {
-    const void* in = cur;
-    if (!post_norm) {
-      norm(cur, b.norm1_w, b.norm1_b, b.eps1, h);
-      in = in_ptr(h);
+  bool projected = false;        // the block's q, k, v came with the previous block's last launch
+  for (size_t i = 0; i < blocks.size(); i++) {
+    const Block& b = blocks[i];
+    if (!projected) {
+      const void* in = cur;
+      if (!post_norm) {
+        norm(cur, b.norm1_w, b.norm1_b, b.eps1, h);
+        in = in_ptr(h);
+      }
+      const auto p = projections(b, n);
+      linear(in, C, {p[0], p[1], p[2]}, nullptr, false);
     }
-    char *ks = slot_of(ck, n), *vs = slot_of(cv, n);
-    linear(in, C, {part(b.q_w, b.q_b, 0, C, out_ptr(q), C), part(b.kv_w, b.kv_b, 0, kv, ks, L * kv), part(b.kv_w, b.kv_b, kv, kv, vs, L * kv)},
-           nullptr, false);
     d.L = n > 0 ? L : 0;
     d.L_valid = (int32_t)n;
-    check_rc(moda_hip_fwd(&d, in_ptr(q), ks, vs, n > 0 ? in_ptr(ck) : nullptr, n > 0 ? in_ptr(cv) : nullptr, out_ptr(h),
-                          (float*)out_ptr(lse), stream),
+    check_rc(moda_hip_fwd(&d, in_ptr(q), slot_of(ck, n), slot_of(cv, n), n > 0 ? in_ptr(ck) : nullptr, n > 0 ? in_ptr(cv) : nullptr,
+                          out_ptr(h), (float*)out_ptr(lse), stream),
              "moda_hip_fwd");
-    linear(in_ptr(h), C, {part(b.proj_w, b.proj_b, 0, C, out_ptr(x1), C)}, cur, false);
-    if (post_norm) {
-      norm(in_ptr(x1), b.norm1_w, b.norm1_b, b.eps1, x1);
-      linear(in_ptr(x1), C, {part(b.fc1_w, b.fc1_b, 0, hidden, out_ptr(hid), hidden)}, nullptr, true);
-      linear(in_ptr(hid), hidden, {part(b.fc2_w, b.fc2_b, 0, C, out_ptr(h), C)}, in_ptr(x1), false);
-      norm(in_ptr(h), b.norm2_w, b.norm2_b, b.eps2, x);
+    const int64_t slots = b.kv_ffn_w.defined() ? 2 : 1;
+    if (tails) {
+      moda_hip_block_tail_args t = {};
+      t.struct_size = sizeof(t);
+      t.dtype = dt;
+      t.rows = M;
+      t.width = C;
+      t.hidden = hidden;
+      t.gelu_table = packed_at(blocks.size());
+      t.attention = in_ptr(h);
+      t.residual = cur;
+      t.x = out_ptr(x);
+      t.proj_w = packed_at(i);
+      t.proj_b = in_ptr(b.proj_b);
+      t.fc1_w = packed_at(i) + C * C * es;
+      t.fc1_b = in_ptr(b.fc1_b);
+      t.fc2_w = packed_at(i) + (C + hidden) * C * es;
+      t.fc2_b = in_ptr(b.fc2_b);
+      const Block* next = i + 1 < blocks.size() ? &blocks[i + 1] : nullptr;
+      t.post_norm = post_norm;
+      t.mid_norm_w = in_ptr(post_norm ? b.norm1_w : b.norm2_w);
+      t.mid_norm_b = in_ptr(post_norm ? b.norm1_b : b.norm2_b);
+      t.mid_norm_eps = (float)(post_norm ? b.eps1 : b.eps2);
+      if (post_norm || next) {
+        t.end_norm_w = in_ptr(post_norm ? b.norm2_w : next->norm1_w);
+        t.end_norm_b = in_ptr(post_norm ? b.norm2_b : next->norm1_b);
+        t.end_norm_eps = (float)(post_norm ? b.eps2 : next->eps1);
+      }
+      if (next) {
+        const auto p = projections(*next, n + slots);
+        std::copy(p.begin(), p.end(), t.parts);
+        const char* qkv = packed_at(i + 1) + (C + 2 * hidden) * C * es;
+        t.parts[0].w = qkv;
+        t.parts[1].w = qkv + C * C * es;
+        t.parts[2].w = qkv + (C + kv) * C * es;
+        t.n_parts = 3;
+      }
+      check_rc(moda_hip_block_tail(&t, stream), "moda_hip_block_tail");
+      projected = true;
     } else {
-      norm(in_ptr(x1), b.norm2_w, b.norm2_b, b.eps2, h);
-      linear(in_ptr(h), C, {part(b.fc1_w, b.fc1_b, 0, hidden, out_ptr(hid), hidden)}, nullptr, true);
-      linear(in_ptr(hid), hidden, {part(b.fc2_w, b.fc2_b, 0, C, out_ptr(x), C)}, in_ptr(x1), false);
+      linear(in_ptr(h), C, {part(b.proj_w, b.proj_b, 0, C, out_ptr(x1), C)}, cur, false);
+      if (post_norm) {
+        norm(in_ptr(x1), b.norm1_w, b.norm1_b, b.eps1, x1);
+        linear(in_ptr(x1), C, {part(b.fc1_w, b.fc1_b, 0, hidden, out_ptr(hid), hidden)}, nullptr, true);
+        linear(in_ptr(hid), hidden, {part(b.fc2_w, b.fc2_b, 0, C, out_ptr(h), C)}, in_ptr(x1), false);
+        norm(in_ptr(h), b.norm2_w, b.norm2_b, b.eps2, x);
+      } else {
+        norm(in_ptr(x1), b.norm2_w, b.norm2_b, b.eps2, h);
+        linear(in_ptr(h), C, {part(b.fc1_w, b.fc1_b, 0, hidden, out_ptr(hid), hidden)}, nullptr, true);
+        linear(in_ptr(hid), hidden, {part(b.fc2_w, b.fc2_b, 0, C, out_ptr(x), C)}, in_ptr(x1), false);
+      }
     }
     cur = in_ptr(x);
     n++;

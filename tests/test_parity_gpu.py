@@ -1952,6 +1952,121 @@ def test_linear_against_fp64(gpu_device, case, dtype):
             assert (y[:, n:] == 7.0).all(), epilogue
 
 
+class _BlockTail:
+    """moda_hip_pack_weights + moda_hip_block_tail through the C entry points, on random weights (or those given)."""
+
+    NAMES = ("proj_w", "proj_b", "fc1_w", "fc1_b", "fc2_w", "fc2_b", "mid_w", "mid_b", "end_w", "end_b")
+
+    def __init__(self, width, hidden, parts, dtype, device, seed=0, **given):
+        import ctypes
+
+        from moda_amd import _lib
+
+        self.lib, self.ct, self.width, self.hidden, self.dtype = _lib.load(), ctypes, width, hidden, dtype
+        gen = torch.Generator(device=device).manual_seed(seed)
+        rn = lambda *s: torch.randn(*s, generator=gen, device=device)
+        made = dict(proj_w=rn(width, width) * width ** -0.5, proj_b=rn(width), fc1_w=rn(hidden, width) * width ** -0.5, fc1_b=rn(hidden),
+                    fc2_w=rn(width, hidden) * hidden ** -0.5, fc2_b=rn(width), mid_w=1 + 0.1 * rn(width), mid_b=rn(width),
+                    end_w=1 + 0.1 * rn(width), end_b=rn(width))
+        self.w = {n: given.get(n, made[n]).to(dtype) for n in self.NAMES}
+        self.parts = [((rn(n, width) * width ** -0.5).to(dtype), rn(n).to(dtype)) for n in parts]
+        ptr, i64 = ctypes.c_void_p, ctypes.c_int64
+
+        class Weight(ctypes.Structure):
+            _fields_ = [("w", ptr), ("packed", ptr), ("n", i64), ("k", i64)]
+
+        ws = [self.w["proj_w"], self.w["fc1_w"], self.w["fc2_w"]] + [w for w, _ in self.parts]
+        self.packed, self.table = [torch.empty_like(w) for w in ws], torch.empty(21504 // 4, device=device)
+        arr = (Weight * len(ws))(*(Weight(w.data_ptr(), p.data_ptr(), *w.shape) for w, p in zip(ws, self.packed)))
+        assert self.lib.moda_hip_pack_weights(arr, len(ws), ptr(self.table.data_ptr()), ptr(torch.cuda.current_stream().cuda_stream)) == 0
+
+    def run(self, attention, residual, post_norm):
+        ptr, i32, i64, f32 = (getattr(self.ct, "c_" + n) for n in ("void_p", "int32", "int64", "float"))
+
+        class Part(self.ct.Structure):
+            _fields_ = [("w", ptr), ("bias", ptr), ("y", ptr), ("ldy", i64), ("n", i64)]
+
+        class Args(self.ct.Structure):
+            _fields_ = [("struct_size", i32), ("dtype", i32), ("rows", i64), ("width", i64), ("hidden", i64), ("attention", ptr),
+                        ("residual", ptr), ("x", ptr), *((n, ptr) for n in self.NAMES), ("gelu_table", ptr), ("mid_eps", f32),
+                        ("end_eps", f32), ("post_norm", i32), ("n_parts", i32), ("parts", Part * 3)]
+
+        rows = attention.shape[0]
+        x = residual.clone()  # in place
+        ys = [torch.full((rows + 1, w.shape[0] + 8), 7.0, device=x.device, dtype=x.dtype) for w, _ in self.parts]
+        a = Args(struct_size=self.ct.sizeof(Args), dtype={torch.bfloat16: 0, torch.float16: 1}[self.dtype], rows=rows, width=self.width,
+                 hidden=self.hidden, attention=attention.data_ptr(), residual=x.data_ptr(), x=x.data_ptr(), gelu_table=self.table.data_ptr(),
+                 mid_eps=1e-6, end_eps=1e-6, post_norm=int(post_norm), n_parts=len(ys))
+        for n in self.NAMES:
+            setattr(a, n, self.w[n].data_ptr())
+        a.proj_w, a.fc1_w, a.fc2_w = (p.data_ptr() for p in self.packed[:3])
+        for i, y in enumerate(ys):
+            a.parts[i] = Part(self.packed[3 + i].data_ptr(), self.parts[i][1].data_ptr(), y.data_ptr(), y.stride(0), self.parts[i][0].shape[0])
+        assert self.lib.moda_hip_block_tail(self.ct.byref(a), ptr(torch.cuda.current_stream().cuda_stream)) == 0
+        return x, ys
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("post_norm", [False, True])
+@pytest.mark.parametrize("case", [
+    # rows, width, hidden, features of each part: one row; ragged rows of both tiles (32 rows, and 64 above 8192), a hidden
+    # width whose last chunk leaves waves without features, 2, 3 and 4 feature blocks a wave, two turns, no part
+    (1, 128, 128, (128, 16, 16)),
+    (45, 256, 640, (256, 64, 64)),
+    (8195, 128, 384, (128,)),
+    (8251, 256, 1024, (256, 128, 128)),
+    (8200, 384, 128, (384, 16)),
+    (8193, 512, 256, (512, 128, 128)),
+    (70, 512, 2048, ()),
+], ids=str)
+def test_block_tail_against_fp64(gpu_device, case, post_norm, dtype):
+    """A block's dense part in one launch against fp64 with a rounding to 16 bits wherever the pieces round.  Those roundings
+    fall alike except where the fp32 sums (K 2^-24 relative at most) move a value across a boundary, one in 2^24 / (K 2^8 or
+    2^11) of them by u = 2^-8 or 2^-11: norm-wise far below one u; a quarter of u is asked for."""
+    rows, width, hidden, parts = case
+    say(f"CASE block tail {case} post_norm={post_norm} {dtype}")
+    t = _BlockTail(width, hidden, parts, dtype, gpu_device, seed=rows)
+    gen = torch.Generator(device=gpu_device).manual_seed(rows + 1)
+    h, res = (torch.randn(rows, width, generator=gen, device=gpu_device).to(dtype) for _ in range(2))
+    x, ys = t.run(h, res, post_norm)
+    r = lambda v: v.to(dtype).double()
+    w = {n: v.double() for n, v in t.w.items()}
+    norm = lambda v, n: r(torch.nn.functional.layer_norm(v, (width,), w[n + "_w"], w[n + "_b"], 1e-6))
+    lin = lambda v, n: r(v @ w[n + "_w"].t() + w[n + "_b"])
+    gelu = lambda v: r(0.5 * v * torch.special.erfc(v * -0.5 ** 0.5))
+    y = r(lin(h.double(), "proj") + res.double())
+    z = norm(y, "mid")
+    y = z if post_norm else y
+    y = r(lin(gelu(lin(z, "fc1")), "fc2") + y)
+    z = norm(y, "end")
+    y = z if post_norm else y
+    u = 2.0 ** -8 if dtype is torch.bfloat16 else 2.0 ** -11
+    off = lambda got, want: ((got.double() - want).norm() / want.norm()).item()
+    assert off(x, y) <= u / 4, off(x, y)
+    for (pw, pb), got in zip(t.parts, ys):
+        n = pw.shape[0]
+        assert off(got[:rows, :n], r(z @ pw.double().t() + pb.double())) <= u / 4
+        assert (got[rows:] == 7.0).all() and (got[:, n:] == 7.0).all()
+
+
+def test_block_tail_gelu_of_every_bf16_value(gpu_device):
+    """The table route of the GELU, value by value: zero rows, the values as the first layer's bias, an identity behind it.
+    One rounding beside the table's own ends: u |y| and 2^-17 relative, and fp32's subnormals."""
+    eye, zero = torch.eye(128, device=gpu_device), torch.zeros(128, device=gpu_device)
+    t = _BlockTail(128, 128, (), torch.bfloat16, gpu_device, mid_w=zero, mid_b=zero, fc2_w=eye, fc2_b=zero, proj_b=zero)
+    row = torch.zeros(1, 128, device=gpu_device, dtype=torch.bfloat16)
+    values = torch.arange(-32768, 32768, device=gpu_device).to(torch.int16).view(torch.bfloat16)
+    values = values[values.isfinite()]
+    got = []
+    for v in values.split(128):
+        t.w["fc1_b"] = torch.nn.functional.pad(v, (0, 128 - v.numel()))
+        got.append(t.run(row, row, False)[0][0, :v.numel()])
+    v = values.double()
+    want = 0.5 * v * torch.special.erfc(v * -0.5 ** 0.5)
+    err = (torch.cat(got).double() - want).abs()
+    assert (err <= (2.0 ** -8 + 8e-6) * want.abs() + 2.0 ** -126).all(), (err / want.abs()).max()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("dim", [8, 128, 136, 256, 264, 512, 520, 1024, 1032, 2048, 2056, 4096])
 def test_layer_norm_against_fp64(gpu_device, dim, dtype):
