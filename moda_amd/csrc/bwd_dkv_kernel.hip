@@ -966,7 +966,8 @@ hipError_t launch_dkv_t(const KArgs& a, hipStream_t stream) {
   const bool flat = takes_dkv_flat(a, HD);
   const int64_t nblk = col_kernel_blocks(a, HD, BN, nseg);
   if (nblk >= (1ll << 31)) return hipErrorInvalidValue;
-  if (nblk > 0 && flat) {
+  if (a.seq_done) {  // formed beside dQ
+  } else if (nblk > 0 && flat) {
     const hipError_t e = launch_dkv_flat(a, std::is_same<T, FP16>::value ? 1 : 0, stream);
     if (e != hipSuccess) return e;
   } else if (nblk > 0) {

@@ -1,0 +1,48 @@
+// dQ and sequence dK/dV of small problems on the 64-wide tiles in one launch: the workgroups of dq_kernel and of
+// dkv_flat_kernel side by side.  Where both together do not fill the machine, each launch is a chain of a few dependent
+// tiles behind its own start and end; together they take as long as the longer one.  The dK/dV workgroups form the row sums
+// of o * do themselves (OWN_DELTA).  2 x 95 tokens, four heads of two query rows, eight slots, fp16: 25.6 -> 19.8
+// us of kernels and a launch less, the replayed training step 35.0 -> 29.3 us; 8 x 197 tokens, six heads, twelve slots 71.1 -> 64.2.
+#include "bwd_dkv_flat.h"
+#include "bwd_dq.h"
+
+namespace moda {
+
+template <typename T, int ADDR, int RW>
+__global__ __launch_bounds__(256, 2) void bwd_short_kernel(const KArgs a, int row_blocks) {
+  if ((int)blockIdx.x < row_blocks)
+    dq_body<T, 64, RowSmall<64>, ADDR>(a, blockIdx.x);
+  else
+    dkv_flat_body<T, 64, false, false, RW, true>(a, (int)blockIdx.x - row_blocks);
+}
+
+template <typename T, int ADDR, int RW>
+hipError_t launch_short_t(const KArgs& a, hipStream_t stream) {
+  constexpr size_t lds_dq = dq_lds<64, RowSmall<64>, ADDR>(), lds_dkv = dkv_flat_lds<64, RW, true>();
+  constexpr size_t smem = lds_dq > lds_dkv ? lds_dq : lds_dkv;
+  static_assert(2 * smem <= 160 * 1024, "two workgroups a compute unit");
+  static LdsAttrState attr;
+  const hipError_t ea = allow_dynamic_lds(attr, reinterpret_cast<const void*>(&bwd_short_kernel<T, ADDR, RW>), smem);
+  if (ea != hipSuccess) return ea;
+  const int64_t columns = dkv_flat_blocks(a, 128 / RW), rows = row_kernel_blocks(a, 128);
+  hipLaunchKernelGGL((bwd_short_kernel<T, ADDR, RW>), dim3((unsigned)(columns + rows)), dim3(256), smem, stream, a, (int)rows);
+  return hipGetLastError();
+}
+
+template <typename T, int RW>
+hipError_t launch_short_a(const KArgs& a, hipStream_t stream) {
+  if (a.L == 0) return launch_short_t<T, 4, RW>(a, stream);
+  return a.Lv != a.L ? launch_short_t<T, 8, RW>(a, stream) : launch_short_t<T, 0, RW>(a, stream);
+}
+
+template <typename T>
+hipError_t launch_short_as(const KArgs& a, hipStream_t stream) {
+  return dkv_flat_row_waves(a) ? launch_short_a<T, 4>(a, stream) : launch_short_a<T, 1>(a, stream);
+}
+
+// dtype: 0 bf16, 1 fp16; the caller asks bwd_one_launch first
+hipError_t launch_bwd_short(const KArgs& a, int dtype, hipStream_t stream) {
+  return dtype == 0 ? launch_short_as<BF16>(a, stream) : launch_short_as<FP16>(a, stream);
+}
+
+}  // namespace moda

@@ -15,6 +15,7 @@ hipError_t launch_fwd(const KArgs& a, int dtype, int hd, hipStream_t stream);
 hipError_t launch_delta(const KArgs& a, int dtype, int hd, hipStream_t stream);
 hipError_t launch_dq(const KArgs& a, int dtype, int hd, hipStream_t stream);
 hipError_t launch_dkv(const KArgs& a, int dtype, int hd, hipStream_t stream);
+hipError_t launch_bwd_short(const KArgs& a, int dtype, hipStream_t stream);
 hipError_t launch_generic(const KArgs& a, int dtype, int D, int Dv, int which, hipStream_t stream);
 hipError_t launch_fp32(const KArgs& a, int which, hipStream_t stream);
 hipError_t launch_reorg(void* const* layers, int64_t n_layers, int64_t slot0, int64_t L_total, int64_t n_tokens,
@@ -468,7 +469,12 @@ int moda_hip_bwd_stages(const moda_hip_desc* d, const void* q, const void* k, co
     // with both stages asked for, the dQ kernel forms the row sums itself (one launch and one pass over o, do less)
     a.own_delta = (stages & MODA_HIP_STAGE_DELTA) && (stages & MODA_HIP_STAGE_DQ) ? 1 : 0;
     if ((stages & MODA_HIP_STAGE_DELTA) && !a.own_delta) e = moda::launch_delta(a, d->dtype, tile_width(d), s);
-    if (e == hipSuccess && (stages & MODA_HIP_STAGE_DQ)) e = moda::launch_dq(a, d->dtype, tile_width(d), s);
+    if ((stages & MODA_HIP_STAGE_DKV) && moda::bwd_one_launch(a, tile_width(d))) {
+      e = moda::launch_bwd_short(a, d->dtype, s);
+      a.seq_done = 1;
+    } else if (e == hipSuccess && (stages & MODA_HIP_STAGE_DQ)) {
+      e = moda::launch_dq(a, d->dtype, tile_width(d), s);
+    }
     if (e == hipSuccess && (stages & MODA_HIP_STAGE_DKV)) e = moda::launch_dkv(a, d->dtype, tile_width(d), s);
   } else if (fp32_matrix(d, a, {{q, d->q}, {k, d->k}, {v, d->v}, {kd, d->kd}, {vd, d->vd}, {o, d->o}, {d_o, d->d_o}, {dq, d->dq},
                                 {dk, d->dk}, {dv, d->dv}, {dkd, d->dkd}, {dvd, d->dvd}})) {

@@ -222,6 +222,20 @@ inline bool dkv_flat_row_waves(const KArgs& a) {
   return !a.cu && a.Tq <= kDkvRowWavesMaxRows && dkv_flat_blocks(a) <= 256;
 }
 
+// whether every streamed (batch, head) slice spans less than 2 GiB
+inline bool narrow_slices(const KArgs& a) {
+  const int64_t seq = (int64_t)a.T * (a.sk.t > a.sv.t ? a.sk.t : a.sv.t), dep = (int64_t)a.T * a.L * (a.skd.t > a.svd.t ? a.skd.t : a.svd.t);
+  return 2 * (seq > dep ? seq : dep) <= 0x7fffffffll;
+}
+// dQ and sequence dK/dV of the 64-wide tiles in one launch (bwd_short_kernel): where the workgroups of both run at once, two a
+// compute unit.  More than that and the launch is longer than the two (64 x 197 tokens, six heads, twelve slots: step 191 ->
+// 206 us; the twelve layers of a depth stream over 64 x 197 tokens of four query rows: 734 -> 794), each of which then has
+// the occupancy that its own registers and LDS allow.
+inline bool bwd_one_launch(const KArgs& a, int HD) {
+  return takes_dkv_flat(a, HD) && !a.cu && a.dkv_split <= 1 && a.own_delta && narrow_slices(a) &&
+         row_kernel_blocks(a, 128) + dkv_flat_blocks(a, dkv_flat_row_waves(a) ? 32 : 128) <= 2 * a.compute_units;
+}
+
 // Row segments of the sequence dK/dV launch (KArgs::dkv_split, dkv_seg_tiles): a launch ends with its longest workgroup,
 // and one with few column tiles leaves compute units idle.  Sized for 256 compute units whatever the partition mode, so
 // that the workspace size depends on the problem alone.

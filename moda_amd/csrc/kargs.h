@@ -29,6 +29,7 @@ struct KArgs {
   int accum_depth;  // dkd, dvd += instead of =
   int own_slot;     // dk, dv += slot Lv of dkd, dvd (the layer's own slot of the stream, complete by now)
   int keep_slots;   // slots l >= Lv of dkd, dvd untouched (always when accumulating) instead of zeroed
+  int seq_done;     // the sequence dK/dV came with the dQ launch (host side)
   int own_delta;    // the dQ kernel forms the row sums of o * do itself and leaves them in `delta` for the later kernels
   // Outside chunk-visible mode a query row sees the Lv depth slots of its own token only.  When the dQ kernel walks
   // them (its waves' own depth columns) it leaves the rounded P and dS of those (row, slot) pairs here,

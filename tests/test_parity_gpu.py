@@ -1874,6 +1874,44 @@ def test_stack_widths_and_which_of_them_run_as_native_launches(gpu_device, case)
     assert off(m.bfloat16()(x) if y is None else y) <= max(1.1 * off(z), 2.0 ** -8), (off(z), y is None or off(y))
 
 
+@pytest.mark.parametrize("case", [
+    # B, T, H, G, D, L, L_valid, mode, dtype: one workgroup; ragged tiles with four row waves; column tiles without them; head
+    # dims below the tile width; a partial stream; no stream; depth gradients of their own launch (G 3); chunk-visible; the
+    # last size in one launch and the first one in two
+    (1, 1, 1, 1, 64, 1, 1, "CAUSAL", "fp16"),
+    (2, 95, 4, 2, 64, 8, 8, "CAUSAL", "fp16"),
+    (3, 257, 1, 4, 64, 3, 3, "NONCAUSAL", "bf16"),
+    (2, 130, 2, 1, 40, 5, 2, "NONCAUSAL", "bf16"),
+    (2, 77, 3, 2, 64, 0, 0, "CAUSAL", "bf16"),
+    (1, 70, 2, 3, 48, 4, 4, "CAUSAL", "fp16"),
+    (1, 100, 2, 4, 64, 3, 3, "CHUNK_VISIBLE", "bf16"),
+    (32, 127, 4, 1, 64, 2, 2, "CAUSAL", "bf16"),
+    (32, 129, 4, 1, 64, 2, 2, "CAUSAL", "bf16"),
+], ids=str)
+def test_backward_in_one_launch_equals_its_stages(gpu_device, case):
+    """dQ and dK/dV of small problems share a launch, whose dK/dV workgroups form the row sums of o * do themselves.  The
+    stages one by one take them from the workspace: same additions in the same order, same bits."""
+    from moda_amd import _lib, ops
+
+    B, T, H, G, D, L, Lv, mode, dtype = case
+    say(f"CASE one launch {case}")
+    dt = {"fp16": torch.float16, "bf16": torch.bfloat16, "fp32": torch.float32}[dtype]
+    gen = torch.Generator(device=gpu_device).manual_seed(T)
+    rn = lambda *s: (0.5 * torch.randn(*s, generator=gen, device=gpu_device)).to(dt)
+    q, k, v, do = rn(B, T * G, H, D), rn(B, T, H, D), rn(B, T, H, D), rn(B, T * G, H, D)
+    kd, vd = (rn(B, T * L, H, D), rn(B, T * L, H, D)) if L else (None, None)
+    m, cb = getattr(_lib, mode), 16 // G if mode == "CHUNK_VISIBLE" else 0
+    valid = dict(depth_valid=Lv) if L else {}
+    o, lse = ops._raw_fwd(m, q, k, v, kd, vd, 0.1, G, cb, **valid)
+    args = (m, q, k, v, kd, vd, o, lse, do, 0.1, G, cb)
+    together = ops._raw_bwd(*args, **valid)
+    ws = torch.empty(max(4, ops.bwd_workspace(m, q, k, v, kd, vd, G, cb).numel()), dtype=torch.uint8, device=gpu_device)
+    apart = ops._raw_bwd(*args, stages=_lib.STAGE_DELTA | _lib.STAGE_DQ, ws=ws, **valid)
+    apart = ops._raw_bwd(*args, stages=_lib.STAGE_DKV, ws=ws, out=apart, **valid)
+    for name, x, y in zip(("dq", "dk", "dv", "dkd", "dvd"), together, apart):
+        assert (x is None and y is None) or torch.equal(x, y), name
+
+
 def _linear(x, parts, residual=None, gelu=False, ldx=None, K=None):
     """moda_hip_linear through the C entry point; parts: (w, bias, y).  Returns its code."""
     import ctypes
