@@ -18,6 +18,7 @@ hipError_t launch_dkv(const KArgs& a, int dtype, int hd, hipStream_t stream);
 hipError_t launch_bwd_short(const KArgs& a, int dtype, hipStream_t stream);
 hipError_t launch_generic(const KArgs& a, int dtype, int D, int Dv, int which, hipStream_t stream);
 hipError_t launch_fp32(const KArgs& a, int which, hipStream_t stream);
+bool fp32_one_launch(const KArgs& a);
 hipError_t launch_reorg(void* const* layers, int64_t n_layers, int64_t slot0, int64_t L_total, int64_t n_tokens,
                         int64_t row_bytes, void* cache, bool to_cache, hipStream_t stream);
 hipError_t launch_slot(void* const (&layer)[2], const int64_t (&strides)[2][3], void* const (&cache)[2], int64_t slot, int64_t L_total,
@@ -479,9 +480,14 @@ int moda_hip_bwd_stages(const moda_hip_desc* d, const void* q, const void* k, co
   } else if (fp32_matrix(d, a, {{q, d->q}, {k, d->k}, {v, d->v}, {kd, d->kd}, {vd, d->vd}, {o, d->o}, {d_o, d->d_o}, {dq, d->dq},
                                 {dk, d->dk}, {dv, d->dv}, {dkd, d->dkd}, {dvd, d->dvd}})) {
     // the dQ kernel forms the row sums for the dK/dV kernel; a dK/dV stage that runs alone has them formed first
-    if (stages & MODA_HIP_STAGE_DQ) e = moda::launch_fp32(a, 1, s);
-    if (e == hipSuccess && !(stages & MODA_HIP_STAGE_DQ) && stages) e = moda::launch_fp32(a, 3, s);
-    if (e == hipSuccess && (stages & MODA_HIP_STAGE_DKV)) e = moda::launch_fp32(a, 2, s);
+    const bool dq = stages & MODA_HIP_STAGE_DQ, dkv = stages & MODA_HIP_STAGE_DKV;
+    if (dq && dkv && moda::fp32_one_launch(a)) {
+      e = moda::launch_fp32(a, 4, s);
+    } else {
+      if (dq) e = moda::launch_fp32(a, 1, s);
+      if (e == hipSuccess && !dq && stages) e = moda::launch_fp32(a, 3, s);
+      if (e == hipSuccess && dkv) e = moda::launch_fp32(a, 2, s);
+    }
   } else {
     // the generic kernels recompute delta inline; the DELTA stage is a no-op for them
     if (stages & MODA_HIP_STAGE_DQ) e = moda::launch_generic(a, d->dtype, (int)d->D, value_dim(d), 1, s);

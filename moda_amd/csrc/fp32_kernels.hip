@@ -300,18 +300,19 @@ __device__ __forceinline__ float neg_delta_of(const f32x4 (&o)[HD / 16], const f
   return -quad_sum_f32(acc);
 }
 
+// `block`: this workgroup's place among the launch's dQ workgroups
 template <int HD, bool FULL>
-__global__ __launch_bounds__(64 * kFp32RowWaves, 2) void fp32_dq_kernel(const KArgs a_in) {
+__device__ __forceinline__ void fp32_dq_body(const KArgs& a_in, int block) {
   constexpr int W = kFp32RowWaves, KS = HD / 16, H4 = HD / 64;
   extern __shared__ __align__(16) float fp32_smem[];
   float* part = fp32_smem;  // [W][16][HD + 4]
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, q = lane >> 4, wave = uniform(tid >> 6);
   KArgs a = a_in;
-  const int BH = a.B * a.Hq, bh = blockIdx.x % BH;
+  const int BH = a.B * a.Hq, bh = block % BH;
   int b = bh / a.Hq;
   const int hq = bh % a.Hq, hkv = hq / a.hdiv;
   enter_sequence(a, b, 2);
-  const int qt = query_tile_of(blockIdx.x, BH, 16, a_in.Tq);
+  const int qt = query_tile_of(block, BH, 16, a_in.Tq);
   if (qt * 16 >= a.Tq) return;
   const int r = qt * 16 + n, rc = imin(r, a.Tq - 1);
   f32x4 Q[KS], dO[KS];
@@ -372,6 +373,11 @@ __global__ __launch_bounds__(64 * kFp32RowWaves, 2) void fp32_dq_kernel(const KA
   }
 }
 
+template <int HD, bool FULL>
+__global__ __launch_bounds__(64 * kFp32RowWaves, 2) void fp32_dq_kernel(const KArgs a) {
+  fp32_dq_body<HD, FULL>(a, blockIdx.x);
+}
+
 // Minus rowsum(o * do) alone, for a dK/dV stage that runs without the dQ stage: one wave per 16 rows.
 template <int HD, bool FULL>
 __global__ __launch_bounds__(64) void fp32_delta_kernel(const KArgs a_in) {
@@ -397,16 +403,18 @@ __global__ __launch_bounds__(64) void fp32_delta_kernel(const KArgs a_in) {
 template <int HD>
 constexpr int kFp32ColWaves = HD <= 64 ? 8 : 4;
 
-template <int HD, bool FULL>
-__global__ __launch_bounds__(64 * kFp32ColWaves<HD>, HD <= 64 ? 2 : 1) void fp32_dkv_kernel(const KArgs a_in) {
+// `block`: this workgroup's place among the launch's dK/dV workgroups.  OWN_DELTA: the row sums of o * do are formed here, block
+// by block (a launch that runs beside the dQ workgroups cannot read theirs); the same additions in the same order as there
+template <int HD, bool FULL, bool OWN_DELTA>
+__device__ __forceinline__ void fp32_dkv_body(const KArgs& a_in, int block) {
   constexpr int W = kFp32ColWaves<HD>, KS = HD / 16, H4 = HD / 64, PART = 16 * kPartRow<HD>;
   extern __shared__ __align__(16) float fp32_smem[];
   float* part = fp32_smem;  // [2 (dk, dv)][W][16][HD + 4]
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, q = lane >> 4, wave = uniform(tid >> 6);
   KArgs a = a_in;
-  const int BHk = a.B * a.Hkv, bh = blockIdx.x % BHk;
+  const int BHk = a.B * a.Hkv, bh = block % BHk;
   int b = bh / a.Hkv;
-  const int hkv = bh % a.Hkv, tile = blockIdx.x / BHk, n_seq_tiles = a_in.has_seq ? (a_in.T + 15) / 16 : 0;
+  const int hkv = bh % a.Hkv, tile = block / BHk, n_seq_tiles = a_in.has_seq ? (a_in.T + 15) / 16 : 0;
   enter_sequence(a, b, 2);
   const bool dep = tile >= n_seq_tiles;
   const int ncols = dep ? a.T * a.Lv : a.T;
@@ -433,6 +441,7 @@ __global__ __launch_bounds__(64 * kFp32ColWaves<HD>, HD <= 64 ? 2 : 1) void fp32
   clear<HD>(dv);
   const float sc = a.scale * kLog2e;
   f32x4 Q[KS], dO[KS], QT[4][H4], dOT[4][H4];
+  f32x4 O[OWN_DELTA ? KS : 1];
   float lse[4], neg_delta[4];
   struct Rows {
     const float *q, *d_o;  // slices of the query head
@@ -452,8 +461,9 @@ __global__ __launch_bounds__(64 * kFp32ColWaves<HD>, HD <= 64 ? 2 : 1) void fp32
     for (int i = 0; i < 4; i++) {
       const int ri = imin(x.r0 + 4 * q + i, a.Tq - 1);
       lse[i] = a.lse[((int64_t)b * a.Tq + ri) * a.Hq + x.hq];
-      neg_delta[i] = a.delta[((int64_t)b * a.Hq + x.hq) * a.delta_pitch + ri];
+      if (!OWN_DELTA) neg_delta[i] = a.delta[((int64_t)b * a.Hq + x.hq) * a.delta_pitch + ri];
     }
+    if constexpr (OWN_DELTA) load_score_operand<HD, FULL>(O, (const float*)a.o + b * a.so.b + x.hq * a.so.h + r * a.so.t, q, a.Dv);
   };
   const int blk0 = dep ? 0 : wave, step = dep ? 1 : W;
   if (blk0 < nblk) load_rows(blk0);
@@ -464,6 +474,11 @@ __global__ __launch_bounds__(64 * kFp32ColWaves<HD>, HD <= 64 ? 2 : 1) void fp32
       const int64_t r = imin(x.r0 + 4 * q + i, a.Tq - 1);
       load_sum_operand<HD, FULL>(QT[i], x.q + r * a.sq.t, n, a.D);
       load_sum_operand<HD, FULL>(dOT[i], x.d_o + r * a.sdo.t, n, a.Dv);
+    }
+    if constexpr (OWN_DELTA) {  // lane (n, .) has the sum of row n, its accumulators hold rows 4 q + i
+      const float row_sum = neg_delta_of<HD>(O, dO);
+#pragma unroll
+      for (int i = 0; i < 4; i++) neg_delta[i] = __shfl(row_sum, 4 * q + i, 64);
     }
     __builtin_amdgcn_sched_barrier(0);
     const f32x4 s = scores<HD>(Q, K, f32x4{0.f, 0.f, 0.f, 0.f});
@@ -528,22 +543,38 @@ __global__ __launch_bounds__(64 * kFp32ColWaves<HD>, HD <= 64 ? 2 : 1) void fp32
   }
 }
 
+template <int HD, bool FULL>
+__global__ __launch_bounds__(64 * kFp32ColWaves<HD>, HD <= 64 ? 2 : 1) void fp32_dkv_kernel(const KArgs a) {
+  fp32_dkv_body<HD, FULL, false>(a, blockIdx.x);
+}
+
+// dQ and dK/dV of a problem that leaves compute units idle in one launch, their workgroups side by side: two chains of a few
+// dependent blocks behind one start and one end.  B=1 T=256 H=4 D=64 L=4 causal: the replayed training step 33.1 -> 23.9 us.
+template <bool FULL>
+__global__ __launch_bounds__(64 * kFp32RowWaves, 2) void fp32_bwd_kernel(const KArgs a, int row_blocks) {
+  static_assert(kFp32ColWaves<64> == kFp32RowWaves, "workgroups of one size");
+  if ((int)blockIdx.x < row_blocks)
+    fp32_dq_body<64, FULL>(a, blockIdx.x);
+  else
+    fp32_dkv_body<64, FULL, true>(a, (int)blockIdx.x - row_blocks);
+}
+
 namespace {
 
-template <typename Kernel>
-hipError_t launch(Kernel kernel, LdsAttrState& attr, const KArgs& a, int64_t nblk, int threads, size_t smem, hipStream_t stream) {
+template <typename Kernel, typename... More>
+hipError_t launch(Kernel kernel, LdsAttrState& attr, const KArgs& a, int64_t nblk, int threads, size_t smem, hipStream_t stream, More... more) {
   if (nblk == 0) return hipSuccess;
   if (nblk >= (1ll << 31)) return hipErrorInvalidValue;
   const hipError_t e = allow_dynamic_lds(attr, reinterpret_cast<const void*>(kernel), smem);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)nblk), dim3(threads), smem, stream, a);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)nblk), dim3(threads), smem, stream, a, more...);
   return hipGetLastError();
 }
 
 template <int HD, bool FULL>
 hipError_t launch_fp32_t(const KArgs& a, int which, hipStream_t stream) {
   constexpr size_t part = (size_t)16 * kPartRow<HD> * sizeof(float);
-  static LdsAttrState attr[4];
+  static LdsAttrState attr[5];
   const int64_t row_tiles = (int64_t)((a.Tq + 15) / 16) * a.B * a.Hq;
   if (which == 0)
     return launch(&fp32_fwd_kernel<HD, FULL>, attr[0], a, row_tiles, 64 * kFp32RowWaves,
@@ -552,12 +583,23 @@ hipError_t launch_fp32_t(const KArgs& a, int which, hipStream_t stream) {
   if (which == 3) return launch(&fp32_delta_kernel<HD, FULL>, attr[3], a, row_tiles, 64, 0, stream);
   constexpr int W = kFp32ColWaves<HD>;
   const int64_t seq = a.has_seq ? (a.T + 15) / 16 : 0, dep = ((int64_t)a.T * a.Lv + 16 * W - 1) / (16 * W);
-  return launch(&fp32_dkv_kernel<HD, FULL>, attr[2], a, (seq + dep) * a.B * a.Hkv, 64 * W, 2 * W * part, stream);
+  const int64_t columns = (seq + dep) * a.B * a.Hkv;
+  if constexpr (HD == 64) {
+    if (which == 4) return launch(&fp32_bwd_kernel<FULL>, attr[4], a, row_tiles + columns, 64 * W, 2 * W * part, stream, (int)row_tiles);
+  }
+  return launch(&fp32_dkv_kernel<HD, FULL>, attr[2], a, columns, 64 * W, 2 * W * part, stream);
 }
 
 }  // namespace
 
-// which: 0 forward, 1 dQ (leaves the row sums of o * do in the workspace), 2 dK/dV (reads them), 3 the row sums alone
+// Whether dQ and dK/dV go as one launch: all workgroups run at once (one per compute unit; head dims above 64 have dK/dV
+// workgroups of another size).  More than that and the row sums, formed twice, cost more than the launch.
+bool fp32_one_launch(const KArgs& a) {
+  const int64_t cols = (a.has_seq ? (a.T + 15) / 16 : 0) + ((int64_t)a.T * a.Lv + 127) / 128;
+  return a.D <= 64 && a.Dv <= 64 && ((int64_t)(a.Tq + 15) / 16 * a.Hq + cols * a.Hkv) * a.B <= a.compute_units;
+}
+
+// which: 4 dQ and dK/dV in one launch; 0 forward, 1 dQ (leaves the row sums of o * do in the workspace), 2 dK/dV (reads them), 3 the row sums alone
 hipError_t launch_fp32(const KArgs& a, int which, hipStream_t stream) {
   const int hd = a.D > a.Dv ? a.D : a.Dv;
   if (hd <= 64) return a.D == 64 && a.Dv == 64 ? launch_fp32_t<64, true>(a, which, stream) : launch_fp32_t<64, false>(a, which, stream);

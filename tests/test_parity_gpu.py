@@ -1887,6 +1887,13 @@ def test_stack_widths_and_which_of_them_run_as_native_launches(gpu_device, case)
     (1, 100, 2, 4, 64, 3, 3, "CHUNK_VISIBLE", "bf16"),
     (32, 127, 4, 1, 64, 2, 2, "CAUSAL", "bf16"),
     (32, 129, 4, 1, 64, 2, 2, "CAUSAL", "bf16"),
+    # fp32: both instantiations, one row, an empty and a partial stream, chunk-visible, the last size in one launch
+    (1, 1, 1, 1, 64, 1, 1, "CAUSAL", "fp32"),
+    (1, 256, 4, 1, 64, 4, 4, "CAUSAL", "fp32"),
+    (2, 61, 2, 2, 36, 3, 2, "NONCAUSAL", "fp32"),
+    (1, 90, 2, 3, 64, 0, 0, "CAUSAL", "fp32"),
+    (1, 70, 2, 4, 20, 3, 3, "CHUNK_VISIBLE", "fp32"),
+    (1, 1024, 1, 2, 64, 8, 8, "CAUSAL", "fp32"),
 ], ids=str)
 def test_backward_in_one_launch_equals_its_stages(gpu_device, case):
     """dQ and dK/dV of small problems share a launch, whose dK/dV workgroups form the row sums of o * do themselves.  The
