@@ -27,11 +27,16 @@
 namespace moda {
 
 // VARLEN: packed variable-length batch (a workgroup enters its sequence; column tiles past its end leave at once)
-// `block`: this workgroup's place among the launch's dK/dV workgroups
+// As a kernel of its own or, MODA_SIDE_BY_SIDE, as a function (see dq_kernel); `block` is the workgroup's place among these
 // OWN_DELTA: the row sums of o * do are formed here, tile by tile (a launch that runs beside the dQ kernel's workgroups
 // cannot read theirs); the same additions in the same order as there
 template <typename T, int HD, bool VARLEN, bool SPLIT, int RW = 1, bool OWN_DELTA = false>
+#ifdef MODA_SIDE_BY_SIDE
 __device__ __forceinline__ void dkv_flat_body(const KArgs& a_in, int block) {
+#else
+__global__ __launch_bounds__(256, RW == 1 ? 3 : 2) void dkv_flat_kernel(const KArgs a_in) {
+  const int block = blockIdx.x;
+#endif
   static_assert(RW == 1 || (RW == 4 && !VARLEN && !SPLIT), "four row waves: fixed length, no segments");
   static_assert(!OWN_DELTA || (!VARLEN && HD == 64), "row sums of fixed-length launches, eight chunks a row");
   constexpr int NB = 2, WM = 32, BM = WM * RW, MBLK = WM / 16, BN = 4 / RW * 16 * NB, KS = HD / 32, MB = HD / 16;

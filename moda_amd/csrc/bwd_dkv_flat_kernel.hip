@@ -4,11 +4,6 @@
 namespace moda {
 
 template <typename T, int HD, bool VARLEN, bool SPLIT, int RW = 1>
-__global__ __launch_bounds__(256, RW == 1 ? 3 : 2) void dkv_flat_kernel(const KArgs a) {
-  dkv_flat_body<T, HD, VARLEN, SPLIT, RW>(a, blockIdx.x);
-}
-
-template <typename T, int HD, bool VARLEN, bool SPLIT, int RW = 1>
 hipError_t launch_dkv_flat_t(const KArgs& a, hipStream_t stream) {
   constexpr size_t smem = dkv_flat_lds<HD, RW, false>();
   static LdsAttrState attr;

@@ -52,11 +52,6 @@ __global__ __launch_bounds__(256) void delta_kernel(const KArgs a_in) {
   if (r < a.Tq && (tid % TPR) == 0) a.delta[((int64_t)b * a.Hq + hq) * a.delta_pitch + r] = -acc;
 }
 
-template <typename T, int HD, typename Shape, int ADDR>
-__global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a) {
-  dq_body<T, HD, Shape, ADDR>(a, blockIdx.x);
-}
-
 template <typename T, int HD>
 hipError_t launch_delta_t(const KArgs& a, hipStream_t stream) {
   if (a.Tq == 0 || a.B * a.Hq == 0) return hipSuccess;

@@ -3,6 +3,7 @@
 // tiles behind its own start and end; together they take as long as the longer one.  The dK/dV workgroups form the row sums
 // of o * do themselves (OWN_DELTA).  2 x 95 tokens, four heads of two query rows, eight slots, fp16: 25.6 -> 19.8
 // us of kernels and a launch less, the replayed training step 35.0 -> 29.3 us; 8 x 197 tokens, six heads, twelve slots 71.1 -> 64.2.
+#define MODA_SIDE_BY_SIDE
 #include "bwd_dkv_flat.h"
 #include "bwd_dq.h"
 
