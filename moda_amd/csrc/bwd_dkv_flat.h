@@ -49,13 +49,11 @@ __global__ __launch_bounds__(256, RW == 1 ? 3 : 2) void dkv_flat_kernel(const KA
 
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, q4 = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int BHk = a_in.B * a_in.Hkv;
-  const int bh = block % BHk;
-  const int ct = block / BHk;
-  int b = bh / a_in.Hkv;
-  const int hkv = bh % a_in.Hkv;
-  const int seq_index = b;
-  SeqArgs<VARLEN> seq(a_in, b);
+  const ColPlace place = col_place<VARLEN>(a_in, (int)block, BN, SPLIT ? a_in.dkv_split : 1);
+  if (VARLEN && !place.active) return;
+  const int ct = place.ct, hkv = place.hkv;
+  int b = place.b;
+  SeqArgs<VARLEN> seq(a_in, b, place.t0, place.T);
   const KArgs& a = seq.a;
   const ColTilePlan plan = col_tile_plan(a_in, a, ct, BN, BM, VARLEN, SPLIT ? a.dkv_split : 1);
   if ((VARLEN || SPLIT) && !plan.active) return;  // a tile beyond its sequence, or a segment beyond its tile
@@ -318,7 +316,7 @@ __global__ __launch_bounds__(256, RW == 1 ? 3 : 2) void dkv_flat_kernel(const KA
   }
   if (SPLIT && plan.nsegs > 1) {  // a row segment: fp32 partial sums, added up by dkv_reduce_kernel
     const int64_t pitch = part_rows(a), plane = (int64_t)(VARLEN ? 1 : a.B) * a.Hkv * pitch * HD;
-    const int first = VARLEN ? a_in.cu[seq_index] : 0;
+    const int first = VARLEN ? place.t0 : 0;
 #pragma unroll
     for (int nb = 0; nb < NB; nb++)
       if (valid[nb]) {

@@ -53,13 +53,11 @@ __global__ __launch_bounds__(512) void dkv_kernel(const KArgs a_in) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kblk = wave & 3;
   const bool role_b = wave >= 4;
-  const int BHk = a_in.B * a_in.Hkv;
-  const int bh = blockIdx.x % BHk;
-  const int ct = blockIdx.x / BHk;
-  int b = bh / a_in.Hkv;
-  const int hkv = bh % a_in.Hkv;
-  const int seq_index = b;
-  SeqArgs<VARLEN> seq(a_in, b);
+  const ColPlace place = col_place<VARLEN>(a_in, (int)blockIdx.x, BN, SPLIT ? a_in.dkv_split : 1);
+  if (VARLEN && !place.active) return;
+  const int ct = place.ct, hkv = place.hkv;
+  int b = place.b;
+  SeqArgs<VARLEN> seq(a_in, b, place.t0, place.T);
   const KArgs& a = seq.a;
   // sequence tiles come `nseg` workgroups each (row segments of one column tile are neighbours in the grid, the
   // heaviest column tile first), then the depth tiles
@@ -363,7 +361,7 @@ __global__ __launch_bounds__(512) void dkv_kernel(const KArgs a_in) {
   if (SPLIT && !dep && plan.nsegs > 1) {
     // a row segment: fp32 partial sums, added up by dkv_reduce_kernel
     const int64_t pitch = part_rows(a), plane = (int64_t)(VARLEN ? 1 : a.B) * a.Hkv * pitch * HD;
-    const int first = VARLEN ? a_in.cu[seq_index] : 0;
+    const int first = VARLEN ? place.t0 : 0;
     const float mul = role_b ? a.scale : 1.f;
 #pragma unroll
     for (int nb = 0; nb < NB; nb++)
@@ -1023,19 +1021,20 @@ hipError_t launch_dkv_t(const KArgs& a, hipStream_t stream) {
   }
   if (depth_by_columns && (int64_t)a.B * a.T > 0) {
     constexpr int CPB = 4 * (64 / (HD / 8));
-    const int64_t nx = (((int64_t)a.T * a.L + CPB - 1) / CPB) * a.B * a.Hkv;
+    const KArgs one = packed_as_one(a);
+    const int64_t nx = (((int64_t)one.T * a.L + CPB - 1) / CPB) * one.B * a.Hkv;
     if (nx >= (1ll << 31)) return hipErrorInvalidValue;
     if constexpr (HD <= 128) {
       if (a.depth_p && a.Gf <= 4) {
         constexpr int TPB = 4 * (64 / (HD / 8));
-        const int64_t nt = (((int64_t)a.T + TPB - 1) / TPB) * a.B * a.Hkv;
-        hipLaunchKernelGGL((depth_token_handed_kernel<T, HD>), dim3((unsigned)nt), dim3(256), 0, stream, a);
+        const int64_t nt = (((int64_t)one.T + TPB - 1) / TPB) * one.B * a.Hkv;
+        hipLaunchKernelGGL((depth_token_handed_kernel<T, HD>), dim3((unsigned)nt), dim3(256), 0, stream, one);
       } else if (a.depth_p)
-        hipLaunchKernelGGL((depth_cols_handed_kernel<T, HD>), dim3((unsigned)nx), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((depth_cols_handed_kernel<T, HD>), dim3((unsigned)nx), dim3(256), 0, stream, one);
       else
-        hipLaunchKernelGGL((depth_cols_kernel<T, HD>), dim3((unsigned)nx), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((depth_cols_kernel<T, HD>), dim3((unsigned)nx), dim3(256), 0, stream, one);
     } else {
-      hipLaunchKernelGGL((depth_cols_kernel<T, HD>), dim3((unsigned)nx), dim3(256), 0, stream, a);
+      hipLaunchKernelGGL((depth_cols_kernel<T, HD>), dim3((unsigned)nx), dim3(256), 0, stream, one);
     }
   }
   return hipGetLastError();

@@ -35,16 +35,13 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
   // so that it cannot disturb the register allocation of their main loop
   constexpr bool NODEPTH = (ADDR & 4) != 0, PARTIAL = (ADDR & 8) != 0;
   static_assert(!(NODEPTH && PARTIAL), "a partially filled depth stream is a depth stream");
-  const int BH = a_in.B * a_in.Hq;
-  const int bh = block % BH;
-  int b = bh / a_in.Hq;
-  const int hq = bh % a_in.Hq, hkv = hq / a_in.hdiv;
-  SeqArgs<VARLEN> seq(a_in, b);
+  const RowPlace place = row_place<VARLEN>(a_in, (int)block, BM);
+  if (VARLEN && !place.active) return;
+  int b = place.b;
+  const int hq = place.hq, hkv = hq / a_in.hdiv, qt = place.qt;
+  SeqArgs<VARLEN> seq(a_in, b, place.t0, place.T);
   const KArgs& a = seq.a;
   const int Ld = NODEPTH ? 0 : a.L;  // depth slots per token
-  const int nqt = (a.Tq + BM - 1) / BM;
-  const int qt = query_tile_of(block, BH, BM, VARLEN ? a_in.Tq : a.Tq);
-  if (VARLEN && qt >= nqt) return;
 
   i32x4 Qr[NB][KS], dOr[NB][KS];
   float lse[NB], delta[NB];

@@ -49,17 +49,13 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
   // so that it cannot disturb the register allocation of their main loop
   constexpr bool NODEPTH = (ADDR & 4) != 0, PARTIAL = (ADDR & 8) != 0;
   static_assert(!(NODEPTH && PARTIAL), "a partially filled depth stream is a depth stream");
-  const int BH = a_in.B * a_in.Hq;
-  const int bh = blockIdx.x % BH;
-  int b = bh / a_in.Hq;
-  const int hq = bh % a_in.Hq, hkv = hq / a_in.hdiv;
-  SeqArgs<VARLEN> seq(a_in, b);
+  const RowPlace place = row_place<VARLEN>(a_in, (int)blockIdx.x, BM);
+  if (VARLEN && !place.active) return;
+  int b = place.b;
+  const int hq = place.hq, hkv = hq / a_in.hdiv, qt = place.qt;
+  SeqArgs<VARLEN> seq(a_in, b, place.t0, place.T);
   const KArgs& a = seq.a;
   const int Ld = NODEPTH ? 0 : a.L;  // depth slots per token
-  const int nqt = (a.Tq + BM - 1) / BM;
-  // heavy (late) tiles first; the positions a shorter sequence of a variable-length batch does not have are dropped
-  const int qt = query_tile_of(blockIdx.x, BH, BM, VARLEN ? a_in.Tq : a.Tq);
-  if (VARLEN && qt >= nqt) return;
   const int r = qt * BM + wave * 32 + n;
   const bool valid = r < a.Tq;
   const int t = r / a.Gf;
@@ -411,16 +407,12 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void fwd_wide_kernel(const KArgs 
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 15, q4 = lane >> 4;
   constexpr bool WIDE = (ADDR & 1) != 0, VARLEN = (ADDR & 2) != 0, PARTIAL = (ADDR & 8) != 0;
-  const int BH = a_in.B * a_in.Hq;
-  const int bh = blockIdx.x % BH;
-  int b = bh / a_in.Hq;
-  const int hq = bh % a_in.Hq, hkv = hq / a_in.hdiv;
-  SeqArgs<VARLEN> seq(a_in, b);
+  const RowPlace place = row_place<VARLEN>(a_in, (int)blockIdx.x, BM);
+  if (VARLEN && !place.active) return;
+  int b = place.b;
+  const int hq = place.hq, hkv = hq / a_in.hdiv, qt = place.qt;
+  SeqArgs<VARLEN> seq(a_in, b, place.t0, place.T);
   const KArgs& a = seq.a;
-  const int nqt = (a.Tq + BM - 1) / BM;
-  // heavy (late) tiles first; the positions a shorter sequence of a variable-length batch does not have are dropped
-  const int qt = query_tile_of(blockIdx.x, BH, BM, VARLEN ? a_in.Tq : a.Tq);
-  if (VARLEN && qt >= nqt) return;
   i32x4 Qr[NB][KS];
   int shi[NB], dlo[NB], dhi[NB];  // per-row visible column intervals [lo, hi) for the two phases
 #pragma unroll

@@ -32,6 +32,125 @@ MODA_HD int64_t depth_row_of(const KArgs& a, int c) {
 // together; a result >= the sequence's own tile count means the workgroup has nothing to do.
 MODA_HD int query_tile_of(int block, int BH, int BM, int Tq_grid) { return (Tq_grid + BM - 1) / BM - 1 - block / BH; }
 
+// Packed order: the tiles of all sequences of a packed batch as one list, by cost level (row kernels: the tile's index;
+// dK/dV: how many column tiles lie behind it), the highest level first and the sequences that reach a level in turn; the
+// heads of a tile are neighbours in the grid.  A workgroup finds its place itself: N(j) = sum of max(0, tiles - j) counts
+// the list's entries at level j or above, its level is the largest j with N(j) > rank.
+// What it replaces, a grid of the longest sequence for every one, launched mostly workgroups without work on unequal
+// lengths, and sent a (sequence, head) to the XCD that its index fell on (block % 8): with B * H a multiple of 8 the longest
+// sequence's tiles stayed on as many XCDs as it has heads.  Training steps: 16 sequences of 113 - 7441 tokens, two heads of
+// four, head dim 64: 3480 -> 737 us; twelve of 338 - 7523, four heads of two: 1296 -> 666; 8192 + 3 x 64 tokens, two heads of
+// two, head dim 128: 1139 -> 766; 16 384 to 2048 tokens, 15 sequences, four heads of four: 10.14 -> 9.84 ms; 200 of 300 each:
+// 1710 -> 1671 us.  Where all workgroups run at once it can go the other way, by which of them share a compute unit (five
+// sequences of 226 - 6188, two heads of two, head dim 64: 356 -> 364).
+// Up to kPackedOrderMax sequences, whose tile counts a wave holds in four registers; more keep that grid.
+constexpr int kPackedOrderMax = 256;
+MODA_HD bool packed_order(const KArgs& a) { return a.cu != nullptr && a.B <= kPackedOrderMax; }
+// length of the list, at most: every sequence has one tile that is not full (rows_per_token: query rows, or 1 for keys)
+MODA_HD int64_t packed_ranks(const KArgs& a, int rows_per_token, int BM) {
+  const int64_t grid = (int64_t)(((int64_t)a.T * rows_per_token + BM - 1) / BM) * a.B;
+  const int64_t list = (int64_t)(a.delta_pitch / a.Gf) * rows_per_token / BM + a.B;
+  return grid < list ? grid : list;
+}
+struct PackedTile {
+  int seq, level;
+  int t0, T;    // the sequence's first token and length
+  bool active;  // false: past the end of the list
+};
+MODA_HD PackedTile packed_tile(const KArgs& a, int rows_per_token, int BM, int rank) {
+  PackedTile p = {0, 0, 0, 0, false};
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int P = kPackedOrderMax / 64;
+  const int lane = threadIdx.x & 63;
+  int tiles[P], t0[P], T[P];
+#pragma unroll
+  for (int i = 0; i < P; i++) {
+    const int s = 64 * i + lane;
+    t0[i] = T[i] = 0;
+    if (s < a.B) {
+      t0[i] = a.cu[s];
+      T[i] = a.cu[s + 1] - t0[i];
+    }
+    tiles[i] = (T[i] * rows_per_token + BM - 1) / BM;
+  }
+  const auto entries_from = [&](int j) {  // N(j)
+    int x = 0;
+#pragma unroll
+    for (int i = 0; i < P; i++) x += imax(0, tiles[i] - j);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8: sums of 16 lanes
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast 15, 31: lane 63 holds all
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+    return __builtin_amdgcn_readlane(x, 63);
+  };
+#else
+  const auto tiles_of = [&](int s) { return ((a.cu[s + 1] - a.cu[s]) * rows_per_token + BM - 1) / BM; };
+  const auto entries_from = [&](int j) {
+    int x = 0;
+    for (int s = 0; s < a.B; s++) x += imax(0, tiles_of(s) - j);
+    return x;
+  };
+#endif
+  if (entries_from(0) <= rank) return p;
+  int lo = 0, hi = (a.T * rows_per_token + BM - 1) / BM, above = 0;  // N(lo) > rank >= N(hi) = above
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) / 2, n = entries_from(mid);
+    if (n > rank) {
+      lo = mid;
+    } else {
+      hi = mid;
+      above = n;
+    }
+  }
+  p.level = lo;
+  int nth = rank - above;  // among the sequences that reach the level
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+  for (int i = 0; i < P; i++) {
+    const uint64_t there = __builtin_amdgcn_ballot_w64(tiles[i] > lo);
+    const int count = __builtin_popcountll(there);
+    if (!p.active && nth < count) {
+      const int before = __builtin_amdgcn_mbcnt_hi((uint32_t)(there >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)there, 0));
+      const int at = __builtin_ctzll(__builtin_amdgcn_ballot_w64(tiles[i] > lo && before == nth));
+      p.seq = 64 * i + at;
+      p.t0 = __builtin_amdgcn_readlane(t0[i], at);
+      p.T = __builtin_amdgcn_readlane(T[i], at);
+      p.active = true;
+    }
+    nth -= count;
+  }
+#else
+  for (int s = 0; s < a.B && !p.active; s++)
+    if (tiles_of(s) > lo && nth-- == 0) {
+      p.seq = s;
+      p.t0 = a.cu[s];
+      p.T = a.cu[s + 1] - p.t0;
+      p.active = true;
+    }
+#endif
+  return p;
+}
+
+// Which (batch entry, query head, query tile) a workgroup of the forward or dQ kernel takes.
+struct RowPlace {
+  int b, hq, qt;
+  int t0, T;  // packed batch: the sequence's first token and length
+  bool active;
+};
+template <bool VARLEN>
+MODA_HD RowPlace row_place(const KArgs& grid, int block, int BM) {
+  if (VARLEN && packed_order(grid)) {
+    const PackedTile p = packed_tile(grid, grid.Gf, BM, block / grid.Hq);
+    return {p.seq, block % grid.Hq, p.level, p.t0, p.T, p.active};
+  }
+  const int BH = grid.B * grid.Hq, bh = block % BH;
+  const int b = bh / grid.Hq, qt = query_tile_of(block, BH, BM, grid.Tq);
+  const int t0 = VARLEN ? grid.cu[b] : 0, T = VARLEN ? grid.cu[b + 1] - t0 : grid.T;
+  return {b, bh % grid.Hq, qt, t0, T, !VARLEN || qt < (T * grid.Gf + BM - 1) / BM};
+}
+
 // Visible column intervals [0, shi) of the sequence keys and [dlo, dhi) of the depth columns (compact axis) for
 // query row r (all zero for a row past the end).  Ld: depth slots per token, 0 when the launch has no depth stream.
 struct RowVis {
@@ -183,6 +302,34 @@ MODA_HD ColTilePlan col_tile_plan(const KArgs& grid, const KArgs& a, int ct, int
   return p;
 }
 
+// Which (batch entry, kv head, column-tile workgroup `ct` of it) a workgroup of the dK/dV kernels takes.  A batch in packed
+// order has the sequence tiles of all its sequences first, then the depth tiles as every other launch has them.
+struct ColPlace {
+  int b, hkv, ct;
+  int t0, T;
+  bool active;
+};
+template <bool VARLEN>
+MODA_HD ColPlace col_place(const KArgs& grid, int block, int BN, int nseg) {
+  const int BHk = grid.B * grid.Hkv;
+  int ct0 = 0;
+  if (VARLEN && packed_order(grid)) {
+    const int n_seq_tiles = grid.has_seq ? (grid.T + BN - 1) / BN : 0;
+    const int seq_blocks = grid.has_seq ? (int)packed_ranks(grid, 1, BN) * nseg * grid.Hkv : 0;
+    if (block < seq_blocks) {
+      const int seg = block / grid.Hkv;  // of all ranks
+      const PackedTile p = packed_tile(grid, 1, BN, seg / nseg);
+      const int tile = grid.causal ? n_seq_tiles - 1 - p.level : p.level;  // as col_tile_plan counts them
+      return {p.seq, block % grid.Hkv, tile * nseg + seg % nseg, p.t0, p.T, p.active};
+    }
+    block -= seq_blocks;
+    ct0 = n_seq_tiles * nseg;
+  }
+  const int bh = block % BHk, b = bh / grid.Hkv;
+  const int t0 = VARLEN ? grid.cu[b] : 0, T = VARLEN ? grid.cu[b + 1] - t0 : grid.T;
+  return {b, bh % grid.Hkv, ct0 + block / BHk, t0, T, true};
+}
+
 // rows of query tile starting at row f_q0 that exist (only a head's top tile can be short)
 MODA_HD int query_tile_rows(const KArgs& a, int f_q0, int BM) { return imax(imin(a.Tq - f_q0, BM), 0); }
 
@@ -198,19 +345,23 @@ inline int64_t linear_blocks(int m_tiles, int n_tiles) { return 8ll * ((m_tiles 
 // Launch grids (host side), one place for the launchers and the walker.
 // ---------------------------------------------------------------------------------------------------
 inline int64_t row_kernel_blocks(const KArgs& a, int rows_per_block) {
+  if (packed_order(a)) return packed_ranks(a, a.Gf, rows_per_block) * a.Hq;
   return (int64_t)((a.Tq + rows_per_block - 1) / rows_per_block) * a.B * a.Hq;
 }
 // chunk-visible depth columns: by whole chunks when a chunk's rows fit one 64-row query tile (tile widths up to 128:
 // the chunk kernel's registers and LDS do not stretch to 256), else as column tiles of the dK/dV kernel
 inline bool depth_by_chunks(const KArgs& a, int HD) { return HD <= 128 && a.L > 0 && a.chunk && (int64_t)a.Cb * a.Gf <= 64; }
+// sequence column tiles of a launch, all batch entries together
+inline int64_t seq_col_tiles(const KArgs& a, int BN) {
+  return !a.has_seq ? 0 : packed_order(a) ? packed_ranks(a, 1, BN) : (int64_t)((a.T + BN - 1) / BN) * a.B;
+}
 inline int64_t col_kernel_blocks(const KArgs& a, int HD, int BN, int nseg) {
-  const int64_t n_seq_tiles = a.has_seq ? (a.T + BN - 1) / BN : 0;
   const int64_t n_dep_tiles = (a.L > 0 && a.chunk && !depth_by_chunks(a, HD)) ? ((int64_t)a.T * a.Lv + BN - 1) / BN : 0;
-  return (n_seq_tiles * nseg + n_dep_tiles) * a.B * a.Hkv;
+  return (seq_col_tiles(a, BN) * nseg + n_dep_tiles * a.B) * a.Hkv;
 }
 // Sequence dK/dV on the 64-wide tiles: dkv_flat_kernel (three workgroups per compute unit, where dkv_kernel fits one)
 // takes every launch of sequence-key column tiles whose kv head is the query head.
-inline int64_t dkv_flat_blocks(const KArgs& a, int BN = 128) { return a.has_seq ? (int64_t)((a.T + BN - 1) / BN) * a.B * a.Hkv : 0; }
+inline int64_t dkv_flat_blocks(const KArgs& a, int BN = 128) { return seq_col_tiles(a, BN) * a.Hkv; }
 inline bool takes_dkv_flat(const KArgs& a, int HD) {
   return HD == 64 && a.has_seq && a.hdiv == 1 && col_kernel_blocks(a, HD, 128, 1) == dkv_flat_blocks(a);
 }

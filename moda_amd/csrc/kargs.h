@@ -60,10 +60,7 @@ __host__ __device__ __forceinline__ int part_rows(const KArgs& a) { return a.cu 
 // sequence's length, so that the code after it addresses the sequence as batch 0 of a fixed-length problem.
 // The launch grid is sized for the longest sequence: callers drop the tiles beyond their own sequence.
 // `units`: 16-bit units per tensor element (the data pointers are typed for 16-bit elements).
-__host__ __device__ __forceinline__ void enter_sequence(KArgs& a, int& b, int units = 1) {
-  if (a.cu == nullptr) return;
-  const int t0 = a.cu[b];
-  const int T = a.cu[b + 1] - t0;
+__host__ __device__ __forceinline__ void enter_sequence_at(KArgs& a, int t0, int T, int units) {
   const int64_t r0 = (int64_t)t0 * a.Gf * units, c0 = (int64_t)t0 * a.L * units, k0 = (int64_t)t0 * units;
   a.q += r0 * a.sq.t;
   a.o += r0 * a.so.t;
@@ -86,7 +83,23 @@ __host__ __device__ __forceinline__ void enter_sequence(KArgs& a, int& b, int un
   }
   a.T = T;
   a.Tq = T * a.Gf;
+}
+__host__ __device__ __forceinline__ void enter_sequence(KArgs& a, int& b, int units = 1) {
+  if (a.cu == nullptr) return;
+  const int t0 = a.cu[b];
+  enter_sequence_at(a, t0, a.cu[b + 1] - t0, units);
   b = 0;
+}
+
+// Depth columns outside chunk-visible mode meet the query rows of their own token only: for them a packed batch is one
+// sequence, and their launch holds no workgroups beyond it.
+__host__ __device__ __forceinline__ KArgs packed_as_one(KArgs a) {
+  if (a.cu == nullptr) return a;
+  a.B = 1;
+  a.T = part_rows(a);
+  a.Tq = a.delta_pitch;
+  a.cu = nullptr;
+  return a;
 }
 
 // The argument block a kernel body works on: the launch's own (fixed-length instantiations, no copy)
@@ -97,11 +110,16 @@ template <>
 struct SeqArgs<false> {
   const KArgs& a;
   __device__ __forceinline__ SeqArgs(const KArgs& in, int&) : a(in) {}
+  __device__ __forceinline__ SeqArgs(const KArgs& in, int&, int, int) : a(in) {}
 };
 template <>
 struct SeqArgs<true> {
   KArgs a;
   __device__ __forceinline__ SeqArgs(const KArgs& in, int& b) : a(in) { enter_sequence(a, b); }
+  __device__ __forceinline__ SeqArgs(const KArgs& in, int& b, int t0, int T) : a(in) {  // its place is known already
+    enter_sequence_at(a, t0, T, 1);
+    b = 0;
+  }
 };
 
 }  // namespace moda

@@ -237,18 +237,16 @@ void walk_row_kernel(const KArgs& a_in, bool dq, int rows_per_wave, bool own_pos
   constexpr int BN = 64, NT = 64 * Shape::W, NST = Shape::NST, DIST = Shape::DIST;
   const int BM = rows_per_wave * Shape::W;
   const bool varlen = a_in.cu != nullptr;
-  const int BH = a_in.B * a_in.Hq;
   const int64_t nblk = row_kernel_blocks(a_in, BM);
   typedef AsyncTileLoader<HD, BN, NT> Loader;
   for (int64_t block = 0; block < nblk; block++) {
-    const int bh = (int)(block % BH);
-    int b = bh / a_in.Hq;
-    const int hq = bh % a_in.Hq, hkv = hq / a_in.hdiv;
+    const RowPlace place = varlen ? row_place<true>(a_in, (int)block, BM) : row_place<false>(a_in, (int)block, BM);
+    if (varlen && !place.active) continue;
+    int b = place.b;
+    const int hq = place.hq, hkv = hq / a_in.hdiv, qt = place.qt;
     const KArgs a = seq_args(a_in, b);
     const int Ld = a.L;
     const int nqt = (a.Tq + BM - 1) / BM;
-    const int qt = query_tile_of((int)block, BH, BM, varlen ? a_in.Tq : a.Tq);
-    if (varlen && qt >= nqt) continue;
     if (qt < 0 || qt >= nqt) fail("%s: query tile %d of %d", kname, qt, nqt);
     const bool own_depth = own_possible && waves_own_depth(a, Ld);
     const RowTilePlan plan = row_tile_plan(a, qt, BM, BN, Ld > 0 && !own_depth);
@@ -460,13 +458,13 @@ void walk_dkv(const KArgs& a_in) {
   const uint32_t stat_byte = NST * 2 * BM * HD * 2 + 2 * 4 * NP * 64 * 16;
   const bool varlen = a_in.cu != nullptr;
   const int nseg = a_in.dkv_split;
-  const int BHk = a_in.B * a_in.Hkv;
   const int64_t nblk = col_kernel_blocks(a_in, HD, BN, nseg);
   typedef AsyncTileLoader<HD, BM, 512> Loader;
   for (int64_t block = 0; block < nblk; block++) {
-    const int bh = (int)(block % BHk), ct = (int)(block / BHk);
-    int b = bh / a_in.Hkv;
-    const int hkv = bh % a_in.Hkv, first = varlen ? a_in.cu[b] : 0;
+    const ColPlace place = varlen ? col_place<true>(a_in, (int)block, BN, nseg) : col_place<false>(a_in, (int)block, BN, nseg);
+    if (varlen && !place.active) continue;
+    int b = place.b;
+    const int ct = place.ct, hkv = place.hkv, first = varlen ? a_in.cu[b] : 0;
     const KArgs a = seq_args(a_in, b);
     const ColTilePlan plan = col_tile_plan(a_in, a, ct, BN, BM, varlen, nseg);
     if (!plan.active) {
@@ -554,13 +552,13 @@ void walk_dkv_flat(const KArgs& a_in) {
   if (RW > 1 && nseg > 1) fail("dkv_flat_kernel: row waves and segments");
   const uint32_t stat_byte = NST * 2 * BM * HD * 2;
   const bool varlen = a_in.cu != nullptr;
-  const int BHk = a_in.B * a_in.Hkv;
   const int64_t nblk = dkv_flat_blocks(a_in, BN) * nseg;
   typedef AsyncTileLoader<HD, BM, 256> Loader;
   for (int64_t block = 0; block < nblk; block++) {
-    const int bh = (int)(block % BHk), ct = (int)(block / BHk);
-    int b = bh / a_in.Hkv;
-    const int hkv = bh % a_in.Hkv, first = varlen ? a_in.cu[b] : 0;
+    const ColPlace place = varlen ? col_place<true>(a_in, (int)block, BN, nseg) : col_place<false>(a_in, (int)block, BN, nseg);
+    if (varlen && !place.active) continue;
+    int b = place.b;
+    const int ct = place.ct, hkv = place.hkv, first = varlen ? a_in.cu[b] : 0;
     const KArgs a = seq_args(a_in, b);
     const ColTilePlan plan = col_tile_plan(a_in, a, ct, BN, BM, varlen, nseg);
     if (!plan.active) {
@@ -765,7 +763,8 @@ void walk_zero_unfilled(const KArgs& a) {
 
 // depth columns outside chunk-visible mode: one column per HD/8 lanes
 template <int HD>
-void walk_depth_cols(const KArgs& a_in) {
+void walk_depth_cols(const KArgs& launch) {
+  const KArgs a_in = packed_as_one(launch);
   constexpr int LPC = HD / 8, CPW = 64 / LPC, CPB = 4 * CPW;
   const int BHk = a_in.B * a_in.Hkv;
   const int64_t nx = (((int64_t)a_in.T * a_in.L + CPB - 1) / CPB) * BHk;
@@ -813,7 +812,8 @@ void walk_depth_cols(const KArgs& a_in) {
 
 // the same organised by token (query groups of up to four rows with the depth scores handed over by the dQ kernel)
 template <int HD>
-void walk_depth_tokens(const KArgs& a_in) {
+void walk_depth_tokens(const KArgs& launch) {
+  const KArgs a_in = packed_as_one(launch);
   constexpr int LPT = HD / 8, TPW = 64 / LPT, TPB = 4 * TPW;
   const int BHk = a_in.B * a_in.Hkv;
   const int64_t nt = (((int64_t)a_in.T + TPB - 1) / TPB) * BHk;

@@ -121,6 +121,17 @@ def test_the_packed_wide_case_that_faulted_stays_inside_its_tensors(walker):
         assert rc == 1 and "VIOLATION" in out, (name, out)
 
 
+@pytest.mark.parametrize("n", [64, 65, 256, 257])
+@pytest.mark.parametrize("shape", [(1, 64, 2, 2, "causal", 0), (2, 128, 2, 1, "noncausal", 0), (1, 96, 2, 4, "chunk_visible", 40)],
+                         ids=lambda s: f"{s[4]}-D{s[1]}")
+def test_packed_batches_of_many_sequences(walker, shape, n):
+    """Every tile of every sequence has one workgroup, in the list of all tiles and (above 256 sequences) in the grid of
+    the longest one."""
+    H, D, L, G, mode, cb = shape
+    rc, out = run(walker, [i * 37 % 50 + (300 if i == 40 else 0) for i in range(n)], H, D, L, G, mode, cb, split=-1)
+    assert rc == 0 and "OK checked" in out, out
+
+
 @pytest.mark.parametrize("case", PACKED, ids=lambda c: f"{c[5]}-{'_'.join(map(str, c[0]))}-D{c[2]}")
 def test_packed_batches(walker, case):
     lengths, H, D, L, G, mode, cb = case

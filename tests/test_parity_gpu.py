@@ -1208,6 +1208,20 @@ def test_small_packed_batches_of_long_sequences_equal_separate_calls_bitwise(gpu
             assert torch.equal(x.grad[:, a * mult[n]:b * mult[n]], one["d" + n]), (a, b, n)
 
 
+@pytest.mark.parametrize("case", [
+    # sequences, H, D, L, G, mode, chunk: a wave holds the tile counts of 64 sequences a register, four registers of them;
+    # more sequences are launched in the order of the longest one; the last has depth tiles behind the sequence tiles
+    (64, 1, 128, 2, 2, "causal", 0),
+    (65, 1, 128, 2, 2, "noncausal", 0),
+    (256, 1, 128, 2, 1, "causal", 0),
+    (257, 1, 128, 2, 1, "causal", 0),
+    (66, 1, 96, 2, 4, "chunk_visible", 40),
+], ids=lambda c: f"{c[5]}-{c[0]}-D{c[2]}")
+def test_packed_batches_of_many_sequences_equal_separate_calls_bitwise(gpu_device, case):
+    lengths = tuple(i * 37 % 90 + (700 if i == 40 else 0) for i in range(case[0]))  # empty ones among them, one long
+    test_small_packed_batches_of_long_sequences_equal_separate_calls_bitwise(gpu_device, (lengths,) + case[1:])
+
+
 def test_packed_batch_on_the_narrow_tiles_against_separate_calls(gpu_device):
     """On the 64-wide tiles the separate (short) calls form dk, dv by waves that share their columns, this packed launch by
     whole column tiles or segments of them: everything else is bit-identical, dk and dv agree to the order of their sums."""
