@@ -708,7 +708,7 @@ bool stack_runs_native(int64_t rows, int64_t width, void* stream) {
 // round is well filled (384: 64 x 145 tokens 670 / 845, 4 x 50 452 / 411; 512: 64 x 145 979 / 1036, in fp16 1134 / 1038, 4 x 50
 // 618 / 446, 64 x 257 2084 / 1839).
 bool tail_is_one_launch(int64_t rows, int64_t width, int64_t hidden, int64_t kv) {
-  if ((width != 128 && width != 256 && width != 384 && width != 512) || hidden % 128 != 0 || kv % 16 != 0) return false;
+  if ((width != 128 && width != 256 && width != 384 && width != 512) || hidden % 128 != 0 || hidden >= 1 << 20 || kv % 16 != 0) return false;
   const int64_t last = ((rows + 63) / 64 - 1) % 256 + 1;
   return width <= 256 || last >= (width <= 384 ? 128 : 192);
 }

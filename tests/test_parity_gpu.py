@@ -1857,6 +1857,7 @@ def test_fp32_non_finite_values_stay_with_the_rows_that_see_them(gpu_device, cas
     (1536, 12, 1, 600, 2.0, True, False),
     (1536, 12, 1, 700, 1.0, False, False),
     (1600, 8, 1, 10, 1.0, False, False),
+    (128, 2, 1, 3, 8192.0, True, True),        # hidden width 2^20: past the block tail's range, its pieces take it
 ])
 def test_stack_widths_and_which_of_them_run_as_native_launches(gpu_device, case):
     """The rule by size, and both ways through the blocks against the same blocks in fp32 on the same 16-bit weights: the
