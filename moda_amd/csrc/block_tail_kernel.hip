@@ -58,9 +58,10 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// GELU of a packed pair of 16-bit values.  A bf16 value has 2 x 2688 magnitudes between 2^-17 and 16, outside of which Phi is
-// 0.5 or 0 and 1 to 3e-6 relative: x Phi(x) with Phi from a table in LDS, 8 vector instructions an element where the
-// formula (which fp16 takes) has 22, 6.5 k cycles for 64 rows x 256 features against 2.4 k (the launch 40 -> 32.7 us).
+// GELU of a packed pair of 16-bit values.  A bf16 value has 2 x 2688 magnitudes between 2^-17 and 16, outside of which the
+// formula's result is x / 2 (to 6e-6, which no rounding to 8 bits sees), or 0 and x.  Inside, a table in LDS holds the formula's
+// result, rounded, over x: times x that is the result again to 2^-23, which rounds to itself.  8 vector instructions an element
+// where the formula (which fp16 takes) has 22, 6.5 k cycles for 64 rows x 256 features against 2.4 k (the launch 40 -> 32.7 us).
 constexpr int kGeluHalf = 21 * 128, kGeluTable = 2 * kGeluHalf, kGeluFirst = (127 - 17) << 7;
 template <typename T>
 constexpr int table_bytes() {
@@ -84,18 +85,30 @@ __device__ __forceinline__ int activated(int w, MODA_LDS const char* table) {
   }
 }
 
-// sum over the TPR neighbouring lanes (8 or 16) of a row
-template <int TPR>
-__device__ __forceinline__ float lane_group_sum(float v) {
-  static_assert(TPR == 8 || TPR == 16, "half or whole rows of sixteen lanes");
+// Sum of a row over the TPR neighbouring lanes (8 or 16) that share it; s[j] is what this lane has of the row's piece
+// lsub + TPR j.  Added as layer_norm_kernel adds them, the two halves of the pieces first (past the last piece: zero).
+template <int TPR, int NL>
+__device__ __forceinline__ float row_sum(const float (&s)[NL]) {
+  static_assert((TPR == 8 || TPR == 16) && NL <= 8, "half or whole rows of sixteen lanes");
+  constexpr int P = NL > 4 ? 8 : NL > 2 ? 4 : NL;
+  float t[P], v = 0.f;
+#pragma unroll
+  for (int j = 0; j < P; j++) t[j] = j < NL ? s[j] : 0.f;
+#pragma unroll
+  for (int h = P / 2; h > 0; h >>= 1)
+#pragma unroll
+    for (int j = 0; j < h; j++) t[j] += t[j + h];
+  v = t[0];
 #if defined(__HIP_DEVICE_COMPILE__)
   auto add = [&](auto ctrl) {
     v += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), decltype(ctrl)::value, 0xf, 0xf, true));
   };
-  add(std::integral_constant<int, 0xB1>{});   // quad_perm 1, 0, 3, 2
-  add(std::integral_constant<int, 0x4E>{});   // quad_perm 2, 3, 0, 1
-  add(std::integral_constant<int, 0x141>{});  // row_half_mirror
-  if (TPR == 16) add(std::integral_constant<int, 0x140>{});  // row_mirror
+  if (TPR == 16) add(std::integral_constant<int, 0x128>{});  // row_ror 8: the lane 8 away
+  const int own = __builtin_bit_cast(int, v);  // the lane 4 away: row_shl 4 for banks 0 and 2, row_shr 4 for 1 and 3
+  const int up = __builtin_amdgcn_update_dpp(0, own, 0x104, 0xf, 0x5, false);
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(up, own, 0x114, 0xf, 0xa, false));
+  add(std::integral_constant<int, 0x4E>{});  // quad_perm 2, 3, 0, 1
+  add(std::integral_constant<int, 0xB1>{});  // quad_perm 1, 0, 3, 2
 #endif
   return v;
 }
@@ -283,14 +296,15 @@ __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
       for (int i = 0; i < 4; i++) unpack2<T>(v[i], f[2 * i], f[2 * i + 1]);
     };
     lds_barrier();
-    float f[NL][8], s = 0.f;
+    float f[NL][8], s[NL];
     i32x4 raw[NL];
 #pragma unroll
     for (int j = 0; j < NL; j++) {
       raw[j] = *reinterpret_cast<MODA_LDS const i32x4*>(X + Rows<C>::off(lrow, lsub + TPR * j));
       load8(raw[j], f[j]);
+      s[j] = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; i++) s += f[j][i];
+      for (int i = 0; i < 8; i++) s[j] += f[j][i];
     }
     const bool store = out && r0 + lrow < a.rows;
     if (!POST && store) {
@@ -298,16 +312,17 @@ __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
       for (int j = 0; j < NL; j++) *reinterpret_cast<i32x4*>(out + (int64_t)(r0 + lrow) * C + (lsub + TPR * j) * 8) = raw[j];
     }
     if (normalise) {
-      const float mean = lane_group_sum<TPR>(s) / C;
-      float v = 0.f;
+      const float mean = row_sum<TPR>(s) / C;
 #pragma unroll
-      for (int j = 0; j < NL; j++)
+      for (int j = 0; j < NL; j++) {
+        s[j] = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
           const float d = f[j][i] - mean;
-          v = __builtin_fmaf(d, d, v);
+          s[j] = __builtin_fmaf(d, d, s[j]);
         }
-      const float rstd = rsqrtf(lane_group_sum<TPR>(v) / C + eps);
+      }
+      const float rstd = rsqrtf(row_sum<TPR>(s) / C + eps);
 #pragma unroll
       for (int j = 0; j < NL; j++) {
         float w[8], b[8];
@@ -360,23 +375,23 @@ __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
   for (int c0 = 0; c0 < a.hidden; c0 += HC) {
     if (has_features(c0)) {
       f32x4 hid[MB1][NB];
+      zero(hid);
+      fc1.template run<C>(X, xbase, C / 32, hid);
 #pragma unroll
-      for (int mb = 0; mb < MB1; mb++) {  // sums start from the bias
+      for (int mb = 0; mb < MB1; mb++) {
         float b[4];
         unpack4(bias1[mb], b);
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) hid[mb][nb] = f32x4{b[0], b[1], b[2], b[3]};
-      }
-      fc1.template run<C>(X, xbase, C / 32, hid);
-#pragma unroll
-      for (int mb = 0; mb < MB1; mb++)
-#pragma unroll
         for (int nb = 0; nb < NB; nb++) {
-          i32x2 w;  // the linear layer's own result is a 16-bit value, as it is when the layers run one by one
-          w[0] = activated<T>(pack2<T>(hid[mb][nb][0], hid[mb][nb][1]), table);
-          w[1] = activated<T>(pack2<T>(hid[mb][nb][2], hid[mb][nb][3]), table);
+          float x[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++) x[i] = hid[mb][nb][i] + b[i];
+          i32x2 w = pack4(x);  // the linear layer's own result is a 16-bit value, as it is when the layers run one by one
+          w[0] = activated<T>(w[0], table);
+          w[1] = activated<T>(w[1], table);
           *reinterpret_cast<MODA_LDS i32x2*>(Hs + Rows<HC>::off(sigma, wave * 2 * MB1 + 2 * mb + (q4 >> 1)) + 4 * (q4 & 1) + 16 * nb * HC) = w;
         }
+      }
     }
 #pragma unroll
     for (int mb = 0; mb < MB2; mb++) fc2.base[mb] = a.fc2_w + (size_t)(f2 + 16 * mb) * a.hidden + c0 * 16;
@@ -453,7 +468,7 @@ __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
 // the sum, per step the 1 KB of a wave's A operand, lane by lane.  In their own order a wave's load touches sixteen rows in each
 // quarter of its lanes, sixteen cache lines where packed it touches two, and a compute unit takes in 13 bytes a cycle instead
 // of 64 (12 608 rows, width 256: 61 us, packed 42 at the time).  Twelve blocks are packed in one launch of 7 us.
-// The last row of workgroups fills the GELU table: Phi of the bf16 values from 2^-17 to 16, then of their negatives.
+// The last row of workgroups fills the GELU table (see activated): bf16 values from 2^-17 to 16, then their negatives.
 constexpr int kPackMatrices = 96;
 struct PackArgs {
   int n;
@@ -467,9 +482,11 @@ struct PackArgs {
 __global__ __launch_bounds__(256) void pack_weights_kernel(const PackArgs a) {
   if ((int)blockIdx.y == a.n) {
     for (int i = blockIdx.x * 256 + threadIdx.x; i < kGeluTable; i += gridDim.x * 256) {
-      const unsigned bits = (unsigned)(kGeluFirst + i % kGeluHalf) << 16;
-      const double x = __builtin_bit_cast(float, bits) * (i < kGeluHalf ? 1.0 : -1.0);
-      a.gelu_table[i] = (float)(0.5 * erfc(-x * 0.70710678118654752440));
+      const int bits = (kGeluFirst + i % kGeluHalf) | (i < kGeluHalf ? 0 : 0x8000);
+      float x, y, none;
+      unpack2<BF16>(bits, x, none);
+      unpack2<BF16>(pack2<BF16>(gelu(x), 0.f), y, none);
+      a.gelu_table[i] = y / x;
     }
     return;
   }

@@ -2109,6 +2109,56 @@ def test_block_tail_against_fp64(gpu_device, case, post_norm, dtype):
         assert (got[rows:] == 7.0).all() and (got[:, n:] == 7.0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("post_norm", [False, True])
+@pytest.mark.parametrize("case", [
+    # rows, width, hidden, features of each part: every width with 32 rows a workgroup and with 64
+    (77, 128, 256, (128, 16, 16)),
+    (8195, 128, 384, (128,)),
+    (45, 256, 640, (256, 64, 64)),
+    (8251, 256, 1024, (256, 128, 128)),
+    (33, 384, 1536, (384, 64)),
+    (8200, 384, 128, (384, 16)),
+    (70, 512, 2048, (512, 64, 64)),
+    (8193, 512, 256, (512, 128, 128)),
+], ids=str)
+def test_block_tail_equals_its_pieces_bitwise(gpu_device, case, post_norm, dtype):
+    """A stack takes the one launch or the pieces by its size: the outputs are the same bits, since every sum adds the same
+    numbers in the same order and every rounding falls in the same place."""
+    import ctypes
+
+    from moda_amd import _lib
+
+    rows, width, hidden, parts = case
+    say(f"CASE block tail bitwise {case} post_norm={post_norm} {dtype}")
+    t = _BlockTail(width, hidden, parts, dtype, gpu_device, seed=rows)
+    gen = torch.Generator(device=gpu_device).manual_seed(rows + 1)
+    h, res = (torch.randn(rows, width, generator=gen, device=gpu_device).to(dtype) for _ in range(2))
+    x, ys = t.run(h, res, post_norm)
+    i64, ptr = ctypes.c_int64, lambda v: ctypes.c_void_p(v.data_ptr())
+
+    def lin(v, w, b, residual=None, gelu=False):
+        y = torch.empty(rows, w.shape[0], dtype=dtype, device=gpu_device)
+        assert _linear(v, [(w, b, y)], residual, gelu) == 0
+        return y
+
+    def norm(v, name):
+        y = torch.empty_like(v)
+        assert _lib.load().moda_hip_layer_norm({torch.bfloat16: 0, torch.float16: 1}[dtype], i64(rows), i64(width), ptr(v), ptr(t.w[name + "_w"]),
+                                               ptr(t.w[name + "_b"]), ctypes.c_float(1e-6), ptr(y),
+                                               ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        return y
+
+    y = lin(h, t.w["proj_w"], t.w["proj_b"], res)
+    z = norm(y, "mid")
+    y = z if post_norm else y
+    y = lin(lin(z, t.w["fc1_w"], t.w["fc1_b"], gelu=True), t.w["fc2_w"], t.w["fc2_b"], y)
+    z = norm(y, "end")
+    assert torch.equal(x, z if post_norm else y), (x != (z if post_norm else y)).float().mean()
+    for (w, b), got in zip(t.parts, ys):
+        assert torch.equal(got[:rows, :w.shape[0]], lin(z, w, b))
+
+
 def test_block_tail_gelu_of_every_bf16_value(gpu_device):
     """The table route of the GELU, value by value: zero rows, the values as the first layer's bias, an identity behind it.
     One rounding beside the table's own ends: u |y| and 2^-17 relative, and fp32's subnormals."""
@@ -2125,6 +2175,26 @@ def test_block_tail_gelu_of_every_bf16_value(gpu_device):
     want = 0.5 * v * torch.special.erfc(v * -0.5 ** 0.5)
     err = (torch.cat(got).double() - want).abs()
     assert (err <= (2.0 ** -8 + 8e-6) * want.abs() + 2.0 ** -126).all(), (err / want.abs()).max()
+
+
+def test_block_tail_gelu_is_the_linear_layers_bitwise(gpu_device):
+    """The table holds the formula's results: every bf16 value gives the bits that moda_hip_linear's GELU gives, infinities and
+    NaN (one at a time, since an identity of infinities is NaN beside them) included.  Where the result is a subnormal, x / 2
+    can lie half way between two of them, and an odd one of the formula's 2^-23 decides: one step of 2^-133 there."""
+    eye, zero = torch.eye(128, device=gpu_device), torch.zeros(128, device=gpu_device)
+    t = _BlockTail(128, 128, (), torch.bfloat16, gpu_device, mid_w=zero, mid_b=zero, fc2_w=eye, fc2_b=zero, proj_b=zero)
+    row, x, w = (torch.zeros(*s, device=gpu_device, dtype=torch.bfloat16) for s in ((1, 128), (1, 64), (128, 64)))
+    bits = torch.arange(-32768, 32768, device=gpu_device).to(torch.int16)
+    finite = bits[bits.view(torch.bfloat16).isfinite()]
+    some = torch.tensor([0x7f80, -0x80, 0x7fc0, -0x40, 0x7f81, -1], device=gpu_device).to(torch.int16)
+    for chunk in (*finite.split(128), *some.split(1)):
+        v = torch.nn.functional.pad(chunk.view(torch.bfloat16), (0, 128 - chunk.numel()))
+        t.w["fc1_b"] = v
+        got, want = t.run(row, row, False)[0][0, :chunk.numel()], torch.empty_like(row)
+        assert _linear(x, [(w, v, want)], gelu=True) == 0
+        want, small = want[0, :chunk.numel()], chunk.view(torch.bfloat16).abs() < 2.0 ** -125
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[~small].nan_to_num(7.0), want[~small].nan_to_num(7.0)), chunk
+        assert ((got - want).double()[small].abs() <= 2.0 ** -133).all(), chunk
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
