@@ -513,7 +513,7 @@ hipError_t launch_tail_t(const TailArgs& a, hipStream_t stream) {
 
 template <typename T, int C>
 hipError_t launch_tail_c(const TailArgs& a, bool post, int cus, hipStream_t stream) {
-  if (a.rows <= 32 * cus) return post ? launch_tail_t<T, C, 2, true>(a, stream) : launch_tail_t<T, C, 2, false>(a, stream);
+  if (block_tail_rows(a.rows, cus) == 32) return post ? launch_tail_t<T, C, 2, true>(a, stream) : launch_tail_t<T, C, 2, false>(a, stream);
   return post ? launch_tail_t<T, C, 4, true>(a, stream) : launch_tail_t<T, C, 4, false>(a, stream);
 }
 

@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "../../include/moda_hip.h"
+#include "tuning.h"
 
 namespace py = pybind11;
 using at::Tensor;
@@ -700,17 +701,12 @@ bool stack_runs_native(int64_t rows, int64_t width, void* stream) {
   return hipStreamIsCapturing((hipStream_t)stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
 }
 
-// Whether a block's dense part runs as one launch (moda_hip_block_tail) or as its pieces.  Eight blocks, 64 x 197 tokens,
-// one launch / pieces: width 128 268 / 455 us, 256 407 / 660, 384 735 / 1005, 512 1110 / 1284.  A workgroup takes 64 rows through
-// all of a block's weights (32 where that still fits one round), so few rows cost what a full round of 256 workgroups
-// does, and a round that is mostly empty as much as a full one: up to width 256 that is still the faster way (4 x 50 tokens
-// 187 / 272 and 272 / 335; 64 x 257, one workgroup too many for a round, 388 / 519 and 683 / 838), above only when the last
-// round is well filled (384: 64 x 145 tokens 670 / 845, 4 x 50 452 / 411; 512: 64 x 145 979 / 1036, in fp16 1134 / 1038, 4 x 50
-// 618 / 446, 64 x 257 2084 / 1839).
-bool tail_is_one_launch(int64_t rows, int64_t width, int64_t hidden, int64_t kv) {
+// Whether a block's dense part runs as one launch (moda_hip_block_tail): the kernel's range, and where it is the faster way.
+bool tail_is_one_launch(bool fp16, int64_t rows, int64_t width, int64_t hidden, int64_t kv, int device) {
   if ((width != 128 && width != 256 && width != 384 && width != 512) || hidden % 128 != 0 || hidden >= 1 << 20 || kv % 16 != 0) return false;
-  const int64_t last = ((rows + 63) / 64 - 1) % 256 + 1;
-  return width <= 256 || last >= (width <= 384 ? 128 : 192);
+  int compute_units = 0;
+  return hipDeviceGetAttribute(&compute_units, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && compute_units > 0 &&
+         moda::block_tail_pays(fp16, rows, width, hidden, kv, compute_units);
 }
 
 // Forward pass of all blocks of one stack, launches only: the residual stream, one depth cache and four work tensors
@@ -748,7 +744,7 @@ std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>
   const auto opt = x_in.options().requires_grad(false);
   const Tensor x0 = x_in.contiguous();
   if ((uintptr_t)x0.const_data_ptr() % 16 != 0) return {};
-  const bool tails = tail_is_one_launch(M, C, hidden, kv);
+  const bool tails = tail_is_one_launch(type == at::kHalf, M, C, hidden, kv, x_in.get_device());
   Tensor x = at::empty({B, N, C}, opt), h = at::empty({M, C}, opt), q = at::empty({M, C}, opt), x1 = tails ? Tensor() : at::empty({M, C}, opt),
          hid = tails ? Tensor() : at::empty({M, hidden}, opt), ck = at::empty({B, N * L, kv}, opt), cv = at::empty({B, N * L, kv}, opt),
          lse = at::empty({M * heads}, opt.dtype(at::kFloat));

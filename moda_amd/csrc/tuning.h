@@ -1,4 +1,4 @@
-// Compile-time launch shapes of the streaming (query-row) kernels: forward and dQ.
+// Compile-time launch shapes of the streaming (query-row) kernels: forward and dQ; rules of the dense ones.
 #pragma once
 
 namespace moda {
@@ -89,6 +89,32 @@ inline LinearTile pick_linear_tile(long long rows, long long K, const int* featu
   if (tall >= 2 * cus) return LinearTile::k128x64;
   if (tall > cus && K >= 512) return LinearTile::k128x64ThreeStages;
   return LinearTile::k64x64;
+}
+
+// Host side, a transformer block's dense part as one launch (block_tail_kernel) or as its pieces (linear and layer-norm
+// launches): rows of a workgroup of the one launch ...
+inline int block_tail_rows(long long rows, int compute_units) { return rows <= 32ll * compute_units ? 32 : 64; }
+// ... and whether it is the faster way.  Measured as the time of stacks of four blocks, both ways, at widths 128, 256, 384
+// and 512, MLPs of once to 64 times the width, 16 to 25 216 rows, both types, and as the time of 218 others of one to eight
+// blocks: the rule takes the slower way nowhere by more than 3 % (1 us of 38, a single block).
+// A workgroup takes its rows through all of the block's weights, which one compute unit takes in at 64 bytes a cycle, however
+// few the rows are.  The pieces spread the weights over the compute units, but are seven launches, and their time grows with
+// the rows.  While 32 rows each are one round, the one launch costs, in us a block and against the pieces, 16 for a million
+// weights; it saves 9 of launches, 3 for 256 features of width, the hidden activations' way through memory (less in fp16, whose
+// GELU is the longer one), and for 1000 rows 1 and 2.2 for a million weights.  Width 256, MLP of 1024, 200 rows: 45 us a block,
+// pieces 64; MLP of 16 384: 235 and 157, at 4 640 rows 236 and 255.  Width 512, MLP of 2048, 200 rows: 76 and 54, 8 128 rows: 86
+// and 107.
+// With 64 rows a round that is mostly empty costs as much as a full one.  Up to width 256 that is still less than the pieces
+// (16 448 rows, a workgroup more than a round: 80 and 94); 384 has to fill half of it (16 448 rows: 161 and 151, 25 216: 174
+// and 216), and so has 512 in bf16 (18 912: 247 and 229, 25 216: 261 and 307).  512 in fp16 spills most registers: three
+// quarters (9 280 rows: 140 and 127, 12 608: 154 and 160).
+inline bool block_tail_pays(bool fp16, long long rows, long long width, long long hidden, long long kv_width, int compute_units) {
+  if (block_tail_rows(rows, compute_units) == 32) {
+    const double weights = 2e-6 * (double)width * (double)(width + kv_width + hidden), k = 0.256 * (double)rows / compute_units;
+    return weights * (16 - 2.2 * k) < 9 + 3 * (width / 256.) + k + (fp16 ? 0.8 : 2.7) * (hidden / 1000.);
+  }
+  const long long last = ((rows + 63) / 64 - 1) % compute_units + 1;  // workgroups of the last round
+  return width <= 256 || 4 * last >= (width > 384 && fp16 ? 3 : 2) * compute_units;
 }
 
 }  // namespace moda

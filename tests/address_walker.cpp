@@ -1269,6 +1269,11 @@ void walk_all(const Case& c, const KArgs& a) {
 int main(int argc, char** argv) {
   const auto arg = [&](int i) { return i < argc ? atoi(argv[i]) : 0; };
   const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "tail_rule") {  // dtype rows width hidden kv compute_units
+    printf("%s, %d rows\n", block_tail_pays(std::string(argv[2]) == "fp16", arg(3), arg(4), arg(5), arg(6), arg(7)) ? "one launch" : "pieces",
+           block_tail_rows(arg(3), arg(7)));
+    return 0;
+  }
   if (what == "linear" || what == "norm" || what == "slot") {
     std::vector<int> parts;
     for (int i = 5; i < argc; i++) parts.push_back(arg(i));

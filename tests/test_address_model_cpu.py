@@ -273,3 +273,36 @@ def test_dense_and_slot_kernels(walker, case):
         r = subprocess.run([walker, *map(str, args)], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, env=e, timeout=600)
         out = r.stdout + r.stderr
         assert r.returncode == want and out.startswith(chosen) and ("VIOLATION" if want else "OK checked") in out, out
+
+
+@pytest.mark.parametrize("case", [
+    # dtype, rows, width, MLP, K/V width, compute units, what has to be chosen: points on both sides of the rule that measured
+    # at least 5 % apart (256 compute units), times of a block in one launch / in pieces
+    ("bf16", 200, 256, 1024, 64, 256, "one launch, 32 rows"),      # 45 / 64 us
+    ("bf16", 16, 256, 4096, 64, 256, "pieces, 32 rows"),           # 67 / 56
+    ("bf16", 2320, 256, 4096, 64, 256, "one launch, 32 rows"),     # 74 / 80
+    ("fp16", 580, 256, 4096, 64, 256, "pieces, 32 rows"),          # 82 / 68
+    ("bf16", 1160, 256, 16384, 64, 256, "pieces, 32 rows"),        # 230 / 182
+    ("bf16", 200, 128, 8192, 64, 256, "pieces, 32 rows"),          # 100 / 85
+    ("fp16", 1160, 128, 8192, 64, 256, "pieces, 32 rows"),         # 115 / 107
+    ("fp16", 4728, 128, 2048, 64, 256, "one launch, 32 rows"),
+    ("bf16", 8128, 384, 1536, 192, 256, "one launch, 32 rows"),    # 63 / 87
+    ("fp16", 200, 384, 384, 192, 256, "one launch, 32 rows"),      # 36 / 39
+    ("bf16", 200, 384, 1536, 192, 256, "pieces, 32 rows"),         # 55 / 48
+    ("fp16", 8128, 384, 6144, 192, 256, "one launch, 32 rows"),    # 151 / 196
+    ("bf16", 8128, 512, 2048, 128, 256, "one launch, 32 rows"),    # 86 / 107
+    ("fp16", 16, 512, 512, 128, 256, "pieces, 32 rows"),           # 41 / 37
+    ("fp16", 8128, 512, 512, 128, 256, "one launch, 32 rows"),     # 55 / 73
+    ("bf16", 16448, 256, 1024, 64, 256, "one launch, 64 rows"),    # 80 / 94
+    ("bf16", 16448, 384, 1536, 192, 256, "pieces, 64 rows"),       # 161 / 151
+    ("fp16", 9280, 384, 1536, 192, 256, "one launch, 64 rows"),    # 90 / 101
+    ("bf16", 9280, 512, 2048, 128, 256, "one launch, 64 rows"),    # 121 / 126
+    ("fp16", 9280, 512, 512, 128, 256, "pieces, 64 rows"),         # 95 / 85
+    ("fp16", 12608, 512, 2048, 128, 256, "one launch, 64 rows"),   # 154 / 160
+    # a partition with fewer compute units: a round holds fewer rows
+    ("bf16", 2048, 384, 1536, 192, 64, "one launch, 32 rows"),
+    ("bf16", 4097, 384, 1536, 192, 64, "pieces, 64 rows"),
+], ids=lambda c: "-".join(map(str, c[:4])))
+def test_a_blocks_dense_part_takes_the_faster_way(walker, case):
+    out = subprocess.run([walker, "tail_rule", *map(str, case[:-1])], stdout=subprocess.PIPE, text=True, check=True).stdout
+    assert out.strip() == case[-1]
