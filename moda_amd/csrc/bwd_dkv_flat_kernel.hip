@@ -9,7 +9,7 @@ hipError_t launch_dkv_flat_t(const KArgs& a, hipStream_t stream) {
   static LdsAttrState attr;
   const hipError_t ea = allow_dynamic_lds(attr, reinterpret_cast<const void*>(&dkv_flat_kernel<T, HD, VARLEN, SPLIT, RW>), smem);
   if (ea != hipSuccess) return ea;
-  const int64_t nblk = dkv_flat_blocks(a, 128 / RW) * (SPLIT ? a.dkv_split : 1);
+  const int64_t nblk = dkv_flat_blocks(a, 128 / RW, SPLIT ? a.dkv_split : 1);
   if (nblk == 0) return hipSuccess;
   if (nblk >= (1ll << 31)) return hipErrorInvalidValue;
   hipLaunchKernelGGL((dkv_flat_kernel<T, HD, VARLEN, SPLIT, RW>), dim3((unsigned)nblk), dim3(256), smem, stream, a);

@@ -41,11 +41,20 @@ MODA_HD int query_tile_of(int block, int BH, int BM, int Tq_grid) { return (Tq_g
 // sequence's tiles stayed on as many XCDs as it has heads.  Training steps: 16 sequences of 113 - 7441 tokens, two heads of
 // four, head dim 64: 3480 -> 737 us; twelve of 338 - 7523, four heads of two: 1296 -> 666; 8192 + 3 x 64 tokens, two heads of
 // two, head dim 128: 1139 -> 766; 16 384 to 2048 tokens, 15 sequences, four heads of four: 10.14 -> 9.84 ms; 200 of 300 each:
-// 1710 -> 1671 us.  Where all workgroups run at once it can go the other way, by which of them share a compute unit (five
-// sequences of 226 - 6188, two heads of two, head dim 64: 356 -> 364).
-// Up to kPackedOrderMax sequences, whose tile counts a wave holds in four registers; more keep that grid.
-constexpr int kPackedOrderMax = 256;
-MODA_HD bool packed_order(const KArgs& a) { return a.cu != nullptr && a.B <= kPackedOrderMax; }
+// 1710 -> 1671 us.
+// Two kinds of launches keep that grid.  Those of up to kPackedOrderGrid workgroups in it, where every workgroup has a compute
+// unit to itself wherever it falls: a place in the list costs a launch 0.4 us (forward of 8 x 14 - 262 tokens, four heads of
+// two, head dim 64: 9.4 us in the list, 9.0 in the grid; two of up to 147, eight heads of four: 8.2 and 7.8).  Above, the list's
+// order is worth more than that (5909 + 433 tokens, four heads, a grid of 376: 108 -> 78).  And those of more than
+// kPackedOrderMax sequences, whose tile counts a wave holds in four registers (one up to 64: 0.3 us less).
+// What is left of the list's price: launches whose workgroups all run at once, two or three a compute unit, end by which of
+// them share one (226, 1800, 6188, 900, 3300 tokens, two heads of two, head dim 64, causal: 268 -> 271 us a step, not causal with
+// four slots 426 -> 413; 12 of 1332 and fewer, four heads: 91 -> 93).
+constexpr int kPackedOrderMax = 256, kPackedOrderGrid = 256;
+// workgroups of the grid of the longest sequence for every one
+MODA_HD int64_t longest_row_grid(const KArgs& a, int BM) { return (int64_t)((a.Tq + BM - 1) / BM) * a.B * a.Hq; }
+MODA_HD int64_t longest_col_grid(const KArgs& a, int BN, int nseg) { return a.has_seq ? (int64_t)((a.T + BN - 1) / BN) * nseg * a.B * a.Hkv : 0; }
+MODA_HD bool packed_order(const KArgs& a, int64_t grid) { return a.cu != nullptr && a.B <= kPackedOrderMax && grid > kPackedOrderGrid; }
 // length of the list, at most: every sequence has one tile that is not full (rows_per_token: query rows, or 1 for keys)
 MODA_HD int64_t packed_ranks(const KArgs& a, int rows_per_token, int BM) {
   const int64_t grid = (int64_t)(((int64_t)a.T * rows_per_token + BM - 1) / BM) * a.B;
@@ -57,10 +66,10 @@ struct PackedTile {
   int t0, T;    // the sequence's first token and length
   bool active;  // false: past the end of the list
 };
-MODA_HD PackedTile packed_tile(const KArgs& a, int rows_per_token, int BM, int rank) {
+template <int P>  // sequences: up to 64 P
+MODA_HD PackedTile packed_tile_of(const KArgs& a, int rows_per_token, int BM, int rank) {
   PackedTile p = {0, 0, 0, 0, false};
 #if defined(__HIP_DEVICE_COMPILE__)
-  constexpr int P = kPackedOrderMax / 64;
   const int lane = threadIdx.x & 63;
   int tiles[P], t0[P], T[P];
 #pragma unroll
@@ -132,6 +141,9 @@ MODA_HD PackedTile packed_tile(const KArgs& a, int rows_per_token, int BM, int r
 #endif
   return p;
 }
+MODA_HD PackedTile packed_tile(const KArgs& a, int rows_per_token, int BM, int rank) {
+  return a.B <= 64 ? packed_tile_of<1>(a, rows_per_token, BM, rank) : packed_tile_of<kPackedOrderMax / 64>(a, rows_per_token, BM, rank);
+}
 
 // Which (batch entry, query head, query tile) a workgroup of the forward or dQ kernel takes.
 struct RowPlace {
@@ -141,7 +153,7 @@ struct RowPlace {
 };
 template <bool VARLEN>
 MODA_HD RowPlace row_place(const KArgs& grid, int block, int BM) {
-  if (VARLEN && packed_order(grid)) {
+  if (VARLEN && packed_order(grid, longest_row_grid(grid, BM))) {
     const PackedTile p = packed_tile(grid, grid.Gf, BM, block / grid.Hq);
     return {p.seq, block % grid.Hq, p.level, p.t0, p.T, p.active};
   }
@@ -304,6 +316,11 @@ MODA_HD ColTilePlan col_tile_plan(const KArgs& grid, const KArgs& a, int ct, int
 
 // Which (batch entry, kv head, column-tile workgroup `ct` of it) a workgroup of the dK/dV kernels takes.  A batch in packed
 // order has the sequence tiles of all its sequences first, then the depth tiles as every other launch has them.
+// Row segments: the last one of every tile first, then the one before it, so that the long tiles, which alone have many,
+// still lead, and the places of segments that a tile does without lie together.  Side by side, as the other launches have
+// them, those places repeat with a period that compute units and XCDs share: the fullest XCD had 1.34 - 1.45 of the mean work
+// (here 1.02).  dK/dV stage, causal, head dim 64, the longest sequence's grid / side by side / here: 2667 and two shorter
+// sequences, eight heads 73 / 82 / 64 us; 3825 and two, one head of four 96 / 108 / 74; 1497 and four, two heads of four 56 / 64 / 57.
 struct ColPlace {
   int b, hkv, ct;
   int t0, T;
@@ -313,14 +330,14 @@ template <bool VARLEN>
 MODA_HD ColPlace col_place(const KArgs& grid, int block, int BN, int nseg) {
   const int BHk = grid.B * grid.Hkv;
   int ct0 = 0;
-  if (VARLEN && packed_order(grid)) {
+  if (VARLEN && packed_order(grid, longest_col_grid(grid, BN, nseg))) {
     const int n_seq_tiles = grid.has_seq ? (grid.T + BN - 1) / BN : 0;
-    const int seq_blocks = grid.has_seq ? (int)packed_ranks(grid, 1, BN) * nseg * grid.Hkv : 0;
+    const int ranks = grid.has_seq ? (int)packed_ranks(grid, 1, BN) : 0, seq_blocks = ranks * nseg * grid.Hkv;
     if (block < seq_blocks) {
-      const int seg = block / grid.Hkv;  // of all ranks
-      const PackedTile p = packed_tile(grid, 1, BN, seg / nseg);
+      const int place = block / grid.Hkv, seg = nseg - 1 - place / ranks;
+      const PackedTile p = packed_tile(grid, 1, BN, place % ranks);
       const int tile = grid.causal ? n_seq_tiles - 1 - p.level : p.level;  // as col_tile_plan counts them
-      return {p.seq, block % grid.Hkv, tile * nseg + seg % nseg, p.t0, p.T, p.active};
+      return {p.seq, block % grid.Hkv, tile * nseg + seg, p.t0, p.T, p.active};
     }
     block -= seq_blocks;
     ct0 = n_seq_tiles * nseg;
@@ -345,23 +362,24 @@ inline int64_t linear_blocks(int m_tiles, int n_tiles) { return 8ll * ((m_tiles 
 // Launch grids (host side), one place for the launchers and the walker.
 // ---------------------------------------------------------------------------------------------------
 inline int64_t row_kernel_blocks(const KArgs& a, int rows_per_block) {
-  if (packed_order(a)) return packed_ranks(a, a.Gf, rows_per_block) * a.Hq;
-  return (int64_t)((a.Tq + rows_per_block - 1) / rows_per_block) * a.B * a.Hq;
+  const int64_t grid = longest_row_grid(a, rows_per_block);
+  return packed_order(a, grid) ? packed_ranks(a, a.Gf, rows_per_block) * a.Hq : grid;
 }
 // chunk-visible depth columns: by whole chunks when a chunk's rows fit one 64-row query tile (tile widths up to 128:
 // the chunk kernel's registers and LDS do not stretch to 256), else as column tiles of the dK/dV kernel
 inline bool depth_by_chunks(const KArgs& a, int HD) { return HD <= 128 && a.L > 0 && a.chunk && (int64_t)a.Cb * a.Gf <= 64; }
-// sequence column tiles of a launch, all batch entries together
-inline int64_t seq_col_tiles(const KArgs& a, int BN) {
-  return !a.has_seq ? 0 : packed_order(a) ? packed_ranks(a, 1, BN) : (int64_t)((a.T + BN - 1) / BN) * a.B;
+// workgroups for the sequence column tiles of a launch
+inline int64_t seq_col_blocks(const KArgs& a, int BN, int nseg) {
+  const int64_t grid = longest_col_grid(a, BN, nseg);
+  return packed_order(a, grid) ? packed_ranks(a, 1, BN) * nseg * a.Hkv : grid;
 }
 inline int64_t col_kernel_blocks(const KArgs& a, int HD, int BN, int nseg) {
   const int64_t n_dep_tiles = (a.L > 0 && a.chunk && !depth_by_chunks(a, HD)) ? ((int64_t)a.T * a.Lv + BN - 1) / BN : 0;
-  return (seq_col_tiles(a, BN) * nseg + n_dep_tiles * a.B) * a.Hkv;
+  return seq_col_blocks(a, BN, nseg) + n_dep_tiles * a.B * a.Hkv;
 }
 // Sequence dK/dV on the 64-wide tiles: dkv_flat_kernel (three workgroups per compute unit, where dkv_kernel fits one)
 // takes every launch of sequence-key column tiles whose kv head is the query head.
-inline int64_t dkv_flat_blocks(const KArgs& a, int BN = 128) { return seq_col_tiles(a, BN) * a.Hkv; }
+inline int64_t dkv_flat_blocks(const KArgs& a, int BN = 128, int nseg = 1) { return seq_col_blocks(a, BN, nseg); }
 inline bool takes_dkv_flat(const KArgs& a, int HD) {
   return HD == 64 && a.has_seq && a.hdiv == 1 && col_kernel_blocks(a, HD, 128, 1) == dkv_flat_blocks(a);
 }

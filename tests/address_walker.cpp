@@ -22,10 +22,12 @@
 // usage: address_walker HD D Dv H G L Lv mode(0..4) chunk_tokens row_segments packed B_or_n len0 [len1 ...]
 //   packed = 0: a fixed-length batch of B sequences of len0 tokens; packed = 1: n sequences on one packed axis.
 //   environment: WALKER_FP32=1 walks the fp32 matrix kernels instead; WALKER_OWN_SLOT=1 a backward that leaves the slots
-//   without data alone and adds slot Lv of the depth gradients to dk, dv.
+//   without data alone and adds slot Lv of the depth gradients to dk, dv; WALKER_ORDER=1 prints the order of a packed
+//   batch's launches instead.
 // usage: address_walker linear rows K gelu n0 [n1 n2]   |   norm rows dim   |   slot B T H D L slot wide to_cache
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -216,6 +218,12 @@ KArgs make_args(const Case& c) {
   return a;
 }
 
+// what a place says of its sequence is what the offsets say
+template <typename Place>
+void check_place(const KArgs& a, const Place& p) {
+  if (p.t0 != a.cu[p.b] || p.T != a.cu[p.b + 1] - a.cu[p.b]) fail("place of sequence %d: tokens %d + %d", p.b, p.t0, p.T);
+}
+
 // argument block of the workgroup: rebased on its sequence for a packed batch
 KArgs seq_args(const KArgs& in, int& b) {
   KArgs a = in;
@@ -242,6 +250,7 @@ void walk_row_kernel(const KArgs& a_in, bool dq, int rows_per_wave, bool own_pos
   for (int64_t block = 0; block < nblk; block++) {
     const RowPlace place = varlen ? row_place<true>(a_in, (int)block, BM) : row_place<false>(a_in, (int)block, BM);
     if (varlen && !place.active) continue;
+    if (varlen) check_place(a_in, place);
     int b = place.b;
     const int hq = place.hq, hkv = hq / a_in.hdiv, qt = place.qt;
     const KArgs a = seq_args(a_in, b);
@@ -463,6 +472,7 @@ void walk_dkv(const KArgs& a_in) {
   for (int64_t block = 0; block < nblk; block++) {
     const ColPlace place = varlen ? col_place<true>(a_in, (int)block, BN, nseg) : col_place<false>(a_in, (int)block, BN, nseg);
     if (varlen && !place.active) continue;
+    if (varlen) check_place(a_in, place);
     int b = place.b;
     const int ct = place.ct, hkv = place.hkv, first = varlen ? a_in.cu[b] : 0;
     const KArgs a = seq_args(a_in, b);
@@ -552,11 +562,12 @@ void walk_dkv_flat(const KArgs& a_in) {
   if (RW > 1 && nseg > 1) fail("dkv_flat_kernel: row waves and segments");
   const uint32_t stat_byte = NST * 2 * BM * HD * 2;
   const bool varlen = a_in.cu != nullptr;
-  const int64_t nblk = dkv_flat_blocks(a_in, BN) * nseg;
+  const int64_t nblk = dkv_flat_blocks(a_in, BN, nseg);
   typedef AsyncTileLoader<HD, BM, 256> Loader;
   for (int64_t block = 0; block < nblk; block++) {
     const ColPlace place = varlen ? col_place<true>(a_in, (int)block, BN, nseg) : col_place<false>(a_in, (int)block, BN, nseg);
     if (varlen && !place.active) continue;
+    if (varlen) check_place(a_in, place);
     int b = place.b;
     const int ct = place.ct, hkv = place.hkv, first = varlen ? a_in.cu[b] : 0;
     const KArgs a = seq_args(a_in, b);
@@ -846,6 +857,29 @@ void walk_depth_tokens(const KArgs& launch) {
         if (in_v) check_access("dvd", a.dvd + b * a.sdvd.b + hkv * a.sdvd.h + c * a.sdvd.t + 8 * sub, 16, true);
       }
     }
+}
+
+// The order of a packed batch's launches on the 64-wide tiles: which grid each takes, and the query tiles that the dK/dV
+// workgroups of the fullest XCD (block % 8) and of the fullest place of one (32 compute units in turn) have, over the mean.
+void packed_launch_order(const KArgs& a) {
+  constexpr int BN = 128, BM = 32;
+  const int nseg = a.dkv_split;
+  std::vector<double> xcd(8, 0.), place(256, 0.);
+  double all = 0.;
+  for (int64_t block = 0; block < dkv_flat_blocks(a, BN, nseg); block++) {
+    const ColPlace p = col_place<true>(a, (int)block, BN, nseg);
+    if (!p.active) continue;
+    int b = p.b;
+    const KArgs one = seq_args(a, b);
+    const ColTilePlan plan = col_tile_plan(a, one, p.ct, BN, BM, true, nseg);
+    if (!plan.active) continue;
+    xcd[block % 8] += plan.nqt;
+    place[block % 256] += plan.nqt;
+    all += plan.nqt;
+  }
+  const auto name = [&](int64_t grid) { return packed_order(a, grid) ? "list" : "grid"; };
+  printf("rows %s columns %s xcd %.2f place %.2f\n", name(longest_row_grid(a, 128)), name(longest_col_grid(a, BN, nseg)),
+         8 * *std::max_element(xcd.begin(), xcd.end()) / all, 256 * *std::max_element(place.begin(), place.end()) / all);
 }
 
 void reset_writes(const char* name) {
@@ -1327,6 +1361,10 @@ int main(int argc, char** argv) {
   }
   if (a.dkv_split > 1)
     a.dkv_part = (float*)add_region("part", 20, (uint64_t)2 * a.dkv_split * (a.cu ? 1 : a.B) * a.Hkv * part_rows(a) * c.HD * 4, 4, true);
+  if (getenv("WALKER_ORDER")) {
+    packed_launch_order(a);
+    return 0;
+  }
   if (g_fp32) {
     if (c.HD > 128) return 2;
     c.HD == 64 ? walk_fp32<64>(a) : walk_fp32<128>(a);

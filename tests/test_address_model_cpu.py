@@ -132,6 +132,39 @@ def test_packed_batches_of_many_sequences(walker, shape, n):
     assert rc == 0 and "OK checked" in out, out
 
 
+@pytest.mark.parametrize("case", [
+    # lengths, H, D, L, G, mode, chunk tokens: more than 256 workgroups in the longest sequence's grid, so that rows and columns
+    # are taken from the list; row segments, depth tiles behind the sequence tiles, an empty and a one-token sequence
+    ((700, 0, 65, 1, 130), 8, 64, 2, 4, "causal", 0),
+    ((700, 33, 300), 16, 64, 0, 2, "noncausal", 0),
+    ((900, 100), 16, 64, 2, 8, "chunk_visible", 40),
+    ((600, 1, 0, 129), 16, 128, 3, 4, "causal", 0),
+], ids=lambda c: f"{c[5]}-{'_'.join(map(str, c[0]))}-D{c[2]}")
+def test_packed_batches_in_the_list_of_all_tiles(walker, case):
+    lengths, H, D, L, G, mode, cb = case
+    rc, out = run(walker, lengths, H, D, L, G, mode, cb, split=-1)
+    assert rc == 0 and "OK checked" in out, out
+
+
+@pytest.mark.parametrize("case", [
+    # lengths, H, G, mode, rows in list or grid, columns, most work of an XCD and of a compute unit's turn over the mean
+    ((2667, 2000, 1798), 8, 1, "causal", "list", "list", 1.05, 1.85),        # in tile order, segments side by side: 1.00, 1.97
+    ((3825, 3400, 3362), 1, 4, "causal", "list", "list", 1.05, 2.5),         # 1.40, 2.11
+    ((1497, 1400, 1300, 1200, 1094), 2, 4, "causal", "list", "list", 1.05, 2.0),   # 1.34, 2.12
+    ((1332, 1300, 1200, 1100, 1050, 1007, 1000, 1000, 950, 950, 900, 900), 4, 1, "causal", "list", "list", 1.05, 1.7),  # 1.45, 1.93
+    ((5909, 433), 4, 1, "causal", "list", "list", 1.05, 1.5),                # 1.10, 1.83
+    ((262, 150, 100, 60, 30, 25, 20, 14), 4, 2, "noncausal", "grid", "grid", 9, 99),  # a compute unit for every workgroup
+    ((2600, 133), 4, 1, "noncausal", "grid", "list", 1.05, 2.0),             # rows 168, columns in segments 672
+], ids=lambda c: f"{c[3]}-{c[0][0]}-H{c[1]}")
+def test_packed_launches_take_the_list_where_it_pays_and_spread_their_work(walker, case):
+    lengths, H, G, mode, rows, columns, xcd, place = case
+    rc, out = run(walker, lengths, H, 64, 0, G, mode, split=-1, env={"WALKER_ORDER": "1"})
+    w = out.split()
+    got = dict(zip(w[-8::2], w[-7::2]))
+    assert rc == 0 and (got["rows"], got["columns"]) == (rows, columns), out
+    assert float(got["xcd"]) <= xcd and float(got["place"]) <= place, out
+
+
 @pytest.mark.parametrize("case", PACKED, ids=lambda c: f"{c[5]}-{'_'.join(map(str, c[0]))}-D{c[2]}")
 def test_packed_batches(walker, case):
     lengths, H, D, L, G, mode, cb = case

@@ -1249,6 +1249,44 @@ def test_packed_batch_on_the_narrow_tiles_against_separate_calls(gpu_device):
             assert ((got - want).abs() <= 2.0 ** -6 * want.abs() + 2e-3).all(), (i, key)
 
 
+@pytest.mark.parametrize("case", [
+    # lengths, H, L, G, mode: the list of all tiles with one register of sequences and with four, its segments, the longest
+    # sequence's grid (257 sequences; few workgroups), an empty list place in every one
+    (tuple(i * 37 % 90 + (700 if i == 40 else 0) for i in range(65)), 1, 2, 2, "causal"),
+    (tuple(i * 37 % 90 + (1300 if i == 200 else 0) for i in range(256)), 1, 1, 2, "causal"),
+    (tuple(i * 37 % 90 for i in range(257)), 1, 1, 1, "noncausal"),
+    ((900, 0, 1, 333, 700), 8, 2, 2, "causal"),
+    ((900, 0, 1, 333, 700), 8, 0, 2, "noncausal"),
+    ((200, 1, 0, 65), 2, 3, 2, "noncausal"),
+], ids=lambda c: f"{c[4]}-{len(c[0])}-H{c[1]}")
+def test_packed_batches_of_the_narrow_tiles_in_every_order(gpu_device, case):
+    """Against separate calls: every result of a query row or depth slot bit for bit, dk and dv (summed in other pieces) to a
+    rounding of the result and one of a piece."""
+    from moda_amd import ops
+
+    lengths, H, L, G, mode = case
+    say(f"CASE packed order {case[1:]} {len(lengths)} sequences")
+    D, cu = 64, _cu(lengths)
+    inp = to_dev(oracle.make_inputs(1, cu[-1], H, D, L, G, seed=47, dtype=torch.bfloat16, std=0.5), gpu_device)
+    m = MODE_ID[mode]
+    packed = ops._packed(torch.tensor(cu, device=gpu_device), inp["q"], G)
+    o, lse = ops._raw_fwd(m, inp["q"], inp["k"], inp["v"], inp["kd"], inp["vd"], D ** -0.5, G, 0, packed=packed)
+    grads = ops._raw_bwd(m, inp["q"], inp["k"], inp["v"], inp["kd"], inp["vd"], o, lse, inp["do"], D ** -0.5, G, 0, packed=packed)
+    whole = dict(zip(("o", "lse", "dq", "dk", "dv", "dkd", "dvd"), (o, lse) + tuple(grads)))
+    mult = {"q": G, "k": 1, "v": 1, "kd": L, "vd": L}
+    for a, b in zip(cu[:-1], cu[1:]):
+        if a == b:
+            continue
+        part = {n: None if inp[n] is None else inp[n][:, a * x:b * x] for n, x in mult.items()}
+        part["do"] = inp["do"][:, a * G:b * G]
+        one = run_hip(part, D ** -0.5, G, mode, no_row_split=True)
+        for key, x in (("o", G), ("lse", G), ("dq", G), ("dkd", L), ("dvd", L)):
+            assert one[key] is None or torch.equal(whole[key][:, a * x:b * x], one[key]), (a, key)
+        for key in ("dk", "dv"):
+            got, want = whole[key][:, a:b].float(), one[key].float()
+            assert ((got - want).abs() <= 2.0 ** -6 * want.abs() + 2e-3).all(), (a, key)
+
+
 def test_packed_plain_gqa_attention(gpu_device):
     import moda_amd
 
