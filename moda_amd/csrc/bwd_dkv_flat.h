@@ -38,7 +38,7 @@ __global__ __launch_bounds__(256, RW == 1 ? 3 : 2) void dkv_flat_kernel(const KA
   const int block = blockIdx.x;
 #endif
   static_assert(RW == 1 || (RW == 4 && !VARLEN && !SPLIT), "four row waves: fixed length, no segments");
-  static_assert(!OWN_DELTA || (!VARLEN && HD == 64), "row sums of fixed-length launches, eight chunks a row");
+  static_assert(!OWN_DELTA || (RW == 4 && HD == 64), "row sums of launches with row waves, eight chunks a row");
   constexpr int NB = 2, WM = 32, BM = WM * RW, MBLK = WM / 16, BN = 4 / RW * 16 * NB, KS = HD / 32, MB = HD / 16;
   constexpr int NST = RW == 1 ? 3 : 2, DIST = NST - 1;  // ring stages, tiles in flight
   constexpr int SP = RW == 1 ? 64 : BM;  // floats per statistic and stage (wave-wide loads)

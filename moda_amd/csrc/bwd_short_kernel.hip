@@ -9,36 +9,32 @@
 
 namespace moda {
 
-template <typename T, int ADDR, int RW>
+template <typename T, int ADDR>
 __global__ __launch_bounds__(256, 2) void bwd_short_kernel(const KArgs a, int row_blocks) {
+  static_assert(16 * RowSmall<64>::NB * RowSmall<64>::W == kBwdShortRows, "the grid's rows are the workgroup's");
   if ((int)blockIdx.x < row_blocks)
     dq_body<T, 64, RowSmall<64>, ADDR>(a, blockIdx.x);
   else
-    dkv_flat_body<T, 64, false, false, RW, true>(a, (int)blockIdx.x - row_blocks);
+    dkv_flat_body<T, 64, false, false, 4, true>(a, (int)blockIdx.x - row_blocks);
 }
 
-template <typename T, int ADDR, int RW>
+template <typename T, int ADDR>
 hipError_t launch_short_t(const KArgs& a, hipStream_t stream) {
-  constexpr size_t lds_dq = dq_lds<64, RowSmall<64>, ADDR>(), lds_dkv = dkv_flat_lds<64, RW, true>();
+  constexpr size_t lds_dq = dq_lds<64, RowSmall<64>, ADDR>(), lds_dkv = dkv_flat_lds<64, 4, true>();
   constexpr size_t smem = lds_dq > lds_dkv ? lds_dq : lds_dkv;
   static_assert(2 * smem <= 160 * 1024, "two workgroups a compute unit");
   static LdsAttrState attr;
-  const hipError_t ea = allow_dynamic_lds(attr, reinterpret_cast<const void*>(&bwd_short_kernel<T, ADDR, RW>), smem);
+  const hipError_t ea = allow_dynamic_lds(attr, reinterpret_cast<const void*>(&bwd_short_kernel<T, ADDR>), smem);
   if (ea != hipSuccess) return ea;
-  const int64_t columns = dkv_flat_blocks(a, 128 / RW), rows = row_kernel_blocks(a, 128);
-  hipLaunchKernelGGL((bwd_short_kernel<T, ADDR, RW>), dim3((unsigned)(columns + rows)), dim3(256), smem, stream, a, (int)rows);
+  const int64_t columns = dkv_flat_blocks(a, 32), rows = row_kernel_blocks(a, kBwdShortRows);
+  hipLaunchKernelGGL((bwd_short_kernel<T, ADDR>), dim3((unsigned)(columns + rows)), dim3(256), smem, stream, a, (int)rows);
   return hipGetLastError();
-}
-
-template <typename T, int RW>
-hipError_t launch_short_a(const KArgs& a, hipStream_t stream) {
-  if (a.L == 0) return launch_short_t<T, 4, RW>(a, stream);
-  return a.Lv != a.L ? launch_short_t<T, 8, RW>(a, stream) : launch_short_t<T, 0, RW>(a, stream);
 }
 
 template <typename T>
 hipError_t launch_short_as(const KArgs& a, hipStream_t stream) {
-  return dkv_flat_row_waves(a) ? launch_short_a<T, 4>(a, stream) : launch_short_a<T, 1>(a, stream);
+  if (a.L == 0) return launch_short_t<T, 4>(a, stream);
+  return a.Lv != a.L ? launch_short_t<T, 8>(a, stream) : launch_short_t<T, 0>(a, stream);
 }
 
 // dtype: 0 bf16, 1 fp16; the caller asks bwd_one_launch first

@@ -18,7 +18,6 @@ hipError_t launch_dkv(const KArgs& a, int dtype, int hd, hipStream_t stream);
 hipError_t launch_bwd_short(const KArgs& a, int dtype, hipStream_t stream);
 hipError_t launch_generic(const KArgs& a, int dtype, int D, int Dv, int which, hipStream_t stream);
 hipError_t launch_fp32(const KArgs& a, int which, hipStream_t stream);
-bool fp32_one_launch(const KArgs& a);
 hipError_t launch_reorg(void* const* layers, int64_t n_layers, int64_t slot0, int64_t L_total, int64_t n_tokens,
                         int64_t row_bytes, void* cache, bool to_cache, hipStream_t stream);
 hipError_t launch_slot(void* const (&layer)[2], const int64_t (&strides)[2][3], void* const (&cache)[2], int64_t slot, int64_t L_total,

@@ -592,13 +592,6 @@ hipError_t launch_fp32_t(const KArgs& a, int which, hipStream_t stream) {
 
 }  // namespace
 
-// Whether dQ and dK/dV go as one launch: all workgroups run at once (one per compute unit; head dims above 64 have dK/dV
-// workgroups of another size).  More than that and the row sums, formed twice, cost more than the launch.
-bool fp32_one_launch(const KArgs& a) {
-  const int64_t cols = (a.has_seq ? (a.T + 15) / 16 : 0) + ((int64_t)a.T * a.Lv + 127) / 128;
-  return a.D <= 64 && a.Dv <= 64 && ((int64_t)(a.Tq + 15) / 16 * a.Hq + cols * a.Hkv) * a.B <= a.compute_units;
-}
-
 // which: 4 dQ and dK/dV in one launch; 0 forward, 1 dQ (leaves the row sums of o * do in the workspace), 2 dK/dV (reads them), 3 the row sums alone
 hipError_t launch_fp32(const KArgs& a, int which, hipStream_t stream) {
   const int hd = a.D > a.Dv ? a.D : a.Dv;

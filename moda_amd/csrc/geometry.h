@@ -396,13 +396,23 @@ inline bool narrow_slices(const KArgs& a) {
   const int64_t seq = (int64_t)a.T * (a.sk.t > a.sv.t ? a.sk.t : a.sv.t), dep = (int64_t)a.T * a.L * (a.skd.t > a.svd.t ? a.skd.t : a.svd.t);
   return 2 * (seq > dep ? seq : dep) <= 0x7fffffffll;
 }
-// dQ and sequence dK/dV of the 64-wide tiles in one launch (bwd_short_kernel): where the workgroups of both run at once, two a
-// compute unit.  More than that and the launch is longer than the two (64 x 197 tokens, six heads, twelve slots: step 191 ->
+// dQ and sequence dK/dV of the 64-wide tiles in one launch (bwd_short_kernel): row waves, and the workgroups of both run at once,
+// two a compute unit.  A replayed backward pass of 48 random such shapes takes 0.71 - 0.99 of the two launches' time (one of
+// 16 us 1.07), 0.75 - 0.88 where the launch holds 300 - 512 workgroups.  More than that and the launch is longer than the two (64 x 197 tokens, six heads, twelve slots: step 191 ->
 // 206 us; the twelve layers of a depth stream over 64 x 197 tokens of four query rows: 734 -> 794), each of which then has
 // the occupancy that its own registers and LDS allow.
+constexpr int kBwdShortRows = 128;  // query rows of a dQ workgroup there
 inline bool bwd_one_launch(const KArgs& a, int HD) {
-  return takes_dkv_flat(a, HD) && !a.cu && a.dkv_split <= 1 && a.own_delta && narrow_slices(a) &&
-         row_kernel_blocks(a, 128) + dkv_flat_blocks(a, dkv_flat_row_waves(a) ? 32 : 128) <= 2 * a.compute_units;
+  return takes_dkv_flat(a, HD) && dkv_flat_row_waves(a) && a.dkv_split <= 1 && a.own_delta && narrow_slices(a) &&
+         row_kernel_blocks(a, kBwdShortRows) + dkv_flat_blocks(a, 32) <= 2 * a.compute_units;
+}
+
+// fp32: whether dQ and dK/dV go as one launch: all workgroups run at once (one per compute unit; head dims above 64 have dK/dV
+// workgroups of another size).  More than that and the row sums, formed twice, cost more than the launch.  Twelve random
+// shapes, replayed: 0.65 - 0.91 of the two launches.
+inline bool fp32_one_launch(const KArgs& a) {
+  const int64_t cols = (a.has_seq ? (a.T + 15) / 16 : 0) + ((int64_t)a.T * a.Lv + 127) / 128;
+  return a.D <= 64 && a.Dv <= 64 && ((int64_t)(a.Tq + 15) / 16 * a.Hq + cols * a.Hkv) * a.B <= a.compute_units;
 }
 
 // Row segments of the sequence dK/dV launch (KArgs::dkv_split, dkv_seg_tiles): a launch ends with its longest workgroup,

@@ -22,8 +22,8 @@
 // usage: address_walker HD D Dv H G L Lv mode(0..4) chunk_tokens row_segments packed B_or_n len0 [len1 ...]
 //   packed = 0: a fixed-length batch of B sequences of len0 tokens; packed = 1: n sequences on one packed axis.
 //   environment: WALKER_FP32=1 walks the fp32 matrix kernels instead; WALKER_OWN_SLOT=1 a backward that leaves the slots
-//   without data alone and adds slot Lv of the depth gradients to dk, dv; WALKER_ORDER=1 prints the order of a packed
-//   batch's launches instead.
+//   without data alone and adds slot Lv of the depth gradients to dk, dv; instead of a walk, WALKER_ORDER=1 prints
+//   the order of a packed batch's launches, WALKER_ROUTE=1 whether a backward pass is one launch.
 // usage: address_walker linear rows K gelu n0 [n1 n2]   |   norm rows dim   |   slot B T H D L slot wide to_cache
 #include <hip/hip_runtime.h>
 
@@ -554,10 +554,11 @@ void walk_dkv(const KArgs& a_in) {
 
 // dkv_flat_kernel: four waves, a wave's 32 columns with K and V in registers, query tiles of 32 rows; or (RW = 4) the
 // waves on the same 32 columns, 32 rows each of a query tile of 128
-template <int HD, int RW>
+// OWN_DELTA: beside the dQ workgroups of a launch (bwd_short_kernel): the waves read o instead of the row sums
+template <int HD, int RW, bool OWN_DELTA = false>
 void walk_dkv_flat(const KArgs& a_in) {
   constexpr int NB = 2, BM = 32 * RW, BN = 4 / RW * 16 * NB, KS = HD / 32, MB = HD / 16, NST = RW == 1 ? 3 : 2, SP = RW == 1 ? 64 : BM;
-  const uint32_t lds_bytes = NST * 2 * BM * HD * 2 + NST * 2 * SP * 4;
+  const uint32_t lds_bytes = NST * 2 * BM * HD * 2 + NST * 2 * SP * 4 + (OWN_DELTA ? 4 * 32 * 4 : 0);
   const int nseg = a_in.dkv_split;
   if (RW > 1 && nseg > 1) fail("dkv_flat_kernel: row waves and segments");
   const uint32_t stat_byte = NST * 2 * BM * HD * 2;
@@ -613,7 +614,7 @@ void walk_dkv_flat(const KArgs& a_in) {
       }
       Loader ld;
       ld.init(tid);
-      const bool st_lse = (wave & 1) == 0;
+      const bool st_lse = OWN_DELTA || (wave & 1) == 0;
       const char* stb = st_lse ? (const char*)(a.lse + (int64_t)b * a.Tq * a.Hq + hkv) : (const char*)(a.delta + ((int64_t)b * a.Hq + hkv) * (varlen ? a.delta_pitch : a.Tq));
       const uint32_t st_row = st_lse ? (uint32_t)a.Hq * 4u : 4u;
       int ld_st = 0;
@@ -632,6 +633,15 @@ void walk_dkv_flat(const KArgs& a_in) {
         }
         const int rows = imax(imin(a.Tq - f_q0, BM), 0), st_first = RW == 1 ? 0 : (wave >> 1) * 64;
         if (rows == 0) fail("dkv_flat_kernel: empty query tile at row %d (Tq %d)", f_q0, a.Tq);
+        if (OWN_DELTA) {  // two lanes a row, four pieces each; the sums lie behind the statistics
+          ctx("bwd_short_kernel", (int)block, wave, lane, "pieces of o");
+          const int r = imin(f_q0 + (RW == 1 ? 0 : wave) * 32 + (lane >> 1), a.Tq - 1);
+          for (int c = 0; c < 4; c++) {
+            const int chunk = 2 * (lane & 1) + (c >> 1) + 4 * (c & 1);
+            check_access("o", a.o + b * a.so.b + hkv * a.so.h + (int64_t)r * a.so.t + (chunk * 8 < a.Dv ? chunk * 8 : 0), 16, false);
+          }
+          if (stat_byte + (uint32_t)(NST * 2 * SP + wave * 32 + (lane >> 1) + 1) * 4 > lds_bytes) fail("row sums past the LDS allocation");
+        }
         ctx("dkv_flat_kernel", (int)block, wave, lane, st_lse ? "query tile lse" : "query tile row sums");
         check_dma(st_lse ? "lse" : "delta", stb + (int64_t)f_q0 * st_row, (uint32_t)(rows - 1) * st_row + 4u,
                   (st_first + lane) * (int)st_row, 0, 4, stat_byte + (uint32_t)(ld_st * 2 * SP + (st_lse ? 0 : SP) + st_first) * 4,
@@ -990,81 +1000,87 @@ void walk_fp32(const KArgs& a_in) {
     }
     if (which == 2) require_full("dq");
   }
-  // dK/dV
-  const int BHk = a_in.B * a_in.Hkv, n_seq_tiles = a_in.has_seq ? (a_in.T + 15) / 16 : 0;
-  const int64_t ndep = ((int64_t)a_in.T * a_in.Lv + 16 * CW - 1) / (16 * CW), nblk = (n_seq_tiles + ndep) * BHk;
-  for (int64_t block = 0; block < nblk; block++) {
-    const int hkv = (int)(block % BHk) % a_in.Hkv, tile = (int)(block / BHk);
-    int b = (int)(block % BHk) / a_in.Hkv;
-    KArgs a = a_in;
-    enter_sequence(a, b, 2);
-    const bool dep = tile >= n_seq_tiles;
-    const int ncols = dep ? a.T * a.Lv : a.T;
-    for (int tid = 0; tid < 64 * CW; tid++) {
-      const int lane = tid & 63, n = lane & 15, q = lane >> 4, wave = tid >> 6;
-      const int c0 = dep ? ((tile - n_seq_tiles) * CW + wave) * 16 : tile * 16;
-      if (c0 >= ncols) continue;
-      const int c = c0 + n, cc = imin(c, ncols - 1);
-      const int64_t crow = dep ? depth_row_of(a, cc) : (int64_t)cc;
-      ctx("fp32_dkv_kernel", (int)block, wave, lane, "stationary K and V rows");
-      score(dep ? "kd" : "k", dep ? f(a.kd) + b * a.skd.b + hkv * a.skd.h + crow * a.skd.t : f(a.k) + b * a.sk.b + hkv * a.sk.h + crow * a.sk.t, q, a.D);
-      score(dep ? "vd" : "v", dep ? f(a.vd) + b * a.svd.b + hkv * a.svd.h + crow * a.svd.t : f(a.v) + b * a.sv.b + hkv * a.sv.h + crow * a.sv.t, q, a.Dv);
-      int lo, hi, unused;
-      q_interval(a, dep, c0, lo, unused);
-      q_interval(a, dep, imin(ncols, c0 + 16) - 1, unused, hi);
-      const int r_first = lo / 16 * 16, nrb = (hi - r_first + 15) / 16, nb = nrb * a.hdiv;
-      ctx("fp32_dkv_kernel", (int)block, wave, lane, "query rows and their statistics");
-      for (int blk = dep ? 0 : wave; blk < nb; blk += dep ? 1 : CW) {
-        const int hq = hkv * a.hdiv + blk / nrb, r0 = r_first + blk % nrb * 16;
-        const float *qp = f(a.q) + b * a.sq.b + hq * a.sq.h, *dop = f(a.d_o) + b * a.sdo.b + hq * a.sdo.h;
-        const int64_t r = imin(r0 + n, a.Tq - 1);
-        score("q", qp + r * a.sq.t, q, a.D);
-        score("do", dop + r * a.sdo.t, q, a.Dv);
-        for (int i = 0; i < 4; i++) {
-          const int64_t ri = imin(r0 + 4 * q + i, a.Tq - 1);
-          check_access("lse", a.lse + ((int64_t)b * a.Tq + ri) * a.Hq + hq, 4, false);
-          check_access("delta", a.delta + ((int64_t)b * a.Hq + hq) * a.delta_pitch + ri, 4, false);
-          sum("q", qp + ri * a.sq.t, n, a.D);
-          sum("do", dop + ri * a.sdo.t, n, a.Dv);
+  // dK/dV: as a launch of its own, and beside the dQ workgroups, where it reads o instead of the row sums
+  const bool one_launch = HD == 64 && fp32_one_launch(a_in);
+  if (one_launch) printf("fp32_bwd_kernel ");
+  for (int own_delta = 0; own_delta <= (one_launch ? 1 : 0); own_delta++) {
+    for (const char* name : {"dk", "dv", "dkd", "dvd"}) reset_writes(name);
+    const int BHk = a_in.B * a_in.Hkv, n_seq_tiles = a_in.has_seq ? (a_in.T + 15) / 16 : 0;
+    const int64_t ndep = ((int64_t)a_in.T * a_in.Lv + 16 * CW - 1) / (16 * CW), nblk = (n_seq_tiles + ndep) * BHk;
+    for (int64_t block = 0; block < nblk; block++) {
+      const int hkv = (int)(block % BHk) % a_in.Hkv, tile = (int)(block / BHk);
+      int b = (int)(block % BHk) / a_in.Hkv;
+      KArgs a = a_in;
+      enter_sequence(a, b, 2);
+      const bool dep = tile >= n_seq_tiles;
+      const int ncols = dep ? a.T * a.Lv : a.T;
+      for (int tid = 0; tid < 64 * CW; tid++) {
+        const int lane = tid & 63, n = lane & 15, q = lane >> 4, wave = tid >> 6;
+        const int c0 = dep ? ((tile - n_seq_tiles) * CW + wave) * 16 : tile * 16;
+        if (c0 >= ncols) continue;
+        const int c = c0 + n, cc = imin(c, ncols - 1);
+        const int64_t crow = dep ? depth_row_of(a, cc) : (int64_t)cc;
+        ctx("fp32_dkv_kernel", (int)block, wave, lane, "stationary K and V rows");
+        score(dep ? "kd" : "k", dep ? f(a.kd) + b * a.skd.b + hkv * a.skd.h + crow * a.skd.t : f(a.k) + b * a.sk.b + hkv * a.sk.h + crow * a.sk.t, q, a.D);
+        score(dep ? "vd" : "v", dep ? f(a.vd) + b * a.svd.b + hkv * a.svd.h + crow * a.svd.t : f(a.v) + b * a.sv.b + hkv * a.sv.h + crow * a.sv.t, q, a.Dv);
+        int lo, hi, unused;
+        q_interval(a, dep, c0, lo, unused);
+        q_interval(a, dep, imin(ncols, c0 + 16) - 1, unused, hi);
+        const int r_first = lo / 16 * 16, nrb = (hi - r_first + 15) / 16, nb = nrb * a.hdiv;
+        ctx("fp32_dkv_kernel", (int)block, wave, lane, "query rows and their statistics");
+        for (int blk = dep ? 0 : wave; blk < nb; blk += dep ? 1 : CW) {
+          const int hq = hkv * a.hdiv + blk / nrb, r0 = r_first + blk % nrb * 16;
+          const float *qp = f(a.q) + b * a.sq.b + hq * a.sq.h, *dop = f(a.d_o) + b * a.sdo.b + hq * a.sdo.h;
+          const int64_t r = imin(r0 + n, a.Tq - 1);
+          score("q", qp + r * a.sq.t, q, a.D);
+          score("do", dop + r * a.sdo.t, q, a.Dv);
+          if (own_delta) score("o", f(a.o) + b * a.so.b + hq * a.so.h + r * a.so.t, q, a.Dv);
+          for (int i = 0; i < 4; i++) {
+            const int64_t ri = imin(r0 + 4 * q + i, a.Tq - 1);
+            check_access("lse", a.lse + ((int64_t)b * a.Tq + ri) * a.Hq + hq, 4, false);
+            if (!own_delta) check_access("delta", a.delta + ((int64_t)b * a.Hq + hq) * a.delta_pitch + ri, 4, false);
+            sum("q", qp + ri * a.sq.t, n, a.D);
+            sum("do", dop + ri * a.sdo.t, n, a.Dv);
+          }
+        }
+        ctx("fp32_dkv_kernel", (int)block, wave, lane, "gradient rows");
+        if (dep) {
+          if (c >= ncols) continue;
+          const float *dkp = f(a.dkd) + b * a.sdkd.b + hkv * a.sdkd.h + crow * a.sdkd.t, *dvp = f(a.dvd) + b * a.sdvd.b + hkv * a.sdvd.h + crow * a.sdvd.t;
+          for (int h = 0; h < H4; h++)
+            for (int i = 0; i < 4; i++) {
+              const int d = 64 * h + 16 * q + 4 * i;
+              if (d < a.D) check_access("dkd", dkp + d, 16, true);
+              if (d < a.Dv) check_access("dvd", dvp + d, 16, true);
+            }
+          if (a.Lv != a.L && !a.keep_slots && c % a.Lv == a.Lv - 1)
+            for (int slot = a.Lv; slot < a.L; slot++) {
+              dkp += a.sdkd.t;
+              dvp += a.sdvd.t;
+              for (int d = 4 * q; d < a.D; d += 16) check_access("dkd", dkp + d, 16, true);
+              for (int d = 4 * q; d < a.Dv; d += 16) check_access("dvd", dvp + d, 16, true);
+            }
+          continue;
+        }
+        if (lane == 0) partial((CW + wave) * PART, 2 * CW * PART * 4);
+        for (int e = tid; e < 2 * 16 * HD / 4; e += 64 * CW) {
+          const int w = e / (16 * HD / 4), row = e % (16 * HD / 4) / (HD / 4), d = (e % (HD / 4)) * 4;
+          if (c0 + row >= ncols || d >= (w ? a.Dv : a.D)) continue;
+          if (w)
+            check_access("dv", f(a.dv) + b * a.sdv.b + hkv * a.sdv.h + (int64_t)(c0 + row) * a.sdv.t + d, 16, true);
+          else
+            check_access("dk", f(a.dk) + b * a.sdk.b + hkv * a.sdk.h + (int64_t)(c0 + row) * a.sdk.t + d, 16, true);
         }
       }
-      ctx("fp32_dkv_kernel", (int)block, wave, lane, "gradient rows");
-      if (dep) {
-        if (c >= ncols) continue;
-        const float *dkp = f(a.dkd) + b * a.sdkd.b + hkv * a.sdkd.h + crow * a.sdkd.t, *dvp = f(a.dvd) + b * a.sdvd.b + hkv * a.sdvd.h + crow * a.sdvd.t;
-        for (int h = 0; h < H4; h++)
-          for (int i = 0; i < 4; i++) {
-            const int d = 64 * h + 16 * q + 4 * i;
-            if (d < a.D) check_access("dkd", dkp + d, 16, true);
-            if (d < a.Dv) check_access("dvd", dvp + d, 16, true);
-          }
-        if (a.Lv != a.L && !a.keep_slots && c % a.Lv == a.Lv - 1)
-          for (int slot = a.Lv; slot < a.L; slot++) {
-            dkp += a.sdkd.t;
-            dvp += a.sdvd.t;
-            for (int d = 4 * q; d < a.D; d += 16) check_access("dkd", dkp + d, 16, true);
-            for (int d = 4 * q; d < a.Dv; d += 16) check_access("dvd", dvp + d, 16, true);
-          }
-        continue;
-      }
-      if (lane == 0) partial((CW + wave) * PART, 2 * CW * PART * 4);
-      for (int e = tid; e < 2 * 16 * HD / 4; e += 64 * CW) {
-        const int w = e / (16 * HD / 4), row = e % (16 * HD / 4) / (HD / 4), d = (e % (HD / 4)) * 4;
-        if (c0 + row >= ncols || d >= (w ? a.Dv : a.D)) continue;
-        if (w)
-          check_access("dv", f(a.dv) + b * a.sdv.b + hkv * a.sdv.h + (int64_t)(c0 + row) * a.sdv.t + d, 16, true);
-        else
-          check_access("dk", f(a.dk) + b * a.sdk.b + hkv * a.sdk.h + (int64_t)(c0 + row) * a.sdk.t + d, 16, true);
-      }
     }
-  }
-  if (a_in.has_seq) {
-    require_full("dk");
-    require_full("dv");
-  }
-  if (a_in.L > 0) {
-    require_depth_rows("dkd", a_in, a_in.D);
-    require_depth_rows("dvd", a_in, a_in.Dv);
+    if (a_in.has_seq) {
+      require_full("dk");
+      require_full("dv");
+    }
+    if (a_in.L > 0) {
+      require_depth_rows("dkd", a_in, a_in.D);
+      require_depth_rows("dvd", a_in, a_in.Dv);
+    }
   }
 }
 
@@ -1295,6 +1311,24 @@ void walk_all(const Case& c, const KArgs& a) {
     require_depth_rows("dkd", a, a.D);
     require_depth_rows("dvd", a, a.Dv);
   }
+  // ---- the whole backward where dQ and dK/dV share a launch (the stages apart are what is walked above)
+  if constexpr (HD == 64)
+    if (bwd_one_launch(a, HD)) {
+      printf("bwd_short_kernel ");
+      if (row_kernel_blocks(a, kBwdShortRows) + dkv_flat_blocks(a, 32) > 2 * a.compute_units) fail("more workgroups than run at once");
+      for (const char* name : {"delta", "dq", "dk", "dv", "dkd", "dvd"}) reset_writes(name);
+      if (a.depth_p)
+        for (const char* name : {"hand_p", "hand_ds"}) reset_writes(name);
+      const uint32_t own = (uint32_t)RowSmall<64>::W * (2 * 64 + 16) * HD * 2;
+      walk_row_kernel<HD, RowSmall<64>, false>(a, true, 32, true, a.L > 0 ? std::max(ring(RowSmall<64>::NST), own) : ring(RowSmall<64>::NST), "bwd_short_kernel");
+      walk_dkv_flat<HD, 4, true>(a);
+      for (const char* name : {"delta", "dq", "dk", "dv"}) require_full(name);
+      if (a.L > 0 && depth_grads_in_dq(a, HD)) {
+        if (a.Lv != a.L && !a.keep_slots) walk_zero_unfilled<HD>(a);
+        require_depth_rows("dkd", a, a.D);
+        require_depth_rows("dvd", a, a.Dv);
+      }
+    }
   (void)c;
 }
 
@@ -1361,6 +1395,11 @@ int main(int argc, char** argv) {
   }
   if (a.dkv_split > 1)
     a.dkv_part = (float*)add_region("part", 20, (uint64_t)2 * a.dkv_split * (a.cu ? 1 : a.B) * a.Hkv * part_rows(a) * c.HD * 4, 4, true);
+  if (getenv("WALKER_ROUTE")) {  // of a whole backward pass; split 1: a workspace without room for segments
+    const bool one = g_fp32 ? c.HD == 64 && fp32_one_launch(a) : bwd_one_launch(a, c.HD);
+    printf("%s\n", one ? "one launch" : "two launches");
+    return 0;
+  }
   if (getenv("WALKER_ORDER")) {
     packed_launch_order(a);
     return 0;

@@ -37,6 +37,38 @@ REFERENCE_MATRIX = [
 ]
 assert len(REFERENCE_MATRIX) == 102
 
+# Backward passes at the edges of what dQ and sequence dK/dV take as one launch (256 compute units):
+# (B, T, H, G, D, L, L_valid, mode, dtype), one launch or not
+ONE_LAUNCH = [
+    # one workgroup; ragged tiles with four row waves; more than 1024 query rows; head dims below the tile width; a partial
+    # stream; no stream; depth gradients of their own launch (G 3); chunk-visible
+    ((1, 1, 1, 1, 64, 1, 1, "CAUSAL", "fp16"), True),
+    ((2, 95, 4, 2, 64, 8, 8, "CAUSAL", "fp16"), True),
+    ((3, 257, 1, 4, 64, 3, 3, "NONCAUSAL", "bf16"), False),
+    ((2, 130, 2, 1, 40, 5, 2, "NONCAUSAL", "bf16"), True),
+    ((2, 77, 3, 2, 64, 0, 0, "CAUSAL", "bf16"), True),
+    ((1, 70, 2, 3, 48, 4, 4, "CAUSAL", "fp16"), True),
+    ((1, 100, 2, 4, 64, 3, 3, "CHUNK_VISIBLE", "bf16"), True),
+    # more than twice the compute units, then the last size in one launch and the first one in two: 510 and 515 workgroups; as
+    # many query rows as row waves take, and one token more
+    ((32, 127, 4, 1, 64, 2, 2, "CAUSAL", "bf16"), False),
+    ((32, 129, 4, 1, 64, 2, 2, "CAUSAL", "bf16"), False),
+    ((51, 127, 2, 1, 64, 2, 2, "CAUSAL", "bf16"), True),
+    ((103, 127, 1, 1, 64, 2, 2, "NONCAUSAL", "bf16"), False),
+    ((3, 256, 4, 4, 64, 2, 2, "CAUSAL", "fp16"), True),
+    ((4, 1024, 3, 1, 64, 1, 1, "NONCAUSAL", "bf16"), True),
+    ((3, 1025, 1, 1, 64, 1, 1, "NONCAUSAL", "bf16"), False),
+    # fp32: both instantiations, one row, an empty and a partial stream, chunk-visible, the last size in one launch and the
+    # first one in two (256 and 260 workgroups)
+    ((1, 1, 1, 1, 64, 1, 1, "CAUSAL", "fp32"), True),
+    ((1, 256, 4, 1, 64, 4, 4, "CAUSAL", "fp32"), True),
+    ((2, 61, 2, 2, 36, 3, 2, "NONCAUSAL", "fp32"), True),
+    ((1, 90, 2, 3, 64, 0, 0, "CAUSAL", "fp32"), True),
+    ((1, 70, 2, 4, 20, 3, 3, "CHUNK_VISIBLE", "fp32"), True),
+    ((1, 1024, 1, 2, 64, 8, 8, "CAUSAL", "fp32"), True),
+    ((1, 1025, 1, 2, 64, 8, 8, "CAUSAL", "fp32"), False),
+]
+
 # Small shapes used to cross-check the oracle's forms on the CPU:
 # (B, T, H, D, L, G, mode, chunk_tokens)
 ORACLE_SMALL = [

@@ -18,6 +18,8 @@ import subprocess
 
 import pytest
 
+from cases import ONE_LAUNCH
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 MODES = {"causal": 0, "noncausal": 1, "chunk_visible": 2, "depth_only": 3, "plain": 4}
 
@@ -253,6 +255,27 @@ def test_own_slot_rows(walker, case):
     assert rc == 0 and "OK checked" in out, out
     rc, out = run(walker, env={"WALKER_OWN_SLOT": "1", "WALKER_SHRINK": f"dkd:{2 * H * D * L}"}, **args)
     assert rc == 1 and "VIOLATION" in out, out
+
+
+@pytest.mark.parametrize("case", ONE_LAUNCH, ids=lambda c: "-".join(map(str, c[0])))
+def test_backward_passes_in_one_launch(walker, case):
+    """The rule takes the cases of the GPU test the way that they are meant to test, and the shared launch stays inside its
+    tensors and writes every gradient once."""
+    (B, T, H, G, D, L, Lv, mode, dtype), one = case
+    args = dict(lengths=(T,), H=H, D=D, L=L, G=G, mode=mode.lower(), cb=16 // G, packed=False, B=B, Lv=Lv if Lv != L else 0, split=-1)
+    env = {"WALKER_FP32": "1"} if dtype == "fp32" else {}
+    rc, out = run(walker, env={"WALKER_ROUTE": "1", **env}, **args)
+    assert rc == 0 and out.endswith("one launch" if one else "two launches"), out
+    if B * T * H * G > 13000:
+        return
+    rc, out = run(walker, env=env, **args)
+    assert rc == 0 and "OK checked" in out and (("bwd_short_kernel" in out) or ("fp32_bwd_kernel" in out)) == one, out
+
+
+def test_long_rows_without_room_for_segments_take_two_launches(walker):
+    for T, one in ((1024, True), (1025, False), (1100, False)):
+        rc, out = run(walker, (T,), 2, 64, 3, 1, "causal", packed=False, B=1, split=1, env={"WALKER_ROUTE": "1"})
+        assert rc == 0 and out.endswith("one launch" if one else "two launches"), out
 
 
 FP32 = [

@@ -16,7 +16,7 @@ import pytest
 import torch
 
 import oracle
-from cases import REFERENCE_MATRIX
+from cases import ONE_LAUNCH, REFERENCE_MATRIX
 
 pytestmark = pytest.mark.gpu
 
@@ -1927,27 +1927,7 @@ def test_stack_widths_and_which_of_them_run_as_native_launches(gpu_device, case)
     assert off(m.bfloat16()(x) if y is None else y) <= max(1.1 * off(z), 2.0 ** -8), (off(z), y is None or off(y))
 
 
-@pytest.mark.parametrize("case", [
-    # B, T, H, G, D, L, L_valid, mode, dtype: one workgroup; ragged tiles with four row waves; column tiles without them; head
-    # dims below the tile width; a partial stream; no stream; depth gradients of their own launch (G 3); chunk-visible; the
-    # last size in one launch and the first one in two
-    (1, 1, 1, 1, 64, 1, 1, "CAUSAL", "fp16"),
-    (2, 95, 4, 2, 64, 8, 8, "CAUSAL", "fp16"),
-    (3, 257, 1, 4, 64, 3, 3, "NONCAUSAL", "bf16"),
-    (2, 130, 2, 1, 40, 5, 2, "NONCAUSAL", "bf16"),
-    (2, 77, 3, 2, 64, 0, 0, "CAUSAL", "bf16"),
-    (1, 70, 2, 3, 48, 4, 4, "CAUSAL", "fp16"),
-    (1, 100, 2, 4, 64, 3, 3, "CHUNK_VISIBLE", "bf16"),
-    (32, 127, 4, 1, 64, 2, 2, "CAUSAL", "bf16"),
-    (32, 129, 4, 1, 64, 2, 2, "CAUSAL", "bf16"),
-    # fp32: both instantiations, one row, an empty and a partial stream, chunk-visible, the last size in one launch
-    (1, 1, 1, 1, 64, 1, 1, "CAUSAL", "fp32"),
-    (1, 256, 4, 1, 64, 4, 4, "CAUSAL", "fp32"),
-    (2, 61, 2, 2, 36, 3, 2, "NONCAUSAL", "fp32"),
-    (1, 90, 2, 3, 64, 0, 0, "CAUSAL", "fp32"),
-    (1, 70, 2, 4, 20, 3, 3, "CHUNK_VISIBLE", "fp32"),
-    (1, 1024, 1, 2, 64, 8, 8, "CAUSAL", "fp32"),
-], ids=str)
+@pytest.mark.parametrize("case", [c for c, _ in ONE_LAUNCH], ids=str)
 def test_backward_in_one_launch_equals_its_stages(gpu_device, case):
     """dQ and dK/dV of small problems share a launch, whose dK/dV workgroups form the row sums of o * do themselves.  The
     stages one by one take them from the workspace: same additions in the same order, same bits."""
@@ -1970,6 +1950,25 @@ def test_backward_in_one_launch_equals_its_stages(gpu_device, case):
     apart = ops._raw_bwd(*args, stages=_lib.STAGE_DKV, ws=ws, out=apart, **valid)
     for name, x, y in zip(("dq", "dk", "dv", "dkd", "dvd"), together, apart):
         assert (x is None and y is None) or torch.equal(x, y), name
+
+
+def test_backward_of_long_rows_with_a_workspace_of_row_sums_alone(gpu_device):
+    """More query rows than row waves take, and no room for the segments that such launches are otherwise cut into: whole
+    column tiles in a launch of their own, same bits as stage by stage."""
+    from moda_amd import _lib, ops
+
+    B, T, H, G, D, L = 1, 1100, 2, 1, 64, 3
+    say("CASE row sums alone")
+    gen = torch.Generator(device=gpu_device).manual_seed(T)
+    rn = lambda *s: (0.5 * torch.randn(*s, generator=gen, device=gpu_device)).bfloat16()
+    q, k, v, do, kd, vd = (rn(B, T * n, H, D) for n in (G, 1, 1, G, L, L))
+    o, lse = ops._raw_fwd(_lib.CAUSAL, q, k, v, kd, vd, 0.1, G, 0)
+    args, ws = (_lib.CAUSAL, q, k, v, kd, vd, o, lse, do, 0.1, G, 0), torch.empty(4 * B * T * G * H, dtype=torch.uint8, device=gpu_device)
+    together = ops._raw_bwd(*args, ws=ws)
+    apart = ops._raw_bwd(*args, stages=_lib.STAGE_DELTA | _lib.STAGE_DQ, ws=ws)
+    apart = ops._raw_bwd(*args, stages=_lib.STAGE_DKV, ws=ws, out=apart)
+    for name, x, y in zip(("dq", "dk", "dv", "dkd", "dvd"), together, apart):
+        assert torch.equal(x, y), name
 
 
 def _linear(x, parts, residual=None, gelu=False, ldx=None, K=None):
