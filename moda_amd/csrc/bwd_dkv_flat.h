@@ -174,7 +174,8 @@ __global__ __launch_bounds__(256, RW == 1 ? 3 : 2) void dkv_flat_kernel(const KA
       }
       float row_sum = sum[0] + sum[1];
       row_sum += __shfl_xor(row_sum, 1, 64);
-      if (own_half == 0) own_stat[own_row] = -row_sum;
+      // a row past the end has zeros everywhere, though the last row's o was read for it
+      if (own_half == 0) own_stat[own_row] = q0 + rw * WM + own_row < a.Tq ? -row_sum : 0.f;
       if (it + 1 < nqt) fetch_o(it + 1);
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_waitcnt(0xC07F);  // the wave reads what its lanes wrote

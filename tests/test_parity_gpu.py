@@ -1952,6 +1952,28 @@ def test_backward_in_one_launch_equals_its_stages(gpu_device, case):
         assert (x is None and y is None) or torch.equal(x, y), name
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_backward_in_one_launch_with_an_infinite_last_row(gpu_device, dtype):
+    """A row past the end takes no share in dK, dV, whatever the last row of o holds (the shared launch reads that row in its
+    place): infinities and NaN where the stages one by one have them."""
+    from moda_amd import _lib, ops
+
+    B, T, H, G, D, L = 2, 37, 2, 1, 64, 2
+    say(f"CASE infinite last row {dtype}")
+    gen = torch.Generator(device=gpu_device).manual_seed(T)
+    rn = lambda *s: (0.5 * torch.randn(*s, generator=gen, device=gpu_device)).to(dtype)
+    q, k, v, do, kd, vd = (rn(B, T * n, H, D) for n in (G, 1, 1, G, L, L))
+    o, lse = ops._raw_fwd(_lib.CAUSAL, q, k, v, kd, vd, 0.1, G, 0)
+    o[0, -1, 0, 3] = float("inf")
+    args = (_lib.CAUSAL, q, k, v, kd, vd, o, lse, do, 0.1, G, 0)
+    together, ws = ops._raw_bwd(*args), ops.bwd_workspace(_lib.CAUSAL, q, k, v, kd, vd, G)
+    apart = ops._raw_bwd(*args, stages=_lib.STAGE_DELTA | _lib.STAGE_DQ, ws=ws)
+    apart = ops._raw_bwd(*args, stages=_lib.STAGE_DKV, ws=ws, out=apart)
+    assert apart[1].isinf().any()
+    for name, x, y in zip(("dq", "dk", "dv", "dkd", "dvd"), together, apart):
+        assert torch.equal(x.isnan(), y.isnan()) and torch.equal(x.nan_to_num(7.0), y.nan_to_num(7.0)), name
+
+
 def test_backward_of_long_rows_with_a_workspace_of_row_sums_alone(gpu_device):
     """More query rows than row waves take, and no room for the segments that such launches are otherwise cut into: whole
     column tiles in a launch of their own, same bits as stage by stage."""
