@@ -32,7 +32,7 @@ struct TailPart {
   const uint16_t *w, *bias;
   uint16_t* y;
   int64_t ldy;
-  int n, block_end;  // output features; 16-feature blocks of this part and of those before it
+  int block_end;  // 16-feature blocks of this part and of those before it
 };
 struct TailArgs {
   const uint16_t *h, *res;  // attention output, residual stream
@@ -63,6 +63,7 @@ __device__ __forceinline__ void lds_barrier() {
 // result, rounded, over x: times x that is the result again to 2^-23, which rounds to itself.  8 vector instructions an element
 // where the formula (which fp16 takes) has 22, 6.5 k cycles for 64 rows x 256 features against 2.4 k (the launch 40 -> 32.7 us).
 constexpr int kGeluHalf = 21 * 128, kGeluTable = 2 * kGeluHalf, kGeluFirst = (127 - 17) << 7;
+static_assert(kGeluTable * sizeof(float) == MODA_HIP_GELU_TABLE_BYTES, "what a caller allocates");
 template <typename T>
 constexpr int table_bytes() {
   return std::is_same<T, BF16>::value ? kGeluTable * 4 : 0;
@@ -576,7 +577,7 @@ hipError_t launch_block_tail(const moda_hip_block_tail_args* t, int compute_unit
   for (int i = 0; i < t->n_parts; i++) {
     const moda_hip_linear_part& p = t->parts[i];
     end += (int)p.n / 16;
-    a.part[i] = TailPart{in(p.w), in(p.bias), (uint16_t*)p.y, p.ldy, (int)p.n, end};
+    a.part[i] = TailPart{in(p.w), in(p.bias), (uint16_t*)p.y, p.ldy, end};
   }
   return t->dtype == 0 ? launch_tail<BF16>(a, (int)t->width, t->post_norm != 0, compute_units, stream)
                        : launch_tail<FP16>(a, (int)t->width, t->post_norm != 0, compute_units, stream);

@@ -637,16 +637,12 @@ __device__ __forceinline__ float group_sum(float x) {
 }
 
 template <typename T, int HD>
-__global__ __launch_bounds__(256) void depth_cols_kernel(const KArgs a_in) {
+__global__ __launch_bounds__(256) void depth_cols_kernel(const KArgs a) {
   constexpr int LPC = HD / 8, CPW = 64 / LPC, CPB = 4 * CPW;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int sub = lane % LPC;
-  KArgs a = a_in;
   const int BHk = a.B * a.Hkv;
-  const int bh = blockIdx.x % BHk;
-  int b = bh / a.Hkv;
-  const int hkv = bh % a.Hkv;
-  enter_sequence(a, b);
+  const int bh = blockIdx.x % BHk, b = bh / a.Hkv, hkv = bh % a.Hkv;
   const int64_t c = (int64_t)(blockIdx.x / BHk) * CPB + wave * CPW + lane / LPC;
   if (c >= (int64_t)a.T * a.L) return;  // whole lane groups leave together
   const int w = (int)(c / a.L), slot = (int)(c - (int64_t)w * a.L);
@@ -725,16 +721,12 @@ __global__ __launch_bounds__(256) void depth_cols_kernel(const KArgs a_in) {
 // (KArgs::depth_p, depth_ds): no kd, vd, no scores -- per column G scalar pairs and the G rows of q and do, which the
 // L columns of a token share through the caches.  The launch moves the gradient rows out and little else.
 template <typename T, int HD>
-__global__ __launch_bounds__(256) void depth_cols_handed_kernel(const KArgs a_in) {
+__global__ __launch_bounds__(256) void depth_cols_handed_kernel(const KArgs a) {
   constexpr int LPC = HD / 8, CPW = 64 / LPC, CPB = 4 * CPW;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int sub = lane % LPC;
-  KArgs a = a_in;
   const int BHk = a.B * a.Hkv;
-  const int bh = blockIdx.x % BHk;
-  int b = bh / a.Hkv;
-  const int hkv = bh % a.Hkv;
-  enter_sequence(a, b);
+  const int bh = blockIdx.x % BHk, b = bh / a.Hkv, hkv = bh % a.Hkv;
   const int64_t c = (int64_t)(blockIdx.x / BHk) * CPB + wave * CPW + lane / LPC;
   if (c >= (int64_t)a.T * a.L) return;  // whole lane groups leave together
   const int w = (int)(c / a.L), slot = (int)(c - (int64_t)w * a.L);
@@ -801,16 +793,12 @@ __global__ __launch_bounds__(256) void depth_cols_handed_kernel(const KArgs a_in
 // dim each) keep the token's rows of q and do in registers and walk its slots, so that q and do are read once per
 // token instead of once per slot and the launch is little more than the stream of gradient rows going out.
 template <typename T, int HD>
-__global__ __launch_bounds__(256) void depth_token_handed_kernel(const KArgs a_in) {
+__global__ __launch_bounds__(256) void depth_token_handed_kernel(const KArgs a) {
   constexpr int LPT = HD / 8, TPW = 64 / LPT, TPB = 4 * TPW, GMAX = 4;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int sub = lane % LPT;
-  KArgs a = a_in;
   const int BHk = a.B * a.Hkv;
-  const int bh = blockIdx.x % BHk;
-  int b = bh / a.Hkv;
-  const int hkv = bh % a.Hkv;
-  enter_sequence(a, b);
+  const int bh = blockIdx.x % BHk, b = bh / a.Hkv, hkv = bh % a.Hkv;
   const int w = (blockIdx.x / BHk) * TPB + wave * TPW + lane / LPT;
   if (w >= a.T) return;  // whole lane groups leave together
   const bool in_k = 8 * sub < a.D, in_v = 8 * sub < a.Dv;

@@ -11,7 +11,6 @@
 // blocks; lane (n, q) owns rows 16*nb + n and, inside a 16-column score block, columns slot_base(q) .. +3.
 // P^T is recomputed from the saved base-2 LSE, dS^T = P^T * (dP^T - delta) is packed straight into the
 // B operand of dQ^T += K^T * dS^T, K^T coming from the LDS transpose read of the K tile.
-#include <algorithm>
 #include <type_traits>
 
 #include "bwd_dq.h"
@@ -93,10 +92,7 @@ hipError_t launch_dq_t_addr(const KArgs& a, bool small, hipStream_t stream) {
 
 template <typename T, int HD>
 hipError_t launch_dq_t(const KArgs& a, hipStream_t stream) {
-  // byte span of the widest streamed (batch, head) slice
-  const int64_t span = 2 * std::max(std::max((int64_t)a.T * a.sk.t, (int64_t)a.T * a.sv.t),
-                                    std::max((int64_t)a.T * a.L * a.skd.t, (int64_t)a.T * a.L * a.svd.t));
-  const bool wide = span > 0x7fffffffll;
+  const bool wide = !narrow_slices(a);
   const bool small = a.cu ? use_small_rows(a.delta_pitch, a.Hq, a.compute_units)  // the rows there are, not those of the grid
                           : use_small_rows(a.Tq, (long long)a.B * a.Hq, a.compute_units);
   switch ((wide ? 1 : 0) | (a.cu ? 2 : 0) | (a.L == 0 ? 4 : 0) | (a.L > 0 && a.Lv != a.L ? 8 : 0)) {

@@ -14,7 +14,6 @@
 // loop over column tiles is split in two: tiles every row of the workgroup sees
 // completely run a body without any masking or visibility tests; boundary and
 // depth tiles run the masked body.
-#include <algorithm>
 #include <type_traits>
 
 #include "geometry.h"
@@ -691,10 +690,7 @@ hipError_t launch_fwd_t_addr(const KArgs& a, bool small, hipStream_t stream) {
 
 template <typename T, int HD>
 hipError_t launch_fwd_t(const KArgs& a, hipStream_t stream) {
-  // byte span of the widest streamed (batch, head) slice
-  const int64_t span = 2 * std::max(std::max((int64_t)a.T * a.sk.t, (int64_t)a.T * a.sv.t),
-                                    std::max((int64_t)a.T * a.L * a.skd.t, (int64_t)a.T * a.L * a.svd.t));
-  const bool wide = span > 0x7fffffffll;
+  const bool wide = !narrow_slices(a);
   const bool small = a.cu ? use_small_rows(a.delta_pitch, a.Hq, a.compute_units)  // the rows there are, not those of the grid
                           : use_small_rows(a.Tq, (long long)a.B * a.Hq, a.compute_units);
   switch ((wide ? 1 : 0) | (a.cu ? 2 : 0) | (a.L == 0 ? 4 : 0) | (a.L > 0 && a.Lv != a.L ? 8 : 0)) {

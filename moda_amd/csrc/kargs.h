@@ -58,7 +58,8 @@ __host__ __device__ __forceinline__ int part_rows(const KArgs& a) { return a.cu 
 
 // Variable-length batches: rebases every tensor on the first row of sequence `b` and shrinks T / Tq to the
 // sequence's length, so that the code after it addresses the sequence as batch 0 of a fixed-length problem.
-// The launch grid is sized for the longest sequence: callers drop the tiles beyond their own sequence.
+// Launches sized for the longest sequence drop the tiles beyond their own; those that take their tiles from a list
+// (geometry.h: packed_tile) have none.
 // `units`: 16-bit units per tensor element (the data pointers are typed for 16-bit elements).
 __host__ __device__ __forceinline__ void enter_sequence_at(KArgs& a, int t0, int T, int units) {
   const int64_t r0 = (int64_t)t0 * a.Gf * units, c0 = (int64_t)t0 * a.L * units, k0 = (int64_t)t0 * units;

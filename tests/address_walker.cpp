@@ -1212,11 +1212,7 @@ void walk_slot(int64_t B, int64_t T, int64_t H, int64_t D, int64_t L, int64_t sl
 
 template <int HD>
 void walk_all(const Case& c, const KArgs& a) {
-  // byte span of the widest streamed (batch, head) slice decides the addressing variant (as the launchers do)
-  const int64_t span = 2 * std::max(std::max((int64_t)a.T * a.sk.t, (int64_t)a.T * a.sv.t),
-                                    std::max((int64_t)a.T * a.L * a.skd.t, (int64_t)a.T * a.L * a.svd.t));
-  const bool wide_addr = span > 0x7fffffffll;
-  if (wide_addr) fail("slices beyond 2 GiB are not walked (the fake tensors would not fit the walker's write maps)");
+  if (!narrow_slices(a)) fail("slices beyond 2 GiB are not walked (the fake tensors would not fit the walker's write maps)");
   const bool small = a.cu ? use_small_rows(a.delta_pitch, a.Hq, a.compute_units) : use_small_rows(a.Tq, (long long)a.B * a.Hq, a.compute_units);
   const ShortRows rows = a.cu ? ShortRows::kNone : pick_short_rows(a.Tq, (long long)a.B * a.Hq, a.causal, a.compute_units);
   // ---- forward
