@@ -1,5 +1,6 @@
 // Device-side pieces shared by the dense kernels of a transformer block (block_kernels.hip, block_tail_kernel.hip).
 #pragma once
+#include "geometry.h"
 #include "tile.h"
 
 namespace moda {
@@ -20,6 +21,22 @@ __device__ __forceinline__ float gelu(float x) {
   r = __builtin_fmaf(r, t, 0.108287916f);
   r = __builtin_fmaf(r, t, 0.107143715f);
   return (x - __builtin_amdgcn_fmed3f(x, kNegInf, 0.f)) - a * t * r * fast_exp2(a * a * (-0.5f * kLog2e));
+}
+
+// Rows of W 16-bit elements in LDS, 16-byte chunks swizzled as Tile<> has them for rows of 256 bytes and more.
+template <int W>
+struct RowLayout {
+  static constexpr int kWidth = W;
+  static_assert(W % 128 == 0, "rows start at bank 0");
+  MODA_HD static int swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+  MODA_HD static int off(int row, int chunk) { return row * W + ((chunk ^ swz(row)) << 3); }
+};
+
+// Packed weights: blocks of 16 features, per block the steps of 32 of the sum, per step (`item`: block * steps + step) the 16
+// bytes of each lane of a wave.  First element of a lane's piece there, and of the same piece in the weight [n][32 * steps].
+MODA_HD int64_t packed_piece(int64_t item, int lane) { return (item * 64 + lane) * 8; }
+MODA_HD int64_t weight_piece(int block, int step, int steps, int lane) {
+  return ((int64_t)(block * 16 + (lane & 15)) * steps + step) * 32 + (lane >> 4) * 8;
 }
 
 }  // namespace moda

@@ -114,12 +114,8 @@ __device__ __forceinline__ float row_sum(const float (&s)[NL]) {
   return v;
 }
 
-// Rows of W 16-bit elements in LDS, 16-byte chunks swizzled as Tile<> has them for rows of 256 bytes and more.
 template <int W>
-struct Rows {
-  static_assert(W % 128 == 0, "rows start at bank 0");
-  __device__ __forceinline__ static int swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
-  __device__ __forceinline__ static int off(int row, int chunk) { return row * W + ((chunk ^ swz(row)) << 3); }
+struct Rows : RowLayout<W> {
   // B operand of rows row0 + sigma(0..15), features 32 ks .. +31 (see Operand16); base: off(sigma(n), q4 + 4 j) for j = 0..3
   __device__ __forceinline__ static i32x4 operand(lds_cptr tile, const int (&base)[4], int row0, int ks) {
     return *reinterpret_cast<MODA_LDS const i32x4*>(tile + base[ks & 3] + row0 * W + (ks >> 2) * 128);
@@ -495,8 +491,8 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(const PackArgs a) {
   const int lane = threadIdx.x & 63, item = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (item >= m.blocks * m.steps) return;
   const int blk = item / m.steps, ks = item - blk * m.steps;
-  const i32x4 v = *reinterpret_cast<const i32x4*>(m.w + ((int64_t)(blk * 16 + (lane & 15)) * m.steps + ks) * 32 + (lane >> 4) * 8);
-  *reinterpret_cast<i32x4*>(m.to + ((int64_t)item * 64 + lane) * 8) = v;
+  const i32x4 v = *reinterpret_cast<const i32x4*>(m.w + weight_piece(blk, ks, m.steps, lane));
+  *reinterpret_cast<i32x4*>(m.to + packed_piece(item, lane)) = v;
 }
 
 namespace {

@@ -25,6 +25,7 @@
 //   without data alone and adds slot Lv of the depth gradients to dk, dv; instead of a walk, WALKER_ORDER=1 prints
 //   the order of a packed batch's launches, WALKER_ROUTE=1 whether a backward pass is one launch.
 // usage: address_walker linear rows K gelu n0 [n1 n2]   |   norm rows dim   |   slot B T H D L slot wide to_cache
+//   |   tail bf16|fp16 rows width hidden post_norm [n0 [n1 [n2]]]   |   pack matrices
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -36,6 +37,8 @@
 #include <string>
 #include <vector>
 
+#include "../include/moda_hip.h"
+#include "../moda_amd/csrc/block.h"
 #include "../moda_amd/csrc/geometry.h"
 #include "../moda_amd/csrc/kargs.h"
 #include "../moda_amd/csrc/tile.h"
@@ -1189,6 +1192,181 @@ void walk_norm(int rows, int dim) {
   require_full("y");
 }
 
+// A block's dense part in one launch: rows in and out, every product's weights, biases, norms and parts; what LDS holds.
+// Weights are read through their packed copies, each piece against the order that pack_weights_kernel leaves.
+template <int C, int NB>
+void walk_tail_of(bool fp16, int rows, int hidden, bool post, const std::vector<int>& parts) {
+  constexpr int BM = 16 * NB, MB2 = C / 128, MB1 = 2, HC = 256, CH = C / 8, TPR = 512 / BM, NL = CH / TPR;
+  const uint32_t table = fp16 ? 0 : MODA_HIP_GELU_TABLE_BYTES, X = table / 2, H = X + BM * C;  // elements
+  const uint32_t lds_bytes = table + (uint32_t)BM * (C + std::max(C, 2 * HC)) * 2;
+  int idx = 0;
+  const auto region2 = [&](const char* name, int64_t n, bool track = false) { return add_region(name, idx++, n * 2, 2, track); };
+  const uint16_t *h = region2("attention", (int64_t)rows * C), *res = region2("residual", (int64_t)rows * C), *x = region2("x", (int64_t)rows * C, true);
+  const uint16_t *proj_w = region2("proj_w", C * C), *proj_b = region2("proj_b", C), *fc1_w = region2("fc1_w", (int64_t)hidden * C);
+  const uint16_t *fc1_b = region2("fc1_b", hidden), *fc2_w = region2("fc2_w", (int64_t)hidden * C), *fc2_b = region2("fc2_b", C);
+  const uint16_t *mid_w = region2("mid_w", C), *mid_b = region2("mid_b", C), *end_w = region2("end_w", C), *end_b = region2("end_b", C);
+  const uint16_t* gelu_table = region2("gelu_table", table / 2);
+  std::vector<const uint16_t*> w, bias, y;
+  std::vector<int> end;
+  std::vector<std::string> wn, bn, yn;
+  for (size_t i = 0; i < parts.size(); i++) {
+    const std::string k = std::to_string(i);
+    wn.push_back("w" + k);
+    bn.push_back("bias" + k);
+    yn.push_back("y" + k);
+    w.push_back(region2(wn[i].c_str(), (int64_t)parts[i] * C));
+    bias.push_back(region2(bn[i].c_str(), parts[i]));
+    y.push_back(region2(yn[i].c_str(), (int64_t)(rows - 1) * (parts[i] + 8) + parts[i], true));
+    end.push_back((end.empty() ? 0 : end.back()) + parts[i] / 16);
+  }
+  const auto lds = [&](uint32_t first, int64_t off, int elems, uint32_t limit, const char* what) {  // [first, limit) elements
+    if (off < 0 || first + off + elems > limit || limit * 2 > lds_bytes) fail("%s at element %lld of LDS", what, (long long)off);
+  };
+  const int nblk = (rows + BM - 1) / BM;
+  for (int block = 0; block < nblk; block++)
+    for (int tid = 0; tid < 512; tid++) {
+      const int lane = tid & 63, n = lane & 15, q4 = lane >> 4, wave = tid >> 6, r0 = block * BM, sigma = slot_base(n >> 2) + (n & 3);
+      const int f2 = wave * 16 * MB2, lrow = tid / TPR, lsub = tid % TPR;
+      const uint32_t all = lds_bytes / 2;
+      // one product: `mb` blocks of 16 features from f on (packed [features][width]), steps first .. first + nk - 1 of 32
+      const auto product = [&](const char* name, const uint16_t* packed, int f, int mbs, int width, int first, int nk, int ahead) {
+        ctx("block_tail_kernel", block, wave, lane, name);
+        if (nk % 4 || ahead > nk) fail("%d steps", nk);
+        for (int mb = 0; mb < mbs; mb++)
+          for (int ks = 0; ks < nk; ks++) {
+            const char* at = (const char*)(packed + (size_t)(f + 16 * mb) * width + first * 512) + lane * 16 + (size_t)ks * 1024;
+            if (at != (const char*)(packed + packed_piece((int64_t)((f + 16 * mb) / 16) * (width / 32) + first + ks, lane))) fail("a piece that is not where it was packed");
+            check_access(name, at, 16, false);
+          }
+      };
+      const auto operand = [&](auto layout, uint32_t base, uint32_t limit, int nk) {
+        typedef decltype(layout) L;
+        for (int ks = 0; ks < nk; ks++)
+          for (int nb = 0; nb < NB; nb++)
+            lds(base, L::off(sigma, 4 * (ks & 3) + q4) + 16 * nb * L::kWidth + (ks >> 2) * 128, 8, limit, "row operand");
+      };
+      const auto pieces = [&](const char* name, const uint16_t* b, int f, int mbs) {
+        for (int mb = 0; mb < mbs; mb++) check_access(name, b + f + 16 * mb + 4 * q4, 8, false);
+      };
+      const auto norm = [&](const char* wn, const uint16_t* weight, const char* bn, const uint16_t* b, bool normalise, bool store) {
+        ctx("block_tail_kernel", block, wave, lane, "layer norm");
+        for (int j = 0; j < NL; j++) {
+          lds(X, RowLayout<C>::off(lrow, lsub + TPR * j), 8, H, "row");
+          if (normalise) {
+            check_access(wn, weight + (lsub + TPR * j) * 8, 16, false);
+            check_access(bn, b + (lsub + TPR * j) * 8, 16, false);
+          }
+          if (store && r0 + lrow < rows) check_access("x", x + (int64_t)(r0 + lrow) * C + (lsub + TPR * j) * 8, 16, true);
+        }
+      };
+      ctx("block_tail_kernel", block, wave, lane, "rows in");
+      for (int j = 0; j < BM * CH / 512; j++) {
+        const int at = (tid + 512 * j) / CH, row = std::min(r0 + at, rows - 1), ch = (tid + 512 * j) % CH;
+        check_access("attention", h + (int64_t)row * C + ch * 8, 16, false);
+        check_access("residual", res + (int64_t)row * C + ch * 8, 16, false);
+        lds(X, RowLayout<C>::off(at, ch), 8, H, "residual row");
+        lds(H, RowLayout<C>::off(at, ch), 8, all, "attention row");
+      }
+      const int nt = table / 16;
+      for (int j = 0; j < (nt + 511) / 512; j++) check_access("gelu_table", gelu_table + (tid + 512 * j < nt ? tid + 512 * j : 0) * 8, 16, false);
+      product("proj_w", proj_w, f2, MB2, C, 0, C / 32, MB2 <= 3 ? 4 : 2);
+      operand(RowLayout<C>{}, H, all, C / 32);
+      pieces("proj_b", proj_b, f2, MB2);
+      for (int mb = 0; mb < MB2; mb++)
+        for (int nb = 0; nb < NB; nb++) lds(X, RowLayout<C>::off(sigma, (f2 >> 3) + 2 * mb + (q4 >> 1)) + 4 * (q4 & 1) + 16 * nb * C, 4, H, "own piece");
+      norm("mid_w", mid_w, "mid_b", mid_b, true, false);
+      for (int c0 = 0, stage = 0; c0 < hidden; c0 += HC, stage ^= 1) {
+        const int f1 = c0 + wave * 16 * MB1, left = std::min(hidden - c0, HC);
+        const uint32_t Hs = H + stage * BM * HC, Hs_end = Hs + BM * HC;
+        if (f1 < hidden) {
+          product("fc1_w", fc1_w, f1, MB1, C, 0, C / 32, 4);
+          operand(RowLayout<C>{}, X, H, C / 32);
+          pieces("fc1_b", fc1_b, f1, MB1);
+          for (int mb = 0; mb < MB1; mb++)
+            for (int nb = 0; nb < NB; nb++)
+              lds(Hs, RowLayout<HC>::off(sigma, wave * 2 * MB1 + 2 * mb + (q4 >> 1)) + 4 * (q4 & 1) + 16 * nb * HC, 4, Hs_end, "hidden piece");
+        }
+        product("fc2_w", fc2_w, f2, MB2, hidden, c0 / 32, left / 32, MB2 <= 3 ? 4 : 2);
+        operand(RowLayout<HC>{}, Hs, Hs_end, left / 32);
+      }
+      pieces("fc2_b", fc2_b, f2, MB2);
+      norm("end_w", end_w, "end_b", end_b, post || !parts.empty(), true);
+      if (parts.empty()) continue;
+      const int blocks = end.back();
+      const auto projections = [&](auto side_by_side) {
+        constexpr int MBQ = decltype(side_by_side)::value, W = 128 * MBQ;
+        for (int first = 0; first < blocks; first += 8 * MBQ) {
+          for (int mb = 0; mb < MBQ; mb++) {
+            const int blk = std::min(first + wave * MBQ + mb, blocks - 1);
+            size_t pi = 0;
+            while (blk >= end[pi]) pi++;
+            const int f = 16 * (blk - (pi ? end[pi - 1] : 0));
+            product(wn[pi].c_str(), w[pi], f, 1, C, 0, C / 32, MBQ <= 3 ? 4 : 2);
+            pieces(bn[pi].c_str(), bias[pi], f, 1);
+            for (int nb = 0; nb < NB; nb++)
+              lds(H, RowLayout<W>::off(sigma, 2 * (wave * MBQ + mb) + (q4 >> 1)) + 4 * (q4 & 1) + 16 * nb * W, 4, all, "projected piece");
+          }
+          ctx("block_tail_kernel", block, wave, lane, "projected rows out");
+          const int chunks = 2 * std::min(blocks - first, 8 * MBQ);
+          for (int ch = lsub; ch < chunks && r0 + lrow < rows; ch += TPR) {
+            const int blk = first + (ch >> 1);
+            size_t pi = 0;
+            while (blk >= end[pi]) pi++;
+            lds(H, RowLayout<W>::off(lrow, ch), 8, all, "projected row");
+            check_access(yn[pi].c_str(), y[pi] + (int64_t)(r0 + lrow) * (parts[pi] + 8) + 8 * (2 * first + ch) - (pi ? 16 * end[pi - 1] : 0), 16, true);
+          }
+        }
+      };
+      if (blocks <= 16)
+        projections(std::integral_constant<int, 2>{});
+      else if (blocks <= 24)
+        projections(std::integral_constant<int, 3>{});
+      else
+        projections(std::integral_constant<int, 4>{});
+    }
+  require_full("x");
+  for (size_t i = 0; i < parts.size(); i++) {
+    Region& r = region(("y" + std::to_string(i)).c_str());
+    for (size_t u = 0; r.track && u < r.writes.size(); u++) {
+      const int want = (int)(u % (size_t)(parts[i] + 8)) < parts[i] ? 1 : 0;
+      if (r.writes[u] != want) fail("%s unit %zu written %d times, not %d", r.name.c_str(), u, (int)r.writes[u], want);
+    }
+  }
+}
+void walk_tail(bool fp16, int rows, int width, int hidden, bool post, const std::vector<int>& parts) {
+  const auto go = [&](auto c) {
+    constexpr int C = decltype(c)::value;
+    block_tail_rows(rows, 256) == 32 ? walk_tail_of<C, 2>(fp16, rows, hidden, post, parts) : walk_tail_of<C, 4>(fp16, rows, hidden, post, parts);
+  };
+  switch (width) {
+    case 128: return go(std::integral_constant<int, 128>{});
+    case 256: return go(std::integral_constant<int, 256>{});
+    case 384: return go(std::integral_constant<int, 384>{});
+    default: return go(std::integral_constant<int, 512>{});
+  }
+}
+
+// weights [n][k] into their packed order: matrices of alternating sizes, as many as given
+void walk_pack(int matrices) {
+  const int sizes[3][2] = {{16, 32}, {48, 128}, {128, 96}};
+  int64_t most = 0;
+  for (const auto& s : sizes) most = std::max(most, (int64_t)(s[0] / 16) * (s[1] / 32));
+  for (int m = 0; m < matrices; m++) {
+    const int n = sizes[m % 3][0], k = sizes[m % 3][1], blocks = n / 16, steps = k / 32;
+    const uint16_t *from = add_region("w", 0, (int64_t)n * k * 2, 2, true), *to = add_region("packed", 1, (int64_t)n * k * 2, 2, true);
+    for (int block = 0; block < (most + 3) / 4; block++)
+      for (int tid = 0; tid < 256; tid++) {
+        const int lane = tid & 63, item = block * 4 + (tid >> 6);
+        if (item >= blocks * steps) continue;
+        ctx("pack_weights_kernel", block, tid >> 6, lane, "piece");
+        check_access("w", from + weight_piece(item / steps, item % steps, steps, lane), 16, true);  // (read, each element once)
+        check_access("packed", to + packed_piece(item, lane), 16, true);
+      }
+    require_full("w");
+    require_full("packed");
+  }
+}
+
 // one layer's K and V (views of one projection: rows 2 H D + 8 elements apart) against slot `slot` of the caches
 void walk_slot(int64_t B, int64_t T, int64_t H, int64_t D, int64_t L, int64_t slot, bool wide, bool to_cache) {
   const int64_t st = 2 * H * D + 8, sb = T * st, piece = wide ? 16 : 2, per_row = D * 2 / piece, units = B * T * H * per_row;
@@ -1336,6 +1514,18 @@ int main(int argc, char** argv) {
   if (what == "tail_rule") {  // dtype rows width hidden kv compute_units
     printf("%s, %d rows\n", block_tail_pays(std::string(argv[2]) == "fp16", arg(3), arg(4), arg(5), arg(6), arg(7)) ? "one launch" : "pieces",
            block_tail_rows(arg(3), arg(7)));
+    return 0;
+  }
+  if (what == "tail") {  // dtype rows width hidden post_norm n0 [n1 n2]
+    std::vector<int> parts;
+    for (int i = 7; i < argc; i++) parts.push_back(arg(i));
+    walk_tail(std::string(argv[2]) == "fp16", arg(3), arg(4), arg(5), arg(6) != 0, parts);
+    printf("OK checked=%lld\n", g_checked);
+    return 0;
+  }
+  if (what == "pack") {
+    walk_pack(arg(2));
+    printf("OK checked=%lld\n", g_checked);
     return 0;
   }
   if (what == "linear" || what == "norm" || what == "slot") {

@@ -5,8 +5,8 @@ kernels' own index arithmetic (``moda_amd/csrc/geometry.h``, ``kargs.h``, ``tile
 and walks every (workgroup, wave, lane, trip) of a forward + backward launch: register operand loads, every tile
 descriptor with each lane's vector and scalar offset (the lanes that fetch past the tensors' head dim included),
 the row-statistics loads, the LDS targets against the launch's dynamic LDS size, and all stores; every output
-element must be written exactly once.  The fp32 matrix kernels, the linear, layer-norm and depth-slot kernels are walked
-the same way.
+element must be written exactly once.  The fp32 matrix kernels, the launches that dQ and dK/dV share, the linear, layer-norm and
+depth-slot kernels, a stack's block tail and the packing of its weights are walked the same way.
 
 The first case is the packed batch that once ended in a GPU memory fault on the packed instantiations of the
 256-wide kernels (switched off since).  The walk finds every access of it inside its tensor: the fault is not an
@@ -329,6 +329,30 @@ def test_dense_and_slot_kernels(walker, case):
         r = subprocess.run([walker, *map(str, args)], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, env=e, timeout=600)
         out = r.stdout + r.stderr
         assert r.returncode == want and out.startswith(chosen) and ("VIOLATION" if want else "OK checked") in out, out
+
+
+@pytest.mark.parametrize("case", [
+    # dtype, rows, width, hidden, post-norm, features of each part: 32 rows a workgroup and 64, a last chunk of the hidden
+    # width that leaves waves without features, 2, 3 and 4 feature blocks a wave, more than one turn, no part
+    ("bf16", 1, 128, 128, 0, 128, 16, 16),
+    ("bf16", 45, 256, 640, 1, 256, 64, 64),
+    ("fp16", 8195, 128, 384, 0, 128),
+    ("bf16", 8251, 256, 256, 0, 256, 128, 128),
+    ("bf16", 8200, 384, 128, 1, 384, 16),
+    ("bf16", 70, 512, 1024, 1),
+    ("fp16", 8193, 512, 256, 0, 512, 128, 128),
+], ids=lambda c: "-".join(map(str, c)))
+def test_block_tail(walker, case):
+    cuts = [None, "x:2", "attention:2", "residual:2", "fc2_w:2", "end_b:2" if case[4] or len(case) > 5 else "mid_b:2"]
+    for shrink in cuts + (["y0:2", f"w{len(case) - 6}:2", "bias0:2"] if len(case) > 5 else []) + (["gelu_table:2"] if case[0] == "bf16" else []):
+        e = dict(os.environ, **({"WALKER_SHRINK": shrink} if shrink else {}))
+        out = subprocess.run([walker, "tail", *map(str, case)], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=e, timeout=600)
+        assert out.returncode == (1 if shrink else 0) and ("VIOLATION" if shrink else "OK checked") in out.stdout, (shrink, out.stdout)
+
+
+def test_packed_weights(walker):
+    out = subprocess.run([walker, "pack", "7"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=600)
+    assert out.returncode == 0 and "OK checked" in out.stdout, out.stdout
 
 
 @pytest.mark.parametrize("case", [

@@ -600,6 +600,68 @@ def test_dense_entry_points_refuse_what_their_kernels_cannot_take():
         assert norm(**bad) == -3, bad
 
 
+def test_block_tail_and_weight_packing_refuse_what_their_kernels_cannot_take():
+    """Codes of moda_hip_block_tail and moda_hip_pack_weights, all returned before a device is looked at (nothing is read)."""
+    from moda_amd import _lib
+
+    lib = _lib.load()
+    i32, i64, ptr = ctypes.c_int32, ctypes.c_int64, ctypes.c_void_p
+    biases, pointers = ("proj_b", "fc1_b", "fc2_b"), ("attention", "residual", "x", "proj_w", "fc1_w", "fc2_w", "mid_norm_w", "mid_norm_b")
+
+    class Part(ctypes.Structure):
+        _fields_ = [("w", ptr), ("bias", ptr), ("y", ptr), ("ldy", i64), ("n", i64)]
+
+    class Tail(ctypes.Structure):
+        _fields_ = [("struct_size", i32), ("dtype", i32), ("rows", i64), ("width", i64), ("hidden", i64), ("attention", ptr),
+                    ("residual", ptr), ("x", ptr), ("proj_w", ptr), ("proj_b", ptr), ("fc1_w", ptr), ("fc1_b", ptr), ("fc2_w", ptr),
+                    ("fc2_b", ptr), ("mid_norm_w", ptr), ("mid_norm_b", ptr), ("end_norm_w", ptr), ("end_norm_b", ptr),
+                    ("gelu_table", ptr), ("mid_norm_eps", ctypes.c_float), ("end_norm_eps", ctypes.c_float), ("post_norm", i32),
+                    ("n_parts", i32), ("parts", Part * 3)]
+
+    class Weight(ctypes.Structure):
+        _fields_ = [("w", ptr), ("packed", ptr), ("n", i64), ("k", i64)]
+
+    def tail(**given):
+        v = dict(struct_size=ctypes.sizeof(Tail), dtype=0, rows=4, width=256, hidden=1024, post_norm=0, n_parts=1, gelu_table=0x1000,
+                 end_norm_w=0x1000, end_norm_b=0x1000, **{n: 0x1000 for n in pointers + biases})
+        part = dict(w=0x2000, bias=0x3000, y=0x4000, ldy=64, n=64)
+        part.update({n: given.pop("part_" + n) for n in list(part) if "part_" + n in given})
+        t = Tail(**{**v, **given})
+        for i in range(3):
+            t.parts[i] = Part(*(part[n] for n in ("w", "bias", "y", "ldy", "n")))
+        return lib.moda_hip_block_tail(ctypes.byref(t), None)
+
+    def pack(n=1, table=0x1000, **given):
+        w = dict(w=0x2000, packed=0x3000, n=32, k=64)
+        w.update({f: given[f] for f in w if f in given})
+        if "rows" in given:
+            w["n"] = given["rows"]
+        return lib.moda_hip_pack_weights((Weight * 2)(*(Weight(w["w"], w["packed"], w["n"], w["k"]) for _ in range(2))), n, ptr(table), None)
+
+    assert tail(rows=0) == 0 and lib.moda_hip_block_tail(None, None) == -1 and lib.moda_hip_pack_weights(None, 1, None, None) == -1
+    for bad in (dict(struct_size=8), dict(dtype=2), dict(rows=-1), dict(width=0), dict(hidden=0), dict(n_parts=-1), dict(n_parts=4),
+                dict(gelu_table=None), dict(end_norm_w=None), dict(end_norm_b=None), dict(n_parts=0, post_norm=1, end_norm_w=None),
+                dict(part_w=None), dict(part_y=None), dict(part_n=0), *({n: None} for n in pointers)):
+        assert tail(**bad) == -1, bad
+    for bad in (dict(width=64), dict(width=640), dict(hidden=64), dict(hidden=1 << 20), dict(rows=1 << 30), dict(part_n=40), dict(part_n=1 << 20)):
+        assert tail(**bad) == -2, bad
+    for bad in (dict(gelu_table=0x1008), dict(end_norm_w=0x1008), dict(part_w=0x2008), dict(part_y=0x4008), dict(part_ldy=68),
+                dict(part_bias=0x3004), *({n: 0x1008} for n in pointers), *({n: 0x1004} for n in biases)):
+        assert tail(**bad) == -3, bad
+    for bad in (dict(n=0), dict(w=None), dict(packed=None), dict(rows=0), dict(k=0)):
+        assert pack(**bad) == -1, bad
+    for bad in (dict(rows=24), dict(k=48), dict(rows=1 << 20), dict(k=1 << 20), dict(rows=1 << 16, k=1 << 15)):
+        assert pack(**bad) == -2, bad
+    for bad in (dict(table=0x1008), dict(w=0x2008), dict(packed=0x3008)):
+        assert pack(**bad) == -3, bad
+    # what need not be there is not asked for: no parts and no norm behind them, no biases, no table in fp16; here no device
+    # either, which is the next thing to be looked at
+    fine = (dict(n_parts=0, end_norm_w=None, end_norm_b=None), dict(proj_b=None, fc1_b=None, fc2_b=None, part_bias=None),
+            dict(dtype=1, gelu_table=None))
+    if not torch.cuda.is_available():
+        assert [tail(**f) for f in fine] == [pack(table=None)] * 3 and pack() not in (0, -1, -2, -3)
+
+
 @pytest.mark.parametrize("way", ["forward hook", "forward pre-hook", "global hook", "dropout", "replaced activation", "tanh GELU",
                                  "derived linear", "patched forward", "derived attention", "swapped parameter", "blocks that differ",
                                  "another scale", "autocast", "gradients", "derived tensor", "rebuilt cache"])

@@ -2074,6 +2074,7 @@ def test_linear_against_fp64(gpu_device, case, dtype):
 class _BlockTail:
     """moda_hip_pack_weights + moda_hip_block_tail through the C entry points, on random weights (or those given)."""
 
+    TABLE = 21504 // 4  # floats of MODA_HIP_GELU_TABLE_BYTES
     NAMES = ("proj_w", "proj_b", "fc1_w", "fc1_b", "fc2_w", "fc2_b", "mid_w", "mid_b", "end_w", "end_b")
 
     def __init__(self, width, hidden, parts, dtype, device, seed=0, **given):
@@ -2095,7 +2096,7 @@ class _BlockTail:
             _fields_ = [("w", ptr), ("packed", ptr), ("n", i64), ("k", i64)]
 
         ws = [self.w["proj_w"], self.w["fc1_w"], self.w["fc2_w"]] + [w for w, _ in self.parts]
-        self.packed, self.table = [torch.empty_like(w) for w in ws], torch.empty(21504 // 4, device=device)
+        self.packed, self.table = [torch.empty_like(w) for w in ws], torch.empty(self.TABLE, device=device)
         arr = (Weight * len(ws))(*(Weight(w.data_ptr(), p.data_ptr(), *w.shape) for w, p in zip(ws, self.packed)))
         assert self.lib.moda_hip_pack_weights(arr, len(ws), ptr(self.table.data_ptr()), ptr(torch.cuda.current_stream().cuda_stream)) == 0
 
@@ -2216,6 +2217,87 @@ def test_block_tail_equals_its_pieces_bitwise(gpu_device, case, post_norm, dtype
     assert torch.equal(x, z if post_norm else y), (x != (z if post_norm else y)).float().mean()
     for (w, b), got in zip(t.parts, ys):
         assert torch.equal(got[:rows, :w.shape[0]], lin(z, w, b))
+
+
+@pytest.mark.parametrize("n", [96, 97, 200])
+def test_weights_beyond_one_packing_launch(gpu_device, n):
+    """96 matrices go in a launch; each ends up in the order of the operands, and the table is filled once, by the first."""
+    import ctypes
+
+    from moda_amd import _lib
+
+    class Weight(ctypes.Structure):
+        _fields_ = [("w", ctypes.c_void_p), ("packed", ctypes.c_void_p), ("n", ctypes.c_int64), ("k", ctypes.c_int64)]
+
+    gen = torch.Generator(device=gpu_device).manual_seed(n)
+    ws = [torch.randn(16 * (1 + i % 3), 32 * (1 + i % 5), generator=gen, device=gpu_device).bfloat16() for i in range(n)]
+    packed = [torch.full_like(w, 7.0) for w in ws]
+    table = torch.full((_BlockTail.TABLE + 8,), 7.0, device=gpu_device)
+    arr = (Weight * n)(*(Weight(w.data_ptr(), p.data_ptr(), *w.shape) for w, p in zip(ws, packed)))
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert _lib.load().moda_hip_pack_weights(arr, n, ctypes.c_void_p(table.data_ptr()), stream) == 0
+    for w, p in zip(ws, packed):
+        r, k = w.shape
+        # [block, feature, step, quarter, 8] -> [block, step, quarter, feature, 8]
+        assert torch.equal(p.flatten(), w.view(r // 16, 16, k // 32, 4, 8).permute(0, 2, 3, 1, 4).flatten())
+    assert (table[:_BlockTail.TABLE] != 7.0).all() and (table[_BlockTail.TABLE:] == 7.0).all()
+
+
+@pytest.mark.parametrize("case", [
+    # width, blocks, batch, tokens, post-norm, dtype: 64 rows a workgroup (more than 8192 rows); more matrices than one packing
+    # launch takes (five a block, without the first block's two)
+    (128, 2, 43, 197, False, torch.bfloat16),
+    (256, 2, 64, 145, True, torch.float16),
+    (128, 24, 2, 50, False, torch.bfloat16),
+], ids=str)
+def test_stack_of_block_tails_equals_its_pieces(gpu_device, case):
+    """Stacks that take the one launch a block, against moda_hip_linear, moda_hip_layer_norm and the attention operator called
+    one by one as such a stack calls its pieces: the same bits."""
+    import ctypes
+
+    import moda_amd
+    from moda_amd import _lib
+
+    C, n, B, N, post, dtype = case
+    say(f"CASE stack of block tails {case}")
+    torch.manual_seed(3)
+    heads = C // 64
+    m = moda_amd.MoDAStack(C, n, heads, 1, mlp_ratio=2.0, post_norm=post).to(gpu_device, dtype).eval().requires_grad_(False)
+    x = (0.5 * torch.randn(B, N, C, device=gpu_device)).to(dtype)
+    with torch.no_grad():
+        got = m._forward_native(x)
+    assert got is not None
+
+    def lin(v, layer, residual=None, gelu=False):
+        v = v.reshape(-1, v.shape[-1])
+        y = torch.empty(v.shape[0], layer.weight.shape[0], dtype=dtype, device=gpu_device)
+        assert _linear(v, [(layer.weight, layer.bias, y)], residual, gelu) == 0
+        return y
+
+    def norm(v, layer):
+        y = torch.empty_like(v)
+        p, i = (lambda t: ctypes.c_void_p(t.data_ptr())), ctypes.c_int64
+        assert _lib.load().moda_hip_layer_norm({torch.bfloat16: 0, torch.float16: 1}[dtype], i(v.shape[0]), i(C), p(v), p(layer.weight), p(layer.bias),
+                                               ctypes.c_float(layer.eps), p(y), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        return y
+
+    kd = vd = None
+    z, keys, values = x.reshape(-1, C), [], []
+    for blk in m.blocks:
+        h = z if post else norm(z, blk.norm1)
+        q, kv = lin(h, blk.attn.q), lin(h, blk.attn.kv)
+        k, v = kv[:, :64].reshape(B, N, 1, 64).contiguous(), kv[:, 64:].reshape(B, N, 1, 64).contiguous()
+        if keys:
+            kd, vd = (torch.stack(t, dim=2).reshape(B, -1, 1, 64) for t in (keys, values))
+        a = moda_amd.parallel_moda(q.reshape(B, N * heads, 1, 64), k, v, cached_k=kd, cached_v=vd, moda_group_num=heads, is_causal=False)
+        keys.append(k)
+        values.append(v)
+        y = lin(a.reshape(-1, C), blk.attn.proj, z)
+        t = norm(y, blk.norm1 if post else blk.norm2)
+        y = t if post else y
+        z = lin(lin(t, blk.mlp[0], gelu=True), blk.mlp[2], y)
+        z = norm(z, blk.norm2) if post else z
+    assert torch.equal(got.reshape(-1, C), z), ((got.reshape(-1, C) != z).float().mean().item(), (got.reshape(-1, C) - z).abs().max().item())
 
 
 def test_block_tail_gelu_of_every_bf16_value(gpu_device):
