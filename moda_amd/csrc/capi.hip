@@ -465,11 +465,16 @@ int moda_hip_bwd_stages(const moda_hip_desc* d, const void* q, const void* k, co
   a.sdvd = cvt(d->dvd);
   hipStream_t s = (hipStream_t)stream;
   hipError_t e = hipSuccess;
+  // Launches one after the other let dk, dv take the place of k, v (a dK/dV workgroup reads its own rows of them first, and the
+  // dQ launch is done) and dq that of o; side by side they would overwrite what the other half still reads.
+  bool in_place = false;
+  for (const void* out : {dq, dk, dv})
+    for (const void* in : {q, k, v, o, d_o}) in_place = in_place || (out && out == in);
   if (use_mfma(d)) {
     // with both stages asked for, the dQ kernel forms the row sums itself (one launch and one pass over o, do less)
     a.own_delta = (stages & MODA_HIP_STAGE_DELTA) && (stages & MODA_HIP_STAGE_DQ) ? 1 : 0;
     if ((stages & MODA_HIP_STAGE_DELTA) && !a.own_delta) e = moda::launch_delta(a, d->dtype, tile_width(d), s);
-    if ((stages & MODA_HIP_STAGE_DKV) && moda::bwd_one_launch(a, tile_width(d))) {
+    if ((stages & MODA_HIP_STAGE_DKV) && !in_place && moda::bwd_one_launch(a, tile_width(d))) {
       e = moda::launch_bwd_short(a, d->dtype, s);
       a.seq_done = 1;
     } else if (e == hipSuccess && (stages & MODA_HIP_STAGE_DQ)) {
@@ -479,12 +484,12 @@ int moda_hip_bwd_stages(const moda_hip_desc* d, const void* q, const void* k, co
   } else if (fp32_matrix(d, a, {{q, d->q}, {k, d->k}, {v, d->v}, {kd, d->kd}, {vd, d->vd}, {o, d->o}, {d_o, d->d_o}, {dq, d->dq},
                                 {dk, d->dk}, {dv, d->dv}, {dkd, d->dkd}, {dvd, d->dvd}})) {
     // the dQ kernel forms the row sums for the dK/dV kernel; a dK/dV stage that runs alone has them formed first
-    const bool dq = stages & MODA_HIP_STAGE_DQ, dkv = stages & MODA_HIP_STAGE_DKV;
-    if (dq && dkv && moda::fp32_one_launch(a)) {
+    const bool rows = stages & MODA_HIP_STAGE_DQ, dkv = stages & MODA_HIP_STAGE_DKV;
+    if (rows && dkv && !in_place && moda::fp32_one_launch(a)) {
       e = moda::launch_fp32(a, 4, s);
     } else {
-      if (dq) e = moda::launch_fp32(a, 1, s);
-      if (e == hipSuccess && !dq && stages) e = moda::launch_fp32(a, 3, s);
+      if (rows) e = moda::launch_fp32(a, 1, s);
+      if (e == hipSuccess && !rows && stages) e = moda::launch_fp32(a, 3, s);
       if (e == hipSuccess && dkv) e = moda::launch_fp32(a, 2, s);
     }
   } else {

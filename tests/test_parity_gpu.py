@@ -1974,6 +1974,32 @@ def test_backward_in_one_launch_with_an_infinite_last_row(gpu_device, dtype):
         assert torch.equal(x.isnan(), y.isnan()) and torch.equal(x.nan_to_num(7.0), y.nan_to_num(7.0)), name
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("case", [
+    # T, heads, query rows a token, slots: sizes whose dQ and dK/dV otherwise share a launch, and one above them
+    (1, 1, 1, 0), (95, 2, 2, 3), (130, 1, 4, 0), (1025, 2, 1, 0),
+], ids=str)
+def test_backward_into_the_buffers_of_its_inputs(gpu_device, case, dtype):
+    """dk, dv in the place of k, v, and dq in that of o: what buffers of their own receive, bit for bit."""
+    from moda_amd import _lib, ops
+
+    T, H, G, L = case
+    say(f"CASE in place {case} {dtype}")
+    gen = torch.Generator(device=gpu_device).manual_seed(T)
+    rn = lambda *s: (0.5 * torch.randn(*s, generator=gen, device=gpu_device)).to(dtype)
+    q, k, v, do = (rn(2, T * n, H, 64) for n in (G, 1, 1, G))
+    kd, vd = (rn(2, T * L, H, 64) for _ in range(2)) if L else (None, None)
+    o, lse = ops._raw_fwd(_lib.CAUSAL, q, k, v, kd, vd, 0.1, G, 0)
+    ws = ops.bwd_workspace(_lib.CAUSAL, q, k, v, kd, vd, G)
+    want = ops._raw_bwd(_lib.CAUSAL, q, k, v, kd, vd, o, lse, do, 0.1, G, 0, ws=ws)
+    k2, v2, o2 = k.clone(), v.clone(), o.clone()
+    depth = tuple(None if t is None else torch.empty_like(t) for t in (kd, vd))
+    got = ops._raw_bwd(_lib.CAUSAL, q, k2, v2, kd, vd, o2, lse, do, 0.1, G, 0, ws=ws, out=(o2, k2, v2, *depth))
+    assert got[1].data_ptr() == k2.data_ptr()
+    for name, x, y in zip(("dq", "dk", "dv", "dkd", "dvd"), got, want):
+        assert (x is None and y is None) or torch.equal(x, y), name
+
+
 def test_backward_of_long_rows_with_a_workspace_of_row_sums_alone(gpu_device):
     """More query rows than row waves take, and no room for the segments that such launches are otherwise cut into: whole
     column tiles in a launch of their own, same bits as stage by stage."""
