@@ -3,7 +3,7 @@
 // local to a row, so a workgroup takes BM rows through the whole chain; what one step hands to the next stays in
 // registers and LDS.  As separate launches (block_kernels.hip) the same rows went to memory and back six times, the
 // hidden activations of the MLP, four times as wide, among them: 12 608 rows of width 256 took 69 us in seven launches
-// (projection 9, norm 6, MLP 23 + 15, norm 6, next projections 10.5), here 32.8.
+// (projection 9, norm 6, MLP 23 + 15, norm 6, next projections 10.5), here 34.6.
 //
 // Eight waves share the BM rows and divide the features of every product.  The weights sit on the matrix instruction's A
 // side (M = features) and go from memory (L2 after the first workgroup of an XCD) straight into the registers that it
@@ -61,7 +61,8 @@ __device__ __forceinline__ void lds_barrier() {
 // GELU of a packed pair of 16-bit values.  A bf16 value has 2 x 2688 magnitudes between 2^-17 and 16, outside of which the
 // formula's result is x / 2 (to 6e-6, which no rounding to 8 bits sees), or 0 and x.  Inside, a table in LDS holds the formula's
 // result, rounded, over x: times x that is the result again to 2^-23, which rounds to itself.  8 vector instructions an element
-// where the formula (which fp16 takes) has 22, 6.5 k cycles for 64 rows x 256 features against 2.4 k (the launch 40 -> 32.7 us).
+// where the formula (which fp16 takes) has 22, 6.5 k cycles for 64 rows x 256 features against 2.4 k (the launch 40 -> 32.7 us,
+// before its sums took the order of the pieces).
 constexpr int kGeluHalf = 21 * 128, kGeluTable = 2 * kGeluHalf, kGeluFirst = (127 - 17) << 7;
 static_assert(kGeluTable * sizeof(float) == MODA_HIP_GELU_TABLE_BYTES, "what a caller allocates");
 template <typename T>
@@ -464,7 +465,7 @@ __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
 // Weights [n][k] into the order in which the products above read them: blocks of 16 features, per block the steps of 32 of
 // the sum, per step the 1 KB of a wave's A operand, lane by lane.  In their own order a wave's load touches sixteen rows in each
 // quarter of its lanes, sixteen cache lines where packed it touches two, and a compute unit takes in 13 bytes a cycle instead
-// of 64 (12 608 rows, width 256: 61 us, packed 42 at the time).  Twelve blocks are packed in one launch of 7 us.
+// of 64 (12 608 rows, width 256: 61 us, packed 42 at the time).  Twelve blocks are packed in one launch of 7.3 us.
 // The last row of workgroups fills the GELU table (see activated): bf16 values from 2^-17 to 16, then their negatives.
 constexpr int kPackMatrices = 96;
 struct PackArgs {

@@ -34,7 +34,8 @@ MODA_HD int query_tile_of(int block, int BH, int BM, int Tq_grid) { return (Tq_g
 
 // Packed order: the tiles of all sequences of a packed batch as one list, by cost level (row kernels: the tile's index;
 // dK/dV: how many column tiles lie behind it), the highest level first and the sequences that reach a level in turn; the
-// heads of a tile are neighbours in the grid.  A workgroup finds its place itself: N(j) = sum of max(0, tiles - j) counts
+// heads of a tile are neighbours in the grid.  (Cost in a causal batch; where every row sees all keys a tile costs what its
+// sequence is long, and the levels only mix the sequences.)  A workgroup finds its place itself: N(j) = sum of max(0, tiles - j) counts
 // the list's entries at level j or above, its level is the largest j with N(j) > rank.
 // What it replaces, a grid of the longest sequence for every one, launched mostly workgroups without work on unequal
 // lengths, and sent a (sequence, head) to the XCD that its index fell on (block % 8): with B * H a multiple of 8 the longest
