@@ -10,10 +10,10 @@
 // loads ahead of the math, V is read with the LDS transpose load.  Depth
 // columns are extra column tiles with a different per-row visible interval.
 //
-// Vector-ALU instructions do not overlap with MFMA on this hardware, so the
-// loop over column tiles is split in two: tiles every row of the workgroup sees
-// completely run a body without any masking or visibility tests; boundary and
-// depth tiles run the masked body.
+// The vector work of the softmax costs as much as the products (more on the
+// 64-wide tiles), so the loop over column tiles is split in two: tiles every row
+// of the workgroup sees completely run a body without any masking or visibility
+// tests; boundary and depth tiles run the masked body, 32 columns at a time.
 #include <type_traits>
 
 #include "geometry.h"
@@ -155,12 +155,17 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
   i32x4 P[4];
   TrPipe<T, HD, 4, 2> pv;
   const std::integral_constant<int, 2> two{};
+  const std::integral_constant<int, 1> one{};
   auto front = [&](auto masked, auto nblk, lds_cptr Kc, int col0, int lo, int hi, auto&& after_scores) {
     constexpr bool MASKED = decltype(masked)::value;
     constexpr int NBLK = decltype(nblk)::value;  // 32-column blocks of the tile
     f32x16 s[NBLK];
     mfma_rows<T, HD, NBLK, 4>(oa, Kc, Qr, s);
     after_scores();
+    // whether the row sees register i of block bb, a column of [lo, hi): by its distance from lo
+    const int before = col0 + 4 * g - lo;
+    const unsigned width = (unsigned)(hi > lo ? hi - lo : 0);
+    auto sees = [&](int bb, int i) { return (unsigned)(before + 32 * bb + acc_row(i, 0)) < width; };
     // row maximum of the raw scores (scale > 0, so it commutes with the max)
     float mx = kNegInf;
 #pragma unroll
@@ -168,8 +173,7 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
 #pragma unroll
       for (int i = 0; i < 16; i++) {
         if (MASKED) {
-          const int c = col0 + 32 * bb + acc_row(i, g);
-          mx = fmaxf(mx, (c >= lo && c < hi) ? s[bb][i] : kNegInf);
+          mx = fmaxf(mx, sees(bb, i) ? s[bb][i] : kNegInf);
         } else {
           mx = fmaxf(mx, s[bb][i]);
         }
@@ -195,10 +199,7 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
 #pragma unroll
       for (int i = 0; i < 16; i++) {
         float p = fast_exp2(__builtin_fmaf(s[bb][i], sc, neg_m));
-        if (MASKED) {
-          const int c = col0 + 32 * bb + acc_row(i, g);
-          p = (c >= lo && c < hi) ? p : 0.f;
-        }
+        if (MASKED) p = sees(bb, i) ? p : 0.f;
         s[bb][i] = p;
         if (i & 1)
           rs1 += p;
@@ -218,6 +219,13 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
     pv.prefetch(oa, Vc);
     pv.run(oa, Vc, P, o);
   };
+  // 32 columns, masked
+  auto half_tile = [&](lds_cptr Kc, lds_cptr Vc, int col0, int lo, int hi) {
+    TrPipe<T, HD, 2, 2> pv1;
+    front(std::true_type{}, one, Kc, col0, lo, hi, [&]() { pv1.prefetch(oa, Vc); });
+    const i32x4 P1[2] = {P[0], P[1]};
+    pv1.run(oa, Vc, P1, o);
+  };
   auto stage_k = [&](int st) { return smem + st * 2 * BN * HD; };
 
   // Ping-pong: the two waves of a SIMD (wave w and w + W/2) would otherwise run the same phase at the
@@ -226,6 +234,56 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
   // previous tile (V product), then does scores and softmax of the current one, so its softmax overlaps
   // the lower half's V product and its V product the lower half's scores.  The previous tile's V must
   // survive one more barrier interval, hence the extra ring stage.
+  // The wave's own depth columns, 32 at a time through wave-private K and V tiles cut out of the ring.  EARLY: the first
+  // ones travel while the last sequence tile is worked on, into the ring stage that is free by then.  Two waves have room
+  // for two whole sets, one in each stage, and fetch a tile ahead all the way; four for K in one stage and V in the other.
+  // A short launch is bound by what one wave has to do, one thing after the other: 64 x 197 tokens of four rows, eleven of
+  // twelve slots filled, 35.5 k cycles a wave with every private tile waited for and 13.7 k of them in this pass; now 29.1 k
+  // and 7.0 k, the launch 16.5 -> 13.9 us (six slots 14.1 -> 12.5, none 8.9 -> 8.5).
+  constexpr bool EARLY = !NODEPTH && !PP && NST == 2 && HD <= 64, TWO_SETS = EARLY && Shape::W <= 2;
+  typedef WaveTileLoader<HD> Own;
+  Own own;
+  const uint16_t *kdp = nullptr, *vdp = nullptr;
+  int c_beg = 0, c_end = 0, tok = 0, slot = 0;  // the span; token and slot of the next tile to be fetched
+  int first_set = 0;
+  bool early = false;
+  auto enter_depth = [&]() {
+    const int rw0 = qt * BM + __builtin_amdgcn_readfirstlane(wave) * 32;
+    if (rw0 >= a.Tq) return;
+    const DepthSpan span = own_depth_span(a, rw0, 32);
+    c_beg = __builtin_amdgcn_readfirstlane(span.c_beg);
+    c_end = __builtin_amdgcn_readfirstlane(span.c_end);
+    tok = __builtin_amdgcn_readfirstlane(span.t_beg);
+    kdp = a.kd + b * a.skd.b + hkv * a.skd.h;
+    vdp = a.vd + b * a.svd.b + hkv * a.svd.h;
+    own.init(lane);
+  };
+  // rows [col0, col0 + 32) of the span (short at its end) into a private tile; d: the tensor's head dim
+  auto fetch = [&](lds_ptr tile, const uint16_t* slice, int64_t stride, int col0, int d) {
+    const int nrows = min(32, c_end - col0);
+    if (PARTIAL)
+      own.fetch_slots(tile, slice, stride, tok, slot, nrows, (int64_t)a.T * a.L, a.L, a.Lv, d);
+    else
+      own.fetch(tile, slice, stride, col0, nrows, d);
+  };
+  auto next_columns = [&]() {
+    if (!PARTIAL) return;
+    const SlotStep s = slot_step(slot, 32, a.Lv);
+    tok += __builtin_amdgcn_readfirstlane(s.tokens);
+    slot = __builtin_amdgcn_readfirstlane(s.slot);
+  };
+  auto own_tile = [&](int set) {  // its V tile, with two sets, lies right behind
+    const int wv = __builtin_amdgcn_readfirstlane(wave);
+    return !EARLY ? smem + wv * (2 * 32 * HD) : stage_k(first_set ^ set) + wv * (TWO_SETS ? 2 * 32 * HD : 32 * HD);
+  };
+  auto fetch_early = [&]() {
+    fetch(own_tile(0), kdp, a.skd.t, c_beg, a.D);
+    if (TWO_SETS) {
+      fetch(own_tile(0) + 32 * HD, vdp, a.svd.t, c_beg, a.Dv);
+      next_columns();
+    }
+  };
+
   const bool late = PP && __builtin_amdgcn_readfirstlane(wave) >= Shape::W / 2;
   int it = 0;
   if (!late) {
@@ -254,17 +312,26 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
     // phase 2: boundary sequence tiles and depth tiles
     for (; it < ntiles; it++) {
       if (it + DIST < ntiles) issue(it + DIST);
+      if (EARLY && own_depth && it + 1 == ntiles) {
+        first_set = c_st ^ 1;
+        enter_depth();
+        if (c_beg < c_end) fetch_early();
+        early = true;
+      }
       const bool dep = !NODEPTH && it >= n_seq;
       const int col0 = dep ? dep0 + (it - n_seq) * BN : it * BN;
       const int lo = dep ? dlo : 0;
       const int hi = dep ? dhi : shi;
-      const bool touches = (hi > col0) && (lo < col0 + BN) && (hi > lo);
-      if (__any(touches)) {
-        lds_cptr Kc = stage_k(c_st);
-        tile(std::true_type{}, Kc, Kc + BN * HD, col0, lo, hi);
+      lds_cptr Kc = stage_k(c_st);
+      if (PP) {
+        if (__any((hi > col0) && (lo < col0 + BN) && (hi > lo))) tile(std::true_type{}, Kc, Kc + BN * HD, col0, lo, hi);
+      } else {  // by halves: the last tile of a sequence is as often as not seen by no row beyond its first half
+#pragma unroll 1
+        for (int c = col0; c < col0 + BN; c += 32, Kc += 32 * HD)
+          if (__any((hi > c) && (lo < c + 32) && (hi > lo))) half_tile(Kc, Kc + BN * HD, c, lo, hi);
       }
       c_st = (c_st + 1 == NST) ? 0 : c_st + 1;
-      wait_tile(it + 1);
+      if (it + 1 < ntiles) wait_tile(it + 1);
       __syncthreads();
     }
   } else {
@@ -324,40 +391,37 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
   }
 
   if (own_depth) {
-    // The wave's own depth columns, 32 at a time through a wave-private K tile and V tile cut out of the ring
-    // (no workgroup barrier after the one that retires the ring).  The next K tile is fetched as soon as the
-    // scores are out, the next V tile once the V product is.
-    __syncthreads();
-    typedef WaveTileLoader<HD> Own;
-    const int wv = __builtin_amdgcn_readfirstlane(wave);
-    lds_ptr Kt = smem + wv * (2 * 32 * HD), Vt = Kt + 32 * HD;
-    const int rw0 = qt * BM + wv * 32;
-    if (rw0 < a.Tq) {
-      const DepthSpan span = own_depth_span(a, rw0, 32);
-      const int c_beg = __builtin_amdgcn_readfirstlane(span.c_beg);
-      const int c_end = __builtin_amdgcn_readfirstlane(span.c_end);
-      const int nh = (c_end - c_beg + 31) / 32;
-      const uint16_t* kdp = a.kd + b * a.skd.b + hkv * a.skd.h;
-      const uint16_t* vdp = a.vd + b * a.svd.b + hkv * a.svd.h;
-      Own own;
-      own.init(lane);
-      // rows [col0, col0 + 32) of the span (short at its end) into a private tile; d: the tensor's head dim
-      auto fetch = [&](lds_ptr tile, const uint16_t* slice, int64_t stride, int col0, int d) {
-        const int nrows = min(32, c_end - col0);
-        if (PARTIAL)
-          own.fetch_mapped(tile, slice, stride, col0, nrows, (int64_t)a.T * a.L, a.L, a.Lv, d);
-        else
-          own.fetch(tile, slice, stride, col0, nrows, d);
-      };
-      fetch(Kt, kdp, a.skd.t, c_beg, a.D);
+    if (!EARLY) __syncthreads();  // (EARLY: every tile ends with one)
+    if (!early) enter_depth();
+    const int nh = (c_end - c_beg + 31) / 32;
+    if (TWO_SETS) {
+      if (!early && nh > 0) fetch_early();
+      for (int j = 0; j < nh; j++) {
+        const int col0 = c_beg + 32 * j;
+        lds_ptr Kt = own_tile(j & 1);
+        if (j + 1 < nh) {
+          fetch(own_tile((j + 1) & 1), kdp, a.skd.t, col0 + 32, a.D);
+          fetch(own_tile((j + 1) & 1) + 32 * HD, vdp, a.svd.t, col0 + 32, a.Dv);
+          next_columns();
+          Own::template wait_but<2 * Own::N>();
+        } else {
+          Own::template wait_but<0>();
+        }
+        half_tile(Kt, Kt + 32 * HD, col0, dlo, dhi);
+        Own::reads_done();
+      }
+    } else if (nh > 0) {
+      // The next K tile is fetched as soon as the scores are out, the next V tile once the V product is.
+      lds_ptr Kt = own_tile(0), Vt = EARLY ? own_tile(1) : Kt + 32 * HD;
+      if (!early) fetch(Kt, kdp, a.skd.t, c_beg, a.D);
       fetch(Vt, vdp, a.svd.t, c_beg, a.Dv);
-      const std::integral_constant<int, 1> one{};
       for (int j = 0; j < nh; j++) {
         const int col0 = c_beg + 32 * j;
         const bool more = j + 1 < nh;
         Own::template wait_but<Own::N>();  // K landed, V may still be on its way
         front(std::true_type{}, one, Kt, col0, dlo, dhi, []() {});
         Own::reads_done();
+        next_columns();
         if (more) fetch(Kt, kdp, a.skd.t, col0 + 32, a.D);
         if (more)
           Own::template wait_but<Own::N>();  // V landed, the next K on its way

@@ -238,11 +238,13 @@ MODA_HD int ring_tile_row0(const RowTilePlan& p, int it, int BN) {
 // Depth columns [c_beg, c_end) that the `rows` query rows starting at rw0 (< Tq) can see.
 struct DepthSpan {
   int c_beg, c_end;
+  int t_beg;  // token of the first one
 };
 MODA_HD DepthSpan own_depth_span(const KArgs& a, int rw0, int rows) {
   const int tw0 = rw0 / a.Gf, tw1 = (imin(a.Tq, rw0 + rows) - 1) / a.Gf;
   DepthSpan s;
-  s.c_beg = (a.chunk ? (tw0 / a.Cb) * a.Cb : tw0) * a.Lv;
+  s.t_beg = a.chunk ? (tw0 / a.Cb) * a.Cb : tw0;
+  s.c_beg = s.t_beg * a.Lv;
   s.c_end = (tw1 + 1) * a.Lv;
   return s;
 }

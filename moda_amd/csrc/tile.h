@@ -364,9 +364,29 @@ constexpr int kPadOffset = 0x7ffffff0;
 // (column c = token * Lv + slot, see geometry.h) and lie in rows token * L + slot of the tensor.  The loaders anchor
 // one descriptor at slot 0 of the first column's token; this is the row, relative to that anchor, of the tile's
 // row `rho`, given the first column's slot l0.
+// `rho` (at most 64) columns behind slot l0 of a token: tokens further, and the slot there.  The quotient is small: an
+// estimate from the reciprocal, low by less than one, and a correction, where a division of integers is 25 vector
+// instructions behind a branch (eight times a 32-row tile of K and V).
+struct SlotStep {
+  int tokens, slot;
+};
+__host__ __device__ __forceinline__ SlotStep slot_step(int l0, int rho, int Lv) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const float inv = __builtin_amdgcn_rcpf((float)Lv) * (1.f - 0x1p-20f);
+#else
+  const float inv = 1.f / (float)Lv * (1.f - 0x1p-20f);
+#endif
+  SlotStep s;
+  s.tokens = (int)((float)(l0 + rho) * inv);
+  s.slot = l0 + rho - s.tokens * Lv;
+  const bool low = s.slot >= Lv;
+  s.slot -= low ? Lv : 0;
+  s.tokens += low ? 1 : 0;
+  return s;
+}
 __host__ __device__ __forceinline__ int mapped_row(int l0, int rho, int L, int Lv) {
-  const int l = l0 + rho, dw = l / Lv;
-  return dw * L + (l - dw * Lv);
+  const SlotStep s = slot_step(l0, rho, Lv);
+  return s.tokens * L + s.slot;
 }
 // bytes the anchored descriptor covers: from the anchor row to the end of the slice (rows_total rows), capped
 __host__ __device__ __forceinline__ uint32_t mapped_bytes(int64_t anchor_row, int64_t rows_total, uint32_t stride_bytes) {
@@ -504,18 +524,25 @@ struct WaveTileLoader {
   __host__ __device__ __forceinline__ int mapped_offset(int i, int l0, int L, int Lv, int nrows, int stride_bytes, int d) const {
     const int row = i * RPW + prow;
     const int lch = pch ^ Tile<HD>::swz(row);
-    return (lch * 8 < d && row < nrows) ? mapped_row(l0, row, L, Lv) * stride_bytes + lch * 16 : kPadOffset;
+    const int off = mapped_row(l0, row, L, Lv) * stride_bytes + lch * 16;
+    return ((lch * 8 < d) & (row < nrows)) ? off : kPadOffset;
   }
-  // compact depth columns [col0, col0 + nrows) of a slice of rows_total rows, L slots per token, Lv of them filled
-  __device__ __forceinline__ void fetch_mapped(lds_ptr tile, const uint16_t* slice, int64_t row_stride, int col0,
-                                               int nrows, int64_t rows_total, int L, int Lv, int d) const {
-    const int w0 = __builtin_amdgcn_readfirstlane(col0 / Lv), l0 = col0 - w0 * Lv;
+  // `nrows` compact depth columns of a slice of rows_total rows, L slots per token, Lv of them filled, from slot l0 (< Lv) of
+  // token w0 on
+  __device__ __forceinline__ void fetch_slots(lds_ptr tile, const uint16_t* slice, int64_t row_stride, int w0, int l0,
+                                              int nrows, int64_t rows_total, int L, int Lv, int d) const {
     const uint32_t stride_bytes = (uint32_t)row_stride * 2u;
     const int64_t anchor = (int64_t)w0 * L;
     const i32x4 rs = rsrc_words(slice + anchor * row_stride, nrows > 0 ? mapped_bytes(anchor, rows_total, stride_bytes) : 0u);
 #pragma unroll
     for (int i = 0; i < N; i++)
       lds_dma<16, NOP>(rs, lds_addr(tile + i * 512), mapped_offset(i, l0, L, Lv, nrows, (int)stride_bytes, d), 0);
+  }
+  // ... from compact column col0 on
+  __device__ __forceinline__ void fetch_mapped(lds_ptr tile, const uint16_t* slice, int64_t row_stride, int col0,
+                                               int nrows, int64_t rows_total, int L, int Lv, int d) const {
+    const int w0 = __builtin_amdgcn_readfirstlane(col0 / Lv);
+    fetch_slots(tile, slice, row_stride, w0, col0 - w0 * Lv, nrows, rows_total, L, Lv, d);
   }
   // at most K of this wave's vector-memory loads (the youngest) still in flight
   template <int K>

@@ -347,7 +347,15 @@ void walk_row_kernel(const KArgs& a_in, bool dq, int rows_per_wave, bool own_pos
       // the wave's own depth columns, 32 at a time through a private K tile and V tile
       if (own_depth) {
         typedef WaveTileLoader<HD> Own;
-        const uint32_t kt = (uint32_t)wave * (2 * 32 * HD) * 2, vt = kt + 32 * HD * 2;
+        uint32_t kt = (uint32_t)wave * (2 * 32 * HD) * 2, vt = kt + 32 * HD * 2;
+        // forward on the 64-wide tiles: the first tiles go to the stage that is free while the last, masked sequence tile
+        // is worked on; two sets a stage apart for two waves, else K in that stage and V in the other
+        const bool early = !dq && HD <= 64 && NST == 2, two_sets = early && Shape::W <= 2;
+        const uint32_t stage = 2 * BN * HD * 2, first = plan.n_full < ntiles ? (uint32_t)(ntiles & 1) : 0u;
+        if (early && !two_sets) {
+          kt = first * stage + (uint32_t)wave * 32 * HD * 2;
+          vt = (first ^ 1) * stage + (uint32_t)wave * 32 * HD * 2;
+        }
         const int rw0 = qt * BM + wave * rows_per_wave;
         if (rw0 < a.Tq) {
           const DepthSpan span = own_depth_span(a, rw0, rows_per_wave);
@@ -359,7 +367,8 @@ void walk_row_kernel(const KArgs& a_in, bool dq, int rows_per_wave, bool own_pos
             const int col0 = span.c_beg + 32 * j;
             const int nrows = imin(32, span.c_end - col0);
             // where the dQ kernel forms the depth gradients it alternates between two sets of private tiles
-            const uint32_t set = dq && depth_grads_in_dq(a, HD) ? (uint32_t)(j & 1) * Shape::W * 64 * HD * 2 : 0u;
+            const uint32_t set = two_sets ? (first ^ (uint32_t)(j & 1)) * stage
+                                          : dq && depth_grads_in_dq(a, HD) ? (uint32_t)(j & 1) * Shape::W * 64 * HD * 2 : 0u;
             for (int i = 0; i < Own::N; i++) {
               if (a.Lv != a.L) {
                 const int w0 = col0 / a.Lv, l0 = col0 - w0 * a.Lv;
@@ -1520,6 +1529,18 @@ int main(int argc, char** argv) {
     std::vector<int> parts;
     for (int i = 7; i < argc; i++) parts.push_back(arg(i));
     walk_tail(std::string(argv[2]) == "fp16", arg(3), arg(4), arg(5), arg(6) != 0, parts);
+    printf("OK checked=%lld\n", g_checked);
+    return 0;
+  }
+  if (what == "slots") {  // the slot arithmetic of partially filled streams against the division it stands for
+    for (int Lv : {1, 2, 3, 5, 7, 11, 12, 24, 31, 33, 63, 64, 65, 72, 127, 1000, 65537, (1 << 24) + 3, (1 << 30) + 1})
+      for (int l0 : {0, 1, Lv / 2, Lv - 2, Lv - 1})
+        for (int rho = 0; rho <= 64; rho++) {
+          if (l0 < 0 || l0 >= Lv) continue;
+          const SlotStep s = slot_step(l0, rho, Lv);
+          if (s.tokens != (l0 + rho) / Lv || s.slot != (l0 + rho) % Lv) fail("slot %d + %d of %d: token %d, slot %d", l0, rho, Lv, s.tokens, s.slot);
+          g_checked++;
+        }
     printf("OK checked=%lld\n", g_checked);
     return 0;
   }

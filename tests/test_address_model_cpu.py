@@ -243,6 +243,12 @@ def test_launch_shapes_of_the_narrow_tiles(walker, case):
     assert rc == 0 and out.startswith(shapes + " OK"), out
 
 
+def test_slot_arithmetic(walker):
+    """Token and slot of a column of a partially filled stream, by a reciprocal and a correction."""
+    p = subprocess.run([walker, "slots"], capture_output=True, text=True)
+    assert p.returncode == 0 and "OK checked" in p.stdout, p.stdout + p.stderr
+
+
 @pytest.mark.parametrize("case", [
     # T, H, D, L, Lv, G, B: a backward that adds slot Lv of the depth gradients: row waves, row segments
     (197, 1, 64, 3, 1, 4, 3),

@@ -2424,3 +2424,42 @@ def test_compiled_autograd_replays_the_native_nodes(gpu_device):
                 total.backward()
             for x, w in zip(xs, want):
                 assert torch.equal(x.grad, w), call.__name__
+
+
+# ---------------------------------------------------------------------------
+# short sequences on the 64-wide tiles: where the last column tile ends, and the waves' own depth tiles
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize("B,T,H,G,L,valid,causal", [
+    # two waves (an odd number of 64-row tiles a head, more 128-row workgroups than compute units)
+    (37, 197, 1, 4, 12, 1, False),    # last tile of 5 columns; one depth tile of 8
+    (37, 197, 1, 4, 12, 4, False),    # ... of 32
+    (37, 197, 1, 4, 12, 11, False),   # ... three, the last one short
+    (37, 197, 1, 4, 12, 12, True),    # a full stream
+    (43, 160, 2, 2, 5, 3, False),     # last tile half full
+    (43, 161, 2, 2, 5, 3, False),     # ... and a column more
+    (65, 192, 2, 1, 40, 37, False),   # last tile full: no tile left to fetch beside; more than 1024 columns a wave
+    (130, 50, 2, 1, 3, 2, True),      # one tile
+    # four waves
+    (3, 197, 2, 2, 12, 7, False),
+    (2, 193, 2, 4, 6, 5, True),
+])
+def test_short_rows_by_tile_and_depth(gpu_device, B, T, H, G, L, valid, causal):
+    from moda_amd import ops
+
+    D, dtype, scale = 64, torch.bfloat16, 0.125
+    inp = oracle.make_inputs(B, T, H, D, L, G, seed=T + valid, dtype=dtype, std=0.5)
+    mode = "causal" if causal else "noncausal"
+    dev = to_dev(inp, gpu_device)
+    for n in ("kd", "vd"):  # unused slots are never read
+        dev[n].view(B, T, L, H, D)[:, :, valid:] = float("nan")
+    o, lse = ops._raw_fwd(MODE_ID[mode], dev["q"], dev["k"], dev["v"], dev["kd"], dev["vd"], scale, G, depth_valid=valid)
+    dq, dk, dv, dkd, dvd = ops._raw_bwd(MODE_ID[mode], dev["q"], dev["k"], dev["v"], dev["kd"], dev["vd"], o, lse, dev["do"],
+                                        scale, G, depth_valid=valid)
+    some = sorted({0, B // 2, B - 1})
+    part = {n: x[some] for n, x in inp.items()}
+    part["kd"], part["vd"] = (oracle.compact_depth(part[n], T, valid) for n in ("kd", "vd"))
+    ref = oracle.moda_dense_fwd_bwd(part, scale, G, mode)
+    for n in ("dkd", "dvd"):
+        ref[n] = oracle.scatter_depth_grad(ref[n], T, L)
+    got = {"o": o, "lse": lse, "dq": dq, "dk": dk, "dv": dv, "dkd": dkd, "dvd": dvd}
+    compare_all({n: x[some] for n, x in got.items()}, ref, dtype, f"B{B} T{T} valid {valid}")
