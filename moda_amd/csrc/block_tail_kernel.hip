@@ -14,10 +14,12 @@
 // 32 rows it waits for them.  (Two workgroups of 32 rows a compute unit instead: 48 us.)
 //
 // What bounds it, per 64 rows at width 256, hidden 1024, a next block with 384 projected features, measured cycles of 63 k: the
-// MLP's products 21 k (16 k of matrix instructions), its activation 9.4 k, waiting for each other 4 k; rows in 5 k, the two
-// projections 9 k, norms and residuals 11 k, rows out 5 k.  The activation's vector work does not overlap with the products:
-// run beside the next chunk's first product, or with the two waves of a SIMD half a chunk apart, it needs more registers than
-// there are (72 spilled, 44 us; with half the weights in flight 37).
+// MLP's products 21 k (16 k of matrix instructions; the rows' operands take all of LDS's 128 bytes a cycle there, and the
+// weights all of the 64 from L2), its activation 9.4 k, waiting for each other 4 k; rows in 5 k, the two projections 9 k, norms
+// and residuals 11 k, rows out 5 k.  With the activation of a chunk beside the second product of the chunk before, an
+// eighth of it after each step, the two waves of a SIMD cover each other: 34.7 -> 33.5 us, 64 x 197 tokens through twelve blocks
+// 571 -> 556, 16 x 197 417 -> 406.  Beside the next chunk's first product, or with the two waves of a SIMD half a chunk apart, it
+// needs more registers than there are (72 spilled, 44 us; with half the weights in flight 37).
 #include <type_traits>
 
 #include "../../include/moda_hip.h"
@@ -136,11 +138,13 @@ struct Product {
     typedef __attribute__((address_space(1))) const i32x4* vec;
     return *(vec)((__attribute__((address_space(1))) const char*)base[mb] + (size_t)voff + (size_t)ks * 1024);
   }
+  __device__ __forceinline__ void load(int j) {
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) w[j % PF][mb] = get(mb, j);
+  }
   __device__ __forceinline__ void start() {
 #pragma unroll
-    for (int j = 0; j < PF; j++)
-#pragma unroll
-      for (int mb = 0; mb < MB; mb++) w[j][mb] = get(mb, j);
+    for (int j = 0; j < PF; j++) load(j);
   }
   template <int W>
   __device__ __forceinline__ static void rows(i32x4 (&x)[NB], lds_cptr tile, const int (&rbase)[4], int ks) {
@@ -173,6 +177,22 @@ struct Product {
       }
     }
   }
+  // NK steps, all unrolled; after step j beside(j): work of another kind, or the loads of the product that follows
+  template <int W, int NK, typename Beside>
+  __device__ __forceinline__ void run_beside(lds_cptr tile, const int (&rbase)[4], f32x4 (&acc)[MB][NB], Beside&& beside) {
+    i32x4 x[2][NB];
+    rows<W>(x[0], tile, rbase, 0);
+#pragma unroll
+    for (int j = 0; j < NK; j++) {
+      if (j + 1 < NK) rows<W>(x[(j + 1) & 1], tile, rbase, j + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      step(w[j % PF], x[j & 1], acc);
+      if (j + PF < NK) load(j + PF);
+      __builtin_amdgcn_sched_barrier(0);
+      beside(j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
 };
 
 }  // namespace
@@ -180,6 +200,9 @@ struct Product {
 template <typename T, int C, int NB, bool POST>
 __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
   constexpr int BM = 16 * NB, MB2 = C / 128, MB1 = 2, HC = 128 * MB1, CH = C / 8, TPR = 512 / BM, NL = CH / TPR;
+  // The activation of a chunk beside the second product of the one before: where the registers are there.  fp16's formula with 64
+  // rows spills 23 (twelve blocks of width 256: 616 us apart, 624 beside), widths above 256 spill more than they do apart.
+  constexpr bool BESIDE = MB2 <= 2 && (NB == 2 || std::is_same<T, BF16>::value);
   static_assert(CH % TPR == 0, "a row's chunks over the threads of the row");
   extern __shared__ __align__(16) unsigned char tail_smem[];
   MODA_LDS const char* table = (MODA_LDS const char*)(lds_ptr)tail_smem;  // kGeluTable floats (bf16)
@@ -352,8 +375,9 @@ __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
   i32x2 bias1[MB1];
   auto has_features = [&](int c0) { return c0 + wave * 16 * MB1 < a.hidden; };
   auto start_fc1 = [&](int c0) MODA_INLINE {
-    if (!has_features(c0)) return;
-    const int f1 = c0 + wave * 16 * MB1;
+    // BESIDE: the waves that a short last chunk has no features for take others' and keep the result to themselves
+    if (!BESIDE && !has_features(c0)) return;
+    const int f1 = !BESIDE || has_features(c0) ? c0 + wave * 16 * MB1 : c0;
 #pragma unroll
     for (int mb = 0; mb < MB1; mb++) fc1.base[mb] = a.fc1_w + (size_t)(f1 + 16 * mb) * C;
     fc1.start();
@@ -370,35 +394,71 @@ __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
   Product<T, MB2, NB> fc2;
   fc2.voff = lane * 16;
   lds_ptr Hs = H;
-  for (int c0 = 0; c0 < a.hidden; c0 += HC) {
-    if (has_features(c0)) {
-      f32x4 hid[MB1][NB];
-      zero(hid);
-      fc1.template run<C>(X, xbase, C / 32, hid);
+  // piece (mb, nb) of a chunk's first product: bias, activation, into the stage `to`
+  auto activate = [&](const f32x4 (&hid)[MB1][NB], int mb, int nb, lds_ptr to) MODA_INLINE {
+    float b[4], x[4];
+    unpack4(bias1[mb], b);
 #pragma unroll
-      for (int mb = 0; mb < MB1; mb++) {
-        float b[4];
-        unpack4(bias1[mb], b);
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
-          float x[4];
-#pragma unroll
-          for (int i = 0; i < 4; i++) x[i] = hid[mb][nb][i] + b[i];
-          i32x2 w = pack4(x);  // the linear layer's own result is a 16-bit value, as it is when the layers run one by one
-          w[0] = activated<T>(w[0], table);
-          w[1] = activated<T>(w[1], table);
-          *reinterpret_cast<MODA_LDS i32x2*>(Hs + Rows<HC>::off(sigma, wave * 2 * MB1 + 2 * mb + (q4 >> 1)) + 4 * (q4 & 1) + 16 * nb * HC) = w;
-        }
-      }
-    }
+    for (int i = 0; i < 4; i++) x[i] = hid[mb][nb][i] + b[i];
+    i32x2 w = pack4(x);  // the linear layer's own result is a 16-bit value, as it is when the layers run one by one
+    w[0] = activated<T>(w[0], table);
+    w[1] = activated<T>(w[1], table);
+    *reinterpret_cast<MODA_LDS i32x2*>(to + Rows<HC>::off(sigma, wave * 2 * MB1 + 2 * mb + (q4 >> 1)) + 4 * (q4 & 1) + 16 * nb * HC) = w;
+  };
+  auto fc2_at = [&](int c0) MODA_INLINE {
 #pragma unroll
     for (int mb = 0; mb < MB2; mb++) fc2.base[mb] = a.fc2_w + (size_t)(f2 + 16 * mb) * a.hidden + c0 * 16;
-    fc2.start();
+  };
+  if constexpr (BESIDE) {
+    static_assert(Product<T, MB1, NB>::PF == Product<T, MB2, NB>::PF && C / 32 >= Product<T, MB1, NB>::PF, "as many steps on their way in both");
+    constexpr int PF = Product<T, MB1, NB>::PF, N1 = C / 32, N2 = HC / 32;
+    static_assert(N2 >= MB1 * NB, "a step for every piece");
+    f32x4 hid[MB1][NB];
+    zero(hid);
+    fc2_at(0);
+    fc1.template run_beside<C, N1>(X, xbase, hid, [&](int j) MODA_INLINE {
+      if (j >= N1 - PF) fc2.load(j - (N1 - PF));
+    });
+    if (has_features(0))
+#pragma unroll
+      for (int mb = 0; mb < MB1; mb++)
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) activate(hid, mb, nb, Hs);
+    for (int c0 = 0; c0 + HC < a.hidden; c0 += HC) {
+      lds_ptr other = Hs == H ? H + BM * HC : H;
+      start_fc1(c0 + HC);
+      lds_barrier();
+      zero(hid);
+      fc1.template run_beside<C, N1>(X, xbase, hid, [](int) {});
+      const bool mine = has_features(c0 + HC);
+      fc2.template run_beside<HC, N2>(Hs, hbase, acc, [&](int j) MODA_INLINE {
+        if (j < MB1 * NB && mine) activate(hid, j / NB, j % NB, other);
+      });
+      fc2_at(c0 + HC);
+      fc2.start();
+      Hs = other;
+    }
     lds_barrier();
-    const int left = a.hidden - c0;
-    fc2.template run<HC>(Hs, hbase, (left < HC ? left : HC) / 32, acc);
-    if (c0 + HC < a.hidden) start_fc1(c0 + HC);
-    Hs = Hs == H ? H + BM * HC : H;
+    fc2.template run<HC>(Hs, hbase, ((a.hidden - 1) % HC + 1) / 32, acc);
+  } else {
+    for (int c0 = 0; c0 < a.hidden; c0 += HC) {
+      if (has_features(c0)) {
+        f32x4 hid[MB1][NB];
+        zero(hid);
+        fc1.template run<C>(X, xbase, C / 32, hid);
+#pragma unroll
+        for (int mb = 0; mb < MB1; mb++)
+#pragma unroll
+          for (int nb = 0; nb < NB; nb++) activate(hid, mb, nb, Hs);
+      }
+      fc2_at(c0);
+      fc2.start();
+      lds_barrier();
+      const int left = a.hidden - c0;
+      fc2.template run<HC>(Hs, hbase, (left < HC ? left : HC) / 32, acc);
+      if (c0 + HC < a.hidden) start_fc1(c0 + HC);
+      Hs = Hs == H ? H + BM * HC : H;
+    }
   }
   pieces(a.fc2_b, f2, bias2);
   const bool end_norm = POST || a.n_parts > 0;

@@ -1285,12 +1285,14 @@ void walk_tail_of(bool fp16, int rows, int hidden, bool post, const std::vector<
         for (int nb = 0; nb < NB; nb++) lds(X, RowLayout<C>::off(sigma, (f2 >> 3) + 2 * mb + (q4 >> 1)) + 4 * (q4 & 1) + 16 * nb * C, 4, H, "own piece");
       norm("mid_w", mid_w, "mid_b", mid_b, true, false);
       for (int c0 = 0, stage = 0; c0 < hidden; c0 += HC, stage ^= 1) {
-        const int f1 = c0 + wave * 16 * MB1, left = std::min(hidden - c0, HC);
+        // (a wave without features of a short last chunk may read others', see the kernel, but leaves nothing)
+        const bool mine = c0 + wave * 16 * MB1 < hidden;
+        const int f1 = mine ? c0 + wave * 16 * MB1 : c0, left = std::min(hidden - c0, HC);
         const uint32_t Hs = H + stage * BM * HC, Hs_end = Hs + BM * HC;
-        if (f1 < hidden) {
-          product("fc1_w", fc1_w, f1, MB1, C, 0, C / 32, 4);
-          operand(RowLayout<C>{}, X, H, C / 32);
-          pieces("fc1_b", fc1_b, f1, MB1);
+        product("fc1_w", fc1_w, f1, MB1, C, 0, C / 32, 4);
+        operand(RowLayout<C>{}, X, H, C / 32);
+        pieces("fc1_b", fc1_b, f1, MB1);
+        if (mine) {
           for (int mb = 0; mb < MB1; mb++)
             for (int nb = 0; nb < NB; nb++)
               lds(Hs, RowLayout<HC>::off(sigma, wave * 2 * MB1 + 2 * mb + (q4 >> 1)) + 4 * (q4 & 1) + 16 * nb * HC, 4, Hs_end, "hidden piece");
