@@ -395,11 +395,10 @@ __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
   fc2.voff = lane * 16;
   lds_ptr Hs = H;
   // piece (mb, nb) of a chunk's first product: bias, activation, into the stage `to`
-  auto activate = [&](const f32x4 (&hid)[MB1][NB], int mb, int nb, lds_ptr to) MODA_INLINE {
-    float b[4], x[4];
-    unpack4(bias1[mb], b);
+  auto activate = [&](const f32x4& sum, const float (&b)[4], int mb, int nb, lds_ptr to) MODA_INLINE {
+    float x[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) x[i] = hid[mb][nb][i] + b[i];
+    for (int i = 0; i < 4; i++) x[i] = sum[i] + b[i];
     i32x2 w = pack4(x);  // the linear layer's own result is a 16-bit value, as it is when the layers run one by one
     w[0] = activated<T>(w[0], table);
     w[1] = activated<T>(w[1], table);
@@ -421,9 +420,12 @@ __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
     });
     if (has_features(0))
 #pragma unroll
-      for (int mb = 0; mb < MB1; mb++)
+      for (int mb = 0; mb < MB1; mb++) {
+        float b[4];
+        unpack4(bias1[mb], b);
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) activate(hid, mb, nb, Hs);
+        for (int nb = 0; nb < NB; nb++) activate(hid[mb][nb], b, mb, nb, Hs);
+      }
     for (int c0 = 0; c0 + HC < a.hidden; c0 += HC) {
       lds_ptr other = Hs == H ? H + BM * HC : H;
       start_fc1(c0 + HC);
@@ -432,7 +434,10 @@ __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
       fc1.template run_beside<C, N1>(X, xbase, hid, [](int) {});
       const bool mine = has_features(c0 + HC);
       fc2.template run_beside<HC, N2>(Hs, hbase, acc, [&](int j) MODA_INLINE {
-        if (j < MB1 * NB && mine) activate(hid, j / NB, j % NB, other);
+        if (j >= MB1 * NB || !mine) return;
+        float b[4];
+        unpack4(bias1[j / NB], b);
+        activate(hid[j / NB][j % NB], b, j / NB, j % NB, other);
       });
       fc2_at(c0 + HC);
       fc2.start();
@@ -447,11 +452,15 @@ __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
         zero(hid);
         fc1.template run<C>(X, xbase, C / 32, hid);
 #pragma unroll
-        for (int mb = 0; mb < MB1; mb++)
+        for (int mb = 0; mb < MB1; mb++) {
+          float b[4];
+          unpack4(bias1[mb], b);
 #pragma unroll
-          for (int nb = 0; nb < NB; nb++) activate(hid, mb, nb, Hs);
+          for (int nb = 0; nb < NB; nb++) activate(hid[mb][nb], b, mb, nb, Hs);
+        }
       }
-      fc2_at(c0);
+#pragma unroll
+      for (int mb = 0; mb < MB2; mb++) fc2.base[mb] = a.fc2_w + (size_t)(f2 + 16 * mb) * a.hidden + c0 * 16;  // (fc2_at: 4 registers more)
       fc2.start();
       lds_barrier();
       const int left = a.hidden - c0;
