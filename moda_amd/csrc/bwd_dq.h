@@ -43,9 +43,48 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
   const KArgs& a = seq.a;
   const int Ld = NODEPTH ? 0 : a.L;  // depth slots per token
 
-  i32x4 Qr[NB][KS], dOr[NB][KS];
+  // Loads of the row operands and, on the 64-wide tiles, of o, which has the row sums wait for it: the first tiles of the ring
+  // are sent for in between, so that all of it travels together.
+  constexpr bool SUMS_LATE = HD <= 64;
+  i32x4 Qr[NB][KS], dOr[NB][KS], Or[NB][KS];
   float lse[NB], delta[NB];
   int shi[NB], dlo[NB], dhi[NB];
+  auto load_o = [&](int nb) {
+    const int r = qt * BM + wave * WR + 16 * nb + n;
+    const uint16_t* orow = a.o + b * a.so.b + hq * a.so.h + (int64_t)r * a.so.t + 8 * q4;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      i32x4 z = {0, 0, 0, 0};
+      Or[nb][ks] = (r < a.Tq && 32 * ks + 8 * q4 < a.Dv) ? *reinterpret_cast<const i32x4*>(orow + 32 * ks) : z;
+    }
+  };
+  auto row_sum = [&](int nb) {
+    const int r = qt * BM + wave * WR + 16 * nb + n;
+    const bool valid = r < a.Tq;
+    float* drow = a.delta + ((int64_t)b * a.Hq + hq) * (VARLEN ? a.delta_pitch : a.Tq) + r;
+    delta[nb] = 0.f;
+    if (a.own_delta) {
+      // minus rowsum(o * do) (moda_v14.py:525-539) from the dO pieces this lane holds anyway and the same pieces of
+      // o; the four lanes of a row add their shares and the first one leaves the sum for the kernels that follow
+      if (!SUMS_LATE) load_o(nb);
+      float acc = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+          float x0, x1, y0, y1;
+          unpack2<T>(Or[nb][ks][w], x0, x1);
+          unpack2<T>(dOr[nb][ks][w], y0, y1);
+          acc = __builtin_fmaf(x0, y0, acc);
+          acc = __builtin_fmaf(x1, y1, acc);
+        }
+      acc = quad_sum(acc);
+      delta[nb] = valid ? -acc : 0.f;
+      if (valid && q4 == 0) *drow = -acc;
+    } else if (valid) {
+      delta[nb] = *drow;
+    }
+  };
 #pragma unroll
   for (int nb = 0; nb < NB; nb++) {
     const int r = qt * BM + wave * WR + 16 * nb + n;
@@ -59,33 +98,11 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
       dOr[nb][ks] = (valid && 32 * ks + 8 * q4 < a.Dv) ? *reinterpret_cast<const i32x4*>(dop + 32 * ks) : z;
     }
     lse[nb] = 0.f;
-    delta[nb] = 0.f;
     if (valid) lse[nb] = a.lse[((int64_t)b * a.Tq + r) * a.Hq + hq];
-    float* drow = a.delta + ((int64_t)b * a.Hq + hq) * (VARLEN ? a.delta_pitch : a.Tq) + r;
-    if (a.own_delta) {
-      // minus rowsum(o * do) (moda_v14.py:525-539) from the dO pieces this lane holds anyway and the same pieces of
-      // o; the four lanes of a row add their shares and the first one leaves the sum for the kernels that follow
-      const uint16_t* orow = a.o + b * a.so.b + hq * a.so.h + (int64_t)r * a.so.t + 8 * q4;
-      float acc = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < KS; ks++) {
-        i32x4 z = {0, 0, 0, 0};
-        const i32x4 ov = (valid && 32 * ks + 8 * q4 < a.Dv) ? *reinterpret_cast<const i32x4*>(orow + 32 * ks) : z;
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-          float x0, x1, y0, y1;
-          unpack2<T>(ov[w], x0, x1);
-          unpack2<T>(dOr[nb][ks][w], y0, y1);
-          acc = __builtin_fmaf(x0, y0, acc);
-          acc = __builtin_fmaf(x1, y1, acc);
-        }
-      }
-      acc = quad_sum(acc);
-      delta[nb] = valid ? -acc : 0.f;
-      if (valid && q4 == 0) *drow = -acc;
-    } else if (valid) {
-      delta[nb] = *drow;
-    }
+    if (!SUMS_LATE)
+      row_sum(nb);
+    else if (a.own_delta)
+      load_o(nb);
     const RowVis vis = row_visibility(a, r, Ld);
     shi[nb] = vis.shi;
     dlo[nb] = vis.dlo;
@@ -157,6 +174,9 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
 #pragma unroll
   for (int j = 0; j < DIST; j++)
     if (j < ntiles) issue(j);
+  if (SUMS_LATE)
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) row_sum(nb);
   // The tile loads are issued behind the compiler's back, and a register operand it still believes pending would cost
   // a vmcnt(0) in every trip of the main loop: both kinds are waited for here, once, having travelled together.
   asm volatile("" ::: "memory");
@@ -186,10 +206,14 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
 #pragma unroll
       for (int nb = 0; nb < NB; nb++) {
         f32x4 pr;
+        // a column of [lo, hi) by its distance from lo (two comparisons where the registers of the distance would spill)
+        const int before = col0 + slot_base(q4) - lo[nb];
+        const unsigned width = (unsigned)(hi[nb] > lo[nb] ? hi[nb] - lo[nb] : 0);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           float p = fast_exp2(__builtin_fmaf(s[mb][nb][i], sc, -lse[nb]));
-          if (MASKED) {
+          if (MASKED && HD <= 64) p = (unsigned)(before + 16 * mb + i) < width ? p : 0.f;
+          if (MASKED && HD > 64) {
             const int c = col0 + 16 * mb + slot_base(q4) + i;
             p = (c >= lo[nb] && c < hi[nb]) ? p : 0.f;
           }
@@ -211,6 +235,7 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
 #pragma unroll
   for (int nb = 0; nb < NB; nb++) none[nb] = 0;
   const std::integral_constant<int, 4> four{};
+  const std::integral_constant<int, 2> two{};
   for (; it < n_full; it++) {
     if (it + DIST < ntiles) issue(it + DIST);
     lds_cptr Kc = smem + c_st * 2 * BN * HD;
@@ -219,38 +244,94 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
     wait_tile(it + 1);
     __syncthreads();
   }
+  // Outside chunk-visible mode (when a token's rows never straddle waves) the pass over the wave's own depth
+  // columns also forms their dK and dV: see the second block below.
+  constexpr bool FUSABLE = !NODEPTH && OWN_FITS && HD <= kDepthGradsInDqMaxWidth;
+  bool fused_depth = false;
+  if constexpr (FUSABLE) fused_depth = depth_grads_in_dq(a, HD);
+  typedef WaveTileLoader<HD, DMA_NOP> Own;
+  // Its private tiles: two sets of a K tile and a V tile for every wave, over the ring.  The first tile is sent for while the
+  // last sequence tile is worked on, into the set that lies outside of that one's stage.
+  constexpr int SET = Shape::W * 64 * HD;
+  static_assert(!FUSABLE || (Shape::W == 2 && SET == 2 * BN * HD) || NST * 2 * BN * HD <= SET, "a set is a stage, or all of the ring");
+  Own own;
+  const uint16_t *kdp = nullptr, *vdp = nullptr;
+  int c_beg = 0, c_end = 0, t_beg = 0, first_set = 0;
+  bool early = false;
+  auto own_tile = [&](int set) { return smem + (first_set ^ set) * SET + __builtin_amdgcn_readfirstlane(wave) * (2 * 32 * HD); };
+  bool pad_k[Own::N], pad_v[Own::N];  // this lane's chunk lies past the head dim
+  int rel[Own::N];                    // this lane's rows of the tile that was sent for last, from the row that `tile_row` names
+  // Token `tok`, slot `slot`: those of column col0.  The rows are counted from slot 0 of the token (a full stream: from the column)
+  auto tile_row = [&](int tok, int col0) { return PARTIAL ? (int64_t)tok * a.L : (int64_t)col0; };
+  auto fetch = [&](int set, int col0, int tok, int slot) {
+#pragma unroll
+    for (int i = 0; i < Own::N; i++) {
+      const int row = i * Own::RPW + own.prow;
+      rel[i] = PARTIAL ? mapped_row(slot, row, a.L, a.Lv) : row;
+      rel[i] = col0 + row < c_end ? rel[i] : -1;
+    }
+    const int64_t row0 = tile_row(tok, col0), rows = (int64_t)a.T * a.L;
+    const uint32_t sk = (uint32_t)a.skd.t * 2u, sv = (uint32_t)a.svd.t * 2u;
+    lds_ptr Kt = own_tile(set);
+    own.fetch_rows(Kt, kdp + row0 * a.skd.t, sk, mapped_bytes(row0, rows, sk), rel, pad_k);
+    own.fetch_rows(Kt + 32 * HD, vdp + row0 * a.svd.t, sv, mapped_bytes(row0, rows, sv), rel, pad_v);
+  };
+  auto enter_depth = [&]() {
+    const int rw0 = qt * BM + __builtin_amdgcn_readfirstlane(wave) * WR;
+    if (rw0 >= a.Tq) return;
+    const DepthSpan span = own_depth_span(a, rw0, WR);
+    c_beg = __builtin_amdgcn_readfirstlane(span.c_beg);
+    c_end = __builtin_amdgcn_readfirstlane(span.c_end);
+    t_beg = __builtin_amdgcn_readfirstlane(span.t_beg);
+    kdp = a.kd + b * a.skd.b + hkv * a.skd.h;
+    vdp = a.vd + b * a.svd.b + hkv * a.svd.h;
+    own.init(lane);
+#pragma unroll
+    for (int i = 0; i < Own::N; i++) {
+      pad_k[i] = own.chunk(i) * 8 >= a.D;
+      pad_v[i] = own.chunk(i) * 8 >= a.Dv;
+    }
+    if (c_beg < c_end) fetch(0, c_beg, t_beg, 0);
+  };
   for (; it < ntiles; it++) {
     if (it + DIST < ntiles) issue(it + DIST);
+    if (FUSABLE && fused_depth && it + 1 == ntiles) {
+      first_set = Shape::W > 2 || c_st == 0 ? 1 : 0;
+      enter_depth();
+      early = true;
+    }
     const bool dep = !NODEPTH && it >= n_seq;
     const int col0 = dep ? dep0 + (it - n_seq) * BN : it * BN;
     int lo[NB], hi[NB];
-    bool touches = false;
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
       lo[nb] = dep ? dlo[nb] : 0;
       hi[nb] = dep ? dhi[nb] : shi[nb];
-      touches = touches || ((hi[nb] > col0) && (lo[nb] < col0 + BN) && (hi[nb] > lo[nb]));
     }
-    if (__any(touches)) {
-      lds_cptr Kc = smem + c_st * 2 * BN * HD;
-      tile(std::true_type{}, four, Kc, Kc + BN * HD, col0, lo, hi, []() {}, [](int, int, const f32x4&, const f32x4&) {});
+    lds_cptr Kc = smem + c_st * 2 * BN * HD;
+    auto part = [&](auto nblk, lds_cptr Kp, int c) {
+      constexpr int COLS = 16 * decltype(nblk)::value;
+      bool touches = false;
+#pragma unroll
+      for (int nb = 0; nb < NB; nb++) touches = touches || ((hi[nb] > c) && (lo[nb] < c + COLS) && (hi[nb] > lo[nb]));
+      if (__any(touches)) tile(std::true_type{}, nblk, Kp, Kp + BN * HD, c, lo, hi, []() {}, [](int, int, const f32x4&, const f32x4&) {});
+    };
+    if constexpr (HD <= 64) {  // by halves: the last tile of a sequence is as often as not seen by no row beyond its first half
+#pragma unroll 1
+      for (int c = col0; c < col0 + BN; c += 32, Kc += 32 * HD) part(two, Kc, c);
+    } else {
+      part(four, Kc, col0);
     }
     c_st = (c_st + 1 == NST) ? 0 : c_st + 1;
-    wait_tile(it + 1);
+    if (it + 1 < ntiles) wait_tile(it + 1);
     __syncthreads();
   }
 
-  // Outside chunk-visible mode (when a token's rows never straddle waves) the pass over the wave's own depth
-  // columns also forms their dK and dV: see the second block below.
-  bool fused_depth = false;
-  constexpr bool FUSABLE = !NODEPTH && OWN_FITS && HD <= kDepthGradsInDqMaxWidth;
-  if constexpr (FUSABLE) fused_depth = depth_grads_in_dq(a, HD);
   if (own_depth && !fused_depth) {
     // The wave's own depth columns, 32 at a time through a wave-private K tile and V tile cut out of the ring
     // (no workgroup barrier after the one that retires the ring).  The next V tile is fetched as soon as the
     // scores are out, the next K tile once dQ has its share.
     __syncthreads();
-    typedef WaveTileLoader<HD, DMA_NOP> Own;
     const int wv = __builtin_amdgcn_readfirstlane(wave);
     lds_ptr Kt = smem + wv * (2 * 32 * HD), Vt = Kt + 32 * HD;
     const int rw0 = qt * BM + wv * WR;
@@ -273,7 +354,6 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
       };
       fetch(Kt, kdp, a.skd.t, c_beg, a.D);
       fetch(Vt, vdp, a.svd.t, c_beg, a.Dv);
-      const std::integral_constant<int, 2> two{};
       // where the depth-gradient kernel takes P and dS from here: this lane's rows of the two arrays
       const bool hand_over = a.depth_p != nullptr;
       uint16_t *hp[NB], *hds[NB];
@@ -325,16 +405,13 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
   if constexpr (FUSABLE) {
     if (fused_depth) {
       static_assert(NB == 2, "the wave's 32 query rows are the 32 summation slots of one matrix instruction");
-      __syncthreads();
-      typedef WaveTileLoader<HD, DMA_NOP> Own;
+      if (!early) enter_depth();  // (every ring tile ends with a barrier)
       const int wv = __builtin_amdgcn_readfirstlane(wave);
-      // two sets of a private K tile and V tile (the next tile's rows travel while this one is worked on), then
-      // the staging block: 16 rows of HD, or 32 x 32 for the dS block
-      lds_ptr Kt = smem + wv * (2 * 32 * HD), Vt = Kt + 32 * HD;
-      constexpr int SET = Shape::W * 64 * HD;
+      // behind the two sets the staging block: 16 rows of HD, or 32 x 32 for the dS block
       lds_ptr stage = smem + 2 * SET + wv * (16 * HD);
       const int rw0 = qt * BM + wv * WR;
       if (rw0 < a.Tq) {
+        lds_ptr Kt = own_tile(1), Vt = Kt + 32 * HD;  // (the first tile is on its way to the other set)
         // Query row 16*nb + n goes to the tile row its lane reads as a row operand, slot_base(n >> 2) + (n & 3):
         // the transposed read then delivers rows 4q + j and 16 + 4q + j as lane group q's eight summation slots,
         // the order of the packed accumulators.
@@ -365,62 +442,109 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
             del4[nb][i] = __shfl(delta[nb], 4 * q4 + i, 64);
           }
         const int gshift = __builtin_ctz(a.Gf);  // Gf divides 32: a power of two
-        const DepthSpan span = own_depth_span(a, rw0, WR);
-        const int c_beg = __builtin_amdgcn_readfirstlane(span.c_beg);
-        const int c_end = __builtin_amdgcn_readfirstlane(span.c_end);
         const int nh = (c_end - c_beg + 31) / 32;
-        const uint16_t* kdp = a.kd + b * a.skd.b + hkv * a.skd.h;
-        const uint16_t* vdp = a.vd + b * a.svd.b + hkv * a.svd.h;
-        uint16_t* dkdp = a.dkd + b * a.sdkd.b + hkv * a.sdkd.h;
-        uint16_t* dvdp = a.dvd + b * a.sdvd.b + hkv * a.sdvd.h;
-        Own own;
-        own.init(lane);
-        auto fetch = [&](lds_ptr tile, const uint16_t* slice, int64_t stride, int col0, int d) {
-          const int nrows = min(32, c_end - col0);
-          if (PARTIAL)
-            own.fetch_mapped(tile, slice, stride, col0, nrows, (int64_t)a.T * a.L, a.L, a.Lv, d);
-          else
-            own.fetch(tile, slice, stride, col0, nrows, d);
-        };
+        // token of the query row on accumulator register i of block nb; -1 past the end
+        int row_token[NB][4];
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) row_token[nb][i] = rq + 16 * nb + i < a.Tq ? (rq + 16 * nb + i) >> gshift : -1;
+        const uint16_t* dkdp = a.dkd + b * a.sdkd.b + hkv * a.sdkd.h;
+        const uint16_t* dvdp = a.dvd + b * a.sdvd.b + hkv * a.sdvd.h;
         const int lrow = slot_base(n >> 2) + (n & 3);  // tile row (of a 16-row block) whose column this lane holds
-        // 16 gradient rows (the columns cbase .. cbase + 15) leave through the staging block: the accumulators
-        // hold 8-byte pieces of 16 different rows per register, which the memory pipeline would take as 16 partial
-        // lines per store; written to LDS and read back by rows, every store covers whole rows.
-        constexpr int RPW = Own::RPW, NPASS = 16 / RPW;
-        auto stage_put = [&](int mb, const f32x4& x, float mul) {
-          i32x2 w;
-          w[0] = pack2<T>(x[0] * mul, x[1] * mul);
-          w[1] = pack2<T>(x[2] * mul, x[3] * mul);
-          *reinterpret_cast<MODA_LDS i32x2*>(stage + Tile<HD>::off(lrow, 2 * mb + (q4 >> 1)) + 4 * (q4 & 1)) = w;
-        };
-        // Accumulating: what this lane's pieces of the tile's gradient rows hold, sent for once the tile's scores are out of
-        // the registers and waited for with the next tile's rows.  Fetched where they are added, every 16 rows stood
-        // still for a trip to memory, the next tile's loads with them (64 x 197 tokens of four query rows, one to eleven
-        // slots: dQ launch 30.0 -> 27.1 us).
-        i32x4 old_k[2][NPASS], old_v[2][NPASS];
-        auto fetch_old = [&](int col0) {
+        // The rounded dS block crosses over through `stage`: per 16 columns and 16 query rows, column by column in lane order,
+        // four rows (8 bytes) a piece; columns 8 .. 15 have their two halves swapped, which spreads the pieces that are written
+        // together over all banks.  The transposed read hands lane group q the columns slot_base(q) .. + 3 of each block.
+        const int xs_put = n * 16 + 4 * (q4 ^ ((n >> 3) << 1)), xs_col = 4 * q4 + (n >> 2), xs_get = xs_col * 16 + 4 * ((n & 3) ^ ((xs_col >> 3) << 1));
+        int tok = t_beg, slot = 0;  // of the tile's first column
+        // Tile j: wait for its rows, send for tile j + 1 (other set), scores, dS and dQ; then its gradient rows, through the
+        // tile's own K and V blocks, which nobody reads any more: the accumulators hold 8-byte pieces of 16 different rows per
+        // register, which the memory pipeline would take as 16 partial lines per store; written to LDS and read back by rows,
+        // every store covers whole rows.  The wave's memory counter covers loads and stores alike: the wait for the next
+        // tile's rows leaves this tile's eight stores, younger than them, on their way.  Such a launch is bound by what a wave has to
+        // issue, one thing after the other (six slots of twelve, 64 x 197 tokens of four rows: 43 k cycles): with 16 rows staged
+        // at a time, guarded 64-bit addresses and dS crossing in 2-byte pieces a backward pass over the stream's layers took
+        // 27.8 us a dQ launch, now 24.9; vision layers (64 x 197, six heads, twelve slots) 190 -> 184 us a step.
+        for (int j = 0; j < nh; j++) {
+          const int col0 = c_beg + 32 * j;
+          lds_ptr Kc = own_tile(j & 1), Vc = Kc + 32 * HD;
+          const SlotStep ahead = slot_step(slot, 32, a.Lv);
+          const int next_tok = tok + __builtin_amdgcn_readfirstlane(ahead.tokens), next_slot = __builtin_amdgcn_readfirstlane(ahead.slot);
+          if (j == 0)
+            Own::template wait_but<0>();
+          else
+            Own::template wait_but<2 * Own::N>();
+          int off_k[Own::N], off_v[Own::N];  // this lane's pieces of the gradient rows
+#pragma unroll
+          for (int i = 0; i < Own::N; i++) {
+            off_k[i] = own.row_offset(i, rel[i], (int)a.sdkd.t * 2, pad_k[i]);
+            off_v[i] = own.row_offset(i, rel[i], (int)a.sdvd.t * 2, pad_v[i]);
+          }
+          const int64_t row0 = tile_row(tok, col0);
+          const RowBuffer dk_rows(dkdp + row0 * a.sdkd.t, kPadOffset), dv_rows(dvdp + row0 * a.sdvd.t, kPadOffset);
+          if (j + 1 < nh) fetch((j + 1) & 1, col0 + 32, next_tok, next_slot);
+          f32x4 s[2][NB], dp[2][NB];
+          mfma16_rows2<T, HD, 2, NB, 2, true>(oa, Kc, Qr, s, Vc, dOr, dp, del4);
+          // Accumulating: what the gradient rows hold, sent for once the scores are out of the registers (where it is added,
+          // every row would stand still for a trip to memory)
+          i32x4 old_k[Own::N], old_v[Own::N], PA[2], DSA[2];
+          if (a.accum_depth) {
+#pragma unroll
+            for (int i = 0; i < Own::N; i++) {
+              old_v[i] = dv_rows.load(off_v[i]);
+              old_k[i] = dk_rows.load(off_k[i]);
+            }
+          }
+#pragma unroll
+          for (int cb = 0; cb < 2; cb++) {
+            const int tokc = col0 + 16 * cb + lrow < c_end ? tok + slot_step(slot, 16 * cb + lrow, a.Lv).tokens : -2;
+            f32x4 p[NB], ds[NB];
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+              for (int i = 0; i < 4; i++) {
+                float pv = fast_exp2(__builtin_fmaf(s[cb][nb][i], sc, -lse4[nb][i]));
+                pv = row_token[nb][i] == tokc ? pv : 0.f;
+                p[nb][i] = pv;
+                ds[nb][i] = pv * dp[cb][nb][i];
+              }
+            PA[cb] = pack_slots<T>(p[0], p[1]);
+            DSA[cb] = pack_slots<T>(ds[0], ds[1]);
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++)
+              *reinterpret_cast<MODA_LDS i32x2*>(stage + (2 * cb + nb) * 256 + xs_put) = i32x2{DSA[cb][2 * nb], DSA[cb][2 * nb + 1]};
+          }
+          Own::reads_done();  // (the counter covers LDS writes as well)
+          i32x4 DS[1][NB];
+#pragma unroll
+          for (int nb = 0; nb < NB; nb++) {
+            const i32x2 lo = __builtin_bit_cast(i32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((MODA_LDS s16x4*)(stage + nb * 256 + xs_get)));
+            const i32x2 hi = __builtin_bit_cast(i32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((MODA_LDS s16x4*)(stage + (2 + nb) * 256 + xs_get)));
+            DS[0][nb] = i32x4{lo[0], lo[1], hi[0], hi[1]};
+          }
+          TrPipe16<T, HD, 1, NB, 3> kt;
+          kt.prefetch(oa, Kc);
+          kt.run(oa, Kc, DS, dq);
+          Own::reads_done();
+          auto put = [&](lds_ptr block, int cb, int mb, const f32x4& x, float mul) {
+            i32x2 w;
+            w[0] = pack2<T>(x[0] * mul, x[1] * mul);
+            w[1] = pack2<T>(x[2] * mul, x[3] * mul);
+            *reinterpret_cast<MODA_LDS i32x2*>(block + 16 * cb * HD + Tile<HD>::off(lrow, 2 * mb + (q4 >> 1)) + 4 * (q4 & 1)) = w;
+          };
+          const f32x4 z = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int cb = 0; cb < 2; cb++)
 #pragma unroll
-            for (int i = 0; i < NPASS; i++) {
-              const int row = i * RPW + own.prow, lch = own.pch ^ Tile<HD>::swz(row), c = col0 + 16 * cb + row;
-              if (c < c_end) {
-                const int64_t r = depth_row_of(a, c);
-                if (lch * 8 < a.D) old_k[cb][i] = *reinterpret_cast<const i32x4*>(dkdp + r * a.sdkd.t + lch * 8);
-                if (lch * 8 < a.Dv) old_v[cb][i] = *reinterpret_cast<const i32x4*>(dvdp + r * a.sdvd.t + lch * 8);
-              }
+            for (int mb = 0; mb < MB; mb++) {
+              put(Vc, cb, mb, mfma16<T>(dOT[mb], PA[cb], z), 1.f);
+              put(Kc, cb, mb, mfma16<T>(QT[mb], DSA[cb], z), a.scale);
             }
-        };
-        auto flush = [&](uint16_t* base, int64_t stride, int cbase, int width, const i32x4 (&old)[NPASS]) {
-          Own::reads_done();  // the block is written
+          Own::reads_done();
+          auto flush = [&](lds_ptr block, const RowBuffer& rows, const int (&off)[Own::N], const i32x4 (&old)[Own::N]) {
 #pragma unroll
-          for (int i = 0; i < NPASS; i++) {
-            const int row = i * RPW + own.prow;
-            i32x4 val = *reinterpret_cast<MODA_LDS const i32x4*>(stage + i * 512 + lane * 8);
-            const int lch = own.pch ^ Tile<HD>::swz(row);
-            const int c = cbase + row;
-            if (c < c_end && lch * 8 < width) {
-              i32x4* dst = reinterpret_cast<i32x4*>(base + depth_row_of(a, c) * stride + lch * 8);
+            for (int i = 0; i < Own::N; i++) {
+              i32x4 val = *reinterpret_cast<MODA_LDS const i32x4*>(block + i * 512 + lane * 8);
               if (a.accum_depth) {  // add to what the row holds (this lane is the only writer of its 16 bytes)
 #pragma unroll
                 for (int w = 0; w < 4; w++) {
@@ -430,83 +554,15 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
                   val[w] = pack2<T>(x0 + y0, x1 + y1);
                 }
               }
-              __builtin_nontemporal_store(val, dst);  // next read by another launch
+              rows.template store<true>(val, off[i]);  // next read by another launch
             }
-          }
-          Own::reads_done();  // the block may be overwritten
-        };
-        fetch(Kt, kdp, a.skd.t, c_beg, a.D);
-        fetch(Vt, vdp, a.svd.t, c_beg, a.Dv);
-        MODA_LDS uint16_t* xs = (MODA_LDS uint16_t*)stage;  // dS block: [32 query rows][32 column slots]
-        // the gradient rows of one tile's columns from its packed P and dS
-        auto gradients = [&](const i32x4 (&PA)[2], const i32x4 (&DSA)[2], int col0) {
-          const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int cb = 0; cb < 2; cb++)
-            if (col0 + 16 * cb < c_end) {
-#pragma unroll
-              for (int mb = 0; mb < MB; mb++) stage_put(mb, mfma16<T>(dOT[mb], PA[cb], z), 1.f);
-              flush(dvdp, a.sdvd.t, col0 + 16 * cb, a.Dv, old_v[cb]);
-#pragma unroll
-              for (int mb = 0; mb < MB; mb++) stage_put(mb, mfma16<T>(QT[mb], DSA[cb], z), a.scale);
-              flush(dkdp, a.sdkd.t, col0 + 16 * cb, a.D, old_k[cb]);
-            }
-        };
-        // Tile j: wait for its rows, send for tile j + 1 (other set), write out the gradient rows of tile j - 1, then
-        // scores, dS and dQ of tile j.  The stores of a tile are thus issued a whole tile before the next wait
-        // (the wave's memory counter covers loads and stores alike), the loads one tile ahead of their use.
-        i32x4 PA[2], DSA[2];
-        for (int j = 0; j < nh; j++) {
-          const int col0 = c_beg + 32 * j;
-          lds_ptr Kc = Kt + (j & 1) * SET, Vc = Vt + (j & 1) * SET;
-          Own::template wait_but<0>();
-          if (j + 1 < nh) {
-            fetch(Kt + ((j + 1) & 1) * SET, kdp, a.skd.t, col0 + 32, a.D);
-            fetch(Vt + ((j + 1) & 1) * SET, vdp, a.svd.t, col0 + 32, a.Dv);
-          }
-          if (j > 0) gradients(PA, DSA, col0 - 32);
-          f32x4 s[2][NB], dp[2][NB];
-          mfma16_rows2<T, HD, 2, NB, 2, true>(oa, Kc, Qr, s, Vc, dOr, dp, del4);
-#pragma unroll
-          for (int cb = 0; cb < 2; cb++) {
-            const int c = col0 + 16 * cb + lrow;
-            const int tokc = c < c_end ? c / a.Lv : -2;
-            f32x4 p[NB], ds[NB];
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-              for (int i = 0; i < 4; i++) {
-                const int r = rq + 16 * nb + i;
-                float pv = fast_exp2(__builtin_fmaf(s[cb][nb][i], sc, -lse4[nb][i]));
-                pv = (r < a.Tq && (r >> gshift) == tokc) ? pv : 0.f;
-                p[nb][i] = pv;
-                ds[nb][i] = pv * dp[cb][nb][i];
-              }
-            PA[cb] = pack_slots<T>(p[0], p[1]);
-            DSA[cb] = pack_slots<T>(ds[0], ds[1]);
-            // the rounded dS block to LDS, a query row per 64-byte line, the column of tile row
-            // 16*cb + slot_base(g) + j in slot 8g + 4*cb + j: lane group g of the dQ product then reads its eight
-            // summation slots (tile rows slot_base(g) + j and 16 + slot_base(g) + j) as one 16-byte piece
-            const int slot = 8 * (n >> 2) + 4 * cb + (n & 3);
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-              for (int i = 0; i < 4; i++) {
-                const int w = DSA[cb][2 * nb + (i >> 1)];
-                xs[(16 * nb + 4 * q4 + i) * 32 + slot] = (uint16_t)((i & 1) ? ((unsigned)w >> 16) : ((unsigned)w & 0xffffu));
-              }
-          }
-          Own::reads_done();
-          i32x4 DS[1][NB];
-#pragma unroll
-          for (int nb = 0; nb < NB; nb++) DS[0][nb] = *reinterpret_cast<MODA_LDS const i32x4*>(xs + (16 * nb + n) * 32 + 8 * q4);
-          if (a.accum_depth) fetch_old(col0);
-          TrPipe16<T, HD, 1, NB, 3> kt;
-          kt.prefetch(oa, Kc);
-          kt.run(oa, Kc, DS, dq);
-          Own::reads_done();  // this set and the staging block are free again
+          };
+          flush(Vc, dv_rows, off_v, old_v);
+          flush(Kc, dk_rows, off_k, old_k);
+          Own::reads_done();  // this set may be loaded over
+          tok = next_tok;
+          slot = next_slot;
         }
-        if (nh > 0) gradients(PA, DSA, c_beg + 32 * (nh - 1));
       }
     }
   }

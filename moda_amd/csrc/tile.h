@@ -348,6 +348,34 @@ __device__ __forceinline__ i32x4 rsrc_words(const void* base, uint32_t nbytes) {
   return r;
 }
 
+// Rows through a raw buffer: a lane whose offset lies past its end (kPadOffset) loads zeros or stores nothing, without the
+// branch and the 64-bit address that a guarded access costs.  `base` wave-uniform, offsets in bytes.
+#if defined(__HIP_DEVICE_COMPILE__)
+struct RowBuffer {
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ __forceinline__ RowBuffer(const void* base, uint32_t nbytes) {
+    const i32x4 w = rsrc_words(base, nbytes);
+    const uint64_t p = (uint64_t)(uint32_t)w[0] | ((uint64_t)(uint32_t)w[1] << 32);
+    rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, w[2], w[3]);
+  }
+  __device__ __forceinline__ i32x4 load(int off) const {
+    return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
+  }
+  template <bool NT>  // nontemporal
+  __device__ __forceinline__ void store(const i32x4& v, int off) const {
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, off, 0, NT ? 2 : 0);
+  }
+};
+#else
+struct RowBuffer {  // host pass of the single-source compile: never executed
+  __device__ RowBuffer(const void*, uint32_t) {}
+  __device__ i32x4 load(int) const { return i32x4{0, 0, 0, 0}; }
+  template <bool NT>
+  __device__ void store(const i32x4&, int) const {}
+};
+#endif
+
 __device__ __forceinline__ uint32_t lds_addr(lds_cptr p) { return (uint32_t)(uintptr_t)p; }
 
 // Global -> LDS staging without registers: gfx950 `buffer_load_dwordx4 ... lds`.
@@ -537,6 +565,18 @@ struct WaveTileLoader {
 #pragma unroll
     for (int i = 0; i < N; i++)
       lds_dma<16, NOP>(rs, lds_addr(tile + i * 512), mapped_offset(i, l0, L, Lv, nrows, (int)stride_bytes, d), 0);
+  }
+  // rows rel[i] of the slice part at `base`, counted from there; below zero: zeros.  `pad[i]`: the lane's chunk lies past the head dim
+  __device__ __forceinline__ void fetch_rows(lds_ptr tile, const uint16_t* base, uint32_t stride_bytes, uint32_t nbytes,
+                                             const int (&rel)[N], const bool (&pad)[N]) const {
+    const i32x4 rs = rsrc_words(base, nbytes);
+#pragma unroll
+    for (int i = 0; i < N; i++) lds_dma<16, NOP>(rs, lds_addr(tile + i * 512), row_offset(i, rel[i], (int)stride_bytes, pad[i]), 0);
+  }
+  __host__ __device__ __forceinline__ int chunk(int i) const { return pch ^ Tile<HD>::swz(i * RPW + prow); }
+  __host__ __device__ __forceinline__ int row_offset(int i, int rel, int stride_bytes, bool pad) const {
+    const int off = rel * stride_bytes + chunk(i) * 16;
+    return (pad | (rel < 0)) ? kPadOffset : off;
   }
   // ... from compact column col0 on
   __device__ __forceinline__ void fetch_mapped(lds_ptr tile, const uint16_t* slice, int64_t row_stride, int col0,

@@ -367,9 +367,31 @@ void walk_row_kernel(const KArgs& a_in, bool dq, int rows_per_wave, bool own_pos
             const int col0 = span.c_beg + 32 * j;
             const int nrows = imin(32, span.c_end - col0);
             // where the dQ kernel forms the depth gradients it alternates between two sets of private tiles
+            const bool fused = dq && depth_grads_in_dq(a, HD);
+            const uint32_t fused_first = plan.n_full < ntiles && (Shape::W > 2 || (ntiles - 1) % NST == 0) ? 1u : 0u;
             const uint32_t set = two_sets ? (first ^ (uint32_t)(j & 1)) * stage
-                                          : dq && depth_grads_in_dq(a, HD) ? (uint32_t)(j & 1) * Shape::W * 64 * HD * 2 : 0u;
+                                          : fused ? (fused_first ^ (uint32_t)(j & 1)) * Shape::W * 64 * HD * 2 : 0u;
             for (int i = 0; i < Own::N; i++) {
+              if (fused) {  // rows of the tile and of its gradients, from slot 0 of the first column's token or the column itself
+                const int tok = col0 / a.Lv, slot = col0 - tok * a.Lv, row = i * Own::RPW + own.prow;
+                const int64_t row0 = a.Lv != a.L ? (int64_t)tok * a.L : (int64_t)col0, rows_total = (int64_t)a.T * a.L;
+                const int rel = row < nrows ? (a.Lv != a.L ? mapped_row(slot, row, a.L, a.Lv) : row) : -1;
+                const bool pad_k = own.chunk(i) * 8 >= a.D, pad_v = own.chunk(i) * 8 >= a.Dv;
+                const int vk = own.row_offset(i, rel, (int)a.skd.t * 2, pad_k), vv = own.row_offset(i, rel, (int)a.svd.t * 2, pad_v);
+                check_dma("kd", a.kd + b * a.skd.b + hkv * a.skd.h + row0 * a.skd.t, mapped_bytes(row0, rows_total, (uint32_t)a.skd.t * 2u), vk, 0,
+                          16, kt + set + i * 1024, lds_bytes, vk == kPadOffset);
+                check_dma("vd", a.vd + b * a.svd.b + hkv * a.svd.h + row0 * a.svd.t, mapped_bytes(row0, rows_total, (uint32_t)a.svd.t * 2u), vv, 0,
+                          16, vt + set + i * 1024, lds_bytes, vv == kPadOffset);
+                const int gk = own.row_offset(i, rel, (int)a.sdkd.t * 2, pad_k), gv = own.row_offset(i, rel, (int)a.sdvd.t * 2, pad_v);
+                ctx(kname, (int)block, wave, lane, "own depth gradients");
+                if (rel >= 0 && (row0 + rel) / a.L >= a.T) fail("%s: depth column %d outside the stream", kname, col0 + row);
+                if (rel >= 0 && (row0 + rel) % a.L >= a.Lv) fail("%s: gradient of slot %d of %d filled", kname, (int)((row0 + rel) % a.L), a.Lv);
+                if (gk < 0 || gv < 0) fail("%s: gradient row offset past 31 bits", kname);
+                if (gk != kPadOffset) check_access("dkd", a.dkd + b * a.sdkd.b + hkv * a.sdkd.h + row0 * a.sdkd.t + gk / 2, 16, true);
+                if (gv != kPadOffset) check_access("dvd", a.dvd + b * a.sdvd.b + hkv * a.sdvd.h + row0 * a.sdvd.t + gv / 2, 16, true);
+                ctx(kname, (int)block, wave, lane, "own depth tile");
+                continue;
+              }
               if (a.Lv != a.L) {
                 const int w0 = col0 / a.Lv, l0 = col0 - w0 * a.Lv;
                 const int64_t anchor = (int64_t)w0 * a.L, rows_total = (int64_t)a.T * a.L;
@@ -413,29 +435,11 @@ void walk_row_kernel(const KArgs& a_in, bool dq, int rows_per_wave, bool own_pos
             }
           }
           // dQ kernel outside chunk-visible mode: the same pass forms dK and dV of the wave's own depth columns.
-          // The gradient rows leave 16 at a time through a staging block behind the private tiles, 16 bytes per lane
-          // (WaveTileLoader's row / chunk split).
+          // The gradient rows leave through the tile's own blocks; behind the two sets lies the block through which dS crosses.
           if (dq && depth_grads_in_dq(a, HD)) {
             if (rows_per_wave != 32) fail("%s: depth gradients need 32 rows per wave", kname);
-            const uint32_t stage = 2u * Shape::W * 64 * HD * 2 + (uint32_t)wave * 16 * HD * 2;
-            if (stage + 16 * HD * 2 > lds_bytes) fail("%s: staging block past the LDS allocation", kname);
-            ctx(kname, (int)block, wave, lane, "own depth gradients");
-            constexpr int RPW = Own::RPW, NPASS = 16 / RPW;
-            for (int j = 0; j < nh; j++)
-              for (int cb = 0; cb < 2; cb++) {
-                const int cbase = span.c_beg + 32 * j + 16 * cb;
-                if (cbase >= span.c_end) continue;
-                for (int i = 0; i < NPASS; i++) {
-                  const int row = i * RPW + own.prow;
-                  const int lch = own.pch ^ Tile<HD>::swz(row);
-                  const int c = cbase + row;
-                  if (c >= span.c_end) continue;
-                  if (c / a.Lv >= a.T) fail("%s: depth column %d outside the stream", kname, c);
-                  const int64_t prow = depth_row_of(a, c);
-                  if (lch * 8 < a.Dv) check_access("dvd", a.dvd + b * a.sdvd.b + hkv * a.sdvd.h + prow * a.sdvd.t + lch * 8, 16, true);
-                  if (lch * 8 < a.D) check_access("dkd", a.dkd + b * a.sdkd.b + hkv * a.sdkd.h + prow * a.sdkd.t + lch * 8, 16, true);
-                }
-              }
+            const uint32_t block_at = 2u * Shape::W * 64 * HD * 2 + (uint32_t)wave * 16 * HD * 2;
+            if (block_at + 32 * 32 * 2 > lds_bytes || 16 * HD * 2 < 32 * 32 * 2) fail("%s: dS block past its LDS", kname);
           }
         }
       }
