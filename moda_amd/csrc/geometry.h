@@ -426,6 +426,9 @@ inline bool fp32_one_launch(const KArgs& a) {
 // ms; head dim 64, 64 heads: 10.4 -> 10.9 ms).  Below that:
 // dkv_kernel, fixed length: the same power of two for every tile, segments of the heaviest of at least 16 trips (a trip:
 // one query tile of one query head).  3057 tokens, 32 query heads on four: 538 -> 430 us when the heads count as trips.
+// While compute units have no workgroup at all, of at least 4: the serial chain of the longest is all there is (training steps, 16
+// and 4: 710 tokens, four heads of four, 16 slots 123 -> 101 us; 1500, two of two, eight slots 142 -> 121; 900, sixteen query
+// heads on four 116 -> 87; at least 6 or 10: up to 8 % more).
 // dkv_kernel, packed, tiles wider than 64: not cut.  There a packed batch returns bit for bit what separate calls return
 // that have no room for segments, and that is kept although the cut is faster (a training step of 2600 + 168 + 900 + 400
 // + 1500 tokens, four heads of four, eight slots: 329 us cut, 435 not; of 6000 + 3000 + 500, two heads of four: 641, 894).
@@ -444,7 +447,7 @@ inline DkvSplit dkv_split_plan(const KArgs& a, int HD) {
   if (tiles >= (flat ? 768 : 512)) return {1, 0};
   if (!flat && !a.cu) {
     int s = 1;
-    while (tiles * s < 512 && s < 8 && nqt * a.hdiv / (2 * s) >= 16 && nqt >= 4 * s) s *= 2;
+    while (tiles * s < 512 && s < 8 && nqt * a.hdiv / (2 * s) >= (tiles * s < 256 ? 4 : 16) && nqt >= 2 * s) s *= 2;
     return {s, 0};
   }
   const int64_t trips = tiles * (a.causal ? (nqt + 1) / 2 : nqt) * a.hdiv / (flat ? 768 : 256);  // of one place
