@@ -196,7 +196,7 @@ MODA_HD bool waves_own_depth(const KArgs& a, int Ld) { return Ld > 0 && (!a.chun
 // depth-column kernel, which every other case runs from the dK/dV launch.
 constexpr int kDepthGradsInDqMaxWidth = 64;
 MODA_HD bool depth_grads_in_dq(const KArgs& a, int HD) {
-  return a.L > 0 && !a.chunk && HD <= kDepthGradsInDqMaxWidth && 32 % a.Gf == 0;
+  return a.L > 0 && !a.chunk && HD <= kDepthGradsInDqMaxWidth && 32 % a.Gf == 0 && !a.far_depth_grads;
 }
 
 // ... and where the dQ kernel's waves walk their own depth columns without forming the gradients (the 128-wide tiles,

@@ -2463,3 +2463,20 @@ def test_short_rows_by_tile_and_depth(gpu_device, B, T, H, G, L, valid, causal):
         ref[n] = oracle.scatter_depth_grad(ref[n], T, L)
     got = {"o": o, "lse": lse, "dq": dq, "dk": dk, "dv": dv, "dkd": dkd, "dvd": dvd}
     compare_all({n: x[some] for n, x in got.items()}, ref, dtype, f"B{B} T{T} valid {valid}")
+
+
+def test_depth_gradients_into_rows_far_apart(gpu_device):
+    """Gradient buffers whose rows lie further apart than a tile's 32-bit offsets reach (the inputs' rows need not)."""
+    from moda_amd import ops
+
+    B, T, H, D, L, G, valid = 1, 3, 1, 64, 64, 2, 1
+    inp = to_dev(oracle.make_inputs(B, T, H, D, L, G, seed=5, dtype=torch.bfloat16, std=0.5), gpu_device)
+    args = [inp[n] for n in ("q", "k", "v", "kd", "vd")]
+    o, lse = ops._raw_fwd(1, *args, 0.125, G, depth_valid=valid)
+    near = ops._raw_bwd(1, *args, o, lse, inp["do"], 0.125, G, depth_valid=valid)
+    row = (1 << 31) // ((64 // valid + 2) * L * 2) + 8
+    row += -row % 8
+    far = [torch.empty_strided((B, T * L, H, D), (T * L * row, row, D, 1), dtype=torch.bfloat16, device=gpu_device) for _ in range(2)]
+    got = ops._raw_bwd(1, *args, o, lse, inp["do"], 0.125, G, depth_valid=valid, out=[torch.empty_like(x) for x in near[:3]] + far)
+    for n, a, b in zip(("dq", "dk", "dv", "dkd", "dvd"), near, got):
+        check(n, b.contiguous(), a.float().cpu(), torch.bfloat16, "rows far apart")
