@@ -2480,3 +2480,42 @@ def test_depth_gradients_into_rows_far_apart(gpu_device):
     got = ops._raw_bwd(1, *args, o, lse, inp["do"], 0.125, G, depth_valid=valid, out=[torch.empty_like(x) for x in near[:3]] + far)
     for n, a, b in zip(("dq", "dk", "dv", "dkd", "dvd"), near, got):
         check(n, b.contiguous(), a.float().cpu(), torch.bfloat16, "rows far apart")
+
+
+@pytest.mark.parametrize("what", ["same", "others", "written", "other stream", "attended twice", "other heads", "wide"])
+def test_a_layer_copied_by_its_attention_call_is_what_was_pushed(gpu_device, what):
+    """The forward launch copies k and v to the slot they would get; what later layers see is what push() was given."""
+    import moda_amd
+
+    B, T, G, D, L = (2, 70, 2, 128 if what == "wide" else 64, 3)
+    gen = torch.Generator().manual_seed(11)
+    new = lambda H: (torch.randn(B, T, H, D, generator=gen) * 0.5).to(gpu_device, torch.bfloat16)
+    stream = moda_amd.DepthStream(L)
+    pushed = []
+    for i in range(3):
+        H = 2 if what == "other heads" and i == 0 else 1
+        q, k, v = (torch.cat([new(H)] * G, 1) if n == "q" else new(H) for n in "qkv")
+        for x in (q, k, v):
+            x.requires_grad_()
+        o = stream.attend(q, k, v, moda_group_num=G, is_causal=False)
+        if i:
+            cache = [moda_amd.stack_depth([p[j] for p in pushed]) for j in (0, 1)]
+            want = moda_amd.parallel_moda(q.detach(), k.detach(), v.detach(), cached_k=cache[0], cached_v=cache[1], moda_group_num=G,
+                                          is_causal=False, need_lse=True, warn_shape=False)[0]
+            check("o", o, want.float().cpu(), torch.bfloat16, what)
+        if what in ("others", "other heads"):
+            k, v = new(1).requires_grad_(), new(1).requires_grad_()
+        if what == "written":
+            with torch.no_grad():
+                k.mul_(-2), v.add_(1)
+        if what == "attended twice":
+            stream.attend(q, new(1).requires_grad_(), new(1).requires_grad_(), moda_group_num=G, is_causal=False)
+        if what == "other stream":
+            side = torch.cuda.Stream()
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                stream.push(k, v)
+            torch.cuda.current_stream().wait_stream(side)
+        else:
+            stream.push(k, v)
+        pushed.append((k.detach().clone(), v.detach().clone()))
