@@ -249,9 +249,12 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
     pv.run(oa, Vc, P, o);
   };
   // 32 columns, masked
-  auto half_tile = [&](lds_cptr Kc, lds_cptr Vc, int col0, int lo, int hi) {
+  auto half_tile = [&](lds_cptr Kc, lds_cptr Vc, int col0, int lo, int hi, auto&& after_scores) {
     TrPipe<T, HD, 2, 2> pv1;
-    front(std::true_type{}, one, Kc, col0, lo, hi, [&]() { pv1.prefetch(oa, Vc); });
+    front(std::true_type{}, one, Kc, col0, lo, hi, [&]() {
+      after_scores();
+      pv1.prefetch(oa, Vc);
+    });
     const i32x4 P1[2] = {P[0], P[1]};
     pv1.run(oa, Vc, P1, o);
   };
@@ -357,7 +360,7 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
       } else {  // by halves: the last tile of a sequence is as often as not seen by no row beyond its first half
 #pragma unroll 1
         for (int c = col0; c < col0 + BN; c += 32, Kc += 32 * HD)
-          if (__any((hi > c) && (lo < c + 32) && (hi > lo))) half_tile(Kc, Kc + BN * HD, c, lo, hi);
+          if (__any((hi > c) && (lo < c + 32) && (hi > lo))) half_tile(Kc, Kc + BN * HD, c, lo, hi, []() {});
       }
       c_st = (c_st + 1 == NST) ? 0 : c_st + 1;
       if (it + 1 < ntiles) wait_tile(it + 1);
@@ -423,7 +426,9 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
     if (!EARLY) __syncthreads();  // (EARLY: every tile ends with one)
     if (!early) enter_depth();
     const int nh = (c_end - c_beg + 31) / 32;
-    if (TWO_SETS) {
+    // (Depth-only launches stream from memory; a second tile on its way costs them 4 %: 102 x 197 tokens of two rows, ten slots, 13.1
+    // and 13.7 us.)
+    if (TWO_SETS && a.has_seq) {
       if (!early && nh > 0) fetch_early();
       for (int j = 0; j < nh; j++) {
         const int col0 = c_beg + 32 * j;
@@ -432,16 +437,21 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
           fetch(own_tile((j + 1) & 1), kdp, a.skd.t, col0 + 32, a.D);
           fetch(own_tile((j + 1) & 1) + 32 * HD, vdp, a.svd.t, col0 + 32, a.Dv);
           next_columns();
-          Own::template wait_but<2 * Own::N>();
+          Own::template wait_but<3 * Own::N>();  // K landed, V may still be on its way
         } else {
-          Own::template wait_but<0>();
+          Own::template wait_but<Own::N>();
         }
-        half_tile(Kt, Kt + 32 * HD, col0, dlo, dhi);
+        half_tile(Kt, Kt + 32 * HD, col0, dlo, dhi, [&]() {
+          if (j + 1 < nh)
+            Own::template wait_but<2 * Own::N>();
+          else
+            Own::template wait_but<0>();
+        });
         Own::reads_done();
       }
     } else if (nh > 0) {
       // The next K tile is fetched as soon as the scores are out, the next V tile once the V product is.
-      lds_ptr Kt = own_tile(0), Vt = EARLY ? own_tile(1) : Kt + 32 * HD;
+      lds_ptr Kt = own_tile(0), Vt = EARLY && !TWO_SETS ? own_tile(1) : Kt + 32 * HD;
       if (!early) fetch(Kt, kdp, a.skd.t, c_beg, a.D);
       fetch(Vt, vdp, a.svd.t, c_beg, a.Dv);
       for (int j = 0; j < nh; j++) {
