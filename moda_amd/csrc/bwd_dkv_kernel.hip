@@ -721,13 +721,13 @@ __global__ __launch_bounds__(256) void depth_cols_kernel(const KArgs a) {
 // (KArgs::depth_p, depth_ds): no kd, vd, no scores -- per column G scalar pairs and the G rows of q and do, which the
 // L columns of a token share through the caches.  The launch moves the gradient rows out and little else.
 template <typename T, int HD>
-__global__ __launch_bounds__(256) void depth_cols_handed_kernel(const KArgs a) {
+__device__ __forceinline__ void depth_cols_handed(const KArgs& a, int wg) {
   constexpr int LPC = HD / 8, CPW = 64 / LPC, CPB = 4 * CPW;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int sub = lane % LPC;
   const int BHk = a.B * a.Hkv;
-  const int bh = blockIdx.x % BHk, b = bh / a.Hkv, hkv = bh % a.Hkv;
-  const int64_t c = (int64_t)(blockIdx.x / BHk) * CPB + wave * CPW + lane / LPC;
+  const int bh = wg % BHk, b = bh / a.Hkv, hkv = bh % a.Hkv;
+  const int64_t c = (int64_t)(wg / BHk) * CPB + wave * CPW + lane / LPC;
   if (c >= (int64_t)a.T * a.L) return;  // whole lane groups leave together
   const int w = (int)(c / a.L), slot = (int)(c - (int64_t)w * a.L);
   uint16_t* dk_out = a.dkd + b * a.sdkd.b + hkv * a.sdkd.h + c * a.sdkd.t + 8 * sub;
@@ -793,13 +793,13 @@ __global__ __launch_bounds__(256) void depth_cols_handed_kernel(const KArgs a) {
 // dim each) keep the token's rows of q and do in registers and walk its slots, so that q and do are read once per
 // token instead of once per slot and the launch is little more than the stream of gradient rows going out.
 template <typename T, int HD>
-__global__ __launch_bounds__(256) void depth_token_handed_kernel(const KArgs a) {
+__device__ __forceinline__ void depth_token_handed(const KArgs& a, int wg) {
   constexpr int LPT = HD / 8, TPW = 64 / LPT, TPB = 4 * TPW, GMAX = 4;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int sub = lane % LPT;
   const int BHk = a.B * a.Hkv;
-  const int bh = blockIdx.x % BHk, b = bh / a.Hkv, hkv = bh % a.Hkv;
-  const int w = (blockIdx.x / BHk) * TPB + wave * TPW + lane / LPT;
+  const int bh = wg % BHk, b = bh / a.Hkv, hkv = bh % a.Hkv;
+  const int w = (wg / BHk) * TPB + wave * TPW + lane / LPT;
   if (w >= a.T) return;  // whole lane groups leave together
   const bool in_k = 8 * sub < a.D, in_v = 8 * sub < a.Dv;
   auto load8 = [&](const uint16_t* p, float (&f)[8], bool in_dim) {
@@ -889,16 +889,16 @@ __global__ __launch_bounds__(256) void zero_unfilled_slots_kernel(const KArgs a,
 // workgroup finished first) and writes dk, dv in the tensor type.  One thread per 8 head-dim elements.  BN, BM: the
 // column and query tiles of the launch that left them; its tiles of one segment have written their rows themselves.
 template <typename T, int HD, bool VARLEN>
-__global__ __launch_bounds__(256) void dkv_reduce_kernel(const KArgs a_in, int BN, int BM) {
+__device__ __forceinline__ void dkv_reduce(const KArgs& a_in, int BN, int BM, int wg) {
   constexpr int TPR = HD / 8, RPB = 256 / TPR;
   const int BHk = a_in.B * a_in.Hkv;
-  const int bh = blockIdx.x % BHk;
+  const int bh = wg % BHk;
   int b = bh / a_in.Hkv;
   const int hkv = bh % a_in.Hkv, sub = threadIdx.x % TPR;
   const int first = VARLEN ? a_in.cu[b] : 0;
   SeqArgs<VARLEN> seq(a_in, b);
   const KArgs& a = seq.a;
-  const int c = (int)(blockIdx.x / BHk) * RPB + threadIdx.x / TPR;
+  const int c = (int)(wg / BHk) * RPB + threadIdx.x / TPR;
   if (c >= a.T) return;
   const int c_first = c / BN * BN, row0 = a.causal ? c_first * a.Gf : 0;
   const int nsegs = tile_segments(a, (a.Tq + BM - 1) / BM - row0 / BM, a.dkv_split);
@@ -941,6 +941,32 @@ __global__ __launch_bounds__(256) void dkv_reduce_kernel(const KArgs a_in, int B
   }
 }
 
+template <typename T, int HD>
+__global__ __launch_bounds__(256) void depth_cols_handed_kernel(const KArgs a) {
+  depth_cols_handed<T, HD>(a, (int)blockIdx.x);
+}
+template <typename T, int HD>
+__global__ __launch_bounds__(256) void depth_token_handed_kernel(const KArgs a) {
+  depth_token_handed<T, HD>(a, (int)blockIdx.x);
+}
+template <typename T, int HD, bool VARLEN>
+__global__ __launch_bounds__(256) void dkv_reduce_kernel(const KArgs a, int BN, int BM) {
+  dkv_reduce<T, HD, VARLEN>(a, BN, BM, (int)blockIdx.x);
+}
+// The last two of a backward pass in one launch, `reduce_blocks` workgroups of the first: both move memory, neither waits for the
+// other, and a launch more is 4 - 5 us (a training step of 710 tokens, four heads of four, 16 slots: 101 -> 96 us; 1500, two heads of
+// two, eight slots: 121 -> 116; 2 x 4096: 644 -> 640).
+template <typename T, int HD, bool BY_TOKEN>
+__global__ __launch_bounds__(256) void reduce_and_depth_kernel(const KArgs a, int BN, int BM, int reduce_blocks) {
+  const int block = (int)blockIdx.x;
+  if (block < reduce_blocks)
+    dkv_reduce<T, HD, false>(a, BN, BM, block);
+  else if (BY_TOKEN)
+    depth_token_handed<T, HD>(a, block - reduce_blocks);
+  else
+    depth_cols_handed<T, HD>(a, block - reduce_blocks);
+}
+
 hipError_t launch_dkv_flat(const KArgs& a, int dtype, hipStream_t stream);  // bwd_dkv_flat_kernel.hip
 
 template <typename T, int HD>
@@ -968,7 +994,26 @@ hipError_t launch_dkv_t(const KArgs& a, hipStream_t stream) {
                               : (nseg > 1 ? go(&dkv_kernel<T, HD, false, true>, attr[2]) : go(&dkv_kernel<T, HD, false>, attr[3]));
     if (e != hipSuccess) return e;
   }
-  if (nseg > 1 && n_seq_tiles > 0) {
+  // depth columns: vector kernel, except in chunk-visible mode where a column has up to G*Cb visible rows
+  const bool in_dq = depth_grads_in_dq(a, HD);  // the dQ launch has formed the depth slots' dK and dV already
+  const bool depth_by_columns = a.L > 0 && !a.chunk && !in_dq;
+  const bool depth_by_chunks = moda::depth_by_chunks(a, HD);
+  const bool reduces = nseg > 1 && n_seq_tiles > 0;
+  if constexpr (HD == 128) {
+    if (reduces && depth_by_columns && a.depth_p && !a.cu && (int64_t)a.B * a.T > 0) {
+      constexpr int RPB = 256 / (HD / 8);  // rows, tokens or columns of a workgroup
+      const bool by_token = a.Gf <= 4;
+      const int64_t heads = (int64_t)a.B * a.Hkv, rows = ((int64_t)a.T + RPB - 1) / RPB * heads;
+      const int64_t n = rows + ((int64_t)a.T * (by_token ? 1 : a.L) + RPB - 1) / RPB * heads;
+      if (n >= (1ll << 31)) return hipErrorInvalidValue;
+      if (by_token)
+        hipLaunchKernelGGL((reduce_and_depth_kernel<T, HD, true>), dim3((unsigned)n), dim3(256), 0, stream, a, BN, BM, (int)rows);
+      else
+        hipLaunchKernelGGL((reduce_and_depth_kernel<T, HD, false>), dim3((unsigned)n), dim3(256), 0, stream, a, BN, BM, (int)rows);
+      return hipGetLastError();
+    }
+  }
+  if (reduces) {
     const int rpb = 256 / (HD / 8), bm = flat ? 32 : BM;
     const dim3 grid((unsigned)(((int64_t)a.T + rpb - 1) / rpb * a.B * a.Hkv));
     if (HD <= 64 && a.cu)
@@ -978,10 +1023,6 @@ hipError_t launch_dkv_t(const KArgs& a, hipStream_t stream) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
-  // depth columns: vector kernel, except in chunk-visible mode where a column has up to G*Cb visible rows
-  const bool in_dq = depth_grads_in_dq(a, HD);  // the dQ launch has formed the depth slots' dK and dV already
-  const bool depth_by_columns = a.L > 0 && !a.chunk && !in_dq;
-  const bool depth_by_chunks = moda::depth_by_chunks(a, HD);
   if (a.L > 0 && (a.chunk || in_dq) && a.Lv != a.L && !a.keep_slots && (int64_t)a.B * a.T > 0) {
     // packed batch: one row axis of all sequences (its length is the row-sum pitch / G), else B x T * L rows
     const int64_t rows = a.cu ? (int64_t)(a.delta_pitch / a.Gf) * a.L : (int64_t)a.T * a.L;
