@@ -721,7 +721,7 @@ __global__ __launch_bounds__(256) void depth_cols_kernel(const KArgs a) {
 // (KArgs::depth_p, depth_ds): no kd, vd, no scores -- per column G scalar pairs and the G rows of q and do, which the
 // L columns of a token share through the caches.  The launch moves the gradient rows out and little else.
 template <typename T, int HD>
-__device__ __forceinline__ void depth_cols_handed(const KArgs& a, int wg) {
+__device__ __forceinline__ void depth_cols_handed(const KArgs& a, unsigned wg) {
   constexpr int LPC = HD / 8, CPW = 64 / LPC, CPB = 4 * CPW;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int sub = lane % LPC;
@@ -793,7 +793,7 @@ __device__ __forceinline__ void depth_cols_handed(const KArgs& a, int wg) {
 // dim each) keep the token's rows of q and do in registers and walk its slots, so that q and do are read once per
 // token instead of once per slot and the launch is little more than the stream of gradient rows going out.
 template <typename T, int HD>
-__device__ __forceinline__ void depth_token_handed(const KArgs& a, int wg) {
+__device__ __forceinline__ void depth_token_handed(const KArgs& a, unsigned wg) {
   constexpr int LPT = HD / 8, TPW = 64 / LPT, TPB = 4 * TPW, GMAX = 4;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int sub = lane % LPT;
@@ -889,7 +889,7 @@ __global__ __launch_bounds__(256) void zero_unfilled_slots_kernel(const KArgs a,
 // workgroup finished first) and writes dk, dv in the tensor type.  One thread per 8 head-dim elements.  BN, BM: the
 // column and query tiles of the launch that left them; its tiles of one segment have written their rows themselves.
 template <typename T, int HD, bool VARLEN>
-__device__ __forceinline__ void dkv_reduce(const KArgs& a_in, int BN, int BM, int wg) {
+__device__ __forceinline__ void dkv_reduce(const KArgs& a_in, int BN, int BM, unsigned wg) {
   constexpr int TPR = HD / 8, RPB = 256 / TPR;
   const int BHk = a_in.B * a_in.Hkv;
   const int bh = wg % BHk;
@@ -943,22 +943,22 @@ __device__ __forceinline__ void dkv_reduce(const KArgs& a_in, int BN, int BM, in
 
 template <typename T, int HD>
 __global__ __launch_bounds__(256) void depth_cols_handed_kernel(const KArgs a) {
-  depth_cols_handed<T, HD>(a, (int)blockIdx.x);
+  depth_cols_handed<T, HD>(a, blockIdx.x);
 }
 template <typename T, int HD>
 __global__ __launch_bounds__(256) void depth_token_handed_kernel(const KArgs a) {
-  depth_token_handed<T, HD>(a, (int)blockIdx.x);
+  depth_token_handed<T, HD>(a, blockIdx.x);
 }
 template <typename T, int HD, bool VARLEN>
 __global__ __launch_bounds__(256) void dkv_reduce_kernel(const KArgs a, int BN, int BM) {
-  dkv_reduce<T, HD, VARLEN>(a, BN, BM, (int)blockIdx.x);
+  dkv_reduce<T, HD, VARLEN>(a, BN, BM, blockIdx.x);
 }
 // The last two of a backward pass in one launch, `reduce_blocks` workgroups of the first: both move memory, neither waits for the
 // other, and a launch more is 4 - 5 us (a training step of 710 tokens, four heads of four, 16 slots: 101 -> 96 us; 1500, two heads of
 // two, eight slots: 121 -> 116; 2 x 4096: 644 -> 640).
 template <typename T, int HD, bool BY_TOKEN>
-__global__ __launch_bounds__(256) void reduce_and_depth_kernel(const KArgs a, int BN, int BM, int reduce_blocks) {
-  const int block = (int)blockIdx.x;
+__global__ __launch_bounds__(256) void reduce_and_depth_kernel(const KArgs a, int BN, int BM, unsigned reduce_blocks) {
+  const unsigned block = blockIdx.x;
   if (block < reduce_blocks)
     dkv_reduce<T, HD, false>(a, BN, BM, block);
   else if (BY_TOKEN)
@@ -1005,12 +1005,15 @@ hipError_t launch_dkv_t(const KArgs& a, hipStream_t stream) {
       const bool by_token = a.Gf <= 4;
       const int64_t heads = (int64_t)a.B * a.Hkv, rows = ((int64_t)a.T + RPB - 1) / RPB * heads;
       const int64_t n = rows + ((int64_t)a.T * (by_token ? 1 : a.L) + RPB - 1) / RPB * heads;
-      if (n >= (1ll << 31)) return hipErrorInvalidValue;
-      if (by_token)
-        hipLaunchKernelGGL((reduce_and_depth_kernel<T, HD, true>), dim3((unsigned)n), dim3(256), 0, stream, a, BN, BM, (int)rows);
-      else
-        hipLaunchKernelGGL((reduce_and_depth_kernel<T, HD, false>), dim3((unsigned)n), dim3(256), 0, stream, a, BN, BM, (int)rows);
-      return hipGetLastError();
+      // By columns up to 32768 workgroups: one launch against two takes 190 to 194 us a training step at 4.1 K workgroups, 310 to 315
+      // at 16.4 K and 429 to 435 at 32.8 K, but 814 to 809 at 65 K and 1918 to 1897 at 122 K.
+      if (n <= (by_token ? (1ll << 31) - 1 : 32768)) {
+        if (by_token)
+          hipLaunchKernelGGL((reduce_and_depth_kernel<T, HD, true>), dim3((unsigned)n), dim3(256), 0, stream, a, BN, BM, (unsigned)rows);
+        else
+          hipLaunchKernelGGL((reduce_and_depth_kernel<T, HD, false>), dim3((unsigned)n), dim3(256), 0, stream, a, BN, BM, (unsigned)rows);
+        return hipGetLastError();
+      }
     }
   }
   if (reduces) {

@@ -2465,6 +2465,24 @@ def test_short_rows_by_tile_and_depth(gpu_device, B, T, H, G, L, valid, causal):
     compare_all({n: x[some] for n, x in got.items()}, ref, dtype, f"B{B} T{T} valid {valid}")
 
 
+@pytest.mark.parametrize("B,T,H,G,L", [(2, 260, 1, 4, 5), (1, 161, 3, 8, 3), (64, 130, 1, 8, 64)], ids=["by-token", "by-columns", "two-launches"])
+def test_partial_sums_and_depth_gradients_of_wide_heads(gpu_device, B, T, H, G, L):
+    """dK/dV in row segments, and the depth gradients from handed-over probabilities in the same launch, or in one of their own where
+    the columns need more than 32768 workgroups (64 batches x (9 + 520)); odd ends of both halves' workgroups of 16 rows."""
+    from moda_amd import ops
+
+    scale = 128**-0.5
+    inp = oracle.make_inputs(B, T, H, 128, L, G, seed=B + T, dtype=torch.bfloat16, std=0.5)
+    dev = to_dev(inp, gpu_device)
+    args = [dev[n] for n in ("q", "k", "v", "kd", "vd")]
+    o, lse = ops._raw_fwd(MODE_ID["causal"], *args, scale, G)
+    grads = ops._raw_bwd(MODE_ID["causal"], *args, o, lse, dev["do"], scale, G)
+    some = sorted({0, B - 1})
+    ref = oracle.moda_dense_fwd_bwd({n: x[some] for n, x in inp.items()}, scale, G, "causal")
+    got = dict(zip(("o", "lse", "dq", "dk", "dv", "dkd", "dvd"), (o, lse, *grads)))
+    compare_all({n: x[some] for n, x in got.items()}, ref, torch.bfloat16, f"B{B} T{T} H{H} G{G} L{L}")
+
+
 def test_depth_gradients_into_rows_far_apart(gpu_device):
     """Gradient buffers whose rows lie further apart than a tile's 32-bit offsets reach (the inputs' rows need not)."""
     from moda_amd import ops
