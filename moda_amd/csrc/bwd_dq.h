@@ -443,12 +443,12 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
           }
         const int gshift = __builtin_ctz(a.Gf);  // Gf divides 32: a power of two
         const int nh = (c_end - c_beg + 31) / 32;
-        // token of the query row on accumulator register i of block nb; -1 past the end
-        int row_token[NB][4];
+        // Token of the query row on accumulator register i of block nb: the first register's and i >> gshift more (rows past the end
+        // belong to tokens that no column has).  Every register counts here: spilled ones, 11 in fp16, cost a launch that streams
+        // from memory 5 %.
+        int row_token[NB];
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-          for (int i = 0; i < 4; i++) row_token[nb][i] = rq + 16 * nb + i < a.Tq ? (rq + 16 * nb + i) >> gshift : -1;
+        for (int nb = 0; nb < NB; nb++) row_token[nb] = (rq + 16 * nb) >> gshift;
         const uint16_t* dkdp = a.dkd + b * a.sdkd.b + hkv * a.sdkd.h;
         const uint16_t* dvdp = a.dvd + b * a.sdvd.b + hkv * a.sdvd.h;
         const int lrow = slot_base(n >> 2) + (n & 3);  // tile row (of a 16-row block) whose column this lane holds
@@ -474,12 +474,11 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
             Own::template wait_but<0>();
           else
             Own::template wait_but<2 * Own::N>();
-          int off_k[Own::N], off_v[Own::N];  // this lane's pieces of the gradient rows
+          int grow[Own::N];  // this lane's rows of the tile
 #pragma unroll
-          for (int i = 0; i < Own::N; i++) {
-            off_k[i] = own.row_offset(i, rel[i], (int)a.sdkd.t * 2, pad_k[i]);
-            off_v[i] = own.row_offset(i, rel[i], (int)a.sdvd.t * 2, pad_v[i]);
-          }
+          for (int i = 0; i < Own::N; i++) grow[i] = rel[i];
+          auto off_k = [&](int i) { return own.row_offset(i, grow[i], (int)a.sdkd.t * 2, pad_k[i]); };
+          auto off_v = [&](int i) { return own.row_offset(i, grow[i], (int)a.sdvd.t * 2, pad_v[i]); };
           const int64_t row0 = tile_row(tok, col0);
           const RowBuffer dk_rows(dkdp + row0 * a.sdkd.t, kPadOffset), dv_rows(dvdp + row0 * a.sdvd.t, kPadOffset);
           if (j + 1 < nh) fetch((j + 1) & 1, col0 + 32, next_tok, next_slot);
@@ -491,8 +490,8 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
           if (a.accum_depth) {
 #pragma unroll
             for (int i = 0; i < Own::N; i++) {
-              old_v[i] = dv_rows.load(off_v[i]);
-              old_k[i] = dk_rows.load(off_k[i]);
+              old_v[i] = dv_rows.load(off_v(i));
+              old_k[i] = dk_rows.load(off_k(i));
             }
           }
 #pragma unroll
@@ -504,7 +503,7 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
 #pragma unroll
               for (int i = 0; i < 4; i++) {
                 float pv = fast_exp2(__builtin_fmaf(s[cb][nb][i], sc, -lse4[nb][i]));
-                pv = row_token[nb][i] == tokc ? pv : 0.f;
+                pv = tokc - row_token[nb] == (i >> gshift) ? pv : 0.f;
                 p[nb][i] = pv;
                 ds[nb][i] = pv * dp[cb][nb][i];
               }
@@ -541,7 +540,7 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
               put(Kc, cb, mb, mfma16<T>(QT[mb], DSA[cb], z), a.scale);
             }
           Own::reads_done();
-          auto flush = [&](lds_ptr block, const RowBuffer& rows, const int (&off)[Own::N], const i32x4 (&old)[Own::N]) {
+          auto flush = [&](lds_ptr block, const RowBuffer& rows, auto&& off, const i32x4 (&old)[Own::N]) {
 #pragma unroll
             for (int i = 0; i < Own::N; i++) {
               i32x4 val = *reinterpret_cast<MODA_LDS const i32x4*>(block + i * 512 + lane * 8);
@@ -554,7 +553,7 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
                   val[w] = pack2<T>(x0 + y0, x1 + y1);
                 }
               }
-              rows.template store<true>(val, off[i]);  // next read by another launch
+              rows.template store<true>(val, off(i));  // next read by another launch
             }
           };
           flush(Vc, dv_rows, off_v, old_v);
