@@ -191,10 +191,12 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
     f32x16 s[NBLK];
     mfma_rows<T, HD, NBLK, 4>(oa, Kc, Qr, s);
     after_scores();
-    // whether the row sees register i of block bb, a column of [lo, hi): by its distance from lo
+    // whether the row sees register i of block bb, a column of [lo, hi): by its distance from lo (0 without depth)
     const int before = col0 + 4 * g - lo;
     const unsigned width = (unsigned)(hi > lo ? hi - lo : 0);
-    auto sees = [&](int bb, int i) { return (unsigned)(before + 32 * bb + acc_row(i, 0)) < width; };
+    auto sees = [&](int bb, int i) {
+      return NODEPTH ? col0 + 32 * bb + acc_row(i, g) < hi : (unsigned)(before + 32 * bb + acc_row(i, 0)) < width;
+    };
     // row maximum of the raw scores (scale > 0, so it commutes with the max)
     float mx = kNegInf;
 #pragma unroll
@@ -271,7 +273,7 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
   // for two whole sets, one in each stage, and fetch a tile ahead all the way; four for K in one stage and V in the other.
   // A short launch is bound by what one wave has to do, one thing after the other: 64 x 197 tokens of four rows, eleven of
   // twelve slots filled, 35.5 k cycles a wave with every private tile waited for and 13.7 k of them in this pass; now 29.1 k
-  // and 7.0 k, the launch 16.5 -> 13.9 us (six slots 14.1 -> 12.5, none 8.9 -> 8.5).
+  // and 7.0 k, the launch 16.5 -> 13.9 us (six slots 14.1 -> 12.5).
   constexpr bool EARLY = !NODEPTH && !PP && NST == 2 && HD <= 64, TWO_SETS = EARLY && Shape::W <= 2;
   typedef WaveTileLoader<HD> Own;
   Own own;
@@ -355,9 +357,11 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
       const int lo = dep ? dlo : 0;
       const int hi = dep ? dhi : shi;
       lds_cptr Kc = stage_k(c_st);
-      if (PP) {
+      if (PP || NODEPTH) {
         if (__any((hi > col0) && (lo < col0 + BN) && (hi > lo))) tile(std::true_type{}, Kc, Kc + BN * HD, col0, lo, hi);
-      } else {  // by halves: the last tile of a sequence is as often as not seen by no row beyond its first half
+      } else {  // by halves: the last tile of a sequence is as often as not seen by no row beyond its first half, and depth needs them anyway.
+        // (Without depth the whole tile at once is faster: 3 x 500 tokens, two heads of eight, causal, 11.7 us by halves and 11.3 whole;
+        // 64 x 240, three of two, 18.4 and 17.7; 64 x 197, six heads, where five columns are left, 13.1 and 12.9.)
 #pragma unroll 1
         for (int c = col0; c < col0 + BN; c += 32, Kc += 32 * HD)
           if (__any((hi > c) && (lo < c + 32) && (hi > lo))) half_tile(Kc, Kc + BN * HD, c, lo, hi, []() {});
