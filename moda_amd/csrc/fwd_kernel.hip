@@ -13,7 +13,7 @@
 // The vector work of the softmax costs as much as the products (more on the
 // 64-wide tiles), so the loop over column tiles is split in two: tiles every row
 // of the workgroup sees completely run a body without any masking or visibility
-// tests; boundary and depth tiles run the masked body, 32 columns at a time.
+// tests; boundary and depth tiles run the masked body.
 #include <type_traits>
 
 #include "geometry.h"
@@ -357,14 +357,15 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
       const int lo = dep ? dlo : 0;
       const int hi = dep ? dhi : shi;
       lds_cptr Kc = stage_k(c_st);
-      if (PP || NODEPTH) {
-        if (__any((hi > col0) && (lo < col0 + BN) && (hi > lo))) tile(std::true_type{}, Kc, Kc + BN * HD, col0, lo, hi);
-      } else {  // by halves: the last tile of a sequence is as often as not seen by no row beyond its first half, and depth needs them anyway.
-        // (Without depth the whole tile at once is faster: 3 x 500 tokens, two heads of eight, causal, 11.7 us by halves and 11.3 whole;
-        // 64 x 240, three of two, 18.4 and 17.7; 64 x 197, six heads, where five columns are left, 13.1 and 12.9.)
-#pragma unroll 1
-        for (int c = col0; c < col0 + BN; c += 32, Kc += 32 * HD)
-          if (__any((hi > c) && (lo < c + 32) && (hi > lo))) half_tile(Kc, Kc + BN * HD, c, lo, hi, []() {});
+      const auto seen = [&](int c, int cols) { return __any((hi > c) && (lo < c + cols) && (hi > lo)); };
+      if (HD <= 64 && !NODEPTH && seen(col0, 32) != seen(col0 + 32, 32)) {
+        // No row of the wave sees the other half, as in every second last tile of a sequence: 32 columns give the bits of the whole tile,
+        // which takes one maximum over all of them.  (Without depth the whole tile is as fast: 64 x 197 tokens, six heads, five columns
+        // left, 13.1 us by halves and 12.9.)
+        const int half = seen(col0, 32) ? 0 : 32;
+        half_tile(Kc + half * HD, Kc + (BN + half) * HD, col0 + half, lo, hi, []() {});
+      } else if (seen(col0, BN)) {
+        tile(std::true_type{}, Kc, Kc + BN * HD, col0, lo, hi);
       }
       c_st = (c_st + 1 == NST) ? 0 : c_st + 1;
       if (it + 1 < ntiles) wait_tile(it + 1);

@@ -1222,6 +1222,41 @@ def test_packed_batches_of_many_sequences_equal_separate_calls_bitwise(gpu_devic
     test_small_packed_batches_of_long_sequences_equal_separate_calls_bitwise(gpu_device, (lengths,) + case[1:])
 
 
+@pytest.mark.parametrize("case", [
+    # lengths, H, D, L, G, mode, chunk: 512 or more workgroups of 256 rows together, fewer each, so that the packed launch takes
+    # eight waves half a tile apart and the separate calls take four: sequences that end in either half of a key tile, in every mode
+    ((1030, 200, 1, 1500, 1399), 8, 128, 3, 4, "causal", 0),
+    ((1030, 200, 1, 1500, 1399), 8, 96, 3, 4, "noncausal", 0),
+    ((1030, 200, 1, 1500, 1399), 8, 128, 2, 4, "chunk_visible", 16),  # chunks of 64 rows: a wave pair's own depth columns
+    ((1030, 200, 1, 1500, 1399), 8, 128, 0, 4, "causal", 0),
+], ids=lambda c: f"{c[5]}-D{c[2]}-L{c[3]}")
+def test_large_packed_batches_equal_separate_calls_bitwise(gpu_device, case):
+    lengths, H, G = case[0], case[1], case[4]
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    blocks = lambda n: (n * G + 255) // 256 * H
+    assert blocks(sum(lengths)) >= 2 * cus > max(blocks(n) for n in lengths)
+    test_small_packed_batches_of_long_sequences_equal_separate_calls_bitwise(gpu_device, case)
+
+
+@pytest.mark.parametrize("mode", ["causal", "noncausal"])
+@pytest.mark.parametrize("D,T,many", [
+    (64, 230, 24),   # two waves a workgroup in the batch, four alone; the last key tile ends in its second half
+    (64, 197, 24),   # ... in its first
+    (128, 300, 28),  # eight waves half a tile apart, and four; the second half
+    (128, 270, 32),  # ... the first
+])
+def test_a_row_does_not_depend_on_the_batch_it_is_in(gpu_device, D, T, many, mode):
+    """Scores spread over more than 2^8, so that the exponent reference of a row follows its maximum tile by tile."""
+    from moda_amd import ops
+
+    H, L, G = 4, 5, 4
+    inp = to_dev(oracle.make_inputs(many, T, H, D, L, G, seed=T, dtype=torch.bfloat16, std=1.6), gpu_device)
+    names = ("q", "k", "v", "kd", "vd")
+    o, lse = ops._raw_fwd(MODE_ID[mode], *(inp[n] for n in names), D ** -0.5, G)
+    one = ops._raw_fwd(MODE_ID[mode], *(inp[n][3:4].contiguous() for n in names), D ** -0.5, G)
+    assert torch.equal(o[3:4], one[0]) and torch.equal(lse[3:4], one[1])
+
+
 def test_packed_batch_on_the_narrow_tiles_against_separate_calls(gpu_device):
     """On the 64-wide tiles the separate (short) calls form dk, dv by waves that share their columns, this packed launch by
     whole column tiles or segments of them: everything else is bit-identical, dk and dv agree to the order of their sums."""
