@@ -252,13 +252,6 @@ int moda_hip_depth_reorg_bwd(const void* d_cache, int64_t n_layers, int64_t slot
 int moda_hip_depth_push(const void* k, const void* v, const moda_hip_strides* sk, const moda_hip_strides* sv, int64_t slot,
                         int64_t L_total, int64_t B, int64_t T, int64_t H, int64_t D, int32_t dtype,
                         void* cache_k, void* cache_v, void* stream);
-/*
- * moda_hip_fwd and, in the same launch, moda_hip_depth_push of its k and v.  MODA_HIP_EUNSUPPORTED, and nothing done, where the
- * forward kernel has no such workgroups (16-bit types up to head dim 64, fixed length, k and v of one head dim, folded layout,
- * no depth stream or a partially filled one have): two calls then.  Slot `slot` must not be among those kd, vd show (L_valid).
- */
-int moda_hip_fwd_push(const moda_hip_desc* d, const void* q, const void* k, const void* v, const void* kd, const void* vd, void* o,
-                      float* lse, void* cache_k, void* cache_v, int64_t slot, int64_t L_total, void* stream);
 int moda_hip_depth_slot_add(void* dk, void* dv, const moda_hip_strides* sdk, const moda_hip_strides* sdv, int64_t slot,
                             int64_t L_total, int64_t B, int64_t T, int64_t H, int64_t D, int32_t dtype,
                             const void* d_cache_k, const void* d_cache_v, void* stream);

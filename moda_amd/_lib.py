@@ -29,7 +29,6 @@ EXPORTS = (
     "moda_hip_depth_reorg_fwd",
     "moda_hip_depth_reorg_bwd",
     "moda_hip_depth_push",
-    "moda_hip_fwd_push",
     "moda_hip_depth_slot_add",
     "moda_hip_linear",
     "moda_hip_layer_norm",

@@ -259,27 +259,23 @@ void* at(void* p, int64_t row, int64_t stride, int esize) { return p ? (char*)p 
 
 }  // namespace
 
-// where a forward launch copies k and v besides
-struct PushTo {
-  void *k, *v;
-  int64_t slot, L_total;
-};
+extern "C" {
 
-static int forward(const moda_hip_desc* d, const void* q, const void* k, const void* v, const void* kd, const void* vd, void* o, float* lse,
-                   const PushTo* push, void* stream) {
+int moda_hip_fwd(const moda_hip_desc* d, const void* q, const void* k, const void* v, const void* kd,
+                 const void* vd, void* o, float* lse, void* stream) {
   KArgs a;
   int rc = fill_geometry(d, a);
   if (rc) return rc;
   if ((int64_t)a.B * a.Tq * a.Hq == 0) return MODA_HIP_OK;
   const int es = elem_size(d->dtype);
   if (per_sequence(d)) {
-    if (push) return MODA_HIP_EUNSUPPORTED;
     MODA_REQ_PTR(lse);
     for (int64_t i = 0; i < d->B; i++) {
       const SeqView s = sequence_view(d, i);
       if (s.d.T == 0) continue;
-      rc = forward(&s.d, at(q, s.q_row, d->q.t, es), at(k, s.k_row, d->k.t, es), at(v, s.k_row, d->v.t, es),
-                   at(kd, s.d_row, d->kd.t, es), at(vd, s.d_row, d->vd.t, es), at(o, s.q_row, d->o.t, es), lse + s.q_row * a.Hq, nullptr, stream);
+      rc = moda_hip_fwd(&s.d, at(q, s.q_row, d->q.t, es), at(k, s.k_row, d->k.t, es), at(v, s.k_row, d->v.t, es),
+                        at(kd, s.d_row, d->kd.t, es), at(vd, s.d_row, d->vd.t, es), at(o, s.q_row, d->o.t, es),
+                        lse + s.q_row * a.Hq, stream);
       if (rc) return rc;
     }
     return MODA_HIP_OK;
@@ -317,16 +313,6 @@ static int forward(const moda_hip_desc* d, const void* q, const void* k, const v
   a.skd = cvt(d->kd);
   a.svd = cvt(d->vd);
   a.so = cvt(d->o);
-  if (push) {
-    if (!use_mfma(d) || !moda::fwd_takes_push(a, tile_width(d))) return MODA_HIP_EUNSUPPORTED;
-    if (!push->k || !push->v || push->slot < 0 || push->slot >= push->L_total) return MODA_HIP_EINVAL;
-    if ((uintptr_t)push->k % 16 != 0 || (uintptr_t)push->v % 16 != 0) return MODA_HIP_EALIGN;
-    const int64_t at = push->slot * a.Hkv * a.D;
-    a.dkd = (uint16_t*)push->k + at;
-    a.dvd = (uint16_t*)push->v + at;
-    a.sdkd = Str3{(int64_t)a.T * push->L_total * a.Hkv * a.D, push->L_total * a.Hkv * a.D, a.D};
-    a.push_blocks = 1;
-  }
   hipError_t e;
   if (use_mfma(d))
     e = moda::launch_fwd(a, d->dtype, tile_width(d), (hipStream_t)stream);
@@ -344,19 +330,6 @@ size_t moda_hip_bwd_workspace_bytes(const moda_hip_desc* d) {
   const size_t hand = depth_handover_bytes(d, a);
   // the row sums, then (each optional) the handed-over depth scores and the partial sums of the row split
   return (part || hand) ? delta_bytes(a) + hand + part : delta_bytes_exact(a);
-}
-
-extern "C" {
-
-int moda_hip_fwd(const moda_hip_desc* d, const void* q, const void* k, const void* v, const void* kd,
-                 const void* vd, void* o, float* lse, void* stream) {
-  return forward(d, q, k, v, kd, vd, o, lse, nullptr, stream);
-}
-
-int moda_hip_fwd_push(const moda_hip_desc* d, const void* q, const void* k, const void* v, const void* kd, const void* vd, void* o,
-                      float* lse, void* cache_k, void* cache_v, int64_t slot, int64_t L_total, void* stream) {
-  const PushTo push = {cache_k, cache_v, slot, L_total};
-  return forward(d, q, k, v, kd, vd, o, lse, &push, stream);
 }
 
 int moda_hip_bwd(const moda_hip_desc* d, const void* q, const void* k, const void* v, const void* kd,

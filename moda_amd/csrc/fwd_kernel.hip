@@ -29,8 +29,7 @@ using FwdLarge = RowLargePP;
 
 // ADDR bit 0: a (batch, head) slice is wider than 2 GiB (descriptors anchored per tile instead of 32-bit
 // offsets inside the slice); bit 1: packed variable-length batch; bit 2: no depth stream; bit 3: partially filled
-// depth stream (only Lv of a token's L slots hold data: depth tiles are loaded through the slot mapping); bit 4: workgroups
-// behind the rows' copy the layer's k and v (KArgs::push_blocks)
+// depth stream (only Lv of a token's L slots hold data: depth tiles are loaded through the slot mapping)
 // On the 64-wide tiles the registers of three waves per SIMD are enough (168, no spills).
 template <typename T, int HD, typename Shape, int ADDR>
 __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(const KArgs a_in) {
@@ -49,34 +48,6 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
   // so that it cannot disturb the register allocation of their main loop
   constexpr bool NODEPTH = (ADDR & 4) != 0, PARTIAL = (ADDR & 8) != 0;
   static_assert(!(NODEPTH && PARTIAL), "a partially filled depth stream is a depth stream");
-  if constexpr ((ADDR & 16) != 0) {
-    // The layer's own k and v on their way to their slot of the cache (a launch of their own: 4 us, and as long again on the
-    // host, of 15 a layer of 64 x 197 tokens; beside the rows' workgroups they are gone before those end).
-    if ((int)blockIdx.x >= (int)gridDim.x - a_in.push_blocks) {
-      const int n = push_pieces(a_in), at = ((int)blockIdx.x - ((int)gridDim.x - a_in.push_blocks)) * NT + tid;
-      i32x4 x[2], y[2];
-#pragma unroll
-      for (int i = 0; i < 2; i++) {
-        const int j = at + i * a_in.push_blocks * NT;
-        if (j < n) {
-          const PushPiece p = push_piece(a_in, j);
-          x[i] = *reinterpret_cast<const i32x4*>(a_in.k + p.b * a_in.sk.b + p.t * a_in.sk.t + p.h * a_in.sk.h + p.e);
-          y[i] = *reinterpret_cast<const i32x4*>(a_in.v + p.b * a_in.sv.b + p.t * a_in.sv.t + p.h * a_in.sv.h + p.e);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 2; i++) {
-        const int j = at + i * a_in.push_blocks * NT;
-        if (j < n) {
-          const PushPiece p = push_piece(a_in, j);
-          const int64_t to = p.b * a_in.sdkd.b + p.t * a_in.sdkd.t + p.h * a_in.sdkd.h + p.e;
-          *reinterpret_cast<i32x4*>(a_in.dkd + to) = x[i];
-          *reinterpret_cast<i32x4*>(a_in.dvd + to) = y[i];
-        }
-      }
-      return;
-    }
-  }
   const RowPlace place = row_place<VARLEN>(a_in, (int)blockIdx.x, BM);
   if (VARLEN && !place.active) return;
   int b = place.b;
@@ -754,18 +725,13 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void fwd_wide_kernel(const KArgs 
 }
 
 template <typename T, int HD, typename Shape, int ADDR>
-hipError_t launch_fwd_t_shape(const KArgs& args, hipStream_t stream) {
-  KArgs a = args;
+hipError_t launch_fwd_t_shape(const KArgs& a, hipStream_t stream) {
   constexpr size_t smem = (size_t)Shape::NST * 2 * 64 * HD * sizeof(uint16_t);  // the ring
   static LdsAttrState attr;
   const hipError_t ea = allow_dynamic_lds(attr, reinterpret_cast<const void*>(&fwd_kernel<T, HD, Shape, ADDR>), smem);
   if (ea != hipSuccess) return ea;
-  int64_t nblk = row_kernel_blocks(a, 32 * Shape::W);
+  const int64_t nblk = row_kernel_blocks(a, 32 * Shape::W);
   if (nblk == 0) return hipSuccess;
-  if (a.push_blocks) {  // asked for: how many, only the shape says
-    a.push_blocks = (push_pieces(a) + 2 * 64 * Shape::W - 1) / (2 * 64 * Shape::W);
-    nblk += a.push_blocks;
-  }
   if (nblk >= (1ll << 31)) return hipErrorInvalidValue;
   hipLaunchKernelGGL((fwd_kernel<T, HD, Shape, ADDR>), dim3((unsigned)nblk), dim3(64 * Shape::W), smem, stream, a);
   return hipGetLastError();
@@ -789,9 +755,6 @@ hipError_t launch_fwd_wide(const KArgs& a, hipStream_t stream) {
 
 template <typename T, int HD, int ADDR>
 hipError_t launch_fwd_t_addr(const KArgs& a, bool small, hipStream_t stream) {
-  if constexpr (HD <= 64 && (ADDR == 4 || ADDR == 8)) {
-    if (a.push_blocks) return launch_fwd_t_addr<T, HD, ADDR | 16>(a, small, stream);
-  }
   if constexpr (HD <= 64) {
     if (!(ADDR & 3) && pick_short_rows(a.Tq, (long long)a.B * a.Hq, a.causal, a.compute_units) == ShortRows::kTwoStages)
       return launch_fwd_t_shape<T, HD, RowShort, ADDR & ~3>(a, stream);

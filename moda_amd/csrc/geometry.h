@@ -183,16 +183,6 @@ MODA_HD RowVis row_visibility(const KArgs& a, int r, int Ld) {
   return v;
 }
 
-// 16-byte piece i of the k (or v) that such a launch copies
-struct PushPiece {
-  int b, t, h, e;  // e: first element of the row
-};
-MODA_HD int push_pieces(const KArgs& a) { return a.B * a.T * a.Hkv * (a.D / 8); }
-MODA_HD PushPiece push_piece(const KArgs& a, int i) {
-  const int row = i / (a.D / 8), tok = row / a.Hkv, b = tok / a.T;
-  return {b, tok - b * a.T, row - tok * a.Hkv, (i - row * (a.D / 8)) * 8};
-}
-
 // Depth columns a wave alone can see (always outside chunk-visible mode, and in it when a chunk's rows fit a
 // wave pair) are not streamed through the workgroup's ring: each wave fetches its own rows' span.
 MODA_HD bool waves_own_depth(const KArgs& a, int Ld) { return Ld > 0 && (!a.chunk || a.Cb * a.Gf <= 64); }
@@ -408,12 +398,6 @@ inline bool dkv_flat_row_waves(const KArgs& a) {
 inline bool narrow_slices(const KArgs& a) {
   const int64_t seq = (int64_t)a.T * (a.sk.t > a.sv.t ? a.sk.t : a.sv.t), dep = (int64_t)a.T * a.L * (a.skd.t > a.svd.t ? a.skd.t : a.svd.t);
   return 2 * (seq > dep ? seq : dep) <= 0x7fffffffll;
-}
-// Forward launches that also copy the layer's own k and v to their slot of a depth cache: the narrow tiles, fixed length,
-// without a depth stream or with a partially filled one.  Pieces of 16 bytes of each tensor, two a thread.
-inline bool fwd_takes_push(const KArgs& a, int HD) {
-  return HD <= 64 && a.has_seq && !a.cu && a.hdiv == 1 && a.D == a.Dv && (a.L == 0 || a.Lv < a.L) && narrow_slices(a) &&
-         (int64_t)a.B * a.T * a.Hkv < (1ll << 27);
 }
 // dQ and sequence dK/dV of the 64-wide tiles in one launch (bwd_short_kernel): row waves, and the workgroups of both run at once,
 // two a compute unit.  A replayed backward pass of 48 random such shapes takes 0.71 - 0.99 of the two launches' time (one of

@@ -264,14 +264,7 @@ moda_hip_desc geometry(const Call& c, const Tensor& q, const Tensor& k, const Te
 // forward and backward
 // ------------------------------------------------------------------------------------------------------------------
 
-// A slot of a stream's cache that a call's own k and v are copied to by the forward launch, where it has room for that.
-struct PushTo {
-  Tensor k, v;
-  int64_t slot, L;
-  bool done = false;
-};
-
-std::pair<Tensor, Tensor> forward(const Call& c, Tensor q, Tensor k, Tensor v, Tensor kd, Tensor vd, PushTo* push = nullptr) {
+std::pair<Tensor, Tensor> forward(const Call& c, Tensor q, Tensor k, Tensor v, Tensor kd, Tensor vd) {
   if (narrows(q)) {
     auto r = forward(c, narrowed(q), narrowed(k), narrowed(v), narrowed(kd), narrowed(vd));
     return {r.first.to(at::kFloat), r.second};
@@ -292,13 +285,6 @@ std::pair<Tensor, Tensor> forward(const Call& c, Tensor q, Tensor k, Tensor v, T
   d.vd = strides_of(vd);
   d.o = strides_of(o);
   c10::OptionalDeviceGuard guard(q.device());
-  if (push) {
-    const int rc = moda_hip_fwd_push(&d, in_ptr(q), in_ptr(k), in_ptr(v), in_ptr(kd), in_ptr(vd), out_ptr(o), (float*)out_ptr(lse),
-                                     out_ptr(push->k), out_ptr(push->v), push->slot, push->L, stream_of(q));
-    push->done = rc == 0;
-    if (push->done) return {o, lse};
-    if (rc != MODA_HIP_EUNSUPPORTED) check_rc(rc, "moda_hip_fwd_push");
-  }
   check_rc(moda_hip_fwd(&d, in_ptr(q), in_ptr(k), in_ptr(v), in_ptr(kd), in_ptr(vd), out_ptr(o), (float*)out_ptr(lse),
                         stream_of(q)),
            "moda_hip_fwd");
@@ -562,7 +548,6 @@ struct StreamCall : c10::intrusive_ptr_target {
   Call call;
   c10::intrusive_ptr<StreamBuffers> buf;
   int64_t n = 0, slot = -1;
-  PushTo* push = nullptr;  // while the call's forward runs
 };
 
 // A tensor that carries no data, only the order of the stream's operations (autograd runs them last to first).
@@ -575,7 +560,7 @@ struct StreamAttend : torch::autograd::Function<StreamAttend> {
   static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const OptTensor& /*token*/,
                                const c10::intrusive_ptr<StreamCall>& call) {
     const bool depth = call->n > 0;
-    auto r = ::forward(call->call, q, k, v, depth ? call->buf->k : Tensor(), depth ? call->buf->v : Tensor(), call->push);
+    auto r = ::forward(call->call, q, k, v, depth ? call->buf->k : Tensor(), depth ? call->buf->v : Tensor());
     ctx->save_for_backward({q, k, v, r.first, r.second});
     ctx->saved_data["state"] = owning(call);
     ctx->set_materialize_grads(false);
@@ -656,23 +641,7 @@ class TrainStream {
     if (n_ > 0) call->call.depth_valid = n_;
     call->buf = buf_;
     call->n = n_;
-    // The layer's k and v are as a rule pushed next: the forward launch copies them to the slot they would get, which nobody reads
-    // before something is pushed there, and push() need not launch (with the copies 706 us a step of twelve layers of 64 x 197
-    // tokens, of which the host took 690).
-    PushTo push{Tensor(), Tensor(), n_, buf_->L};
-    copied_ = Copied();
-    struct Ends {  // the call outlives its forward
-      StreamCall& call;
-      ~Ends() { call.push = nullptr; }
-    } ends{*call};
-    if (copies_early(q, k, v)) {
-      if (!buf_->k.defined()) allocate(k);
-      push.k = buf_->k;
-      push.v = buf_->v;
-      call->push = &push;
-    }
     const variable_list r = StreamAttend::apply(q, k, v, token_.defined() ? OptTensor(token_) : OptTensor(), call);
-    if (push.done) copied_ = Copied{true, k._version(), v._version(), stream_of(k)};
     token_ = r[1];
     last_ = r[0].requires_grad() ? call : c10::intrusive_ptr<StreamCall>();
     last_k_ = k;
@@ -683,11 +652,11 @@ class TrainStream {
   void push(const Tensor& k, const Tensor& v) {
     py::gil_scoped_release nogil;
     CONTRACT(k.dim() == 4, "k must be [B, T, H, D]");
-    if (!buf_->k.defined() || (n_ == 0 && !cache_fits(k))) allocate(k);
-    const bool copied = copied_.done && k.is_same(last_k_) && v.is_same(last_v_) && k._version() == copied_.k_version &&
-                        v._version() == copied_.v_version && stream_of(k) == copied_.stream;
-    if (!copied) depth_push(k, v, buf_->k, buf_->v, n_, buf_->L);
-    copied_ = Copied();
+    if (!buf_->k.defined()) {
+      buf_->k = at::empty({k.size(0), k.size(1) * buf_->L, k.size(2), k.size(3)}, k.options());
+      for (Tensor* x : {&buf_->v, &buf_->gk, &buf_->gv}) *x = at::empty_like(buf_->k);
+    }
+    depth_push(k, v, buf_->k, buf_->v, n_, buf_->L);
     if (at::GradMode::is_enabled()) {
       if (last_ && k.is_same(last_k_) && v.is_same(last_v_)) {
         last_->slot = n_;
@@ -704,26 +673,6 @@ class TrainStream {
   }
 
  private:
-  bool cache_fits(const Tensor& k) const {
-    return has_shape(buf_->k, {k.size(0), k.size(1) * buf_->L, k.size(2), k.size(3)}) && k.scalar_type() == buf_->k.scalar_type() &&
-           k.device() == buf_->k.device();
-  }
-  void allocate(const Tensor& k) {
-    buf_->k = at::empty({k.size(0), k.size(1) * buf_->L, k.size(2), k.size(3)}, k.options().requires_grad(false));
-    for (Tensor* x : {&buf_->v, &buf_->gk, &buf_->gv}) *x = at::empty_like(buf_->k);
-  }
-  // Whether an attention call may copy its k, v to slot n_: tensors a push of them would take as they are.
-  bool copies_early(const Tensor& q, const Tensor& k, const Tensor& v) const {
-    return n_ < buf_->L && q.is_cuda() && k.is_cuda() && k.dim() == 4 && k.sizes() == v.sizes() && k.scalar_type() == v.scalar_type() &&
-           k.device() == q.device() && v.device() == q.device() && (k.scalar_type() == at::kBFloat16 || k.scalar_type() == at::kHalf) &&
-           k.size(3) <= 64 && !k.is_inference() && !v.is_inference() && (!buf_->k.defined() || cache_fits(k));
-  }
-  struct Copied {  // the latest attention call's k and v lie in slot n_ already, as they were on that stream
-    bool done = false;
-    int64_t k_version = 0, v_version = 0;
-    void* stream = nullptr;
-  };
-  Copied copied_;
   c10::intrusive_ptr<StreamBuffers> buf_;
   c10::intrusive_ptr<StreamCall> last_;  // the latest attention call, until something is pushed
   Tensor token_, last_k_, last_v_;

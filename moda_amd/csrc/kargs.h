@@ -30,7 +30,6 @@ struct KArgs {
   int own_slot;     // dk, dv += slot Lv of dkd, dvd (the layer's own slot of the stream, complete by now)
   int keep_slots;   // slots l >= Lv of dkd, dvd untouched (always when accumulating) instead of zeroed
   int far_depth_grads;  // rows of dkd or dvd too far apart for the 32-bit offsets of a tile (host and kernels: depth_grads_in_dq)
-  int push_blocks;  // forward: workgroups behind the rows' that copy k, v to a slot of the caches at dkd, dvd (strides sdkd)
   int seq_done;     // the sequence dK/dV came with the dQ launch (host side)
   int own_delta;    // the dQ kernel forms the row sums of o * do itself and leaves them in `delta` for the later kernels
   // Outside chunk-visible mode a query row sees the Lv depth slots of its own token only.  When the dQ kernel walks

@@ -1550,20 +1550,6 @@ int main(int argc, char** argv) {
     printf("OK checked=%lld\n", g_checked);
     return 0;
   }
-  if (what == "push") {  // B T H D L_total: every piece of k once, in bounds, to a place of its own in the slot
-    KArgs a = {};
-    a.B = arg(2), a.T = arg(3), a.Hkv = arg(4), a.D = arg(5);
-    std::vector<int> seen((size_t)a.B * a.T * a.Hkv * (a.D / 8));
-    for (int i = 0; i < push_pieces(a); i++) {
-      const PushPiece p = push_piece(a, i);
-      if (p.b < 0 || p.b >= a.B || p.t < 0 || p.t >= a.T || p.h < 0 || p.h >= a.Hkv || p.e < 0 || p.e + 8 > a.D || p.e % 8) fail("piece %d", i);
-      if (seen[(((size_t)p.b * a.T + p.t) * a.Hkv + p.h) * (a.D / 8) + p.e / 8]++) fail("piece %d twice", i);
-      g_checked++;
-    }
-    if ((size_t)g_checked != seen.size()) fail("%lld pieces of %zu", g_checked, seen.size());
-    printf("OK checked=%lld\n", g_checked);
-    return 0;
-  }
   if (what == "pack") {
     walk_pack(arg(2));
     printf("OK checked=%lld\n", g_checked);

@@ -243,12 +243,6 @@ def test_launch_shapes_of_the_narrow_tiles(walker, case):
     assert rc == 0 and out.startswith(shapes + " OK"), out
 
 
-@pytest.mark.parametrize("shape", [(1, 1, 1, 8), (3, 17, 2, 40), (64, 197, 1, 64)])
-def test_pieces_of_a_layer_copied_by_its_forward(walker, shape):
-    p = subprocess.run([walker, "push"] + [str(x) for x in shape], capture_output=True, text=True)
-    assert p.returncode == 0 and "OK checked" in p.stdout, p.stdout + p.stderr
-
-
 def test_slot_arithmetic(walker):
     """Token and slot of a column of a partially filled stream, by a reciprocal and a correction."""
     p = subprocess.run([walker, "slots"], capture_output=True, text=True)

@@ -2535,9 +2535,11 @@ def test_depth_gradients_into_rows_far_apart(gpu_device):
         check(n, b.contiguous(), a.float().cpu(), torch.bfloat16, "rows far apart")
 
 
-@pytest.mark.parametrize("what", ["same", "others", "written", "other stream", "attended twice", "other heads", "wide"])
-def test_a_layer_copied_by_its_attention_call_is_what_was_pushed(gpu_device, what):
-    """The forward launch copies k and v to the slot they would get; what later layers see is what push() was given."""
+@pytest.mark.parametrize("what", ["same", "others", "written", "other stream", "attended twice", "other heads", "wide",
+                                  "written past autograd", "unordered"])
+def test_later_layers_see_what_was_pushed(gpu_device, what):
+    """... as it was then, whatever an attention call got before it and on whichever stream: attend() reads the stream's cache and
+    leaves nothing in it."""
     import moda_amd
 
     B, T, G, D, L = (2, 70, 2, 128 if what == "wide" else 64, 3)
@@ -2561,6 +2563,8 @@ def test_a_layer_copied_by_its_attention_call_is_what_was_pushed(gpu_device, wha
         if what == "written":
             with torch.no_grad():
                 k.mul_(-2), v.add_(1)
+        if what == "written past autograd":  # no version counter moves
+            k.data.mul_(-2), v.data.add_(1)
         if what == "attended twice":
             stream.attend(q, new(1).requires_grad_(), new(1).requires_grad_(), moda_group_num=G, is_causal=False)
         if what == "other stream":
@@ -2569,6 +2573,24 @@ def test_a_layer_copied_by_its_attention_call_is_what_was_pushed(gpu_device, wha
             with torch.cuda.stream(side):
                 stream.push(k, v)
             torch.cuda.current_stream().wait_stream(side)
+        elif what == "unordered":  # an attention call of a side stream that gets there last
+            side, others = torch.cuda.Stream(), [new(1).requires_grad_() for _ in range(2)]
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                torch.cuda._sleep(1 << 22)
+                stream.attend(q, *others, moda_group_num=G, is_causal=False)
+            stream.push(k, v)
+            torch.cuda.synchronize()
         else:
             stream.push(k, v)
         pushed.append((k.detach().clone(), v.detach().clone()))
+
+
+def test_a_stream_that_nothing_is_pushed_to_holds_no_cache(gpu_device):
+    import moda_amd
+
+    q, k, v = (torch.randn(2, n, 1, 64, device=gpu_device, dtype=torch.bfloat16, requires_grad=True) for n in (140, 70, 70))
+    stream = moda_amd.DepthStream(512)
+    before = torch.cuda.memory_allocated()
+    o = stream.attend(q, k, v, moda_group_num=2, is_causal=False)
+    assert torch.cuda.memory_allocated() - before < 512 * k.nbytes and o.requires_grad
