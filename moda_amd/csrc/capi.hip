@@ -58,11 +58,6 @@ bool mapped_span_ok(const KArgs& a, const moda_hip_strides& s, int esize) {
   return (int64_t)(64 / a.Lv + 2) * a.L * s.t * esize < (1ll << 31);
 }
 
-// The dQ kernel that forms the depth gradients stores a tile's rows in the same way, of a full stream 32 of them.
-bool far_grad_rows(const KArgs& a, const moda_hip_strides& s, int esize) {
-  return a.L > 0 && (s.t < 0 || 32 * s.t * esize >= (1ll << 31) || !mapped_span_ok(a, s, esize));
-}
-
 // The fp32 matrix kernels move 16-byte pieces of rows; fp32 tensors that are not laid out for that run on the vector-ALU
 // kernels, which ask for element alignment only (the host therefore does not copy fp32 views).
 struct TensorAt {
@@ -134,7 +129,9 @@ int fill_geometry(const moda_hip_desc* d, KArgs& a) {
   a.own_slot = (d->flags & MODA_HIP_FLAG_ADD_OWN_SLOT) ? 1 : 0;
   a.accum_depth = (d->flags & MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS) ? 1 : 0;
   a.keep_slots = (d->flags & (MODA_HIP_FLAG_ACCUMULATE_DEPTH_GRADS | MODA_HIP_FLAG_KEEP_DEPTH_SLOTS)) ? 1 : 0;
-  a.far_depth_grads = far_grad_rows(a, d->dkd, elem_size(d->dtype)) || far_grad_rows(a, d->dvd, elem_size(d->dtype));
+  // The dQ kernel that forms the depth gradients stores a tile's rows in the same way as it reads them; of a full stream 32 rows in
+  // a row, which row_stride_ok keeps within 512 MiB.
+  a.far_depth_grads = !mapped_span_ok(a, d->dkd, elem_size(d->dtype)) || !mapped_span_ok(a, d->dvd, elem_size(d->dtype));
   a.nqt = (a.Tq + 127) / 128;
   a.scale = d->scale;
   a.delta_pitch = a.Tq;
