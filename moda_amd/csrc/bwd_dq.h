@@ -298,7 +298,7 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
   for (; it < ntiles; it++) {
     if (it + DIST < ntiles) issue(it + DIST);
     if (FUSABLE && fused_depth && it + 1 == ntiles) {
-      first_set = Shape::W > 2 || c_st == 0 ? 1 : 0;
+      first_set = dq_first_private_set(Shape::W, c_st);
       enter_depth();
       early = true;
     }

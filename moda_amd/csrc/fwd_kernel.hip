@@ -318,7 +318,7 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
     for (; it < ntiles; it++) {
       if (it + DIST < ntiles) issue(it + DIST);
       if (EARLY && own_depth && it + 1 == ntiles) {
-        first_set = c_st ^ 1;
+        first_set = fwd_first_private_set(c_st);
         enter_depth();
         if (c_beg < c_end) fetch_early();
         early = true;

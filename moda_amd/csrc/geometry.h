@@ -207,6 +207,12 @@ MODA_HD bool depth_scores_from_dq(const KArgs& a, int HD) {
   return a.L > 0 && !a.chunk && HD <= 128 && !depth_grads_in_dq(a, HD);
 }
 
+// Private depth tiles that are sent for while the last ring tile, in stage `last`, is worked on: the first of two sets, or of K and V
+// places, that lies outside of that stage.  Forward: a set is one of two stages.  dQ with the depth gradients: a set is a stage of two
+// or three, or (four waves) as large as the whole ring.
+MODA_HD int fwd_first_private_set(int last) { return last ^ 1; }
+MODA_HD int dq_first_private_set(int waves, int last) { return waves > 2 || last == 0 ? 1 : 0; }
+
 // The column tiles of query tile qt: n_seq sequence tiles, of which the first n_full are seen completely by every
 // row of the workgroup, then n_dep depth tiles starting at flattened depth column dep0 (ring_depth: the depth
 // columns go through the ring at all).

@@ -351,7 +351,9 @@ void walk_row_kernel(const KArgs& a_in, bool dq, int rows_per_wave, bool own_pos
         // forward on the 64-wide tiles: the first tiles go to the stage that is free while the last, masked sequence tile
         // is worked on; two sets a stage apart for two waves, else K in that stage and V in the other
         const bool early = !dq && HD <= 64 && NST == 2, two_sets = early && Shape::W <= 2;
-        const uint32_t stage = 2 * BN * HD * 2, first = plan.n_full < ntiles ? (uint32_t)(ntiles & 1) : 0u;
+        const bool fused = dq && depth_grads_in_dq(a, HD), beside = plan.n_full < ntiles;  // (a masked tile to travel beside)
+        const int last = beside ? (ntiles - 1) % NST : 0;
+        const uint32_t stage = 2 * BN * HD * 2, first = beside ? (uint32_t)fwd_first_private_set(last) : 0u;
         if (early && !two_sets) {
           kt = first * stage + (uint32_t)wave * 32 * HD * 2;
           vt = (first ^ 1) * stage + (uint32_t)wave * 32 * HD * 2;
@@ -367,10 +369,14 @@ void walk_row_kernel(const KArgs& a_in, bool dq, int rows_per_wave, bool own_pos
             const int col0 = span.c_beg + 32 * j;
             const int nrows = imin(32, span.c_end - col0);
             // where the dQ kernel forms the depth gradients it alternates between two sets of private tiles
-            const bool fused = dq && depth_grads_in_dq(a, HD);
-            const uint32_t fused_first = plan.n_full < ntiles && (Shape::W > 2 || (ntiles - 1) % NST == 0) ? 1u : 0u;
+            const uint32_t fused_first = beside ? (uint32_t)dq_first_private_set(Shape::W, last) : 0u;
             const uint32_t set = two_sets ? (first ^ (uint32_t)(j & 1)) * stage
                                           : fused ? (fused_first ^ (uint32_t)(j & 1)) * Shape::W * 64 * HD * 2 : 0u;
+            if (j == 0 && beside && (early || fused)) {  // other waves may still read the last ring tile
+              const auto clear = [&](uint32_t at) { return at + 32 * HD * 2 <= last * stage || at >= (last + 1) * stage; };
+              if (!clear(kt + set)) fail("%s: first private K tile in the stage of the last ring tile", kname);
+              if ((two_sets || fused) && !clear(vt + set)) fail("%s: first private V tile in the stage of the last ring tile", kname);
+            }
             for (int i = 0; i < Own::N; i++) {
               if (fused) {  // rows of the tile and of its gradients, from slot 0 of the first column's token or the column itself
                 const int tok = col0 / a.Lv, slot = col0 - tok * a.Lv, row = i * Own::RPW + own.prow;
