@@ -307,17 +307,23 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic.json")
 # kernel of the same runs): FETCH_SIZE counts half of the bytes read, WRITE_SIZE all bytes written
 PMC_SCALE = {"FETCH_SIZE": 2.0, "WRITE_SIZE": 1.0}
 KERNEL_NAMES = ("fwd_kernel", "fwd_wide_kernel", "delta_kernel", "dq_kernel", "dkv_kernel", "dkv_flat_kernel", "dkv_reduce_kernel", "depth_cols_kernel",
-                "depth_token_handed_kernel", "depth_cols_handed_kernel", "chunk_depth_kernel", "reorg_kernel")
+                "depth_token_handed_kernel", "depth_cols_handed_kernel", "reduce_and_depth_kernel", "chunk_depth_kernel", "reorg_kernel")
 
 
-def depth_gradient_kernel(mode, D, G):
+def depth_gradient_kernel(mode, B, T, Hkv, G, D, L):
     """Name of the launch that forms dkd, dvd after dkv_kernel (moda_amd/csrc/geometry.h: depth_grads_in_dq,
-    depth_scores_from_dq), or None where the dQ kernel forms them itself."""
+    depth_scores_from_dq, dkv_split_plan; bwd_dkv_kernel.hip), or None where the dQ kernel forms them itself."""
     if mode == "chunk_visible":
         return "chunk_depth_kernel"
     if D <= 64 and 32 % G == 0:
         return None
+    if D <= 64:
+        return "depth_token_handed_kernel" if G <= 4 else "depth_cols_handed_kernel"
     if D <= 128:
+        tiles, query_tiles = -(-T // 128) * B * Hkv, -(-T * G // 64)
+        cut = mode != "depth_only" and tiles < 512 and query_tiles // 2 >= (4 if tiles < 256 else 16)
+        if cut and (G <= 4 or (-(-T // 16) + -(-T * L // 16)) * B * Hkv <= 32768):
+            return "reduce_and_depth_kernel"
         return "depth_token_handed_kernel" if G <= 4 else "depth_cols_handed_kernel"
     return "depth_cols_kernel"
 
@@ -522,8 +528,8 @@ def main():
     dom = max(("fwd_kernel", "dq_kernel", "dkv_kernel"), key=lambda n: kernels[n]["ms"])
     traffic = recorded_traffic(args.workload) or {}
     # the dK/dV stage is timed as a whole: dkv_kernel followed by the HBM-bound launch that forms the depth gradients
-    # (where the dQ kernel does not form them itself; light launches add dkv_reduce_kernel)
-    depth_kernel = depth_gradient_kernel(mode, D, G) if L > 0 else None
+    # (where the dQ kernel does not form them itself; light launches add dkv_reduce_kernel or have it in the same launch)
+    depth_kernel = depth_gradient_kernel(mode, B, T, Hkv, G, D, L) if L > 0 else None
     two_launches = dom == "dkv_kernel" and depth_kernel is not None
     dom_traffic = None
     if dom in traffic:

@@ -3,7 +3,7 @@
 // local to a row, so a workgroup takes BM rows through the whole chain; what one step hands to the next stays in
 // registers and LDS.  As separate launches (block_kernels.hip) the same rows went to memory and back six times, the
 // hidden activations of the MLP, four times as wide, among them: 12 608 rows of width 256 took 69 us in seven launches
-// (projection 9, norm 6, MLP 23 + 15, norm 6, next projections 10.5), here 34.6.
+// (projection 9, norm 6, MLP 23 + 15, norm 6, next projections 10.5), here 33.1.
 //
 // Eight waves share the BM rows and divide the features of every product.  The weights sit on the matrix instruction's A
 // side (M = features) and go from memory (L2 after the first workgroup of an XCD) straight into the registers that it
@@ -200,8 +200,10 @@ struct Product {
 template <typename T, int C, int NB, bool POST>
 __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
   constexpr int BM = 16 * NB, MB2 = C / 128, MB1 = 2, HC = 128 * MB1, CH = C / 8, TPR = 512 / BM, NL = CH / TPR;
-  // The activation of a chunk beside the second product of the one before: where the registers are there.  fp16's formula with 64
-  // rows spills 23 (twelve blocks of width 256: 616 us apart, 624 beside), widths above 256 spill more than they do apart.
+  // The activation of a chunk beside the second product of the one before.  At width 256 that takes 15 to 31 registers more: with 32 rows
+  // and POST room for two waves a SIMD instead of three (a workgroup has two, a second one never fitted), with 64 rows of bf16 five of
+  // them spilled.  fp16's formula with 64 rows spills 23 (twelve blocks of width 256: 616 us apart, 624 beside), widths above 256 spill
+  // more than they do apart.
   constexpr bool BESIDE = MB2 <= 2 && (NB == 2 || std::is_same<T, BF16>::value);
   static_assert(CH % TPR == 0, "a row's chunks over the threads of the row");
   extern __shared__ __align__(16) unsigned char tail_smem[];

@@ -954,8 +954,8 @@ __global__ __launch_bounds__(256) void dkv_reduce_kernel(const KArgs a, int BN, 
   dkv_reduce<T, HD, VARLEN>(a, BN, BM, blockIdx.x);
 }
 // The last two of a backward pass in one launch, `reduce_blocks` workgroups of the first: both move memory, neither waits for the
-// other, and a launch more is 4 - 5 us (a training step of 710 tokens, four heads of four, 16 slots: 101 -> 96 us; 1500, two heads of
-// two, eight slots: 121 -> 116; 2 x 4096: 644 -> 640).
+// other, and a launch more is 5 - 7 us (backward pass, medians of two launches and one in turn, quartiles within 0.3 us: 710 tokens, four
+// heads of four, 16 slots 78.7 and 73.3 us; 1500, two of two, eight slots 86.7 and 81.0).
 template <typename T, int HD, bool BY_TOKEN>
 __global__ __launch_bounds__(256) void reduce_and_depth_kernel(const KArgs a, int BN, int BM, unsigned reduce_blocks) {
   const unsigned block = blockIdx.x;
@@ -1005,9 +1005,11 @@ hipError_t launch_dkv_t(const KArgs& a, hipStream_t stream) {
       const bool by_token = a.Gf <= 4;
       const int64_t heads = (int64_t)a.B * a.Hkv, rows = ((int64_t)a.T + RPB - 1) / RPB * heads;
       const int64_t n = rows + ((int64_t)a.T * (by_token ? 1 : a.L) + RPB - 1) / RPB * heads;
-      // By columns up to 32768 workgroups: one launch against two takes 190 to 194 us a training step at 4.1 K workgroups, 310 to 315
-      // at 16.4 K and 429 to 435 at 32.8 K, but 814 to 809 at 65 K and 1918 to 1897 at 122 K.
-      if (n <= (by_token ? (1ll << 31) - 1 : 32768)) {
+      // By columns up to 32768 workgroups: the dK/dV stage in two launches and in one, medians taken in turn, takes 53.2 and 46.1 us at
+      // 1.6 K workgroups, 126.8 and 123.9 at 16.5 K, 289.9 both at 33 K, 424.9 and 430.9 at 65 K, 989 and 1008 at 122 K (quartiles
+      // within 0.3 %).  By token there are fewer than 8192 (512 column tiles are not cut): 297.6 and 295.1 at 4.1 K, 132.7 and
+      // 132.9, 675.0 and 674.4, 1398 and 1385 at 8 K.
+      if (by_token || n <= 32768) {
         if (by_token)
           hipLaunchKernelGGL((reduce_and_depth_kernel<T, HD, true>), dim3((unsigned)n), dim3(256), 0, stream, a, BN, BM, (unsigned)rows);
         else

@@ -403,13 +403,13 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
   // dKd^T = Q^T dS: one matrix instruction per 16 columns x 16 head-dim elements, nothing to accumulate across
   // tiles.  Q^T and dO^T in that slot order are read once, through the private tiles before the first fetch.
   // dQ needs dS with the columns as summation index: the rounded dS block crosses over through a small LDS block
-  // of the wave, which afterwards stages the gradient rows on their way out.
+  // of the wave.
   if constexpr (FUSABLE) {
     if (fused_depth) {
       static_assert(NB == 2, "the wave's 32 query rows are the 32 summation slots of one matrix instruction");
       if (!early) enter_depth();  // (every ring tile ends with a barrier)
       const int wv = __builtin_amdgcn_readfirstlane(wave);
-      // behind the two sets the staging block: 16 rows of HD, or 32 x 32 for the dS block
+      // behind the two sets the 32 x 32 dS block
       lds_ptr stage = smem + 2 * SET + wv * (16 * HD);
       const int rw0 = qt * BM + wv * WR;
       if (rw0 < a.Tq) {
@@ -593,8 +593,8 @@ __global__ __launch_bounds__(64 * Shape::W, 2) void dq_kernel(const KArgs a_in) 
 }
 
 // LDS of a workgroup: the ring, or one 32-column K tile and V tile per wave for the waves' own depth columns
-// ... and, where the kernel forms the depth gradients, a second set of those and a 16-row block per wave through
-// which the gradients leave
+// ... and, where the kernel forms the depth gradients, a second set of those and a 32 x 32 block per wave (16 rows of HD) through
+// which dS crosses over
 template <int HD, typename Shape, int ADDR>
 constexpr size_t dq_lds() {
   constexpr size_t ring = (size_t)Shape::NST * 2 * 64 * HD * sizeof(uint16_t),

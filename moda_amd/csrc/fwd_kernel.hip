@@ -233,12 +233,6 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
   };
   auto stage_k = [&](int st) { return smem + st * 2 * BN * HD; };
 
-  // Ping-pong: the two waves of a SIMD (wave w and w + W/2) would otherwise run the same phase at the
-  // same time -- matrix pipe contended during the MFMA phases, idle during both softmaxes.  The upper
-  // half of the workgroup therefore runs half a tile behind: between two barriers it first finishes the
-  // previous tile (V product), then does scores and softmax of the current one, so its softmax overlaps
-  // the lower half's V product and its V product the lower half's scores.  The previous tile's V must
-  // survive one more barrier interval, hence the extra ring stage.
   // The wave's own depth columns, 32 at a time through wave-private K and V tiles cut out of the ring.  EARLY: the first
   // ones travel while the last sequence tile is worked on, into the ring stage that is free by then.  Two waves have room
   // for two whole sets, one in each stage, and fetch a tile ahead all the way; four for K in one stage and V in the other.
@@ -289,6 +283,12 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
     }
   };
 
+  // Ping-pong: the two waves of a SIMD (wave w and w + W/2) would otherwise run the same phase at the
+  // same time -- matrix pipe contended during the MFMA phases, idle during both softmaxes.  The upper
+  // half of the workgroup therefore runs half a tile behind: between two barriers it first finishes the
+  // previous tile (V product), then does scores and softmax of the current one, so its softmax overlaps
+  // the lower half's V product and its V product the lower half's scores.  The previous tile's V must
+  // survive one more barrier interval, hence the extra ring stage.
   const bool late = PP && __builtin_amdgcn_readfirstlane(wave) >= Shape::W / 2;
   int it = 0;
   if (!late) {
@@ -331,8 +331,9 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
       const auto seen = [&](int c, int cols) { return __any((hi > c) && (lo < c + cols) && (hi > lo)); };
       if (HD <= 64 && !NODEPTH && seen(col0, 32) != seen(col0 + 32, 32)) {
         // No row of the wave sees the other half, as in every second last tile of a sequence: 32 columns give the bits of the whole tile,
-        // which takes one maximum over all of them.  (Without depth the whole tile is as fast: 64 x 197 tokens, six heads, five columns
-        // left, 13.1 us by halves and 12.9.)
+        // which takes one maximum over all of them.  Serving twelve blocks of 64 x 197 tokens, five columns in the last tile: 566 us
+        // with whole tiles, 559 so; one such layer of six heads 199 both.  (Without depth the whole tile is as fast: 13.1 us by halves and
+        // 12.9.)
         const int half = seen(col0, 32) ? 0 : 32;
         half_tile(Kc + half * HD, Kc + (BN + half) * HD, col0 + half, lo, hi, []() {});
       } else if (seen(col0, BN)) {

@@ -388,10 +388,6 @@ __device__ __forceinline__ uint32_t lds_addr(lds_cptr p) { return (uint32_t)(uin
 // zero-padded): past the end of every descriptor, so the range check fills the chunk with zeros.
 constexpr int kPadOffset = 0x7ffffff0;
 
-// Depth tiles when only Lv of a token's L slots hold data: the tile's columns are counted on the compact axis
-// (column c = token * Lv + slot, see geometry.h) and lie in rows token * L + slot of the tensor.  The loaders anchor
-// one descriptor at slot 0 of the first column's token; this is the row, relative to that anchor, of the tile's
-// row `rho`, given the first column's slot l0.
 // `rho` (at most 64) columns behind slot l0 of a token: tokens further, and the slot there.  The quotient is small: an
 // estimate from the reciprocal, low by less than one, and a correction, where a division of integers is 25 vector
 // instructions behind a branch (eight times a 32-row tile of K and V).
@@ -412,6 +408,10 @@ __host__ __device__ __forceinline__ SlotStep slot_step(int l0, int rho, int Lv) 
   s.tokens += low ? 1 : 0;
   return s;
 }
+// Depth tiles when only Lv of a token's L slots hold data: the tile's columns are counted on the compact axis
+// (column c = token * Lv + slot, see geometry.h) and lie in rows token * L + slot of the tensor.  The loaders anchor
+// one descriptor at slot 0 of the first column's token; this is the row, relative to that anchor, of the tile's
+// row `rho`, given the first column's slot l0.
 __host__ __device__ __forceinline__ int mapped_row(int l0, int rho, int L, int Lv) {
   const SlotStep s = slot_step(l0, rho, Lv);
   return s.tokens * L + s.slot;

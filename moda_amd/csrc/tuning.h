@@ -94,20 +94,21 @@ inline LinearTile pick_linear_tile(long long rows, long long K, const int* featu
 // Host side, a transformer block's dense part as one launch (block_tail_kernel) or as its pieces (linear and layer-norm
 // launches): rows of a workgroup of the one launch ...
 inline int block_tail_rows(long long rows, int compute_units) { return rows <= 32ll * compute_units ? 32 : 64; }
-// ... and whether it is the faster way.  Measured as the time of stacks of four blocks, both ways, at widths 128, 256, 384
-// and 512, MLPs of once to 64 times the width, 16 to 25 216 rows, both types, and as the time of 218 others of one to eight
-// blocks: the rule takes the slower way nowhere by more than 3 % (1 us of 38, a single block).
+// ... and whether it is the faster way.  Measured as the time of stacks of four blocks, both ways in turn, at widths 128, 256, 384
+// and 512, MLPs of 1, 4, 16 and 64 times the width, 200 to 25 216 rows, both types: of 312 such stacks the rule takes the faster way or
+// one within 3 % of it for 286.  The others: MLPs of 16 times the width and more near the line, 3 - 14 % behind; widths 384 and 512
+// with two fifths of the last round full (22 852 rows), 4 - 15 % behind at an MLP of four times the width, up to 46 % at sixteen.
 // A workgroup takes its rows through all of the block's weights, which one compute unit takes in at 64 bytes a cycle, however
 // few the rows are.  The pieces spread the weights over the compute units, but are seven launches, and their time grows with
 // the rows.  While 32 rows each are one round, the one launch costs, in us a block and against the pieces, 16 for a million
 // weights; it saves 9 of launches, 3 for 256 features of width, the hidden activations' way through memory (less in fp16, whose
-// GELU is the longer one), and for 1000 rows 1 and 2.2 for a million weights.  Width 256, MLP of 1024, 200 rows: 45 us a block,
-// pieces 64; MLP of 16 384: 235 and 157, at 4 640 rows 236 and 255.  Width 512, MLP of 2048, 200 rows: 76 and 54, 8 128 rows: 86
-// and 107.
+// GELU is the longer one), and for 1000 rows 1 and 2.2 for a million weights.  Width 256, MLP of 1024, 200 rows: 34 us a block,
+// pieces 42; MLP of 16 384: 219 and 156, at 4 632 rows 211 and 255.  Width 512, MLP of 2048, 200 rows: 78 and 56, 8 128 rows: 92
+// and 112.
 // With 64 rows a round that is mostly empty costs as much as a full one.  Up to width 256 that is still less than the pieces
-// (16 448 rows, a workgroup more than a round: 80 and 94); 384 has to fill half of it (16 448 rows: 161 and 151, 25 216: 174
-// and 216), and so has 512 in bf16 (18 912: 247 and 229, 25 216: 261 and 307).  512 in fp16 spills most registers: three
-// quarters (9 280 rows: 140 and 127, 12 608: 154 and 160).
+// (16 464 rows, two workgroups more than a round: 80 and 97); 384 has to fill half of it (16 464 rows: 165 and 154, 25 216: 179
+// and 217), and so has 512 in bf16 (18 912: 259 and 237, 25 216: 280 and 320).  512 in fp16 spills most registers: three
+// quarters (9 259 rows: 150 and 135, 12 608: 162 and 172).
 inline bool block_tail_pays(bool fp16, long long rows, long long width, long long hidden, long long kv_width, int compute_units) {
   if (block_tail_rows(rows, compute_units) == 32) {
     const double weights = 2e-6 * (double)width * (double)(width + kv_width + hidden), k = 0.256 * (double)rows / compute_units;
