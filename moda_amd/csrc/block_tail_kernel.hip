@@ -3,7 +3,7 @@
 // local to a row, so a workgroup takes BM rows through the whole chain; what one step hands to the next stays in
 // registers and LDS.  As separate launches (block_kernels.hip) the same rows went to memory and back six times, the
 // hidden activations of the MLP, four times as wide, among them: 12 608 rows of width 256 took 69 us in seven launches
-// (projection 9, norm 6, MLP 23 + 15, norm 6, next projections 10.5), here 33.1.
+// (projection 9, norm 6, MLP 23 + 15, norm 6, next projections 10.5), here 33 - 34.
 //
 // Eight waves share the BM rows and divide the features of every product.  The weights sit on the matrix instruction's A
 // side (M = features) and go from memory (L2 after the first workgroup of an XCD) straight into the registers that it
