@@ -311,6 +311,16 @@ typedef struct moda_hip_weight {
 } moda_hip_weight;
 int moda_hip_pack_weights(const moda_hip_weight* weights, int32_t n, void* gelu_table, void* stream);
 int moda_hip_block_tail(const moda_hip_block_tail_args* args, void* stream);
+/*
+ * The attention of a block and its tail in one launch: what moda_hip_fwd(desc, q, k, v, kd, vd, o, lse) and then
+ * moda_hip_block_tail with `attention` = o leave, bit for bit, without o and lse (args->attention is not read).
+ * For tokens as the tail's rows (args->rows = desc's B * T, token by token), one key/value head and G = 2 or 4 query heads of
+ * 64 (feature g * 64 + i of a token's attention output: element i of its query row g), args->width 64 G, no packed batch;
+ * MODA_HIP_EUNSUPPORTED otherwise.  The outputs of the tail may be the buffers of q and of the residual, but not of k, v, kd, vd:
+ * slots of the depth cache that this call does not read, and rows of k, v elsewhere, are fine.
+ */
+int moda_hip_attend_block_tail(const moda_hip_desc* desc, const void* q, const void* k, const void* v, const void* kd, const void* vd,
+                               const moda_hip_block_tail_args* args, void* stream);
 
 /*
  * Which kernels a descriptor runs on: 1 = the matrix-core kernels (tensor rows must then be 16-byte aligned, see

@@ -28,6 +28,7 @@ hipError_t launch_layer_norm(int dtype, int64_t rows, int64_t dim, const void* x
                              hipStream_t stream);
 hipError_t launch_pack_weights(const moda_hip_weight* w, int n, float* gelu_table, hipStream_t stream);
 hipError_t launch_block_tail(const moda_hip_block_tail_args* args, int compute_units, hipStream_t stream);
+hipError_t launch_attend_tail(const moda_hip_block_tail_args* args, const KArgs& attention, hipStream_t stream);
 }  // namespace moda
 
 using moda::KArgs;
@@ -605,21 +606,23 @@ int moda_hip_pack_weights(const moda_hip_weight* w, int32_t n, void* gelu_table,
   return moda::launch_pack_weights(w, n, (float*)gelu_table, (hipStream_t)stream) == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
 }
 
-int moda_hip_block_tail(const moda_hip_block_tail_args* t, void* stream) {
+namespace {
+// what both launches ask of a block tail's arguments; `attention`: with the attention output
+int check_tail(const moda_hip_block_tail_args* t, bool attention) {
   if (!t || t->struct_size != (int32_t)sizeof(*t) || (t->dtype != MODA_HIP_BF16 && t->dtype != MODA_HIP_FP16)) return MODA_HIP_EINVAL;
   if (t->rows < 0 || t->width <= 0 || t->hidden <= 0 || t->n_parts < 0 || t->n_parts > 3) return MODA_HIP_EINVAL;
   if (t->rows == 0) return MODA_HIP_OK;
   if (t->dtype == MODA_HIP_BF16 && !t->gelu_table) return MODA_HIP_EINVAL;
   if ((uintptr_t)t->gelu_table % 16 != 0) return MODA_HIP_EALIGN;
   const bool end_norm = t->post_norm || t->n_parts > 0;
-  for (const void* p : {t->attention, t->residual, (const void*)t->x, t->proj_w, t->fc1_w, t->fc2_w, t->mid_norm_w, t->mid_norm_b,
-                        end_norm ? t->end_norm_w : t->x, end_norm ? t->end_norm_b : t->x})
+  for (const void* p : {attention ? t->attention : t->residual, t->residual, (const void*)t->x, t->proj_w, t->fc1_w, t->fc2_w, t->mid_norm_w,
+                        t->mid_norm_b, end_norm ? t->end_norm_w : t->x, end_norm ? t->end_norm_b : t->x})
     if (!p) return MODA_HIP_EINVAL;
   if ((t->width != 128 && t->width != 256 && t->width != 384 && t->width != 512) || t->hidden % 128 != 0 || t->hidden >= (1 << 20) ||
       t->rows >= (1ll << 30))
     return MODA_HIP_EUNSUPPORTED;
-  for (const void* p : {t->attention, t->residual, (const void*)t->x, t->proj_w, t->fc1_w, t->fc2_w, t->mid_norm_w, t->mid_norm_b,
-                        end_norm ? t->end_norm_w : t->x, end_norm ? t->end_norm_b : t->x})
+  for (const void* p : {attention ? t->attention : t->residual, t->residual, (const void*)t->x, t->proj_w, t->fc1_w, t->fc2_w, t->mid_norm_w,
+                        t->mid_norm_b, end_norm ? t->end_norm_w : t->x, end_norm ? t->end_norm_b : t->x})
     if ((uintptr_t)p % 16 != 0) return MODA_HIP_EALIGN;
   for (const void* p : {t->proj_b, t->fc1_b, t->fc2_b})
     if ((uintptr_t)p % 8 != 0) return MODA_HIP_EALIGN;
@@ -629,10 +632,54 @@ int moda_hip_block_tail(const moda_hip_block_tail_args* t, void* stream) {
     if (p.n % 16 != 0 || p.n >= (1 << 20)) return MODA_HIP_EUNSUPPORTED;
     if ((uintptr_t)p.w % 16 != 0 || (uintptr_t)p.y % 16 != 0 || p.ldy % 8 != 0 || (uintptr_t)p.bias % 8 != 0) return MODA_HIP_EALIGN;
   }
-  int cus = 0;
-  const int rc = check_device(&cus);
-  if (rc) return rc;
+  return MODA_HIP_OK;
+}
+}  // namespace
+
+int moda_hip_block_tail(const moda_hip_block_tail_args* t, void* stream) {
+  int cus = 0, rc = check_tail(t, true);
+  if (rc || t->rows == 0) return rc;
+  if ((rc = check_device(&cus))) return rc;
   return moda::launch_block_tail(t, cus, (hipStream_t)stream) == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
+}
+
+int moda_hip_attend_block_tail(const moda_hip_desc* d, const void* q, const void* k, const void* v, const void* kd, const void* vd,
+                               const moda_hip_block_tail_args* t, void* stream) {
+  KArgs a;
+  int rc = fill_geometry(d, a);
+  if (rc || (rc = check_tail(t, false))) return rc;
+  if (t->rows != (int64_t)a.B * a.T || t->dtype != d->dtype) return MODA_HIP_EINVAL;
+  if (a.D != 64 || a.Dv != 64 || a.Hkv != 1 || a.hdiv != 1 || (a.Gf != 2 && a.Gf != 4) || t->width != 64 * a.Gf || !a.has_seq || a.cu)
+    return MODA_HIP_EUNSUPPORTED;
+  if (t->rows == 0) return MODA_HIP_OK;
+  const int es = elem_size(d->dtype);
+  const bool vec16 = true;
+  MODA_REQ_PTR(q);
+  MODA_REQ_PTR(k);
+  MODA_REQ_PTR(v);
+  MODA_REQ_ALIGN(q, d->q);
+  MODA_REQ_ALIGN(k, d->k);
+  MODA_REQ_ALIGN(v, d->v);
+  if (a.L > 0) {
+    MODA_REQ_PTR(kd);
+    MODA_REQ_PTR(vd);
+    MODA_REQ_ALIGN(kd, d->kd);
+    MODA_REQ_ALIGN(vd, d->vd);
+    if (!(mapped_span_ok(a, d->kd, es) && mapped_span_ok(a, d->vd, es))) return MODA_HIP_EUNSUPPORTED;
+  }
+  a.q = (const uint16_t*)q;
+  a.k = (const uint16_t*)k;
+  a.v = (const uint16_t*)v;
+  a.kd = (const uint16_t*)kd;
+  a.vd = (const uint16_t*)vd;
+  a.sq = cvt(d->q);
+  a.sk = cvt(d->k);
+  a.sv = cvt(d->v);
+  a.skd = cvt(d->kd);
+  a.svd = cvt(d->vd);
+  if (!moda::narrow_slices(a)) return MODA_HIP_EUNSUPPORTED;
+  if ((rc = check_device(&a.compute_units))) return rc;
+  return moda::launch_attend_tail(t, a, (hipStream_t)stream) == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
 }
 
 int moda_hip_uses_matrix_cores(const moda_hip_desc* d) {

@@ -164,6 +164,17 @@ MODA_HD RowPlace row_place(const KArgs& grid, int block, int BM) {
   return {b, bh % grid.Hq, qt, t0, T, !VARLEN || qt < (T * grid.Gf + BM - 1) / BM};
 }
 
+// Which tokens a workgroup of attend_tail_kernel takes: tile `tile` (of `tokens` each) of sequence b, rows [first_row, rows_end) of
+// the [B * T] rows; a sequence's tiles are B workgroups apart, on one XCD (one L2) if B is a multiple of eight.
+struct AttendTailPlace {
+  int b, tile, first_row, rows_end;
+};
+MODA_HD AttendTailPlace attend_tail_place(const KArgs& a, int block, int tokens) {
+  const int tile = block / a.B, b = block % a.B;
+  return {b, tile, b * a.T + tile * tokens, (b + 1) * a.T};
+}
+inline int64_t attend_tail_blocks(const KArgs& a, int tokens) { return (int64_t)a.B * ((a.T + tokens - 1) / tokens); }
+
 // Visible column intervals [0, shi) of the sequence keys and [dlo, dhi) of the depth columns (compact axis) for
 // query row r (all zero for a row past the end).  Ld: depth slots per token, 0 when the launch has no depth stream.
 struct RowVis {

@@ -709,6 +709,12 @@ bool tail_is_one_launch(bool fp16, int64_t rows, int64_t width, int64_t hidden, 
          moda::block_tail_pays(fp16, rows, width, hidden, kv, compute_units);
 }
 
+bool attention_joins(const Tensor& x, int64_t heads, int64_t kv_heads) {
+  int compute_units = 0;
+  return hipDeviceGetAttribute(&compute_units, hipDeviceAttributeMultiprocessorCount, x.get_device()) == hipSuccess && compute_units > 0 &&
+         moda::attention_joins_tail(x.size(0), x.size(1), x.size(2), heads, kv_heads, compute_units);
+}
+
 // Forward pass of all blocks of one stack, launches only: the residual stream, one depth cache and four work tensors
 // are all there is.  A layer's K and V are projected straight into their slot of the cache, where its own attention reads
 // them as the sequence and later layers as a depth slot.  Returns nothing where a kernel's contract is not met (the
@@ -745,9 +751,10 @@ std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>
   const Tensor x0 = x_in.contiguous();
   if ((uintptr_t)x0.const_data_ptr() % 16 != 0) return {};
   const bool tails = tail_is_one_launch(type == at::kHalf, M, C, hidden, kv, x_in.get_device());
+  const bool joined = tails && attention_joins(x_in, heads, kv_heads);  // attention and tail as one launch
   Tensor x = at::empty({B, N, C}, opt), h = at::empty({M, C}, opt), q = at::empty({M, C}, opt), x1 = tails ? Tensor() : at::empty({M, C}, opt),
          hid = tails ? Tensor() : at::empty({M, hidden}, opt), ck = at::empty({B, N * L, kv}, opt), cv = at::empty({B, N * L, kv}, opt),
-         lse = at::empty({M * heads}, opt.dtype(at::kFloat));
+         lse = joined ? Tensor() : at::empty({M * heads}, opt.dtype(at::kFloat));
   auto part = [&](const Tensor& w, const Tensor& b, int64_t first, int64_t n, void* y, int64_t ldy) {
     return moda_hip_linear_part{(const char*)in_ptr(w) + first * w.size(1) * es, b.defined() ? (const char*)in_ptr(b) + first * es : nullptr, y,
                                 ldy, n};
@@ -815,9 +822,10 @@ std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>
     }
     d.L = n > 0 ? L : 0;
     d.L_valid = (int32_t)n;
-    check_rc(moda_hip_fwd(&d, in_ptr(q), slot_of(ck, n), slot_of(cv, n), n > 0 ? in_ptr(ck) : nullptr, n > 0 ? in_ptr(cv) : nullptr,
-                          out_ptr(h), (float*)out_ptr(lse), stream),
-             "moda_hip_fwd");
+    if (!joined)
+      check_rc(moda_hip_fwd(&d, in_ptr(q), slot_of(ck, n), slot_of(cv, n), n > 0 ? in_ptr(ck) : nullptr, n > 0 ? in_ptr(cv) : nullptr,
+                            out_ptr(h), (float*)out_ptr(lse), stream),
+               "moda_hip_fwd");
     const int64_t slots = b.kv_ffn_w.defined() ? 2 : 1;
     if (tails) {
       moda_hip_block_tail_args t = {};
@@ -855,7 +863,12 @@ std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>
         t.parts[2].w = qkv + (C + kv) * C * es;
         t.n_parts = 3;
       }
-      check_rc(moda_hip_block_tail(&t, stream), "moda_hip_block_tail");
+      if (joined)
+        check_rc(moda_hip_attend_block_tail(&d, in_ptr(q), slot_of(ck, n), slot_of(cv, n), n > 0 ? in_ptr(ck) : nullptr,
+                                            n > 0 ? in_ptr(cv) : nullptr, &t, stream),
+                 "moda_hip_attend_block_tail");
+      else
+        check_rc(moda_hip_block_tail(&t, stream), "moda_hip_block_tail");
       projected = true;
     } else {
       linear(in_ptr(h), C, {part(b.proj_w, b.proj_b, 0, C, out_ptr(x1), C)}, cur, false);

@@ -18,35 +18,44 @@ namespace moda {
 // 181 -> 145 us and 217 -> 187 us at 3 x 4 144 tokens, 16 query heads without a depth stream.
 struct RowLarge {
   static constexpr int W = 8, NST = 3, DIST = 2, NB = 2;
-  static constexpr bool PP = false;
+  static constexpr bool PP = false, APART = false;
 };
 // RowLarge with the upper half of the workgroup running half a tile behind the lower half (see the
 // forward kernel); one more ring stage keeps the previous tile's V alive for it.
 struct RowLargePP {
   static constexpr int W = 8, NST = 4, DIST = 2, NB = 2;
-  static constexpr bool PP = true;
+  static constexpr bool PP = true, APART = false;
 };
 template <int HD>
 struct RowSmall {
   static constexpr int W = 4, NST = 2, DIST = 1, NB = 2;  // 64 KB of LDS at 128, 32 KB at 64
-  static constexpr bool PP = false;
+  static constexpr bool PP = false, APART = false;
 };
 // 64-wide tiles, short sequences: two waves, for a row count whose last 128-row tile would be half empty.
 struct RowShort {
   static constexpr int W = 2, NST = 2, DIST = 1, NB = 2;
-  static constexpr bool PP = false;
+  static constexpr bool PP = false, APART = false;
 };
 // ... and with a third ring stage, for dQ launches of equal, HBM-bound workgroups (see pick_short_rows).
 struct RowShort3 {
   static constexpr int W = 2, NST = 3, DIST = 2, NB = 2;
-  static constexpr bool PP = false;
+  static constexpr bool PP = false, APART = false;
+};
+
+// The attention of a block with its dense part in one launch (attend_tail_kernel): eight waves load the tiles, WORK of them take 32
+// query rows each, those of the workgroup's 64 or 32 tokens of all heads.  Each of those has a private K and V tile apart from the
+// ring.
+template <int WORK>
+struct RowBlock {
+  static constexpr int W = 8, NST = 4, DIST = 3, NB = 2, WORKING = WORK;
+  static constexpr bool PP = false, APART = true;
 };
 
 // Head dims above 128 (tile width 256, 16x16x32 kernels only): 16 query rows per wave, so that the wave's Q (and
 // dO) operands and its 256-wide accumulator still fit the register file; two ring stages of 64 KB.
 struct RowWide {
   static constexpr int W = 8, NST = 2, DIST = 1, NB = 1;
-  static constexpr bool PP = false;
+  static constexpr bool PP = false, APART = false;
 };
 
 // Host side, 128-wide tiles: the small shape is used when the large one would not even give every compute unit
@@ -116,6 +125,14 @@ inline bool block_tail_pays(bool fp16, long long rows, long long width, long lon
   }
   const long long last = ((rows + 63) / 64 - 1) % compute_units + 1;  // workgroups of the last round
   return width <= 256 || 4 * last >= (width > 384 && fp16 ? 3 : 2) * compute_units;
+}
+
+// ... and whether the block's attention joins it (attend_tail_kernel): workgroups of 64 (or 32) tokens of one sequence, which a
+// sequence's last one has few of, as long as they take no more rounds than workgroups of as many rows of all.
+inline bool attention_joins_tail(long long batch, long long tokens, long long width, long long heads, long long kv_heads, int compute_units) {
+  const long long rows = batch * tokens, bm = block_tail_rows(rows, compute_units), cus = compute_units;
+  const long long tiles = (rows + bm - 1) / bm, with = batch * ((tokens + bm - 1) / bm);
+  return (heads == 2 || heads == 4) && width == 64 * heads && kv_heads == 1 && (with + cus - 1) / cus == (tiles + cus - 1) / cus;
 }
 
 }  // namespace moda

@@ -1213,11 +1213,18 @@ void walk_norm(int rows, int dim) {
 
 // A block's dense part in one launch: rows in and out, every product's weights, biases, norms and parts; what LDS holds.
 // Weights are read through their packed copies, each piece against the order that pack_weights_kernel leaves.
+// `tokens` > 0: with the attention before it (attend_tail_kernel), workgroups of BM tokens of one of rows / tokens sequences.
 template <int C, int NB>
-void walk_tail_of(bool fp16, int rows, int hidden, bool post, const std::vector<int>& parts) {
+void walk_tail_of(bool fp16, int rows, int hidden, bool post, const std::vector<int>& parts, int tokens) {
   constexpr int BM = 16 * NB, MB2 = C / 128, MB1 = 2, HC = 256, CH = C / 8, TPR = 512 / BM, NL = CH / TPR;
   const uint32_t table = fp16 ? 0 : MODA_HIP_GELU_TABLE_BYTES, X = table / 2, H = X + BM * C;  // elements
-  const uint32_t lds_bytes = table + (uint32_t)BM * (C + std::max(C, 2 * HC)) * 2;
+  KArgs att = {};
+  att.B = tokens ? rows / tokens : 0;
+  att.T = tokens;
+  typedef RowBlock<BM * (C / 64) / 32> Attend;
+  const uint32_t ring = std::max(Attend::NST * 2 * 64 * 64, BM * 2 * HC), apart = Attend::WORKING * 32 * 64;  // elements
+  const uint32_t lds_bytes = table + (tokens ? (BM * C + ring + apart) * 2 : (uint32_t)BM * (C + std::max(C, 2 * HC)) * 2);
+  if (tokens && (X + apart > H || H + ring + apart > lds_bytes / 2)) fail("private K and V tiles of the attention");
   int idx = 0;
   const auto region2 = [&](const char* name, int64_t n, bool track = false) { return add_region(name, idx++, n * 2, 2, track); };
   const uint16_t *h = region2("attention", (int64_t)rows * C), *res = region2("residual", (int64_t)rows * C), *x = region2("x", (int64_t)rows * C, true);
@@ -1241,10 +1248,13 @@ void walk_tail_of(bool fp16, int rows, int hidden, bool post, const std::vector<
   const auto lds = [&](uint32_t first, int64_t off, int elems, uint32_t limit, const char* what) {  // [first, limit) elements
     if (off < 0 || first + off + elems > limit || limit * 2 > lds_bytes) fail("%s at element %lld of LDS", what, (long long)off);
   };
-  const int nblk = (rows + BM - 1) / BM;
+  const int nblk = tokens ? (int)attend_tail_blocks(att, BM) : (rows + BM - 1) / BM;
   for (int block = 0; block < nblk; block++)
     for (int tid = 0; tid < 512; tid++) {
-      const int lane = tid & 63, n = lane & 15, q4 = lane >> 4, wave = tid >> 6, r0 = block * BM, sigma = slot_base(n >> 2) + (n & 3);
+      const AttendTailPlace place = tokens ? attend_tail_place(att, block, BM) : AttendTailPlace{0, block, block * BM, rows};
+      const int rows_end = place.rows_end;
+      if (place.first_row >= rows_end) fail("a workgroup without rows");
+      const int lane = tid & 63, n = lane & 15, q4 = lane >> 4, wave = tid >> 6, r0 = place.first_row, sigma = slot_base(n >> 2) + (n & 3);
       const int f2 = wave * 16 * MB2, lrow = tid / TPR, lsub = tid % TPR;
       const uint32_t all = lds_bytes / 2;
       // one product: `mb` blocks of 16 features from f on (packed [features][width]), steps first .. first + nk - 1 of 32
@@ -1275,13 +1285,13 @@ void walk_tail_of(bool fp16, int rows, int hidden, bool post, const std::vector<
             check_access(wn, weight + (lsub + TPR * j) * 8, 16, false);
             check_access(bn, b + (lsub + TPR * j) * 8, 16, false);
           }
-          if (store && r0 + lrow < rows) check_access("x", x + (int64_t)(r0 + lrow) * C + (lsub + TPR * j) * 8, 16, true);
+          if (store && r0 + lrow < rows_end) check_access("x", x + (int64_t)(r0 + lrow) * C + (lsub + TPR * j) * 8, 16, true);
         }
       };
       ctx("block_tail_kernel", block, wave, lane, "rows in");
       for (int j = 0; j < BM * CH / 512; j++) {
-        const int at = (tid + 512 * j) / CH, row = std::min(r0 + at, rows - 1), ch = (tid + 512 * j) % CH;
-        check_access("attention", h + (int64_t)row * C + ch * 8, 16, false);
+        const int at = (tid + 512 * j) / CH, row = std::min(r0 + at, rows_end - 1), ch = (tid + 512 * j) % CH;
+        if (!tokens) check_access("attention", h + (int64_t)row * C + ch * 8, 16, false);
         check_access("residual", res + (int64_t)row * C + ch * 8, 16, false);
         lds(X, RowLayout<C>::off(at, ch), 8, H, "residual row");
         lds(H, RowLayout<C>::off(at, ch), 8, all, "attention row");
@@ -1329,7 +1339,7 @@ void walk_tail_of(bool fp16, int rows, int hidden, bool post, const std::vector<
           }
           ctx("block_tail_kernel", block, wave, lane, "projected rows out");
           const int chunks = 2 * std::min(blocks - first, 8 * MBQ);
-          for (int ch = lsub; ch < chunks && r0 + lrow < rows; ch += TPR) {
+          for (int ch = lsub; ch < chunks && r0 + lrow < rows_end; ch += TPR) {
             const int blk = first + (ch >> 1);
             size_t pi = 0;
             while (blk >= end[pi]) pi++;
@@ -1354,10 +1364,11 @@ void walk_tail_of(bool fp16, int rows, int hidden, bool post, const std::vector<
     }
   }
 }
-void walk_tail(bool fp16, int rows, int width, int hidden, bool post, const std::vector<int>& parts) {
+void walk_tail(bool fp16, int rows, int width, int hidden, bool post, const std::vector<int>& parts, int tokens = 0) {
   const auto go = [&](auto c) {
     constexpr int C = decltype(c)::value;
-    block_tail_rows(rows, 256) == 32 ? walk_tail_of<C, 2>(fp16, rows, hidden, post, parts) : walk_tail_of<C, 4>(fp16, rows, hidden, post, parts);
+    block_tail_rows(rows, 256) == 32 ? walk_tail_of<C, 2>(fp16, rows, hidden, post, parts, tokens)
+                                     : walk_tail_of<C, 4>(fp16, rows, hidden, post, parts, tokens);
   };
   switch (width) {
     case 128: return go(std::integral_constant<int, 128>{});
@@ -1542,6 +1553,17 @@ int main(int argc, char** argv) {
     for (int i = 7; i < argc; i++) parts.push_back(arg(i));
     walk_tail(std::string(argv[2]) == "fp16", arg(3), arg(4), arg(5), arg(6) != 0, parts);
     printf("OK checked=%lld\n", g_checked);
+    return 0;
+  }
+  if (what == "attend_tail") {  // dtype sequences tokens width hidden post_norm n0 [n1 n2]
+    std::vector<int> parts;
+    for (int i = 8; i < argc; i++) parts.push_back(arg(i));
+    walk_tail(std::string(argv[2]) == "fp16", arg(3) * arg(4), arg(5), arg(6), arg(7) != 0, parts, arg(4));
+    printf("OK checked=%lld\n", g_checked);
+    return 0;
+  }
+  if (what == "attend_tail_rule") {  // sequences tokens width heads kv_heads compute_units
+    printf("%s\n", attention_joins_tail(arg(2), arg(3), arg(4), arg(5), arg(6), arg(7)) ? "joins" : "apart");
     return 0;
   }
   if (what == "slots") {  // the slot arithmetic of partially filled streams against the division it stands for

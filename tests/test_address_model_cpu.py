@@ -356,6 +356,41 @@ def test_block_tail(walker, case):
         assert out.returncode == (1 if shrink else 0) and ("VIOLATION" if shrink else "OK checked") in out.stdout, (shrink, out.stdout)
 
 
+@pytest.mark.parametrize("case", [
+    # dtype, sequences, tokens, width, hidden, post-norm, features of each part: 32 tokens a workgroup and 64; one token, whole
+    # workgroups, a last one of one token
+    ("bf16", 1, 1, 128, 128, 0, 128, 16, 16),
+    ("bf16", 3, 33, 256, 256, 1, 256, 64, 64),
+    ("fp16", 65, 129, 128, 128, 0, 128, 64, 64),
+    ("bf16", 129, 64, 256, 256, 0, 256, 64, 64),
+], ids=lambda c: "-".join(map(str, c)))
+def test_attention_with_block_tail(walker, case):
+    """The rows of the dense part where the attention joins it; the attention's own accesses are the forward kernel's."""
+    for shrink in (None, "x:2", "residual:2", "y0:2", "end_w:2"):
+        e = dict(os.environ, **({"WALKER_SHRINK": shrink} if shrink else {}))
+        out = subprocess.run([walker, "attend_tail", *map(str, case)], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=e, timeout=600)
+        assert out.returncode == (1 if shrink else 0) and ("VIOLATION" if shrink else "OK checked") in out.stdout, (shrink, out.stdout)
+
+
+@pytest.mark.parametrize("case", [
+    # sequences, tokens, width, heads, key/value heads, compute units: rounds of workgroups by sequences against those of all rows;
+    # six blocks, us apart / joined
+    (64, 197, 256, 4, 1, 256, "joins"),   # 281 / 256
+    (36, 197, 256, 4, 1, 256, "joins"),   # 218 / 193: 252 workgroups of 32 tokens
+    (37, 197, 256, 4, 1, 256, "apart"),   # 259 of them
+    (64, 257, 256, 4, 1, 256, "joins"),   # 462 / 464: two rounds either way
+    (100, 145, 256, 4, 1, 256, "apart"),  # 300 workgroups of 64 tokens, 227 of 64 rows
+    (64, 50, 128, 2, 1, 256, "joins"),    # 130 / 108
+    (64, 197, 256, 4, 2, 256, "apart"),   # what the kernel does not take
+    (64, 197, 256, 2, 1, 256, "apart"),
+    (64, 197, 512, 8, 1, 256, "apart"),
+    (64, 197, 384, 6, 1, 256, "apart"),
+], ids=lambda c: "-".join(map(str, c[:6])))
+def test_when_a_blocks_attention_joins_its_tail(walker, case):
+    out = subprocess.run([walker, "attend_tail_rule", *map(str, case[:-1])], stdout=subprocess.PIPE, text=True, check=True).stdout
+    assert out.strip() == case[-1]
+
+
 def test_packed_weights(walker):
     out = subprocess.run([walker, "pack", "7"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=600)
     assert out.returncode == 0 and "OK checked" in out.stdout, out.stdout

@@ -621,7 +621,7 @@ def test_block_tail_and_weight_packing_refuse_what_their_kernels_cannot_take():
     class Weight(ctypes.Structure):
         _fields_ = [("w", ptr), ("packed", ptr), ("n", i64), ("k", i64)]
 
-    def tail(**given):
+    def tail(joined=None, **given):
         v = dict(struct_size=ctypes.sizeof(Tail), dtype=0, rows=4, width=256, hidden=1024, post_norm=0, n_parts=1, gelu_table=0x1000,
                  end_norm_w=0x1000, end_norm_b=0x1000, **{n: 0x1000 for n in pointers + biases})
         part = dict(w=0x2000, bias=0x3000, y=0x4000, ldy=64, n=64)
@@ -629,7 +629,18 @@ def test_block_tail_and_weight_packing_refuse_what_their_kernels_cannot_take():
         t = Tail(**{**v, **given})
         for i in range(3):
             t.parts[i] = Part(*(part[n] for n in ("w", "bias", "y", "ldy", "n")))
-        return lib.moda_hip_block_tail(ctypes.byref(t), None)
+        if joined is None:
+            return lib.moda_hip_block_tail(ctypes.byref(t), None)
+        d = _lib.Desc()
+        d.struct_size, d.mode, d.B, d.T, d.H, d.G, d.D, d.scale = ctypes.sizeof(d), 1, 2, 2, 1, 4, 64, 1.0
+        at = dict(q=0x1000, k=0x1000, v=0x1000, kd=None, vd=None)
+        at.update({n: joined[n] for n in at if n in joined})
+        for n, x in joined.items():
+            if n not in at:
+                setattr(d, n, x)
+        for n in ("q", "k", "v", "kd", "vd", "o"):
+            setattr(d, n, _lib.Strides(1024, 64, 64))
+        return lib.moda_hip_attend_block_tail(ctypes.byref(d), *(at[n] for n in ("q", "k", "v", "kd", "vd")), ctypes.byref(t), None)
 
     def pack(n=1, table=0x1000, **given):
         w = dict(w=0x2000, packed=0x3000, n=32, k=64)
@@ -648,6 +659,15 @@ def test_block_tail_and_weight_packing_refuse_what_their_kernels_cannot_take():
     for bad in (dict(gelu_table=0x1008), dict(end_norm_w=0x1008), dict(part_w=0x2008), dict(part_y=0x4008), dict(part_ldy=68),
                 dict(part_bias=0x3004), *({n: 0x1008} for n in pointers), *({n: 0x1004} for n in biases)):
         assert tail(**bad) == -3, bad
+    # the same with the attention before it, whose output is not asked for
+    assert tail({"B": 0}, rows=0) == 0 and tail({}, attention=None) == tail({})
+    for bad in (dict(rows=5), dict(dtype=1), dict(residual=None), *({"joined": {n: None}} for n in "qkv"), dict(joined=dict(L=3))):
+        assert tail(**{"joined": {}, **bad}) == -1, bad
+    for bad in (dict(joined=dict(G=2)), dict(joined=dict(G=1), width=128), dict(joined=dict(G=8), width=512), dict(joined=dict(H=2)),
+                dict(joined=dict(D=32)), dict(joined=dict(D=128)), dict(joined=dict(Dv=32)), dict(width=384)):
+        assert tail(**{"joined": {}, **bad}) == -2, bad
+    for bad in (*({"joined": {n: 0x1008}} for n in "qkv"), dict(joined=dict(L=3, kd=0x1008, vd=0x1000)), dict(x=0x1008)):
+        assert tail(**{"joined": {}, **bad}) == -3, bad
     for bad in (dict(n=0), dict(w=None), dict(packed=None), dict(rows=0), dict(k=0)):
         assert pack(**bad) == -1, bad
     for bad in (dict(rows=24), dict(k=48), dict(rows=1 << 20), dict(k=1 << 20), dict(rows=1 << 16, k=1 << 15)):

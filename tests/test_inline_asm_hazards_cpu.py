@@ -86,7 +86,7 @@ def assembly(tmp_path_factory):
         return dst
 
     with ThreadPoolExecutor(4) as ex:
-        return list(ex.map(build, ["fwd_kernel", "bwd_dq_kernel", "bwd_dkv_kernel", "bwd_dkv_flat_kernel", "bwd_short_kernel"]))
+        return list(ex.map(build, ["fwd_kernel", "bwd_dq_kernel", "bwd_dkv_kernel", "bwd_dkv_flat_kernel", "bwd_short_kernel", "attend_tail_kernel"]))
 
 
 def test_scanner_sees_the_hazard():

@@ -2161,7 +2161,8 @@ class _BlockTail:
         arr = (Weight * len(ws))(*(Weight(w.data_ptr(), p.data_ptr(), *w.shape) for w, p in zip(ws, self.packed)))
         assert self.lib.moda_hip_pack_weights(arr, len(ws), ptr(self.table.data_ptr()), ptr(torch.cuda.current_stream().cuda_stream)) == 0
 
-    def run(self, attention, residual, post_norm):
+    def run(self, attention, residual, post_norm, attend=None):
+        """`attend(args)`: makes the call instead, with the attention before it."""
         ptr, i32, i64, f32 = (getattr(self.ct, "c_" + n) for n in ("void_p", "int32", "int64", "float"))
 
         class Part(self.ct.Structure):
@@ -2172,18 +2173,19 @@ class _BlockTail:
                         ("residual", ptr), ("x", ptr), *((n, ptr) for n in self.NAMES), ("gelu_table", ptr), ("mid_eps", f32),
                         ("end_eps", f32), ("post_norm", i32), ("n_parts", i32), ("parts", Part * 3)]
 
-        rows = attention.shape[0]
+        rows = residual.shape[0]
         x = residual.clone()  # in place
         ys = [torch.full((rows + 1, w.shape[0] + 8), 7.0, device=x.device, dtype=x.dtype) for w, _ in self.parts]
         a = Args(struct_size=self.ct.sizeof(Args), dtype={torch.bfloat16: 0, torch.float16: 1}[self.dtype], rows=rows, width=self.width,
-                 hidden=self.hidden, attention=attention.data_ptr(), residual=x.data_ptr(), x=x.data_ptr(), gelu_table=self.table.data_ptr(),
+                 hidden=self.hidden, attention=None if attend else attention.data_ptr(), residual=x.data_ptr(), x=x.data_ptr(), gelu_table=self.table.data_ptr(),
                  mid_eps=1e-6, end_eps=1e-6, post_norm=int(post_norm), n_parts=len(ys))
         for n in self.NAMES:
             setattr(a, n, self.w[n].data_ptr())
         a.proj_w, a.fc1_w, a.fc2_w = (p.data_ptr() for p in self.packed[:3])
         for i, y in enumerate(ys):
             a.parts[i] = Part(self.packed[3 + i].data_ptr(), self.parts[i][1].data_ptr(), y.data_ptr(), y.stride(0), self.parts[i][0].shape[0])
-        assert self.lib.moda_hip_block_tail(self.ct.byref(a), ptr(torch.cuda.current_stream().cuda_stream)) == 0
+        stream = ptr(torch.cuda.current_stream().cuda_stream)
+        assert (attend(self.ct.byref(a), stream) if attend else self.lib.moda_hip_block_tail(self.ct.byref(a), stream)) == 0
         return x, ys
 
 
@@ -2278,6 +2280,73 @@ def test_block_tail_equals_its_pieces_bitwise(gpu_device, case, post_norm, dtype
     assert torch.equal(x, z if post_norm else y), (x != (z if post_norm else y)).float().mean()
     for (w, b), got in zip(t.parts, ys):
         assert torch.equal(got[:rows, :w.shape[0]], lin(z, w, b))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", [
+    # sequences, tokens, heads, slots, filled ones, mode, chunk: workgroups of 32 tokens (up to 8192 rows) and of 64; a sequence of
+    # one token, ends of workgroups, half tiles, more tiles than the ring holds; no, one, few and many slots (one to six private
+    # tiles a wave); causal; chunks that a wave walks itself and chunks through the ring
+    (1, 1, 4, 0, 0, "noncausal", 0),
+    (3, 1, 2, 3, 2, "causal", 0),
+    (2, 31, 4, 12, 11, "noncausal", 0),
+    (5, 33, 2, 12, 1, "noncausal", 0),
+    (3, 64, 4, 5, 5, "causal", 0),
+    (2, 65, 4, 40, 21, "noncausal", 0),
+    (2, 300, 2, 6, 4, "causal", 0),
+    (2, 261, 4, 0, 0, "causal", 0),
+    (2, 100, 4, 12, 7, "chunk", 16),
+    (2, 150, 2, 3, 2, "chunk", 48),
+    (66, 128, 4, 12, 11, "noncausal", 0),
+    (43, 197, 4, 12, 5, "noncausal", 0),
+    (65, 129, 2, 4, 3, "causal", 0),
+    (1, 8257, 2, 2, 1, "causal", 0),
+    (84, 100, 4, 6, 5, "chunk", 16),
+], ids=str)
+def test_attention_with_block_tail_equals_the_two_launches_bitwise(gpu_device, case, dtype):
+    """moda_hip_attend_block_tail against the forward kernel and moda_hip_block_tail, one after the other.  k and v lie in the first free
+    slot of the depth cache (as a stack has them) where there is one; slots that hold nothing are NaN."""
+    import ctypes
+
+    from moda_amd import _lib, ops
+
+    B, T, heads, L, filled, mode, chunk = case
+    say(f"CASE attention with block tail {case} {dtype}")
+    width, rows, post_norm = 64 * heads, B * T, (B + T) % 2 == 1
+    t = _BlockTail(width, 384, (width, 64, 64), dtype, gpu_device, seed=T)
+    gen = torch.Generator(device=gpu_device).manual_seed(rows + L)
+    rn = lambda *s: (0.5 * torch.randn(*s, generator=gen, device=gpu_device)).to(dtype)
+    q, res = rn(B, T * heads, 1, 64), rn(rows, width)
+    slots = max(L, 1)
+    ck, cv = (rn(B, T, slots, 64) for _ in range(2))
+    if filled < L:
+        ck[:, :, filled:], cv[:, :, filled:] = float("nan"), float("nan")
+        k, v = ck[:, :, filled:filled + 1], cv[:, :, filled:filled + 1]
+        k.copy_(rn(B, T, 1, 64))
+        v.copy_(rn(B, T, 1, 64))
+    else:
+        k, v = rn(B, T, 1, 64), rn(B, T, 1, 64)
+    kd, vd = (None, None) if L == 0 else (ck.view(B, T * L, 1, 64), cv.view(B, T * L, 1, 64))
+    code = {"causal": _lib.CAUSAL, "noncausal": _lib.NONCAUSAL, "chunk": _lib.CHUNK_VISIBLE}[mode]
+    kw = dict(chunk_tokens=chunk) if chunk else {}
+    if L and filled < L:
+        kw["depth_valid"] = filled
+    o, _ = ops._raw_fwd(code, q, k, v, kd, vd, 0.125, heads, **kw)
+    want = t.run(o.reshape(rows, width), res, post_norm)
+
+    d = _lib.Desc()
+    d.struct_size, d.dtype, d.mode, d.L_valid = ctypes.sizeof(d), {torch.bfloat16: 0, torch.float16: 1}[dtype], code, filled if L else 0
+    d.B, d.T, d.H, d.G, d.D, d.Dv, d.L, d.chunk_tokens, d.scale = B, T, 1, heads, 64, 64, L, chunk, 0.125
+    strides = lambda x: _lib.Strides(x.stride(0), x.stride(1), x.stride(2))
+    d.q, d.o, d.k, d.v = strides(q), strides(q), strides(k), strides(v)
+    if L:
+        d.kd, d.vd = strides(kd), strides(vd)
+    p = lambda x: ctypes.c_void_p(None if x is None else x.data_ptr())
+    got = t.run(None, res, post_norm, lambda args, stream: t.lib.moda_hip_attend_block_tail(ctypes.byref(d), p(q), p(k), p(v), p(kd), p(vd), args, stream))
+    assert torch.isfinite(want[0].float()).all()
+    assert torch.equal(got[0], want[0]), (got[0] != want[0]).float().mean()
+    for a, b in zip(got[1], want[1]):
+        assert torch.equal(a, b), (a != b).float().mean()
 
 
 @pytest.mark.parametrize("n", [96, 97, 200])
