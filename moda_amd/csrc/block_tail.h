@@ -183,13 +183,14 @@ struct Product {
 // Elements of the LDS that the ring of a block's attention and then the hidden activations have (see attend_tail_kernel)
 template <typename Shape, int BM>
 constexpr int attend_ring() {
-  return Shape::NST * 2 * 64 * 64 > BM * 2 * 256 ? Shape::NST * 2 * 64 * 64 : BM * 2 * 256;
+  constexpr int rings = 8 / Shape::W * Shape::NST * 2 * 64 * 64;
+  return rings > BM * 2 * 256 ? rings : BM * 2 * 256;
 }
 
 // The same body with the block's attention before it (MODA_SIDE_BY_SIDE, attend_tail_kernel.hip): the workgroup forms the rows of H
 // itself, from the arguments `att` of the forward kernel (fwd.h).  Its rows are then BM tokens of one sequence.
 #ifdef MODA_SIDE_BY_SIDE
-template <typename T, int C, int NB, bool POST, int ADDR>
+template <typename T, int C, int NB, bool POST, int ADDR, int KV_HEADS>
 __global__ __launch_bounds__(512, 2) void attend_tail_kernel(const TailArgs a, const KArgs att) {
 #else
 template <typename T, int C, int NB, bool POST>
@@ -270,9 +271,12 @@ __global__ __launch_bounds__(512, 2) void block_tail_kernel(const TailArgs a) {
     fetch(a.res, res);
 #pragma unroll
     for (int j = 0; j < (NT + 511) / 512; j++) tab[j] = reinterpret_cast<const i32x4*>(a.gelu_table)[tid + 512 * j < NT ? tid + 512 * j : 0];
-    typedef RowBlock<BM * (C / 64) / 32> Shape;
-    fwd_body<T, 64, Shape, ADDR>(att, RowPlace{at.b, 0, at.tile, 0, 0, true}, H, X, H + attend_ring<Shape, BM>(), [&](int row, int chunk, int half, const i32x2& w) MODA_INLINE {
-      *reinterpret_cast<MODA_LDS i32x2*>(H + Rows<C>::off(row / (C / 64), row % (C / 64) * 8 + chunk) + 4 * half) = w;
+    constexpr int G = C / 64 / KV_HEADS, WORK = BM * G / 32;
+    typedef RowBlock<KV_HEADS, WORK> Shape;
+    const int head = KV_HEADS > 1 ? wave / Shape::W : 0;
+    fwd_body<T, 64, Shape, ADDR>(att, RowPlace{at.b, head, at.tile, 0, 0, true}, H + head * (Shape::NST * 2 * 64 * 64), X + head * (WORK * 32 * 64),
+                                 H + attend_ring<Shape, BM>() + head * (WORK * 32 * 64), [&](int row, int chunk, int half, const i32x2& w) MODA_INLINE {
+      *reinterpret_cast<MODA_LDS i32x2*>(H + Rows<C>::off(row / G, (row % G * KV_HEADS + head) * 8 + chunk) + 4 * half) = w;
     });
 #pragma unroll
     for (int mb = 0; mb < MB2; mb++) proj.base[mb] = a.proj_w + (size_t)(f2 + 16 * mb) * C;

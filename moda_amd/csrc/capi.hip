@@ -9,6 +9,7 @@
 #include "../../include/moda_hip.h"
 #include "geometry.h"
 #include "kargs.h"
+#include "tuning.h"
 
 namespace moda {
 hipError_t launch_fwd(const KArgs& a, int dtype, int hd, hipStream_t stream);
@@ -649,7 +650,7 @@ int moda_hip_attend_block_tail(const moda_hip_desc* d, const void* q, const void
   int rc = fill_geometry(d, a);
   if (rc || (rc = check_tail(t, false))) return rc;
   if (t->rows != (int64_t)a.B * a.T || t->dtype != d->dtype) return MODA_HIP_EINVAL;
-  if (a.D != 64 || a.Dv != 64 || a.Hkv != 1 || a.hdiv != 1 || (a.Gf != 2 && a.Gf != 4) || t->width != 64 * a.Gf || !a.has_seq || a.cu)
+  if (a.D != 64 || a.Dv != 64 || a.hdiv != 1 || !a.has_seq || a.cu || !moda::attend_tail_takes(t->width, (int64_t)a.Hkv * a.Gf, a.Hkv, 32))
     return MODA_HIP_EUNSUPPORTED;
   if (t->rows == 0) return MODA_HIP_OK;
   const int es = elem_size(d->dtype);
@@ -679,6 +680,7 @@ int moda_hip_attend_block_tail(const moda_hip_desc* d, const void* q, const void
   a.svd = cvt(d->vd);
   if (!moda::narrow_slices(a)) return MODA_HIP_EUNSUPPORTED;
   if ((rc = check_device(&a.compute_units))) return rc;
+  if (!moda::attend_tail_takes(t->width, (int64_t)a.Hkv * a.Gf, a.Hkv, moda::block_tail_rows(t->rows, a.compute_units))) return MODA_HIP_EUNSUPPORTED;
   return moda::launch_attend_tail(t, a, (hipStream_t)stream) == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
 }
 

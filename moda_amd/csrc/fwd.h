@@ -40,7 +40,12 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
   lds_ptr smem = (lds_ptr)smem_raw;  // ring stage st: K tile at smem + st * 2*BN*HD, V tile right behind it
 #endif
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 31, g = lane >> 5;
+#ifdef MODA_SIDE_BY_SIDE
+  const int tid = (int)threadIdx.x % (64 * Shape::W);  // (half of the workgroup may be at another head: as many barriers there)
+#else
+  const int tid = threadIdx.x;
+#endif
+  const int lane = tid & 63, wave = tid >> 6, n = lane & 31, g = lane >> 5;
   constexpr bool WIDE = (ADDR & 1) != 0, VARLEN = (ADDR & 2) != 0;
   // bit 2: launched without a depth stream (the plain and sequence-only calls): the depth code is compiled out,
   // so that it cannot disturb the register allocation of their main loop

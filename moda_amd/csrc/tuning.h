@@ -42,13 +42,14 @@ struct RowShort3 {
   static constexpr bool PP = false, APART = false;
 };
 
-// The attention of a block with its dense part in one launch (attend_tail_kernel): eight waves load the tiles, WORK of them take 32
-// query rows each, those of the workgroup's 64 or 32 tokens of all heads.  Each of those has a private K and V tile apart from the
-// ring.
-template <int WORK>
+// The attention of a block with its dense part in one launch (attend_tail_kernel): the eight waves of a workgroup, or four for each of
+// two key/value heads with half the ring, load the tiles; WORK of them take 32 query rows each, those of the workgroup's 64 or 32
+// tokens of all the head's query heads.  Each of those has a private K and V tile apart from the ring.
+template <int KV_HEADS, int WORK>
 struct RowBlock {
-  static constexpr int W = 8, NST = 4, DIST = 3, NB = 2, WORKING = WORK;
+  static constexpr int W = 8 / KV_HEADS, NST = 4 / KV_HEADS, DIST = NST - 1, NB = 2, WORKING = WORK;
   static constexpr bool PP = false, APART = true;
+  static_assert(WORK >= 1 && WORK <= W, "the query rows of the workgroup's tokens over its waves");
 };
 
 // Head dims above 128 (tile width 256, 16x16x32 kernels only): 16 query rows per wave, so that the wave's Q (and
@@ -129,10 +130,15 @@ inline bool block_tail_pays(bool fp16, long long rows, long long width, long lon
 
 // ... and whether the block's attention joins it (attend_tail_kernel): workgroups of 64 (or 32) tokens of one sequence, which a
 // sequence's last one has few of, as long as they take no more rounds than workgroups of as many rows of all.
+inline bool attend_tail_takes(long long width, long long heads, long long kv_heads, long long tokens) {
+  const long long group = kv_heads > 0 ? heads / kv_heads : 0;
+  return (kv_heads == 1 || kv_heads == 2) && heads == group * kv_heads && (group == 2 || group == 4) && width == 64 * heads &&
+         tokens * heads <= 256;  // query rows, 32 a wave
+}
 inline bool attention_joins_tail(long long batch, long long tokens, long long width, long long heads, long long kv_heads, int compute_units) {
   const long long rows = batch * tokens, bm = block_tail_rows(rows, compute_units), cus = compute_units;
   const long long tiles = (rows + bm - 1) / bm, with = batch * ((tokens + bm - 1) / bm);
-  return (heads == 2 || heads == 4) && width == 64 * heads && kv_heads == 1 && (with + cus - 1) / cus == (tiles + cus - 1) / cus;
+  return attend_tail_takes(width, heads, kv_heads, bm) && (with + cus - 1) / cus == (tiles + cus - 1) / cus;
 }
 
 }  // namespace moda

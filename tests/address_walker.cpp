@@ -1221,10 +1221,10 @@ void walk_tail_of(bool fp16, int rows, int hidden, bool post, const std::vector<
   KArgs att = {};
   att.B = tokens ? rows / tokens : 0;
   att.T = tokens;
-  typedef RowBlock<BM * (C / 64) / 32> Attend;
-  const uint32_t ring = std::max(Attend::NST * 2 * 64 * 64, BM * 2 * HC), apart = Attend::WORKING * 32 * 64;  // elements
-  const uint32_t lds_bytes = table + (tokens ? (BM * C + ring + apart) * 2 : (uint32_t)BM * (C + std::max(C, 2 * HC)) * 2);
-  if (tokens && (X + apart > H || H + ring + apart > lds_bytes / 2)) fail("private K and V tiles of the attention");
+  const uint32_t ring = std::max(4 * 2 * 64 * 64, BM * 2 * HC), apart = BM * (C / 64);  // elements; 64 a query row, K or V
+  if (tokens && BM * (C / 64) > 256) fail("more query rows than eight waves take");
+  const uint32_t lds_bytes = table + (tokens ? (BM * C + ring + 64 * apart) * 2 : (uint32_t)BM * (C + std::max(C, 2 * HC)) * 2);
+  if (tokens && (X + 64 * apart > H || H + ring + 64 * apart > lds_bytes / 2)) fail("private K and V tiles of the attention");
   int idx = 0;
   const auto region2 = [&](const char* name, int64_t n, bool track = false) { return add_region(name, idx++, n * 2, 2, track); };
   const uint16_t *h = region2("attention", (int64_t)rows * C), *res = region2("residual", (int64_t)rows * C), *x = region2("x", (int64_t)rows * C, true);

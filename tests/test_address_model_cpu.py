@@ -363,6 +363,7 @@ def test_block_tail(walker, case):
     ("bf16", 3, 33, 256, 256, 1, 256, 64, 64),
     ("fp16", 65, 129, 128, 128, 0, 128, 64, 64),
     ("bf16", 129, 64, 256, 256, 0, 256, 64, 64),
+    ("bf16", 3, 33, 512, 256, 0, 512, 128, 128),
 ], ids=lambda c: "-".join(map(str, c)))
 def test_attention_with_block_tail(walker, case):
     """The rows of the dense part where the attention joins it; the attention's own accesses are the forward kernel's."""
@@ -381,7 +382,10 @@ def test_attention_with_block_tail(walker, case):
     (64, 257, 256, 4, 1, 256, "joins"),   # 462 / 464: two rounds either way
     (100, 145, 256, 4, 1, 256, "apart"),  # 300 workgroups of 64 tokens, 227 of 64 rows
     (64, 50, 128, 2, 1, 256, "joins"),    # 130 / 108
-    (64, 197, 256, 4, 2, 256, "apart"),   # what the kernel does not take
+    (64, 197, 256, 4, 2, 256, "joins"),
+    (36, 197, 512, 8, 2, 256, "joins"),
+    (64, 197, 512, 8, 2, 256, "apart"),   # what the kernel does not take: 64 tokens of eight heads
+    (64, 197, 128, 2, 2, 256, "apart"),
     (64, 197, 256, 2, 1, 256, "apart"),
     (64, 197, 512, 8, 1, 256, "apart"),
     (64, 197, 384, 6, 1, 256, "apart"),

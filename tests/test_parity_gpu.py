@@ -2284,7 +2284,7 @@ def test_block_tail_equals_its_pieces_bitwise(gpu_device, case, post_norm, dtype
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("case", [
-    # sequences, tokens, heads, slots, filled ones, mode, chunk: workgroups of 32 tokens (up to 8192 rows) and of 64; a sequence of
+    # sequences, tokens, heads (or key/value heads x query heads on each), slots, filled ones, mode, chunk: workgroups of 32 tokens (up to 8192 rows) and of 64; a sequence of
     # one token, ends of workgroups, half tiles, more tiles than the ring holds; no, one, few and many slots (one to six private
     # tiles a wave); causal; chunks that a wave walks itself and chunks through the ring
     (1, 1, 4, 0, 0, "noncausal", 0),
@@ -2302,6 +2302,12 @@ def test_block_tail_equals_its_pieces_bitwise(gpu_device, case, post_norm, dtype
     (65, 129, 2, 4, 3, "causal", 0),
     (1, 8257, 2, 2, 1, "causal", 0),
     (84, 100, 4, 6, 5, "chunk", 16),
+    (3, 33, (2, 2), 12, 11, "noncausal", 0),
+    (2, 261, (2, 4), 6, 2, "causal", 0),
+    (1, 1, (2, 4), 0, 0, "noncausal", 0),
+    (64, 129, (2, 2), 4, 3, "noncausal", 0),
+    (85, 100, (2, 2), 6, 5, "chunk", 16),
+    (2, 150, (2, 4), 3, 2, "chunk", 48),
 ], ids=str)
 def test_attention_with_block_tail_equals_the_two_launches_bitwise(gpu_device, case, dtype):
     """moda_hip_attend_block_tail against the forward kernel and moda_hip_block_tail, one after the other.  k and v lie in the first free
@@ -2311,32 +2317,33 @@ def test_attention_with_block_tail_equals_the_two_launches_bitwise(gpu_device, c
     from moda_amd import _lib, ops
 
     B, T, heads, L, filled, mode, chunk = case
+    H, G = heads if isinstance(heads, tuple) else (1, heads)
     say(f"CASE attention with block tail {case} {dtype}")
-    width, rows, post_norm = 64 * heads, B * T, (B + T) % 2 == 1
-    t = _BlockTail(width, 384, (width, 64, 64), dtype, gpu_device, seed=T)
+    width, rows, post_norm = 64 * H * G, B * T, (B + T) % 2 == 1
+    t = _BlockTail(width, 384, (width, 64 * H, 64 * H), dtype, gpu_device, seed=T)
     gen = torch.Generator(device=gpu_device).manual_seed(rows + L)
     rn = lambda *s: (0.5 * torch.randn(*s, generator=gen, device=gpu_device)).to(dtype)
-    q, res = rn(B, T * heads, 1, 64), rn(rows, width)
+    q, res = rn(B, T * G, H, 64), rn(rows, width)
     slots = max(L, 1)
-    ck, cv = (rn(B, T, slots, 64) for _ in range(2))
+    ck, cv = (rn(B, T, slots, H, 64) for _ in range(2))
     if filled < L:
         ck[:, :, filled:], cv[:, :, filled:] = float("nan"), float("nan")
-        k, v = ck[:, :, filled:filled + 1], cv[:, :, filled:filled + 1]
-        k.copy_(rn(B, T, 1, 64))
-        v.copy_(rn(B, T, 1, 64))
+        k, v = ck[:, :, filled], cv[:, :, filled]
+        k.copy_(rn(B, T, H, 64))
+        v.copy_(rn(B, T, H, 64))
     else:
-        k, v = rn(B, T, 1, 64), rn(B, T, 1, 64)
-    kd, vd = (None, None) if L == 0 else (ck.view(B, T * L, 1, 64), cv.view(B, T * L, 1, 64))
+        k, v = rn(B, T, H, 64), rn(B, T, H, 64)
+    kd, vd = (None, None) if L == 0 else (ck.view(B, T * L, H, 64), cv.view(B, T * L, H, 64))
     code = {"causal": _lib.CAUSAL, "noncausal": _lib.NONCAUSAL, "chunk": _lib.CHUNK_VISIBLE}[mode]
     kw = dict(chunk_tokens=chunk) if chunk else {}
     if L and filled < L:
         kw["depth_valid"] = filled
-    o, _ = ops._raw_fwd(code, q, k, v, kd, vd, 0.125, heads, **kw)
+    o, _ = ops._raw_fwd(code, q, k, v, kd, vd, 0.125, G, **kw)
     want = t.run(o.reshape(rows, width), res, post_norm)
 
     d = _lib.Desc()
     d.struct_size, d.dtype, d.mode, d.L_valid = ctypes.sizeof(d), {torch.bfloat16: 0, torch.float16: 1}[dtype], code, filled if L else 0
-    d.B, d.T, d.H, d.G, d.D, d.Dv, d.L, d.chunk_tokens, d.scale = B, T, 1, heads, 64, 64, L, chunk, 0.125
+    d.B, d.T, d.H, d.G, d.D, d.Dv, d.L, d.chunk_tokens, d.scale = B, T, H, G, 64, 64, L, chunk, 0.125
     strides = lambda x: _lib.Strides(x.stride(0), x.stride(1), x.stride(2))
     d.q, d.o, d.k, d.v = strides(q), strides(q), strides(k), strides(v)
     if L:
