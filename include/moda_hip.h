@@ -313,7 +313,8 @@ int moda_hip_pack_weights(const moda_hip_weight* weights, int32_t n, void* gelu_
 int moda_hip_block_tail(const moda_hip_block_tail_args* args, void* stream);
 /*
  * The attention of a block and its tail in one launch: what moda_hip_fwd(desc, q, k, v, kd, vd, o, lse) and then
- * moda_hip_block_tail with `attention` = o leave, bit for bit, without o and lse (args->attention is not read).
+ * moda_hip_block_tail with `attention` = o leave, bit for bit (chunks of more than 64 query rows: up to the order in which their depth
+ * columns are summed, which follows a workgroup's rows), without o and lse (args->attention is not read).
  * For tokens as the tail's rows (args->rows = desc's B * T, token by token), H = 1 or 2 key/value heads and G = 2 or 4 query heads
  * of 64 on each (feature (g * H + h) * 64 + i of a token's attention output: element i of head h of its query row g), args->width
  * 64 G H (512: as many rows as go 32 a workgroup, 32 times the compute units), no packed batch;

@@ -751,7 +751,9 @@ std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>
   const Tensor x0 = x_in.contiguous();
   if ((uintptr_t)x0.const_data_ptr() % 16 != 0) return {};
   const bool tails = tail_is_one_launch(type == at::kHalf, M, C, hidden, kv, x_in.get_device());
-  const bool joined = tails && attention_joins(x_in, heads, kv_heads);  // attention and tail as one launch
+  // Attention and tail as one launch.  (Of chunks of more than 64 query rows the depth columns are summed from where a workgroup's own
+  // begin: those keep the forward kernel's workgroups, and with them the bits.)
+  const bool joined = tails && chunk_tokens * (heads / kv_heads) <= 64 && attention_joins(x_in, heads, kv_heads);
   Tensor x = at::empty({B, N, C}, opt), h = at::empty({M, C}, opt), q = at::empty({M, C}, opt), x1 = tails ? Tensor() : at::empty({M, C}, opt),
          hid = tails ? Tensor() : at::empty({M, hidden}, opt), ck = at::empty({B, N * L, kv}, opt), cv = at::empty({B, N * L, kv}, opt),
          lse = joined ? Tensor() : at::empty({M * heads}, opt.dtype(at::kFloat));
