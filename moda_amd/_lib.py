@@ -33,6 +33,7 @@ EXPORTS = (
     "moda_hip_linear",
     "moda_hip_layer_norm",
     "moda_hip_pack_weights",
+    "moda_hip_pack_weights_and_norm",
     "moda_hip_block_tail",
     "moda_hip_attend_block_tail",
     "moda_hip_uses_matrix_cores",

@@ -23,6 +23,58 @@ __device__ __forceinline__ float gelu(float x) {
   return (x - __builtin_amdgcn_fmed3f(x, kNegInf, 0.f)) - a * t * r * fast_exp2(a * a * (-0.5f * kLog2e));
 }
 
+// Layer norm of 256 / LPR rows, LPR lanes a row with CH pieces of eight each (block_kernels.hip).
+template <typename T, int LPR, int CH>
+__device__ __forceinline__ void layer_norm_rows(unsigned block, const uint16_t* x, const uint16_t* weight, const uint16_t* bias, float eps, uint16_t* y,
+                                                int rows, int dim) {
+  const int tid = threadIdx.x, sub = tid % LPR;
+  const int row = (int)block * (256 / LPR) + tid / LPR;
+  if (row >= rows) return;  // whole lane groups leave together
+  auto sum = [](float v) {
+#pragma unroll
+    for (int s = LPR / 2; s > 0; s >>= 1) v += __shfl_xor(v, s, 64);
+    return v;
+  };
+  auto load8 = [](const uint16_t* p, float (&f)[8]) {
+    const i32x4 v = *reinterpret_cast<const i32x4*>(p);
+#pragma unroll
+    for (int i = 0; i < 4; i++) unpack2<T>(v[i], f[2 * i], f[2 * i + 1]);
+  };
+  float f[CH][8], s = 0.f;
+#pragma unroll
+  for (int c = 0; c < CH; c++) {
+    const int e = (c * LPR + sub) * 8;
+#pragma unroll
+    for (int i = 0; i < 8; i++) f[c][i] = 0.f;
+    if (e < dim) load8(x + (int64_t)row * dim + e, f[c]);
+#pragma unroll
+    for (int i = 0; i < 8; i++) s += f[c][i];
+  }
+  const float mean = sum(s) / dim;
+  float v = 0.f;
+#pragma unroll
+  for (int c = 0; c < CH; c++)
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const float d = f[c][i] - mean;
+      if ((c * LPR + sub) * 8 < dim) v = __builtin_fmaf(d, d, v);
+    }
+  const float rstd = rsqrtf(sum(v) / dim + eps);
+#pragma unroll
+  for (int c = 0; c < CH; c++) {
+    const int e = (c * LPR + sub) * 8;
+    if (e >= dim) continue;
+    float w[8], b[8];
+    load8(weight + e, w);
+    load8(bias + e, b);
+    i32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      o[i] = pack2<T>((f[c][2 * i] - mean) * rstd * w[2 * i] + b[2 * i], (f[c][2 * i + 1] - mean) * rstd * w[2 * i + 1] + b[2 * i + 1]);
+    *reinterpret_cast<i32x4*>(y + (int64_t)row * dim + e) = o;
+  }
+}
+
 // Rows of W 16-bit elements in LDS, 16-byte chunks swizzled as Tile<> has them for rows of 256 bytes and more.
 template <int W>
 struct RowLayout {

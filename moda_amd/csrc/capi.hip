@@ -27,7 +27,7 @@ hipError_t launch_linear(int dtype, int64_t rows, int64_t K, const void* x, int6
                          const void* residual, int64_t ld_res, bool gelu, int compute_units, hipStream_t stream);
 hipError_t launch_layer_norm(int dtype, int64_t rows, int64_t dim, const void* x, const void* weight, const void* bias, float eps, void* y,
                              hipStream_t stream);
-hipError_t launch_pack_weights(const moda_hip_weight* w, int n, float* gelu_table, hipStream_t stream);
+hipError_t launch_pack_weights(const moda_hip_weight* w, int n, float* gelu_table, const moda_hip_norm_rows* norm, hipStream_t stream);
 hipError_t launch_block_tail(const moda_hip_block_tail_args* args, int compute_units, hipStream_t stream);
 hipError_t launch_attend_tail(const moda_hip_block_tail_args* args, const KArgs& attention, hipStream_t stream);
 }  // namespace moda
@@ -581,19 +581,29 @@ int moda_hip_linear(int32_t dtype, int64_t rows, int64_t K, const void* x, int64
   return e == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
 }
 
-int moda_hip_layer_norm(int32_t dtype, int64_t rows, int64_t dim, const void* x, const void* weight, const void* bias, float eps, void* y,
-                        void* stream) {
+namespace {
+int check_norm(int32_t dtype, int64_t rows, int64_t dim, std::initializer_list<const void*> pointers) {
   if ((dtype != MODA_HIP_BF16 && dtype != MODA_HIP_FP16) || rows < 0 || dim <= 0) return MODA_HIP_EINVAL;
   if (rows == 0) return MODA_HIP_OK;
-  if (!x || !weight || !bias || !y) return MODA_HIP_EINVAL;
+  for (const void* p : pointers)
+    if (!p) return MODA_HIP_EINVAL;
   if (dim % 8 != 0 || dim > 4096 || rows >= (1ll << 31)) return MODA_HIP_EUNSUPPORTED;
-  for (const void* p : {x, weight, bias, (const void*)y})
+  for (const void* p : pointers)
     if ((uintptr_t)p % 16 != 0) return MODA_HIP_EALIGN;
+  return MODA_HIP_OK;
+}
+}  // namespace
+
+int moda_hip_layer_norm(int32_t dtype, int64_t rows, int64_t dim, const void* x, const void* weight, const void* bias, float eps, void* y,
+                        void* stream) {
+  const int rc = check_norm(dtype, rows, dim, {x, weight, bias, y});
+  if (rc || rows == 0) return rc;
   const hipError_t e = moda::launch_layer_norm(dtype, rows, dim, x, weight, bias, eps, y, (hipStream_t)stream);
   return e == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
 }
 
-int moda_hip_pack_weights(const moda_hip_weight* w, int32_t n, void* gelu_table, void* stream) {
+namespace {
+int pack(const moda_hip_weight* w, int32_t n, void* gelu_table, const moda_hip_norm_rows* norm, void* stream) {
   if (!w || n < 1) return MODA_HIP_EINVAL;
   if ((uintptr_t)gelu_table % 16 != 0) return MODA_HIP_EALIGN;
   for (int i = 0; i < n; i++) {
@@ -604,7 +614,18 @@ int moda_hip_pack_weights(const moda_hip_weight* w, int32_t n, void* gelu_table,
   }
   const int rc = check_device();
   if (rc) return rc;
-  return moda::launch_pack_weights(w, n, (float*)gelu_table, (hipStream_t)stream) == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
+  return moda::launch_pack_weights(w, n, (float*)gelu_table, norm, (hipStream_t)stream) == hipSuccess ? MODA_HIP_OK : MODA_HIP_ELAUNCH;
+}
+}  // namespace
+
+int moda_hip_pack_weights(const moda_hip_weight* w, int32_t n, void* gelu_table, void* stream) { return pack(w, n, gelu_table, nullptr, stream); }
+
+int moda_hip_pack_weights_and_norm(const moda_hip_weight* w, int32_t n, void* gelu_table, const moda_hip_norm_rows* norm, void* stream) {
+  if (!norm) return MODA_HIP_EINVAL;
+  const int rc = check_norm(norm->dtype, norm->rows, norm->dim, {norm->x, norm->weight, norm->bias, norm->y});
+  if (rc) return rc;
+  if (norm->dim > 512) return MODA_HIP_EUNSUPPORTED;
+  return pack(w, n, gelu_table, norm, stream);
 }
 
 namespace {

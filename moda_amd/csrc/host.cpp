@@ -805,7 +805,11 @@ std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>
         to += w->numel() * es;
       }
     }
-    check_rc(moda_hip_pack_weights(weights.data(), (int32_t)weights.size(), packed_at(blocks.size()), stream), "moda_hip_pack_weights");
+    const Block& b = blocks[0];
+    const moda_hip_norm_rows first = {in_ptr(x0), in_ptr(b.norm1_w), in_ptr(b.norm1_b), out_ptr(h), M, C, (float)b.eps1, dt};
+    check_rc(post_norm ? moda_hip_pack_weights(weights.data(), (int32_t)weights.size(), packed_at(blocks.size()), stream)
+                       : moda_hip_pack_weights_and_norm(weights.data(), (int32_t)weights.size(), packed_at(blocks.size()), &first, stream),
+             "moda_hip_pack_weights");
   }
 
   const void* cur = in_ptr(x0);  // the residual stream
@@ -816,7 +820,7 @@ std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>
     if (!projected) {
       const void* in = cur;
       if (!post_norm) {
-        norm(cur, b.norm1_w, b.norm1_b, b.eps1, h);
+        if (!tails) norm(cur, b.norm1_w, b.norm1_b, b.eps1, h);  // (the first block's, else: with the weights)
         in = in_ptr(h);
       }
       const auto p = projections(b, n);

@@ -674,6 +674,19 @@ def test_block_tail_and_weight_packing_refuse_what_their_kernels_cannot_take():
         assert pack(**bad) == -2, bad
     for bad in (dict(table=0x1008), dict(w=0x2008), dict(packed=0x3008)):
         assert pack(**bad) == -3, bad
+
+    class Norm(ctypes.Structure):
+        _fields_ = [("x", ptr), ("weight", ptr), ("bias", ptr), ("y", ptr), ("rows", i64), ("dim", i64), ("eps", ctypes.c_float), ("dtype", i32)]
+
+    def both(n=1, **given):
+        v = dict(x=0x1000, weight=0x1000, bias=0x1000, y=0x1000, rows=4, dim=256, eps=1e-6, dtype=0)
+        return lib.moda_hip_pack_weights_and_norm((Weight * 1)(Weight(0x2000, 0x3000, 32, 64)), n, ptr(0x1000), ctypes.byref(Norm(**{**v, **given})), None)
+
+    assert lib.moda_hip_pack_weights_and_norm((Weight * 1)(Weight(0x2000, 0x3000, 32, 64)), 1, ptr(0x1000), None, None) == -1
+    for want, bads in ((-1, [dict(n=0), dict(dtype=2), dict(rows=-1), dict(dim=0), *({n: None} for n in ("x", "weight", "bias", "y"))]),
+                       (-2, [dict(dim=100), dict(dim=520), dict(dim=4104), dict(rows=1 << 31)]), (-3, [{n: 0x1008} for n in ("x", "weight", "bias", "y")])):
+        for bad in bads:
+            assert both(**bad) == want, bad
     # what need not be there is not asked for: no parts and no norm behind them, no biases, no table in fp16; here no device
     # either, which is the next thing to be looked at
     fine = (dict(n_parts=0, end_norm_w=None, end_norm_b=None), dict(proj_b=None, fc1_b=None, fc2_b=None, part_bias=None),

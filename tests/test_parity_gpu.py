@@ -2380,6 +2380,45 @@ def test_weights_beyond_one_packing_launch(gpu_device, n):
     assert (table[:_BlockTail.TABLE] != 7.0).all() and (table[_BlockTail.TABLE:] == 7.0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows, dim, n", [(1, 128, 1), (9, 256, 96), (16, 8, 2), (3, 264, 97), (4097, 512, 5), (0, 128, 2)])
+def test_norm_beside_weight_packing(gpu_device, rows, dim, n, dtype):
+    """moda_hip_pack_weights_and_norm against its two parts: the same bits, weights beyond the first launch and rows past the last
+    workgroup's included."""
+    import ctypes
+
+    from moda_amd import _lib
+
+    ptr, i64 = ctypes.c_void_p, ctypes.c_int64
+
+    class Weight(ctypes.Structure):
+        _fields_ = [("w", ptr), ("packed", ptr), ("n", i64), ("k", i64)]
+
+    class Norm(ctypes.Structure):
+        _fields_ = [("x", ptr), ("weight", ptr), ("bias", ptr), ("y", ptr), ("rows", i64), ("dim", i64), ("eps", ctypes.c_float), ("dtype", ctypes.c_int32)]
+
+    lib, stream = _lib.load(), ptr(torch.cuda.current_stream().cuda_stream)
+    say(f"CASE norm beside weight packing {rows} x {dim}, {n} matrices {dtype}")
+    gen = torch.Generator(device=gpu_device).manual_seed(rows + dim)
+    x, w, b = ((torch.randn(*s, generator=gen, device=gpu_device) + 1).to(dtype) for s in ((rows, dim), (dim,), (dim,)))
+    ws = [torch.randn(16 * (1 + i % 3), 32 * (1 + i % 5), generator=gen, device=gpu_device).to(dtype) for i in range(n)]
+    code, got, want = {torch.bfloat16: 0, torch.float16: 1}[dtype], [], []
+    for joined, out in ((True, got), (False, want)):
+        y, packed = torch.full((rows + 1, dim), 7.0, device=gpu_device, dtype=dtype), [torch.full_like(t, 7.0) for t in ws]
+        table = torch.full((_BlockTail.TABLE,), 7.0, device=gpu_device)
+        arr = (Weight * n)(*(Weight(t.data_ptr(), p.data_ptr(), *t.shape) for t, p in zip(ws, packed)))
+        if joined:
+            r = Norm(x.data_ptr(), w.data_ptr(), b.data_ptr(), y.data_ptr(), rows, dim, 1e-6, code)
+            assert lib.moda_hip_pack_weights_and_norm(arr, n, ptr(table.data_ptr()), ctypes.byref(r), stream) == 0
+        else:
+            assert lib.moda_hip_pack_weights(arr, n, ptr(table.data_ptr()), stream) == 0
+            assert lib.moda_hip_layer_norm(code, i64(rows), i64(dim), ptr(x.data_ptr()), ptr(w.data_ptr()), ptr(b.data_ptr()), ctypes.c_float(1e-6),
+                                           ptr(y.data_ptr()), stream) == 0
+        out.extend([y, table, *packed])
+    for a, c in zip(got, want):
+        assert torch.equal(a, c)
+
+
 @pytest.mark.parametrize("case", [
     # width, blocks, batch, tokens, post-norm, dtype: 64 rows a workgroup (more than 8192 rows); more matrices than one packing
     # launch takes (five a block, without the first block's two)
