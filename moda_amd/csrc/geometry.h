@@ -4,6 +4,7 @@
 // every descriptor, load and store of a launch on the CPU and checks them against the tensor extents.
 #pragma once
 #include "kargs.h"
+#include "tuning.h"
 
 #define MODA_HD __host__ __device__ __forceinline__
 
@@ -414,7 +415,7 @@ inline bool dkv_flat_row_waves(const KArgs& a) {
 // whether every streamed (batch, head) slice spans less than 2 GiB
 inline bool narrow_slices(const KArgs& a) {
   const int64_t seq = (int64_t)a.T * (a.sk.t > a.sv.t ? a.sk.t : a.sv.t), dep = (int64_t)a.T * a.L * (a.skd.t > a.svd.t ? a.skd.t : a.svd.t);
-  return 2 * (seq > dep ? seq : dep) <= 0x7fffffffll;
+  return narrow_slice(1, seq > dep ? seq : dep);
 }
 // dQ and sequence dK/dV of the 64-wide tiles in one launch (bwd_short_kernel): row waves, and the workgroups of both run at once,
 // two a compute unit.  A replayed backward pass of 48 random such shapes takes 0.71 - 0.99 of the two launches' time (one of

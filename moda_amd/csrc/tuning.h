@@ -128,17 +128,24 @@ inline bool block_tail_pays(bool fp16, long long rows, long long width, long lon
   return width <= 256 || 4 * last >= (width > 384 && fp16 ? 3 : 2) * compute_units;
 }
 
+// Whether 32-bit byte offsets reach all of a (batch, head) slice: `rows` rows, `stride` 16-bit elements apart.
+inline bool narrow_slice(long long rows, long long stride) { return 2 * rows * stride <= 0x7fffffffll; }
+
 // ... and whether the block's attention joins it (attend_tail_kernel): workgroups of 64 (or 32) tokens of one sequence, which a
 // sequence's last one has few of, as long as they take no more rounds than workgroups of as many rows of all.
+// `slots`: of a token in the depth cache, whose rows are a layer's k and v as well as its depth rows.  Slices that 32-bit offsets do
+// not reach are the forward kernel's alone.
 inline bool attend_tail_takes(long long width, long long heads, long long kv_heads, long long tokens) {
   const long long group = kv_heads > 0 ? heads / kv_heads : 0;
   return (kv_heads == 1 || kv_heads == 2) && heads == group * kv_heads && (group == 2 || group == 4) && width == 64 * heads &&
          tokens * heads <= 256;  // query rows, 32 a wave
 }
-inline bool attention_joins_tail(long long batch, long long tokens, long long width, long long heads, long long kv_heads, int compute_units) {
+inline bool attention_joins_tail(long long batch, long long tokens, long long width, long long heads, long long kv_heads, long long slots,
+                                 int compute_units) {
   const long long rows = batch * tokens, bm = block_tail_rows(rows, compute_units), cus = compute_units;
   const long long tiles = (rows + bm - 1) / bm, with = batch * ((tokens + bm - 1) / bm);
-  return attend_tail_takes(width, heads, kv_heads, bm) && (with + cus - 1) / cus == (tiles + cus - 1) / cus;
+  return attend_tail_takes(width, heads, kv_heads, bm) && narrow_slice(tokens, slots * kv_heads * 64) &&
+         (with + cus - 1) / cus == (tiles + cus - 1) / cus;
 }
 
 }  // namespace moda

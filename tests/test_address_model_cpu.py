@@ -395,6 +395,55 @@ def test_when_a_blocks_attention_joins_its_tail(walker, case):
     assert out.strip() == case[-1]
 
 
+@pytest.mark.parametrize("case", [
+    # tokens, heads, key/value heads, slots: one sequence on either side of 2 GiB a slice (tokens x slots x key/value features)
+    (65536, 4, 2, 128, "apart"),
+    (65535, 4, 2, 128, "joins"),
+    (87382, 4, 2, 96, "apart"),
+    (87381, 4, 2, 96, "joins"),
+    (349526, 4, 2, 24, "apart"),
+    (174763, 2, 1, 96, "apart"),
+    (174762, 2, 1, 96, "joins"),
+    (16777216, 4, 1, 1, "apart"),
+], ids=lambda c: "-".join(map(str, c[:4])))
+def test_a_blocks_attention_joins_only_what_the_joined_launch_takes(walker, case):
+    """Chunk-visible stacks of one long sequence, whose workgroups all cost the same.  Slices of 2 GiB and more go apart: the joined call
+    refuses them, the forward call takes them, as far as can be seen without a device."""
+    import ctypes
+
+    import torch
+
+    from moda_amd import _lib
+
+    tokens, heads, kv_heads, slots, want = case
+    width, kv = 64 * heads, 64 * kv_heads
+    out = subprocess.run([walker, "attend_tail_rule", "1", *map(str, (tokens, width, heads, kv_heads, 256, slots))], stdout=subprocess.PIPE, text=True, check=True).stdout
+    assert out.strip() == want
+    if torch.cuda.is_available():
+        return  # made-up addresses
+
+    i32, i64, f32, ptr = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p
+    named = ("attention", "residual", "x", "proj_w", "proj_b", "fc1_w", "fc1_b", "fc2_w", "fc2_b", "mid_norm_w", "mid_norm_b", "end_norm_w", "end_norm_b", "gelu_table")
+
+    class Tail(ctypes.Structure):  # moda_hip_block_tail_args, without parts
+        _fields_ = [("struct_size", i32), ("dtype", i32), ("rows", i64), ("width", i64), ("hidden", i64), *((n, ptr) for n in named),
+                    ("mid_norm_eps", f32), ("end_norm_eps", f32), ("post_norm", i32), ("n_parts", i32), ("parts", i64 * 15)]
+
+    t = Tail(struct_size=ctypes.sizeof(Tail), rows=tokens, width=width, hidden=4 * width, **{n: 0x1000 for n in named})
+    d = _lib.Desc()
+    d.struct_size, d.mode, d.chunk_tokens, d.scale = ctypes.sizeof(d), _lib.CHUNK_VISIBLE, 16, 0.125
+    d.B, d.T, d.H, d.G, d.D, d.Dv = 1, tokens, kv_heads, heads // kv_heads, 64, 64
+    d.q = d.o = _lib.Strides(tokens * width, kv, 64)
+    d.k = d.v = _lib.Strides(tokens * slots * kv, slots * kv, 64)
+    d.kd = d.vd = _lib.Strides(tokens * slots * kv, kv, 64)
+    p, lib, refused, no_device = ptr(0x1000), _lib.load(), -2, -6
+    for filled in {0, 1, slots // 2}:  # a stack's first block, and later ones
+        d.L, d.L_valid = (slots, filled) if filled else (0, 0)
+        assert lib.moda_hip_fwd(ctypes.byref(d), p, p, p, p, p, p, p, None) == no_device
+        got = lib.moda_hip_attend_block_tail(ctypes.byref(d), p, p, p, p, p, ctypes.byref(t), None)
+        assert got == (no_device if want == "joins" else refused), filled
+
+
 def test_packed_weights(walker):
     out = subprocess.run([walker, "pack", "7"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=600)
     assert out.returncode == 0 and "OK checked" in out.stdout, out.stdout
