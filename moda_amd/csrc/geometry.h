@@ -166,12 +166,14 @@ MODA_HD RowPlace row_place(const KArgs& grid, int block, int BM) {
 }
 
 // Which tokens a workgroup of attend_tail_kernel takes: tile `tile` (of `tokens` each) of sequence b, rows [first_row, rows_end) of
-// the [B * T] rows; a sequence's tiles are B workgroups apart, on one XCD (one L2) if B is a multiple of eight.
+// the [B * T] rows; a sequence's tiles are B workgroups apart, on one XCD (one L2) if B is a multiple of eight.  Causal: the late, heavy
+// tiles first, as in query_tile_of.  Six blocks of width 256 on causal sequences, us with the light ones first and so: 4 x 8192 tokens
+// (two rounds) 1654 and 1360, 1 x 65 536 (four) 20 440 and 15 290, 64 x 512 (two) 517 and 505; one round 1864 and 1854 (1 x 16 384).
 struct AttendTailPlace {
   int b, tile, first_row, rows_end;
 };
 MODA_HD AttendTailPlace attend_tail_place(const KArgs& a, int block, int tokens) {
-  const int tile = block / a.B, b = block % a.B;
+  const int nth = block / a.B, b = block % a.B, tile = a.causal ? (a.T + tokens - 1) / tokens - 1 - nth : nth;
   return {b, tile, b * a.T + tile * tokens, (b + 1) * a.T};
 }
 inline int64_t attend_tail_blocks(const KArgs& a, int tokens) { return (int64_t)a.B * ((a.T + tokens - 1) / tokens); }

@@ -1566,6 +1566,19 @@ int main(int argc, char** argv) {
     printf("%s\n", attention_joins_tail(arg(2), arg(3), arg(4), arg(5), arg(6), argc > 8 ? arg(8) : 12, arg(7)) ? "joins" : "apart");
     return 0;
   }
+  if (what == "attend_tail_order") {  // sequences tokens tokens_of_a_workgroup causal: sequence and tile of every workgroup
+    KArgs a = {};
+    a.B = arg(2);
+    a.T = arg(3);
+    a.causal = arg(5);
+    for (int block = 0; block < attend_tail_blocks(a, arg(4)); block++) {
+      const AttendTailPlace p = attend_tail_place(a, block, arg(4));
+      if (p.first_row != p.b * a.T + p.tile * arg(4) || p.rows_end != (p.b + 1) * a.T) fail("rows of workgroup %d", block);
+      printf("%d:%d ", p.b, p.tile);
+    }
+    printf("\n");
+    return 0;
+  }
   if (what == "slots") {  // the slot arithmetic of partially filled streams against the division it stands for
     for (int Lv : {1, 2, 3, 5, 7, 11, 12, 24, 31, 33, 63, 64, 65, 72, 127, 1000, 65537, (1 << 24) + 3, (1 << 30) + 1})
       for (int l0 : {0, 1, Lv / 2, Lv - 2, Lv - 1})

@@ -395,6 +395,17 @@ def test_when_a_blocks_attention_joins_its_tail(walker, case):
     assert out.strip() == case[-1]
 
 
+@pytest.mark.parametrize("sequences, tokens, of_a_workgroup", [(1, 1, 32), (3, 64, 32), (8, 197, 64), (1, 8257, 64), (5, 33, 32)])
+def test_order_of_the_joined_launch(walker, sequences, tokens, of_a_workgroup):
+    """Every tile of every sequence once; where they differ in cost (causal), those with the most keys first."""
+    tiles = -(-tokens // of_a_workgroup)
+    for causal in (0, 1):
+        out = subprocess.run([walker, "attend_tail_order", *map(str, (sequences, tokens, of_a_workgroup, causal))], stdout=subprocess.PIPE, text=True, check=True).stdout
+        places = [tuple(map(int, p.split(":"))) for p in out.split()]
+        assert sorted(places) == [(b, t) for b in range(sequences) for t in range(tiles)]
+        assert [t for _, t in places] == sorted((t for _, t in places), reverse=bool(causal))
+
+
 @pytest.mark.parametrize("case", [
     # tokens, heads, key/value heads, slots: one sequence on either side of 2 GiB a slice (tokens x slots x key/value features)
     (65536, 4, 2, 128, "apart"),
