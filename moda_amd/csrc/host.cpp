@@ -709,10 +709,10 @@ bool tail_is_one_launch(bool fp16, int64_t rows, int64_t width, int64_t hidden, 
          moda::block_tail_pays(fp16, rows, width, hidden, kv, compute_units);
 }
 
-bool attention_joins(const Tensor& x, int64_t heads, int64_t kv_heads, int64_t slots) {
+bool attention_joins(const Tensor& x, int64_t heads, int64_t kv_heads, int64_t slots, bool causal) {
   int compute_units = 0;
   return hipDeviceGetAttribute(&compute_units, hipDeviceAttributeMultiprocessorCount, x.get_device()) == hipSuccess && compute_units > 0 &&
-         moda::attention_joins_tail(x.size(0), x.size(1), x.size(2), heads, kv_heads, slots, compute_units);
+         moda::attention_joins_tail(x.size(0), x.size(1), x.size(2), heads, kv_heads, slots, causal, compute_units);
 }
 
 // Forward pass of all blocks of one stack, launches only: the residual stream, one depth cache and four work tensors
@@ -753,7 +753,7 @@ std::optional<Tensor> stack_forward(const Tensor& x_in, const std::vector<Block>
   const bool tails = tail_is_one_launch(type == at::kHalf, M, C, hidden, kv, x_in.get_device());
   // Attention and tail as one launch.  (Of chunks of more than 64 query rows the depth columns are summed from where a workgroup's own
   // begin: those keep the forward kernel's workgroups, and with them the bits.)
-  const bool joined = tails && chunk_tokens * (heads / kv_heads) <= 64 && attention_joins(x_in, heads, kv_heads, L);
+  const bool joined = tails && chunk_tokens * (heads / kv_heads) <= 64 && attention_joins(x_in, heads, kv_heads, L, is_causal || chunk_tokens > 0);
   Tensor x = at::empty({B, N, C}, opt), h = at::empty({M, C}, opt), q = at::empty({M, C}, opt), x1 = tails ? Tensor() : at::empty({M, C}, opt),
          hid = tails ? Tensor() : at::empty({M, hidden}, opt), ck = at::empty({B, N * L, kv}, opt), cv = at::empty({B, N * L, kv}, opt),
          lse = joined ? Tensor() : at::empty({M * heads}, opt.dtype(at::kFloat));

@@ -135,17 +135,48 @@ inline bool narrow_slice(long long rows, long long stride) { return 2 * rows * s
 // sequence's last one has few of, as long as they take no more rounds than workgroups of as many rows of all.
 // `slots`: of a token in the depth cache, whose rows are a layer's k and v as well as its depth rows.  Slices that 32-bit offsets do
 // not reach are the forward kernel's alone.
+// The joined launch saves a block 3.5 us of starts and ends (causal: 4.5, and 7 where 32 tokens a workgroup leave the light ones time to
+// take in weights), and the attention takes as long or longer in it, which grows with the sequence.  Of 64 keys, a SIMD takes 0.73 us for
+// one wave's 32 rows, 1.16 for those of two waves, 1.62 of three.  The joined launch has one workgroup a compute unit, so one
+// working wave a SIMD, or two (four query heads and 64 tokens; two key/value heads, whose halves' working waves share SIMDs), round
+// after round; the forward launch up to three.  Causal, a round of the one lasts as long as its longest row, while the other's
+// workgroups, all there at once, make room for each other.  Over several rounds less is saved: the dense launch by itself overlaps a
+// round's end with the next one's start (width 128 most of all).
+// Measured: stacks of two, six and twelve blocks, both ways in turn, 20 - 65 536 tokens, one to eight rounds, causal and not, both types,
+// MLPs of two to eight times the width, the heads that the kernel takes.  The rule was fitted to 1595 of them that take as many rounds
+// either way; 1585 go the faster way or one within 3 % of it, and 1381 of 1398 random ones drawn afterwards, the others within 7 %, one
+// 11 % behind.  Of the 1595, always joined, 373 would lose more than 3 %, up to 31 %, and always apart 805, up to 30 %.  us of six
+// blocks apart and joined, one key/value head: four query heads, 64 x 197 tokens 281 and 256; causal, 1 x 16 384 1475 and 1854, 2 x 8192
+// 869 and 1042, 2 x 4096 478 and 429; two query heads, 4 x 16 384 3836 and 4950, 1 x 16 384 1284 and 1256; two key/value heads of two,
+// 1 x 4096 472 and 590, 4 x 4096 716 and 703.
 inline bool attend_tail_takes(long long width, long long heads, long long kv_heads, long long tokens) {
   const long long group = kv_heads > 0 ? heads / kv_heads : 0;
   return (kv_heads == 1 || kv_heads == 2) && heads == group * kv_heads && (group == 2 || group == 4) && width == 64 * heads &&
          tokens * heads <= 256;  // query rows, 32 a wave
 }
 inline bool attention_joins_tail(long long batch, long long tokens, long long width, long long heads, long long kv_heads, long long slots,
-                                 int compute_units) {
+                                 bool causal, int compute_units) {
   const long long rows = batch * tokens, bm = block_tail_rows(rows, compute_units), cus = compute_units;
-  const long long tiles = (rows + bm - 1) / bm, with = batch * ((tokens + bm - 1) / bm);
-  return attend_tail_takes(width, heads, kv_heads, bm) && narrow_slice(tokens, slots * kv_heads * 64) &&
-         (with + cus - 1) / cus == (tiles + cus - 1) / cus;
+  const long long tiles = (rows + bm - 1) / bm, with = batch * ((tokens + bm - 1) / bm), rounds = (with + cus - 1) / cus;
+  if (!attend_tail_takes(width, heads, kv_heads, bm) || !narrow_slice(tokens, slots * kv_heads * 64) || rounds != (tiles + cus - 1) / cus) return false;
+  constexpr double one = 0.73, two = 1.16, three = 1.62;
+  const double keys = (double)((tokens + 63) / 64);  // tiles of the longest row
+  const bool pairs = kv_heads == 2 || bm * heads > 128;  // waves at work two a SIMD
+  const double joined = (pairs ? two : one) * (!causal ? (double)rounds : with > 2 * cus ? 0.5 * with / cus : 1);
+  // the forward launch's workgroups, 128 rows each, a compute unit; up to three are there at once
+  const double n = (double)(batch * kv_heads * ((tokens * (heads / kv_heads) + 127) / 128)) / cus;
+  double apart;
+  if (n > 3) {
+    apart = three / 3 * n * (causal ? 0.5 : 1);
+  } else if (causal) {  // those of the unit that has the longest row: the second and third have so much of it
+    const double second = n > 1 ? 1 - 1 / n : 0, third = n > 2 ? 1 - 2 / n : 0;
+    apart = third * three + (second - third) * two + (1 - second) * one;
+  } else {
+    apart = n <= 1 ? one : n <= 2 ? two : three;
+  }
+  if (rounds > 2 && !pairs) return false;
+  const double saved = rounds == 1 ? (!causal ? 3.5 : bm == 32 ? 7 : 4.5) : !pairs ? 1.3 : causal ? 4 : kv_heads == 1 ? 3.5 : 2;
+  return (joined - apart) * keys <= saved + 1e-6;
 }
 
 }  // namespace moda

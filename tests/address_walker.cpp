@@ -1562,8 +1562,8 @@ int main(int argc, char** argv) {
     printf("OK checked=%lld\n", g_checked);
     return 0;
   }
-  if (what == "attend_tail_rule") {  // sequences tokens width heads kv_heads compute_units [slots]
-    printf("%s\n", attention_joins_tail(arg(2), arg(3), arg(4), arg(5), arg(6), argc > 8 ? arg(8) : 12, arg(7)) ? "joins" : "apart");
+  if (what == "attend_tail_rule") {  // sequences tokens width heads kv_heads compute_units [slots [causal]]
+    printf("%s\n", attention_joins_tail(arg(2), arg(3), arg(4), arg(5), arg(6), argc > 8 ? arg(8) : 12, arg(9) != 0, arg(7)) ? "joins" : "apart");
     return 0;
   }
   if (what == "attend_tail_order") {  // sequences tokens tokens_of_a_workgroup causal: sequence and tile of every workgroup

@@ -395,6 +395,39 @@ def test_when_a_blocks_attention_joins_its_tail(walker, case):
     assert out.strip() == case[-1]
 
 
+@pytest.mark.parametrize("case", [
+    # sequences, tokens, heads, key/value heads, causal; us of six blocks apart / joined on 256 compute units
+    (1, 16384, 2, 1, False, "joins"),  # 1284 / 1256: one round of one wave a SIMD, as apart
+    (16, 1024, 2, 1, True, "joins"),   # 235 / 200
+    (1, 16384, 2, 1, True, "joins"),   # 1275 / 1239
+    (64, 512, 2, 1, False, "apart"),   # 303 / 313: two rounds of one wave, apart one of two
+    (96, 197, 2, 1, False, "joins"),   # 270 / 259
+    (4, 6144, 2, 1, True, "joins"),    # 666 / 550: apart the unit with the longest row has two more
+    (4, 16384, 2, 1, False, "apart"),  # 3836 / 4959
+    (1, 65536, 2, 1, True, "apart"),   # 7509 / 9688
+    (192, 256, 2, 1, True, "apart"),   # 369 / 395: three rounds
+    (1, 16384, 4, 1, False, "joins"),  # 2022 / 1991: one round of two waves, as apart
+    (32, 512, 4, 1, True, "joins"),    # 303 / 286
+    (8, 2048, 4, 1, True, "apart"),    # 416 / 434: ends with its longest row, where apart the others make room
+    (1, 16384, 4, 1, True, "apart"),   # 1475 / 1854
+    (1, 8192, 4, 1, True, "joins"),    # 755 / 703: 32 tokens, one wave
+    (64, 512, 4, 1, False, "joins"),   # 578 / 556
+    (4, 8192, 4, 1, False, "apart"),   # 2147 / 2172
+    (32, 1024, 4, 1, True, "joins"),   # 589 / 554
+    (1, 65536, 4, 1, True, "apart"),   # 13 993 / 15 286
+    (8, 512, 4, 2, True, "joins"),     # 231 / 218: 32 tokens, the halves' waves on the same SIMDs
+    (2, 2048, 4, 2, False, "apart"),   # 331 / 382
+    (4, 4096, 4, 2, False, "joins"),   # 716 / 703
+    (4, 4096, 4, 2, True, "apart"),    # 579 / 656
+    (8, 1024, 8, 2, True, "joins"),    # 563 / 506
+    (1, 8192, 8, 2, True, "apart"),    # 1090 / 1235
+], ids=lambda c: "-".join(map(str, c[:5])))
+def test_what_length_mask_and_heads_say_of_joining(walker, case):
+    sequences, tokens, heads, kv_heads, causal, want = case
+    out = subprocess.run([walker, "attend_tail_rule", *map(str, (sequences, tokens, 64 * heads, heads, kv_heads, 256, 6, int(causal)))], stdout=subprocess.PIPE, text=True, check=True).stdout
+    assert out.strip() == want
+
+
 @pytest.mark.parametrize("sequences, tokens, of_a_workgroup", [(1, 1, 32), (3, 64, 32), (8, 197, 64), (1, 8257, 64), (5, 33, 32)])
 def test_order_of_the_joined_launch(walker, sequences, tokens, of_a_workgroup):
     """Every tile of every sequence once; where they differ in cost (causal), those with the most keys first."""
@@ -408,17 +441,18 @@ def test_order_of_the_joined_launch(walker, sequences, tokens, of_a_workgroup):
 
 @pytest.mark.parametrize("case", [
     # tokens, heads, key/value heads, slots: one sequence on either side of 2 GiB a slice (tokens x slots x key/value features)
+    (16384, 2, 1, 1024, "apart"),
+    (16384, 2, 1, 1023, "joins"),
+    (8192, 4, 1, 2048, "apart"),
+    (8192, 4, 1, 2047, "joins"),
+    (8192, 8, 2, 1024, "apart"),
     (65536, 4, 2, 128, "apart"),
-    (65535, 4, 2, 128, "joins"),
     (87382, 4, 2, 96, "apart"),
-    (87381, 4, 2, 96, "joins"),
     (349526, 4, 2, 24, "apart"),
-    (174763, 2, 1, 96, "apart"),
-    (174762, 2, 1, 96, "joins"),
     (16777216, 4, 1, 1, "apart"),
 ], ids=lambda c: "-".join(map(str, c[:4])))
 def test_a_blocks_attention_joins_only_what_the_joined_launch_takes(walker, case):
-    """Chunk-visible stacks of one long sequence, whose workgroups all cost the same.  Slices of 2 GiB and more go apart: the joined call
+    """Chunk-visible stacks of one sequence, as long as attention could join or longer.  Slices of 2 GiB and more go apart: the joined call
     refuses them, the forward call takes them, as far as can be seen without a device."""
     import ctypes
 
