@@ -310,8 +310,8 @@ typedef struct moda_hip_weight {
   int64_t n, k;
 } moda_hip_weight;
 int moda_hip_pack_weights(const moda_hip_weight* weights, int32_t n, void* gelu_table, void* stream);
-/* The same, and in its first launch what moda_hip_layer_norm(dtype, rows, dim, x, weight, bias, eps, y) does, bit for bit, for dim up to
- * 512: a stack packs its weights while its input is normalised.  None of the packed copies may be an input of the norm, nor y a weight. */
+/* The same, and in its first launch (or, where a grid does not hold both, one of its own) what moda_hip_layer_norm(dtype, rows, dim, x,
+ * weight, bias, eps, y) does, bit for bit, for dim up to 512: a stack packs its weights while its input is normalised.  None of the packed copies may be an input of the norm, nor y a weight. */
 typedef struct moda_hip_norm_rows {
   const void *x, *weight, *bias;
   void* y;

@@ -109,6 +109,9 @@ hipError_t launch_tail(const TailArgs& a, int width, bool post, int cus, hipStre
 
 }  // namespace
 
+hipError_t launch_layer_norm(int dtype, int64_t rows, int64_t dim, const void* x, const void* weight, const void* bias, float eps, void* y,
+                             hipStream_t stream);  // block_kernels.hip
+
 hipError_t launch_pack_weights(const moda_hip_weight* w, int n, float* gelu_table, const moda_hip_norm_rows* norm, hipStream_t stream) {
   for (int first = 0; first < n; first += kPackMatrices) {
     PackArgs a = {};
@@ -123,12 +126,15 @@ hipError_t launch_pack_weights(const moda_hip_weight* w, int n, float* gelu_tabl
     a.n = count;
     a.gelu_table = first == 0 ? gelu_table : nullptr;
     const unsigned pack_blocks = (unsigned)((most + 3) / 4), parts = count + (a.gelu_table ? 1 : 0);
+    bool joint = false;
     if (first == 0 && norm && norm->rows > 0) {
       const auto go = [&](auto type, auto lanes) {
         constexpr int LPR = decltype(lanes)::value, RPB = 256 / LPR;
         const NormArgs r = {(const uint16_t*)norm->x, (const uint16_t*)norm->weight, (const uint16_t*)norm->bias, (uint16_t*)norm->y, norm->eps,
                             (int)norm->rows, (int)norm->dim, (int)((norm->rows + RPB - 1) / RPB)};
-        hipLaunchKernelGGL((pack_and_norm_kernel<decltype(type), LPR>), dim3((unsigned)r.blocks + pack_blocks * parts), dim3(256), 0, stream, a, r, (int)pack_blocks);
+        const int64_t nblk = pack_and_norm_blocks(norm->rows, RPB, pack_blocks, parts);
+        if ((joint = nblk > 0))
+          hipLaunchKernelGGL((pack_and_norm_kernel<decltype(type), LPR>), dim3((unsigned)nblk), dim3(256), 0, stream, a, r, (int)pack_blocks);
       };
       const auto by_width = [&](auto type) {  // as launch_layer_norm
         if (norm->dim <= 128) return go(type, std::integral_constant<int, 16>{});
@@ -136,9 +142,12 @@ hipError_t launch_pack_weights(const moda_hip_weight* w, int n, float* gelu_tabl
         return go(type, std::integral_constant<int, 64>{});
       };
       norm->dtype == 0 ? by_width(BF16{}) : by_width(FP16{});
-    } else {
-      hipLaunchKernelGGL(pack_weights_kernel, dim3(pack_blocks, parts), dim3(256), 0, stream, a);
+      if (!joint) {
+        const hipError_t en = launch_layer_norm(norm->dtype, norm->rows, norm->dim, norm->x, norm->weight, norm->bias, norm->eps, norm->y, stream);
+        if (en != hipSuccess) return en;
+      }
     }
+    if (!joint) hipLaunchKernelGGL(pack_weights_kernel, dim3(pack_blocks, parts), dim3(256), 0, stream, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

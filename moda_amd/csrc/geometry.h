@@ -178,6 +178,13 @@ MODA_HD AttendTailPlace attend_tail_place(const KArgs& a, int block, int tokens)
 }
 inline int64_t attend_tail_blocks(const KArgs& a, int tokens) { return (int64_t)a.B * ((a.T + tokens - 1) / tokens); }
 
+// Workgroups of the launch that packs weights (`packing` for each of `parts`) and normalises rows (pack_and_norm_kernel), or 0 where the
+// 2^32 threads of a grid's one dimension do not hold both: two launches then, as large as each may be by itself.
+inline int64_t pack_and_norm_blocks(int64_t rows, int rows_per_block, int64_t packing, int64_t parts) {
+  const int64_t n = (rows + rows_per_block - 1) / rows_per_block + packing * parts;
+  return n * 256 < (1ll << 32) ? n : 0;
+}
+
 // Visible column intervals [0, shi) of the sequence keys and [dlo, dhi) of the depth columns (compact axis) for
 // query row r (all zero for a row past the end).  Ld: depth slots per token, 0 when the launch has no depth stream.
 struct RowVis {

@@ -1566,6 +1566,10 @@ int main(int argc, char** argv) {
     printf("%s\n", attention_joins_tail(arg(2), arg(3), arg(4), arg(5), arg(6), argc > 8 ? arg(8) : 12, arg(9) != 0, arg(7)) ? "joins" : "apart");
     return 0;
   }
+  if (what == "pack_and_norm") {  // rows rows_of_a_workgroup packing_workgroups parts
+    printf("%lld\n", (long long)pack_and_norm_blocks(atoll(argv[2]), arg(3), atoll(argv[4]), arg(5)));
+    return 0;
+  }
   if (what == "attend_tail_order") {  // sequences tokens tokens_of_a_workgroup causal: sequence and tile of every workgroup
     KArgs a = {};
     a.B = arg(2);

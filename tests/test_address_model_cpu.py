@@ -489,6 +489,22 @@ def test_a_blocks_attention_joins_only_what_the_joined_launch_takes(walker, case
         assert got == (no_device if want == "joins" else refused), filled
 
 
+@pytest.mark.parametrize("case", [
+    # rows, rows a workgroup, packing workgroups of the widest matrix, matrices (and the table); workgroups of one launch, 0: two
+    (12608, 8, 128, 61, 1576 + 128 * 61),
+    (1, 16, 1, 2, 3),
+    ((1 << 26) - 4 * 97, 4, 1, 96, (1 << 24) - 1),
+    ((1 << 26) - 4 * 97 + 1, 4, 1, 97, 0),
+    (4, 4, 1 << 18, 64, 0),  # 64 matrices of 2^29 elements
+    (4, 4, 1 << 20, 97, 0),  # (as many as a launch takes, the largest there are)
+    ((1 << 30) - 1, 4, 1 << 20, 97, 0),
+], ids=str)
+def test_weights_and_norm_in_one_grid(walker, case):
+    """A dimension of a grid ends below 2^32 threads, which 256 a workgroup reach at 2^24."""
+    out = subprocess.run([walker, "pack_and_norm", *map(str, case[:4])], stdout=subprocess.PIPE, text=True, check=True).stdout
+    assert int(out) == case[4]
+
+
 def test_packed_weights(walker):
     out = subprocess.run([walker, "pack", "7"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=600)
     assert out.returncode == 0 and "OK checked" in out.stdout, out.stdout

@@ -2419,6 +2419,44 @@ def test_norm_beside_weight_packing(gpu_device, rows, dim, n, dtype):
         assert torch.equal(a, c)
 
 
+def test_norm_and_weight_packing_beyond_one_grid(gpu_device):
+    """Rows and pieces of weights that a grid of 2^32 threads does not hold together: two launches, the bits of the two calls."""
+    import ctypes
+
+    from moda_amd import _lib
+
+    ptr, i64 = ctypes.c_void_p, ctypes.c_int64
+
+    class Weight(ctypes.Structure):
+        _fields_ = [("w", ptr), ("packed", ptr), ("n", i64), ("k", i64)]
+
+    class Norm(ctypes.Structure):
+        _fields_ = [("x", ptr), ("weight", ptr), ("bias", ptr), ("y", ptr), ("rows", i64), ("dim", i64), ("eps", ctypes.c_float), ("dtype", ctypes.c_int32)]
+
+    lib, stream = _lib.load(), ptr(torch.cuda.current_stream().cuda_stream)
+    rows, dim = (1 << 28) - 32, 8  # sixteen rows a workgroup: two fewer than a grid has, and three that pack
+    say(f"CASE norm and weight packing {rows} x {dim}")
+    gen = torch.Generator(device=gpu_device).manual_seed(0)
+    some = torch.randn(1 << 16, dim, generator=gen, device=gpu_device).to(torch.bfloat16)
+    x = some.repeat(1 << 12, 1)[:rows]
+    w, b = (torch.randn(dim, generator=gen, device=gpu_device).to(torch.bfloat16) for _ in range(2))
+    ws = [torch.randn(16, 32, generator=gen, device=gpu_device).to(torch.bfloat16) for _ in range(2)]
+    packed, want_packed = ([torch.full_like(t, 7.0) for t in ws] for _ in range(2))
+    table, want_table = (torch.full((_BlockTail.TABLE,), 7.0, device=gpu_device) for _ in range(2))
+    y, want = torch.full((rows + 1, dim), 7.0, device=gpu_device, dtype=torch.bfloat16), torch.empty_like(some)
+    pieces = lambda to: (Weight * 2)(*(Weight(t.data_ptr(), p.data_ptr(), *t.shape) for t, p in zip(ws, to)))
+    norm = Norm(x.data_ptr(), w.data_ptr(), b.data_ptr(), y.data_ptr(), rows, dim, 1e-6, 0)
+    assert lib.moda_hip_pack_weights_and_norm(pieces(packed), 2, ptr(table.data_ptr()), ctypes.byref(norm), stream) == 0
+    assert lib.moda_hip_pack_weights(pieces(want_packed), 2, ptr(want_table.data_ptr()), stream) == 0
+    assert lib.moda_hip_layer_norm(0, i64(1 << 16), i64(dim), ptr(some.data_ptr()), ptr(w.data_ptr()), ptr(b.data_ptr()), ctypes.c_float(1e-6),
+                                   ptr(want.data_ptr()), stream) == 0
+    assert all(torch.equal(p, q) for p, q in zip(packed, want_packed)) and torch.equal(table, want_table)
+    assert (y[rows] == 7.0).all()
+    for first in range(0, rows, 1 << 24):
+        got = y[first:min(rows, first + (1 << 24))]
+        assert torch.equal(got, want.repeat(1 << 8, 1)[:len(got)])
+
+
 @pytest.mark.parametrize("case", [
     # width, blocks, batch, tokens, post-norm, dtype: 64 rows a workgroup (more than 8192 rows); more matrices than one packing
     # launch takes (five a block, without the first block's two)
