@@ -180,13 +180,6 @@ struct Product {
 
 }  // namespace
 
-// Elements of the LDS that the ring of a block's attention and then the hidden activations have (see attend_tail_kernel)
-template <typename Shape, int BM>
-constexpr int attend_ring() {
-  constexpr int rings = 8 / Shape::W * Shape::NST * 2 * 64 * 64;
-  return rings > BM * 2 * 256 ? rings : BM * 2 * 256;
-}
-
 // The same body with the block's attention before it (MODA_SIDE_BY_SIDE, attend_tail_kernel.hip): the workgroup forms the rows of H
 // itself, from the arguments `att` of the forward kernel (fwd.h).  Its rows are then BM tokens of one sequence.
 #ifdef MODA_SIDE_BY_SIDE

@@ -51,6 +51,12 @@ struct RowBlock {
   static constexpr bool PP = false, APART = true;
   static_assert(WORK >= 1 && WORK <= W, "the query rows of the workgroup's tokens over its waves");
 };
+// Elements of the LDS that the ring of a block's attention and then the hidden activations have (see attend_tail_kernel)
+template <typename Shape, int BM>
+constexpr int attend_ring() {
+  constexpr int rings = 8 / Shape::W * Shape::NST * 2 * 64 * 64;
+  return rings > BM * 2 * 256 ? rings : BM * 2 * 256;
+}
 
 // Head dims above 128 (tile width 256, 16x16x32 kernels only): 16 query rows per wave, so that the wave's Q (and
 // dO) operands and its 256-wide accumulator still fit the register file; two ring stages of 64 KB.

@@ -26,6 +26,7 @@
 //   the order of a packed batch's launches, WALKER_ROUTE=1 whether a backward pass is one launch.
 // usage: address_walker linear rows K gelu n0 [n1 n2]   |   norm rows dim   |   slot B T H D L slot wide to_cache
 //   |   tail bf16|fp16 rows width hidden post_norm [n0 [n1 [n2]]]   |   pack matrices
+//   |   attention bf16|fp16 sequences tokens heads group slots filled mode chunk_tokens
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -238,6 +239,70 @@ void ctx(const char* kernel, int block, int wave, int lane, const char* what) {
   g_where = {kernel, block, wave, lane, what};
 }
 
+// One tile of the workgroup's ring, this lane's loads: sequence rows (of the tensors `k_name`, `v_name`) or depth columns from row0 on
+template <int HD, int NT, bool WIDE_ADDR>
+void ring_tile_loads(const KArgs& a, int b, int hkv, const AsyncTileLoader<HD, 64, NT>& ld, const typename AsyncTileLoader<HD, 64, NT>::Source& srcK,
+                     const typename AsyncTileLoader<HD, 64, NT>::Source& srcV, int row0, bool dep, bool mapped, uint32_t kt, uint32_t lds_bytes,
+                     const char* k_name, const char* v_name) {
+  typedef AsyncTileLoader<HD, 64, NT> Loader;
+  constexpr int BN = 64;
+  for (int i = 0; i < Loader::N; i++) {
+    const uint32_t ldsK = kt + (uint32_t)ld.lds_elems(i) * 2, ldsV = ldsK + BN * HD * 2;
+    if (dep && mapped) {  // partially filled stream: one descriptor anchored at the first column's token
+      const int w0 = row0 / a.Lv, l0 = row0 - w0 * a.Lv;
+      const int64_t anchor = (int64_t)w0 * a.L, rows_total = (int64_t)a.T * a.L;
+      check_dma("kd", a.kd + b * a.skd.b + hkv * a.skd.h + anchor * a.skd.t,
+                mapped_bytes(anchor, rows_total, (uint32_t)a.skd.t * 2u),
+                ld.mapped_offset(i, l0, a.L, a.Lv, (int)a.skd.t * 2, a.D), 0, 16, ldsK, lds_bytes, ld.pads(a.D));
+      check_dma("vd", a.vd + b * a.svd.b + hkv * a.svd.h + anchor * a.svd.t,
+                mapped_bytes(anchor, rows_total, (uint32_t)a.svd.t * 2u),
+                ld.mapped_offset(i, l0, a.L, a.Lv, (int)a.svd.t * 2, a.Dv), 0, 16, ldsV, lds_bytes, ld.pads(a.Dv));
+      // a lane in range must have fetched a slot that holds data
+      const int rel = mapped_row(l0, Loader::rows_before(i) + ld.row_in_pass, a.L, a.Lv);
+      if ((anchor + rel) % a.L >= a.Lv) fail("mapped depth tile reads slot %d of %d filled", (int)((anchor + rel) % a.L), a.Lv);
+    } else if (WIDE_ADDR) {
+      const int row_end = dep ? a.T * a.L : a.T;
+      const uint16_t* kb = dep ? a.kd + b * a.skd.b + hkv * a.skd.h : a.k + b * a.sk.b + hkv * a.sk.h;
+      const uint16_t* vb = dep ? a.vd + b * a.svd.b + hkv * a.svd.h : a.v + b * a.sv.b + hkv * a.sv.h;
+      const int64_t ks = dep ? a.skd.t : a.sk.t, vs = dep ? a.svd.t : a.sv.t;
+      check_dma(dep ? "kd" : k_name, kb + (int64_t)row0 * ks, Loader::anchored_bytes(ks, row0, row_end),
+                ld.lane_offset((int)ks * 2, a.D), Loader::rows_before(i) * (int)ks * 2, 16, ldsK, lds_bytes, ld.pads(a.D));
+      check_dma(dep ? "vd" : v_name, vb + (int64_t)row0 * vs, Loader::anchored_bytes(vs, row0, row_end),
+                ld.lane_offset((int)vs * 2, a.Dv), Loader::rows_before(i) * (int)vs * 2, 16, ldsV, lds_bytes, ld.pads(a.Dv));
+    } else {
+      check_dma(dep ? "kd" : k_name, srcK.base, srcK.nbytes, srcK.voff, Loader::source_soffset(srcK, row0, i), 16, ldsK,
+                lds_bytes, ld.pads(a.D));
+      check_dma(dep ? "vd" : v_name, srcV.base, srcV.nbytes, srcV.voff, Loader::source_soffset(srcV, row0, i), 16, ldsV,
+                lds_bytes, ld.pads(a.Dv));
+    }
+  }
+}
+// Load i of a wave's own K and V tile of depth columns [col0, col0 + nrows)
+template <int HD>
+void own_tile_load(const KArgs& a, int b, int hkv, const WaveTileLoader<HD>& own, int i, int col0, int nrows, bool mapped, uint32_t kt, uint32_t vt,
+                   uint32_t lds_bytes) {
+  if (mapped) {
+    const int w0 = col0 / a.Lv, l0 = col0 - w0 * a.Lv;
+    const int64_t anchor = (int64_t)w0 * a.L, rows_total = (int64_t)a.T * a.L;
+    const int vk = own.mapped_offset(i, l0, a.L, a.Lv, nrows, (int)a.skd.t * 2, a.D);
+    const int vv = own.mapped_offset(i, l0, a.L, a.Lv, nrows, (int)a.svd.t * 2, a.Dv);
+    check_dma("kd", a.kd + b * a.skd.b + hkv * a.skd.h + anchor * a.skd.t,
+              nrows > 0 ? mapped_bytes(anchor, rows_total, (uint32_t)a.skd.t * 2u) : 0u, vk, 0, 16, kt + i * 1024,
+              lds_bytes, vk == kPadOffset);
+    check_dma("vd", a.vd + b * a.svd.b + hkv * a.svd.h + anchor * a.svd.t,
+              nrows > 0 ? mapped_bytes(anchor, rows_total, (uint32_t)a.svd.t * 2u) : 0u, vv, 0, 16, vt + i * 1024,
+              lds_bytes, vv == kPadOffset);
+    return;
+  }
+  const int voffk = own.lane_offset(i, (int)a.skd.t * 2, a.D), voffv = own.lane_offset(i, (int)a.svd.t * 2, a.Dv);
+  check_dma("kd", a.kd + b * a.skd.b + hkv * a.skd.h + (int64_t)col0 * a.skd.t,
+            nrows > 0 ? (uint32_t)nrows * (uint32_t)a.skd.t * 2u : 0u, voffk, 0, 16, kt + i * 1024, lds_bytes,
+            voffk == kPadOffset);
+  check_dma("vd", a.vd + b * a.svd.b + hkv * a.svd.h + (int64_t)col0 * a.svd.t,
+            nrows > 0 ? (uint32_t)nrows * (uint32_t)a.svd.t * 2u : 0u, voffv, 0, 16, vt + i * 1024, lds_bytes,
+            voffv == kPadOffset);
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // forward / dQ: the ring of K+V tiles and the waves' own depth tiles.  `dq`: also dO, lse, delta reads, dq stores.
 // ROWS_PER_WAVE: 32 (forward on 32x32x16) or 16 * NB.
@@ -313,36 +378,7 @@ void walk_row_kernel(const KArgs& a_in, bool dq, int rows_per_wave, bool own_pos
         }
         const int row0 = ring_tile_row0(plan, it, BN);
         ctx(kname, (int)block, wave, lane, dep ? "ring depth tile" : "ring sequence tile");
-        for (int i = 0; i < Loader::N; i++) {
-          const uint32_t ldsK = kt + (uint32_t)ld.lds_elems(i) * 2, ldsV = ldsK + BN * HD * 2;
-          if (dep && a.Lv != a.L) {  // partially filled stream: one descriptor anchored at the first column's token
-            const int w0 = row0 / a.Lv, l0 = row0 - w0 * a.Lv;
-            const int64_t anchor = (int64_t)w0 * a.L, rows_total = (int64_t)a.T * a.L;
-            check_dma("kd", a.kd + b * a.skd.b + hkv * a.skd.h + anchor * a.skd.t,
-                      mapped_bytes(anchor, rows_total, (uint32_t)a.skd.t * 2u),
-                      ld.mapped_offset(i, l0, a.L, a.Lv, (int)a.skd.t * 2, a.D), 0, 16, ldsK, lds_bytes, ld.pads(a.D));
-            check_dma("vd", a.vd + b * a.svd.b + hkv * a.svd.h + anchor * a.svd.t,
-                      mapped_bytes(anchor, rows_total, (uint32_t)a.svd.t * 2u),
-                      ld.mapped_offset(i, l0, a.L, a.Lv, (int)a.svd.t * 2, a.Dv), 0, 16, ldsV, lds_bytes, ld.pads(a.Dv));
-            // a lane in range must have fetched a slot that holds data
-            const int rel = mapped_row(l0, Loader::rows_before(i) + ld.row_in_pass, a.L, a.Lv);
-            if ((anchor + rel) % a.L >= a.Lv) fail("mapped depth tile reads slot %d of %d filled", (int)((anchor + rel) % a.L), a.Lv);
-          } else if (WIDE_ADDR) {
-            const int row_end = dep ? a.T * a.L : a.T;
-            const uint16_t* kb = dep ? a.kd + b * a.skd.b + hkv * a.skd.h : a.k + b * a.sk.b + hkv * a.sk.h;
-            const uint16_t* vb = dep ? a.vd + b * a.svd.b + hkv * a.svd.h : a.v + b * a.sv.b + hkv * a.sv.h;
-            const int64_t ks = dep ? a.skd.t : a.sk.t, vs = dep ? a.svd.t : a.sv.t;
-            check_dma(dep ? "kd" : "k", kb + (int64_t)row0 * ks, Loader::anchored_bytes(ks, row0, row_end),
-                      ld.lane_offset((int)ks * 2, a.D), Loader::rows_before(i) * (int)ks * 2, 16, ldsK, lds_bytes, ld.pads(a.D));
-            check_dma(dep ? "vd" : "v", vb + (int64_t)row0 * vs, Loader::anchored_bytes(vs, row0, row_end),
-                      ld.lane_offset((int)vs * 2, a.Dv), Loader::rows_before(i) * (int)vs * 2, 16, ldsV, lds_bytes, ld.pads(a.Dv));
-          } else {
-            check_dma(dep ? "kd" : "k", srcK.base, srcK.nbytes, srcK.voff, Loader::source_soffset(srcK, row0, i), 16, ldsK,
-                      lds_bytes, ld.pads(a.D));
-            check_dma(dep ? "vd" : "v", srcV.base, srcV.nbytes, srcV.voff, Loader::source_soffset(srcV, row0, i), 16, ldsV,
-                      lds_bytes, ld.pads(a.Dv));
-          }
-        }
+        ring_tile_loads<HD, NT, WIDE_ADDR>(a, b, hkv, ld, srcK, srcV, row0, dep, a.Lv != a.L, kt, lds_bytes, "k", "v");
       }
       // the wave's own depth columns, 32 at a time through a private K tile and V tile
       if (own_depth) {
@@ -398,26 +434,7 @@ void walk_row_kernel(const KArgs& a_in, bool dq, int rows_per_wave, bool own_pos
                 ctx(kname, (int)block, wave, lane, "own depth tile");
                 continue;
               }
-              if (a.Lv != a.L) {
-                const int w0 = col0 / a.Lv, l0 = col0 - w0 * a.Lv;
-                const int64_t anchor = (int64_t)w0 * a.L, rows_total = (int64_t)a.T * a.L;
-                const int vk = own.mapped_offset(i, l0, a.L, a.Lv, nrows, (int)a.skd.t * 2, a.D);
-                const int vv = own.mapped_offset(i, l0, a.L, a.Lv, nrows, (int)a.svd.t * 2, a.Dv);
-                check_dma("kd", a.kd + b * a.skd.b + hkv * a.skd.h + anchor * a.skd.t,
-                          nrows > 0 ? mapped_bytes(anchor, rows_total, (uint32_t)a.skd.t * 2u) : 0u, vk, 0, 16, kt + set + i * 1024,
-                          lds_bytes, vk == kPadOffset);
-                check_dma("vd", a.vd + b * a.svd.b + hkv * a.svd.h + anchor * a.svd.t,
-                          nrows > 0 ? mapped_bytes(anchor, rows_total, (uint32_t)a.svd.t * 2u) : 0u, vv, 0, 16, vt + set + i * 1024,
-                          lds_bytes, vv == kPadOffset);
-                continue;
-              }
-              const int voffk = own.lane_offset(i, (int)a.skd.t * 2, a.D), voffv = own.lane_offset(i, (int)a.svd.t * 2, a.Dv);
-              check_dma("kd", a.kd + b * a.skd.b + hkv * a.skd.h + (int64_t)col0 * a.skd.t,
-                        nrows > 0 ? (uint32_t)nrows * (uint32_t)a.skd.t * 2u : 0u, voffk, 0, 16, kt + set + i * 1024, lds_bytes,
-                        voffk == kPadOffset);
-              check_dma("vd", a.vd + b * a.svd.b + hkv * a.svd.h + (int64_t)col0 * a.svd.t,
-                        nrows > 0 ? (uint32_t)nrows * (uint32_t)a.svd.t * 2u : 0u, voffv, 0, 16, vt + set + i * 1024, lds_bytes,
-                        voffv == kPadOffset);
+              own_tile_load<HD>(a, b, hkv, own, i, col0, nrows, a.Lv != a.L, kt + set, vt + set, lds_bytes);
             }
           }
           // dQ kernel handing P and dS of its rows' visible depth columns to the depth-gradient kernel: lane (n, q4)
@@ -1211,6 +1228,100 @@ void walk_norm(int rows, int dim) {
   require_full("y");
 }
 
+// The attention of attend_tail_kernel: the forward kernel's body on RowBlock shapes.  Query rows, the ring of each key/value head (half the
+// waves and half the ring each where there are two), both private sets of depth tiles, the rows left for the dense part; who has which
+// part of LDS while the ring is in use (first set beside it) and after its last tile (second set over it).
+template <int C, int NB, int KV_HEADS>
+void walk_attention(bool fp16, const KArgs& a, const char* k_name, const char* v_name) {
+  constexpr int BM = 16 * NB, G = C / 64 / KV_HEADS, WORK = BM * G / 32, HD = 64, BN = 64;
+  typedef RowBlock<KV_HEADS, WORK> Shape;
+  constexpr int W = Shape::W, NT = 64 * W, NST = Shape::NST, DIST = Shape::DIST, ROWS = 32 * WORK;
+  static_assert(ROWS == BM * G && W * KV_HEADS == 8 && Shape::APART, "a head's query rows of the workgroup's tokens");
+  const char* kname = "attend_tail_kernel";
+  const uint32_t table = fp16 ? 0 : MODA_HIP_GELU_TABLE_BYTES, X = table, H = X + BM * C * 2;  // bytes
+  const uint32_t behind = H + attend_ring<Shape, BM>() * 2, lds_bytes = behind + KV_HEADS * WORK * 32 * HD * 2;
+  if (lds_bytes > 160 * 1024) fail("%u bytes of LDS", lds_bytes);
+  typedef AsyncTileLoader<HD, BN, NT> Loader;
+  typedef WaveTileLoader<HD> Own;
+  const bool own_depth = waves_own_depth(a, a.L);
+  for (int block = 0; block < attend_tail_blocks(a, BM); block++) {
+    const AttendTailPlace place = attend_tail_place(a, block, BM);
+    const int b = place.b, qt = place.tile;
+    if (place.first_row != b * a.T + qt * BM || qt < 0 || qt * BM >= a.T) fail("%s: tile %d of sequence %d", kname, qt, b);
+    const RowTilePlan plan = row_tile_plan(a, qt, ROWS, BN, a.L > 0 && !own_depth);
+    const int ntiles = plan.n_seq + plan.n_dep;
+    // owners of LDS, 16 bytes each: while the ring is in use, and after it; times an element of the attention rows was written
+    static std::vector<int> during, after;  // (static: a walk may end in the middle)
+    static std::vector<uint8_t> left;
+    during.assign(lds_bytes / 16, -1);
+    after.assign(lds_bytes / 16, -1);
+    left.assign(BM * C / 4, 0);
+    const auto take = [lds_bytes, kname](std::vector<int>& lds, uint32_t from, uint32_t bytes, int who) {
+      for (uint32_t i = from / 16; i < (from + bytes) / 16; i++) {
+        if (from + bytes > lds_bytes || (lds[i] != -1 && lds[i] != who)) fail("%s: byte %u of LDS is another's", kname, 16 * i);
+        lds[i] = who;
+      }
+    };
+    for (int tid = 0; tid < 512; tid++) {
+      const int lane = tid & 63, head = tid / NT, wave = tid % NT / 64, who = tid / 64;  // (wave: of the head's)
+      const bool idle = wave >= WORK;
+      const uint32_t ring = H + (uint32_t)head * NST * 2 * BN * HD * 2;
+      const int r = qt * ROWS + wave * 32 + (lane & 31);
+      ctx(kname, block, who, lane, "Q register rows");
+      if (!idle && r < a.Tq)
+        for (int e = 8 * (lane >> 5); e < HD; e += 16) check_access("q", a.q + b * a.sq.b + head * a.sq.h + (int64_t)r * a.sq.t + e, 16, false);
+      Loader ld;
+      ld.init(tid % NT);
+      auto srcK = ld.source(a.k + b * a.sk.b + head * a.sk.h, a.sk.t, 0, a.T, a.D), srcV = ld.source(a.v + b * a.sv.b + head * a.sv.h, a.sv.t, 0, a.T, a.Dv);
+      for (int it = 0; it < ntiles; it++) {
+        const bool dep = it >= plan.n_seq;
+        ctx(kname, block, who, lane, dep ? "ring depth tile" : "ring sequence tile");
+        for (int ahead = 1; ahead <= DIST; ahead++)
+          if ((it + ahead) % NST == it % NST) fail("%s: a tile on its way into the stage that is read", kname);
+        const uint32_t kt = ring + (uint32_t)(it % NST) * 2 * BN * HD * 2;
+        ring_tile_loads<HD, NT, false>(a, b, head, ld, srcK, srcV, ring_tile_row0(plan, it, BN), dep, true, kt, lds_bytes, k_name, v_name);
+        if (lane == 0)
+          for (int i = 0; i < Loader::N; i++)
+            for (uint32_t v : {0u, (uint32_t)BN * HD * 2}) take(during, kt + v + (uint32_t)ld.lds_elems(i) * 2, 1024, 100 + head);
+      }
+      const int rw0 = qt * ROWS + wave * 32;
+      if (own_depth && !idle && rw0 < a.Tq) {
+        const DepthSpan span = own_depth_span(a, rw0, 32);
+        Own own;
+        own.init(lane);
+        ctx(kname, block, who, lane, "own depth tile");
+        for (int j = 0; 32 * j < span.c_end - span.c_beg; j++) {
+          const int col0 = span.c_beg + 32 * j, nrows = imin(32, span.c_end - col0);
+          const uint32_t tile = 32 * HD * 2, kt = j % 2 ? ring + (uint32_t)wave * 2 * tile : X + (uint32_t)(head * WORK + wave) * tile;
+          const uint32_t vt = j % 2 ? kt + tile : behind + (uint32_t)(head * WORK + wave) * tile;
+          for (int i = 0; i < Own::N; i++) own_tile_load<HD>(a, b, head, own, i, col0, nrows, true, kt, vt, lds_bytes);
+          if (lane == 0)
+            for (uint32_t at : {kt, vt}) {
+              take(after, at, tile, who);
+              if (j == 0) take(during, at, tile, who);
+              if (j % 2 && (at < ring || at + tile > ring + NST * 2 * BN * HD * 2)) fail("%s: second private set outside of the head's ring", kname);
+            }
+        }
+      }
+      ctx(kname, block, who, lane, "attention rows");
+      for (int chunk = 0; !idle && chunk < HD / 8; chunk++) {
+        const int row = wave * 32 + (lane & 31), at = RowLayout<C>::off(row / G, (row % G * KV_HEADS + head) * 8 + chunk) + 4 * (lane >> 5);
+        if (at < 0 || at + 4 > BM * C || left[at / 4]++) fail("%s: element %d of the attention rows", kname, at);
+      }
+    }
+    for (size_t i = 0; i < left.size(); i++)
+      if (!left[i]) fail("%s: attention rows %zu of workgroup %d not written", kname, 4 * i, block);
+  }
+}
+void walk_attention(bool fp16, const KArgs& a, const char* k_name, const char* v_name) {
+  const int kv = a.Hkv, width = 64 * kv * a.Gf, bm = block_tail_rows((int64_t)a.B * a.T, a.compute_units);
+  if (!attend_tail_takes(width, kv * a.Gf, kv, bm)) fail("heads that the joined launch does not take");
+  if (width == 128) return bm == 32 ? walk_attention<128, 2, 1>(fp16, a, k_name, v_name) : walk_attention<128, 4, 1>(fp16, a, k_name, v_name);
+  if (width == 256 && kv == 1) return bm == 32 ? walk_attention<256, 2, 1>(fp16, a, k_name, v_name) : walk_attention<256, 4, 1>(fp16, a, k_name, v_name);
+  if (width == 256) return bm == 32 ? walk_attention<256, 2, 2>(fp16, a, k_name, v_name) : walk_attention<256, 4, 2>(fp16, a, k_name, v_name);
+  walk_attention<512, 2, 2>(fp16, a, k_name, v_name);
+}
+
 // A block's dense part in one launch: rows in and out, every product's weights, biases, norms and parts; what LDS holds.
 // Weights are read through their packed copies, each piece against the order that pack_weights_kernel leaves.
 // `tokens` > 0: with the attention before it (attend_tail_kernel), workgroups of BM tokens of one of rows / tokens sequences.
@@ -1560,6 +1671,19 @@ int main(int argc, char** argv) {
     for (int i = 8; i < argc; i++) parts.push_back(arg(i));
     walk_tail(std::string(argv[2]) == "fp16", arg(3) * arg(4), arg(5), arg(6), arg(7) != 0, parts, arg(4));
     printf("OK checked=%lld\n", g_checked);
+    return 0;
+  }
+  if (what == "attention") {  // dtype sequences tokens heads group slots filled mode chunk_tokens
+    Case c = {64, 64, 64, arg(5), arg(6), arg(7), arg(8), arg(9), arg(10), 0, arg(3), {}, {}, arg(4), arg(4)};
+    KArgs a = make_args(c);
+    const bool in_cache = c.Lv > 0 && c.Lv < c.L;  // k and v in the first free slot, as a stack has them
+    if (in_cache) {
+      a.k = a.kd + c.Lv * c.H * 64;
+      a.v = a.vd + c.Lv * c.H * 64;
+      a.sk = a.sv = Str3{a.skd.b, (int64_t)c.L * c.H * 64, 64};
+    }
+    walk_attention(std::string(argv[2]) == "fp16", a, in_cache ? "kd" : "k", in_cache ? "vd" : "v");
+    printf("OK checked=%lld dma_in_range=%lld dma_zero_filled=%lld\n", g_checked, g_dma_in, g_dma_out);
     return 0;
   }
   if (what == "attend_tail_rule") {  // sequences tokens width heads kv_heads compute_units [slots [causal]]

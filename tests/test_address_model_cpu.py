@@ -6,7 +6,7 @@ and walks every (workgroup, wave, lane, trip) of a forward + backward launch: re
 descriptor with each lane's vector and scalar offset (the lanes that fetch past the tensors' head dim included),
 the row-statistics loads, the LDS targets against the launch's dynamic LDS size, and all stores; every output
 element must be written exactly once.  The fp32 matrix kernels, the launches that dQ and dK/dV share, the linear, layer-norm and
-depth-slot kernels, a stack's block tail and the packing of its weights are walked the same way.
+depth-slot kernels, a stack's block tail, the attention that joins it and the packing of its weights are walked the same way.
 
 The first case is the packed batch that once ended in a GPU memory fault on the packed instantiations of the
 256-wide kernels (switched off since).  The walk finds every access of it inside its tensor: the fault is not an
@@ -371,6 +371,46 @@ def test_attention_with_block_tail(walker, case):
         e = dict(os.environ, **({"WALKER_SHRINK": shrink} if shrink else {}))
         out = subprocess.run([walker, "attend_tail", *map(str, case)], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=e, timeout=600)
         assert out.returncode == (1 if shrink else 0) and ("VIOLATION" if shrink else "OK checked") in out.stdout, (shrink, out.stdout)
+
+
+@pytest.mark.parametrize("case", [
+    # dtype, sequences, tokens, key/value heads, query heads on each, slots, filled ones, mode, chunk tokens: the cases of the GPU test of
+    # the joined launch; 32 tokens a workgroup and 64, waves that only load, one and two heads, none to many private tiles, rings of depth
+    ("bf16", 1, 1, 1, 4, 0, 0, "noncausal", 0),
+    ("bf16", 3, 1, 1, 2, 3, 2, "causal", 0),
+    ("fp16", 2, 31, 1, 4, 12, 11, "noncausal", 0),
+    ("bf16", 5, 33, 1, 2, 12, 1, "noncausal", 0),
+    ("bf16", 3, 64, 1, 4, 5, 5, "causal", 0),
+    ("bf16", 2, 65, 1, 4, 40, 21, "noncausal", 0),
+    ("fp16", 2, 300, 1, 2, 6, 4, "causal", 0),
+    ("bf16", 2, 261, 1, 4, 0, 0, "causal", 0),
+    ("bf16", 2, 100, 1, 4, 12, 7, "chunk_visible", 16),
+    ("bf16", 2, 150, 1, 2, 3, 2, "chunk_visible", 48),
+    ("bf16", 65, 129, 1, 4, 12, 11, "noncausal", 0),
+    ("fp16", 65, 129, 1, 2, 4, 3, "causal", 0),
+    ("bf16", 84, 100, 1, 4, 6, 5, "chunk_visible", 16),
+    ("bf16", 84, 100, 1, 2, 3, 2, "chunk_visible", 48),
+    ("bf16", 3, 33, 2, 2, 12, 11, "noncausal", 0),
+    ("fp16", 2, 261, 2, 4, 6, 2, "causal", 0),
+    ("bf16", 1, 1, 2, 4, 0, 0, "noncausal", 0),
+    ("bf16", 64, 129, 2, 2, 4, 3, "noncausal", 0),
+    ("bf16", 85, 100, 2, 2, 6, 5, "chunk_visible", 16),
+    ("bf16", 2, 150, 2, 4, 3, 2, "chunk_visible", 48),
+], ids=lambda c: "-".join(map(str, c)))
+def test_attention_of_the_joined_launch(walker, case):
+    """What test_attention_with_block_tail leaves out: the attention before the dense part, whose shapes no forward launch has."""
+    args = [walker, "attention", *map(str, case[:7]), str(MODES[case[7]]), str(case[8])]
+    small = case[1] * case[2] <= 600
+    for shrink in (None, "q:2", "k:2", "v:2", "kd:2", "vd:2") if small else (None, "q:2"):
+        in_cache = 0 < case[6] < case[5]
+        if shrink and (shrink[0] in "kv" and (case[5] == 0 if shrink[1] == "d" else in_cache)):
+            continue  # a tensor that the case does without
+        e = dict(os.environ, **({"WALKER_SHRINK": shrink} if shrink else {}))
+        out = subprocess.run(args, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, env=e, timeout=600)
+        if shrink and shrink[1] == "d" and in_cache and case[6] + 1 < case[5]:
+            assert "OK checked" in out.stdout, (shrink, out.stdout)  # the last slot holds nothing
+        else:
+            assert out.returncode == (1 if shrink else 0) and ("VIOLATION" if shrink else "OK checked") in out.stdout, (shrink, out.stdout)
 
 
 @pytest.mark.parametrize("case", [
