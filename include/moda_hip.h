@@ -327,8 +327,8 @@ int moda_hip_block_tail(const moda_hip_block_tail_args* args, void* stream);
  * columns are summed, which follows a workgroup's rows), without o and lse (args->attention is not read).
  * For tokens as the tail's rows (args->rows = desc's B * T, token by token), H = 1 or 2 key/value heads and G = 2 or 4 query heads
  * of 64 on each (feature (g * H + h) * 64 + i of a token's attention output: element i of head h of its query row g), args->width
- * 64 G H (512: as many rows as go 32 a workgroup, 32 times the compute units), no packed batch;
- * MODA_HIP_EUNSUPPORTED otherwise.  The outputs of the tail may be the buffers of q and of the residual, but not of k, v, kd, vd:
+ * 64 G H (512: as many rows as go 32 a workgroup, 32 times the compute units), no packed batch, no (batch, head) slice of k, v, kd
+ * or vd of 2 GiB and more (which moda_hip_fwd takes); MODA_HIP_EUNSUPPORTED otherwise.  The outputs of the tail may be the buffers of q and of the residual, but not of k, v, kd, vd:
  * slots of the depth cache that this call does not read, and rows of k, v elsewhere, are fine.
  */
 int moda_hip_attend_block_tail(const moda_hip_desc* desc, const void* q, const void* k, const void* v, const void* kd, const void* vd,

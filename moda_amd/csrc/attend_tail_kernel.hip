@@ -1,15 +1,17 @@
 // A block's attention and its dense part (block_tail_kernel.hip) in one launch, without gradients: a workgroup takes the query rows of
-// 64 (or 32) tokens of a sequence, two or four heads of 64 on each of one or two key/value heads, through the forward kernel's body (fwd.h) and leaves their
-// attention output in LDS, where the dense part takes it up.  Bits as from the two launches.
+// 64 (or 32) tokens of a sequence, two or four heads of 64 on each of one or two key/value heads, through the forward kernel's body (fwd.h)
+// and leaves their attention output in LDS, where the dense part takes it up.  Bits as from the two launches.  For short sequences, and long
+// ones of one round: tuning.h, attention_joins_tail, says which and what they take either way.
 //
 // Both launches are short, and a good part of a short launch is its start and end.  Twelve blocks of width 256 on 64 x 197 tokens: 557 ->
 // 516 us.  Six blocks, apart and joined: 64 x 197 tokens 281 and 256 (fp16 312 and 281), 16 x 197 206 and 184, 8 x 50 194 and 172, 2 x
 // 8192 1134 and 1086; width 128, 64 x 197 178 and 153, 4 x 197 139 and 119; two key/value heads, width 256, 64 x 197 298 and 283, 36 x 197
-// 239 and 217, width 512, 36 x 197 508 and 486.  Of 92 k cycles of the largest (width 256, eleven slots)
-// 9.7 k are the first loads, 12.6 k four tiles of keys, 9 k three private tiles of depth slots, the rest the dense part.  What the dense
-// part wants from memory at its start, the residual rows and the table, travels with the attention's first tiles and waits in registers;
-// ring and private K tiles lie where the hidden activations and the rows go later.  Tried: no barriers where the ring holds all tiles, a
-// higher priority for every second wave of a SIMD: 519 and 521 us where this takes 517.
+// 239 and 217, width 512, 36 x 197 508 and 486.  Of 92 k cycles of the largest (width 256, eleven slots) 9.7 k are the first
+// loads, 12.6 k four tiles of keys, 9 k three private tiles of depth slots, the rest the dense part.  What the dense part wants from memory
+// at its start, the residual rows and the table, travels with the attention's first tiles and waits in registers; ring and private K tiles
+// lie where the hidden activations and the rows go later.  Registers of a wave: all 256 with 64 rows of width 256 and the norm before the
+// block, where bf16 spills five to seven; width 512 in fp16 eleven; no others, but 45 - 69 scalar ones with a depth stream.  Tried: no
+// barriers where the ring holds all tiles, a higher priority for every second wave of a SIMD: 519 and 521 us where this takes 517.
 #define MODA_SIDE_BY_SIDE
 #include "block_tail.h"
 

@@ -500,7 +500,9 @@ __global__ __launch_bounds__(64 * Shape::W, HD <= 64 ? 3 : 2) void fwd_kernel(co
 #ifdef MODA_SIDE_BY_SIDE
   __syncthreads();
   if (idle) return;
-  const float inv = l > 0.f ? 1.f / l : 0.f;  // (a row past the end sees nothing: zeros)
+  // (A row past the end comes with what the unmasked tiles gave its zero query, the mean of their V rows: whoever takes the rows keeps
+  // them apart and does not store it.)
+  const float inv = l > 0.f ? 1.f / l : 0.f;
 #pragma unroll
   for (int d = 0; d < DB; d++)
 #pragma unroll
