@@ -2419,6 +2419,21 @@ def test_norm_beside_weight_packing(gpu_device, rows, dim, n, dtype):
         assert torch.equal(a, c)
 
 
+def test_stack_whose_cache_slices_reach_two_gib(gpu_device):
+    """Such a stack goes without the joined launch, which does not reach all of its slices.  Causal: its first tokens against the stack on
+    them alone, whose slices are short and whose attention joins; the same bits."""
+    import moda_amd
+
+    say("CASE stack with slices of 2 GiB")
+    torch.manual_seed(5)
+    m = moda_amd.MoDAStack(128, 512, 2, 1, mlp_ratio=1.0, is_causal=True, ffn_kv=True).to(gpu_device, torch.bfloat16).eval().requires_grad_(False)
+    x = (0.5 * torch.randn(1, 16384, 128, device=gpu_device)).to(torch.bfloat16)  # 1024 slots of 128 bytes a token
+    with torch.no_grad():
+        got, want = m._forward_native(x), m._forward_native(x[:, :1000].contiguous())
+    assert got is not None and torch.isfinite(got.float()).all()
+    assert torch.equal(got[:, :1000], want)
+
+
 def test_norm_and_weight_packing_beyond_one_grid(gpu_device):
     """Rows and pieces of weights that a grid of 2^32 threads does not hold together: two launches, the bits of the two calls."""
     import ctypes
